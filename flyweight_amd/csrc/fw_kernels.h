@@ -34,6 +34,11 @@ int fw_rmsnorm_rows(const float* x, const float* weight, void* out, int out_dtyp
 // 1: out (float32) += result (the residual sum).
 int fw_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, const float* bias,
                     void* out, int out_dtype, int out_mode, int M, int N, int K, void* stream);
+// The same for float32 operands aligned to 16 bytes and K a multiple of 4, on the float32 matrix instruction; each output is
+// summed in an order that depends on K alone. mode 0: store as out_dtype; 1: out (float32) += result; 2: w is [2N][K], gate
+// rows then up rows, out (float32) = silu(a . gate^T) * (a . up^T), no bias.
+int fw_gemm_float32(const float* a, const float* w, const float* bias, void* out, int out_dtype, int mode,
+                    int M, int N, int K, void* stream);
 
 // bfloat16 matrix products on the matrix cores, float32 accumulation. a [M][K], w [N][K], K a
 // multiple of 8. mode 0: out = a . w^T (+ bias) stored as out_dtype (also 2, here and in every storing product below:

@@ -1,0 +1,79 @@
+"""The product of float32 operands on the float32 matrix instruction: edges of its tiles, of K's quarters and groups of 16,
+its three epilogues, and that a row's result does not depend on the rows beside it."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from flyweight_amd.kernels import ops as module
+    module.library()
+    return module
+
+
+def draw(*shape, seed=0):
+    generator = torch.Generator().manual_seed(seed)
+    return torch.randn(*shape, generator=generator)
+
+
+def bound(a, w):
+    """K rounded products and sums: at most (K + 1) * 2^-24 of the sum of the products' sizes."""
+    return (a.shape[1] + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+
+
+# one row and the last of a tile, one past each tile's edge; outputs that fill no tile; K below a quarter's group, of whole
+# groups, with a piece of a group left in the last or in an earlier quarter, and one quarter empty
+SHAPES = [(1, 16, 64), (1, 1024, 4608), (16, 33, 100), (17, 64, 4), (32, 65, 20), (33, 130, 132), (64, 96, 208), (65, 1000, 1024),
+          (129, 48, 36), (301, 515, 76), (3, 9216, 12)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_product_of_float32_operands(ops, M, N, K):
+    a, w, bias = draw(M, K), draw(N, K, seed=1), draw(N, seed=2)
+    limit, exact = bound(a, w), a.double() @ w.double().T
+    A, W, B = a.to(DEV), w.to(DEV), bias.to(DEV)
+    assert ((ops.gemm(A, W).cpu().double() - exact).abs() <= limit).all()
+    with_bias = ops.gemm(A, W, B).cpu().double()
+    assert ((with_bias - exact - bias.double()).abs() <= limit + 2.0 ** -23 * with_bias.abs()).all()
+    residual = draw(M, N, seed=3)
+    into = residual.to(DEV)
+    ops.gemm(A, W, accumulate_into=into)
+    total = exact + residual.double()
+    assert ((into.cpu().double() - total).abs() <= limit + 2.0 ** -23 * total.abs()).all()
+    rounded = ops.gemm(A, W, out_dtype=torch.bfloat16).cpu().double()
+    assert ((rounded - exact).abs() <= limit + 2.0 ** -8 * exact.abs()).all()
+
+
+@pytest.mark.parametrize("M,F,K", [(1, 16, 64), (5, 77, 100), (33, 130, 132), (301, 515, 76), (64, 4608, 1024)])
+def test_gated_product_of_float32_operands(ops, M, F, K):
+    a, w = draw(M, K) * K ** -0.5, draw(2 * F, K, seed=1)
+    limit, sums = bound(a, w), a.double() @ w.double().T
+    g, u = sums[:, :F], sums[:, F:]
+    exact = torch.nn.functional.silu(g) * u
+    # silu's slope is below 1.1; the unit's own roundings are a few units in the last place
+    allowed = 1.1 * limit[:, :F] * u.abs() + limit[:, F:] * g.abs() + 2.0 ** -20 * exact.abs() + 1e-12
+    assert ((ops.gemm_swiglu(a.to(DEV), w.to(DEV)).cpu().double() - exact).abs() <= allowed).all()
+
+
+def test_a_row_does_not_depend_on_the_rows_beside_it(ops):
+    for N, K in ((1024, 4608), (70, 36), (9216, 1024)):
+        a, w = draw(330, K).to(DEV), draw(N, K, seed=1).to(DEV)
+        whole = ops.gemm(a, w)
+        for first, last in ((0, 1), (7, 23), (40, 57), (3, 36), (250, 330), (17, 301)):
+            assert torch.equal(ops.gemm(a[first:last].contiguous(), w), whole[first:last])
+        gated = ops.gemm_swiglu(a, w)
+        assert torch.equal(ops.gemm_swiglu(a[5:6].contiguous(), w)[0], gated[5])
+
+
+def test_what_its_loads_cannot_take_goes_to_the_plain_tiles(ops):
+    a, w = draw(5, 66), draw(40, 66, seed=1)                       # K no multiple of 4
+    exact = a.double() @ w.double().T
+    assert ((ops.gemm(a.to(DEV), w.to(DEV)).cpu().double() - exact).abs() <= bound(a, w)).all()
+    flat = torch.cat([torch.zeros(1), draw(5, 64).reshape(-1)]).to(DEV)     # rows that do not start at 16 bytes
+    b, v = flat[1:].view(5, 64), draw(40, 64, seed=1)
+    exact = b.cpu().double() @ v.double().T
+    assert ((ops.gemm(b, v.to(DEV)).cpu().double() - exact).abs() <= bound(b.cpu(), v)).all()
