@@ -364,10 +364,15 @@ int fw_token_shift_mix(const float* x, const float* norm_weight, float eps, int 
 int fw_tanh_rows(const float* x, void* out, int out_dtype, long long count, void* stream);
 // Per head: o_t = S^T r_t + (r_t . (u k_t)) v_t; S <- diag(exp(-exp(a_t + w0))) S + k_t v_t^T. r, k, v float32 rows of
 // rkv_stride floats (heads * dim used), a rows of a_stride; w0 [heads * dim], u [heads * dim]; state float32
-// [slots][heads][dim (key)][dim (value)]; out float32 [rows][heads * dim].
+// [slots][heads][dim (key)][dim (value)]; out float32 [rows][heads * dim]. With chunks > 0 segments of more than long_rows rows
+// are walked in chunks of fw_wkv_chunk_rows() rows side by side (places as for fw_decay_recurrence; workspace: chunks * heads *
+// dim * (dim + 1) floats).
 int fw_wkv_recurrence(const float* r, const float* k, const float* v, int rkv_stride, const float* a, int a_stride,
                       const float* w0, const float* u, float* state, int slots, float* out, const int32_t* seg_row0,
-                      const int32_t* seg_slot, int rows, int segments, int heads, int dim, void* stream);
+                      const int32_t* seg_slot, int rows, int segments, int heads, int dim, const int32_t* chunk_seg,
+                      const int32_t* chunk_row0, const int32_t* seg_chunk0, int chunks, int long_rows, int all_long,
+                      float* workspace, void* stream);
+int fw_wkv_chunk_rows(void);
 
 // ---- a mixture of feed-forward units chosen per token ------------------------------------------------------
 // chosen / weight [rows][top]: the `top` largest of logits[r] + bias (float32 [rows][experts]; ties: the lowest

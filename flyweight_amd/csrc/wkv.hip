@@ -120,22 +120,30 @@ __device__ __forceinline__ float wkv_row_sum(float x) {
     return x;
 }
 
-template <int RPT, int WKV_CHUNK>
+//
+// CUT: a workgroup walks a chunk of WKV_ROWS rows of a long segment (chunk_seg, chunk_row0) from a zero state; the state
+// behind it goes to local[chunk][head] and the product of its decays per key channel to shrink[chunk][head]. Otherwise a
+// workgroup walks a segment, and leaves those of more than long_rows rows alone (long_rows > 0).
+#define WKV_ROWS 64
+template <int RPT, int WKV_CHUNK, bool CUT>
 __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
     const float* __restrict__ r, const float* __restrict__ k, const float* __restrict__ v, int rkv_stride,
     const float* __restrict__ a, int a_stride, const float* __restrict__ w0, const float* __restrict__ u, float* __restrict__ state,
-    float* __restrict__ out, const int32_t* __restrict__ seg_row0, const int32_t* __restrict__ seg_slot, int heads, int dim) {
+    float* __restrict__ out, const int32_t* __restrict__ seg_row0, const int32_t* __restrict__ seg_slot, int heads, int dim, int long_rows,
+    const int32_t* __restrict__ chunk_seg, const int32_t* __restrict__ chunk_row0, float* __restrict__ local, float* __restrict__ shrink) {
     constexpr int DP = WKV_LANES * RPT;                 // key channels as the lanes hold them
     constexpr int TOKEN = 3 * DP + WKV_COLUMNS;         // a staged token: r, k, decay, the block's values
     constexpr int PIECES = (WKV_CHUNK * DP + 255) / 256;    // elements of a chunk's r (and k, and a) per thread, at most
     __shared__ __attribute__((aligned(16))) float staged[WKV_CHUNK * TOKEN];
     __shared__ float results[WKV_CHUNK * WKV_COLUMNS];
     constexpr int VALUE_PIECES = (WKV_CHUNK * WKV_COLUMNS + 255) / 256;     // of the block's values of a chunk per thread
-    const int seg = blockIdx.x, head = blockIdx.y, block = blockIdx.z;
-    const int local = threadIdx.x / WKV_LANES, part = threadIdx.x % WKV_LANES;
-    const int column = block * WKV_COLUMNS + local;
+    const int seg = CUT ? chunk_seg[blockIdx.x] : blockIdx.x, head = blockIdx.y, block = blockIdx.z;
+    const int own = threadIdx.x / WKV_LANES, part = threadIdx.x % WKV_LANES;
+    const int column = block * WKV_COLUMNS + own;
     const bool live = column < dim;
-    const int first = seg_row0[seg], count = seg_row0[seg + 1] - first;
+    const int first = CUT ? chunk_row0[blockIdx.x] : seg_row0[seg];
+    const int rows = seg_row0[seg + 1] - first, count = CUT && rows > WKV_ROWS ? WKV_ROWS : rows;
+    if (!CUT && long_rows > 0 && count > long_rows) return;     // its chunks are walked side by side
     const size_t head_at = (size_t)head * dim;
     // This thread's elements of every chunk: element e = thread + 256 i of the chunk's [tokens][dim] block of r,
     // of k and of a alike (token e / dim, channel e % dim), and one of the block's values (token thread / 16,
@@ -201,12 +209,14 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
             if (value_token[j] >= 0 && value_token[j] < tokens) staged[value_token[j] * TOKEN + 3 * DP + threadIdx.x % WKV_COLUMNS] = held_v[j];
     };
     ask(0);
-    float* mine = state + ((size_t)seg_slot[seg] * heads + head) * dim * dim + (live ? column : 0);
+    float* mine = (CUT ? local + ((size_t)blockIdx.x * heads + head) * dim * dim
+                       : state + ((size_t)seg_slot[seg] * heads + head) * dim * dim) + (live ? column : 0);
+    float product = 1.0f;       // CUT, the first block: of this thread's channel's decays
     float S[RPT], bonus[RPT];
 #pragma unroll
     for (int t = 0; t < RPT; ++t) {
         const int key = part * RPT + t;
-        S[t] = (live && key < dim) ? mine[(size_t)key * dim] : 0.0f;
+        S[t] = (!CUT && live && key < dim) ? mine[(size_t)key * dim] : 0.0f;
         bonus[t] = key < dim ? u[head_at + key] : 0.0f;
     }
     __syncthreads();        // the zeros are in place
@@ -226,7 +236,7 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
                 k_next[t] = t0[DP + part * RPT + t];
                 w_next[t] = t0[2 * DP + part * RPT + t];
             }
-            v_next = t0[3 * DP + local];
+            v_next = t0[3 * DP + own];
         };
         fetch(0);
         for (int token = 0; token < tokens; ++token) {
@@ -241,7 +251,7 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
             fetch(token + 1 < staged_tokens ? token + 1 : token);       // (behind the chunk's last token: read again, not used)
             read = wkv_row_sum(read);
             ruk = wkv_row_sum(ruk);
-            if (part == 0) results[token * WKV_COLUMNS + local] = fmaf(ruk, value, read);
+            if (part == 0) results[token * WKV_COLUMNS + own] = fmaf(ruk, value, read);
         }
         // (barriers that order LDS traffic only: the next chunk's loads stay in flight across them)
         fw_lds_barrier();
@@ -251,9 +261,13 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
             if (block * WKV_COLUMNS + c < dim)
                 out[((size_t)first + base + token) * heads * dim + head_at + block * WKV_COLUMNS + c] = results[i];
         }
+        if (CUT && block == 0 && threadIdx.x < dim)
+            for (int token = 0; token < tokens; ++token) product *= staged[token * TOKEN + 2 * DP + threadIdx.x];
+        if constexpr (CUT) fw_lds_barrier();
         if (more) put(base + WKV_CHUNK);
         fw_lds_barrier();
     }
+    if (CUT && block == 0 && threadIdx.x < dim) shrink[((size_t)blockIdx.x * heads + head) * dim + threadIdx.x] = product;
     if (live) {
 #pragma unroll
         for (int t = 0; t < RPT; ++t) {
@@ -263,26 +277,185 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
     }
 }
 
+// ---- a long segment in chunks ---------------------------------------------------------------------
+// A segment's serial walk is 0.2 us a row on heads x dim / 16 workgroups, whatever the chip could do beside it. Cut into chunks
+// of WKV_ROWS rows, the walks run side by side from zero states (the kernel above, CUT); with P_t the product of the
+// chunk's decays before row t and S_in the state ahead of the chunk,
+//     o_t += S_in^T (P_t r_t);      S_out = diag(shrink) S_in + local
+// Bound by the walks' instructions once the chip is full of them. 2,048 rows of 32 heads of 64 channels: 420 us in order ->
+// 108 us (the walks) + 14 (the states) + 20 (the read-outs, which read and write every output once more).
+
+// local[chunk] becomes the state ahead of the chunk, the slot moves on to the state behind the segment. A thread per element of
+// (segment, head): loads and one multiply-add per chunk, eight chunks asked for at once.
+__global__ __launch_bounds__(256) void wkv_chunk_state_kernel(float* __restrict__ local, const float* __restrict__ shrink, float* __restrict__ state,
+                                                              const int32_t* __restrict__ seg_chunk0, const int32_t* __restrict__ seg_slot,
+                                                              int heads, int dim) {
+    const int seg = blockIdx.x, head = blockIdx.y;
+    const int begin = seg_chunk0[seg], chunks = seg_chunk0[seg + 1] - begin;
+    const int i = blockIdx.z * 256 + threadIdx.x;
+    if (chunks <= 0 || i >= dim * dim) return;
+    float* slot = state + ((size_t)seg_slot[seg] * heads + head) * dim * dim + i;
+    float* at = local + ((size_t)begin * heads + head) * dim * dim + i;
+    const float* decay = shrink + ((size_t)begin * heads + head) * dim + i / dim;
+    const size_t step = (size_t)heads * dim * dim, decay_step = (size_t)heads * dim;
+    float S = *slot;
+    for (int c = 0; c < chunks; c += 8) {
+        float own[8], by[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int chunk = c + u < chunks ? c + u : chunks - 1;
+            own[u] = at[(size_t)chunk * step];
+            by[u] = decay[(size_t)chunk * decay_step];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            if (c + u >= chunks) break;
+            at[(size_t)(c + u) * step] = S;
+            S = fmaf(by[u], S, own[u]);
+        }
+    }
+    *slot = S;
+}
+
+// out[t] += S_in^T (P_t r_t) of a chunk and head. The threads form P_t r_t in LDS, DP channels by 256 / DP runs of rows: a run's
+// decays first (their product tells the later runs where to start), then its rows. The product runs on the matrix cores in
+// float32 (v_mfma_f32_32x32x2f32), a 32 x 32 tile a wave at a time; a step takes eight channels, lanes 0..31 the first four,
+// lanes 32..63 the next four. S_in comes straight from memory.
+typedef __attribute__((ext_vector_type(16))) float wkv_f32x16;
+typedef __attribute__((ext_vector_type(4))) float wkv_f32x4;
+template <int DP>
+__global__ __launch_bounds__(256) void wkv_chunk_read_kernel(const float* __restrict__ r, int rkv_stride, const float* __restrict__ a, int a_stride,
+                                                             const float* __restrict__ w0, const float* __restrict__ local, float* __restrict__ out,
+                                                             const int32_t* __restrict__ chunk_seg, const int32_t* __restrict__ chunk_row0,
+                                                             const int32_t* __restrict__ seg_row0, int heads, int dim) {
+    constexpr int RUNS = 256 / DP, RUN = WKV_ROWS / RUNS, PITCH = DP + 4;
+    extern __shared__ __attribute__((aligned(16))) float scaled[];      // [WKV_ROWS][PITCH], then the runs' products [RUNS][DP]
+    float* products = scaled + WKV_ROWS * PITCH;
+    const int chunk = blockIdx.x, head = blockIdx.y;
+    const int row0 = chunk_row0[chunk], end = seg_row0[chunk_seg[chunk] + 1];
+    const int tokens = end - row0 < WKV_ROWS ? end - row0 : WKV_ROWS;
+    const size_t head_at = (size_t)head * dim;
+    const int channel = threadIdx.x % DP, run = threadIdx.x / DP;
+    const int safe = channel < dim ? channel : dim - 1;
+    float decay[RUN], query[RUN];
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) {                     // rows past the end: the last one again, not stored
+        const int token = run * RUN + t < tokens ? run * RUN + t : tokens - 1;
+        decay[t] = a[(size_t)(row0 + token) * a_stride + head_at + safe];
+        query[t] = r[(size_t)(row0 + token) * rkv_stride + head_at + safe];
+    }
+    const float base = w0[head_at + safe];
+    float product = 1.0f;
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) {
+        decay[t] = expf(-expf(decay[t] + base));
+        product *= decay[t];
+    }
+    products[run * DP + channel] = product;
+    __syncthreads();
+    float before = 1.0f;
+    for (int u = 0; u < run; ++u) before *= products[u * DP + channel];
+#pragma unroll
+    for (int t = 0; t < RUN; ++t) {
+        scaled[(run * RUN + t) * PITCH + channel] = channel < dim ? query[t] * before : 0.0f;
+        before *= decay[t];
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, half = lane >> 5, within = lane & 31;
+    const float* S_in = local + ((size_t)chunk * heads + head) * dim * dim;
+    const int tiles = WKV_ROWS / 32 * ((dim + 31) / 32);
+    for (int tile = wave; tile < tiles; tile += 4) {
+        const int token0 = tile % (WKV_ROWS / 32) * 32, col = tile / (WKV_ROWS / 32) * 32 + within;
+        const int from = col < dim ? col : dim - 1;
+        float* to = out + (size_t)(row0 + token0) * heads * dim + head_at + col;
+        const size_t step = (size_t)heads * dim;
+        float old[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int t = 8 * (i >> 2) + 4 * half + (i & 3);
+            old[i] = token0 + t < tokens && col < dim ? to[(size_t)t * step] : 0.0f;
+        }
+        wkv_f32x16 acc;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+        const float* rows = scaled + (token0 + within) * PITCH + 4 * half;
+#pragma unroll
+        for (int c = 0; c < DP; c += 8) {
+            const wkv_f32x4 x = *reinterpret_cast<const wkv_f32x4*>(rows + c);
+            float b[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int key = c + 4 * half + e;       // (channels past dim meet zeros; they are read at the last one)
+                b[e] = S_in[(size_t)(key < dim ? key : dim - 1) * dim + from];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], b[e], acc, 0, 0, 0);
+        }
+        fw_mfma_drain();
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int t = 8 * (i >> 2) + 4 * half + (i & 3);
+            if (token0 + t < tokens && col < dim) to[(size_t)t * step] = old[i] + acc[i];
+        }
+    }
+}
+
+extern "C" int fw_wkv_chunk_rows(void) { return WKV_ROWS; }
+
 extern "C" int fw_wkv_recurrence(const float* r, const float* k, const float* v, int rkv_stride, const float* a, int a_stride,
                                  const float* w0, const float* u, float* state, int slots, float* out, const int32_t* seg_row0,
-                                 const int32_t* seg_slot, int rows, int segments, int heads, int dim, void* stream) {
+                                 const int32_t* seg_slot, int rows, int segments, int heads, int dim, const int32_t* chunk_seg,
+                                 const int32_t* chunk_row0, const int32_t* seg_chunk0, int chunks, int long_rows, int all_long,
+                                 float* workspace, void* stream) {
     FW_REQUIRE(rows >= 0 && segments >= 0 && heads > 0 && heads <= 65535 && slots > 0, "wkv_recurrence: bad sizes rows=%d segments=%d heads=%d", rows, segments, heads);
     FW_REQUIRE(dim >= 1 && dim <= 256, "wkv_recurrence: a head of %d channels (1..256)", dim);
     FW_REQUIRE(rkv_stride >= heads * dim && a_stride >= heads * dim, "wkv_recurrence: rows of %d / %d values do not hold %d heads of %d", rkv_stride, a_stride, heads, dim);
+    FW_REQUIRE(chunks >= 0 && (chunks == 0 || (chunk_seg && chunk_row0 && seg_chunk0 && workspace && long_rows > 0)),
+               "wkv_recurrence: chunks come with their places, a workspace and the length from which they are used");
     if (rows == 0 || segments == 0) return 0;
-    dim3 grid(segments, heads, (dim + WKV_COLUMNS - 1) / WKV_COLUMNS);
     hipStream_t s = (hipStream_t)stream;
-#define FW_WKV_LAUNCH(RPT, CHUNK) \
-    wkv_recurrence_kernel<RPT, CHUNK><<<grid, 256, 0, s>>>(r, k, v, rkv_stride, a, a_stride, w0, u, state, out, seg_row0, seg_slot, heads, dim)
-    // (the chunk's length changes what is staged together, not one sum: steps of single tokens take short chunks,
-    // whose bookkeeping at the start is a few loads)
-    const bool few = rows <= 4 * segments;
-    if (dim <= 16) { if (few) FW_WKV_LAUNCH(1, 4); else FW_WKV_LAUNCH(1, 32); }
-    else if (dim <= 32) { if (few) FW_WKV_LAUNCH(2, 4); else FW_WKV_LAUNCH(2, 32); }
-    else if (dim <= 64) { if (few) FW_WKV_LAUNCH(4, 4); else FW_WKV_LAUNCH(4, 32); }
-    else if (dim <= 128) FW_WKV_LAUNCH(8, 8);
-    else FW_WKV_LAUNCH(16, 4);
+    float* shrink = workspace ? workspace + (size_t)chunks * heads * dim * dim : nullptr;
+#define FW_WKV_LAUNCH(RPT, CHUNK, CUT)                                                                                                     \
+    wkv_recurrence_kernel<RPT, CHUNK, CUT><<<dim3(CUT ? chunks : segments, heads, (dim + WKV_COLUMNS - 1) / WKV_COLUMNS), 256, 0, s>>>(    \
+        r, k, v, rkv_stride, a, a_stride, w0, u, state, out, seg_row0, seg_slot, heads, dim, chunks > 0 ? long_rows : 0, chunk_seg,        \
+        chunk_row0, workspace, shrink)
+    if (chunks == 0 || !all_long) {
+        // (the chunk's length changes what is staged together, not one sum: steps of single tokens take short chunks,
+        // whose bookkeeping at the start is a few loads)
+        const bool few = rows <= 4 * segments;
+        if (dim <= 16) { if (few) FW_WKV_LAUNCH(1, 4, false); else FW_WKV_LAUNCH(1, 32, false); }
+        else if (dim <= 32) { if (few) FW_WKV_LAUNCH(2, 4, false); else FW_WKV_LAUNCH(2, 32, false); }
+        else if (dim <= 64) { if (few) FW_WKV_LAUNCH(4, 4, false); else FW_WKV_LAUNCH(4, 32, false); }
+        else if (dim <= 128) FW_WKV_LAUNCH(8, 8, false);
+        else FW_WKV_LAUNCH(16, 4, false);
+        FW_LAUNCH_CHECK("wkv_recurrence");
+    }
+    if (chunks == 0) return 0;
+    if (dim <= 16) FW_WKV_LAUNCH(1, 32, true);
+    else if (dim <= 32) FW_WKV_LAUNCH(2, 32, true);
+    else if (dim <= 64) FW_WKV_LAUNCH(4, 32, true);
+    else if (dim <= 128) FW_WKV_LAUNCH(8, 8, true);
+    else FW_WKV_LAUNCH(16, 4, true);
 #undef FW_WKV_LAUNCH
-    FW_LAUNCH_CHECK("wkv_recurrence");
+    FW_LAUNCH_CHECK("wkv_recurrence (chunks)");
+    wkv_chunk_state_kernel<<<dim3(segments, heads, fw_ceil_div(dim * dim, 256)), 256, 0, s>>>(workspace, shrink, state, seg_chunk0, seg_slot, heads, dim);
+    FW_LAUNCH_CHECK("wkv_recurrence (states)");
+#define FW_WKV_READ(DP)                                                                                                                 \
+    wkv_chunk_read_kernel<DP><<<dim3(chunks, heads), 256, (WKV_ROWS * (DP + 4) + 256) * sizeof(float), s>>>(r, rkv_stride, a, a_stride, \
+        w0, workspace, out, chunk_seg, chunk_row0, seg_row0, heads, dim)
+    if (dim <= 64) FW_WKV_READ(64);
+    else if (dim <= 128) FW_WKV_READ(128);
+    else {
+        static bool configured = false;
+        if (!configured) {
+            hipError_t status = hipFuncSetAttribute((const void*)wkv_chunk_read_kernel<256>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                    (WKV_ROWS * 260 + 256) * sizeof(float));
+            FW_REQUIRE(status == hipSuccess, "wkv_recurrence: cannot reserve LDS: %s", hipGetErrorString(status));
+            configured = true;
+        }
+        FW_WKV_READ(256);
+    }
+#undef FW_WKV_READ
+    FW_LAUNCH_CHECK("wkv_recurrence (read)");
     return 0;
 }

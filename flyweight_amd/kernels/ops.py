@@ -1679,10 +1679,12 @@ def tanh_rows(x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
 
 
 def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.Tensor, w0: torch.Tensor, u: torch.Tensor,
-                   state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor, segments: int, heads: int, dim: int) -> torch.Tensor:
+                   state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor, segments: int, heads: int, dim: int,
+                   chunks: Optional[tuple] = None) -> torch.Tensor:
     """Per head o_t = S^T r_t + (r_t . (u k_t)) v_t, then S <- diag(exp(-exp(a_t + w0))) S + k_t v_t^T, over each segment's rows
     in order. ``r``, ``k``, ``v`` float32 [rows, heads dim] with one row stride (views of wider rows will do), ``a``
-    likewise; ``state`` float32 [slots, heads, dim, dim] is read and moved on. Returns float32 [rows, heads dim]."""
+    likewise; ``state`` float32 [slots, heads, dim, dim] is read and moved on. ``chunks``: as for ``decay_recurrence``. Returns
+    float32 [rows, heads dim]."""
     _dev(w0, u, state, seg_row0, seg_slot)
     rows = r.shape[0]
     width = heads * dim
@@ -1709,8 +1711,13 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.T
         if t.numel() < n:
             raise KernelError(f"wkv_recurrence: {name} holds {t.numel()} entries, needs {n}")
     out = torch.empty((rows, width), dtype=torch.float32, device=r.device)
+    places, count, *how = _chunks("wkv_recurrence", chunks, segments)
+    if count and library().fw_wkv_chunk_rows() != DECAY_CHUNK:
+        raise KernelError("the kernel library's chunks are of another length")
+    workspace = torch.empty(count * width * (dim + 1), dtype=torch.float32, device=r.device) if count else None
     _check(library().fw_wkv_recurrence(_p(r), _p(k), _p(v), stride(r), _p(a), stride(a), _p(w0), _p(u), _p(state), state.shape[0], _p(out),
-                                       _p(seg_row0), _p(seg_slot), rows, int(segments), heads, dim, _stream()))
+                                       _p(seg_row0), _p(seg_slot), rows, int(segments), heads, dim, *(_p(t) for t in places), count, *how,
+                                       _p(workspace), _stream()))
     return out
 
 

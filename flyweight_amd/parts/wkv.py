@@ -7,7 +7,7 @@ Per head, with the state S [key channel, value channel] (zero at the start):
 
     o_t = (S + diag(u) k_t v_t^T)^T r_t;      S <- diag(w_t) S + k_t v_t^T
 
-(u, the bonus, counts for the current token only). Each head's o is divided by its root mean square, times a
+(u, the bonus, counts for the current token only; long segments walk in chunks side by side). Each head's o is divided by its root mean square, times a
 weight per head and channel, times the gate; out = W_o of the heads side by side. The mixes, the decay with
 its exponentials, the state, the read-out and the heads' norm are float32 whatever the run's dtype; a request
 keeps S and its last h. The inner width of the decay's low-rank map is ``decay_rank``.
@@ -24,6 +24,7 @@ from ..config.spec import ConfigError
 from ..kernels import ops
 from ..weights.loader import TensorDecl
 from .base import Mixer, register_mixer
+from .chunks import RecurrenceChunks
 from .linear import Linear
 from .norm import LazyNorm
 
@@ -33,8 +34,9 @@ _MIXES = ("r", "k", "v", "g", "w")
 
 
 @register_mixer("wkv")
-class Wkv(Mixer):
+class Wkv(RecurrenceChunks, Mixer):
     graph_safe = True
+    LONG_ROWS = 128                 # 32 heads of 64 channels, one segment: 96 rows 25.6 us in order, 27.1 in chunks; 128 rows 32.3 and 27.6
     accepts_lazy_norm = True        # the norm in front is taken into the kernel that forms the mixes
     wants_unnormed_rows = True      # ... in float32, from the residual rows themselves: it asks for them also where the normed rows exist
 
@@ -58,6 +60,18 @@ class Wkv(Mixer):
 
     def _name(self, which: str) -> str:
         return self.prefix + self.names[which]
+
+    def step_arrays(self, batch):
+        # a float32 run gives the same bits however a sequence is cut into steps: its rows are walked in order
+        return super().step_arrays(batch) if self.dtype == torch.bfloat16 else {}
+
+    def chunk_arguments(self, ctx) -> dict:
+        """The walk in order takes 0.22 us a row of the longest segment, however many there are; the chunks about 20 us and, the chip
+        being full, 1 us for 2,200 rows of a workgroup's 16 value channels of one head. (32 heads of 64 channels: one segment
+        of 2,048 rows 441 us in order, 140 in chunks; four of 512 rows 125 and 129.)"""
+        lengths = [b - a for a, b in zip(ctx.host_seg_row0, ctx.host_seg_row0[1:])]
+        work = sum(n for n in lengths if n > self.LONG_ROWS) * self.heads * -(-self.dim // 16)
+        return super().chunk_arguments(ctx) if 20.0 + work / 2200.0 < 0.22 * max(lengths) else {}
 
     def mixing_flops(self, rows: int, keys_before: int = 0) -> int:
         """Flops of the recurrence itself: per token and head a read and a write of the state, a multiply and an add each
@@ -100,7 +114,7 @@ class Wkv(Mixer):
         inner = ops.tanh_rows(self.w1.forward(mixes[4], out_dtype=torch.float32), self.dtype)
         a = self.w2.forward(inner, out_dtype=torch.float32)
         o = ops.wkv_recurrence(r, k, v, a, self.w0, self.u, cache["state"].state, ctx.seg_row0, ctx.seg_slot, ctx.num_segments,
-                               self.heads, self.dim)
+                               self.heads, self.dim, **self.chunk_arguments(ctx))
         return ops.gated_head_norm(o, gate, self.norm_weight, self.heads, self.dim, self.eps, self.dtype, gate_silu=True)
 
     def output(self, h, ctx, cache) -> torch.Tensor:

@@ -138,6 +138,37 @@ def test_wkv_recurrence_gives_the_same_bits_however_the_tokens_are_cut(ops):
         assert torch.equal(found, whole) and torch.equal(other, state), f"cut as {cuts}"
 
 
+@pytest.mark.parametrize("heads,dim", [(3, 4), (2, 24), (4, 64), (1, 100), (2, 128), (1, 256)])
+def test_wkv_recurrence_in_chunks(ops, heads, dim):
+    """Segments of one row beside ones of exactly a chunk, a row less and more, several chunks and a rest; from states that are
+    not zero; decays from barely forgetting to forgetting at once. The same tolerance as for the walk in order, of whose
+    products and sums the chunks are another order (every factor is at most one)."""
+    rng = np.random.default_rng(dim)
+    lengths, slots, long_rows = [1, 64, 40, 63, 65, 130, 32, 257], [4, 0, 5, 2, 1, 7, 6, 3], 40
+    width, rows = heads * dim, sum(lengths)
+    seg_row0, _ = segments_of(lengths)
+    state = rng.normal(size=(9, heads, dim, dim)).astype(np.float32) * 0.3
+    w0, u = rng.normal(size=width).astype(np.float32) * 2.0 - 2.0, rng.normal(size=width).astype(np.float32)
+    r, k, v = (rng.normal(size=(rows, width)).astype(np.float32) * dim ** -0.25 for _ in range(3))
+    a = rng.normal(size=(rows, width)).astype(np.float32)
+    decay = np.exp(-np.exp(a.astype(np.float64) + w0))
+    S, expected = state.astype(np.float64).copy(), np.zeros((rows, width))
+    for s, slot in enumerate(slots):
+        cut = slice(seg_row0[s], seg_row0[s + 1])
+        expected[cut] = plain_recurrence(r[cut].astype(np.float64), k[cut].astype(np.float64), v[cut].astype(np.float64), decay[cut],
+                                         u.astype(np.float64), S[slot], heads, dim)
+    counts = [-(-n // 64) if n > long_rows else 0 for n in lengths]
+    seg = np.repeat(np.arange(len(lengths)), counts)
+    row0 = np.concatenate([seg_row0[s] + 64 * np.arange(c) for s, c in enumerate(counts)])
+    chunks = (ints(seg), ints(row0), ints(np.concatenate([[0], np.cumsum(counts)])), long_rows, False)
+    device_state = dev(state)
+    found = ops.wkv_recurrence(dev(r), dev(k), dev(v), dev(a), dev(w0), dev(u), device_state, ints(seg_row0), ints(slots), len(slots),
+                               heads, dim, chunks=chunks)
+    assert np.abs(host(found) - expected).max() <= 2e-5 * max(1.0, np.abs(expected).max())
+    assert np.abs(host(device_state) - S).max() <= 2e-5 * max(1.0, np.abs(S).max())
+    assert np.array_equal(host(device_state)[8], state[8].astype(np.float64)), "a slot of no request was touched"
+
+
 def test_wkv_bonus_counts_for_the_current_token_only(ops):
     """A state of zeros and one token: the read-out is (r . (u k)) v; the token after it sees k v^T without u."""
     dim = 16
