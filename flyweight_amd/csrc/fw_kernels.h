@@ -44,10 +44,8 @@ int fw_gemm_float32(const float* a, const float* w, const float* bias, void* out
 // multiple of 8. mode 0: out = a . w^T (+ bias) stored as out_dtype (also 2, here and in every storing product below:
 // gelu(a . w^T (+ bias)), the error-function form, in bfloat16); mode 1: out (float32) +=
 // a . w^T (+ bias); mode 2 (SwiGLU): w is [2N][K], gate rows then up rows, out [M][N] bfloat16 =
-// silu(a . gate^T) * (a . up^T), or with out_dtype 3 gelu_tanh(a . gate^T) * (a . up^T). fw_gemm_skinny streams w once for M <= 64 (decode);
-// fw_gemm_mfma tiles both operands through LDS (prompts).
-int fw_gemm_skinny(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
-                   int M, int N, int K, void* stream);
+// silu(a . gate^T) * (a . up^T), or with out_dtype 3 gelu_tanh(a . gate^T) * (a . up^T). fw_gemm_mfma tiles both operands
+// through LDS (prompts).
 int fw_gemm_mfma(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                  int M, int N, int K, void* stream);
 // The prompt product with large tiles (256 x 256 or 256 x 192; storing products also 128 rows by as many columns,
@@ -72,19 +70,20 @@ int fw_gemm_mfma_split_plan(int mode, int M, int N, int K, size_t* workspace_byt
 int fw_gemm_mfma_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                        int M, int N, int K, void* workspace, size_t workspace_bytes, int* counters,
                        int counters_len, void* stream);
-// The same product for 1..64 rows with K split over workgroups, so that a is not re-read by every
-// few features (decode steps of 17..64 requests). fw_gemm_medium_plan says what a shape needs:
-// bytes of workspace (0: none) and int32 counters (0: none) that are zero before the first call;
-// the kernel leaves them zero. Calls that overlap on one device need their own of both.
-// The accumulating product can leave what the norm after it needs, as fw_gemm_decode does
-// (next_activations [M][N] bfloat16, next_squares [squares_rows][16 for M <= 16, else 64]), and
-// any mode takes such prepared activations as a, with squares / squares_rows / eps.
-int fw_gemm_medium_plan(int M, int N, int K, int mode, size_t* workspace_bytes, int* counters, int* squares_rows);
-int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode,
-                   int M, int N, int K, void* workspace, size_t workspace_bytes, int* counters,
-                   int counters_len, const float* next_norm_weight, int next_one_centered,
-                   void* next_activations, float* next_squares, const float* squares, int squares_rows,
-                   float eps, float glu_limit, float glu_alpha, float glu_shift, void* stream);
+// The product for 1..64 rows and a very wide output: mode 0 alone; takes prepared activations as a (squares [squares_rows][16
+// for M <= 16, else 64], eps).
+int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int M, int N, int K,
+                   const float* squares, int squares_rows, float eps, void* stream);
+// The product for 1..4096 rows in modes 0, 1 and 2 (the gated unit: glu_limit and its like as for fw_gemm_decode) with K split over
+// a workgroup's waves alone: no workspace, no counters. Up to 64 rows the accumulating product can leave what the norm after
+// it needs, as fw_gemm_decode does (next_activations [M][N] bfloat16, next_squares [fw_gemm_rows_squares(M, N)][16 for M <= 16,
+// else 64]), and any mode takes such prepared activations as a, with squares / squares_rows / eps. fw_gemm_rows_round: whether
+// its tiles are at most one round over the compute units.
+int fw_gemm_rows(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
+                 const float* next_norm_weight, int next_one_centered, void* next_activations, float* next_squares, const float* squares,
+                 int squares_rows, float eps, float glu_limit, float glu_alpha, float glu_shift, void* stream);
+int fw_gemm_rows_squares(int M, int N);
+int fw_gemm_rows_round(int mode, int M, int N);
 
 // Fused product for decode steps of up to 16 rows. prologue 0: a is bfloat16 [M][K]; 1: a is
 // float32 rows, RMS-normed with norm_weight/eps (rows gathered through row_index if given) inside
@@ -96,10 +95,10 @@ int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias,
 // [M][N] = x_new * w_next and next_squares [fw_gemm_decode_accumulate_tiles(N)][16], per-tile sums
 // of x_new^2 of every row. A later call takes them with prologue 2 (a = those activations,
 // squares/squares_tiles = those sums, eps) and applies the row's scale in its epilogue.
-// glu_limit / glu_alpha / glu_shift (here and in fw_gemm_medium, epilogue 2 only): with a limit of 0 the
+// glu_limit / glu_alpha / glu_shift (here and in fw_gemm_rows, epilogue 2 only): with a limit of 0 the
 // gated unit is SwiGLU, silu(gate) * up; with a negative one gelu_tanh(gate) * up; with a positive one its halves are clamped, g = min(gate,
 // limit), u = clamp(up, -limit, limit), and out = g * sigmoid(alpha * g) * (u + shift).
-// w_tiled (here and in fw_gemm_medium): w is not row-major [rows][K] but lies in operand tiles,
+// w_tiled (here, in fw_gemm_medium and in fw_gemm_rows): w is not row-major [rows][K] but lies in operand tiles,
 // [rows / 16][K / 32][4][16][8]: tile (i, j) holds rows 16 i .. 16 i + 15, columns 32 j .. 32 j + 31 as
 // 1 KB in the order in which a wave loads a matrix-core operand (lane = 16 * (column / 8) + row), so
 // that a wave reads whole contiguous kilobytes (rows padded with zeros to a multiple of 16; K a

@@ -525,20 +525,17 @@ def gather_rows(rows: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
 
 def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                w_tiled: Optional[torch.Tensor] = None) -> None:
-    """bfloat16 operands on the matrix cores: the skinny kernel for up to 16 rows, the medium one
-    (K split over workgroups) for up to 64, the tiled ones beyond (large tiles where they fill the
-    chip, K cut into slices where even the small tiles are too few)."""
+    """bfloat16 operands on the matrix cores: up to 64 rows, and with weights in operand tiles as long as its tiles are one
+    round over the chip, the product whose waves split K; the tiled ones beyond (large tiles where they fill the chip, K cut into slices where
+    even the small tiles are too few)."""
     M, K = a.shape
-    if SKINNY_MAX_ROWS < M <= MEDIUM_MAX_ROWS or (M <= SKINNY_MAX_ROWS and w.numel() >= MEDIUM_LARGE and K % 8 == 0):
-        # also a few rows of a large W (a vocabulary's head: 65,536 x 2,048 at 8 rows 52 against 61 us)
+    if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and M <= ROWS_MAX and library().fw_gemm_rows_round(mode, M, N)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
             gemm_medium_into(a, w, bias, target, BF16, mode, N, w_tiled=w_tiled, glu=GEGLU)
         else:
             gemm_medium_into(a, w, bias, target, out_code, mode, N, w_tiled=w_tiled)
         return
-    if M <= SKINNY_MAX_ROWS:
-        entry = library().fw_gemm_skinny
-    elif M > BIG_MIN_ROWS and library().fw_gemm_mfma_big_tiles(mode, M, N, K) >= BIG_TILES_MIN:
+    if M > BIG_MIN_ROWS and library().fw_gemm_mfma_big_tiles(mode, M, N, K) >= BIG_TILES_MIN:
         entry = library().fw_gemm_mfma_big      # enough 256 x 256 tiles to fill the chip
     elif K >= (DEEP_MIN_K if mode == 1 else DEEP_MIN_K_STORE) and _deep_columns(mode, M, N, K):
         # whole rounds of one tile per compute unit: the waves split K
@@ -568,9 +565,14 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     _check(entry(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
 
 
-SKINNY_MAX_ROWS = 16
 MEDIUM_MAX_ROWS = 64
-MEDIUM_LARGE = 1 << 25    # weights from which the medium product beats the skinny one at any number of rows
+# Beyond 64 rows the waves-split-K product (gemm_rows.hip) is taken for weights in operand tiles while its tiles, of at most 64 x 64, are one round over the 256
+# compute units; measured against the tiled products, every weight from memory: adding 2,048 features (K 8,192) at 128 / 256 / 512
+# rows 20.6 / 26.2 / 34.8 against 25.0 / 30.6 / 44.1 us, K 2,048 8.2 / 10.6 / 14.3 against 14.8 / 15.1 / 18.9; storing 3,072 features at
+# 256 rows 14.4 against 18.1, 6,144 at 128 rows 15.3 against 18.9. With two rounds it loses (6,144 features at 192 rows 25.9 against
+# 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27).
+ROWS_MAX = 1024
+WIDE_STORE = 24576        # outputs from which a storing product of up to 64 rows takes the tiles of a vocabulary (65,536 at 64 rows: 62 against 70 us)
 BIG_TILES_MIN = 192      # 256 x 256 tiles from which the large-tile prompt product is used (256 compute units)
 DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)
 DEEP_MIN_K_STORE = 4096   # storing: no old values travel during the exchange at a tile's end, a short K gains nothing
@@ -696,31 +698,29 @@ def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tenso
                      next_norm_weight: Optional[torch.Tensor] = None, next_one_centered: bool = False,
                      squares: Optional[torch.Tensor] = None, eps: float = 0.0, w_tiled: Optional[torch.Tensor] = None,
                      glu: Optional[tuple] = None):
-    """The product for 1..64 rows with K split over workgroups (fw_gemm_medium). With
+    """The product for 1..64 rows (more where nothing is prepared). With
     ``squares`` ``a`` holds prepared activations (x * w of an RMS norm) and the rows' 1/rms is
     formed from those sums. With ``next_norm_weight`` (accumulating product) returns what the
     norm after it needs: (activations x * w_next, sums of squares)."""
     M, K = a.shape
-    need_bytes, need_counters, squares_rows = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
-    _check(library().fw_gemm_medium_plan(M, N, K, mode, ctypes.byref(need_bytes), ctypes.byref(need_counters),
-                                         ctypes.byref(squares_rows)))
-    workspace = counters = next_activations = next_squares = None
-    if need_bytes.value:
-        workspace = torch.empty(need_bytes.value // 4, dtype=torch.float32, device=a.device)
-        counters = _medium_counters(a.device, need_counters.value)
+    next_activations = next_squares = None
     stride = 16 if M <= DECODE_MAX_ROWS else 64
-    if next_norm_weight is not None:
-        next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-        next_squares = torch.empty((squares_rows.value, stride), dtype=torch.float32, device=a.device)
     if squares is not None and (squares.dtype != torch.float32 or squares.dim() != 2 or squares.shape[1] != stride
                                 or not squares.is_contiguous()):
         raise KernelError(f"gemm_medium: sums of squares for {M} rows are float32 [n, {stride}]")
+    squares_rows = 0 if squares is None else squares.shape[0]
     w_tiled = _tiled_for(w, w_tiled)
-    _check(library().fw_gemm_medium(_p(a), _p(w if w_tiled is None else w_tiled), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K, _p(workspace),
-                                    ctypes.c_size_t(need_bytes.value), _p(counters),
-                                    0 if counters is None else counters.numel(), _p(next_norm_weight),
-                                    int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
-                                    0 if squares is None else squares.shape[0], ctypes.c_float(eps), *_glu(glu), _stream()))
+    operand = w if w_tiled is None else w_tiled
+    if mode == 0 and N >= WIDE_STORE and M <= MEDIUM_MAX_ROWS and target.data_ptr() % 16 == 0:
+        _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, M, N, K, _p(squares),
+                                        squares_rows, ctypes.c_float(eps), _stream()))
+        return None
+    if next_norm_weight is not None:
+        next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+        next_squares = torch.empty((library().fw_gemm_rows_squares(M, N), stride), dtype=torch.float32, device=a.device)
+    _check(library().fw_gemm_rows(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
+                                  _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
+                                  squares_rows, ctypes.c_float(eps), *_glu(glu), _stream()))
     if next_norm_weight is not None:
         return next_activations, next_squares
     return None
@@ -935,9 +935,8 @@ def gemm_decode(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Option
                                          or next_norm_weight.shape != (N,)):
         raise KernelError("gemm_decode: only the accumulating product prepares the next norm, whose weight is float32 [N]")
     if epilogue == EPILOGUE_ACCUMULATE and K >= LONG_K and N <= 4096 and not (w_tiled is not None and rows <= LONG_K_TILED_ROWS):
-        # few features and a long K: the kernel that splits K over workgroups streams W faster (from operand
-        # tiles only beyond eight rows: 2,048 features over K 8,192 at 8 rows 11.4 against 11.0 us, at 16
-        # rows 11.3 against 13.4)
+        # few features and a long K: the product on tiles of few rows (from operand tiles only beyond eight rows:
+        # 2,048 features over K 8,192 at 8 rows 11.4 us on this one, at 16 rows 13.4 against 12.6 us)
         left = gemm_medium_into(a, w, bias, target, F32, 1, N, next_norm_weight, next_one_centered, w_tiled=w_tiled)
         return target if left is None else left
     if next_norm_weight is not None:

@@ -6,7 +6,7 @@ stream in the kernel's epilogue, so the residual sum never leaves float32; ``swi
 here from the operand types and the number of rows: for up to 16 rows of a bfloat16 model one
 fused kernel takes the RMS norm before the product (handed over as a :class:`LazyNorm`) and
 the epilogue after it, and the product that adds to the residual stream prepares the norm
-that follows; otherwise the norm runs on its own and the skinny, tiled or generic
+that follows; otherwise the norm runs on its own and the tiled, float32 or generic
 product follows.
 """
 
@@ -66,22 +66,19 @@ class Linear:
     def _tensor_of(a: Input) -> torch.Tensor:
         return a.tensor() if isinstance(a, LazyNorm) else a
 
-    # From this many weights on the product that splits K over workgroups also serves a few rows: its
-    # workgroups walk K from different chunks on, and a large W in row-major order then streams faster
-    # than through the fused decode product (16,384 x 2,048 with SwiGLU at 8 rows: 17.6 against 19.1 us;
-    # equal at one row). From operand tiles the fused product streams faster than either (gate|up at 8
-    # rows 12.9 against 14.9 us, a vocabulary of 65,536 45.3 against 49.5 us); only the widest outputs
-    # go to the split-K product, from nine rows on, where every workgroup's own read of all of a
-    # begins to weigh (the vocabulary at 16 rows: 50.4 against 52.2 us).
+    # From this many weights on the products of a few dozen rows also serve fewer: a large W in row-major order streams
+    # faster through them than through the fused decode product (16,384 x 2,048 with SwiGLU at 12 rows 15.7 us against 19.1 at
+    # eight). From operand tiles the fused product streams faster (gate|up at 8 rows 12.9 against 14.7 us, a
+    # vocabulary of 65,536 45.3 against 49.5 us); only the widest outputs go there from nine rows on, where every
+    # workgroup's own read of all of a begins to weigh (the vocabulary at 16 rows: 50.4 against 52.2 us).
     LARGE = 1 << 25
     LARGE_MIN_ROWS = 3
     LARGE_TILED = 1 << 26
     LARGE_TILED_MIN_ROWS = 9
 
     def _medium(self, a: Input) -> bool:
-        """17..64 rows of a bfloat16 model, and fewer rows of a large weight: the product that splits
-        K over workgroups, which takes prepared activations and prepares the next norm as the fused
-        decode product does."""
+        """17..64 rows of a bfloat16 model, and fewer rows of a large weight: the products of a few dozen
+        rows, which take prepared activations and prepare the next norm as the fused decode product does."""
         if self.weight.dtype != torch.bfloat16 or a.dtype != torch.bfloat16 or self.in_features % 8:
             return False
         rows = a.rows if isinstance(a, LazyNorm) else a.shape[0]
