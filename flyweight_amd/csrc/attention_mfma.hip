@@ -287,8 +287,14 @@ __device__ __forceinline__ void load_query(Columns<HD>& c, const uint16_t* __res
 // them into the accumulation registers, and the softmax's rescaling of the output and the masks on
 // the scores then cost a move out and a move back per value and page (112 + 80 of the ~560 vector
 // instructions of two pages).
-template <int HD, int NH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((HD <= 64 && NH == 1) ? 2 : 1))) void attention_prefill_kernel(
+//
+// PARTS 2: eight waves, the pages shared out between two halves of four waves (every second page each, with buffers
+// of its own), which merge at the end, the first half's rows first. With NH 2 every key and value read from LDS serves
+// two heads, and there are as many waves as with one half and NH 1. (The reads from LDS, 16 KB a wave and page, bound the
+// kernel beside the softmax: one head 452 TFLOP/s over a prompt of 32,768 tokens, 16 heads in 8 groups; two heads in halves
+// 560.)
+template <int HD, int NH, int PARTS>
+__global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu((HD <= 64 && NH <= 2) ? 2 : 1))) void attention_prefill_kernel(
     const uint16_t* __restrict__ q, uint16_t* __restrict__ out, const uint16_t* __restrict__ k_pages,
     const uint16_t* __restrict__ v_pages, const int32_t* __restrict__ block_table, int table_stride,
     const int32_t* __restrict__ tile_seg, const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ seg_row0,
@@ -299,10 +305,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((HD <= 64 &
     constexpr int k_stride = HD + KV_PAD;
     const int v_stride = PAGE + KV_PAD;
     const int k_elems = PAGE * k_stride, v_elems = v_dim * v_stride;
-    uint16_t* lds = reinterpret_cast<uint16_t*>(lds_raw);      // [buffer][K tile | V tile]
+    const int half = PARTS > 1 ? threadIdx.x >> 8 : 0, tid = threadIdx.x & 255;
+    uint16_t* lds = reinterpret_cast<uint16_t*>(lds_raw) + (size_t)half * 2 * (k_elems + v_elems);     // [half][buffer][K tile | V tile]
     if (head_dim < HD) {
         const int runs_per_row = (HD - head_dim) / 8;          // head_dim is a multiple of 16
-        for (int run = threadIdx.x; run < 2 * PAGE * runs_per_row; run += 256) {
+        for (int run = tid; run < 2 * PAGE * runs_per_row; run += 256) {
             const int buffer = run / (PAGE * runs_per_row), row = run / runs_per_row % PAGE, at = run % runs_per_row;
             *reinterpret_cast<u32x4*>(lds + (size_t)buffer * (k_elems + v_elems) + row * k_stride + head_dim + at * 8) = u32x4{0u, 0u, 0u, 0u};
         }
@@ -312,7 +319,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((HD <= 64 &
     const int per_tile = num_kv_heads * runs;
     const int tile = blockIdx.x / per_tile, of_tile = blockIdx.x % per_tile;
     const int kvh = of_tile / runs, first_in_group = (of_tile % runs) * NH;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
+    const int lane = tid & 63, wave = tid >> 6, col = lane & 15, g = lane >> 4;
     const int seg = tile_seg[tile];
     const int tile_first_row = tile_row0[tile];
     const int seg_end = seg_row0[seg + 1];
@@ -412,24 +419,56 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((HD <= 64 &
         }
     };
 
-    // page b travels: global -> register set (b - first) % 2, requested two pages ahead -> LDS
-    // buffer (b - first) % 2, stored while page b - 1 is worked on -> attended
-    fetch(hold_k0, hold_v0, 0);
-    fetch(hold_k1, hold_v1, 1);
-    stash(hold_k0, hold_v0, 0, 0);
+    // a half's page number i travels: global -> register set i % 2, requested two pages ahead -> LDS
+    // buffer i % 2, stored while page i - 1 is worked on -> attended
+    auto step_of = [&](int i) { return PARTS * i + half; };
+    const int pages = (last_step + PARTS) / PARTS;              // of the first half; the other may have one less (a page past the end)
+    fetch(hold_k0, hold_v0, step_of(0));
+    fetch(hold_k1, hold_v1, step_of(1));
+    stash(hold_k0, hold_v0, 0, step_of(0));
     fw_lds_barrier();
-    for (int step = 0; step <= last_step; step += 2) {
-        fetch(hold_k0, hold_v0, step + 2);
+    for (int i = 0; i < pages; i += 2) {
+        fetch(hold_k0, hold_v0, step_of(i + 2));
         __builtin_amdgcn_sched_barrier(0);      // keep the requests ahead of the work they overlap
-        attend(step, 0);
-        stash(hold_k1, hold_v1, 1, step + 1);
+        attend(step_of(i), 0);
+        stash(hold_k1, hold_v1, 1, step_of(i + 1));
         fw_lds_barrier();
-        if (step + 1 > last_step) break;
-        fetch(hold_k1, hold_v1, step + 3);
+        if (i + 1 >= pages) break;
+        fetch(hold_k1, hold_v1, step_of(i + 3));
         __builtin_amdgcn_sched_barrier(0);
-        attend(step + 1, 1);
-        stash(hold_k0, hold_v0, 0, step + 2);
+        attend(step_of(i + 1), 1);
+        stash(hold_k0, hold_v0, 0, step_of(i + 2));
         fw_lds_barrier();
+    }
+    if constexpr (PARTS > 1) {
+        // the second half leaves its maximum, sum and output to the same lane of the first
+        constexpr int VALUES = HD / 4 + 2;
+        float* left = reinterpret_cast<float*>(lds_raw) + tid;                  // [NH][VALUES][256]
+        __syncthreads();
+        if (half == 1)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                left[(h * VALUES + HD / 4) * 256] = c[h].m;
+                left[(h * VALUES + HD / 4 + 1) * 256] = c[h].l;
+#pragma unroll
+                for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) left[(h * VALUES + t * 4 + r) * 256] = c[h].o[t][r];
+            }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float other = left[(h * VALUES + HD / 4) * 256], top = fmaxf(c[h].m, other);
+            // (a half without any key of this row keeps NEG_BIG: its factor is 0)
+            const float mine = __builtin_amdgcn_exp2f(c[h].m - top), theirs = __builtin_amdgcn_exp2f(other - top);
+            c[h].m = top;
+            c[h].l = c[h].l * mine + left[(h * VALUES + HD / 4 + 1) * 256] * theirs;
+#pragma unroll
+            for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c[h].o[t][r] = c[h].o[t][r] * mine + left[(h * VALUES + t * 4 + r) * 256] * theirs;
+        }
     }
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
@@ -856,7 +895,7 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
                                     const int32_t* tile_row0, int tiles, const int32_t* seg_row0,
                                     const int32_t* row_pos, int rows, int num_heads, int num_kv_heads, int head_dim,
                                     int v_dim, float scale, int window, int chunk, float softcap, int keep_first, const float* sinks,
-                                    const float* slopes, int page_size, int num_pages, int heads_together, void* stream) {
+                                    const float* slopes, int page_size, int num_pages, int heads_together, int halves, void* stream) {
     FW_REQUIRE(keep_first >= 0 && (keep_first == 0 || chunk == 0), "attention_prefill: %d first keys are kept beside a window, not beside chunks", keep_first);
     if (check_common("attention_prefill", rows, num_heads, num_kv_heads, head_dim, v_dim, page_size, window, num_pages, table_stride, chunk, softcap)) return -1;
     const ScoreRule rule = score_rule(scale, softcap);
@@ -865,36 +904,40 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
     const int most_together = widest <= 64 ? 4 : 1;
     FW_REQUIRE(heads_together == 0 || heads_together == 1 || (heads_together == 4 && most_together == 4),
                "attention_prefill: %d heads together with head_dim %d (1, or 4 up to head_dim 64)", heads_together, head_dim);
+    FW_REQUIRE(!halves || (widest <= 64 && heads_together == 0), "attention_prefill: the pages are shared out between halves up to head_dim 64, two heads together");
     if (rows == 0 || tiles == 0) return 0;
     const int group = num_heads / num_kv_heads;
+    if (halves) heads_together = 2;
     if (heads_together == 0)
         heads_together = most_together == 4 && group >= 4 && (long long)tiles * num_kv_heads * ((group + 3) / 4) >= 1024 ? 4 : 1;
     const long long blocks = (long long)tiles * num_kv_heads * ((group + heads_together - 1) / heads_together);
     FW_REQUIRE(blocks < (1ll << 31), "attention_prefill: too many tiles and heads");
     dim3 grid((unsigned)blocks);
-#define LAUNCH(HD, NH)                                                                                             \
+#define LAUNCH(HD, NH, PARTS)                                                                                      \
     {                                                                                                              \
-        const int lds_bytes = 2 * (PAGE * (HD + KV_PAD) + v_dim * (PAGE + KV_PAD)) * 2;                            \
+        const int lds_bytes = PARTS * 2 * (PAGE * (HD + KV_PAD) + v_dim * (PAGE + KV_PAD)) * 2;                    \
+        const int merge_bytes = PARTS > 1 ? NH * (HD / 4 + 2) * 256 * 4 : 0;                                       \
+        const int bytes = lds_bytes > merge_bytes ? lds_bytes : merge_bytes;                                       \
         static int configured = 0;                                                                                 \
-        if (lds_bytes > configured) {                                                                              \
-            hipError_t status = hipFuncSetAttribute((const void*)attention_prefill_kernel<HD, NH>,                 \
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);        \
-            FW_REQUIRE(status == hipSuccess, "attention_prefill: cannot reserve %d bytes of LDS", lds_bytes);      \
-            configured = lds_bytes;                                                                                \
+        if (bytes > configured) {                                                                                  \
+            hipError_t status = hipFuncSetAttribute((const void*)attention_prefill_kernel<HD, NH, PARTS>,          \
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, bytes);            \
+            FW_REQUIRE(status == hipSuccess, "attention_prefill: cannot reserve %d bytes of LDS", bytes);          \
+            configured = bytes;                                                                                    \
         }                                                                                                          \
-        attention_prefill_kernel<HD, NH><<<grid, 256, lds_bytes, (hipStream_t)stream>>>(                            \
+        attention_prefill_kernel<HD, NH, PARTS><<<grid, 256 * PARTS, bytes, (hipStream_t)stream>>>(                 \
             (const uint16_t*)q, (uint16_t*)out, (const uint16_t*)k_pages, (const uint16_t*)v_pages, block_table,    \
             table_stride, tile_seg, tile_row0, seg_row0, row_pos, num_heads, num_kv_heads, head_dim, v_dim,        \
             rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, keep_first, sinks, slopes);                  \
     }
     if (widest <= 32) {
-        if (heads_together == 4) LAUNCH(32, 4) else LAUNCH(32, 1)
+        if (halves) LAUNCH(32, 2, 2) else if (heads_together == 4) LAUNCH(32, 4, 1) else LAUNCH(32, 1, 1)
     } else if (widest <= 64) {
-        if (heads_together == 4) LAUNCH(64, 4) else LAUNCH(64, 1)
+        if (halves) LAUNCH(64, 2, 2) else if (heads_together == 4) LAUNCH(64, 4, 1) else LAUNCH(64, 1, 1)
     } else if (widest <= 128) {
-        LAUNCH(128, 1)
+        LAUNCH(128, 1, 1)
     } else {
-        LAUNCH(256, 1)
+        LAUNCH(256, 1, 1)
     }
 #undef LAUNCH
     FW_LAUNCH_CHECK("attention_prefill");

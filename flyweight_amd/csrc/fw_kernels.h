@@ -168,13 +168,14 @@ int fw_attention_generic(const void* q, void* out, int dtype, const void* k_page
 // tile_row0), in any order: workgroups start in the order of the tiles, so the caller lists those
 // that see the most keys first. heads_together: how many query heads of a kv group one workgroup takes, reading
 // the keys and values once for all of them (1, or 4 up to head_dim 64: 4 pays behind a long
-// context, 1 evens out a short causal prompt); 0: chosen from the shape alone.
+// context, 1 evens out a short causal prompt); 0: chosen from the shape alone. halves (with heads_together 0, up to head_dim
+// 64): two heads together, a tile's pages shared out between two halves of a workgroup that merge at the end.
 int fw_attention_prefill(const void* q, void* out, const void* k_pages, const void* v_pages,
                          const int32_t* block_table, int table_stride, const int32_t* tile_seg,
                          const int32_t* tile_row0, int tiles, const int32_t* seg_row0, const int32_t* row_pos,
                          int rows, int num_heads, int num_kv_heads, int head_dim, int v_dim, float scale, int window,
                          int chunk, float softcap, int keep_first, const float* sinks, const float* slopes, int page_size, int num_pages,
-                         int heads_together, void* stream);
+                         int heads_together, int halves, void* stream);
 // Decode (one row per request): the keys are split between workgroups in runs of 4 pages and
 // merged in order by the workgroup that finishes last. partial: float32 workspace
 // [rows][heads][max_splits][v_dim + 4]; max_context: an upper bound on position + 1 of every

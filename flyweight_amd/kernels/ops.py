@@ -988,9 +988,9 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
                       seg_row0: torch.Tensor, row_pos: torch.Tensor, scale: float, window: int = 0,
                       heads_together: int = 0, out: Optional[torch.Tensor] = None, v_dim: Optional[int] = None,
                       chunk: int = 0, softcap: float = 0.0, keep_first: int = 0, sinks: Optional[torch.Tensor] = None,
-                      slopes: Optional[torch.Tensor] = None) -> torch.Tensor:
+                      slopes: Optional[torch.Tensor] = None, halves: bool = False) -> torch.Tensor:
     """``heads_together``: query heads of a kv group per workgroup (1, or 4 up to head_dim 64), 0: the
-    kernel's choice. Only the rows of the given tiles are written (into ``out`` if given)."""
+    kernel's choice. ``halves`` (up to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. Only the rows of the given tiles are written (into ``out`` if given)."""
     _dev(q, k_pages, v_pages, block_table, tile_seg, tile_row0, seg_row0, row_pos)
     _want(q, torch.bfloat16, "q")
     rows = q.shape[0]
@@ -1011,7 +1011,7 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         _p(q), _p(out), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(tile_seg), _p(tile_row0),
         tile_seg.numel(), _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale),
         int(window), int(chunk), ctypes.c_float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages,
-        int(heads_together), _stream()))
+        int(heads_together), int(halves), _stream()))
     return out
 
 
@@ -1142,15 +1142,16 @@ def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
         if tile_seg is None or tile_row0 is None:
             raise KernelError("attention: the tiled kernel needs the step's query tiles")
         single = getattr(ctx, "decode_prefix", 0)       # leading segments of one row: rows and tiles 0 .. single - 1
-        # four query heads of a kv group per workgroup pay where the rows sit behind a long context
-        # (a page is read once for the four); from the start of a prompt one head per workgroup
-        # gives more and shorter workgroups, which evens out the causal triangle
-        rows = q.shape[0] - single
+        # Where a row may see some thousand keys, two heads of a kv group per workgroup read a page's keys and values from LDS
+        # once for both, its two halves sharing the pages out so that as many waves are at work (2,048 rows, head_dim 64,
+        # against one head: 32 heads in 8 groups behind 0 / 2,048 / 30,720 keys 46.9 / 106 / 871 against 48.2 / 143 / 1,078 us,
+        # 16 heads 37.7 / 66 / 455 against 39.6 / 78 / 562; 777 rows from position 0 20.1 against 18.8). Four heads
+        # together, which a long context once took, lose to either (64 rows behind 8,000 keys 270 against 116 us).
         keys = min([n for n in (window, chunk) if n] + [ctx.max_context])      # the most keys a row can see
-        together = 4 if max(head_dim, v_dim) <= 64 and num_heads // num_kv_heads >= 4 and keys >= 4 * rows else 0
+        halves = max(head_dim, v_dim) <= 64 and num_heads // num_kv_heads >= 2 and keys >= 3072
         if single == 0:
             return attention_prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, tile_seg,
-                                     tile_row0, ctx.seg_row0, ctx.row_pos, scale, window, heads_together=together, v_dim=v_dim,
+                                     tile_row0, ctx.seg_row0, ctx.row_pos, scale, window, halves=halves, v_dim=v_dim,
                                      chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)
         out = torch.empty((q.shape[0], num_heads * v_dim), dtype=q.dtype, device=q.device)
         attention_decode(q[:single], num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, ctx.row_seg,
@@ -1158,7 +1159,7 @@ def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
                          chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)
         return attention_prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table,
                                  tile_seg[single:], tile_row0[single:], ctx.seg_row0, ctx.row_pos, scale, window,
-                                 heads_together=together, out=out, v_dim=v_dim, chunk=chunk, softcap=softcap,
+                                 halves=halves, out=out, v_dim=v_dim, chunk=chunk, softcap=softcap,
                                  keep_first=keep_first, sinks=sinks, slopes=slopes)
     return attention_generic(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, ctx.row_seg,
                              ctx.row_pos, scale, window, v_dim=v_dim, chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)

@@ -694,6 +694,38 @@ def test_attention_prefill_takes_four_heads_of_a_group_together(ops, nh, nkv, hd
         run(2)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,window,keep_first,sink", [(4, 2, 64, 0, 0, False), (3, 1, 48, 0, 0, False), (6, 1, 64, 0, 0, True), (2, 2, 32, 0, 0, False),
+                                                              (8, 4, 64, 70, 0, False), (4, 2, 64, 64, 5, True), (4, 1, 16, 1, 0, False)])
+def test_attention_prefill_whose_halves_share_the_pages(ops, nh, nkv, hd, window, keep_first, sink):
+    """Tiles of one page (the second half has none), of an even and an odd number of pages, rows whose own page is the second
+    half's, groups of one, three and six heads, windows that leave a half without a key, kept first keys and a sink. Against
+    the reference; rows differ from the plain kernel's by the rounding of the halves' weights alone."""
+    lengths = [150, 200, 64, 65, 33, 320]
+    starts = [0, 120, 63, 64, 16, 5]
+    keys, values, table, k_pages, v_pages = _mfma_setup(nh, nkv, hd, lengths, num_pages=19, seed=5)
+    counts = [n - s for n, s in zip(lengths, starts)]
+    seg_row0 = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    row_pos = np.concatenate([np.arange(s, n) for s, n in zip(starts, lengths)]).astype(np.int32)
+    row_seg = np.concatenate([np.full(c, i) for i, c in enumerate(counts)]).astype(np.int32)
+    tile_seg, tile_row0 = ops.query_tiles(seg_row0.tolist())
+    rows = int(seg_row0[-1])
+    q = as_dev(gen(rows, nh * hd, seed=4), torch.bfloat16)
+    scale = 1 / math.sqrt(hd)
+    sinks = torch.randn(nh, generator=torch.Generator().manual_seed(1)).to(DEV) if sink else None
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    run = lambda **how: ops.attention_prefill(q, nh, nkv, hd, k_pages, v_pages, d(table), d(tile_seg), d(tile_row0), d(seg_row0),  # noqa: E731
+                                              d(row_pos), scale, window, keep_first=keep_first, sinks=sinks, **how)
+    found, plain = run(halves=True), run(heads_together=1)
+    close(found, back(plain), torch.bfloat16)
+    if not sink and not keep_first:
+        want = torch.stack([attention_reference(back(q)[r].reshape(nh, hd), keys[row_seg[r]], values[row_seg[r]], int(row_pos[r]),
+                                                scale, window, nh // nkv).reshape(-1) for r in range(rows)])
+        close(found, want, torch.bfloat16)
+    assert torch.equal(found, run(halves=True))
+    with pytest.raises(ops.KernelError, match="halves"):
+        run(halves=True, heads_together=1)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,window", [(4, 2, 16, 0), (3, 1, 48, 0), (6, 3, 80, 0), (32, 8, 64, 0), (2, 2, 128, 0),
                                               (20, 1, 256, 0), (4, 2, 32, 300), (4, 4, 64, 64), (2, 1, 64, 1)])
 def test_attention_decode_on_the_matrix_cores(ops, nh, nkv, hd, window):
