@@ -186,8 +186,9 @@ __device__ __forceinline__ float delta_row_sum(float x) {
 }
 
 // Workgroup (segment, head, block of 16 value channels); thread = 16 * column + part: a column of S
-// is shared out over the 16 lanes of a row of the wave, RPT rows each (rows part, part + 16, ...: the
-// sixteen lanes then read sixteen neighbouring floats of q, k and g from LDS, one bank each; rows from
+// is shared out over the 16 lanes of a row of the wave, RPT rows each (from four rows on in runs of four, 4 part .. + 3 of
+// every 64: a lane then reads four floats of q, k and g from LDS at a time, the sixteen lanes all banks once. Read one
+// float at a time, 26 reads a token and wave kept LDS busier than the sums kept the vector unit: FIGURES; rows from
 // dim on hold zeros), so that a head is spread over many compute units: the walk along the
 // tokens is one dependent chain per column, and only its width can be bought. LDS per staged token:
 // q, k, g (16 * RPT each; past the record's padded dim they stay zero), beta and three unused, then the
@@ -201,6 +202,7 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     const int32_t* __restrict__ seg_row0, const int32_t* __restrict__ seg_slot, int heads, int dim, int vdim) {
     typedef __attribute__((ext_vector_type(4))) float f32x4;
     constexpr int DP = DELTA_LANES * RPT;
+    constexpr int RUN = RPT >= 4 ? 4 : 1;                                // neighbouring rows of a lane
     constexpr int TOKEN = 3 * DP + 4 + DELTA_COLUMNS;
     constexpr int PIECES = (DELTA_CHUNK * (TOKEN / 4) + 255) / 256;      // 16-byte pieces of a chunk per thread, at most
     __shared__ __attribute__((aligned(16))) float staged[DELTA_CHUNK * TOKEN];
@@ -261,14 +263,16 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     ask(0);
     float* mine = state + (((size_t)seg_slot[seg] * heads + head) * vdim + (live ? column : 0)) * dim;
     float S[RPT];
+    auto row_of = [&](int t) { return t / RUN * (RUN * DELTA_LANES) + part * RUN + t % RUN; };
 #pragma unroll
-    for (int t = 0; t < RPT; ++t) {
-        const int i = t * DELTA_LANES + part;
-        S[t] = (live && i < dim) ? mine[i] : 0.0f;
-    }
+    for (int t = 0; t < RPT; ++t) S[t] = (live && row_of(t) < dim) ? mine[row_of(t)] : 0.0f;
     __syncthreads();        // the zeros are in place
     put(0);
     __syncthreads();
+    // The state has arrived here, for the compiler too: its first use being inside the loop, every token waited for all loads
+    // in flight, the next chunk's among them.
+#pragma unroll
+    for (int t = 0; t < RPT; ++t) asm volatile("" : "+v"(S[t]));
     for (int base = 0; base < count; base += DELTA_CHUNK) {
         const int tokens = count - base < DELTA_CHUNK ? count - base : DELTA_CHUNK;
         const bool more = base + DELTA_CHUNK < count;
@@ -277,11 +281,25 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
         float q_next[RPT], k_next[RPT], g_next[RPT], b_next, v_next;
         auto fetch = [&](int token) {
             const float* t0 = staged + token * TOKEN;
+            if constexpr (RUN == 4) {
 #pragma unroll
-            for (int t = 0; t < RPT; ++t) {
-                q_next[t] = t0[t * DELTA_LANES + part];
-                k_next[t] = t0[DP + t * DELTA_LANES + part];
-                g_next[t] = t0[2 * DP + t * DELTA_LANES + part];
+                for (int t = 0; t < RPT; t += 4) {
+                    const f32x4 q = *reinterpret_cast<const f32x4*>(t0 + row_of(t)), k = *reinterpret_cast<const f32x4*>(t0 + DP + row_of(t));
+                    const f32x4 g = *reinterpret_cast<const f32x4*>(t0 + 2 * DP + row_of(t));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        q_next[t + e] = q[e];
+                        k_next[t + e] = k[e];
+                        g_next[t + e] = g[e];
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int t = 0; t < RPT; ++t) {
+                    q_next[t] = t0[row_of(t)];
+                    k_next[t] = t0[DP + row_of(t)];
+                    g_next[t] = t0[2 * DP + row_of(t)];
+                }
             }
             b_next = t0[3 * DP];
             v_next = t0[3 * DP + 4 + local];
@@ -324,10 +342,8 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     }
     if (live) {
 #pragma unroll
-        for (int t = 0; t < RPT; ++t) {
-            const int i = t * DELTA_LANES + part;
-            if (i < dim) mine[i] = S[t];
-        }
+        for (int t = 0; t < RPT; ++t)
+            if (row_of(t) < dim) mine[row_of(t)] = S[t];
     }
 }
 

@@ -76,14 +76,14 @@ int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias,
                    const float* squares, int squares_rows, float eps, void* stream);
 // The product for 1..4096 rows in modes 0, 1 and 2 (the gated unit: glu_limit and its like as for fw_gemm_decode) with K split over
 // a workgroup's waves alone: no workspace, no counters. Up to 64 rows the accumulating product can leave what the norm after
-// it needs, as fw_gemm_decode does (next_activations [M][N] bfloat16, next_squares [fw_gemm_rows_squares(M, N)][16 for M <= 16,
-// else 64]), and any mode takes such prepared activations as a, with squares / squares_rows / eps. fw_gemm_rows_round: whether
+// it needs, as fw_gemm_decode does (next_activations [M][N] bfloat16, next_squares [fw_gemm_rows_square_tiles(M, N)][16 for M <= 16,
+// else 64]), and any mode takes such prepared activations as a, with squares / squares_rows / eps. fw_gemm_rows_round_fits: whether
 // its tiles are at most one round over the compute units.
 int fw_gemm_rows(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
                  const float* next_norm_weight, int next_one_centered, void* next_activations, float* next_squares, const float* squares,
                  int squares_rows, float eps, float glu_limit, float glu_alpha, float glu_shift, void* stream);
-int fw_gemm_rows_squares(int M, int N);
-int fw_gemm_rows_round(int mode, int M, int N);
+int fw_gemm_rows_square_tiles(int M, int N);
+int fw_gemm_rows_round_fits(int mode, int M, int N);
 
 // Fused product for decode steps of up to 16 rows. prologue 0: a is bfloat16 [M][K]; 1: a is
 // float32 rows, RMS-normed with norm_weight/eps (rows gathered through row_index if given) inside
@@ -365,14 +365,14 @@ int fw_tanh_rows(const float* x, void* out, int out_dtype, long long count, void
 // Per head: o_t = S^T r_t + (r_t . (u k_t)) v_t; S <- diag(exp(-exp(a_t + w0))) S + k_t v_t^T. r, k, v float32 rows of
 // rkv_stride floats (heads * dim used), a rows of a_stride; w0 [heads * dim], u [heads * dim]; state float32
 // [slots][heads][dim (key)][dim (value)]; out float32 [rows][heads * dim]. With chunks > 0 segments of more than long_rows rows
-// are walked in chunks of fw_wkv_chunk_rows() rows side by side (places as for fw_decay_recurrence; workspace: chunks * heads *
+// are walked in chunks of fw_wkv_chunk_plan() rows side by side (places as for fw_decay_recurrence; workspace: chunks * heads *
 // dim * (dim + 1) floats).
 int fw_wkv_recurrence(const float* r, const float* k, const float* v, int rkv_stride, const float* a, int a_stride,
                       const float* w0, const float* u, float* state, int slots, float* out, const int32_t* seg_row0,
                       const int32_t* seg_slot, int rows, int segments, int heads, int dim, const int32_t* chunk_seg,
                       const int32_t* chunk_row0, const int32_t* seg_chunk0, int chunks, int long_rows, int all_long,
                       float* workspace, void* stream);
-int fw_wkv_chunk_rows(void);
+int fw_wkv_chunk_plan(void);
 
 // ---- a mixture of feed-forward units chosen per token ------------------------------------------------------
 // chosen / weight [rows][top]: the `top` largest of logits[r] + bias (float32 [rows][experts]; ties: the lowest

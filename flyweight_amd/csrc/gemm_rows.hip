@@ -428,9 +428,9 @@ int rows_mode(const RowsArgs& args, const RowsPlan& plan, int out_dtype, int mod
 }  // namespace
 
 // how many rows the sums of squares left for the next norm take (the second extent: 16 for M <= 16, else 64)
-extern "C" int fw_gemm_rows_squares(int M, int N) { return rows_plan(M, N, GR_ACCUMULATE).tiles_n; }
+extern "C" int fw_gemm_rows_square_tiles(int M, int N) { return rows_plan(M, N, GR_ACCUMULATE).tiles_n; }
 
-extern "C" int fw_gemm_rows_round(int mode, int M, int N) {
+extern "C" int fw_gemm_rows_round_fits(int mode, int M, int N) {
     const RowsPlan plan = rows_plan(M, N, mode);
     return M >= 1 && M <= 4096 && (long long)plan.tiles_m * plan.tiles_n <= 256;
 }

@@ -222,6 +222,10 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
     __syncthreads();        // the zeros are in place
     put(0);
     __syncthreads();
+    // The state and the bonus have arrived here, for the compiler too: their first use being inside the loop, every token waited
+    // for all loads in flight, the next chunk's among them.
+#pragma unroll
+    for (int t = 0; t < RPT; ++t) asm volatile("" : "+v"(S[t]), "+v"(bonus[t]));
     for (int base = 0; base < count; base += WKV_CHUNK) {
         const int tokens = count - base < WKV_CHUNK ? count - base : WKV_CHUNK;
         const bool more = base + WKV_CHUNK < count;
@@ -400,7 +404,7 @@ __global__ __launch_bounds__(256) void wkv_chunk_read_kernel(const float* __rest
     }
 }
 
-extern "C" int fw_wkv_chunk_rows(void) { return WKV_ROWS; }
+extern "C" int fw_wkv_chunk_plan(void) { return WKV_ROWS; }
 
 extern "C" int fw_wkv_recurrence(const float* r, const float* k, const float* v, int rkv_stride, const float* a, int a_stride,
                                  const float* w0, const float* u, float* state, int slots, float* out, const int32_t* seg_row0,

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
 import time
 from typing import Dict, Optional
 
@@ -21,7 +22,7 @@ F32, BF16, BF16_GELU, BF16_GEGLU = 0, 1, 2, 3
 PAGE_SIZE = 64          # tokens per cache page: the width of a wavefront
 MAX_HEAD_DIM = 256          # of the matrix-core attention kernels
 MAX_PLAIN_HEAD_DIM = 1024   # of the plain attention kernels, which serve what the others do not take
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 _lib = None
 
@@ -99,6 +100,22 @@ def kernel_profile_report() -> Dict[str, Dict[str, float]]:
     return _profiled.report() if _profiled is not None else {}
 
 
+_C_TYPES = {"int": ctypes.c_int, "float": ctypes.c_float, "size_t": ctypes.c_size_t, "long long": ctypes.c_longlong}
+
+
+def _declare(lib) -> None:
+    """Gives every entry point the argument types that the kernels' header declares: addresses and numbers then go
+    through as they are. Wrapped one by one (an object per argument, about twenty of them a launch) they were a sixth of
+    what the host spends on a launch, and a short prompt's step, some hundred launches, is bound by that."""
+    with open(os.path.join(_build.CSRC, "fw_kernels.h"), "r", encoding="utf-8") as handle:
+        header = re.sub(r"//[^\n]*", "", handle.read())
+    for name, arguments in re.findall(r"\bint\s+(fw_\w+)\s*\(([^;{]*)\)\s*;", header):
+        types = [" ".join(argument.split()) for argument in arguments.split(",")]
+        entry = getattr(lib, name)
+        entry.restype = ctypes.c_int
+        entry.argtypes = [ctypes.c_void_p if "*" in t else _C_TYPES[t.rpartition(" ")[0]] for t in types if t not in ("", "void")]
+
+
 def library():
     """Loads (building first if nothing is built) the kernel library."""
     global _lib
@@ -107,8 +124,8 @@ def library():
     if _lib is None:
         path = _build.ensure_built()
         lib = ctypes.CDLL(path)
+        _declare(lib)
         lib.fw_last_error.restype = ctypes.c_char_p
-        lib.fw_abi_version.restype = ctypes.c_int
         if lib.fw_abi_version() != ABI_VERSION:
             raise KernelError(f"{path}: kernel library ABI {lib.fw_abi_version()} != {ABI_VERSION}; rebuild it")
         _lib = lib
@@ -159,19 +176,18 @@ def _stride(t: torch.Tensor) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], t.stride(0))
 
 
-def _p(t: Optional[torch.Tensor]) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def _p(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # (the tensors at hand have initialised the GPU)
 
 
-def _stream() -> ctypes.c_void_p:
+def _stream() -> int:
     """The current HIP stream of the current device (asked for at every launch: a graph
     capture or a caller's stream context changes it)."""
-    if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return _raw_stream(_device()) if _raw_stream is not None else torch.cuda.current_stream().cuda_stream
 
 
 def _want(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
@@ -200,7 +216,7 @@ def embed_rows(table: torch.Tensor, ids: torch.Tensor, out: Optional[torch.Tenso
     if copies < 1 or out.shape != ((rows, hidden) if copies == 1 else (rows, copies, hidden)):
         raise KernelError(f"embed_rows: out is {tuple(out.shape)}, expected {(rows, hidden)} ({copies} copies)")
     _check(library().fw_embed_rows(_p(table), _code(table.dtype), _p(ids), _p(out), rows, hidden, vocab,
-                                   ctypes.c_float(scale), _p(places_table), _code(places_table.dtype) if places_table is not None else F32,
+                                   float(scale), _p(places_table), _code(places_table.dtype) if places_table is not None else F32,
                                    _p(places), places_table.shape[0] if places_table is not None else 0, int(copies), _stream()))
     return out
 
@@ -211,7 +227,7 @@ def scale_softcap_(x: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> tor
     _want(x, torch.float32, "x")
     if cap < 0:
         raise KernelError("scale_softcap: the cap must not be negative")
-    _check(library().fw_scale_softcap(_p(x), ctypes.c_longlong(x.numel()), ctypes.c_float(scale), ctypes.c_float(cap), _stream()))
+    _check(library().fw_scale_softcap(_p(x), int(x.numel()), float(scale), float(cap), _stream()))
     return x
 
 
@@ -232,7 +248,7 @@ def rmsnorm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: t
     if out.shape != (rows, hidden) or out.dtype != out_dtype:
         raise KernelError("rmsnorm: out has the wrong shape or dtype")
     _check(library().fw_rmsnorm_rows(_p(x), _p(weight), _p(out), _code(out_dtype), _p(row_index), rows, hidden,
-                                     ctypes.c_float(eps), int(one_centered), _stream()))
+                                     float(eps), int(one_centered), _stream()))
     return out
 
 
@@ -312,7 +328,7 @@ def query_temperature(positions: torch.Tensor, coef: float, every: int) -> torch
     _dev(positions)
     _want(positions, torch.int32, "positions")
     out = torch.empty((positions.numel(),), dtype=torch.float32, device=positions.device)
-    _check(library().fw_query_temperature(_p(positions), _p(out), positions.numel(), ctypes.c_float(coef), int(every), _stream()))
+    _check(library().fw_query_temperature(_p(positions), _p(out), positions.numel(), float(coef), int(every), _stream()))
     return out
 
 
@@ -399,7 +415,7 @@ def qk_norm_rope_kv_write(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, 
     q_out = torch.empty((rows, num_heads * head_dim), dtype=k_pages.dtype, device=qkv.device)
     _row_scale(q_row_scale, rows)
     _check(library().fw_qk_norm_rope_kv_write(
-        _p(qkv), _code(qkv.dtype), _stride(qkv), _p(q_out), _code(k_pages.dtype), _p(q_norm_weight), _p(k_norm_weight), ctypes.c_float(eps), _p(cos), _p(sin),
+        _p(qkv), _code(qkv.dtype), _stride(qkv), _p(q_out), _code(k_pages.dtype), _p(q_norm_weight), _p(k_norm_weight), float(eps), _p(cos), _p(sin),
         rotary_dim, _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(row_seg), _p(row_pos), rows,
         num_heads, num_kv_heads, head_dim, v_dim, PAGE_SIZE, pages, int(write_kv), int(interleaved), int(q_only), _p(q_row_scale), _stream()))
     return q_out
@@ -455,8 +471,8 @@ def attention_generic(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     out = torch.empty((rows, num_heads * v_dim), dtype=q.dtype, device=q.device)
     _check(library().fw_attention_generic(
         _p(q), _p(out), _code(q.dtype), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(row_seg),
-        _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale), int(window), int(chunk),
-        ctypes.c_float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages, _stream()))
+        _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale), int(window), int(chunk),
+        float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages, _stream()))
     return out
 
 
@@ -506,15 +522,15 @@ def sample_rows(logits: torch.Tensor, settings: torch.Tensor, states: torch.Tens
 
 def fill_zero(t: torch.Tensor) -> None:
     _dev(t)
-    _check(library().fw_fill_zero(_p(t), ctypes.c_longlong(t.numel() * t.element_size()), _stream()))
+    _check(library().fw_fill_zero(_p(t), int(t.numel() * t.element_size()), _stream()))
 
 
 def fill_zero_pieces(first: torch.Tensor, pieces: int, stride_bytes: int) -> None:
     """Clears ``pieces`` runs of memory the size of ``first`` (contiguous), ``stride_bytes`` apart,
     beginning with ``first`` itself: the caller vouches that all of them lie in one allocation."""
     _dev(first)
-    _check(library().fw_fill_zero_pieces(_p(first), int(pieces), ctypes.c_longlong(first.numel() * first.element_size()),
-                                         ctypes.c_longlong(int(stride_bytes)), _stream()))
+    _check(library().fw_fill_zero_pieces(_p(first), int(pieces), int(first.numel() * first.element_size()),
+                                         int(int(stride_bytes)), _stream()))
 
 
 def gather_rows(rows: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
@@ -529,7 +545,7 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     round over the chip, the product whose waves split K; the tiled ones beyond (large tiles where they fill the chip, K cut into slices where
     even the small tiles are too few)."""
     M, K = a.shape
-    if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and M <= ROWS_MAX and library().fw_gemm_rows_round(mode, M, N)):
+    if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and M <= ROWS_MAX and library().fw_gemm_rows_round_fits(mode, M, N)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
             gemm_medium_into(a, w, bias, target, BF16, mode, N, w_tiled=w_tiled, glu=GEGLU)
         else:
@@ -713,14 +729,14 @@ def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tenso
     operand = w if w_tiled is None else w_tiled
     if mode == 0 and N >= WIDE_STORE and M <= MEDIUM_MAX_ROWS and target.data_ptr() % 16 == 0:
         _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, M, N, K, _p(squares),
-                                        squares_rows, ctypes.c_float(eps), _stream()))
+                                        squares_rows, float(eps), _stream()))
         return None
     if next_norm_weight is not None:
         next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-        next_squares = torch.empty((library().fw_gemm_rows_squares(M, N), stride), dtype=torch.float32, device=a.device)
+        next_squares = torch.empty((library().fw_gemm_rows_square_tiles(M, N), stride), dtype=torch.float32, device=a.device)
     _check(library().fw_gemm_rows(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
                                   _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
-                                  squares_rows, ctypes.c_float(eps), *_glu(glu), _stream()))
+                                  squares_rows, float(eps), *_glu(glu), _stream()))
     if next_norm_weight is not None:
         return next_activations, next_squares
     return None
@@ -859,11 +875,11 @@ def _glu(glu):
     """The three numbers a gated epilogue takes: (0, 1, 0) is SwiGLU, (-1, 1, 0) the same around the tanh form of gelu
     (``GEGLU``); else (limit > 0, alpha, shift)."""
     if glu is None or glu == GEGLU:
-        return ctypes.c_float(0.0 if glu is None else -1.0), ctypes.c_float(1.0), ctypes.c_float(0.0)
+        return float(0.0 if glu is None else -1.0), float(1.0), float(0.0)
     limit, alpha, shift = glu
     if not limit > 0:
         raise KernelError("a gated unit with clamped halves needs a positive limit")
-    return ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift)
+    return float(limit), float(alpha), float(shift)
 DECODE_MAX_ROWS = 16
 LONG_K = 4096
 LONG_K_TILED_ROWS = 8
@@ -947,7 +963,7 @@ def gemm_decode(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Option
         raise KernelError("gemm_decode: gelu goes with a plain storing product of bfloat16")
     w_tiled = _tiled_for(w, w_tiled)
     _check(library().fw_gemm_decode(
-        prologue, _p(a), _p(norm_weight), _p(row_index), ctypes.c_float(eps), int(one_centered),
+        prologue, _p(a), _p(norm_weight), _p(row_index), float(eps), int(one_centered),
         _p(w if w_tiled is None else w_tiled), int(w_tiled is not None), _p(bias),
         _p(target), BF16_GELU if gelu else _code(out_dtype), int(epilogue), rows, N, K, _p(taps), _p(conv_bias), _p(state), _p(seg_slot),
         int(kernel_size), _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares),
@@ -1009,8 +1025,8 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         raise KernelError("attention: out must be bfloat16 [rows, heads * v_dim]")
     _check(library().fw_attention_prefill(
         _p(q), _p(out), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(tile_seg), _p(tile_row0),
-        tile_seg.numel(), _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale),
-        int(window), int(chunk), ctypes.c_float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages,
+        tile_seg.numel(), _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale),
+        int(window), int(chunk), float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages,
         int(heads_together), int(halves), _stream()))
     return out
 
@@ -1057,8 +1073,8 @@ def attention_decode(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_di
     _check(library().fw_attention_decode(
         _p(q), _p(out), _p(partial), splits, int(max_context), _work(decode_work), _p(tickets), tickets.numel(), _p(k_pages), _p(v_pages),
         _p(block_table),
-        block_table.shape[1], _p(row_seg), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale),
-        int(window), int(chunk), ctypes.c_float(softcap), keep_first, sinks_at, slopes_at, PAGE_SIZE, pages, _stream()))
+        block_table.shape[1], _p(row_seg), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale),
+        int(window), int(chunk), float(softcap), keep_first, sinks_at, slopes_at, PAGE_SIZE, pages, _stream()))
     return out
 
 
@@ -1105,10 +1121,10 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, num_kv_heads: int,
     tickets = _medium_counters(qkv.device, rows * num_kv_heads * ((group + 15) // 16))
     _row_scale(q_row_scale, rows)
     _check(library().fw_attention_decode_fused(
-        _p(qkv), _p(q_norm_weight), _p(k_norm_weight), ctypes.c_float(eps), _p(cos), _p(sin), int(rotary_dim), int(write_kv), _p(out),
+        _p(qkv), _p(q_norm_weight), _p(k_norm_weight), float(eps), _p(cos), _p(sin), int(rotary_dim), int(write_kv), _p(out),
         _p(partial), splits, int(max_context), _work(decode_work), _p(tickets), tickets.numel(), _p(k_pages), _p(v_pages), _p(block_table),
-        block_table.shape[1], _p(row_seg), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale), int(window),
-        int(chunk), ctypes.c_float(softcap), int(interleaved), int(q_only), keep_first, sinks_at, slopes_at, _p(q_row_scale), PAGE_SIZE, pages,
+        block_table.shape[1], _p(row_seg), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale), int(window),
+        int(chunk), float(softcap), int(interleaved), int(q_only), keep_first, sinks_at, slopes_at, _p(q_row_scale), PAGE_SIZE, pages,
         _stream()))
     return out
 
@@ -1210,7 +1226,7 @@ def sigmoid_attention_generic(q: torch.Tensor, num_heads: int, num_kv_heads: int
     out = torch.empty((rows, num_heads * v_dim), dtype=q.dtype, device=q.device)
     _check(library().fw_sigmoid_attention_generic(
         _p(q), _p(out), _code(q.dtype), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(row_seg), _p(row_pos), rows,
-        num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale), int(window), _p(bias), _p(mix), _p(gate),
+        num_heads, num_kv_heads, head_dim, v_dim, float(scale), int(window), _p(bias), _p(mix), _p(gate),
         _stride(gate) if gate is not None else 0, PAGE_SIZE, pages, _stream()))
     return out
 
@@ -1242,8 +1258,8 @@ def sigmoid_attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int
     partial = torch.empty((floats.value,), dtype=torch.float32, device=q.device) if parts > 1 else None
     tickets = _medium_counters(q.device, counters.value)
     _check(library().fw_sigmoid_attention_prefill(
-        _p(q), _p(out), _p(partial), ctypes.c_longlong(floats.value), _p(tickets), tickets.numel(), parts, _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(tile_seg), _p(tile_row0), tile_seg.numel(),
-        _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale), int(window), _p(bias), _p(mix),
+        _p(q), _p(out), _p(partial), int(floats.value), _p(tickets), tickets.numel(), parts, _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(tile_seg), _p(tile_row0), tile_seg.numel(),
+        _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale), int(window), _p(bias), _p(mix),
         _p(gate), _stride(gate) if gate is not None else 0, PAGE_SIZE, pages, _stream()))
     return out
 
@@ -1291,9 +1307,9 @@ def sigmoid_attention_decode(num_heads: int, num_kv_heads: int, head_dim: int, v
     elif out.shape != (rows, num_heads * v_dim) or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise KernelError("sigmoid_attention: out must be bfloat16 [rows, heads * v_dim]")
     _check(library().fw_sigmoid_attention_decode(
-        _p(q), _p(qkv), _stride(qkv) if qkv is not None else 0, int(qk_norm), ctypes.c_float(eps), int(write_kv), _p(out), _p(partial), splits,
+        _p(q), _p(qkv), _stride(qkv) if qkv is not None else 0, int(qk_norm), float(eps), int(write_kv), _p(out), _p(partial), splits,
         each, int(max_context), _p(tickets), tickets.numel(), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(row_seg),
-        _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, ctypes.c_float(scale), int(window), _p(bias), _p(mix), _p(gate),
+        _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale), int(window), _p(bias), _p(mix), _p(gate),
         _stride(gate) if gate is not None else 0, PAGE_SIZE, pages, _stream()))
     return out
 
@@ -1408,7 +1424,7 @@ def gated_head_norm(o: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, h
         raise KernelError(f"gated_head_norm: o {tuple(o.shape)}, gate {tuple(gate.shape)}, weight {tuple(weight.shape)} do not fit {heads} x {vdim}")
     out = torch.empty((rows, heads * vdim), dtype=out_dtype, device=o.device)
     _check(library().fw_gated_head_norm(_p(o), _p(gate), _code(gate.dtype), gate.stride(0) if rows > 1 else max(heads * vdim, gate.stride(0)), _p(weight), int(per_head), _p(out), _code(out_dtype), rows,
-                                        heads, vdim, ctypes.c_float(eps), int(gate_silu), _stream()))
+                                        heads, vdim, float(eps), int(gate_silu), _stream()))
     return out
 
 
@@ -1429,8 +1445,8 @@ def norm_scale_add_(x: torch.Tensor, a: torch.Tensor, weight: torch.Tensor, eps:
     if weight.shape != (hidden,):
         raise KernelError(f"norm_scale_add: weight is {tuple(weight.shape)}, row width is {hidden}")
     rounded = torch.empty((rows, hidden), dtype=rounded_dtype, device=x.device) if rounded_dtype is not None else None
-    _check(library().fw_norm_scale_add(_p(x), _p(a), _p(b), ctypes.c_float(scale_a), ctypes.c_float(scale_b), _p(weight),
-                                       int(one_centered), ctypes.c_float(eps), ctypes.c_float(mult), _p(rounded),
+    _check(library().fw_norm_scale_add(_p(x), _p(a), _p(b), float(scale_a), float(scale_b), _p(weight),
+                                       int(one_centered), float(eps), float(mult), _p(rounded),
                                        _code(rounded_dtype) if rounded_dtype is not None else F32, rows, hidden, _stream()))
     return rounded
 
@@ -1442,7 +1458,7 @@ def round_rows(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
         return x
     _dev(x)
     out = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device)
-    _check(library().fw_round_rows(_p(x), _p(out), ctypes.c_longlong(x.numel()), _stream()))
+    _check(library().fw_round_rows(_p(x), _p(out), int(x.numel()), _stream()))
     return out
 
 
@@ -1454,7 +1470,7 @@ def clamped_glu(gate_up: torch.Tensor, limit: float, alpha: float, shift: float,
         raise KernelError("clamped_glu: the input holds gate and up halves, contiguous")
     out = torch.empty((rows, width // 2), dtype=out_dtype, device=gate_up.device)
     _check(library().fw_clamped_glu(_p(gate_up), _code(gate_up.dtype), _p(out), _code(out_dtype), rows, width // 2,
-                                    ctypes.c_float(limit), ctypes.c_float(alpha), ctypes.c_float(shift), _stream()))
+                                    float(limit), float(alpha), float(shift), _stream()))
     return out
 
 
@@ -1479,7 +1495,7 @@ def layernorm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype:
         _want(row_index, torch.int32, "row_index")
     out = torch.empty((rows, hidden), dtype=out_dtype, device=x.device)
     _check(library().fw_layernorm_rows(_p(x), _p(weight), _p(bias), _p(out), _code(out_dtype), _p(row_index), rows, hidden,
-                                       ctypes.c_float(eps), _stream()))
+                                       float(eps), _stream()))
     return out
 
 
@@ -1514,8 +1530,8 @@ def norm_add_norm_(x: torch.Tensor, a: torch.Tensor, weight: torch.Tensor, cente
         _dev_rows(out, "next_out")
         if out.shape != (rows, hidden) or (next_dtype is not None and out.dtype != next_dtype):
             raise KernelError(f"norm_add_norm: next_out is {tuple(out.shape)} {out.dtype}, expected {(rows, hidden)} {next_dtype}")
-    _check(library().fw_norm_add_norm(_p(x), _p(a), _p(weight), _p(bias), ctypes.c_float(mult), int(centered), ctypes.c_float(eps),
-                                      int(next_kind), _p(next_weight), _p(next_bias), ctypes.c_float(next_eps), _p(out),
+    _check(library().fw_norm_add_norm(_p(x), _p(a), _p(weight), _p(bias), float(mult), int(centered), float(eps),
+                                      int(next_kind), _p(next_weight), _p(next_bias), float(next_eps), _p(out),
                                       _code(out.dtype) if out is not None else F32, _stride(out) if out is not None else 0, rows, hidden,
                                       _stream()))
     return out
@@ -1538,7 +1554,7 @@ def gelu_rows(z: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _dev(z)
     _want(z, torch.float32, "z")
     out = torch.empty(z.shape, dtype=out_dtype, device=z.device)
-    _check(library().fw_gelu_rows(_p(z), _p(out), _code(out_dtype), ctypes.c_longlong(z.numel()), _stream()))
+    _check(library().fw_gelu_rows(_p(z), _p(out), _code(out_dtype), int(z.numel()), _stream()))
     return out
 
 
@@ -1584,7 +1600,7 @@ def latent_norm_write(raw: torch.Tensor, weight: torch.Tensor, eps: float, k_pag
     if block_table.dim() != 2 or row_seg.numel() < rows or row_pos.numel() < rows:
         raise KernelError("latent_norm_write: batch index arrays are too short")
     _check(library().fw_latent_norm_write(_p(raw), raw.stride(0) if rows > 1 else max(rank + int(rot), raw.stride(0)), 0, _p(weight),
-                                          ctypes.c_float(eps), _p(k_pages), _p(v_pages), _code(k_pages.dtype), _p(block_table),
+                                          float(eps), _p(k_pages), _p(v_pages), _code(k_pages.dtype), _p(block_table),
                                           block_table.shape[1], _p(row_seg), _p(row_pos), rows, rank, int(rot), turn, int(interleaved), _p(cos), _p(sin),
                                           PAGE_SIZE, pages, _stream()))
 
@@ -1664,7 +1680,7 @@ def token_shift_mix(x: torch.Tensor, norm_weight: Optional[torch.Tensor], eps: f
         if t.numel() < n:
             raise KernelError(f"token_shift_mix: {name} holds {t.numel()} entries, needs {n}")
     out = torch.empty((mu.shape[0], rows, hidden), dtype=out_dtype, device=x.device)
-    _check(library().fw_token_shift_mix(_p(x), _p(norm_weight), ctypes.c_float(eps), int(one_centered), _p(mu), mu.shape[0], _p(last),
+    _check(library().fw_token_shift_mix(_p(x), _p(norm_weight), float(eps), int(one_centered), _p(mu), mu.shape[0], _p(last),
                                         last.shape[0], _p(row_seg), _p(seg_row0), _p(seg_slot), _p(out), _code(out_dtype), rows,
                                         int(segments), hidden, _stream()))
     return out
@@ -1674,7 +1690,7 @@ def tanh_rows(x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
     _dev(x)
     _want(x, torch.float32, "x")
     out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
-    _check(library().fw_tanh_rows(_p(x), _p(out), _code(out_dtype), ctypes.c_longlong(x.numel()), _stream()))
+    _check(library().fw_tanh_rows(_p(x), _p(out), _code(out_dtype), int(x.numel()), _stream()))
     return out
 
 
@@ -1712,7 +1728,7 @@ def wkv_recurrence(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a: torch.T
             raise KernelError(f"wkv_recurrence: {name} holds {t.numel()} entries, needs {n}")
     out = torch.empty((rows, width), dtype=torch.float32, device=r.device)
     places, count, *how = _chunks("wkv_recurrence", chunks, segments)
-    if count and library().fw_wkv_chunk_rows() != DECAY_CHUNK:
+    if count and library().fw_wkv_chunk_plan() != DECAY_CHUNK:
         raise KernelError("the kernel library's chunks are of another length")
     workspace = torch.empty(count * width * (dim + 1), dtype=torch.float32, device=r.device) if count else None
     _check(library().fw_wkv_recurrence(_p(r), _p(k), _p(v), stride(r), _p(a), stride(a), _p(w0), _p(u), _p(state), state.shape[0], _p(out),
@@ -1753,7 +1769,7 @@ def moe_route(logits: torch.Tensor, bias: Optional[torch.Tensor], top: int, grou
     chosen = torch.empty((rows, top), dtype=torch.int32, device=logits.device)
     weight = torch.empty((rows, top), dtype=torch.float32, device=logits.device)
     _check(library().fw_moe_route(_p(logits), _stride(logits), _p(bias), _p(correction), _p(chosen), _p(weight), rows, experts, int(top),
-                                  int(groups), int(keep), int(group_pair), MOE_SCORES.index(scores), ctypes.c_float(weight_scale),
+                                  int(groups), int(keep), int(group_pair), MOE_SCORES.index(scores), float(weight_scale),
                                   int(normalize), _stream()))
     return chosen, weight
 
@@ -1884,7 +1900,7 @@ def rglru_scan(u: torch.Tensor, gates: torch.Tensor, y: torch.Tensor, r_bias: to
         return t.stride(0) if rows > 1 else max(channels, t.stride(0))
 
     _check(library().fw_rglru_scan(_p(u), stride(u), _p(gates), 2 * channels, _p(y), stride(y), _p(r_bias), _p(i_bias), _p(lam),
-                                   ctypes.c_float(rate), _p(state), _p(seg_row0), _p(seg_slot), _p(out), _code(out_dtype), rows,
+                                   float(rate), _p(state), _p(seg_row0), _p(seg_slot), _p(out), _code(out_dtype), rows,
                                    int(segments), channels, int(block_width), state.shape[0], _p(workspace), _stream()))
     return out
 
@@ -1976,8 +1992,8 @@ def stream_join_(x: torch.Tensor, ls: torch.Tensor, mix: torch.Tensor, out_weigh
         raise KernelError(f"stream_join: a is {tuple(a.shape)}, expected {(places, hidden)}")
     out = torch.empty((rows, hidden), dtype=next_dtype or torch.float32, device=x.device) if next_kind != NEXT_NOTHING else None
     _check(library().fw_stream_join(
-        _p(x), streams, _p(ls), _p(mix), _p(out_weight), source, _p(a), _p(b), _p(weight_a), _p(weight_b), ctypes.c_float(scale_a),
-        ctypes.c_float(scale_b), ctypes.c_float(eps), _p(choice_weight), _p(pair_place), int(top), _p(gate),
+        _p(x), streams, _p(ls), _p(mix), _p(out_weight), source, _p(a), _p(b), _p(weight_a), _p(weight_b), float(scale_a),
+        float(scale_b), float(eps), _p(choice_weight), _p(pair_place), int(top), _p(gate),
         _stride(gate) if gate is not None else 0, *_reader(next_kind, streams, hidden, next_in, next_weight, next_bias, next_alpha), _p(out),
         _code(out.dtype) if out is not None else F32, rows, hidden, _stream()))
     return out
