@@ -185,29 +185,44 @@ __device__ __forceinline__ float delta_row_sum(float x) {
     return x;
 }
 
-// Workgroup (segment, head, block of 16 value channels); thread = 16 * column + part: a column of S
-// is shared out over the 16 lanes of a row of the wave, RPT rows each (from four rows on in runs of four, 4 part .. + 3 of
+template <int DELTA_LANES>
+__device__ __forceinline__ float delta_lanes_sum(float x) {
+    x = delta_row_sum(x);
+    if (DELTA_LANES == 32) {
+        float mine, partner;
+        fw_quad_partners16(x, mine, partner);
+        x = mine + partner;
+    }
+    return x;
+}
+
+// Workgroup (segment, head, block of 16 value channels, or 8 on 32 lanes); thread = lanes * column + part: a column of S is
+// shared out over 16 or 32 lanes of the wave, RPT rows each (from four rows on in runs of four, 4 part .. + 3 of
 // every 64: a lane then reads four floats of q, k and g from LDS at a time, the sixteen lanes all banks once. Read one
-// float at a time, 26 reads a token and wave kept LDS busier than the sums kept the vector unit: FIGURES; rows from
+// float at a time, 26 reads a token and wave kept LDS busier than the sums kept the vector unit; rows from
 // dim on hold zeros), so that a head is spread over many compute units: the walk along the
 // tokens is one dependent chain per column, and only its width can be bought. LDS per staged token:
 // q, k, g (16 * RPT each; past the record's padded dim they stay zero), beta and three unused, then the
 // block's 16 values. A thread copies the same pieces of every chunk (16-byte pieces: where each lies in
 // a token's record and in LDS is worked out once).
-#define DELTA_LANES 16
-#define DELTA_COLUMNS (256 / DELTA_LANES)
-template <int RPT>
+// The walk is bound by how fast one wave a SIMD issues its chain (about 7 clocks an instruction, twice what several waves get):
+// a prompt's heads of more than 64 key channels take 32 lanes a column, half the arithmetic a wave on twice the
+// workgroups. 16 heads of 128 channels, 694 rows in the mean: 205 us with operands read one float at a time, 172 read four at a
+// time, 146 on 32 lanes. (Two tokens at a time, their sums travelling together, gained nothing more: 147; nor did chunks of 32
+// tokens.) Steps of single rows lose on 32 lanes (8 rows 8.4 against 11.5 us).
+template <int RPT, int DELTA_LANES>
 __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     const float* __restrict__ records, float* __restrict__ state, float* __restrict__ out,
     const int32_t* __restrict__ seg_row0, const int32_t* __restrict__ seg_slot, int heads, int dim, int vdim) {
     typedef __attribute__((ext_vector_type(4))) float f32x4;
+    constexpr int DELTA_COLUMNS = 256 / DELTA_LANES;
     constexpr int DP = DELTA_LANES * RPT;
     constexpr int RUN = RPT >= 4 ? 4 : 1;                                // neighbouring rows of a lane
     constexpr int TOKEN = 3 * DP + 4 + DELTA_COLUMNS;
     constexpr int PIECES = (DELTA_CHUNK * (TOKEN / 4) + 255) / 256;      // 16-byte pieces of a chunk per thread, at most
     __shared__ __attribute__((aligned(16))) float staged[DELTA_CHUNK * TOKEN];
     __shared__ float results[DELTA_CHUNK * DELTA_COLUMNS];
-    static_assert(DELTA_CHUNK * DELTA_COLUMNS == 256, "a chunk's read-outs are one per thread");
+    static_assert(DELTA_CHUNK * DELTA_COLUMNS <= 256, "a chunk's read-outs are at most one per thread");
     const int seg = blockIdx.x, head = blockIdx.y, block = blockIdx.z;
     const int local = threadIdx.x / DELTA_LANES, part = threadIdx.x % DELTA_LANES;
     const int column = block * DELTA_COLUMNS + local;
@@ -321,9 +336,9 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
                 kq = fmaf(k_now[t], q_next[t], kq);
             }
             fetch(token + 1 < DELTA_CHUNK ? token + 1 : token);      // (behind the chunk's last token: read again, not used)
-            seen = delta_row_sum(seen);
-            read_before = delta_row_sum(read_before);
-            kq = delta_row_sum(kq);
+            seen = delta_lanes_sum<DELTA_LANES>(seen);
+            read_before = delta_lanes_sum<DELTA_LANES>(read_before);
+            kq = delta_lanes_sum<DELTA_LANES>(kq);
             const float u = b * (v - seen);
 #pragma unroll
             for (int t = 0; t < RPT; ++t) S[t] = fmaf(k_now[t], u, S[t]);
@@ -349,21 +364,21 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
 
 extern "C" int fw_gated_delta_rule(const float* records, float* state, float* out, const int32_t* seg_row0,
                                    const int32_t* seg_slot, int rows, int segments, int heads, int dim, int vdim,
-                                   int slots, void* stream) {
+                                   int slots, int spread, void* stream) {
     FW_REQUIRE(rows >= 0 && segments >= 0 && heads > 0, "gated_delta_rule: bad sizes rows=%d segments=%d heads=%d", rows, segments, heads);
     FW_REQUIRE(dim > 0 && dim <= 256 && vdim > 0, "gated_delta_rule: dim %d must lie in 1..256 and vdim %d be positive", dim, vdim);
     FW_REQUIRE(slots > 0 && segments <= 65535 && heads <= 65535, "gated_delta_rule: too many segments or heads, or no slots");
     FW_REQUIRE((uintptr_t)records % 16 == 0, "gated_delta_rule: the records must lie at a multiple of 16 bytes");
     if (rows == 0 || segments == 0) return 0;
-    dim3 grid(segments, heads, (vdim + DELTA_COLUMNS - 1) / DELTA_COLUMNS);
     hipStream_t s = (hipStream_t)stream;
-#define FW_DELTA_LAUNCH(RPT) \
-    gated_delta_rule_kernel<RPT><<<grid, 256, 0, s>>>(records, state, out, seg_row0, seg_slot, heads, dim, vdim)
-    if (dim <= 16) FW_DELTA_LAUNCH(1);
-    else if (dim <= 32) FW_DELTA_LAUNCH(2);
-    else if (dim <= 64) FW_DELTA_LAUNCH(4);
-    else if (dim <= 128) FW_DELTA_LAUNCH(8);
-    else FW_DELTA_LAUNCH(16);
+#define FW_DELTA_LAUNCH(RPT, LANES)                                                                                     \
+    gated_delta_rule_kernel<RPT, LANES><<<dim3(segments, heads, fw_ceil_div(vdim, 256 / LANES)), 256, 0, s>>>(          \
+        records, state, out, seg_row0, seg_slot, heads, dim, vdim)
+    if (dim <= 16) FW_DELTA_LAUNCH(1, 16);
+    else if (dim <= 32) FW_DELTA_LAUNCH(2, 16);
+    else if (dim <= 64) FW_DELTA_LAUNCH(4, 16);
+    else if (dim <= 128) { if (spread) FW_DELTA_LAUNCH(4, 32); else FW_DELTA_LAUNCH(8, 16); }
+    else { if (spread) FW_DELTA_LAUNCH(8, 32); else FW_DELTA_LAUNCH(16, 16); }
 #undef FW_DELTA_LAUNCH
     FW_LAUNCH_CHECK("gated_delta_rule");
     return 0;

@@ -294,10 +294,11 @@ int fw_delta_prepare(const void* proj, int dtype, int proj_stride, int beta_col,
                      int heads, int kv_heads, int dim, int vdim, int taps_count, int slots, int decay_per_head, void* stream);
 // Per segment and head, token by token: S <- diag(g) S; u = beta (v - S^T k); S <- S + k u^T;
 // o = S^T q. records [rows][H][fw_delta_record_floats]. state [slots][H][vd][d] (S transposed), read
-// at the segment's start and written at its end. out [rows][H vd].
+// at the segment's start and written at its end. out [rows][H vd]. spread: heads of more than 64 key channels on twice the
+// workgroups (for prompts; other sums over key channels, so other roundings).
 int fw_gated_delta_rule(const float* records, float* state, float* out, const int32_t* seg_row0,
                         const int32_t* seg_slot, int rows, int segments, int heads, int dim, int vdim,
-                        int slots, void* stream);
+                        int slots, int spread, void* stream);
 // out[r][h][j] = o[r][h][j] * rsqrt(mean_j o[r][h]^2 + eps) * weight[j] * act(gate[r][h vd + j]);
 // act is the sigmoid, or with gate_silu z * sigmoid(z)
 int fw_gated_head_norm(const float* o, const void* gate, int gate_dtype, int gate_stride, const float* weight, int weight_per_head,

@@ -1387,8 +1387,9 @@ def delta_record_floats(dim: int, vdim: int) -> int:
 
 
 def gated_delta_rule(records: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor,
-                     segments: int, heads: int, dim: int, vdim: int) -> torch.Tensor:
-    """The recurrence over each segment's rows. ``records`` [rows, heads, delta_record_floats]: what
+                     segments: int, heads: int, dim: int, vdim: int, spread: bool = False) -> torch.Tensor:
+    """The recurrence over each segment's rows (``spread``: large heads on twice the workgroups, for prompts).
+    ``records`` [rows, heads, delta_record_floats]: what
     ``delta_prepare`` made. ``state`` [slots, heads, vdim, dim] float32 (the matrix transposed) is read
     at a segment's start and written at its end. Returns [rows, heads vdim]."""
     _dev(records, state, seg_row0, seg_slot)
@@ -1405,7 +1406,7 @@ def gated_delta_rule(records: torch.Tensor, state: torch.Tensor, seg_row0: torch
             raise KernelError(f"gated_delta_rule: {name} holds {t.numel()} entries, needs {n}")
     out = torch.empty((rows, heads * vdim), dtype=torch.float32, device=records.device)
     _check(library().fw_gated_delta_rule(_p(records), _p(state), _p(out), _p(seg_row0), _p(seg_slot), rows, int(segments), heads,
-                                         dim, vdim, state.shape[0], _stream()))
+                                         dim, vdim, state.shape[0], int(spread), _stream()))
     return out
 
 

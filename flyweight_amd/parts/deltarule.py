@@ -164,8 +164,9 @@ class GatedDeltaRule(Mixer):
         records = ops.delta_prepare(proj, self.beta_col, a, self.taps, self._conv_state(cache), self.A_log, self.dt_bias,
                                     ctx.row_seg, ctx.seg_row0, ctx.seg_slot, ctx.num_segments, self.heads, self.kv_heads,
                                     self.dim, self.vdim, decay_per_head=per_head)
+        # (a float32 run gives the same bits however a sequence is cut into steps: its prompts walk as its single rows do)
         o = ops.gated_delta_rule(records, cache["state"].state, ctx.seg_row0, ctx.seg_slot, ctx.num_segments,
-                                 self.heads, self.dim, self.vdim)
+                                 self.heads, self.dim, self.vdim, spread=self.dtype == torch.bfloat16 and not ctx.all_decode)
         return ops.gated_head_norm(o, gate, self.norm_weight, self.heads, self.vdim, self.eps, self.dtype,
                                    gate_silu=self.gate == "silu")
 

@@ -123,6 +123,37 @@ def test_what_the_recurrence_reads(taps):
             np.testing.assert_allclose(after[slot], np.concatenate([before, x])[-(taps - 1):].T, atol=1e-6)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 20), (3, 66, 70), (2, 128, 40), (1, 130, 129), (1, 256, 9)])
+def test_recurrence_spread_over_more_workgroups(heads, dim, vdim):
+    """Segments at the edges of a chunk of 16 tokens, heads whose key channels fill their lanes or not and whose value channels end
+    inside a block of 8; channels that never forget and some that forget at once. The tolerance of the walk on 16 lanes."""
+    from flyweight_amd.kernels import ops
+    rng = np.random.default_rng(dim)
+    lengths, slots_of = [1, 2, 15, 16, 17, 33, 48], [6, 0, 5, 1, 4, 2, 3]
+    rows = sum(lengths)
+    q, k = plain.unit(rng.normal(size=(rows, heads, dim))) * dim ** -0.5, plain.unit(rng.normal(size=(rows, heads, dim)))
+    v, beta = rng.normal(size=(rows, heads, vdim)), rng.uniform(0.1, 1.0, size=(rows, heads))
+    decay = rng.uniform(0.5, 1.0, size=(rows, heads, dim))
+    decay[:, 0, ::2], decay[::5, :, 1] = 1.0, 0.0
+    start = rng.normal(size=(7, heads, dim, vdim))
+    state = dev(start.transpose(0, 1, 3, 2))
+    at = record_layout(dim, vdim)
+    records = np.zeros((rows, heads, at["floats"]))
+    for name, part, width in (("q", q, dim), ("k", k, dim), ("g", decay, dim), ("v", v, vdim)):
+        records[:, :, at[name]:at[name] + width] = part
+    records[:, :, at["beta"]] = beta
+    seg_row0 = np.concatenate([[0], np.cumsum(lengths)])
+    out = ops.gated_delta_rule(dev(records), state, ints(seg_row0), ints(slots_of), len(lengths), heads, dim, vdim, spread=True)
+    out, after = out.cpu().numpy().reshape(rows, heads, vdim), state.cpu().numpy().transpose(0, 1, 3, 2)
+    for seg, slot in enumerate(slots_of):
+        for head in range(heads):
+            S = start[slot, head].copy()
+            for t in range(seg_row0[seg], seg_row0[seg + 1]):
+                S, o = plain.delta_rule_step(S, q[t, head], k[t, head], v[t, head], beta[t, head], decay[t, head])
+                np.testing.assert_allclose(out[t, head], o, rtol=0, atol=2e-5 * max(1.0, np.abs(o).max()))
+            np.testing.assert_allclose(after[slot, head], S, rtol=0, atol=2e-5 * max(1.0, np.abs(S).max()))
+
+
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_gated_head_norm(out_dtype):
     from flyweight_amd.kernels import ops
