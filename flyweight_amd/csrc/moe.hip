@@ -177,11 +177,14 @@ extern "C" int fw_moe_route(const float* logits, int logits_stride, const float*
 
 // ---- sorting the pairs by expert ------------------------------------------------------------------------
 // One workgroup of 16 waves; the pairs are cut into 16 runs, one a wave, in order. Pass 1: every wave counts
-// its run's pairs per expert (LDS counters [wave][expert]). A thread per expert then turns the counts into
-// where the expert begins (a scan over the experts by one thread) and where each wave's pairs of it begin.
-// Pass 2: every wave walks its run 64 pairs at a time; the lanes that chose the same expert number themselves
-// by a prefix count (ballot), one expert after the other, behind the wave's running place for that expert.
-// So an expert's places hold its pairs in the order (row, choice), whatever the timing.
+// its run's pairs per expert (LDS counters [wave][expert]). The counts become where the expert begins (a scan
+// by the first wave, 64 experts at a time) and where each wave's pairs of it begin (a thread per expert).
+// Pass 2: every wave walks its run 64 pairs at a time. A lane finds the lanes that chose its expert by one vote
+// a bit of the expert's number, its place among them by a prefix count, and puts its pair behind the wave's
+// running place for that expert. So an expert's places hold its pairs in the order (row, choice), whatever the
+// timing. Bound by latency: a round of 64 pairs is a load (the next round's is asked for ahead), the votes (at
+// most 10) and an LDS read. Votes a bit against votes an expert (up to 64 rounds of shuffle, vote and LDS one
+// after the other): 2,048 rows choosing 6 of 64 experts 87 -> 12 us, 8 of 256 159 -> 18 us, 8 rows 7.6 -> 3.2 us.
 // expert_begin [experts + 1]; place_row [pairs]; pair_place [pairs].
 #define MOE_ARRANGE_THREADS 1024
 #define MOE_ARRANGE_WAVES (MOE_ARRANGE_THREADS / 64)
@@ -195,6 +198,7 @@ __global__ __launch_bounds__(MOE_ARRANGE_THREADS) void moe_arrange_kernel(const 
     const int run0 = wave * run, run_end = run0 + run < pairs ? run0 + run : pairs;
     for (int i = tid; i < MOE_ARRANGE_WAVES * experts; i += MOE_ARRANGE_THREADS) counts[i] = 0;
     __syncthreads();
+#pragma unroll 4
     for (int i = run0 + lane; i < run_end; i += 64) atomicAdd(&counts[wave * experts + chosen[i]], 1);
     __syncthreads();
     for (int e = tid; e < experts; e += MOE_ARRANGE_THREADS) {
@@ -203,14 +207,20 @@ __global__ __launch_bounds__(MOE_ARRANGE_THREADS) void moe_arrange_kernel(const 
         begins[e] = total;
     }
     __syncthreads();
-    if (tid == 0) {
-        int running = 0;
-        for (int e = 0; e < experts; ++e) {
-            const int n = begins[e];
-            begins[e] = running;
-            running += n;
+    if (wave == 0) {
+        int behind = 0;                         // pairs of the experts before these 64
+        for (int e0 = 0; e0 < experts; e0 += 64) {
+            const int n = e0 + lane < experts ? begins[e0 + lane] : 0;
+            int sum = n;
+#pragma unroll
+            for (int step = 1; step < 64; step <<= 1) {
+                const int before = __shfl_up(sum, step, 64);
+                if (lane >= step) sum += before;
+            }
+            if (e0 + lane < experts) begins[e0 + lane] = behind + sum - n;
+            behind += __shfl(sum, 63, 64);
         }
-        begins[experts] = running;
+        if (lane == 0) begins[experts] = behind;
     }
     __syncthreads();
     for (int e = tid; e <= experts; e += MOE_ARRANGE_THREADS) expert_begin[e] = begins[e];
@@ -224,23 +234,26 @@ __global__ __launch_bounds__(MOE_ARRANGE_THREADS) void moe_arrange_kernel(const 
     }
     __syncthreads();
     int32_t* next = counts + wave * experts;    // this wave's running place for every expert; only this wave touches it
+    const int bits = experts > 1 ? 32 - __clz(experts - 1) : 0;
+    int e = run0 + lane < run_end ? chosen[run0 + lane] : -1;
     for (int i0 = run0; i0 < run_end; i0 += 64) {
         const int i = i0 + lane;
-        const int e = i < run_end ? chosen[i] : -1;
-        unsigned long long left = __ballot(e >= 0);
-        while (left) {
-            const int leader = __ffsll((long long)left) - 1;
-            const int expert = __shfl(e, leader, 64);
-            const unsigned long long votes = __ballot(e == expert);
-            const int first = next[expert];
-            if (e == expert) {
-                const int place = first + __popcll(votes & ((1ull << lane) - 1ull));
-                place_row[place] = i / top;
-                pair_place[i] = place;
-            }
-            if (lane == leader) next[expert] = first + __popcll(votes);
-            left &= ~votes;
+        const int e_next = i + 64 < run_end ? chosen[i + 64] : -1;
+        unsigned long long same = __ballot(e >= 0);
+        for (int bit = 0; bit < bits; ++bit) {
+            const bool set = (e >> bit) & 1;
+            const unsigned long long votes = __ballot(set);
+            same &= set ? votes : ~votes;
         }
+        if (e >= 0) {
+            const int rank = __popcll(same & ((1ull << lane) - 1ull));
+            const int first = next[e];
+            place_row[first + rank] = i / top;
+            pair_place[i] = first + rank;
+            if ((same >> lane) == 1) next[e] = first + rank + 1;        // the last of the lanes that chose it
+        }
+        __builtin_amdgcn_wave_barrier();
+        e = e_next;
     }
 }
 

@@ -219,6 +219,18 @@ def test_moe_arrange_keeps_an_experts_pairs_in_their_order(ops):
             assert list(place_row[begin[e]:begin[e + 1]]) == list(mine // top)
 
 
+@pytest.mark.parametrize("rows,experts,top", [(1, 1, 1), (1100, 1, 1), (513, 64, 6), (170, 65, 64), (200, 1024, 8), (2049, 33, 5)])
+def test_moe_arrange_at_the_edges_of_its_rounds(ops, rows, experts, top):
+    """One expert (no vote at all), all lanes of a round on one expert, experts around the scan's 64 and at its most."""
+    rng = np.random.default_rng(rows)
+    chosen = np.stack([rng.permutation(experts)[:top] for _ in range(rows)]).astype(np.int32)
+    chosen[: rows // 3] = chosen[0]
+    begin, place_row, pair_place = (t.cpu().numpy() for t in ops.moe_arrange(ints(chosen), experts))
+    order = np.argsort(chosen.reshape(-1), kind="stable")
+    assert list(begin) == [0] + list(np.cumsum(np.bincount(chosen.reshape(-1), minlength=experts)))
+    assert list(place_row) == list(order // top) and list(pair_place.reshape(-1)[order]) == list(range(rows * top))
+
+
 # ---- the experts' products ---------------------------------------------------------------------------------
 def plain_grouped(a, rows_of_places, w, begin, gated):
     out = []
