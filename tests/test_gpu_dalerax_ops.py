@@ -205,6 +205,20 @@ def test_moe_route(ops, experts, top):
     assert list(no_bias[3]) == list(range(top))
 
 
+@pytest.mark.parametrize("experts", [1, 64, 65, 128, 129, 256, 257, 1024])
+def test_moe_route_where_the_slots_of_a_lane_end(ops, experts):
+    """Few values and many ties, which the lowest expert wins: the choice is a stable sort's, whatever the slot it lies in."""
+    rng = np.random.default_rng(experts)
+    top = min(experts, 8)
+    logits = (rng.integers(-3, 4, size=(40, experts)) / 4).astype(np.float32)
+    logits[0, -1] = 2.0
+    chosen, weight = ops.moe_route(dev(logits), None, top)
+    want = np.argsort(-logits, axis=1, kind="stable")[:, :top]
+    assert np.array_equal(chosen.cpu().numpy(), want)
+    shares = np.exp(np.take_along_axis(logits, want, 1).astype(np.float64))
+    assert np.abs(host(weight) - shares / shares.sum(1, keepdims=True)).max() < 1e-6     # float32 exponentials and one division
+
+
 def test_moe_arrange_keeps_an_experts_pairs_in_their_order(ops):
     rng = np.random.default_rng(5)
     for rows, experts, top in ((1, 4, 2), (37, 5, 3), (700, 12, 4), (3000, 130, 2)):
