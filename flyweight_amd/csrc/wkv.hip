@@ -286,8 +286,8 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
 // of WKV_ROWS rows, the walks run side by side from zero states (the kernel above, CUT); with P_t the product of the
 // chunk's decays before row t and S_in the state ahead of the chunk,
 //     o_t += S_in^T (P_t r_t);      S_out = diag(shrink) S_in + local
-// Bound by the walks' instructions once the chip is full of them. 2,048 rows of 32 heads of 64 channels: 420 us in order ->
-// 108 us (the walks) + 14 (the states) + 20 (the read-outs, which read and write every output once more).
+// Bound by the walks' instructions once the chip is full of them. 2,048 rows of 32 heads of 64 channels: 401 us in order ->
+// 111 us (the walks) + 14 (the states) + 21 (the read-outs, which read and write every output once more).
 
 // local[chunk] becomes the state ahead of the chunk, the slot moves on to the state behind the segment. A thread per element of
 // (segment, head): loads and one multiply-add per chunk, eight chunks asked for at once.

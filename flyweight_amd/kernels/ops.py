@@ -665,7 +665,7 @@ TICKET_COUNTERS = 1 << 20      # 4 MB per device
 
 def _medium_counters(device: torch.device, count: int) -> torch.Tensor:
     """Zeroed int32 counters for the tickets of the kernels whose last workgroup finishes the
-    work of the others (the medium product, decode attention), one set per device: each kernel
+    work of the others (products whose K is cut over workgroups, decode attention), one set per device: each kernel
     leaves them at zero, and calls on one device follow each other in stream order (work on
     several streams of one device at once would need a set per stream). The set is allocated
     once and never replaced: recorded graphs hold its address."""

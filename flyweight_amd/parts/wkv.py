@@ -36,7 +36,7 @@ _MIXES = ("r", "k", "v", "g", "w")
 @register_mixer("wkv")
 class Wkv(RecurrenceChunks, Mixer):
     graph_safe = True
-    LONG_ROWS = 128                 # 32 heads of 64 channels, one segment: 96 rows 25.6 us in order, 27.1 in chunks; 128 rows 32.3 and 27.6
+    LONG_ROWS = 128                 # 32 heads of 64 channels, one segment: 96 rows 23.9 us in order, 27.2 in chunks; 128 rows 30.3 and 27.5
     accepts_lazy_norm = True        # the norm in front is taken into the kernel that forms the mixes
     wants_unnormed_rows = True      # ... in float32, from the residual rows themselves: it asks for them also where the normed rows exist
 
@@ -66,9 +66,9 @@ class Wkv(RecurrenceChunks, Mixer):
         return super().step_arrays(batch) if self.dtype == torch.bfloat16 else {}
 
     def chunk_arguments(self, ctx) -> dict:
-        """The walk in order takes 0.22 us a row of the longest segment, however many there are; the chunks about 20 us and, the chip
+        """The walk in order takes 0.20 to 0.24 us a row of the longest segment, however many there are; the chunks about 20 us and, the chip
         being full, 1 us for 2,200 rows of a workgroup's 16 value channels of one head. (32 heads of 64 channels: one segment
-        of 2,048 rows 441 us in order, 140 in chunks; four of 512 rows 125 and 129.)"""
+        of 2,048 rows 401 us in order, 147 in chunks; four of 512 rows 117 and 127.)"""
         lengths = [b - a for a, b in zip(ctx.host_seg_row0, ctx.host_seg_row0[1:])]
         work = sum(n for n in lengths if n > self.LONG_ROWS) * self.heads * -(-self.dim // 16)
         return super().chunk_arguments(ctx) if 20.0 + work / 2200.0 < 0.22 * max(lengths) else {}
