@@ -11,15 +11,18 @@ from __future__ import annotations
 
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
 import tempfile
 import time
+import zlib
 from concurrent.futures import ThreadPoolExecutor
-from typing import List, Optional
+from typing import List, Optional, Tuple
 
 CSRC = os.path.normpath(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "csrc"))
+HEADER = os.path.join(CSRC, "fw_kernels.h")
 LIB_NAME = "libflyweight_hip.so"
 ARCH = "gfx950"
 # packed float32 instructions are switched off: the compiler otherwise forms them from
@@ -36,13 +39,36 @@ def sources() -> List[str]:
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
 
 
+def declarations(header: Optional[str] = None) -> List[Tuple[str, List[str]]]:
+    """(name, arguments as they are declared) of every entry point that the kernels' header declares to return an int."""
+    if header is None:
+        with open(HEADER, "r", encoding="utf-8") as handle:
+            header = handle.read()
+    header = re.sub(r"//[^\n]*", "", header)
+    found = []
+    for name, arguments in re.findall(r"\bint\s+(fw_\w+)\s*\(([^;{]*)\)\s*;", header):
+        words = [" ".join(argument.split()) for argument in arguments.split(",")]
+        found.append((name, [word for word in words if word not in ("", "void")]))
+    return found
+
+
+def abi_version(header: Optional[str] = None) -> int:
+    """The number by which the package and a built library know that they mean the same entry points: formed from their
+    declarations, so no signature changes without it."""
+    return zlib.crc32(repr(declarations(header)).encode()) & 0x7fffffff
+
+
+def compile_flags() -> List[str]:
+    return [*FLAGS, f"-DFW_ABI_VERSION={abi_version()}"]
+
+
 def _fingerprint() -> str:
     digest = hashlib.sha256()
     for path in sources() + sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")):
         digest.update(os.path.basename(path).encode())
         with open(path, "rb") as handle:
             digest.update(handle.read())
-    digest.update(" ".join(FLAGS).encode())
+    digest.update(" ".join(compile_flags()).encode())
     return digest.hexdigest()
 
 
@@ -97,6 +123,7 @@ def build(verbose: bool = True) -> str:
     hipcc = _hipcc()
     folder = _writable_dir()
     files = sources()
+    flags = compile_flags()
     started = time.time()
     if verbose:
         _say(f"building {LIB_NAME} for {ARCH} from {len(files)} sources in {folder}")
@@ -106,7 +133,7 @@ def build(verbose: bool = True) -> str:
     def compile_one(path: str) -> str:
         obj = os.path.join(folder, os.path.basename(path)[:-4] + ".o")
         begun = time.time()
-        result = subprocess.run([hipcc, *FLAGS, "-c", path, "-o", obj], capture_output=True, text=True, env=env)
+        result = subprocess.run([hipcc, *flags, "-c", path, "-o", obj], capture_output=True, text=True, env=env)
         if result.returncode != 0:
             raise RuntimeError(f"hipcc failed on {path}:\n{result.stderr}")
         if verbose:

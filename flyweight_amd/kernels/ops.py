@@ -9,7 +9,6 @@ from __future__ import annotations
 
 import ctypes
 import os
-import re
 import time
 from typing import Dict, Optional
 
@@ -22,7 +21,6 @@ F32, BF16, BF16_GELU, BF16_GEGLU = 0, 1, 2, 3
 PAGE_SIZE = 64          # tokens per cache page: the width of a wavefront
 MAX_HEAD_DIM = 256          # of the matrix-core attention kernels
 MAX_PLAIN_HEAD_DIM = 1024   # of the plain attention kernels, which serve what the others do not take
-ABI_VERSION = 19
 
 _lib = None
 
@@ -107,13 +105,10 @@ def _declare(lib) -> None:
     """Gives every entry point the argument types that the kernels' header declares: addresses and numbers then go
     through as they are. Wrapped one by one (an object per argument, about twenty of them a launch) they were a sixth of
     what the host spends on a launch, and a short prompt's step, some hundred launches, is bound by that."""
-    with open(os.path.join(_build.CSRC, "fw_kernels.h"), "r", encoding="utf-8") as handle:
-        header = re.sub(r"//[^\n]*", "", handle.read())
-    for name, arguments in re.findall(r"\bint\s+(fw_\w+)\s*\(([^;{]*)\)\s*;", header):
-        types = [" ".join(argument.split()) for argument in arguments.split(",")]
+    for name, arguments in _build.declarations():
         entry = getattr(lib, name)
         entry.restype = ctypes.c_int
-        entry.argtypes = [ctypes.c_void_p if "*" in t else _C_TYPES[t.rpartition(" ")[0]] for t in types if t not in ("", "void")]
+        entry.argtypes = [ctypes.c_void_p if "*" in argument else _C_TYPES[argument.rpartition(" ")[0]] for argument in arguments]
 
 
 def library():
@@ -124,10 +119,12 @@ def library():
     if _lib is None:
         path = _build.ensure_built()
         lib = ctypes.CDLL(path)
-        _declare(lib)
         lib.fw_last_error.restype = ctypes.c_char_p
-        if lib.fw_abi_version() != ABI_VERSION:
-            raise KernelError(f"{path}: kernel library ABI {lib.fw_abi_version()} != {ABI_VERSION}; rebuild it")
+        lib.fw_abi_version.restype = ctypes.c_int
+        wanted = _build.abi_version()       # compared first: a library of another interface may lack what is declared now
+        if lib.fw_abi_version() != wanted:
+            raise KernelError(f"{path}: kernel library ABI {lib.fw_abi_version()} != {wanted}; rebuild it")
+        _declare(lib)
         _lib = lib
         if os.environ.get("FLYWEIGHT_KERNEL_PROFILE", "")[:1] == "1":
             kernel_profile(True)
