@@ -123,7 +123,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
 #pragma unroll
         for (int i = 0; i < SLOTS; ++i) best = fmaxf(best, z[i]);
         best = wave_max(best);
-        int best_id = 0x7fffffff;               // the lowest expert that holds it
+        int best_id = 0;                        // the lowest expert that holds it; a row of NaN alone has none, and its NaN weights go to expert 0
 #pragma unroll
         for (int i = SLOTS - 1; i >= 0; --i) {
             const unsigned long long holders = __ballot(z[i] == best && lane + 64 * i < experts);

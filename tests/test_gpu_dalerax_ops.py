@@ -219,6 +219,24 @@ def test_moe_route_where_the_slots_of_a_lane_end(ops, experts):
     assert np.abs(host(weight) - shares / shares.sum(1, keepdims=True)).max() < 1e-6     # float32 exponentials and one division
 
 
+@pytest.mark.parametrize("experts,scores", [(7, "softmax_chosen"), (64, "softmax_all"), (300, "sigmoid")])
+def test_moe_route_names_experts_that_exist_for_a_row_of_nan(ops, experts, scores):
+    """What the sort by expert and the corrected scores index with has to stay within the experts; the row's weights are NaN, the
+    other rows as without it."""
+    rng = np.random.default_rng(experts)
+    logits = rng.normal(size=(5, experts)).astype(np.float32)
+    correction = dev(rng.normal(size=experts)) if scores == "sigmoid" else None
+    plain_chosen, plain_weight = ops.moe_route(dev(logits), None, 3, scores=scores, correction=correction)
+    logits[2] = np.nan
+    chosen, weight = ops.moe_route(dev(logits), None, 3, scores=scores, correction=correction)
+    assert int(chosen.min()) >= 0 and int(chosen.max()) < experts
+    assert bool(weight[2].isnan().all())
+    others = [0, 1, 3, 4]
+    assert torch.equal(chosen[others], plain_chosen[others]) and torch.equal(weight[others], plain_weight[others])
+    begin, place_row, _ = ops.moe_arrange(chosen, experts)
+    assert int(begin[-1]) == 15 and sorted(place_row.tolist()) == sorted([0, 1, 2, 3, 4] * 3)
+
+
 def test_moe_arrange_keeps_an_experts_pairs_in_their_order(ops):
     rng = np.random.default_rng(5)
     for rows, experts, top in ((1, 4, 2), (37, 5, 3), (700, 12, 4), (3000, 130, 2)):
