@@ -6,7 +6,8 @@
 // walked K in order.
 //
 //  * K is cut into sixteen parts. For a few tiles a workgroup has sixteen waves, a part each; otherwise four, which
-//    walk four parts in turn. Each wave computes the whole tile over its parts; the partial tiles meet in LDS. A
+//    walk four parts in turn. (Below 256 k a part is at most a group of 16: the four waves then take groups in turn, as the first of
+//    four would otherwise have most of them.) Each wave computes the whole tile over its parts; the partial tiles meet in LDS. A
 //    tile of 64 x 64 reads 8 KB a wave for 2,048 cycles of matrix work: L2 carries that easily.
 //  * Operands go straight into LDS (global_load_lds_dwordx4), each wave's into a ring of its own, a few groups of 16 k
 //    ahead, and from there into registers one group ahead: nothing is shared between waves before the end, so there
@@ -51,7 +52,7 @@ __device__ __forceinline__ void multiply_group(const Operands<TM, TN>& f, f32x4 
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int n = 0; n < TN; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[i][j], f.w[n][j], acc[i][n], 0, 0, 0);
+            for (int n = 0; n < TN; ++n) acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[n][j], f.a[i][j], acc[i][n], 0, 0, 0);
 }
 
 // groups of a wave in LDS or on their way there
@@ -65,15 +66,13 @@ struct Ring {
 // SwiGLU: w holds N gate rows, then N up rows; column tiles alternate between 16 gate rows and the up rows of the same
 // features, so that one thread meets both at the end.
 template <int TM, int TN, int WAVES, int MODE, typename TO>
-__global__ __launch_bounds__(WAVES * 64) void gemm_float32_kernel(const float* __restrict__ a, const float* __restrict__ w,
-                                                                  const float* __restrict__ bias, TO* __restrict__ out, int M, int N,
-                                                                  int K, int tiles_m, int tiles_n, int per_xcd) {
+__device__ __forceinline__ void gemm_float32_tile(const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias,
+                                                  TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int quads) {
     constexpr int ROWS = TM * 16, WIDE = TN * 16;                       // of a tile, in rows of a and of w
     constexpr int FEATURES = MODE == MF_SWIGLU ? WIDE / 2 : WIDE;       // outputs of a tile's row
     constexpr int LOADS = Ring<TM, TN, WAVES>::LOADS, STAGES = Ring<TM, TN, WAVES>::STAGES;
     constexpr bool FOLDS = WAVES < PARTS;                               // a wave walks several parts
     __shared__ __attribute__((aligned(1024))) unsigned char lds[WAVES * Ring<TM, TN, WAVES>::BYTES];
-    float(*partial)[ROWS][WIDE] = reinterpret_cast<float(*)[ROWS][WIDE]>(lds);     // [WAVES], behind the loop
     static_assert(sizeof(float) * WAVES * ROWS * WIDE <= sizeof(lds), "the partial tiles take the rings' place");
     // workgroups are dealt to the dies in turn: a die gets neighbouring tiles, all rows of a column of tiles in a row
     const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -100,13 +99,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_kernel(const float* _
         for (int n = 0; n < TN; ++n) acc[i][n] = total[i][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
     const int part = (K + PARTS * 16 - 1) / (PARTS * 16);               // groups of 16 k in a part
-    const int k_begin = wave * (PARTS / WAVES) * part * 16;
-    const int k_end = min(K, k_begin + (PARTS / WAVES) * part * 16);
-    const int groups = k_end > k_begin ? (k_end - k_begin + 15) / 16 : 0;
+    const bool in_turn = FOLDS && K < PARTS * 16;
+    const int k_step = in_turn ? WAVES * 16 : 16, k_begin = in_turn ? wave * 16 : wave * (PARTS / WAVES) * part * 16;
+    const int k_end = in_turn ? K : min(K, k_begin + (PARTS / WAVES) * part * 16);
+    const int groups = k_end > k_begin ? (k_end - k_begin + k_step - 1) / k_step : 0;
     unsigned char* ring = lds + wave * Ring<TM, TN, WAVES>::BYTES;
     auto request = [&](int group) {
         unsigned char* stage = ring + group % STAGES * (LOADS * 1024);
-        const int k = min(k_begin + group * 16 + ask_piece * 4, K - 4);     // pieces past the end of K are set to zero below
+        const int k = min(k_begin + group * k_step + ask_piece * 4, K - 4);     // pieces past the end of K are set to zero below
 #pragma unroll
         for (int n = 0; n < TN; ++n)
             __builtin_amdgcn_global_load_lds(w_row[n] + k, reinterpret_cast<uint32_t*>(stage + n * 1024), 16, 0, 0);
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_kernel(const float* _
             if (g + 1 < groups) {
                 wait_for_all_but(min(groups, g + 1 + STAGES) - 2 - g);
                 read(next, g + 1);
-            } else if (k_begin + g * 16 + piece * 4 >= K) {             // K is no multiple of 16
+            } else if (k_begin + g * k_step + piece * 4 >= K) {         // K is no multiple of 16
 #pragma unroll
                 for (int n = 0; n < TN; ++n) now.w[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -197,45 +197,97 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_float32_kernel(const float* _
     __syncthreads();                                                    // every wave has left its ring
     fw_mfma_drain();
 
-    // lane (column l % 16) holds rows 4 * (l / 16) + r of each 16 x 16 product
+    // Lane (row l % 16 of a) holds features 4 * (l / 16) + r of each 16 x 16 product. A row's runs of four features lie permuted,
+    // run q in place q ^ r (the low bits), so that sixteen rows' runs are written to all banks.
+    constexpr int RUNS = WIDE / 4, OUT_RUNS = FEATURES / 4, ITEMS = ROWS * OUT_RUNS, THREADS = WAVES * 64;
+    constexpr int PER_THREAD = (ITEMS + THREADS - 1) / THREADS;         // runs of four outputs
+    f32x4* partial = reinterpret_cast<f32x4*>(lds);                     // [WAVES][ROWS][RUNS]
+    auto place_of = [&](int r, int run) { return r * RUNS + (run ^ (r & (RUNS - 1))); };
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int n = 0; n < TN; ++n)
+            partial[wave * ROWS * RUNS + place_of(i * 16 + row, n * 4 + piece)] = FOLDS ? total[i][n] + acc[i][n] : acc[i][n];
+    f32x4 old[PER_THREAD];
+    if constexpr (MODE == MF_ACCUMULATE) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                partial[wave][i * 16 + piece * 4 + r][n * 16 + row] = FOLDS ? total[i][n][r] + acc[i][n][r] : acc[i][n][r];
+        for (int u = 0; u < PER_THREAD; ++u) {
+            const int item = tid + u * THREADS, m = m0 + item / OUT_RUNS, n = n0 + item % OUT_RUNS * 4;
+            if (quads && item < ITEMS && m < M && n < N) old[u] = *reinterpret_cast<const f32x4*>(out + (size_t)m * N + n);
+        }
+    }
     fw_lds_barrier();
 
-    auto sum = [&](int r, int c) {
-        float quarter[4];
+    auto sum = [&](int r, int run) {
+        const f32x4* from = partial + place_of(r, run);
+        f32x4 quarter[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            quarter[q] = partial[q * (WAVES / 4)][r][c];
+            quarter[q] = from[q * (WAVES / 4) * ROWS * RUNS];
 #pragma unroll
-            for (int p = 1; p < WAVES / 4; ++p) quarter[q] += partial[q * (WAVES / 4) + p][r][c];
+            for (int p = 1; p < WAVES / 4; ++p) quarter[q] += from[(q * (WAVES / 4) + p) * ROWS * RUNS];
         }
         return ((quarter[0] + quarter[1]) + quarter[2]) + quarter[3];
     };
-    for (int e = tid; e < ROWS * FEATURES; e += WAVES * 64) {
-        const int r = e / FEATURES, f = e % FEATURES;
+#pragma unroll
+    for (int u = 0; u < PER_THREAD; ++u) {
+        const int item = tid + u * THREADS, r = item / OUT_RUNS, f = item % OUT_RUNS * 4;
         const int m = m0 + r, n = n0 + f;
-        if (m >= M || n >= N) continue;
-        const size_t at = (size_t)m * N + n;
-        if (MODE == MF_SWIGLU) {
-            const int column = (f >> 4) * 32 + (f & 15);
-            const float g = sum(r, column), u = sum(r, column + 16);
-            store_from_float(out, at, g * sigmoid_float32(g) * u);
+        if (item >= ITEMS || m >= M || n >= N) continue;
+        f32x4 v;
+        if constexpr (MODE == MF_SWIGLU) {
+            const int run = ((f >> 4) * 32 + (f & 15)) / 4;
+            const f32x4 g = sum(r, run), up = sum(r, run + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = g[e] * sigmoid_float32(g[e]) * up[e];
         } else {
-            float value = sum(r, f);
-            if (bias) value += bias[n];
-            if (MODE == MF_ACCUMULATE) value += load_as_float(out, at);
-            store_from_float(out, at, value);
+            v = sum(r, f / 4);
+            if (bias)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += n + e < N ? bias[n + e] : 0.0f;
+        }
+        TO* to = out + (size_t)m * N + n;
+        if (quads) {
+            if constexpr (MODE == MF_ACCUMULATE) v += old[u];
+            if constexpr (sizeof(TO) == 4) {
+                *reinterpret_cast<f32x4*>(to) = v;
+            } else {
+                uint2 packed;
+                packed.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
+                packed.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
+                *reinterpret_cast<uint2*>(to) = packed;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (n + e >= N) continue;
+                if constexpr (MODE == MF_ACCUMULATE) v[e] += load_as_float(to, e);
+                store_from_float(to, e, v[e]);
+            }
         }
     }
 }
 
+template <int TM, int TN, int WAVES, int MODE, typename TO>
+__global__ __launch_bounds__(WAVES * 64) void gemm_float32_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                                  const float* __restrict__ bias, TO* __restrict__ out, int M, int N,
+                                                                  int K, int tiles_m, int tiles_n, int per_xcd, int quads) {
+    gemm_float32_tile<TM, TN, WAVES, MODE, TO>(a, w, bias, out, M, N, K, tiles_m, tiles_n, per_xcd, quads);
+}
+// The same in 256 registers, two workgroups on a compute unit (a tile of 64 x 64 otherwise takes 356): for a short K, where a tile
+// is mostly its start and its end. 8,192 outputs, K 64, 4,096 rows: 144 -> 83 us, 2,048 outputs 38 -> 24; from K 512 on two
+// tiles beside each other get in each other's way (1,024 outputs, K 4,608, 2,048 rows: 186 -> 220; K 1,024, 2,048 outputs, 1,000
+// rows: 50 -> 58).
+template <int TM, int TN, int WAVES, int MODE, typename TO>
+__global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2))) void gemm_float32_short_kernel(
+    const float* __restrict__ a, const float* __restrict__ w, const float* __restrict__ bias, TO* __restrict__ out, int M, int N, int K,
+    int tiles_m, int tiles_n, int per_xcd, int quads) {
+    gemm_float32_tile<TM, TN, WAVES, MODE, TO>(a, w, bias, out, M, N, K, tiles_m, tiles_n, per_xcd, quads);
+}
+
 namespace {
+
+constexpr int SHORT_K = 512;        // below it the form for a short K
 
 // The tile that loads the busiest compute unit least. A wave's group of 16 k costs a compute unit the matrix time of
 // TM x TN products (128 cycles each on its SIMD) or the reading of TM + TN operands by four waves (about as many cycles
@@ -263,7 +315,14 @@ template <int TM, int TN, int WAVES, int MODE, typename TO>
 void run(const float* a, const float* w, const float* bias, void* out, int M, int N, int K, hipStream_t stream) {
     const int tiles_m = fw_ceil_div(M, TM * 16), tiles_n = fw_ceil_div(N, MODE == MF_SWIGLU ? TN * 8 : TN * 16);
     const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n, 8);
-    gemm_float32_kernel<TM, TN, WAVES, MODE, TO><<<per_xcd * 8, WAVES * 64, 0, stream>>>(a, w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd);
+    const int quads = N % 4 == 0 && (uintptr_t)out % 16 == 0;
+    if constexpr (TM * TN == 16) {
+        if (K < SHORT_K) {
+            gemm_float32_short_kernel<TM, TN, WAVES, MODE, TO><<<per_xcd * 8, WAVES * 64, 0, stream>>>(a, w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, quads);
+            return;
+        }
+    }
+    gemm_float32_kernel<TM, TN, WAVES, MODE, TO><<<per_xcd * 8, WAVES * 64, 0, stream>>>(a, w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, quads);
 }
 
 template <int MODE, typename TO>

@@ -69,6 +69,18 @@ def test_a_row_does_not_depend_on_the_rows_beside_it(ops):
         assert torch.equal(ops.gemm_swiglu(a[5:6].contiguous(), w)[0], gated[5])
 
 
+@pytest.mark.parametrize("K", [16, 64, 128, 192, 260, 272, 300, 512, 520, 4100])
+def test_every_part_of_k_is_walked_once(ops, K):
+    """Parts of one group and of several, the last of them cut short or empty, for waves that walk one part and waves that walk
+    four: the same sums to the bit."""
+    a, w = draw(70, K), draw(150, K, seed=1)
+    A, W = a.to(DEV), w.to(DEV)
+    whole = ops.gemm(A, W)
+    assert ((whole.cpu().double() - a.double() @ w.double().T).abs() <= bound(a, w)).all()
+    for first, last in ((0, 1), (3, 20), (30, 70)):
+        assert torch.equal(ops.gemm(A[first:last].contiguous(), W), whole[first:last])
+
+
 def test_what_its_loads_cannot_take_goes_to_the_plain_tiles(ops):
     a, w = draw(5, 66), draw(40, 66, seed=1)                       # K no multiple of 4
     exact = a.double() @ w.double().T
