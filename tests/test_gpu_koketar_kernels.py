@@ -154,6 +154,27 @@ def test_recurrence_spread_over_more_workgroups(heads, dim, vdim):
             np.testing.assert_allclose(after[slot, head], S, rtol=0, atol=2e-5 * max(1.0, np.abs(S).max()))
 
 
+@pytest.mark.parametrize("spread", [False, True])
+@pytest.mark.parametrize("dim", [64, 66, 128, 200, 256])
+def test_recurrence_takes_a_state_that_lies_anywhere(dim, spread):
+    """States aligned to 16 bytes travel four floats at a time, others one by one: the same bits."""
+    from flyweight_amd.kernels import ops
+    heads, vdim, lengths = 2, 20, [1, 1, 18]
+    rows = sum(lengths)
+    generator = torch.Generator().manual_seed(dim)
+    records = (torch.randn(rows, heads, ops.delta_record_floats(dim, vdim), generator=generator) * 0.05).to("cuda:0")
+    start = torch.randn(3, heads, vdim, dim, generator=generator).to("cuda:0")
+    row0, slots = ints(np.concatenate([[0], np.cumsum(lengths)])), ints([2, 0, 1])
+    aligned = start.clone()
+    flat = torch.full((start.numel() + 5,), 7.0, device="cuda:0")
+    shifted = flat[1:1 + start.numel()].view_as(start)
+    shifted.copy_(start)
+    out = ops.gated_delta_rule(records, aligned, row0, slots, 3, heads, dim, vdim, spread=spread)
+    assert torch.equal(ops.gated_delta_rule(records, shifted, row0, slots, 3, heads, dim, vdim, spread=spread), out)
+    assert torch.equal(shifted, aligned) and not torch.equal(aligned, start)
+    assert float(flat[0]) == 7.0 and bool((flat[1 + start.numel():] == 7.0).all())
+
+
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_gated_head_norm(out_dtype):
     from flyweight_amd.kernels import ops
