@@ -207,9 +207,9 @@ __device__ __forceinline__ float delta_lanes_sum(float x) {
 // a token's record and in LDS is worked out once).
 // The walk is bound by how fast one wave a SIMD issues its chain (about 7 clocks an instruction, twice what several waves get):
 // a prompt's heads of more than 64 key channels take 32 lanes a column, half the arithmetic a wave on twice the
-// workgroups. 16 heads of 128 channels, 694 rows in the mean: 205 us with operands read one float at a time, 172 read four at a
+// workgroups, while those have a compute unit each (the caller says: GatedDeltaRule.spread). 16 heads of 128 channels, 694 rows in the mean: 205 us with operands read one float at a time, 172 read four at a
 // time, 146 on 32 lanes. (Two tokens at a time, their sums travelling together, gained nothing more: 147; nor did chunks of 32
-// tokens.) Steps of single rows lose on 32 lanes (8 rows 8.4 against 11.5 us).
+// tokens.) Beyond that 32 lanes lose: four prompts of 694 rows 222 against 320 us, 8 single rows 8.9 against 12.1.
 template <int RPT, int DELTA_LANES>
 __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     const float* __restrict__ records, float* __restrict__ state, float* __restrict__ out,

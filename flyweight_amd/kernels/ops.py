@@ -19,6 +19,7 @@ from . import build as _build
 # (the last two: a storing product leaves gelu of its float32 sums; a gated product gelu_tanh(gate) * up)
 F32, BF16, BF16_GELU, BF16_GEGLU = 0, 1, 2, 3
 PAGE_SIZE = 64          # tokens per cache page: the width of a wavefront
+COMPUTE_UNITS = 256     # of the chip
 MAX_HEAD_DIM = 256          # of the matrix-core attention kernels
 MAX_PLAIN_HEAD_DIM = 1024   # of the plain attention kernels, which serve what the others do not take
 

@@ -147,6 +147,18 @@ class GatedDeltaRule(Mixer):
             self._no_conv_state = torch.zeros((cache["state"].state.shape[0], self.channels, 0), dtype=torch.float32, device=self.device)
         return self._no_conv_state
 
+    def spread(self, row0) -> bool:
+        """Whether a step's columns of state are shared out over 32 lanes (``row0``: the first row of each segment, and the end).
+        A walk is bound by how fast one wave issues its chain of instructions, so half the arithmetic a wave pays as long as its
+        workgroups, of 8 value channels, have a compute unit each. 16 heads of 128 channels, prompts of 694 rows: one
+        173 -> 150 us, but two 177 -> 196 and four 222 -> 320; 4 heads: four prompts 173 -> 148, eight of 300 rows
+        82 -> 91. Segments that are short beside the longest leave early and do not count."""
+        if self.dtype != torch.bfloat16 or self.dim <= 64:
+            return False        # (a float32 run gives the same bits however a sequence is cut into steps: its prompts walk as its single rows do)
+        longest = max(b - a for a, b in zip(row0, row0[1:]))
+        abreast = int((row0[-1] - row0[0]) / longest + 0.75)
+        return longest > 1 and abreast * self.heads * -(-self.vdim // 8) <= ops.COMPUTE_UNITS
+
     def heads_output(self, h, ctx, cache) -> torch.Tensor:
         """The heads' normed and gated read-outs [rows, heads * vdim] in the activation dtype; the
         request's state moves on by the step's rows."""
@@ -164,9 +176,8 @@ class GatedDeltaRule(Mixer):
         records = ops.delta_prepare(proj, self.beta_col, a, self.taps, self._conv_state(cache), self.A_log, self.dt_bias,
                                     ctx.row_seg, ctx.seg_row0, ctx.seg_slot, ctx.num_segments, self.heads, self.kv_heads,
                                     self.dim, self.vdim, decay_per_head=per_head)
-        # (a float32 run gives the same bits however a sequence is cut into steps: its prompts walk as its single rows do)
         o = ops.gated_delta_rule(records, cache["state"].state, ctx.seg_row0, ctx.seg_slot, ctx.num_segments,
-                                 self.heads, self.dim, self.vdim, spread=self.dtype == torch.bfloat16 and not ctx.all_decode)
+                                 self.heads, self.dim, self.vdim, spread=not ctx.all_decode and self.spread(ctx.host_seg_row0))
         return ops.gated_head_norm(o, gate, self.norm_weight, self.heads, self.vdim, self.eps, self.dtype,
                                    gate_silu=self.gate == "silu")
 
