@@ -223,9 +223,11 @@ __global__ __launch_bounds__(256) void wkv_recurrence_kernel(
     put(0);
     __syncthreads();
     // The state and the bonus have arrived here, for the compiler too: their first use being inside the loop, every token waited
-    // for all loads in flight, the next chunk's among them.
+    // for all loads in flight, the next chunk's among them. (Not with sixteen channels a lane: 1,024 rows 719 us so, 683 without.)
+    if constexpr (RPT < 16) {
 #pragma unroll
-    for (int t = 0; t < RPT; ++t) asm volatile("" : "+v"(S[t]), "+v"(bonus[t]));
+        for (int t = 0; t < RPT; ++t) asm volatile("" : "+v"(S[t]), "+v"(bonus[t]));
+    }
     for (int base = 0; base < count; base += WKV_CHUNK) {
         const int tokens = count - base < WKV_CHUNK ? count - base : WKV_CHUNK;
         const bool more = base + WKV_CHUNK < count;

@@ -65,13 +65,27 @@ class Wkv(RecurrenceChunks, Mixer):
         # a float32 run gives the same bits however a sequence is cut into steps: its rows are walked in order
         return super().step_arrays(batch) if self.dtype == torch.bfloat16 else {}
 
+    # What each form takes, by the key channels that the kernels hold (their instantiations), in us: the walk in order a row of the
+    # longest segment; the chunks beyond what the walk in order takes at its start: at least, with few workgroups, else a start and
+    # one per so many rows of a workgroup's 16 value channels of one head. Measured, in order / in chunks: 32 heads of 64, one
+    # segment of 2,048 rows 403 / 136, four of 512 119 / 123, two of 129 32.8 / 33.7; 32 heads of 16, four of 129 22.6 / 25.6;
+    # 16 heads of 128, one of 129 47.8 / 50.8, two of 256 85 / 75; of 256, one of 256 180 / 224, of 1,024 683 / 658; 4 heads of
+    # 256, two of 129 99 / 144, two of 256 178 / 147.
+    _COSTS = {16: (0.14, 17.0, 15.0, 2700.0), 32: (0.147, 18.5, 10.0, 2800.0), 64: (0.197, 21.0, 10.0, 2250.0),
+              128: (0.31, 37.0, 23.0, 1400.0), 256: (0.67, 107.0, 69.0, 450.0)}
+
+    def cuts(self, row0) -> bool:
+        """Whether a step's long segments are walked in chunks (``row0``: the first row of each segment, and the end). The short
+        ones beside them are then walked in order by a launch of its own."""
+        row, least, start, rate = self._COSTS[next(held for held in self._COSTS if self.dim <= held)]
+        lengths = [b - a for a, b in zip(row0, row0[1:])]
+        rows = sum(-(-n // self.CHUNK_ROWS) for n in lengths if n > self.LONG_ROWS) * self.CHUNK_ROWS
+        short = max([n for n in lengths if n <= self.LONG_ROWS], default=0)
+        in_chunks = max(least, start + rows * self.heads * -(-self.dim // 16) / rate) + (4.0 + row * short if short else 0.0)
+        return rows > 0 and in_chunks < row * max(lengths)
+
     def chunk_arguments(self, ctx) -> dict:
-        """The walk in order takes 0.20 to 0.24 us a row of the longest segment, however many there are; the chunks about 20 us and, the chip
-        being full, 1 us for 2,200 rows of a workgroup's 16 value channels of one head. (32 heads of 64 channels: one segment
-        of 2,048 rows 401 us in order, 147 in chunks; four of 512 rows 117 and 127.)"""
-        lengths = [b - a for a, b in zip(ctx.host_seg_row0, ctx.host_seg_row0[1:])]
-        work = sum(n for n in lengths if n > self.LONG_ROWS) * self.heads * -(-self.dim // 16)
-        return super().chunk_arguments(ctx) if 20.0 + work / 2200.0 < 0.22 * max(lengths) else {}
+        return super().chunk_arguments(ctx) if self.cuts(ctx.host_seg_row0) else {}
 
     def mixing_flops(self, rows: int, keys_before: int = 0) -> int:
         """Flops of the recurrence itself: per token and head a read and a write of the state, a multiply and an add each

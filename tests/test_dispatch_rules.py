@@ -30,3 +30,16 @@ def _delta_rule(heads, dim, vdim, dtype=torch.bfloat16):
 def test_delta_rule_spreads_its_columns_while_every_workgroup_has_a_compute_unit(heads, dim, vdim, lengths, spread):
     assert _delta_rule(heads, dim, vdim).spread(_row0(lengths)) == spread
     assert not _delta_rule(heads, dim, vdim, torch.float32).spread(_row0(lengths))
+
+
+@pytest.mark.parametrize("heads,dim,lengths,cuts", [
+    (32, 64, [2048], True), (32, 64, [512] * 4, False), (32, 64, [129] * 2, False), (32, 64, [2048] * 2, True), (32, 64, [128], False),
+    (32, 16, [129] * 4, False), (32, 16, [512] * 4, True), (32, 32, [129] * 4, False), (32, 32, [256] * 4, True),
+    (16, 128, [129], False), (16, 128, [256] * 2, True), (16, 128, [256] * 4, False),
+    (16, 256, [256], False), (16, 256, [1024], True), (4, 256, [129] * 2, False), (4, 256, [256] * 2, True), (4, 256, [256] * 4, False),
+    (32, 64, [1] * 24, False), (32, 64, [1] * 24 + [300], True), (8, 64, [128, 200], False)])   # short segments beside a long one
+def test_wkv_cuts_long_segments_where_the_chunks_are_faster(heads, dim, lengths, cuts):
+    from flyweight_amd.config.spec import PartSpec
+    from flyweight_amd.parts.wkv import Wkv
+    part = Wkv(PartSpec("wkv", {"hidden_size": 64, "num_heads": heads, "head_dim": dim, "decay_rank": 8, "norm_eps": 1e-5}))
+    assert part.cuts(_row0(lengths)) == cuts
