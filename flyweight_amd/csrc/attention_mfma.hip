@@ -908,8 +908,7 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
     if (rows == 0 || tiles == 0) return 0;
     const int group = num_heads / num_kv_heads;
     if (halves) heads_together = 2;
-    if (heads_together == 0)
-        heads_together = most_together == 4 && group >= 4 && (long long)tiles * num_kv_heads * ((group + 3) / 4) >= 1024 ? 4 : 1;
+    if (heads_together == 0) heads_together = 1;
     const long long blocks = (long long)tiles * num_kv_heads * ((group + heads_together - 1) / heads_together);
     FW_REQUIRE(blocks < (1ll << 31), "attention_prefill: too many tiles and heads");
     dim3 grid((unsigned)blocks);

@@ -1003,8 +1003,8 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
                       heads_together: int = 0, out: Optional[torch.Tensor] = None, v_dim: Optional[int] = None,
                       chunk: int = 0, softcap: float = 0.0, keep_first: int = 0, sinks: Optional[torch.Tensor] = None,
                       slopes: Optional[torch.Tensor] = None, halves: bool = False) -> torch.Tensor:
-    """``heads_together``: query heads of a kv group per workgroup (1, or 4 up to head_dim 64), 0: the
-    kernel's choice. ``halves`` (up to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. Only the rows of the given tiles are written (into ``out`` if given)."""
+    """``heads_together``: query heads of a kv group per workgroup (0 and 1: one; 4 up to head_dim 64). ``halves`` (up
+    to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. Only the rows of the given tiles are written (into ``out`` if given)."""
     _dev(q, k_pages, v_pages, block_table, tile_seg, tile_row0, seg_row0, row_pos)
     _want(q, torch.bfloat16, "q")
     rows = q.shape[0]
@@ -1133,6 +1133,28 @@ def attention_is_tiled(head_dim: int) -> bool:
     return head_dim % 16 == 0 and 16 <= head_dim <= MAX_HEAD_DIM
 
 
+def prompt_halves(tiles: int, num_heads: int, num_kv_heads: int, widest: int, keys: int) -> bool:
+    """Whether a prompt's attention takes the form of two heads a workgroup (fw_attention_prefill), whose two halves share the
+    pages out: ``tiles`` tiles of rows, of which the rows see up to ``keys`` keys, heads of up to ``widest`` channels.
+    Its workgroups have a compute unit each, those of the form of one head share one by two to four. So it pays where
+    its rounds over the chip are full, and where rows see enough keys for the merge at the end to be little. us, one head /
+    halves, heads of 64: 32 heads in 8 groups, 2,048 rows (2 rounds) behind 0 / 2,048 / 30,720 keys 44 / 45, 133 / 102, 1,084 /
+    870; 1,500 rows (1.5 rounds) behind 3,072 97 / 115; 1,700 (1.7) behind 2,048 123 / 95; 777 (0.8) behind 0 / 512 18.0 / 19.1,
+    27.2 / 26.2; 6,000 (5.9) behind 4,096 687 / 624, 3,500 (3.4) 329 / 336; 20 prompts of 300 (6.3) behind 1,300 188 / 202. 16
+    heads in 8 groups, 777 rows (0.4) behind 2,048 / 30,720 45.7 / 46.0, 453 / 430. With an odd number of heads a group one wave
+    in so many idles (24 in 8 groups, 2,048 rows behind 8,192 223 / 267), and heads of 32 channels leave LDS less to bound
+    (2,048 rows behind 8,192 188 / 213)."""
+    group = num_heads // num_kv_heads
+    if not 32 < widest <= 64 or group % 2:
+        return False
+    workgroups = tiles * num_kv_heads * (group // 2)
+    rounds = -(-workgroups // COMPUTE_UNITS)
+    if 2 * workgroups <= COMPUTE_UNITS:
+        return keys >= 16384
+    fill, least = ((0.5, 1280), (0.84, 1280), (0.95, 3072))[min(rounds, 3) - 1]
+    return workgroups >= fill * rounds * COMPUTE_UNITS and keys >= least
+
+
 def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, k_pages: torch.Tensor,
               v_pages: torch.Tensor, block_table: torch.Tensor, ctx, scale: float, window: int = 0,
               tile_seg: Optional[torch.Tensor] = None, tile_row0: Optional[torch.Tensor] = None,
@@ -1156,13 +1178,9 @@ def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
         if tile_seg is None or tile_row0 is None:
             raise KernelError("attention: the tiled kernel needs the step's query tiles")
         single = getattr(ctx, "decode_prefix", 0)       # leading segments of one row: rows and tiles 0 .. single - 1
-        # Where a row may see some thousand keys, two heads of a kv group per workgroup read a page's keys and values from LDS
-        # once for both, its two halves sharing the pages out so that as many waves are at work (2,048 rows, head_dim 64,
-        # against one head: 32 heads in 8 groups behind 0 / 2,048 / 30,720 keys 46.9 / 106 / 871 against 48.2 / 143 / 1,078 us,
-        # 16 heads 37.7 / 66 / 455 against 39.6 / 78 / 562; 777 rows from position 0 20.1 against 18.8). Four heads
-        # together, which a long context once took, lose to either (64 rows behind 8,000 keys 270 against 116 us).
-        keys = min([n for n in (window, chunk) if n] + [ctx.max_context])      # the most keys a row can see
-        halves = max(head_dim, v_dim) <= 64 and num_heads // num_kv_heads >= 2 and keys >= 3072
+        lengths = getattr(ctx, "new_lengths", None)     # what each segment sees in the end; the single rows' contexts are not the tiles'
+        keys = min([n for n in (window, chunk) if n] + [max(lengths[single:]) if lengths else ctx.max_context])
+        halves = prompt_halves(tile_seg.numel() - single, num_heads, num_kv_heads, max(head_dim, v_dim), keys)
         if single == 0:
             return attention_prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, tile_seg,
                                      tile_row0, ctx.seg_row0, ctx.row_pos, scale, window, halves=halves, v_dim=v_dim,

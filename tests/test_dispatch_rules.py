@@ -43,3 +43,32 @@ def test_wkv_cuts_long_segments_where_the_chunks_are_faster(heads, dim, lengths,
     from flyweight_amd.parts.wkv import Wkv
     part = Wkv(PartSpec("wkv", {"hidden_size": 64, "num_heads": heads, "head_dim": dim, "decay_rank": 8, "norm_eps": 1e-5}))
     assert part.cuts(_row0(lengths)) == cuts
+
+
+@pytest.mark.parametrize("rows,behind,heads,groups,widest,halves", [
+    (2048, 2048, 32, 8, 64, True), (2048, 30720, 16, 8, 64, True), (1500, 3072, 32, 8, 64, False), (1700, 2048, 32, 8, 64, True),
+    (1500, 3072, 16, 8, 64, True), (777, 0, 32, 8, 64, False), (777, 2048, 32, 8, 64, True), (777, 2048, 16, 8, 64, False),
+    (777, 30720, 16, 8, 64, True), (64, 3000, 32, 8, 64, False), (6000, 4096, 32, 8, 64, True), (3500, 4096, 32, 8, 64, False),
+    (2048, 8192, 24, 8, 64, False), (2048, 8192, 32, 8, 32, False), (2048, 8192, 32, 8, 48, True), (2048, 8192, 32, 8, 128, False),
+    (2048, 8192, 8, 8, 64, False)])
+def test_prompt_attention_shares_pages_between_halves_where_its_rounds_are_full(rows, behind, heads, groups, widest, halves):
+    from flyweight_amd.kernels import ops
+    assert ops.prompt_halves(-(-rows // 64), heads, groups, widest, rows + behind) == halves
+
+
+def test_decode_rows_do_not_choose_the_form_of_a_prompt_beside_them(monkeypatch):
+    """A new prompt of 777 rows beside a request that decodes behind 20,000 keys takes the form that it takes alone."""
+    from types import SimpleNamespace
+
+    from flyweight_amd.kernels import ops
+    taken = []
+    monkeypatch.setattr(ops, "attention_prefill", lambda *a, halves, **k: taken.append(halves))
+    monkeypatch.setattr(ops, "attention_decode", lambda *a, **k: None)
+    for decoding, behind, halves in (([], 0, False), ([20000], 0, False), ([20000], 4000, True), ([], 4000, True), ([30], 4000, True)):
+        single = len(decoding)
+        tiles = torch.zeros(single + 13, dtype=torch.int32)
+        rows = single + 777
+        ctx = SimpleNamespace(all_decode=False, decode_prefix=single, max_context=max(decoding + [behind + 777]),
+                              new_lengths=decoding + [behind + 777], row_seg=None, row_pos=None, seg_row0=None)
+        ops.attention(torch.zeros(rows, 32 * 64, dtype=torch.bfloat16), 32, 8, 64, None, None, None, ctx, 0.125, 0, tiles, tiles)
+        assert taken.pop() == halves
