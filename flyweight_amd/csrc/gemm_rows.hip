@@ -12,7 +12,10 @@
 //    for its own loads alone, counted. Eight neighbouring lanes ask for the 128 bytes of a row that are a line of L2: asked
 //    for 64 at a time, with every compute unit at it, rows come in at 42-66 KB/us a compute unit instead of 85-120 (and at
 //    37 in the order of the matrix operands, sixteen rows at neighbouring lanes).
-//  * The partial tiles meet in LDS and are added in the order of the waves: the order of a sum depends on K alone.
+//  * The partial tiles meet in LDS and are added in the order of the waves: the order of a sum depends on K and on the number of
+//    waves, which the tile decides (M, N and the mode choose it), not on the other rows or on timing. (Eight parts of K whatever
+//    the tile, the waves of a tile of four walking two each in sums of their own, would take M out of it; the tiles of four waves
+//    were 3 to 8 % slower so, and four waves for the small tiles 10 to 25 %.)
 //
 // Measured against the product that cut K over workgroups, which met through a workspace and a ticket (every weight from
 // memory; 64 rows, us): adding 2,048 features over K 8,192 / 2,048 17.7 -> 15.8 / 11.7 -> 7.0, 1,024 over 4,608 / 1,024 13.6 -> 8.4 /

@@ -56,6 +56,26 @@ def test_product_of_a_few_rows(ops, M, N, K):
         assert torch.equal(flat[1:].view(M, N), into)
 
 
+@pytest.mark.parametrize("N,K", [(3072, 1024), (1024, 968), (2048, 96)])
+def test_a_row_among_other_rows(ops, N, K):
+    """Among as many rows a row's result depends neither on the others nor on its place; the number of rows chooses the tile, and with it
+    the number of waves that K is dealt to (at 3,072 features eight up to 32 rows, four beyond), so across numbers of rows it is the
+    same up to the order of the sum."""
+    a, w = draw(64, K), draw(N, K, seed=1)
+    A, W = a.to(DEV), w.to(DEV)
+    limit = bound(a, w)
+    found = {}
+    for M in (12, 17, 32, 33, 64):
+        found[M] = ops.gemm(A[:M].contiguous(), W, out_dtype=torch.float32)
+        turned = torch.roll(A[:M], 5, 0).contiguous()
+        turned[0] = 3.0
+        again = ops.gemm(turned, W, out_dtype=torch.float32)
+        assert torch.equal(again[6:], found[M].roll(5, 0)[6:]), M
+        assert torch.equal(ops.gemm(A[:M].contiguous(), W, out_dtype=torch.float32), found[M])
+    for M in found:
+        assert ((found[M] - found[64][:M]).abs().cpu().double() <= 2 * limit[:M]).all()
+
+
 @pytest.mark.parametrize("M,F,K", [(1, 16, 64), (17, 77, 520), (40, 130, 96), (64, 4608, 1024), (190, 1000, 224)])
 def test_gated_product_of_a_few_rows(ops, M, F, K):
     a, w = draw(M, K, scale=K ** -0.5), draw(2 * F, K, seed=1)
