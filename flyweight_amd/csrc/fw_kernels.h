@@ -70,10 +70,18 @@ int fw_gemm_mfma_split_plan(int mode, int M, int N, int K, size_t* workspace_byt
 int fw_gemm_mfma_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                        int M, int N, int K, void* workspace, size_t workspace_bytes, int* counters,
                        int counters_len, void* stream);
-// The product for 1..64 rows and a very wide output: mode 0 alone; takes prepared activations as a (squares [squares_rows][16
-// for M <= 16, else 64], eps).
-int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int M, int N, int K,
-                   const float* squares, int squares_rows, float eps, void* stream);
+// The same product for 1..64 rows with K split over workgroups, for the shapes that fw_gemm_rows serves worse.
+// fw_gemm_medium_plan says what a shape needs: bytes of workspace (0: none) and int32 counters (0: none) that are zero before
+// the first call; the kernel leaves them zero. Calls that overlap on one device need their own of both.
+// The accumulating product can leave what the norm after it needs, as fw_gemm_decode does
+// (next_activations [M][N] bfloat16, next_squares [squares_rows][16 for M <= 16, else 64]), and
+// any mode takes such prepared activations as a, with squares / squares_rows / eps.
+int fw_gemm_medium_plan(int M, int N, int K, int mode, size_t* workspace_bytes, int* counters, int* squares_rows);
+int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode,
+                   int M, int N, int K, void* workspace, size_t workspace_bytes, int* counters,
+                   int counters_len, const float* next_norm_weight, int next_one_centered,
+                   void* next_activations, float* next_squares, const float* squares, int squares_rows,
+                   float eps, float glu_limit, float glu_alpha, float glu_shift, void* stream);
 // The product for 1..4096 rows in modes 0, 1 and 2 (the gated unit: glu_limit and its like as for fw_gemm_decode) with K split over
 // a workgroup's waves alone: no workspace, no counters. Up to 64 rows the accumulating product can leave what the norm after
 // it needs, as fw_gemm_decode does (next_activations [M][N] bfloat16, next_squares [fw_gemm_rows_square_tiles(M, N)][16 for M <= 16,
@@ -95,7 +103,7 @@ int fw_gemm_rows_round_fits(int mode, int M, int N);
 // [M][N] = x_new * w_next and next_squares [fw_gemm_decode_accumulate_tiles(N)][16], per-tile sums
 // of x_new^2 of every row. A later call takes them with prologue 2 (a = those activations,
 // squares/squares_tiles = those sums, eps) and applies the row's scale in its epilogue.
-// glu_limit / glu_alpha / glu_shift (here and in fw_gemm_rows, epilogue 2 only): with a limit of 0 the
+// glu_limit / glu_alpha / glu_shift (here, in fw_gemm_medium and in fw_gemm_rows, epilogue 2 only): with a limit of 0 the
 // gated unit is SwiGLU, silu(gate) * up; with a negative one gelu_tanh(gate) * up; with a positive one its halves are clamped, g = min(gate,
 // limit), u = clamp(up, -limit, limit), and out = g * sigmoid(alpha * g) * (u + shift).
 // w_tiled (here, in fw_gemm_medium and in fw_gemm_rows): w is not row-major [rows][K] but lies in operand tiles,

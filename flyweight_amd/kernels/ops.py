@@ -586,7 +586,6 @@ MEDIUM_MAX_ROWS = 64
 # 256 rows 14.4 against 18.1, 6,144 at 128 rows 15.3 against 18.9. With two rounds it loses (6,144 features at 192 rows 25.9 against
 # 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27).
 ROWS_MAX = 1024
-WIDE_STORE = 24576        # outputs from which a storing product of up to 64 rows takes the tiles of a vocabulary (65,536 at 64 rows: 62 against 70 us)
 BIG_TILES_MIN = 192      # 256 x 256 tiles from which the large-tile prompt product is used (256 compute units)
 DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)
 DEEP_MIN_K_STORE = 4096   # storing: no old values travel during the exchange at a tile's end, a short K gains nothing
@@ -708,6 +707,41 @@ def _tiled_for(w: torch.Tensor, w_tiled: Optional[torch.Tensor]) -> Optional[tor
     return w_tiled
 
 
+# K from which a product that stores or adds up to 1,024 / 2,048 / 4,095 / 4,096 features splits it over workgroups, by the most rows
+_LONG_K = ((16, (6144, 6144, 6144, 12288)), (32, (10240, 10240, 6144, 10240)), (48, (16384, 16384, 12288, 1 << 30)),
+           (64, (16384, 10240, 6144, 1 << 30)))
+
+
+def medium_splits_k(mode: int, M: int, N: int, K: int) -> bool:
+    """Whether a product of up to 64 rows goes to the kernel that splits K over workgroups (fw_gemm_medium, several workgroups on a
+    compute unit) and not to the one whose waves do (fw_gemm_rows, tiles of up to 64 x 64, one workgroup on a compute unit). The
+    latter loses, every weight from memory, us (splitting / waves):
+
+    * with more than one round of its largest tiles: storing 20,480 features over K 2,048 at 17 / 64 rows 19.1 / 24.0, 29.3 / 30.8,
+      65,536 at 64 rows 62 / 70, gated 10,752 over 2,048 22.5 / 24.6, 28.0 / 31.3 (not over K 2,056, in row-major order: 32.7 / 30.9);
+    * with a short K on wide tiles: gated 4,608 over 1,024 at 32 rows 8.5 / 8.9, over 1,536 10.5 / 11.1, storing 16,384 over 1,024 at 17
+      rows 9.4 / 10.8, 8,192 over 2,048 8.9 / 9.4 (10,240 over 2,048 leave the former's second round empty: 13.6 / 12.4);
+    * with a long K and few tiles: adding 2,048 features over K 8,192 at 16 rows 12.0 / 13.0, over 12,288 13.1 / 18.3, at 32 rows
+      15.2 / 18.2, at 64 21.3 / 23.3, over 10,240 at 64 19.5 / 20.4 but at 48 18.6 / 17.6; 1,024 over 10,240 at 32 rows 13.0 /
+      14.6, at 64 17.3 / 14.1; 2,560, whose tiles of 16 leave a third of the chip without work, over 6,144 at 32 rows 12.0 /
+      13.9; where the slices of K are more than a round they lose again (3,072 over 8,192 at 32 rows 20.3 / 17.2)."""
+    if mode == 2:
+        return K % 32 == 0 and (N > 8192 or (N > 4096 and M > DECODE_MAX_ROWS and K <= (1536 if M <= 48 else 1024)))
+    if N > 16384:
+        return True
+    if N > 4096:
+        if M <= DECODE_MAX_ROWS:
+            return False
+        if M <= 32:
+            return K <= 1024 or (K <= 2048 and not 8192 < N <= 12288)
+        return N > 8192 and K <= (1024 if N > 12288 and M <= 48 else 512)
+    tiles = -(-N // 32)
+    if tiles * ((COMPUTE_UNITS + tiles // 2) // tiles) > COMPUTE_UNITS or (N <= 512 and M > DECODE_MAX_ROWS):
+        return False
+    least = next(by_features for rows, by_features in _LONG_K if M <= rows)
+    return K >= least[0 if N <= 1024 else 1 if N <= 2048 else 2 if N < 4096 else 3]
+
+
 def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                      next_norm_weight: Optional[torch.Tensor] = None, next_one_centered: bool = False,
                      squares: Optional[torch.Tensor] = None, eps: float = 0.0, w_tiled: Optional[torch.Tensor] = None,
@@ -725,16 +759,27 @@ def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tenso
     squares_rows = 0 if squares is None else squares.shape[0]
     w_tiled = _tiled_for(w, w_tiled)
     operand = w if w_tiled is None else w_tiled
-    if mode == 0 and N >= WIDE_STORE and M <= MEDIUM_MAX_ROWS and target.data_ptr() % 16 == 0:
-        _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, M, N, K, _p(squares),
-                                        squares_rows, float(eps), _stream()))
-        return None
+    splits_k = M <= MEDIUM_MAX_ROWS and target.data_ptr() % 16 == 0 and medium_splits_k(mode, M, N, K)
+    if splits_k:
+        need_bytes, need_counters, prepared_rows = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
+        _check(library().fw_gemm_medium_plan(M, N, K, mode, ctypes.byref(need_bytes), ctypes.byref(need_counters), ctypes.byref(prepared_rows)))
     if next_norm_weight is not None:
+        rows = prepared_rows.value if splits_k else library().fw_gemm_rows_square_tiles(M, N)
         next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-        next_squares = torch.empty((library().fw_gemm_rows_square_tiles(M, N), stride), dtype=torch.float32, device=a.device)
-    _check(library().fw_gemm_rows(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
-                                  _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
-                                  squares_rows, float(eps), *_glu(glu), _stream()))
+        next_squares = torch.empty((rows, stride), dtype=torch.float32, device=a.device)
+    if splits_k:
+        workspace = counters = None
+        if need_bytes.value:
+            workspace = torch.empty(need_bytes.value // 4, dtype=torch.float32, device=a.device)
+            counters = _medium_counters(a.device, need_counters.value)
+        _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
+                                        _p(workspace), need_bytes.value, _p(counters), 0 if counters is None else counters.numel(),
+                                        _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
+                                        squares_rows, float(eps), *_glu(glu), _stream()))
+    else:
+        _check(library().fw_gemm_rows(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
+                                      _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
+                                      squares_rows, float(eps), *_glu(glu), _stream()))
     if next_norm_weight is not None:
         return next_activations, next_squares
     return None

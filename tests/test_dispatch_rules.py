@@ -72,3 +72,15 @@ def test_decode_rows_do_not_choose_the_form_of_a_prompt_beside_them(monkeypatch)
                               new_lengths=decoding + [behind + 777], row_seg=None, row_pos=None, seg_row0=None)
         ops.attention(torch.zeros(rows, 32 * 64, dtype=torch.bfloat16), 32, 8, 64, None, None, None, ctx, 0.125, 0, tiles, tiles)
         assert taken.pop() == halves
+
+
+@pytest.mark.parametrize("mode,M,N,K,splits", [
+    (1, 16, 2048, 8192, True), (1, 9, 512, 8192, True), (1, 16, 2048, 4608, False), (1, 16, 4096, 8192, False), (1, 16, 4096, 12288, True),
+    (1, 32, 2048, 12288, True), (1, 32, 2048, 8192, False), (1, 48, 2048, 12288, False), (1, 64, 2048, 12288, True),
+    (1, 32, 2560, 6144, True), (1, 32, 3072, 8192, False), (1, 16, 3072, 8192, False), (1, 64, 1024, 12288, False), (1, 32, 512, 16384, False),
+    (0, 17, 20480, 2048, True), (0, 8, 65536, 2048, True), (0, 64, 65536, 2048, True), (0, 17, 16384, 1024, True), (0, 64, 16384, 1024, False),
+    (0, 32, 8192, 2048, True), (0, 32, 10240, 2048, False), (0, 33, 8192, 2048, False), (0, 17, 4096, 1024, False), (0, 4, 6144, 2048, False),
+    (2, 32, 4608, 1024, True), (2, 64, 4608, 2048, False), (2, 32, 4096, 1024, False), (2, 17, 10752, 2048, True), (2, 17, 10752, 2056, False)])
+def test_products_of_few_rows_split_k_over_workgroups_where_that_is_faster(mode, M, N, K, splits):
+    from flyweight_amd.kernels import ops
+    assert ops.medium_splits_k(mode, M, N, K) == splits
