@@ -44,8 +44,10 @@ int fw_gemm_float32(const float* a, const float* w, const float* bias, void* out
 // multiple of 8. mode 0: out = a . w^T (+ bias) stored as out_dtype (also 2, here and in every storing product below:
 // gelu(a . w^T (+ bias)), the error-function form, in bfloat16); mode 1: out (float32) +=
 // a . w^T (+ bias); mode 2 (SwiGLU): w is [2N][K], gate rows then up rows, out [M][N] bfloat16 =
-// silu(a . gate^T) * (a . up^T), or with out_dtype 3 gelu_tanh(a . gate^T) * (a . up^T). fw_gemm_mfma tiles both operands
-// through LDS (prompts).
+// silu(a . gate^T) * (a . up^T), or with out_dtype 3 gelu_tanh(a . gate^T) * (a . up^T). fw_gemm_skinny is for up to 16
+// rows and a short K; fw_gemm_mfma tiles both operands through LDS (prompts).
+int fw_gemm_skinny(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
+                   int M, int N, int K, void* stream);
 int fw_gemm_mfma(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                  int M, int N, int K, void* stream);
 // The prompt product with large tiles (256 x 256 or 256 x 192; storing products also 128 rows by as many columns,

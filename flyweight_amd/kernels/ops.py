@@ -537,12 +537,22 @@ def gather_rows(rows: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
     return embed_rows(rows, index)
 
 
+def skinny_takes(M: int, N: int, K: int) -> bool:
+    """Whether a product of up to 16 rows goes to the kernel without rings of operands in LDS (fw_gemm_skinny): with a short K, as far as
+    its narrow loads of W do not show. Storing, from memory, us (skinny / waves that split K): 16 features over K 256 2.2 / 2.9, 2,048
+    over 768 at 16 rows 3.8 / 4.0, over 1,024 at 8 4.2 / 4.3, at 16 4.6 / 4.4; 12,288 over 512 6.0 / 6.1, over 1,024 9.0 / 8.2."""
+    return N <= 16384 and K <= (512 if N > 8192 else 1024 if M <= 8 else 768)
+
+
 def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                w_tiled: Optional[torch.Tensor] = None) -> None:
-    """bfloat16 operands on the matrix cores: up to 64 rows, and with weights in operand tiles as long as its tiles are one
+    """bfloat16 operands on the matrix cores: up to 16 rows of a short K the skinny kernel; up to 64 rows, and with weights in operand tiles as long as its tiles are one
     round over the chip, the product whose waves split K; the tiled ones beyond (large tiles where they fill the chip, K cut into slices where
     even the small tiles are too few)."""
     M, K = a.shape
+    if M <= DECODE_MAX_ROWS and skinny_takes(M, N, K):
+        _check(library().fw_gemm_skinny(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
+        return
     if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and M <= ROWS_MAX and library().fw_gemm_rows_round_fits(mode, M, N)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
             gemm_medium_into(a, w, bias, target, BF16, mode, N, w_tiled=w_tiled, glu=GEGLU)

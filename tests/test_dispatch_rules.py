@@ -84,3 +84,10 @@ def test_decode_rows_do_not_choose_the_form_of_a_prompt_beside_them(monkeypatch)
 def test_products_of_few_rows_split_k_over_workgroups_where_that_is_faster(mode, M, N, K, splits):
     from flyweight_amd.kernels import ops
     assert ops.medium_splits_k(mode, M, N, K) == splits
+
+
+@pytest.mark.parametrize("M,N,K,takes", [(1, 16, 256, True), (16, 2048, 768, True), (8, 2048, 1024, True), (16, 2048, 1024, False),
+                                         (1, 4096, 2048, False), (4, 12288, 512, True), (1, 12288, 640, False), (1, 65536, 64, False)])
+def test_products_of_up_to_sixteen_rows_over_a_short_k_take_the_skinny_kernel(M, N, K, takes):
+    from flyweight_amd.kernels import ops
+    assert ops.skinny_takes(M, N, K) == takes

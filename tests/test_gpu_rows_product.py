@@ -29,7 +29,8 @@ def bound(a, w):
 # (rows, features, K): every tile height and its edges; features that end inside a tile or a quad; K of one piece, of a rest, of
 # fewer groups than waves, of a half group for operand tiles; one tile and a whole round of them
 SHAPES = [(1, 16, 8), (16, 40, 64), (17, 96, 520), (32, 33, 2048), (33, 130, 96), (48, 2048, 1056), (64, 515, 168), (64, 6144, 256),
-          (65, 1000, 1024), (130, 1024, 4608), (257, 3072, 224), (512, 2048, 96)]
+          (65, 1000, 1024), (130, 1024, 4608), (257, 3072, 224), (512, 2048, 96),
+          (1, 40, 1032), (5, 2064, 2048), (16, 515, 1112)]      # up to 16 rows only beyond K 1,024
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
