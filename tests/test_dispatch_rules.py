@@ -24,8 +24,7 @@ def _delta_rule(heads, dim, vdim, dtype=torch.bfloat16):
     (16, 128, 128, [694], True), (16, 128, 128, [694, 694], False), (16, 128, 128, [300] * 4, False), (32, 128, 128, [694], False),
     (4, 128, 128, [300] * 4, True), (4, 128, 128, [300] * 8, False), (8, 256, 256, [2048], True), (8, 256, 256, [694] * 2, False),
     (2, 96, 96, [64] * 8, True), (2, 96, 96, [64] * 24, False),
-    (16, 128, 128, [1] * 24 + [694], True),     # single rows leave at once
-    (16, 128, 128, [1] * 64 + [40], False), (16, 128, 128, [600, 694], False), (16, 128, 128, [50, 694], True),
+    (16, 128, 128, [1] * 6 + [1500], False), (16, 128, 128, [1, 694], False), (2, 128, 128, [1] * 6 + [1500], True),
     (16, 64, 64, [694], False)])
 def test_delta_rule_spreads_its_columns_while_every_workgroup_has_a_compute_unit(heads, dim, vdim, lengths, spread):
     assert _delta_rule(heads, dim, vdim).spread(_row0(lengths)) == spread
