@@ -560,11 +560,11 @@ def test_fast_gemm_rows_do_not_depend_on_the_batch(ops):
 
 
 @pytest.mark.parametrize("M", [17, 33, 48, 64])
-@pytest.mark.parametrize("N,K", [(64, 4096), (96, 520), (2048, 8192), (6144, 2048), (25000, 72)])
+@pytest.mark.parametrize("N,K", [(64, 4096), (96, 520), (2048, 8192), (6144, 2048), (25000, 72), (2048, 16384)])
 def test_medium_gemm_splits_k_over_workgroups(ops, M, N, K):
-    """Few features and a long K: slices of K go to different workgroups and the last one to
-    arrive sums them in slice order. Twice in a row (the tickets are left at zero), every
-    epilogue, and bitwise the same whichever workgroup came last."""
+    """The products of a few dozen rows in every epilogue, several times in a row with other rows between: tiles whose waves
+    split K, tiles over all of K of a wide output, and (the last shape) slices of K on different workgroups, of which the last
+    to arrive sums all in slice order, through a workspace and tickets that every call leaves at zero."""
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     bias = gen(N, seed=2).float().to(DEV)
