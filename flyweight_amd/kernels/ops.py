@@ -1004,8 +1004,8 @@ def gemm_decode(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Option
                                          or next_norm_weight.shape != (N,)):
         raise KernelError("gemm_decode: only the accumulating product prepares the next norm, whose weight is float32 [N]")
     if epilogue == EPILOGUE_ACCUMULATE and K >= LONG_K and N <= 4096 and not (w_tiled is not None and rows <= LONG_K_TILED_ROWS):
-        # few features and a long K: the product on tiles of few rows (from operand tiles only beyond eight rows:
-        # 2,048 features over K 8,192 at 8 rows 11.4 us on this one, at 16 rows 13.4 against 12.6 us)
+        # few features and a long K: the products of a few dozen rows (from operand tiles only beyond eight rows:
+        # 2,048 features over K 8,192 at 8 rows 11.8 us on this one, at 12 / 16 rows 14.1 / 14.7 against 11.8 / 11.7)
         left = gemm_medium_into(a, w, bias, target, F32, 1, N, next_norm_weight, next_one_centered, w_tiled=w_tiled)
         return target if left is None else left
     if next_norm_weight is not None:

@@ -67,10 +67,10 @@ class Linear:
         return a.tensor() if isinstance(a, LazyNorm) else a
 
     # From this many weights on the products of a few dozen rows also serve fewer: a large W in row-major order streams
-    # faster through them than through the fused decode product (16,384 x 2,048 with SwiGLU at 12 rows 15.7 us against 19.1 at
-    # eight). From operand tiles the fused product streams faster (gate|up at 8 rows 12.9 against 14.7 us, a
-    # vocabulary of 65,536 45.3 against 49.5 us); only the widest outputs go there from nine rows on, where every
-    # workgroup's own read of all of a begins to weigh (the vocabulary at 16 rows: 50.4 against 52.2 us).
+    # faster through them than through the fused decode product (gated, 16,384 x 2,056, at 4 / 12 rows 17.3 / 17.6 us against
+    # 19.4 / 22.0). From operand tiles the fused product streams faster (gate|up 16,384 x 2,048 at 8 rows 14.3 against 14.8 us, a
+    # vocabulary of 65,536 48.1 against 49.5 us); only the widest outputs go there from nine rows on, where every
+    # workgroup's own read of all of a begins to weigh (the vocabulary at 16 rows: 49.0 against 53.9 us).
     LARGE = 1 << 25
     LARGE_MIN_ROWS = 3
     LARGE_TILED = 1 << 26
@@ -169,7 +169,7 @@ class Linear:
                           seg_slot: torch.Tensor, out_dtype: torch.dtype) -> Optional[torch.Tensor]:
         """For single-token segments: the weight holds B, C and x rows; returns C * conv(B * x)
         with the state shifted, or None when the fused kernel does not take the shape. (Beyond 16
-        rows the product and the convolution run apart: as an epilogue of the split-K product a
+        rows the product and the convolution run apart: as an epilogue of a product that splits K over workgroups a
         workgroup would have to own B, C and x of its channels, which leaves a third as many tiles
         and a fourfold split of K: 41 us against 15.3 + 4.8 us at 64 rows.)"""
         if not self._fused(a, self.out_features // 3, ops.EPILOGUE_CONV):

@@ -128,7 +128,7 @@ def test_sampler_draws_the_reference_samplers_tokens(ops, ref):
         wide_states = want_states
 
 
-# rows that pick every product kernel: the fused decode product (<= 16), the split-K one (17..64),
+# rows that pick every product kernel: the fused decode product (<= 16), those of a few dozen rows (17..64),
 # the tiled prompt kernels (beyond), and the plain float32 kernel
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 72, 200), (7, 200, 264), (16, 1000, 136), (33, 136, 520), (64, 96, 1032), (150, 200, 264)])

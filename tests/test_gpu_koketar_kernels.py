@@ -297,7 +297,7 @@ def test_matrix_core_attention_with_values_of_their_own_size(head_dim, v_dim, wi
 @pytest.mark.parametrize("rows", [1, 8, 16, 40, 64, 200])
 def test_clamped_gated_unit_behind_its_product(rows):
     """Few rows: the unit is the epilogue of the gate|up product (the decode product up to 16 rows, the
-    split-K product up to 64); more rows: float32 sums and the unit's own kernel. All against the plain formula."""
+    products of a few dozen rows up to 64); more rows: float32 sums and the unit's own kernel. All against the plain formula."""
     from flyweight_amd.parts.linear import Linear
     rng = np.random.default_rng(rows)
     hidden, inter, limit = 320, 448, 0.9
