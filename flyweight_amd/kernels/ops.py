@@ -8,6 +8,7 @@ or without a GPU these functions raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import time
 from typing import Dict, Optional
@@ -722,6 +723,7 @@ _LONG_K = ((16, (6144, 6144, 6144, 12288)), (32, (10240, 10240, 6144, 10240)), (
            (64, (16384, 10240, 6144, 1 << 30)))
 
 
+@functools.lru_cache(maxsize=4096)      # (asked at every launch: 0.2 to 0.7 us of the host's time worked out)
 def medium_splits_k(mode: int, M: int, N: int, K: int) -> bool:
     """Whether a product of up to 64 rows goes to the kernel that splits K over workgroups (fw_gemm_medium, several workgroups on a
     compute unit) and not to the one whose waves do (fw_gemm_rows, tiles of up to 64 x 64, one workgroup on a compute unit). The
@@ -752,6 +754,14 @@ def medium_splits_k(mode: int, M: int, N: int, K: int) -> bool:
     return K >= least[0 if N <= 1024 else 1 if N <= 2048 else 2 if N < 4096 else 3]
 
 
+@functools.lru_cache(maxsize=4096)
+def _medium_plan(mode: int, M: int, N: int, K: int):
+    """What the product that splits K over workgroups needs of a shape: bytes of workspace, counters, rows of sums of squares."""
+    need_bytes, need_counters, squares_rows = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
+    _check(library().fw_gemm_medium_plan(M, N, K, mode, ctypes.byref(need_bytes), ctypes.byref(need_counters), ctypes.byref(squares_rows)))
+    return need_bytes.value, need_counters.value, squares_rows.value
+
+
 def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                      next_norm_weight: Optional[torch.Tensor] = None, next_one_centered: bool = False,
                      squares: Optional[torch.Tensor] = None, eps: float = 0.0, w_tiled: Optional[torch.Tensor] = None,
@@ -769,21 +779,20 @@ def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tenso
     squares_rows = 0 if squares is None else squares.shape[0]
     w_tiled = _tiled_for(w, w_tiled)
     operand = w if w_tiled is None else w_tiled
-    splits_k = M <= MEDIUM_MAX_ROWS and target.data_ptr() % 16 == 0 and medium_splits_k(mode, M, N, K)
+    splits_k = M <= MEDIUM_MAX_ROWS and medium_splits_k(mode, M, N, K) and target.data_ptr() % 16 == 0
     if splits_k:
-        need_bytes, need_counters, prepared_rows = ctypes.c_size_t(0), ctypes.c_int(0), ctypes.c_int(0)
-        _check(library().fw_gemm_medium_plan(M, N, K, mode, ctypes.byref(need_bytes), ctypes.byref(need_counters), ctypes.byref(prepared_rows)))
+        need_bytes, need_counters, prepared_rows = _medium_plan(mode, M, N, K)
     if next_norm_weight is not None:
-        rows = prepared_rows.value if splits_k else library().fw_gemm_rows_square_tiles(M, N)
+        rows = prepared_rows if splits_k else library().fw_gemm_rows_square_tiles(M, N)
         next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
         next_squares = torch.empty((rows, stride), dtype=torch.float32, device=a.device)
     if splits_k:
         workspace = counters = None
-        if need_bytes.value:
-            workspace = torch.empty(need_bytes.value // 4, dtype=torch.float32, device=a.device)
-            counters = _medium_counters(a.device, need_counters.value)
+        if need_bytes:
+            workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
+            counters = _medium_counters(a.device, need_counters)
         _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
-                                        _p(workspace), need_bytes.value, _p(counters), 0 if counters is None else counters.numel(),
+                                        _p(workspace), need_bytes, _p(counters), 0 if counters is None else counters.numel(),
                                         _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
                                         squares_rows, float(eps), *_glu(glu), _stream()))
     else:
