@@ -719,8 +719,8 @@ def _tiled_for(w: torch.Tensor, w_tiled: Optional[torch.Tensor]) -> Optional[tor
 
 
 # K from which a product that stores or adds up to 1,024 / 2,048 / 4,095 / 4,096 features splits it over workgroups, by the most rows
-_LONG_K = ((16, (6144, 6144, 6144, 12288)), (32, (10240, 10240, 6144, 10240)), (48, (16384, 16384, 12288, 1 << 30)),
-           (64, (16384, 10240, 6144, 1 << 30)))
+_LONG_K = ((8, (12288, 10240, 12288, 1 << 30)), (11, (8192, 10240, 8192, 12288)), (16, (6144, 6144, 6144, 12288)), (32, (10240, 10240, 6144, 10240)),
+           (48, (16384, 16384, 12288, 1 << 30)), (64, (16384, 10240, 6144, 1 << 30)))
 
 
 @functools.lru_cache(maxsize=4096)      # (asked at every launch: 0.2 to 0.7 us of the host's time worked out)
@@ -736,7 +736,11 @@ def medium_splits_k(mode: int, M: int, N: int, K: int) -> bool:
     * with a long K and few tiles: adding 2,048 features over K 8,192 at 16 rows 12.0 / 13.0, over 12,288 13.1 / 18.3, at 32 rows
       15.2 / 18.2, at 64 21.3 / 23.3, over 10,240 at 64 19.5 / 20.4 but at 48 18.6 / 17.6; 1,024 over 10,240 at 32 rows 13.0 /
       14.6, at 64 17.3 / 14.1; 2,560, whose tiles of 16 leave a third of the chip without work, over 6,144 at 32 rows 12.0 /
-      13.9; where the slices of K are more than a round they lose again (3,072 over 8,192 at 32 rows 20.3 / 17.2)."""
+      13.9; where the slices of K are more than a round they lose again (3,072 over 8,192 at 32 rows 20.3 / 17.2). Fewer rows
+      pay the exchange later: adding 2,048 over 8,192 at 10 rows 11.9 / 11.7 (a decode step of 9 requests, 16 such products, 814 / 804,
+      of 12 831 / 831, of 16 865 / 882), over 12,288 13.5 / 16.7; 1,024 over 6,144 at 9 rows 9.1 / 9.0, over 8,192 9.7 / 11.0. Up to
+      eight rows come here in row-major order alone: 2,048 over 8,192 at 1 / 8 rows 13.2 / 11.0, 13.0 / 12.0, over 12,288
+      15.4 / 14.9, 15.3 / 16.8, 4,096 over 12,288 26.9 / 22.5."""
     if mode == 2:
         return K % 32 == 0 and (N > 8192 or (N > 4096 and M > DECODE_MAX_ROWS and K <= (1536 if M <= 48 else 1024)))
     if N > 16384:

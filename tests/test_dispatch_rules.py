@@ -74,7 +74,9 @@ def test_decode_rows_do_not_choose_the_form_of_a_prompt_beside_them(monkeypatch)
 
 
 @pytest.mark.parametrize("mode,M,N,K,splits", [
-    (1, 16, 2048, 8192, True), (1, 9, 512, 8192, True), (1, 16, 2048, 4608, False), (1, 16, 4096, 8192, False), (1, 16, 4096, 12288, True),
+    (1, 16, 2048, 8192, True), (1, 9, 512, 8192, True), (1, 8, 512, 8192, False),
+    (1, 11, 2048, 8192, False), (1, 12, 2048, 8192, True), (1, 9, 2048, 10752, True), (1, 8, 4096, 12288, False), (1, 11, 4096, 12288, True),
+    (1, 16, 2048, 4608, False), (1, 16, 4096, 8192, False), (1, 16, 4096, 12288, True),
     (1, 32, 2048, 12288, True), (1, 32, 2048, 8192, False), (1, 48, 2048, 12288, False), (1, 64, 2048, 12288, True),
     (1, 32, 2560, 6144, True), (1, 32, 3072, 8192, False), (1, 16, 3072, 8192, False), (1, 64, 1024, 12288, False), (1, 32, 512, 16384, False),
     (0, 17, 20480, 2048, True), (0, 8, 65536, 2048, True), (0, 64, 65536, 2048, True), (0, 17, 16384, 1024, True), (0, 64, 16384, 1024, False),

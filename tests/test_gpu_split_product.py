@@ -34,9 +34,9 @@ def close(found, exact, limit, rounding):
 
 # K in slices of several workgroups (three to sixteen); tiles of 32 features in a round and in two; tiles of 64 features over all
 # of K, K x N beyond 2^24 (the walk starts elsewhere in each workgroup) and below; K of half a chunk more
-SHAPES = [(1, 512, 6144), (9, 1000, 8224), (16, 2048, 8192), (17, 2048, 10272), (32, 2552, 6176), (40, 2560, 12320), (64, 2046, 12288),
-          (17, 5000, 1024), (20, 16400, 296), (33, 20470, 520), (1, 25000, 1056), (9, 25000, 1056), (16, 25000, 1056), (17, 25000, 1056),
-          (40, 25000, 1056), (64, 25000, 1056), (64, 24580, 72)]
+SHAPES = [(1, 512, 12288), (12, 512, 6144), (9, 1000, 8224), (16, 2048, 8192), (17, 2048, 10272), (32, 2552, 6176),
+          (40, 2560, 12320), (64, 2046, 12288), (17, 5000, 1024), (20, 16400, 296), (33, 20470, 520), (1, 25000, 1056),
+          (9, 25000, 1056), (16, 25000, 1056), (17, 25000, 1056), (40, 25000, 1056), (64, 25000, 1056), (64, 24580, 72)]
 
 
 @pytest.mark.parametrize("M,N,K", SHAPES)
