@@ -88,12 +88,12 @@ int fw_gemm_medium(const void* a, const void* w, int w_tiled, const float* bias,
 // a workgroup's waves alone: no workspace, no counters. Up to 64 rows the accumulating product can leave what the norm after
 // it needs, as fw_gemm_decode does (next_activations [M][N] bfloat16, next_squares [fw_gemm_rows_square_tiles(M, N)][16 for M <= 16,
 // else 64]), and any mode takes such prepared activations as a, with squares / squares_rows / eps. fw_gemm_rows_round_fits: whether
-// its tiles are at most one round over the compute units.
+// its tiles are at most one round over the compute units and, with this K, faster than the products that tile both operands.
 int fw_gemm_rows(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
                  const float* next_norm_weight, int next_one_centered, void* next_activations, float* next_squares, const float* squares,
                  int squares_rows, float eps, float glu_limit, float glu_alpha, float glu_shift, void* stream);
 int fw_gemm_rows_square_tiles(int M, int N);
-int fw_gemm_rows_round_fits(int mode, int M, int N);
+int fw_gemm_rows_round_fits(int mode, int M, int N, int K);
 
 // Fused product for decode steps of up to 16 rows. prologue 0: a is bfloat16 [M][K]; 1: a is
 // float32 rows, RMS-normed with norm_weight/eps (rows gathered through row_index if given) inside

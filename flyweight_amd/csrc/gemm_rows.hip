@@ -433,9 +433,19 @@ int rows_mode(const RowsArgs& args, const RowsPlan& plan, int out_dtype, int mod
 // how many rows the sums of squares left for the next norm take (the second extent: 16 for M <= 16, else 64)
 extern "C" int fw_gemm_rows_square_tiles(int M, int N) { return rows_plan(M, N, GR_ACCUMULATE).tiles_n; }
 
-extern "C" int fw_gemm_rows_round_fits(int mode, int M, int N) {
+// Whether the tiles are one round over the compute units, and serve better than the products that tile both operands. With a long K
+// those have caught up with the large tiles unless their own leave much of a round empty, which these do not where 200 to 240 (up
+// to K 8,192 more) of them are wanted. us, here / there, storing 2,560 features at 128 rows over K 4,096 / 8,192 15.1 / 18.2,
+// 28.2 / 25.5, at 160 rows over 8,192 26.0 / 32.8; gated 1,536 at 192 rows over 4,096 / 8,192 22.7 / 23.7, 39.2 / 33.4, at 320 rows over
+// 8,192 37.9 / 58.1; gated 4,096 at 128 rows over 8,192 / 10,752 40.9 / 45.9, 61.9 / 53.9. (Storing, the tiles of 64 x 64 win at any K.)
+extern "C" int fw_gemm_rows_round_fits(int mode, int M, int N, int K) {
     const RowsPlan plan = rows_plan(M, N, mode);
-    return M >= 1 && M <= 4096 && (long long)plan.tiles_m * plan.tiles_n <= 256;
+    const long long tiles = (long long)plan.tiles_m * plan.tiles_n;
+    if (M < 1 || M > 4096 || tiles > 256) return 0;
+    const int products = plan.tm * plan.tn;
+    if (mode == GR_ACCUMULATE || products < 8 || (tiles >= 200 && (K <= 8192 || tiles <= 240))) return 1;
+    if (products == 8) return K < 8192 || M <= 96;
+    return mode == GR_STORE || K <= 5120;
 }
 
 extern "C" int fw_gemm_rows(const void* a, const void* w, int w_tiled, const float* bias, void* out, int out_dtype, int mode, int M, int N,

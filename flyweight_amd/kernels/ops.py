@@ -545,6 +545,12 @@ def skinny_takes(M: int, N: int, K: int) -> bool:
     return N <= 16384 and K <= (512 if N > 8192 else 1024 if M <= 8 else 768)
 
 
+@functools.lru_cache(maxsize=4096)
+def rows_fit(mode: int, M: int, N: int, K: int) -> bool:
+    """Whether a product of more than 64 rows, its weights in operand tiles, goes to the kernel whose waves split K."""
+    return M <= ROWS_MAX and bool(library().fw_gemm_rows_round_fits(mode, M, N, K))
+
+
 def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                w_tiled: Optional[torch.Tensor] = None) -> None:
     """bfloat16 operands on the matrix cores: up to 16 rows of a short K the skinny kernel; up to 64 rows, and with weights in operand tiles as long as its tiles are one
@@ -554,7 +560,7 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     if M <= DECODE_MAX_ROWS and skinny_takes(M, N, K):
         _check(library().fw_gemm_skinny(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
         return
-    if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and M <= ROWS_MAX and library().fw_gemm_rows_round_fits(mode, M, N)):
+    if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and rows_fit(mode, M, N, K)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
             gemm_medium_into(a, w, bias, target, BF16, mode, N, w_tiled=w_tiled, glu=GEGLU)
         else:
@@ -595,7 +601,8 @@ MEDIUM_MAX_ROWS = 64
 # compute units; measured against the tiled products, every weight from memory: adding 2,048 features (K 8,192) at 128 / 256 / 512
 # rows 20.6 / 26.2 / 34.8 against 25.0 / 30.6 / 44.1 us, K 2,048 8.2 / 10.6 / 14.3 against 14.8 / 15.1 / 18.9; storing 3,072 features at
 # 256 rows 14.4 against 18.1, 6,144 at 128 rows 15.3 against 18.9. With two rounds it loses (6,144 features at 192 rows 25.9 against
-# 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27).
+# 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27), and so it does with a long K where the others' tiles
+# fill their round (fw_gemm_rows_round_fits).
 ROWS_MAX = 1024
 BIG_TILES_MIN = 192      # 256 x 256 tiles from which the large-tile prompt product is used (256 compute units)
 DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)

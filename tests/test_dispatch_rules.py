@@ -92,3 +92,13 @@ def test_products_of_few_rows_split_k_over_workgroups_where_that_is_faster(mode,
 def test_products_of_up_to_sixteen_rows_over_a_short_k_take_the_skinny_kernel(M, N, K, takes):
     from flyweight_amd.kernels import ops
     assert ops.skinny_takes(M, N, K) == takes
+
+
+@pytest.mark.parametrize("mode,M,N,K,fits", [
+    (1, 512, 2048, 8192, True), (1, 128, 2560, 10752, True), (0, 192, 6144, 2048, False), (0, 128, 6144, 2048, True), (2, 128, 8192, 2048, False),
+    (0, 128, 2560, 7168, True), (0, 128, 2560, 8192, False), (0, 96, 3072, 10752, True), (0, 160, 2560, 10752, True), (0, 256, 2048, 8192, True),
+    (0, 256, 2048, 10752, False), (0, 256, 4096, 10752, True), (2, 192, 1536, 5120, True), (2, 192, 1536, 6144, False), (2, 320, 1536, 10752, True),
+    (2, 128, 4096, 8192, True), (2, 128, 4096, 10752, False), (2, 96, 1536, 10752, True), (2, 128, 1536, 8192, False), (1, 1025, 64, 64, False)])
+def test_products_beyond_64_rows_are_dealt_to_waves_where_that_is_faster(mode, M, N, K, fits):
+    from flyweight_amd.kernels import ops
+    assert ops.rows_fit(mode, M, N, K) == fits
