@@ -856,7 +856,7 @@ def test_fused_decode_product(ops, M, N, K):
     before = residual.cpu().double()
     ops.gemm_decode(a, w, ops.EPILOGUE_ACCUMULATE, accumulate_into=residual, bias=bias.to(DEV))
     close(residual, before + plain + bias.double(), torch.float32, 2.0)
-    # the same product from the skinny kernel agrees to float32 rounding
+    # the same product from the kernels without a norm in front agrees to float32 rounding
     close(ops.gemm(a, w, out_dtype=torch.float32), plain, torch.float32, 2.0)
     if N % 2 == 0:
         half = N // 2
@@ -905,7 +905,8 @@ def test_fused_decode_product_prepares_the_next_norm(ops, M, H, N, one_centered,
     """The product that adds to the residual stream leaves x * w of the norm after it and sums
     of squares per tile; the next product takes both instead of norming itself. Checked: what
     is left, and the next product (every epilogue that may follow) against a plain norm. With a
-    long K the accumulating product is the one that splits K over workgroups."""
+    long K and few features the accumulating product is one of the products of a few dozen rows (at 16 rows the one that splits K
+    over workgroups, below the one whose waves split it)."""
     a = as_dev(gen(M, K, seed=1), torch.bfloat16)
     w_out = as_dev(gen(H, K, seed=2, scale=K ** -0.5), torch.bfloat16)
     residual = gen(M, H, seed=3, scale=2).float().to(DEV)

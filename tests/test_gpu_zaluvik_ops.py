@@ -253,7 +253,7 @@ def test_layer_norms_with_bias_around_a_sublayer(ops, hidden):
         assert np.array_equal(host(joined)[:, hidden:], stored(x.astype(np.float32), dtype))
 
 
-# every product that stores: the fused one, the one that splits K, the skinny one (K no multiple of 32), the tiled ones
+# every product that stores: the fused one, the skinny one (a short K without operand tiles), the one whose waves split K, the tiled ones
 @pytest.mark.parametrize("rows,N,K", [(1, 40, 96), (8, 3200, 256), (13, 100, 40), (40, 300, 128), (64, 96, 2048), (100, 200, 64), (300, 1024, 512), (700, 4096, 256),
                                       (2048, 4096, 128), (200, 130, 44), (256, 6144, 4096)])
 def test_gelu_in_the_products(ops, rows, N, K):
