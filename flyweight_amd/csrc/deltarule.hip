@@ -280,8 +280,9 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     float S[RPT];
     auto row_of = [&](int t) { return t / RUN * (RUN * DELTA_LANES) + part * RUN + t % RUN; };
     // a lane's runs of four rows as they are where every run is whole (dim a multiple of 4, the state aligned to 16 bytes): for a
-    // single token the state is nearly all that travels (64 of them, 32 heads of 128 channels: 89 us one float at a time, 64 so)
-    if (RUN == 4 && runs_whole) {
+    // single token the state is nearly all that travels (64 of them, 32 heads of 128 channels: 89 us one float at a time, 64 so). Not on
+    // 32 lanes, which prompts alone take: their walk became slower by it (16 heads, 1,111 rows 228 -> 232)
+    if (RUN == 4 && DELTA_LANES == 16 && runs_whole) {
 #pragma unroll
         for (int t = 0; t < RPT; t += RUN) {
             f32x4 run = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
         fw_lds_barrier();
     }
     if (!live) return;
-    if (RUN == 4 && runs_whole) {
+    if (RUN == 4 && DELTA_LANES == 16 && runs_whole) {
 #pragma unroll
         for (int t = 0; t < RPT; t += RUN)
             if (row_of(t) < dim) {
