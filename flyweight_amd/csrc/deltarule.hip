@@ -14,12 +14,10 @@
 // The state is stored transposed, [slot][head][vdim][dim], so that the columns a wave holds are one
 // contiguous piece of memory.
 #include "fw_common.h"
+#include "deltarule.h"
 #include "fw_kernels.h"
 
 #define DELTA_CHUNK 16          // tokens staged in LDS at a time
-
-__device__ __forceinline__ float fw_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float fw_softplus(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
 
 // ---- what the recurrence reads, from the projections -----------------------------------------------
 // One wave per (row, vector). Vectors 0..G-1: query heads, G..2G-1: key heads (dim channels each,
@@ -125,6 +123,13 @@ __global__ void conv_state_kernel(const TI* __restrict__ proj, int proj_stride, 
     }
 }
 
+void fw_launch_conv_state(const void* proj, int dtype, int proj_stride, float* conv_state, const int32_t* seg_row0, const int32_t* seg_slot,
+                          int channels, int taps_count, int segments, hipStream_t stream) {
+    const dim3 grid((channels + 127) / 128, segments);
+    if (dtype == FW_F32) conv_state_kernel<float><<<grid, 128, 0, stream>>>((const float*)proj, proj_stride, conv_state, seg_row0, seg_slot, channels, taps_count);
+    else conv_state_kernel<bf16_t><<<grid, 128, 0, stream>>>((const bf16_t*)proj, proj_stride, conv_state, seg_row0, seg_slot, channels, taps_count);
+}
+
 extern "C" int fw_delta_prepare(const void* proj, int dtype, int proj_stride, int beta_col, const void* a, int a_stride, const float* taps,
                                 float* conv_state, const float* A_log, const float* dt_bias, const int32_t* row_seg,
                                 const int32_t* seg_row0, const int32_t* seg_slot, float* records, int rows, int segments,
@@ -143,7 +148,6 @@ extern "C" int fw_delta_prepare(const void* proj, int dtype, int proj_stride, in
     if (rows == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
     dim3 grid(rows, 2 * kv_heads + 2 * heads);
-    dim3 state_grid((channels + 127) / 128, segments);
     const bool single = rows == segments;       // every segment one row: the memory moves on inside the one kernel
 #define FW_PREPARE_LAUNCH(TI, SINGLE)                                                                                         \
     delta_prepare_kernel<TI, SINGLE><<<grid, 64, 0, s>>>((const TI*)proj, proj_stride, beta_col, (const TI*)a, a_stride, taps, \
@@ -152,38 +156,20 @@ extern "C" int fw_delta_prepare(const void* proj, int dtype, int proj_stride, in
     if (dtype == FW_F32) {
         if (single) FW_PREPARE_LAUNCH(float, true);
         else FW_PREPARE_LAUNCH(float, false);
-        if (taps_count > 1 && !single)
-            conv_state_kernel<float><<<state_grid, 128, 0, s>>>((const float*)proj, proj_stride, conv_state, seg_row0, seg_slot, channels, taps_count);
     } else if (dtype == FW_BF16) {
         if (single) FW_PREPARE_LAUNCH(bf16_t, true);
         else FW_PREPARE_LAUNCH(bf16_t, false);
-        if (taps_count > 1 && !single)
-            conv_state_kernel<bf16_t><<<state_grid, 128, 0, s>>>((const bf16_t*)proj, proj_stride, conv_state, seg_row0, seg_slot, channels, taps_count);
     } else {
         FW_REQUIRE(false, "delta_prepare: unknown dtype %d", dtype);
     }
 #undef FW_PREPARE_LAUNCH
+    if (taps_count > 1 && !single) fw_launch_conv_state(proj, dtype, proj_stride, conv_state, seg_row0, seg_slot, channels, taps_count, segments, s);
     FW_LAUNCH_CHECK("delta_prepare");
     return 0;
 }
 
 // ---- the recurrence -----------------------------------------------------------------------------
 extern "C" int fw_delta_record_floats(int dim, int vdim) { return 3 * ((dim + 3) & ~3) + 4 + ((vdim + 3) & ~3); }
-
-// A sum over the 16 lanes of a row of the wave (every lane gets it): neighbours, pairs, then the two
-// mirrors, all inside the vector unit (no trip through the LDS crossbar). After each step the lanes
-// that have met hold one value, so the mirrors may stand for the exchanges between quads and halves.
-template <int CTRL>
-__device__ __forceinline__ float delta_dpp(float x) {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), CTRL, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float delta_row_sum(float x) {
-    x += delta_dpp<0xB1>(x);        // quad_perm [1, 0, 3, 2]
-    x += delta_dpp<0x4E>(x);        // quad_perm [2, 3, 0, 1]
-    x += delta_dpp<0x141>(x);       // row_half_mirror
-    x += delta_dpp<0x140>(x);       // row_mirror
-    return x;
-}
 
 template <int DELTA_LANES>
 __device__ __forceinline__ float delta_lanes_sum(float x) {

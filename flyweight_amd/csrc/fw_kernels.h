@@ -309,6 +309,15 @@ int fw_delta_prepare(const void* proj, int dtype, int proj_stride, int beta_col,
 int fw_gated_delta_rule(const float* records, float* state, float* out, const int32_t* seg_row0,
                         const int32_t* seg_slot, int rows, int segments, int heads, int dim, int vdim,
                         int slots, int spread, void* stream);
+// Both at once for steps with long segments, float32 projections: sixteen tokens of a segment at a time as float32 matrix products (other
+// sums than token by token, so other roundings). packets: fw_delta_chunk_slots(rows, segments) x H x fw_delta_packet_floats(d, vd)
+// floats of workspace, 16-byte aligned. The other arguments are fw_delta_prepare's and fw_gated_delta_rule's.
+int fw_delta_packet_floats(int dim, int vdim);
+int fw_delta_chunk_slots(int rows, int segments);
+int fw_delta_chunks(const float* proj, int proj_stride, int beta_col, const float* a, int a_stride, const float* taps, float* conv_state,
+                    const float* A_log, const float* dt_bias, const int32_t* seg_row0, const int32_t* seg_slot, float* packets,
+                    float* state, float* out, int rows, int segments, int heads, int kv_heads, int dim, int vdim, int taps_count,
+                    int slots, int decay_per_head, void* stream);
 // out[r][h][j] = o[r][h][j] * rsqrt(mean_j o[r][h]^2 + eps) * weight[j] * act(gate[r][h vd + j]);
 // act is the sigmoid, or with gate_silu z * sigmoid(z)
 int fw_gated_head_norm(const float* o, const void* gate, int gate_dtype, int gate_stride, const float* weight, int weight_per_head,

@@ -46,7 +46,7 @@ class _ProfiledLibrary:
 
     def __getattr__(self, name):
         entry = getattr(self._library, name)
-        if not name.startswith("fw_") or name in ("fw_last_error", "fw_abi_version") or name.endswith(("_plan", "_fits", "_tiles")):
+        if not name.startswith("fw_") or name in ("fw_last_error", "fw_abi_version") or name.endswith(("_plan", "_fits", "_tiles", "_floats", "_slots")):
             return entry
 
         def timed(*args):
@@ -1431,6 +1431,33 @@ def sigmoid_attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
 
 
 # ---- the gated delta rule -----------------------------------------------------------------------------
+def _delta_inputs(name: str, proj, a, taps, conv_state, A_log, dt_bias, seg_row0, seg_slot, segments: int, heads: int, kv_heads: int, dim: int,
+                  vdim: int, decay_per_head: bool):
+    """Checks what the gated delta rule's kernels are given; (rows, floats between rows, channels, taps, decays of a row)."""
+    _dev(proj, taps, conv_state, A_log, dt_bias, seg_row0, seg_slot)
+    _dev_rows(a, "a")
+    rows, stride = proj.shape
+    channels = 2 * kv_heads * dim + heads * vdim
+    count = taps.shape[1]
+    if proj.dtype != a.dtype or not proj.is_contiguous() or a.dim() != 2 or a.stride(1) != 1:
+        raise KernelError(f"{name}: the projections and the decays' arguments come in one dtype, rows contiguous")
+    decays = heads if decay_per_head else heads * dim
+    if a.shape != (rows, decays):
+        raise KernelError(f"{name}: a is {tuple(a.shape)}, expected {(rows, decays)} (a view of wider rows will do)")
+    for what, t, shape in (("taps", taps, (channels, count)), ("A_log", A_log, (heads,)), ("dt_bias", dt_bias, (decays,))):
+        _want(t, torch.float32, what)
+        if t.shape != shape or not t.is_contiguous():
+            raise KernelError(f"{name}: {what} is {tuple(t.shape)}, expected {shape}")
+    _want(conv_state, torch.float32, "conv_state")
+    if conv_state.dim() != 3 or conv_state.shape[1:] != (channels, count - 1) or not conv_state.is_contiguous():
+        raise KernelError(f"{name}: the convolutions' state is {tuple(conv_state.shape)}, expected [slots, {channels}, {count - 1}]")
+    for what, t, n in (("seg_row0", seg_row0, segments + 1), ("seg_slot", seg_slot, segments)):
+        _want(t, torch.int32, what)
+        if t.numel() < n:
+            raise KernelError(f"{name}: {what} holds {t.numel()} entries, needs {n}")
+    return rows, stride, channels, count, decays
+
+
 def delta_prepare(proj: torch.Tensor, beta_col: int, a: torch.Tensor, taps: torch.Tensor, conv_state: torch.Tensor,
                   A_log: torch.Tensor, dt_bias: torch.Tensor, row_seg: torch.Tensor, seg_row0: torch.Tensor,
                   seg_slot: torch.Tensor, segments: int, heads: int, kv_heads: int, dim: int, vdim: int,
@@ -1442,27 +1469,12 @@ def delta_prepare(proj: torch.Tensor, beta_col: int, a: torch.Tensor, taps: torc
     moved on. ``decay_per_head``: one decay for all key channels of a head (``a`` [rows, heads],
     ``dt_bias`` [heads]). Returns float32 records [rows, heads, delta_record_floats(dim, vdim)]: per row and head
     q | k | g | beta | v as the recurrence reads them (q and k of the head's group)."""
-    _dev(proj, taps, conv_state, A_log, dt_bias, row_seg, seg_row0, seg_slot)
-    _dev_rows(a, "a")
-    rows, stride = proj.shape
-    channels = 2 * kv_heads * dim + heads * vdim
-    count = taps.shape[1]
-    if proj.dtype != a.dtype or not proj.is_contiguous() or a.dim() != 2 or a.stride(1) != 1:
-        raise KernelError("delta_prepare: the projections and the decays' arguments come in one dtype, rows contiguous")
-    decays = heads if decay_per_head else heads * dim
-    if a.shape != (rows, decays):
-        raise KernelError(f"delta_prepare: a is {tuple(a.shape)}, expected {(rows, decays)} (a view of wider rows will do)")
-    for name, t, shape in (("taps", taps, (channels, count)), ("A_log", A_log, (heads,)), ("dt_bias", dt_bias, (decays,))):
-        _want(t, torch.float32, name)
-        if t.shape != shape or not t.is_contiguous():
-            raise KernelError(f"delta_prepare: {name} is {tuple(t.shape)}, expected {shape}")
-    _want(conv_state, torch.float32, "conv_state")
-    if conv_state.dim() != 3 or conv_state.shape[1:] != (channels, count - 1) or not conv_state.is_contiguous():
-        raise KernelError(f"delta_prepare: the convolutions' state is {tuple(conv_state.shape)}, expected [slots, {channels}, {count - 1}]")
-    for name, t, n in (("row_seg", row_seg, rows), ("seg_row0", seg_row0, segments + 1), ("seg_slot", seg_slot, segments)):
-        _want(t, torch.int32, name)
-        if t.numel() < n:
-            raise KernelError(f"delta_prepare: {name} holds {t.numel()} entries, needs {n}")
+    _dev(row_seg)
+    _want(row_seg, torch.int32, "row_seg")
+    if row_seg.numel() < proj.shape[0]:
+        raise KernelError(f"delta_prepare: row_seg holds {row_seg.numel()} entries, needs {proj.shape[0]}")
+    rows, stride, channels, count, decays = _delta_inputs("delta_prepare", proj, a, taps, conv_state, A_log, dt_bias, seg_row0, seg_slot,
+                                                          segments, heads, kv_heads, dim, vdim, decay_per_head)
     records = torch.empty((rows, heads, delta_record_floats(dim, vdim)), dtype=torch.float32, device=proj.device)
     _check(library().fw_delta_prepare(_p(proj), _code(proj.dtype), stride, int(beta_col), _p(a), a.stride(0) if rows > 1 else max(decays, a.stride(0)),
                                       _p(taps), _p(conv_state), _p(A_log), _p(dt_bias), _p(row_seg), _p(seg_row0), _p(seg_slot),
@@ -1477,6 +1489,13 @@ def delta_record_floats(dim: int, vdim: int) -> int:
     return 3 * ((dim + 3) // 4 * 4) + 4 + (vdim + 3) // 4 * 4
 
 
+def _delta_state(name: str, state: torch.Tensor, heads: int, dim: int, vdim: int) -> None:
+    _dev(state)
+    _want(state, torch.float32, "state")
+    if state.dim() != 4 or state.shape[1:] != (heads, vdim, dim):
+        raise KernelError(f"{name}: the state is {tuple(state.shape)}, expected [slots, {heads}, {vdim}, {dim}]")
+
+
 def gated_delta_rule(records: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor,
                      segments: int, heads: int, dim: int, vdim: int, spread: bool = False) -> torch.Tensor:
     """The recurrence over each segment's rows (``spread``: large heads on twice the workgroups, for prompts).
@@ -1488,9 +1507,7 @@ def gated_delta_rule(records: torch.Tensor, state: torch.Tensor, seg_row0: torch
     _want(records, torch.float32, "records")
     if records.shape != (rows, heads, delta_record_floats(dim, vdim)) or not records.is_contiguous():
         raise KernelError(f"gated_delta_rule: records are {tuple(records.shape)}, expected {(rows, heads, delta_record_floats(dim, vdim))}")
-    _want(state, torch.float32, "state")
-    if state.dim() != 4 or state.shape[1:] != (heads, vdim, dim) or not state.is_contiguous():
-        raise KernelError(f"gated_delta_rule: the state is {tuple(state.shape)}, expected [slots, {heads}, {vdim}, {dim}]")
+    _delta_state("gated_delta_rule", state, heads, dim, vdim)
     for name, t, n in (("seg_row0", seg_row0, segments + 1), ("seg_slot", seg_slot, segments)):
         _want(t, torch.int32, name)
         if t.numel() < n:
@@ -1498,6 +1515,26 @@ def gated_delta_rule(records: torch.Tensor, state: torch.Tensor, seg_row0: torch
     out = torch.empty((rows, heads * vdim), dtype=torch.float32, device=records.device)
     _check(library().fw_gated_delta_rule(_p(records), _p(state), _p(out), _p(seg_row0), _p(seg_slot), rows, int(segments), heads,
                                          dim, vdim, state.shape[0], int(spread), _stream()))
+    return out
+
+
+def delta_chunks(proj: torch.Tensor, beta_col: int, a: torch.Tensor, taps: torch.Tensor, conv_state: torch.Tensor, A_log: torch.Tensor,
+                 dt_bias: torch.Tensor, state: torch.Tensor, seg_row0: torch.Tensor, seg_slot: torch.Tensor, segments: int, heads: int,
+                 kv_heads: int, dim: int, vdim: int, decay_per_head: bool = False) -> torch.Tensor:
+    """``delta_prepare`` and ``gated_delta_rule`` at once for steps with long segments, float32 projections: sixteen tokens of a segment at a
+    time as matrix products (float32 throughout; other sums than token by token). Returns [rows, heads vdim]."""
+    rows, stride, channels, count, decays = _delta_inputs("delta_chunks", proj, a, taps, conv_state, A_log, dt_bias, seg_row0, seg_slot,
+                                                          segments, heads, kv_heads, dim, vdim, decay_per_head)
+    _want(proj, torch.float32, "proj")
+    _delta_state("delta_chunks", state, heads, dim, vdim)
+    lib = library()
+    packets = torch.empty((lib.fw_delta_chunk_slots(rows, int(segments)), heads, lib.fw_delta_packet_floats(dim, vdim)), dtype=torch.float32,
+                          device=proj.device)
+    out = torch.empty((rows, heads * vdim), dtype=torch.float32, device=proj.device)
+    _check(lib.fw_delta_chunks(_p(proj), stride, int(beta_col), _p(a), a.stride(0) if rows > 1 else max(decays, a.stride(0)), _p(taps),
+                               _p(conv_state), _p(A_log), _p(dt_bias), _p(seg_row0), _p(seg_slot), _p(packets), _p(state), _p(out), rows,
+                               int(segments), heads, kv_heads, dim, vdim, count, min(conv_state.shape[0], state.shape[0]),
+                               int(decay_per_head), _stream()))
     return out
 
 

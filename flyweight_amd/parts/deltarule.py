@@ -148,7 +148,8 @@ class GatedDeltaRule(Mixer):
         return self._no_conv_state
 
     def spread(self, row0) -> bool:
-        """Whether a step's columns of state are shared out over 32 lanes (``row0``: the first row of each segment, and the end).
+        """Whether the columns of state of a step that is walked token by token are shared out over 32 lanes (``row0``: the first row of each
+        segment, and the end).
         A walk is bound by how fast one wave issues its chain of instructions, so half the arithmetic a wave pays as long as its
         workgroups, of 8 value channels, have a compute unit each. 16 heads of 128 channels, prompts of 694 rows: one
         173 -> 150 us, but two 177 -> 196 and four 222 -> 320; 4 heads: four prompts 173 -> 148, eight of 300 rows
@@ -157,6 +158,17 @@ class GatedDeltaRule(Mixer):
         if self.dtype != torch.bfloat16 or self.dim <= 64:
             return False        # (a float32 run gives the same bits however a sequence is cut into steps: its prompts walk as its single rows do)
         return (len(row0) - 1) * self.heads * -(-self.vdim // 8) <= ops.COMPUTE_UNITS
+
+    def chunked(self, row0) -> bool:
+        """Whether a step's segments are walked sixteen tokens at a time (``row0``: the first row of each segment, and the end). That takes
+        one launch more and a chunk's work for a segment of one row, and gains 0.05 to 0.17 us a token of the longest segment. 16 heads of
+        128 channels, convolutions included: one prompt of 64 rows 25 -> 23 us, of 96 33 -> 26, of 1,111 272 -> 117, sixteen of 96 169 -> 112;
+        2 heads of 16 channels: 64 rows 16.5 -> 18.9, 96 rows 21.3 -> 20.4. Beside 24 single rows 64 rows lose (46 -> 56) and 128 gain
+        (70 -> 65), beside 60 single rows 128 lose (84 -> 116) and 500 gain (233 -> 150)."""
+        if self.dtype != torch.bfloat16:
+            return False        # (a float32 run gives the same bits however a sequence is cut into steps)
+        lengths = [b - a for a, b in zip(row0, row0[1:])]
+        return max(lengths, default=0) >= 96 + 2 * sum(n < 16 for n in lengths)
 
     def heads_output(self, h, ctx, cache) -> torch.Tensor:
         """The heads' normed and gated read-outs [rows, heads * vdim] in the activation dtype; the
@@ -172,11 +184,16 @@ class GatedDeltaRule(Mixer):
             gate = proj[:, self.gate_col:self.gate_col + self.heads * self.vdim]
         else:
             gate = both[:, both.shape[1] - self.heads * self.vdim:]
-        records = ops.delta_prepare(proj, self.beta_col, a, self.taps, self._conv_state(cache), self.A_log, self.dt_bias,
-                                    ctx.row_seg, ctx.seg_row0, ctx.seg_slot, ctx.num_segments, self.heads, self.kv_heads,
-                                    self.dim, self.vdim, decay_per_head=per_head)
-        o = ops.gated_delta_rule(records, cache["state"].state, ctx.seg_row0, ctx.seg_slot, ctx.num_segments,
-                                 self.heads, self.dim, self.vdim, spread=not ctx.all_decode and self.spread(ctx.host_seg_row0))
+        if not ctx.all_decode and self.chunked(ctx.host_seg_row0):
+            o = ops.delta_chunks(proj, self.beta_col, a, self.taps, self._conv_state(cache), self.A_log, self.dt_bias, cache["state"].state,
+                                 ctx.seg_row0, ctx.seg_slot, ctx.num_segments, self.heads, self.kv_heads, self.dim, self.vdim,
+                                 decay_per_head=per_head)
+        else:
+            records = ops.delta_prepare(proj, self.beta_col, a, self.taps, self._conv_state(cache), self.A_log, self.dt_bias,
+                                        ctx.row_seg, ctx.seg_row0, ctx.seg_slot, ctx.num_segments, self.heads, self.kv_heads,
+                                        self.dim, self.vdim, decay_per_head=per_head)
+            o = ops.gated_delta_rule(records, cache["state"].state, ctx.seg_row0, ctx.seg_slot, ctx.num_segments,
+                                     self.heads, self.dim, self.vdim, spread=not ctx.all_decode and self.spread(ctx.host_seg_row0))
         return ops.gated_head_norm(o, gate, self.norm_weight, self.heads, self.vdim, self.eps, self.dtype,
                                    gate_silu=self.gate == "silu")
 

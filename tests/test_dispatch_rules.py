@@ -31,6 +31,14 @@ def test_delta_rule_spreads_its_columns_while_every_workgroup_has_a_compute_unit
     assert not _delta_rule(heads, dim, vdim, torch.float32).spread(_row0(lengths))
 
 
+@pytest.mark.parametrize("lengths,chunked", [
+    ([95], False), ([96], True), ([64] * 16, False), ([96] * 16, True), ([1111], True), ([1] * 24 + [128], False), ([1] * 24 + [144], True),
+    ([1] * 60 + [200], False), ([1] * 60 + [500], True), ([1] * 8, False), ([15, 300], True)])
+def test_delta_rule_walks_prompts_in_chunks_where_those_are_faster(lengths, chunked):
+    assert _delta_rule(16, 128, 128).chunked(_row0(lengths)) == chunked
+    assert not _delta_rule(16, 128, 128, torch.float32).chunked(_row0(lengths))
+
+
 @pytest.mark.parametrize("heads,dim,lengths,cuts", [
     (32, 64, [2048], True), (32, 64, [512] * 4, False), (32, 64, [129] * 2, False), (32, 64, [2048] * 2, True), (32, 64, [128], False),
     (32, 16, [129] * 4, False), (32, 16, [512] * 4, True), (32, 32, [129] * 4, False), (32, 32, [256] * 4, True),
