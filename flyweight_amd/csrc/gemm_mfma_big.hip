@@ -36,6 +36,7 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 #define BK 32                   // k per slab: an LDS row is 64 bytes, four 16-byte chunks
 #define BSTAGES 4               // slabs in LDS: one is multiplied, three are on their way
 #define BSLAB (BT * BK * 2)     // bytes of one operand's slab
+#define BK_MOST (1 << 22)
 #define BGROUP_M 4
 #define B_LOADS 4               // most wave-wide loads (16 rows of 64 bytes) per wave per operand per slab
 
@@ -69,7 +70,13 @@ struct BigTile {
     static constexpr int SLAB_LOADS = A_LOADS + W_LOADS;   // and for a slab of both operands
 };
 
-// K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way).
+// K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way), and at most BK_MOST (a
+// lane's place in a tile's 256 rows is 32 bits).
+//
+// Bound by the matrix cores at the clock that their power leaves (1.5 to 1.7 GHz in long runs): 72 to 76 % of the cycles in MFMAs,
+// the rest between the steps and at a tile's start and end. 2,048 x 8,192 gated x 2,048: 128.2 -> 117.5 us against reads and loads
+// spread over whole steps with 64-bit addresses in vector registers; 2,048 x 6,144: 51.9 -> 49.4; 8,192^3: 1,185 -> 1,296 TFLOP/s.
+// One barrier for two slabs (five stages) gave nothing more.
 // TN: 32-column product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144
 // features gives 192 tiles of 256 columns for 256 compute units, but exactly 256 tiles of 192).
 // TM: 32-row product tiles per wave, 4 (256 rows a tile) or 2 (128 rows).
@@ -94,7 +101,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int features = MODE == MB_SWIGLU ? BT / 2 : WIDE;
     const int m0 = pid_m * ROWS, n0 = pid_n * features;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
 
     // The copy: a wave-wide load writes 1,024 contiguous bytes of LDS, lane l its 16 bytes at
@@ -102,38 +109,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // stored permuted (chunk c of row r in slot c ^ ((r / 4) % 4)), so that the 16-byte operand
     // reads of 16 consecutive rows cover all 64 banks once (rows r, r + 4, r + 8, r + 12 would
     // otherwise share theirs). Lane l therefore ASKS for chunk (l % 4) ^ ((r / 4) % 4) of row
-    // r = l / 4 of its 16 rows.
-    const uint16_t* a_src[B_LOADS];
-    const uint16_t* w_src[B_LOADS];     // W_LOADS of them are used (with w_src[W_LOADS] the host pass emitted no launch stub)
+    // r = l / 4 of its 16 rows. Addresses are a base that the wave shares (the tile's first row; of a gated
+    // product's w the first gate or up row: a wave's loads of w are all of one kind), a 32-bit
+    // offset of the lane, and the slab's offset in a scalar register: a slab costs no vector arithmetic.
+    const int w_part = MODE == MB_SWIGLU && wave >= 2 ? 1 : 0;
+    const int w_first = MODE == MB_SWIGLU ? w_part * up_offset + n0 : n0;
+    const uint16_t* a_base = a + (size_t)m0 * K;
+    const uint16_t* w_base = w + (size_t)w_first * K;
+    uint32_t a_at[A_LOADS], w_at[B_LOADS];
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
         const int row = (wave * A_LOADS + i) * 16 + (lane >> 2);
         const int chunk = (lane & 3) ^ ((row >> 2) & 3);
-        int am = m0 + row;
-        am = am < M ? am : M - 1;                       // rows past the end are computed and dropped
-        a_src[i] = a + (size_t)am * K + chunk * 8;
+        a_at[i] = (uint32_t)(row < M - m0 ? row : M - m0 - 1) * (uint32_t)(2 * K) + chunk * 16;     // rows past the end are computed and dropped
     }
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
         const int row = (wave * W_LOADS + i) * 16 + (lane >> 2);
         const int chunk = (lane & 3) ^ ((row >> 2) & 3);
-        int wr;
-        if (MODE == MB_SWIGLU) wr = row < BT / 2 ? n0 + row : up_offset + n0 + row - BT / 2;
-        else wr = n0 + row;
-        const int limit = MODE == MB_SWIGLU ? (row < BT / 2 ? N : up_offset + N) : N;
-        wr = wr < limit ? wr : limit - 1;
-        w_src[i] = w + (size_t)wr * K + chunk * 8;
+        const int of_part = MODE == MB_SWIGLU ? row - w_part * (BT / 2) : row;
+        w_at[i] = (uint32_t)(of_part < N - n0 ? of_part : N - n0 - 1) * (uint32_t)(2 * K) + chunk * 16;
     }
-    auto request = [&](int slab) {
+    const fw_buffer a_rows = fw_make_buffer(a_base), w_rows = fw_make_buffer(w_base);
+    // loads from .. to - 1 of this wave's SLAB_LOADS for a slab
+    auto request_part = [&](int slab, int from, int to) {
         unsigned char* stage = lds + (slab % BSTAGES) * 2 * BSLAB;
-        const int k0 = slab * BK;
+        const int k0 = slab * (BK * 2);
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds(a_src[i] + k0, reinterpret_cast<uint32_t*>(stage + (wave * A_LOADS + i) * 1024), 16, 0, 0);
+            if (i >= from && i < to) fw_buffer_to_lds(a_rows, stage + (wave * A_LOADS + i) * 1024, a_at[i], k0);
 #pragma unroll
         for (int i = 0; i < W_LOADS; ++i)
-            __builtin_amdgcn_global_load_lds(w_src[i] + k0, reinterpret_cast<uint32_t*>(stage + BSLAB + (wave * W_LOADS + i) * 1024), 16, 0, 0);
+            if (A_LOADS + i >= from && A_LOADS + i < to) fw_buffer_to_lds(w_rows, stage + BSLAB + (wave * W_LOADS + i) * 1024, w_at[i], k0);
     };
+    auto request = [&](int slab) { request_part(slab, 0, SLAB_LOADS); };
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -200,10 +209,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
     // Four stages: while slab s is multiplied, slabs s + 1 .. s + 3 are in LDS or on their way.
     // The two k16 steps of a slab are software-pipelined by hand, because with one wave per SIMD
-    // nothing else hides the latency of LDS: the operands of the next step are read between the
-    // MFMAs of this step. In the middle of step 0 of slab s the wave makes sure that slab s + 1
-    // has landed (its own loads: vmcnt; everybody's: the barrier), which also tells that every
-    // wave has read the last of slab s, whose stage then takes slab s + 4.
+    // nothing else hides the latency of LDS: the operands of the next step are read behind the first
+    // MFMAs of this one, a read each, so that they have arrived when the step is through. Between
+    // the two steps the wave makes sure that slab s + 1 has landed (its own loads: vmcnt;
+    // everybody's: the barrier), which also tells that every wave has read the last of slab s,
+    // whose stage then takes slab s + 4. Its loads are issued behind every second one of the later MFMAs, half
+    // of them in the next slab's step 0: a compute unit takes a wave's load in 16 clocks, and four
+    // waves that each issued one behind every MFMA (32 clocks) stood still at them.
     const int steps = K / BK;
     for (int s = 0; s < BSTAGES && s < steps; ++s) request(s);
     wait_for_all_but((steps < BSTAGES ? steps : BSTAGES) - 1);
@@ -211,29 +223,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     Operands f0, f1;
     read(f0, 0, 0);
     int s = 0;
-    // steady state: slab s + 4 exists, nothing is conditional, so that each part is one run of
-    // instructions the scheduler can interleave
-    for (; s + BSTAGES < steps; ++s) {
-        // first half of step 0 of slab s, with the reads of step 1 between its MFMAs
-        arrived(f0);
-        read(f1, s, 1);
-        multiply(f0, 0, TM / 2);
-        FW_INTERLEAVE(TM / 2 * TN, 1, 0x100)    // (where the reads outnumber the MFMAs the rest is left to the scheduler)
+    constexpr int EARLY = SLAB_LOADS / 2;
+    // (where the reads outnumber the MFMAs the rest is left to the scheduler)
+#define FW_STEP_SCHEDULE()                                                                   \
+    FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)                          \
+    FW_INTERLEAVE((TM + TN < TM * TN ? (TM * TN - TM - TN) / 2 : 0), 2, 0x020)                \
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + BSTAGES < steps) {
+        read(f1, 0, 1);
+        multiply(f0, 0, TM);
+        FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)
         __builtin_amdgcn_sched_barrier(0);
-        arrived(f1);                                        // slab s has been read
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SLAB_LOADS) : "memory");   // slab s + 1 has landed; s + 2 and s + 3 may still fly
+        // a turn: step 1 of slab s and step 0 of slab s + 1, with the loads of slab s + 4. Nothing in it is
+        // conditional, so that each step is one run of instructions the scheduler can interleave
+        do {
+            arrived(f1);                                    // slab s has been read
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SLAB_LOADS) : "memory");   // slab s + 1 has landed; s + 2 and s + 3 may still fly
+            __builtin_amdgcn_s_barrier();
+            read(f0, s + 1, 0);
+            request_part(s + BSTAGES, 0, EARLY);
+            multiply(f1, 0, TM);
+            FW_STEP_SCHEDULE()
+            read(f1, s + 1, 1);
+            request_part(s + BSTAGES, EARLY, SLAB_LOADS);
+            multiply(f0, 0, TM);
+            FW_STEP_SCHEDULE()
+            ++s;
+        } while (s + BSTAGES < steps);
+        // step 1 of slab s = steps - 4, of which step 0 is done
+        arrived(f1);
+        wait_for_all_but(2);
         __builtin_amdgcn_s_barrier();
-        // second half, with the requests for slab s + 4 between its MFMAs
-        request(s + BSTAGES);
-        multiply(f0, TM / 2, TM / 2);
-        FW_INTERLEAVE(TM / 2 * TN, 1, 0x020)
-        __builtin_amdgcn_sched_barrier(0);
-        // step 1, with the reads of step 0 of slab s + 1 between its MFMAs
         read(f0, s + 1, 0);
         multiply(f1, 0, TM);
-        FW_INTERLEAVE(2 * TN, TM / 2, 0x100)
         __builtin_amdgcn_sched_barrier(0);
+        ++s;
     }
+#undef FW_STEP_SCHEDULE
     // the last slabs: nothing more to request
     for (; s < steps; ++s) {
         arrived(f0);
@@ -402,13 +428,13 @@ static BigPlan big_plan(int mode, int M, int N) {
 // whether that fills the chip); 0 if the kernel does not take the shape (K must be a multiple
 // of 32).
 extern "C" int fw_gemm_mfma_big_tiles(int mode, int M, int N, int K) {
-    if (K <= 0 || K % BK || M < 1 || N < 1) return 0;
+    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1) return 0;
     return big_plan(mode, M, N).tiles;
 }
 
 // The same with the tile's edges: what the caller needs to tell how much of the tiles the output fills.
 extern "C" int fw_gemm_mfma_big_plan(int mode, int M, int N, int K, int* rows, int* columns) {
-    if (K <= 0 || K % BK || M < 1 || N < 1) return 0;
+    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1) return 0;
     const BigPlan plan = big_plan(mode, M, N);
     if (rows) *rows = plan.rows;
     if (columns) *columns = plan.columns;
@@ -430,7 +456,7 @@ static int launch_planned(const BigPlan& plan, const void* a, const void* w, con
 // Same contract as fw_gemm_mfma.
 extern "C" int fw_gemm_mfma_big(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                                 int M, int N, int K, void* stream) {
-    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && K % BK == 0, "gemm_mfma_big: K (%d) must be a positive multiple of %d; M=%d N=%d", K, BK, M, N);
+    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && K <= BK_MOST && K % BK == 0, "gemm_mfma_big: K (%d) must be a positive multiple of %d; M=%d N=%d", K, BK, M, N);
     FW_REQUIRE(mode >= 0 && mode <= 2, "gemm_mfma_big: unknown mode %d", mode);
     FW_REQUIRE(mode != MB_ACCUMULATE || out_dtype == FW_F32, "gemm_mfma_big: accumulation needs a float32 destination");
     FW_REQUIRE(mode != MB_SWIGLU || ((out_dtype == FW_BF16 || out_dtype == FW_BF16_GEGLU) && bias == nullptr), "gemm_mfma_big: SwiGLU stores bfloat16 and takes no bias");
