@@ -74,9 +74,14 @@ __device__ __forceinline__ void fw_mfma_drain() {
 // A run of memory whose first byte all lanes of a wave share, for loads at a 32-bit offset of the lane and another that the wave
 // shares. 16 bytes a lane straight into LDS, lane l's at `lds` + 16 l (lds: the same for all lanes).
 typedef __amdgpu_buffer_rsrc_t fw_buffer;
-__device__ __forceinline__ fw_buffer fw_make_buffer(const void* first) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(first), 0, -1, 0x00020000);
+__device__ __forceinline__ fw_buffer fw_make_buffer(const void* first, uint32_t bytes = 0xffffffffu) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(first), 0, (int)bytes, 0x00020000);
 }
+// ... loads of places at or beyond its end give zero, stores there do nothing
+__device__ __forceinline__ float fw_buffer_load_float(fw_buffer from, uint32_t at) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
+}
+__device__ __forceinline__ void fw_buffer_store(fw_buffer to, uint32_t at, uint32_t word) { __builtin_amdgcn_raw_buffer_store_b32(word, to, at, 0, 0); }
 __device__ __forceinline__ void fw_buffer_to_lds(fw_buffer from, void* lds, uint32_t at, int shared_at) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)lds, 16, at, shared_at, 0, 0);
 }

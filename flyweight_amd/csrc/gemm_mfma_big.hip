@@ -37,6 +37,8 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 #define BSTAGES 4               // slabs in LDS: one is multiplied, three are on their way
 #define BSLAB (BT * BK * 2)     // bytes of one operand's slab
 #define BK_MOST (1 << 22)
+#define BN_MOST (1 << 20)       // 256 rows of the output lie below BOUNDS
+#define BOUNDS 0x80000000u
 #define BGROUP_M 4
 #define B_LOADS 4               // most wave-wide loads (16 rows of 64 bytes) per wave per operand per slab
 
@@ -71,7 +73,7 @@ struct BigTile {
 };
 
 // K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way), and at most BK_MOST (a
-// lane's place in a tile's 256 rows is 32 bits).
+// lane's place in a tile's 256 rows is 32 bits, as it is in the output: N at most BN_MOST).
 //
 // Bound by the matrix cores at the clock that their power leaves (1.5 to 1.7 GHz in long runs): 72 to 76 % of the cycles in MFMAs,
 // the rest between the steps and at a tile's start and end. 2,048 x 8,192 gated x 2,048: 128.2 -> 117.5 us against reads and loads
@@ -281,18 +283,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // D layout of the 32x32 product: lane holds column lane % 32; register r is row
     // 8 * (r / 4) + 4 * (lane / 32) + r % 4
     const int col = lane & 31, row_base = (lane >> 5) * 4;
-    // A tile that lies wholly inside the output (and an even N for the two-byte kinds) takes the
-    // quick way: no bounds, no branches, pointers stepped by rows, and for bfloat16 two
-    // neighbouring lanes swap one value each so that each stores a pair of columns as one word.
-    // With one workgroup per compute unit nothing runs beside the epilogue, so its length counts.
-    const bool inside = m0 + ROWS <= M && n0 + features <= N && (sizeof(TO) == 4 || (N & 1) == 0);
+    // The output leaves through a buffer that ends behind the tile's last row, so that rows past the end are dropped by its
+    // bounds and a lane of a column past the end by a place beyond them: no branch. (With a branch an element the last tile
+    // of a ragged product took 5 us longer than a whole one, with one only a row 4 us: 192 x 1,536 gated x 1,024 28.7 us
+    // against 22.1 for 256 rows.) For bfloat16 two neighbouring lanes swap one value each so that each stores a pair of
+    // columns as one word, which takes an even N. With one workgroup per compute unit nothing runs beside
+    // the epilogue, so its length counts.
+    constexpr int SIZE = sizeof(TO) == 4 ? 4 : 2;
+    const int rows_here = M - m0 < ROWS ? M - m0 : ROWS;
+    const fw_buffer to = fw_make_buffer(out + (size_t)m0 * N + n0, (uint32_t)(rows_here * N - n0) * SIZE);
+    const uint32_t row_step = (uint32_t)N * SIZE;
     const bool odd = lane & 1;
-    if constexpr (MODE == MB_SWIGLU) {
-        if (inside) {
+    const uint32_t first_row = (uint32_t)(wm * (TM * 32) + row_base);      // of this lane, of the tile
+    if (SIZE == 4 || (N & 1) == 0) {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                uint16_t* pair = reinterpret_cast<uint16_t*>(out) + (size_t)(m0 + wm * (TM * 32) + row_base) * N +
-                                 (n0 + wn * 64 + j * 32 + (col & ~1));
+        for (int j = 0; j < (MODE == MB_SWIGLU ? 2 : TN); ++j) {
+            const int c = (MODE == MB_SWIGLU ? wn * 64 : wn * (TN * 32)) + j * 32 + col;        // column of the tile
+            const bool there = n0 + c < N;
+            if constexpr (SIZE == 4) {
+                const float b = bias && there ? bias[n0 + c] : 0.0f;
+                const uint32_t at = there ? first_row * row_step + c * 4 : BOUNDS;
+                float old[MODE == MB_ACCUMULATE ? TM * 16 : 1];
+                if constexpr (MODE == MB_ACCUMULATE) {
+#pragma unroll
+                    for (int u = 0; u < TM * 16; ++u)
+                        old[u] = fw_buffer_load_float(to, at + (uint32_t)((u >> 4) * 32 + 8 * ((u & 15) >> 2) + (u & 3)) * row_step);
+                }
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        float value = acc[i][j][r] + b;
+                        if (MODE == MB_ACCUMULATE) value += old[i * 16 + r];
+                        fw_buffer_store(to, at + (uint32_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * row_step, __builtin_bit_cast(uint32_t, value));
+                    }
+            } else {
+                const float b = MODE != MB_SWIGLU && bias && there ? bias[n0 + c] : 0.0f;
+                const uint32_t at = there ? (first_row + (odd ? 1 : 0)) * row_step + (c & ~1) * 2 : BOUNDS;
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -300,80 +327,41 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
                             const int r = 4 * q + 2 * h;        // rows 8 q + 2 h and the one below, of row tile i
-                            const float upper = fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r];
-                            const float lower = fw_gate_of<TO>(acc[i][j][r + 1], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r + 1];
+                            float upper, lower;
+                            if constexpr (MODE == MB_SWIGLU) {
+                                upper = fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r];
+                                lower = fw_gate_of<TO>(acc[i][j][r + 1], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r + 1];
+                            } else {
+                                upper = fw_before_store<TO>(acc[i][j][r] + b);
+                                lower = fw_before_store<TO>(acc[i][j][r + 1] + b);
+                            }
                             const float got = from_neighbour(odd ? upper : lower);
                             const uint32_t word = odd ? pack_bf16x2(got, lower) : pack_bf16x2(upper, got);
-                            const int row = i * 32 + 8 * q + 2 * h + (odd ? 1 : 0);
-                            *reinterpret_cast<uint32_t*>(pair + (size_t)row * N) = word;
+                            fw_buffer_store(to, at + (uint32_t)(i * 32 + 8 * q + 2 * h) * row_step, word);
                         }
             }
-            return;
         }
+        return;
+    }
+    // two bytes an element and an odd N
+    if constexpr (SIZE == 2) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + wn * 64 + j * 32 + col;
+        for (int j = 0; j < (MODE == MB_SWIGLU ? 2 : TN); ++j) {
+            const int n = n0 + (MODE == MB_SWIGLU ? wn * 64 : wn * (TN * 32)) + j * 32 + col;
             if (n >= N) continue;
+            const float b = MODE != MB_SWIGLU && bias ? bias[n] : 0.0f;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int m = m0 + wm * (TM * 32) + i * 32 + 8 * (r >> 2) + row_base + (r & 3);
-                    if (m < M) store_from_float(out, (size_t)m * N + n, fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r]);
+                    const int m = m0 + (int)first_row + i * 32 + 8 * (r >> 2) + (r & 3);
+                    if (m >= M) continue;
+                    if constexpr (MODE == MB_SWIGLU)
+                        store_from_float(out, (size_t)m * N + n, fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r]);
+                    else
+                        store_from_float(out, (size_t)m * N + n, acc[i][j][r] + b);
                 }
         }
-        return;
-    }
-    if (inside) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int n = n0 + wn * (TN * 32) + j * 32 + col;
-            const float b = bias ? bias[n] : 0.0f;
-            if constexpr (sizeof(TO) == 4) {
-                float* column = reinterpret_cast<float*>(out) + (size_t)(m0 + wm * (TM * 32) + row_base) * N + n;
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        float* to = column + (size_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * N;
-                        float value = acc[i][j][r] + b;
-                        if (MODE == MB_ACCUMULATE) value += *to;
-                        *to = value;
-                    }
-            } else {
-                uint16_t* pair = reinterpret_cast<uint16_t*>(out) + (size_t)(m0 + wm * (TM * 32) + row_base) * N + (n & ~1);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const int r = 4 * q + 2 * h;
-                            const float upper = fw_before_store<TO>(acc[i][j][r] + b), lower = fw_before_store<TO>(acc[i][j][r + 1] + b);
-                            const float got = from_neighbour(odd ? upper : lower);
-                            const uint32_t word = odd ? pack_bf16x2(got, lower) : pack_bf16x2(upper, got);
-                            *reinterpret_cast<uint32_t*>(pair + (size_t)(i * 32 + 8 * q + 2 * h + (odd ? 1 : 0)) * N) = word;
-                        }
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int n = n0 + wn * (TN * 32) + j * 32 + col;
-        if (n >= N) continue;
-        const float b = bias ? bias[n] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = m0 + wm * (TM * 32) + i * 32 + 8 * (r >> 2) + row_base + (r & 3);
-                if (m >= M) continue;
-                const size_t at = (size_t)m * N + n;
-                float value = acc[i][j][r] + b;
-                if (MODE == MB_ACCUMULATE) value += load_as_float(out, at);
-                store_from_float(out, at, value);
-            }
     }
 }
 
@@ -401,10 +389,9 @@ static int launch_big(const void* a, const void* w, const float* bias, void* out
 // The tile a storing or accumulating product is cut into: 256 or 128 rows by 256 or 192 columns,
 // whichever takes the least time by this count: rounds of tiles over the chip's 256 compute units
 // times the tile's area, a tile of 128 rows counting a quarter more than its area (it moves more
-// bytes per flop). Gated products (SwiGLU) keep 256 x 256, and accumulating ones 256 rows: their
-// epilogue reads the old values where nothing hides the read, and twice the tiles for the same
-// output pay that twice as often (2,048 x 3,072 x 2,048: storing 50.9 -> 35.6 us with tiles of
-// 128 x 192, accumulating 51.6 -> 58.5 us).
+// bytes per flop). Gated products (SwiGLU) keep 256 x 256. (2,048 x 3,072 x 2,048: storing 50.9 -> 35.6 us with tiles of
+// 128 x 192. Accumulating ones asked for each old value behind the store of the one before it and lost with twice the tiles; asked
+// for a column of the tile at a time they gain as well.)
 struct BigPlan {
     int rows, columns, tiles;
 };
@@ -412,7 +399,7 @@ static BigPlan big_plan(int mode, int M, int N) {
     if (mode == MB_SWIGLU) return {BT, BT / 2, fw_ceil_div(M, BT) * fw_ceil_div(N, BT / 2)};
     BigPlan best = {0, 0, 0};
     long long best_cost = 0;
-    for (int rows = BT; rows >= (mode == MB_STORE ? BT / 2 : BT); rows /= 2)
+    for (int rows = BT; rows >= BT / 2; rows /= 2)
         for (int columns = BT; columns >= 192; columns -= 64) {
             const long long tiles = (long long)fw_ceil_div(M, rows) * fw_ceil_div(N, columns);
             const long long cost = fw_ceil_div(tiles, 256) * (rows / 32) * (columns / 32) * (rows == BT ? 4 : 5);
@@ -428,13 +415,13 @@ static BigPlan big_plan(int mode, int M, int N) {
 // whether that fills the chip); 0 if the kernel does not take the shape (K must be a multiple
 // of 32).
 extern "C" int fw_gemm_mfma_big_tiles(int mode, int M, int N, int K) {
-    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1) return 0;
+    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1 || N > BN_MOST) return 0;
     return big_plan(mode, M, N).tiles;
 }
 
 // The same with the tile's edges: what the caller needs to tell how much of the tiles the output fills.
 extern "C" int fw_gemm_mfma_big_plan(int mode, int M, int N, int K, int* rows, int* columns) {
-    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1) return 0;
+    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1 || N > BN_MOST) return 0;
     const BigPlan plan = big_plan(mode, M, N);
     if (rows) *rows = plan.rows;
     if (columns) *columns = plan.columns;
@@ -444,19 +431,17 @@ extern "C" int fw_gemm_mfma_big_plan(int mode, int M, int N, int K, int* rows, i
 template <int MODE, typename TO>
 static int launch_planned(const BigPlan& plan, const void* a, const void* w, const float* bias, void* out, int M, int N, int K,
                           hipStream_t stream) {
-    if (plan.rows == BT || MODE != MB_STORE)
+    if (plan.rows == BT)
         return plan.columns == BT ? launch_big<MODE, TO, 4, 4>(a, w, bias, out, M, N, K, stream)
                                   : launch_big<MODE, TO, 3, 4>(a, w, bias, out, M, N, K, stream);
-    if constexpr (MODE == MB_STORE)
-        return plan.columns == BT ? launch_big<MODE, TO, 4, 2>(a, w, bias, out, M, N, K, stream)
-                                  : launch_big<MODE, TO, 3, 2>(a, w, bias, out, M, N, K, stream);
-    return -1;
+    return plan.columns == BT ? launch_big<MODE, TO, 4, 2>(a, w, bias, out, M, N, K, stream)
+                              : launch_big<MODE, TO, 3, 2>(a, w, bias, out, M, N, K, stream);
 }
 
 // Same contract as fw_gemm_mfma.
 extern "C" int fw_gemm_mfma_big(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                                 int M, int N, int K, void* stream) {
-    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && K <= BK_MOST && K % BK == 0, "gemm_mfma_big: K (%d) must be a positive multiple of %d; M=%d N=%d", K, BK, M, N);
+    FW_REQUIRE(M >= 1 && N > 0 && N <= BN_MOST && K > 0 && K <= BK_MOST && K % BK == 0, "gemm_mfma_big: K (%d) must be a positive multiple of %d; M=%d N=%d", K, BK, M, N);
     FW_REQUIRE(mode >= 0 && mode <= 2, "gemm_mfma_big: unknown mode %d", mode);
     FW_REQUIRE(mode != MB_ACCUMULATE || out_dtype == FW_F32, "gemm_mfma_big: accumulation needs a float32 destination");
     FW_REQUIRE(mode != MB_SWIGLU || ((out_dtype == FW_BF16 || out_dtype == FW_BF16_GEGLU) && bias == nullptr), "gemm_mfma_big: SwiGLU stores bfloat16 and takes no bias");

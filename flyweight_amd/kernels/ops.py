@@ -554,8 +554,7 @@ def rows_fit(mode: int, M: int, N: int, K: int) -> bool:
 def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                w_tiled: Optional[torch.Tensor] = None) -> None:
     """bfloat16 operands on the matrix cores: up to 16 rows of a short K the skinny kernel; up to 64 rows, and with weights in operand tiles as long as its tiles are one
-    round over the chip, the product whose waves split K; the tiled ones beyond (large tiles where they fill the chip, K cut into slices where
-    even the small tiles are too few)."""
+    round over the chip, the product whose waves split K; the tiled ones beyond."""
     M, K = a.shape
     if M <= DECODE_MAX_ROWS and skinny_takes(M, N, K):
         _check(library().fw_gemm_skinny(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
@@ -566,34 +565,80 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
         else:
             gemm_medium_into(a, w, bias, target, out_code, mode, N, w_tiled=w_tiled)
         return
-    if M > BIG_MIN_ROWS and library().fw_gemm_mfma_big_tiles(mode, M, N, K) >= BIG_TILES_MIN:
-        entry = library().fw_gemm_mfma_big      # enough 256 x 256 tiles to fill the chip
-    elif K >= (DEEP_MIN_K if mode == 1 else DEEP_MIN_K_STORE) and _deep_columns(mode, M, N, K):
-        # whole rounds of one tile per compute unit: the waves split K
-        _check(library().fw_gemm_mfma_deep(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K,
-                                           _deep_columns(mode, M, N, K), _stream()))
+    kind, columns = tiled_plan(mode, M, N, K)
+    if kind == "deep":
+        _check(library().fw_gemm_mfma_deep(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, columns, _stream()))
         return
-    elif _deep_columns_few_rows(mode, M, N, K, one_round=True):
-        _check(library().fw_gemm_mfma_deep(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K,
-                                           _deep_columns_few_rows(mode, M, N, K), _stream()))
+    if kind == "split":
+        need_bytes, need_counters = _split_needs(mode, M, N, K)
+        workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
+        counters = _medium_counters(a.device, need_counters)
+        _check(library().fw_gemm_mfma_split(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _p(workspace),
+                                            ctypes.c_size_t(need_bytes), _p(counters), counters.numel(), _stream()))
         return
-    elif M > BIG_MIN_ROWS and _big_tiles_store_well(mode, M, N, K):
-        entry = library().fw_gemm_mfma_big      # fewer large tiles than compute units, but every other way takes two rounds
-    elif _deep_columns_few_rows(mode, M, N, K):
-        _check(library().fw_gemm_mfma_deep(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K,
-                                           _deep_columns_few_rows(mode, M, N, K), _stream()))
-        return
-    else:
-        need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
-        _check(library().fw_gemm_mfma_split_plan(mode, M, N, K, ctypes.byref(need_bytes), ctypes.byref(need_counters)))
-        if need_bytes.value:                    # fewer tiles than compute units: K is cut into slices
-            workspace = torch.empty(need_bytes.value // 4, dtype=torch.float32, device=a.device)
-            counters = _medium_counters(a.device, need_counters.value)
-            _check(library().fw_gemm_mfma_split(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _p(workspace),
-                                                ctypes.c_size_t(need_bytes.value), _p(counters), counters.numel(), _stream()))
-            return
-        entry = library().fw_gemm_mfma
+    entry = library().fw_gemm_mfma_big if kind == "big" else library().fw_gemm_mfma
     _check(entry(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
+
+
+def _split_needs(mode: int, M: int, N: int, K: int):
+    """(bytes of workspace, counters) of the product that cuts K over workgroups; zeros where it does not take the shape."""
+    need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
+    _check(library().fw_gemm_mfma_split_plan(mode, M, N, K, ctypes.byref(need_bytes), ctypes.byref(need_counters)))
+    return need_bytes.value, need_counters.value
+
+
+# What the tiled products take, us: start + rounds * round + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of their
+# tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to 600
+# shapes of 65 to 2,048 rows by 1,024 to 8,192 features over K 1,024 to 8,192, every weight from memory, to 2 to 9 % (mean square).
+_TIME_DEEP = {0: {128: (1.1, 10.8, 4.4, 2.5), 64: (1.4, 5.0, 3.0, 1.6)}, 1: {128: (1.0, 12.7, 4.4, 2.5), 64: (1.4, 5.9, 3.0, 1.6)}}
+_TIME_TILES = {0: {128: (0.8, 5.8, 3.9, 6.4), 64: (8.7, -1.8, 5.9, 0.5)}, 1: {128: (-2.8, 13.0, 3.5, 6.9), 64: (7.3, -0.1, 6.2, 1.0)},
+               2: {64: (8.3, -0.1, 7.9, 1.3)}}
+_TIME_BIG_GATED = (-1.2, 8.6, 13.8, 8.7)
+_TIME_BIG = {0: {128: (1.9, 1.9, 0.33, 0.23), 256: (5.3, 5.3, 0.05, 0.38)},     # by the tile's rows; walk and fill by 32 x 32 of its area
+             1: {128: (2.3, 2.3, 0.32, 0.25), 256: (7.5, 7.5, -0.02, 0.47)}}
+_TIME_SPLIT = {0: (8.0, 1.2, 6.1), 1: (8.0, 1.2, 6.1), 2: (6.5, 3.5, 10.0)}      # start, a slice's part in the sum at the end, 1,024 k of a slice
+
+
+def _tiled_time(tiles: int, K: int, start: float, each_round: float, walk: float, fill: float) -> float:
+    rounds = -(-tiles // DEEP_ROUND)
+    return start + rounds * each_round + K / 1024 * (rounds * walk + tiles / DEEP_ROUND * fill)
+
+
+@functools.lru_cache(maxsize=4096)
+def tiled_plan(mode: int, M: int, N: int, K: int):
+    """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
+    256 columns), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through registers), "split" (those with K cut over
+    workgroups). The least estimated time decides: over the shapes that it was fitted to 10 % less in the geometric mean than by
+    fixed numbers of tiles (storing, before -> now: 1,111 rows by 2,048 features over K 8,192 97 -> 57 us, over 2,048 29 -> 24; 640 by 2,048 over
+    2,048 22 -> 14; 1,300 by 3,072 over 2,048 44 -> 28; gated, 801 by 1,536 over 2,048 35 -> 26; 1,111 by 4,608 over 2,048 63 -> 46).
+    What adds into at most 2,048 features stays with the tiles whose waves split K wherever those fill their rounds: the fastest
+    or level with it from K 2,048 on (over K 1,024 large tiles would take 17 us instead of 22 for 2,048 rows)."""
+    lib = library()
+    if mode == 1 and K >= DEEP_MIN_K and N <= DEEP_NARROW and _deep_columns(mode, M, N, K):
+        return "deep", _deep_columns(mode, M, N, K)
+    wide, narrow = -(-M // 128) * -(-N // 128), -(-M // 128) * -(-N // 64)
+    columns = 64 if mode == 2 or wide < DEEP_ROUND or (wide == DEEP_ROUND and K < LONG_K) else 128        # as fw_gemm_mfma chooses
+    times = {("tiles", 0): _tiled_time(narrow if columns == 64 else wide, K, *_TIME_TILES[mode][columns])}
+    if mode != 2:
+        for columns in (128, 64):
+            tiles = lib.fw_gemm_mfma_deep_tiles(mode, M, N, K, columns)
+            if tiles:
+                times["deep", columns] = _tiled_time(tiles, K, *_TIME_DEEP[mode][columns])
+    if M > BIG_MIN_ROWS:
+        rows, columns = ctypes.c_int(0), ctypes.c_int(0)
+        tiles = lib.fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns))
+        if tiles and mode == 2:
+            times["big", 0] = _tiled_time(tiles, K, *_TIME_BIG_GATED)
+        elif tiles:
+            start, each_round, walk, fill = _TIME_BIG[mode][rows.value]
+            area = rows.value * columns.value / 1024
+            times["big", 0] = _tiled_time(tiles, K, start, each_round, walk * area, fill * area)
+    need_bytes, tiles = _split_needs(mode, M, N, K)
+    if need_bytes:
+        slices = need_bytes // (tiles * 128 * (128 if mode == 2 else 64) * 4)
+        start, each, walk = _TIME_SPLIT[mode]
+        times["split", 0] = start + each * slices + walk * K / 1024 / slices * -(-tiles * slices // DEEP_ROUND)
+    return min(times, key=times.get)
 
 
 MEDIUM_MAX_ROWS = 64
@@ -604,9 +649,9 @@ MEDIUM_MAX_ROWS = 64
 # 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27), and so it does with a long K where the others' tiles
 # fill their round (fw_gemm_rows_round_fits).
 ROWS_MAX = 1024
-BIG_TILES_MIN = 192      # 256 x 256 tiles from which the large-tile prompt product is used (256 compute units)
+BIG_TILES_MIN = 192      # large tiles that are nearly a round over the 256 compute units
+DEEP_NARROW = 2048       # features up to which a product that adds into the residual prefers the tiles whose waves split K
 DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)
-DEEP_MIN_K_STORE = 4096   # storing: no old values travel during the exchange at a tile's end, a short K gains nothing
 DEEP_ROUND = 256          # tiles of a round: one per compute unit
 DEEP_FILL = 0.85          # least share of the rounds' places that the tiles must fill (640 narrow tiles, 0.83: 193 vs 189 us)
 # adding into the residual, 2,048 features: 144 wide tiles (1,152 rows) K 8,192 72 vs 103 us, K 2,048 28 vs 35 us; 160
@@ -635,23 +680,7 @@ DEEP_FEW_TILES_WIDE = 192   # tiles of 128 columns from which those are taken, e
 DEEP_FEW_TILES = 96       # tiles of 64 columns from which those are
 
 
-BIG_TILES_MIN_STORE = 96      # large tiles from which a storing product takes them, if the output fills
-BIG_FILL_STORE = 0.95         # at least this share of them
-
-
-def _big_tiles_store_well(mode: int, M: int, N: int, K: int) -> bool:
-    """A storing product that no kernel serves in one round of small tiles takes the large
-    tiles from 96 of them on if they are well filled: 768 x 3,072 (K 1,024) 18.7 -> 14.9 us,
-    512 x 4,608 21.1 -> 14.6 us, 1,024 x 3,072 (K 2,048) 29.5 -> 25.0 us; 2,048 x 1,024 (96 tiles
-    of 192 columns, an eighth of them outside the output) would lose, 14.1 -> 17.5 us."""
-    if mode != 0:
-        return False
-    rows, columns = ctypes.c_int(0), ctypes.c_int(0)
-    tiles = library().fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns))
-    return tiles >= BIG_TILES_MIN_STORE and M * N >= BIG_FILL_STORE * tiles * rows.value * columns.value
-
-
-def _deep_columns_few_rows(mode: int, M: int, N: int, K: int, one_round: bool = False) -> int:
+def _deep_columns_few_rows(mode: int, M: int, N: int, K: int) -> int:
     """A few hundred rows (decode steps of that many requests, short prompts) give the 128 x 128
     tiles of the register-staged product less than a round over the chip; the tiles whose waves
     split K bring their operands straight into LDS, three slabs ahead, and a workgroup alone on
@@ -666,7 +695,7 @@ def _deep_columns_few_rows(mode: int, M: int, N: int, K: int, one_round: bool = 
     narrow = library().fw_gemm_mfma_deep_tiles(mode, M, N, K, 64)
     if mode == 0 and DEEP_FEW_TILES_WIDE <= wide <= DEEP_ROUND:
         return 128
-    if DEEP_FEW_TILES <= narrow <= (1 if one_round else 2) * DEEP_ROUND:
+    if DEEP_FEW_TILES <= narrow <= 2 * DEEP_ROUND:
         return 64
     return 0
 
