@@ -414,7 +414,8 @@ int fw_moe_arrange(const int32_t* chosen, int32_t* expert_begin, int32_t* place_
 // out[place] = a[place_row ? place_row[place] : place] . w[expert of place]^T; w [experts][N][K], or with
 // gated [experts][2 N][K] (gate rows, then up rows) and out = silu(gate) * up, or with a glu_limit > 0 the clamped
 // unit g sigmoid(glu_alpha g) (u + glu_shift), g = min(gate, limit), u = clamp(up, -limit, limit). out [places][N].
-int fw_grouped_gemm(const void* a, int a_dtype, const int32_t* place_row, const void* w, int w_dtype,
+// a holds a_rows rows; place_row names no other.
+int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                     const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
                     float glu_limit, float glu_alpha, float glu_shift, void* stream);
 // x[r] += sum_j weight[r][j] * y[pair_place[r][j]], j in order, and with b (null: none) + sigmoid(gate[r * gate_stride]) b[r]; float32

@@ -25,6 +25,7 @@
 // (native/include/flyweight_v2_native_kernels.hpp:233-311).
 #include "fw_common.h"
 #include "fw_kernels.h"
+#include "grouped.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
@@ -63,6 +64,13 @@ __device__ __forceinline__ float from_neighbour(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, true));
 }
 
+// A grouped product: places begin[e] .. begin[e + 1] - 1 are expert e's rows (row place_row[p] of a, or row p), w holds the experts' weights one
+// behind the other.
+struct BigGroups {
+    const int32_t *place_row, *begin;
+    int experts;
+};
+
 template <int TM, int TN>
 struct BigTile {
     static constexpr int ROWS = 2 * TM * 32;               // rows of a tile
@@ -82,26 +90,41 @@ struct BigTile {
 // TN: 32-column product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144
 // features gives 192 tiles of 256 columns for 256 compute units, but exactly 256 tiles of 192).
 // TM: 32-row product tiles per wave, 4 (256 rows a tile) or 2 (128 rows).
-template <int MODE, typename TO, int TN, int TM>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void gemm_mfma_big_kernel(
+template <int MODE, typename TO, int TN, int TM, int STAGES, bool GROUPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3 ? 2 : 1, STAGES == 3 ? 2 : 1))) void gemm_mfma_big_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const float* __restrict__ bias,
-    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset) {
+    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [stage][a slab | w slab]
-    const int total = tiles_m * tiles_n;
-    const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= total) return;
-    const int width = BGROUP_M * tiles_n;
-    const int group = logical / width;
-    const int first_m = group * BGROUP_M;
-    const int group_size = tiles_m - first_m < BGROUP_M ? tiles_m - first_m : BGROUP_M;
-    const int pid_m = first_m + (logical % width) % group_size;
-    const int pid_n = (logical % width) / group_size;
-    static_assert((TN == 4 && TM == 4) || (MODE != MB_SWIGLU && (TN == 3 || TN == 4) && (TM == 2 || TM == 4)),
-                  "narrower or lower tiles: store and accumulate only");
     constexpr int ROWS = BigTile<TM, TN>::ROWS, WIDE = BigTile<TM, TN>::WIDE;
     constexpr int A_LOADS = BigTile<TM, TN>::A_LOADS, W_LOADS = BigTile<TM, TN>::W_LOADS, SLAB_LOADS = BigTile<TM, TN>::SLAB_LOADS;
+    constexpr int A_SLAB = ROWS * BK * 2, STAGE = A_SLAB + WIDE * BK * 2;       // bytes
     const int features = MODE == MB_SWIGLU ? BT / 2 : WIDE;
-    const int m0 = pid_m * ROWS, n0 = pid_n * features;
+    static_assert(MODE != MB_SWIGLU || TN == 4, "the gated tile holds 128 gate and 128 up rows");
+    int m0, n0;
+    const int32_t* groups_rows = nullptr;
+    if constexpr (GROUPED) {
+        const GroupedTile tile = grouped_tile(groups.begin, groups.experts, ROWS, tiles_n);
+        const int expert = tile.expert;
+        if (expert < 0) return;
+        m0 = tile.row_tile * ROWS;
+        n0 = tile.column_tile * features;
+        const int first = groups.begin[expert];
+        M = groups.begin[expert + 1] - first;           // rows of this expert: places first .. first + M - 1
+        w += (size_t)expert * (MODE == MB_SWIGLU ? 2 : 1) * N * K;
+        out += (size_t)first * N;
+        if (groups.place_row) groups_rows = groups.place_row + first;
+        else a += (size_t)first * K;
+    } else {
+        const int total = tiles_m * tiles_n;
+        const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+        if (logical >= total) return;
+        const int width = BGROUP_M * tiles_n;
+        const int group = logical / width;
+        const int first_m = group * BGROUP_M;
+        const int group_size = tiles_m - first_m < BGROUP_M ? tiles_m - first_m : BGROUP_M;
+        m0 = (first_m + (logical % width) % group_size) * ROWS;
+        n0 = (logical % width) / group_size * features;
+    }
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -116,14 +139,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // offset of the lane, and the slab's offset in a scalar register: a slab costs no vector arithmetic.
     const int w_part = MODE == MB_SWIGLU && wave >= 2 ? 1 : 0;
     const int w_first = MODE == MB_SWIGLU ? w_part * up_offset + n0 : n0;
-    const uint16_t* a_base = a + (size_t)m0 * K;
+    const uint16_t* a_base = GROUPED && groups_rows ? a : a + (size_t)m0 * K;
     const uint16_t* w_base = w + (size_t)w_first * K;
     uint32_t a_at[A_LOADS], w_at[B_LOADS];
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
         const int row = (wave * A_LOADS + i) * 16 + (lane >> 2);
         const int chunk = (lane & 3) ^ ((row >> 2) & 3);
-        a_at[i] = (uint32_t)(row < M - m0 ? row : M - m0 - 1) * (uint32_t)(2 * K) + chunk * 16;     // rows past the end are computed and dropped
+        uint32_t from = row < M - m0 ? row : M - m0 - 1;        // rows past the end are computed and dropped
+        if (GROUPED && groups_rows) from = groups_rows[m0 + (int)from];
+        a_at[i] = from * (uint32_t)(2 * K) + chunk * 16;
     }
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
@@ -135,14 +160,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const fw_buffer a_rows = fw_make_buffer(a_base), w_rows = fw_make_buffer(w_base);
     // loads from .. to - 1 of this wave's SLAB_LOADS for a slab
     auto request_part = [&](int slab, int from, int to) {
-        unsigned char* stage = lds + (slab % BSTAGES) * 2 * BSLAB;
+        unsigned char* stage = lds + (slab % STAGES) * STAGE;
         const int k0 = slab * (BK * 2);
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i)
             if (i >= from && i < to) fw_buffer_to_lds(a_rows, stage + (wave * A_LOADS + i) * 1024, a_at[i], k0);
 #pragma unroll
         for (int i = 0; i < W_LOADS; ++i)
-            if (A_LOADS + i >= from && A_LOADS + i < to) fw_buffer_to_lds(w_rows, stage + BSLAB + (wave * W_LOADS + i) * 1024, w_at[i], k0);
+            if (A_LOADS + i >= from && A_LOADS + i < to) fw_buffer_to_lds(w_rows, stage + A_SLAB + (wave * W_LOADS + i) * 1024, w_at[i], k0);
     };
     auto request = [&](int slab) { request_part(slab, 0, SLAB_LOADS); };
 
@@ -172,8 +197,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         bf16x8 fa[TM], fb[TN];
     };
     auto read = [&](Operands& f, int slab, int t) {
-        const unsigned char* sa = lds + (slab % BSTAGES) * 2 * BSLAB;
-        const unsigned char* sb = sa + BSLAB;
+        const unsigned char* sa = lds + (slab % STAGES) * STAGE;
+        const unsigned char* sb = sa + A_SLAB;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
             f.fa[i] = *reinterpret_cast<const bf16x8*>(sa + (a_row0 + 32 * i) * (BK * 2) + slot[t]);
@@ -219,8 +244,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // of them in the next slab's step 0: a compute unit takes a wave's load in 16 clocks, and four
     // waves that each issued one behind every MFMA (32 clocks) stood still at them.
     const int steps = K / BK;
-    for (int s = 0; s < BSTAGES && s < steps; ++s) request(s);
-    wait_for_all_but((steps < BSTAGES ? steps : BSTAGES) - 1);
+    for (int s = 0; s < STAGES && s < steps; ++s) request(s);
+    wait_for_all_but((steps < STAGES ? steps : STAGES) - 1);
     __builtin_amdgcn_s_barrier();
     Operands f0, f1;
     read(f0, 0, 0);
@@ -231,30 +256,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)                          \
     FW_INTERLEAVE((TM + TN < TM * TN ? (TM * TN - TM - TN) / 2 : 0), 2, 0x020)                \
     __builtin_amdgcn_sched_barrier(0);
-    if (s + BSTAGES < steps) {
+    if (s + STAGES < steps) {
         read(f1, 0, 1);
         multiply(f0, 0, TM);
         FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)
         __builtin_amdgcn_sched_barrier(0);
-        // a turn: step 1 of slab s and step 0 of slab s + 1, with the loads of slab s + 4. Nothing in it is
+        // a turn: step 1 of slab s and step 0 of slab s + 1, with the loads of slab s + STAGES. Nothing in it is
         // conditional, so that each step is one run of instructions the scheduler can interleave
         do {
             arrived(f1);                                    // slab s has been read
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SLAB_LOADS) : "memory");   // slab s + 1 has landed; s + 2 and s + 3 may still fly
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * SLAB_LOADS) : "memory");   // slab s + 1 has landed; those behind it may still fly
             __builtin_amdgcn_s_barrier();
             read(f0, s + 1, 0);
-            request_part(s + BSTAGES, 0, EARLY);
+            request_part(s + STAGES, 0, EARLY);
             multiply(f1, 0, TM);
             FW_STEP_SCHEDULE()
             read(f1, s + 1, 1);
-            request_part(s + BSTAGES, EARLY, SLAB_LOADS);
+            request_part(s + STAGES, EARLY, SLAB_LOADS);
             multiply(f0, 0, TM);
             FW_STEP_SCHEDULE()
             ++s;
-        } while (s + BSTAGES < steps);
-        // step 1 of slab s = steps - 4, of which step 0 is done
+        } while (s + STAGES < steps);
+        // step 1 of slab s = steps - STAGES, of which step 0 is done
         arrived(f1);
-        wait_for_all_but(2);
+        wait_for_all_but(STAGES - 2);
         __builtin_amdgcn_s_barrier();
         read(f0, s + 1, 0);
         multiply(f1, 0, TM);
@@ -294,6 +319,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const fw_buffer to = fw_make_buffer(out + (size_t)m0 * N + n0, (uint32_t)(rows_here * N - n0) * SIZE);
     const uint32_t row_step = (uint32_t)N * SIZE;
     const bool odd = lane & 1;
+    // (the grouped product has the unit of its form for few places, bit for bit)
+    auto unit = [](float g) { return GROUPED ? silu_big(g) : silu_quick(g); };
     const uint32_t first_row = (uint32_t)(wm * (TM * 32) + row_base);      // of this lane, of the tile
     if (SIZE == 4 || (N & 1) == 0) {
 #pragma unroll
@@ -329,8 +356,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                             const int r = 4 * q + 2 * h;        // rows 8 q + 2 h and the one below, of row tile i
                             float upper, lower;
                             if constexpr (MODE == MB_SWIGLU) {
-                                upper = fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r];
-                                lower = fw_gate_of<TO>(acc[i][j][r + 1], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r + 1];
+                                upper = fw_gate_of<TO>(acc[i][j][r], unit) * acc[i][j + 2][r];
+                                lower = fw_gate_of<TO>(acc[i][j][r + 1], unit) * acc[i][j + 2][r + 1];
                             } else {
                                 upper = fw_before_store<TO>(acc[i][j][r] + b);
                                 lower = fw_before_store<TO>(acc[i][j][r + 1] + b);
@@ -357,7 +384,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                     const int m = m0 + (int)first_row + i * 32 + 8 * (r >> 2) + (r & 3);
                     if (m >= M) continue;
                     if constexpr (MODE == MB_SWIGLU)
-                        store_from_float(out, (size_t)m * N + n, fw_gate_of<TO>(acc[i][j][r], [](float g) { return silu_quick(g); }) * acc[i][j + 2][r]);
+                        store_from_float(out, (size_t)m * N + n, fw_gate_of<TO>(acc[i][j][r], unit) * acc[i][j + 2][r]);
                     else
                         store_from_float(out, (size_t)m * N + n, acc[i][j][r] + b);
                 }
@@ -365,15 +392,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
 }
 
-template <int MODE, typename TO, int TN = 4, int TM = 4>
-static int launch_big(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, hipStream_t stream) {
-    const int features = MODE == MB_SWIGLU ? BT / 2 : 2 * TN * 32;
-    const int tiles_m = fw_ceil_div(M, 2 * TM * 32), tiles_n = fw_ceil_div(N, features);
+template <int MODE, typename TO, int TN, int TM, int STAGES, bool GROUPED>
+static int launch_tiles(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, int tiles_m, const BigGroups& groups,
+                        hipStream_t stream) {
+    const int tiles_n = fw_ceil_div(N, MODE == MB_SWIGLU ? BT / 2 : BigTile<TM, TN>::WIDE);
     const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n, 8);
-    const int lds_bytes = BSTAGES * 2 * BSLAB;
+    const int lds_bytes = STAGES * (BigTile<TM, TN>::ROWS + BigTile<TM, TN>::WIDE) * BK * 2;
     static bool configured = false;     // per instantiation
     if (!configured) {
-        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM>,
+        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, STAGES, GROUPED>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (status != hipSuccess) {
             fw_set_error("gemm_mfma_big: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(status));
@@ -381,9 +408,23 @@ static int launch_big(const void* a, const void* w, const float* bias, void* out
         }
         configured = true;
     }
-    gemm_mfma_big_kernel<MODE, TO, TN, TM><<<per_xcd * 8, 256, lds_bytes, stream>>>(
-        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N);
+    gemm_mfma_big_kernel<MODE, TO, TN, TM, STAGES, GROUPED><<<per_xcd * 8, 256, lds_bytes, stream>>>(
+        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups);
     return 0;
+}
+template <int MODE, typename TO, int TN = 4, int TM = 4>
+static int launch_big(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, hipStream_t stream) {
+    return launch_tiles<MODE, TO, TN, TM, BSTAGES, false>(a, w, bias, out, M, N, K, fw_ceil_div(M, BigTile<TM, TN>::ROWS), BigGroups(), stream);
+}
+
+// The grouped product of fw_grouped_gemm on tiles of 128 places by 256 rows of W, for K a multiple of 32 and a of less than 4 GB.
+bool fw_grouped_big_takes(int a_rows, int N, int K) { return K % BK == 0 && K <= BK_MOST && N <= BN_MOST && 2ll * a_rows * K <= 0xffff0000ll; }
+int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
+                          int experts, int N, int K, hipStream_t stream) {
+    const BigGroups groups = {place_row, expert_begin, experts};
+    const int tiles_m = places / 128 + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
+    if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+    return launch_tiles<MB_STORE, float, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
 }
 
 // The tile a storing or accumulating product is cut into: 256 or 128 rows by 256 or 192 columns,

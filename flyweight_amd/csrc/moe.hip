@@ -11,6 +11,7 @@
 // depends on the row alone, never on what else is in the step.
 #include "fw_common.h"
 #include "fw_kernels.h"
+#include "grouped.h"
 
 // ---- routing ---------------------------------------------------------------------------------------
 // A wave per row. The logits (float32 [rows][experts], bias added here) stay in registers, SLOTS a lane: 1, 2 or 4 where
@@ -391,9 +392,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const TA* __restrict_
 //           and every workgroup streams rows of W that no other reads.
 // GATED: W is [2 N][K], gate rows then up rows; a tile takes as many gate rows as up rows of the same
 // features, a wave holds gate and up of one element in one lane and stores silu(gate) * up.
-// Which tile a workgroup has: an expert with n places has ceil(n / rows) tiles of places, each times the
-// tiles of features; a wave finds its expert by a prefix sum of 64 experts' tile counts at a time. The grid
-// holds as many tiles as there can be at most; a workgroup beyond the last leaves.
+// Which tile a workgroup has: grouped.h. The grid holds as many tiles as there can be at most; a workgroup beyond the last leaves.
 // A place's sum over k is formed in one order whatever the tile's shape and whoever shares the tile.
 typedef __attribute__((ext_vector_type(8))) __bf16 gg_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float gg_f32x16;
@@ -410,7 +409,7 @@ __device__ __forceinline__ float gg_silu(float g) {
 template <bool GATED, bool BIG, int NJ, typename TO>
 __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     const uint16_t* __restrict__ a, const int32_t* __restrict__ place_row, const uint16_t* __restrict__ w,
-    const int32_t* __restrict__ expert_begin, TO* __restrict__ out, int experts, int N, int K, int tiles_m, int tiles_n, int per_xcd,
+    const int32_t* __restrict__ expert_begin, TO* __restrict__ out, int experts, int N, int K, int tiles_n,
     const GatedUnit unit) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     constexpr int TMR = BIG ? 128 : 32;                 // places of a tile
@@ -420,43 +419,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     constexpr int A_CHUNKS = TMR / 32, W_CHUNKS = BN / 32;
     constexpr int A_SLAB = TMR * GGM_ROW_BYTES, W_SLAB = BN * GGM_ROW_BYTES;
     static_assert(!GATED || NJ == 2, "the gated tile holds gate and up side by side");
-    const int total = tiles_m * tiles_n;
-    const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= total) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
-    // Workgroups are numbered expert by expert, within an expert feature tile by feature tile, and within that
-    // over the expert's tiles of places: the two or three tiles that read the same rows of W run side by side,
-    // and an expert's places (a megabyte or so) stay in the L2 of the XCD that works through the expert.
-    int expert = -1, tile_in_expert = 0, pid_n = 0;
-    {
-        int before = 0;
-        for (int e0 = 0; e0 < experts; e0 += 64) {
-            const int e = e0 + lane;
-            const int mine = e < experts ? (expert_begin[e + 1] - expert_begin[e] + TMR - 1) / TMR : 0;
-            int upto = mine * tiles_n;
-#pragma unroll
-            for (int offset = 1; offset < 64; offset <<= 1) {
-                const int other = __shfl_up(upto, offset, 64);
-                if (lane >= offset) upto += other;
-            }
-            const unsigned long long holds = __ballot(logical < before + upto);
-            if (holds) {
-                const int at = __ffsll((long long)holds) - 1;
-                const int tiles_here = __shfl(mine, at, 64);
-                const int rest = logical - (before + __shfl(upto, at, 64) - tiles_here * tiles_n);
-                expert = e0 + at;
-                tile_in_expert = rest % tiles_here;
-                pid_n = rest / tiles_here;
-                break;
-            }
-            before += __shfl(upto, 63, 64);
-        }
-    }
+    const GroupedTile tile = grouped_tile(expert_begin, experts, TMR, tiles_n);
+    const int expert = tile.expert;
     if (expert < 0) return;
-    const int first = expert_begin[expert] + tile_in_expert * TMR, end = expert_begin[expert + 1];
+    const int first = expert_begin[expert] + tile.row_tile * TMR, end = expert_begin[expert + 1];
     const int features = GATED ? BN / 2 : BN;
-    const int n0 = pid_n * features;
+    const int n0 = tile.column_tile * features;
     const int wm = BIG ? wave >> 1 : 0, wn = BIG ? wave & 1 : wave;
     const uint16_t* we = w + (size_t)expert * (GATED ? 2 : 1) * N * K;
 
@@ -620,11 +590,16 @@ static int grouped_mfma_launch(const void* a, const int32_t* place_row, const vo
         configured = true;
     }
     grouped_gemm_mfma_kernel<GATED, BIG, NJ, TO><<<per_xcd * 8, 256, lds_bytes, stream>>>(
-        (const uint16_t*)a, place_row, (const uint16_t*)w, expert_begin, (TO*)out, experts, N, K, (int)tiles_m, (int)tiles_n, per_xcd, unit);
+        (const uint16_t*)a, place_row, (const uint16_t*)w, expert_begin, (TO*)out, experts, N, K, (int)tiles_n, unit);
     return 0;
 }
 
-extern "C" int fw_grouped_gemm(const void* a, int a_dtype, const int32_t* place_row, const void* w, int w_dtype,
+// gemm_mfma_big.hip
+bool fw_grouped_big_takes(int a_rows, int N, int K);
+int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
+                          int experts, int N, int K, hipStream_t stream);
+
+extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                                const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
                                float glu_limit, float glu_alpha, float glu_shift, void* stream) {
     const GatedUnit unit = {glu_limit, glu_alpha, glu_shift};
@@ -638,7 +613,9 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, const int32_t* place_
         (out_dtype == FW_F32 || (out_dtype == FW_BF16 && gated))) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
-        if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
+        if (big && glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && fw_grouped_big_takes(a_rows, N, K))
+            status = fw_launch_grouped_big(a, place_row, w, expert_begin, out, gated, places, experts, N, K, s);
+        else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
                                 : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);
         else status = big ? grouped_mfma_launch<false, true, 2, float>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
                           : grouped_mfma_launch<false, false, 1, float>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);

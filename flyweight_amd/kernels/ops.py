@@ -1963,7 +1963,7 @@ def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: torch.Te
     elif a.shape[0] < places:
         raise KernelError("grouped_gemm: fewer rows than places")
     out = torch.empty((places, N), dtype=out_dtype, device=a.device)
-    _check(library().fw_grouped_gemm(_p(a), _code(a.dtype), _p(place_row), _p(w), _code(w.dtype), _p(expert_begin), _p(out),
+    _check(library().fw_grouped_gemm(_p(a), _code(a.dtype), a.shape[0], _p(place_row), _p(w), _code(w.dtype), _p(expert_begin), _p(out),
                                      _code(out_dtype), int(gated), int(places), experts, N, K, *_glu(glu if gated else None), _stream()))
     return out
 
