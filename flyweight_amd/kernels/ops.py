@@ -588,15 +588,16 @@ def _split_needs(mode: int, M: int, N: int, K: int):
 
 
 # What the tiled products take, us: start + rounds * round + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of their
-# tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to 600
-# shapes of 65 to 2,048 rows by 1,024 to 8,192 features over K 1,024 to 8,192, every weight from memory, to 2 to 9 % (mean square).
+# tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to
+# 1,000 shapes of 65 to 3,900 rows by 32 to 8,192 features over K 256 to 8,192, the large weights from memory, to 2 to 9 % (mean square).
 _TIME_DEEP = {0: {128: (1.1, 10.8, 4.4, 2.5), 64: (1.4, 5.0, 3.0, 1.6)}, 1: {128: (1.0, 12.7, 4.4, 2.5), 64: (1.4, 5.9, 3.0, 1.6)}}
 _TIME_TILES = {0: {128: (0.8, 5.8, 3.9, 6.4), 64: (8.7, -1.8, 5.9, 0.5)}, 1: {128: (-2.8, 13.0, 3.5, 6.9), 64: (7.3, -0.1, 6.2, 1.0)},
                2: {64: (8.3, -0.1, 7.9, 1.3)}}
 _TIME_BIG_GATED = (-1.2, 8.6, 13.8, 8.7)
 _TIME_BIG = {0: {128: (1.9, 1.9, 0.33, 0.23), 256: (5.3, 5.3, 0.05, 0.38)},     # by the tile's rows; walk and fill by 32 x 32 of its area
              1: {128: (2.3, 2.3, 0.32, 0.25), 256: (7.5, 7.5, -0.02, 0.47)}}
-_TIME_SPLIT = {0: (8.0, 1.2, 6.1), 1: (8.0, 1.2, 6.1), 2: (6.5, 3.5, 10.0)}      # start, a slice's part in the sum at the end, 1,024 k of a slice
+# ... with K cut: start, a slice's part in the sum at the end, 1,024 k of a slice in each round, 256 workgroups
+_TIME_SPLIT = {0: (8.1, 0.3, 6.2, 2.4), 1: (8.1, 0.3, 6.2, 2.4), 2: (8.2, 0.7, 10.7, 3.8)}
 
 
 def _tiled_time(tiles: int, K: int, start: float, each_round: float, walk: float, fill: float) -> float:
@@ -636,8 +637,9 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
     need_bytes, tiles = _split_needs(mode, M, N, K)
     if need_bytes:
         slices = need_bytes // (tiles * 128 * (128 if mode == 2 else 64) * 4)
-        start, each, walk = _TIME_SPLIT[mode]
-        times["split", 0] = start + each * slices + walk * K / 1024 / slices * -(-tiles * slices // DEEP_ROUND)
+        start, each, walk, fill = _TIME_SPLIT[mode]
+        workgroups = tiles * slices
+        times["split", 0] = start + each * slices + walk * K / 1024 / slices * -(-workgroups // DEEP_ROUND) + fill * workgroups / DEEP_ROUND
     return min(times, key=times.get)
 
 
