@@ -8,7 +8,7 @@
 //    v_mfma_f32_32x32x16_bf16, its 256 accumulators in the accumulation registers; one wave per
 //    SIMD, so the overlap of loads, LDS reads and MFMAs is inside the wave;
 //  * 256 x 32 slabs of both operands travel from global memory STRAIGHT into LDS
-//    (global_load_lds_dwordx4: no staging registers, which the accumulators leave no room for),
+//    (buffer_load_dwordx4 .. lds: no staging registers, which the accumulators leave no room for),
 //    three slabs ahead of the one being multiplied, four stages, one barrier per slab; rows are
 //    not padded, their chunks are stored permuted against bank conflicts;
 //  * workgroups are numbered so that each XCD works on a compact group of tiles.
@@ -18,10 +18,10 @@
 // Such a tile moves more bytes per flop through LDS and the memory path, so it is used only where
 // it fills the chip better.
 //
-// It needs enough tiles to fill the chip (the caller checks): 2,048 rows by 8,192 gated features
+// It serves where its tiles fill the chip (the caller compares the products' estimated times): 2,048 rows by 8,192 gated features
 // are 512 tiles. Epilogues as the other products: store, add into the residual stream, SwiGLU
 // (a tile holds 128 gate and the 128 up features of the same columns; a lane holds both of an
-// element). The reference's prompt GEMM is a 64x64 tile of plain FMAs without tensor cores
+// element). The experts' grouped product of a prompt runs in the same loop, its tiles numbered as grouped.h says. The reference's prompt GEMM is a 64x64 tile of plain FMAs without tensor cores
 // (native/include/flyweight_v2_native_kernels.hpp:233-311).
 #include "fw_common.h"
 #include "fw_kernels.h"
@@ -417,7 +417,10 @@ static int launch_big(const void* a, const void* w, const float* bias, void* out
     return launch_tiles<MODE, TO, TN, TM, BSTAGES, false>(a, w, bias, out, M, N, K, fw_ceil_div(M, BigTile<TM, TN>::ROWS), BigGroups(), stream);
 }
 
-// The grouped product of fw_grouped_gemm on tiles of 128 places by 256 rows of W, for K a multiple of 32 and a of less than 4 GB.
+// The grouped product of fw_grouped_gemm on tiles of 128 places by 256 rows of W, for K a multiple of 32 and a of less than 4 GB. Bound by
+// the experts' weights from memory (600 MB for both products of 32 experts of 1,536 features: 127 us) and by tiles that an expert's last places fill partly.
+// Two workgroups share a compute unit (three stages of 24 KB each), so that one multiplies while the other starts, ends or waits. 2,048 rows, 4 of 32
+// experts, gated 1,536 over 2,048: 158 us; with four stages and one workgroup 175, on tiles of 256 places 186; through registers (moe.hip) 241.
 bool fw_grouped_big_takes(int a_rows, int N, int K) { return K % BK == 0 && K <= BK_MOST && N <= BN_MOST && 2ll * a_rows * K <= 0xffff0000ll; }
 int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
                           int experts, int N, int K, hipStream_t stream) {

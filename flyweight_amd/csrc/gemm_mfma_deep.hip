@@ -11,7 +11,7 @@
 // finishes four of the sixteen 32 x 32 product tiles (the parts added in the order of the waves).
 //
 //  * slabs of 128 rows x 64 k of both operands travel from global memory straight into LDS
-//    (global_load_lds_dwordx4), three slabs ahead of the one being multiplied, four stages of
+//    (buffer_load_dwordx4 .. lds), three slabs ahead of the one being multiplied, four stages of
 //    32 KB; a row is 128 bytes, its eight 16-byte chunks stored permuted (chunk c of row r in slot
 //    c ^ ((r / 2) % 8)) so that the operand reads of sixteen consecutive rows, two rows to 256
 //    bytes, cover all 64 banks once (with c ^ (r % 8) rows r and r + 8 met in the same banks:

@@ -118,7 +118,7 @@ def test_products_beyond_64_rows_are_dealt_to_waves_where_that_is_faster(mode, M
     (0, 320, 6144, 2048, ("deep", 128)), (0, 320, 1024, 8192, ("split", 0)), (0, 128, 3072, 8192, ("split", 0)), (0, 300, 2500, 520, ("tiles", 0)),
     (0, 100, 8192, 32, ("tiles", 0)), (2, 801, 1536, 2048, ("tiles", 0)), (2, 1111, 4608, 2048, ("big", 0)), (2, 640, 1536, 2048, ("split", 0)),
     (0, 1111, 64, 4096, ("split", 0)), (0, 2048, 64, 1024, ("deep", 64)), (2, 300, 64, 2048, ("split", 0)),
-    (2, 2048, 8192, 2048, ("big", 0)), (2, 128, 8192, 1024, ("tiles", 0)), (2, 2048, 2048, 2048, ("big", 0)),
+    (2, 2048, 8192, 2048, ("big", 0)), (2, 128, 8192, 1024, ("tiles", 0)), (2, 2048, 2048, 2048, ("tiles", 0)),
     (1, 2048, 2048, 8192, ("deep", 128)), (1, 2048, 1024, 1024, ("deep", 64)), (1, 512, 2048, 2048, ("deep", 64)), (1, 256, 2048, 8192, ("split", 0)),
     (1, 2048, 8192, 2048, ("big", 0))])
 def test_tiled_products_take_the_tiles_that_were_the_fastest(mode, M, N, K, plan):
