@@ -426,6 +426,8 @@ int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w
                           int experts, int N, int K, hipStream_t stream) {
     const BigGroups groups = {place_row, expert_begin, experts};
     const int tiles_m = places / 128 + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
+    // (what the product through registers, whose tiles have half the features, would refuse is refused here too)
+    FW_REQUIRE((long long)tiles_m * fw_ceil_div(N, gated ? BT / 4 : BT / 2) < (1ll << 30), "grouped_gemm: too many tiles");
     if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
     return launch_tiles<MB_STORE, float, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
 }
