@@ -296,13 +296,15 @@ extern "C" int fw_gemm_mfma_deep_tiles(int mode, int M, int N, int K, int column
 // fw_gemm_mfma's contract for modes 0 and 1, on tiles of 128 rows and `columns` (128 or 64) columns.
 extern "C" int fw_gemm_mfma_deep(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                                  int M, int N, int K, int columns, void* stream) {
-    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && K <= DK_MOST && K % DK == 0, "gemm_mfma_deep: K (%d) must be a positive multiple of %d; M=%d N=%d", K, DK, M, N);
+    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && K % DK == 0, "gemm_mfma_deep: K (%d) must be a positive multiple of %d; M=%d N=%d", K, DK, M, N);
     FW_REQUIRE(mode == MD_STORE || mode == MD_ACCUMULATE, "gemm_mfma_deep: mode %d is not served", mode);
     FW_REQUIRE(columns == 128 || columns == 64, "gemm_mfma_deep: tiles have 128 or 64 columns, not %d", columns);
     FW_REQUIRE(mode != MD_ACCUMULATE || out_dtype == FW_F32, "gemm_mfma_deep: accumulation needs a float32 destination");
     FW_REQUIRE(out_dtype == FW_F32 || out_dtype == FW_BF16 || (out_dtype == FW_BF16_GELU && mode == MD_STORE), "gemm_mfma_deep: unknown out dtype %d", out_dtype);
     FW_REQUIRE(((uintptr_t)a % 16 == 0) && ((uintptr_t)w % 16 == 0), "gemm_mfma_deep: operands must be 16-byte aligned");
     FW_REQUIRE((long long)fw_ceil_div(M, DT) * fw_ceil_div(N, 64) < (1ll << 30), "gemm_mfma_deep: too many tiles");
+    // rows too long for a lane's 32-bit places (8 MB) go through registers, with 64-bit addresses
+    if (K > DK_MOST) return fw_gemm_mfma(a, w, bias, out, out_dtype, mode, M, N, K, stream);
     hipStream_t s = (hipStream_t)stream;
     int status;
     if (columns == 128) {
