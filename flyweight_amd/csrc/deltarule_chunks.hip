@@ -51,12 +51,12 @@ __device__ __forceinline__ float delta_softplus(float z) {
     sum = fmaf(y * s, sum, s);
     return fmaf(2.0f, sum, fmaxf(z, 0.0f));
 }
-// 1 / (1 + e^-x), the quotient as a reciprocal and one step of Newton's method (as exact as the division; below -87 the divisor would pass
-// the largest float, so x stops there: the result is 1.6e-38 instead of less)
+// 1 / (1 + e^-x), the quotient as a reciprocal and one step of Newton's method (as exact as the division). Below -88.7 the divisor is
+// infinite and the step would be infinity times zero: the result is 0, as the division's.
 __device__ __forceinline__ float delta_sigmoid(float x) {
-    const float d = 1.0f + expf(fminf(-x, 87.0f));
+    const float d = 1.0f + expf(-x);
     const float r = __builtin_amdgcn_rcpf(d);
-    return x != x ? x : fmaf(fmaf(-d, r, 1.0f), r, r);
+    return r == 0.0f ? r : fmaf(fmaf(-d, r, 1.0f), r, r);
 }
 
 // What up to REACH tokens from token j on see of its key: over the channels at .. at + 3, at + stride .., summed over the sixteen lanes of

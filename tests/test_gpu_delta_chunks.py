@@ -57,3 +57,28 @@ def test_prompts_in_chunks(heads, kv_heads, dim, vdim, taps, per_head, lengths, 
                 S, o = plain.delta_rule_step(S, q[t, group], k[t, group], v[t, head], beta[t, head], g[t, head])
                 np.testing.assert_allclose(out[r0 + t, head], o, rtol=0, atol=2e-5 * max(1.0, np.abs(o).max()))
             np.testing.assert_allclose(after[slot, head], S, rtol=0, atol=2e-5 * max(1.0, np.abs(S).max()))
+
+
+def test_inputs_far_below_zero_pass_nothing():
+    """silu(x) goes to -0 as x falls: a convolution's sum of -1e38 writes nothing and turns no key, one of -90 as good as nothing."""
+    from flyweight_amd.kernels import ops
+    rng = np.random.default_rng(5)
+    rows, dim, vdim = 40, 64, 16
+    channels = 2 * dim + vdim
+    proj = rng.normal(size=(rows, channels + 1)).astype(np.float32)
+    values = np.float32([-3e38, -1e38, -1e30, -1e6, -200, -104, -90, -89, -88.7, -88, -87.5, -87, -80, -60, -20, 1])
+    proj[:, 2 * dim:channels] = values
+    proj[::3, 5], proj[::4, dim + 7] = -1e38, -3e38
+    a, A_log, dt_bias = rng.normal(size=(rows, dim)).astype(np.float32), np.zeros(1, np.float32), np.zeros(dim, np.float32)
+    state = dev(np.zeros((1, 1, vdim, dim)))
+    out = ops.delta_chunks(dev(proj), channels, dev(a), dev(np.ones((channels, 1))), dev(np.zeros((1, channels, 0))), dev(A_log), dev(dt_bias), state,
+                           ints([0, rows]), ints([0]), 1, 1, 1, dim, vdim).cpu().numpy()
+    x = proj.astype(np.float64)
+    with np.errstate(over="ignore"):
+        y = x[:, :channels] / (1.0 + np.exp(-x[:, :channels]))
+    q, k = plain.unit(y[:, :dim]) * dim ** -0.5, plain.unit(y[:, dim:2 * dim])
+    S = np.zeros((dim, vdim))
+    for t in range(rows):
+        S, o = plain.delta_rule_step(S, q[t], k[t], y[t, 2 * dim:], plain.sigmoid(x[t, channels]), np.exp(-plain.softplus(a[t].astype(np.float64))))
+        # (a sum of fifty factors is 2^-18 off; below 1e-34 a float loses bits, and below 1e-38 all of them)
+        assert (np.abs(out[t] - o) <= 2e-5 * np.abs(y[0, 2 * dim:]) + 1e-34).all()
