@@ -82,6 +82,7 @@ __device__ __forceinline__ float fw_buffer_load_float(fw_buffer from, uint32_t a
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0));
 }
 __device__ __forceinline__ void fw_buffer_store(fw_buffer to, uint32_t at, uint32_t word) { __builtin_amdgcn_raw_buffer_store_b32(word, to, at, 0, 0); }
+__device__ __forceinline__ void fw_buffer_store(fw_buffer to, uint32_t at, uint16_t half) { __builtin_amdgcn_raw_buffer_store_b16(half, to, at, 0, 0); }
 __device__ __forceinline__ void fw_buffer_to_lds(fw_buffer from, void* lds, uint32_t at, int shared_at) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)lds, 16, at, shared_at, 0, 0);
 }

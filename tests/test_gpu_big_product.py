@@ -60,3 +60,35 @@ def test_a_width_beyond_its_offsets_goes_elsewhere(ops):
     assert ops.library().fw_gemm_mfma_big_tiles(0, 4096, 8192, 1 << 22) > 0
     assert ops.library().fw_gemm_mfma_big_tiles(0, 4096, 8192, (1 << 22) + 32) == 0
     assert ops.library().fw_gemm_mfma_big_plan(0, 4096, 8192, (1 << 22) + 32, ctypes.byref(rows), ctypes.byref(columns)) == 0
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("M,N", [(300, 185), (130, 184), (129, 1), (1, 2), (700, 8193)])
+def test_two_byte_outputs_of_any_width_and_place(ops, M, N, shift):
+    """Pairs of columns as one word where rows and output lie at multiples of four bytes, else every element by itself; the places around
+    the output stay as they are."""
+    K = 96
+    a, w = draw(M, K), draw(2 * N, K, seed=1)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2))
+    A, W, B = a.to(DEV), w.to(DEV), bias.to(DEV)
+    exact, limit = a.double() @ w.double().T, bound(a, w)
+    gate, up = exact[:, :N], exact[:, N:]
+
+    def run(mode, code, with_bias):
+        room = torch.full((M * N + 8,), 7.0, device=DEV, dtype=torch.bfloat16)
+        out = room[2 + shift:2 + shift + M * N]
+        ops._check(ops.library().fw_gemm_mfma_big(ops._p(A), ops._p(W), ops._p(B) if with_bias else None, ops._p(out), code, mode, M, N, K, ops._stream()))
+        assert (room[:2 + shift] == 7.0).all() and (room[2 + shift + M * N:] == 7.0).all()
+        return out.view(M, N).cpu().double()
+
+    summed = exact[:, :N] + bias.double()
+    assert ((run(STORE, BF16, True) - summed).abs() <= limit[:, :N] + 2.0 ** -8 * summed.abs()).all()
+    # (gelu's slope is below 1.13; its short error function is within 1.5e-7, times half of z)
+    want = torch.nn.functional.gelu(summed)
+    assert ((run(STORE, ops.BF16_GELU, True) - want).abs() <= 1.13 * limit[:, :N] + 1e-6 + 1e-6 * summed.abs() + 2.0 ** -8 * want.abs()).all()
+    slack = 1.1 * limit[:, :N] * (up.abs() + limit[:, N:]) + gate.abs() * limit[:, N:] + 2.0 ** -133
+    want = gate * torch.sigmoid(gate) * up
+    assert ((run(GATED, BF16, False) - want).abs() <= slack + 2.0 ** -7 * want.abs()).all()
+    # (the slope of the tanh form is below 1.13 as well)
+    want = torch.nn.functional.gelu(gate, approximate="tanh") * up
+    assert ((run(GATED, ops.BF16_GEGLU, False) - want).abs() <= 1.03 * slack + 1e-5 * (gate * up).abs() + 2.0 ** -7 * want.abs()).all()
