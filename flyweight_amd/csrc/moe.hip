@@ -386,8 +386,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const TA* __restrict_
 // registers (two slabs ahead of the one multiplied) -> LDS (one ahead), two LDS buffers, one barrier an
 // iteration, LDS rows padded to 144 bytes. Two shapes of tile:
 //   BIG     128 places x 128 rows of W; four waves as 2 x 2, each 64 x 64. For steps in which an expert
-//           has hundreds of places (prompts), a clamped unit or a K that is no multiple of 32 (others go straight to LDS:
-//           fw_launch_grouped_big).
+//           has hundreds of places (prompts) and that do not go straight to LDS (fw_grouped_gemm_large_fits): a clamped
+//           unit, a K that is no multiple of 32, few tiles over a long K.
 //   small    32 places x (128 NJ) rows of W; four waves side by side, each 32 x (32 NJ). For steps of
 //           few places an expert (decoding): the product is bound by how fast the experts' weights stream,
 //           and every workgroup streams rows of W that no other reads.
@@ -595,10 +595,19 @@ static int grouped_mfma_launch(const void* a, const int32_t* place_row, const vo
     return 0;
 }
 
-// gemm_mfma_big.hip
-bool fw_grouped_big_takes(int a_rows, int N, int K);
-int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
-                          int experts, int N, int K, hipStream_t stream);
+// Whether a product of many places an expert (bfloat16, the plain unit) goes straight to LDS on the large tiles: with a short K, and where
+// they are about a round over the chip (every expert's last tile half full in the mean). Fewer of them over a long K leave the streaming of W
+// to too few workgroups: 8 experts, 200 / 384 / 1,111 places, 1,024 features over K 2,048 28 / 29 / 29 us against 25 / 26 / 28 through registers, 32
+// experts of 100 places, 288 over 16,832 311 against 173; over K 576 to 960 they win down to 8 tiles (10.5 us against 11.6, 14.3 against 15.3).
+// 140 tiles over K 1,952 35.5 against 42.8, but 148 over 3,232 53.7 against 45.5. Tiles that are half padding win while they are less than a round (10.9 us
+// against 12.8) and lose beyond (32 features of 128 experts, 41,352 places 12.3 against 11.5).
+extern "C" int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int experts, int N, int K) {
+    if ((long long)places < 48ll * experts || !fw_grouped_big_takes(a_rows, N, K)) return 0;
+    const int features = gated ? 128 : 256;
+    const long long tiles = (places / 128 + experts / 2) * (long long)fw_ceil_div(N, features);
+    if (2 * N <= features && tiles >= 256) return 0;
+    return K <= 1024 || tiles >= 192;
+}
 
 extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                                const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
@@ -615,7 +624,7 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
         (out_dtype == FW_F32 || (out_dtype == FW_BF16 && gated))) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
-        if (big && glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && fw_grouped_big_takes(a_rows, N, K))
+        if (glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K))
             status = fw_launch_grouped_big(a, place_row, w, expert_begin, out, gated, places, experts, N, K, s);
         else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
                                 : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);
