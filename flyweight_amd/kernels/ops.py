@@ -587,59 +587,68 @@ def _split_needs(mode: int, M: int, N: int, K: int):
     return need_bytes.value, need_counters.value
 
 
-# What the tiled products take, us: start + rounds * round + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of their
-# tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to
-# 1,000 shapes of 65 to 3,900 rows by 32 to 8,192 features over K 256 to 8,192, the large weights from memory, to 2 to 9 % (mean square).
-_TIME_DEEP = {0: {128: (1.1, 10.8, 4.4, 2.5), 64: (1.4, 5.0, 3.0, 1.6)}, 1: {128: (1.0, 12.7, 4.4, 2.5), 64: (1.4, 5.9, 3.0, 1.6)}}
-_TIME_TILES = {0: {128: (0.8, 5.8, 3.9, 6.4), 64: (8.7, -1.8, 5.9, 0.5)}, 1: {128: (-2.8, 13.0, 3.5, 6.9), 64: (7.3, -0.1, 6.2, 1.0)},
-               2: {64: (8.3, -0.1, 7.9, 1.3)}}
-_TIME_BIG_GATED = (1.8, 8.6, 13.8, 8.7)      # 3 us more than fitted: at a tie the small tiles, which use every compute unit, are faster inside a step
-_TIME_BIG = {0: {128: (1.9, 1.9, 0.33, 0.23), 256: (5.3, 5.3, 0.05, 0.38)},     # by the tile's rows; walk and fill by 32 x 32 of its area
-             1: {128: (2.3, 2.3, 0.32, 0.25), 256: (7.5, 7.5, -0.02, 0.47)}}
-# ... with K cut: start, a slice's part in the sum at the end, 1,024 k of a slice in each round, 256 workgroups
-_TIME_SPLIT = {0: (8.1, 0.3, 6.2, 2.4), 1: (8.1, 0.3, 6.2, 2.4), 2: (8.2, 0.7, 10.7, 3.8)}
+# What the tiled products take, us: start + rounds * round + tiles / 256 * tile + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of
+# their tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to 2,200
+# shapes of 65 to 16,384 rows by 32 to 16,384 features over K 32 to 12,288, the weights from memory, to 4 to 12 % (mean square), with no part
+# below zero: parts that were, fitted to shapes of few rounds, made many rounds over a short K free.
+_TIME_DEEP = {0: {128: (3.2, 9.1, 1.4, 4.76, 3.28), 64: (2.6, 3.9, 1.2, 3.56, 1.54)},
+              1: {128: (2.7, 10.4, 1.9, 4.84, 2.64), 64: (2.4, 4.5, 1.3, 3.62, 1.26)}}
+_TIME_DEEP_FEW_ROWS = 1.25     # of a long K where at most three rows of tiles share what they read of the weights (256 x 2,112 over 7,872: 53 us, by the parts alone 38)
+# ... through registers, where two workgroups share a compute unit, two parts more: for each pair of rounds, for 1,024 k of it
+_TIME_TILES = {0: {128: (5.1, 0.0, 1.5, 6.32, 2.84, 6.2, 0.92), 64: (0.0, 0.3, 0.8, 3.64, 1.42, 6.2, 2.54)},
+               1: {128: (0.3, 0.0, 6.1, 5.87, 1.06, 11.7, 3.78), 64: (0.0, 1.1, 1.3, 2.55, 2.66, 5.1, 3.81)},
+               2: {64: (3.4, 0.7, 0.6, 5.46, 1.69, 2.6, 3.74)}}
+_TIME_RAGGED = 3.0       # ... adding into features that end inside a tile of 64, and the same with K cut: a branch and a load an element
+_TIME_BIG = {0: {128: (1.9, 2.0, 2.9, 0.337, 0.197), 256: (2.4, 4.4, 4.2, 0.174, 0.239)},     # by the tile's rows; walk and fill by 32 x 32 of its area
+             1: {128: (0.6, 3.6, 3.9, 0.341, 0.192), 256: (0.7, 3.9, 13.9, 0.203, 0.21)}, 2: {256: (2.2, 4.4, 2.1, 0.247, 0.144)}}
+_TIME_BIG_ODD = 4.0      # a round more of gated products with an odd number of features, which leave element by element
+# ... with K cut: start, a slice's part in the sum at the end, 1,024 k of a slice in each round and for 256 workgroups, 256 workgroups
+_TIME_SPLIT = {0: (8.3, 0.44, 4.6, 3.4, 1.5), 1: (7.3, 0.55, 4.8, 4.55, 4.0), 2: (8.3, 0.77, 8.7, 3.96, 2.5)}
 
 
-def _tiled_time(tiles: int, K: int, start: float, each_round: float, walk: float, fill: float) -> float:
-    rounds = -(-tiles // DEEP_ROUND)
-    return start + rounds * each_round + K / 1024 * (rounds * walk + tiles / DEEP_ROUND * fill)
+def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: float, walk: float, fill: float, each_pair: float = 0.0,
+                walk_pair: float = 0.0) -> float:
+    rounds, pairs = -(-tiles // DEEP_ROUND), -(-tiles // (2 * DEEP_ROUND))
+    share = tiles / DEEP_ROUND
+    return (start + rounds * each_round + share * each_tile + pairs * each_pair
+            + K / 1024 * (rounds * walk + share * fill + pairs * walk_pair))
 
 
 @functools.lru_cache(maxsize=4096)
 def tiled_plan(mode: int, M: int, N: int, K: int):
     """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
     256 columns), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through registers), "split" (those with K cut over
-    workgroups). The least estimated time decides: over the shapes that it was fitted to 10 % less in the geometric mean than by
-    fixed numbers of tiles (storing, before -> now: 1,111 rows by 2,048 features over K 8,192 97 -> 57 us, over 2,048 29 -> 24; 640 by 2,048 over
-    2,048 22 -> 14; 1,300 by 3,072 over 2,048 44 -> 28; gated, 801 by 1,536 over 2,048 35 -> 26; 1,111 by 4,608 over 2,048 63 -> 46).
-    What adds into at most 2,048 features stays with the tiles whose waves split K wherever those fill their rounds: the fastest
-    or level with it from K 2,048 on (over K 1,024 large tiles would take 17 us instead of 22 for 2,048 rows)."""
+    workgroups). The least estimated time decides: on the shapes that it was fitted to 0.2 % above the fastest in the
+    geometric mean, on 430 others 0.2 to 0.6 %. Fixed numbers of tiles were 10 % above it (storing, 1,111 rows by 2,048 features over K 8,192 97 us
+    against 57, 640 by 2,048 over 2,048 22 against 14, 1,300 by 3,072 over 2,048 44 against 28; gated, 1,111 by 4,608 over 2,048 63 against 46), adding
+    products of up to 2,048 features held to the tiles whose waves split K 5 % (6,200 by 2,048 over 7,168 269 against 163, 2,690 by 1,536 over 1,024 32
+    against 18; they keep what is one round over a long K: 2,048 by 2,048 over 4,096 41 against 48)."""
     lib = library()
-    if mode == 1 and K >= DEEP_MIN_K and N <= DEEP_NARROW and _deep_columns(mode, M, N, K):
-        return "deep", _deep_columns(mode, M, N, K)
     wide, narrow = -(-M // 128) * -(-N // 128), -(-M // 128) * -(-N // 64)
     columns = 64 if mode == 2 or wide < DEEP_ROUND or (wide == DEEP_ROUND and K < LONG_K) else 128        # as fw_gemm_mfma chooses
-    times = {("tiles", 0): _tiled_time(narrow if columns == 64 else wide, K, *_TIME_TILES[mode][columns])}
+    ragged = _TIME_RAGGED if mode == 1 and N % 64 else 0.0
+    times = {("tiles", 0): _tiled_time(narrow if columns == 64 else wide, K, *_TIME_TILES[mode][columns]) + (ragged if columns == 64 else 0.0)}
     if mode != 2:
         for columns in (128, 64):
             tiles = lib.fw_gemm_mfma_deep_tiles(mode, M, N, K, columns)
             if tiles:
-                times["deep", columns] = _tiled_time(tiles, K, *_TIME_DEEP[mode][columns])
+                times["deep", columns] = _tiled_time(tiles, K, *_TIME_DEEP[mode][columns]) * (_TIME_DEEP_FEW_ROWS if columns == 64 and M <= 384 and K > 2560 else 1.0)
     if M > BIG_MIN_ROWS:
         rows, columns = ctypes.c_int(0), ctypes.c_int(0)
         tiles = lib.fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns))
-        if tiles and mode == 2:
-            times["big", 0] = _tiled_time(tiles, K, *_TIME_BIG_GATED)
-        elif tiles:
-            start, each_round, walk, fill = _TIME_BIG[mode][rows.value]
-            area = rows.value * columns.value / 1024
-            times["big", 0] = _tiled_time(tiles, K, start, each_round, walk * area, fill * area)
+        if tiles:
+            start, each_round, each_tile, walk, fill = _TIME_BIG[mode][rows.value]
+            area = rows.value * (256 if mode == 2 else columns.value) / 1024        # (a gated tile has gate and up columns)
+            odd = _TIME_BIG_ODD if mode == 2 and N % 2 else 0.0
+            times["big", 0] = _tiled_time(tiles, K, start, each_round + odd, each_tile, walk * area, fill * area)
     need_bytes, tiles = _split_needs(mode, M, N, K)
     if need_bytes:
         slices = need_bytes // (tiles * 128 * (128 if mode == 2 else 64) * 4)
-        start, each, walk, fill = _TIME_SPLIT[mode]
+        start, each, walk, fill, all_at_once = _TIME_SPLIT[mode]
         workgroups = tiles * slices
-        times["split", 0] = start + each * slices + walk * K / 1024 / slices * -(-workgroups // DEEP_ROUND) + fill * workgroups / DEEP_ROUND
+        share = workgroups / DEEP_ROUND
+        times["split", 0] = (start + ragged + each * slices + share * all_at_once
+                             + K / 1024 / slices * (walk * -(-workgroups // DEEP_ROUND) + fill * share))
     return min(times, key=times.get)
 
 
@@ -652,7 +661,6 @@ MEDIUM_MAX_ROWS = 64
 # fill their round (fw_gemm_rows_round_fits).
 ROWS_MAX = 1024
 BIG_TILES_MIN = 192      # large tiles that are nearly a round over the 256 compute units
-DEEP_NARROW = 2048       # features up to which a product that adds into the residual prefers the tiles whose waves split K
 DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)
 DEEP_ROUND = 256          # tiles of a round: one per compute unit
 DEEP_FILL = 0.85          # least share of the rounds' places that the tiles must fill (640 narrow tiles, 0.83: 193 vs 189 us)

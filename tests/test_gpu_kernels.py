@@ -497,14 +497,12 @@ def test_tiles_whose_waves_split_k(ops, M, N, K, columns):
 
 
 @pytest.mark.parametrize("M,N,K,expected", [(2048, 2048, 4096, 128), (1800, 1990, 4160, 128), (2048, 1024, 2048, 64),
-                                            (1152, 2048, 2048, 128), (576, 2048, 1024, 64), (2304, 2048, 1024, 64)])
+                                            (1152, 2048, 4096, 128), (576, 2048, 1024, 64), (1100, 1024, 2048, 64)])
 def test_the_prompt_product_of_one_round_of_tiles_over_a_long_k(ops, M, N, K, expected):
-    """What the dispatch sends to those tiles: about one 128 x 128 tile per compute unit and a
-    long K (the w2 product of a 2,048-token prompt); for a product that adds into the residual
-    also rounds that are little more than half full, on the width that fills them better."""
-    columns = ops._deep_columns(1, M, N, K)
-    assert columns == expected and K >= ops.DEEP_MIN_K
-    assert ops._deep_columns(1, 512, 2048, 8192) == 0 and ops._deep_columns(0, 1152, 2048, 8192) == 0
+    """What the dispatch sends to those tiles of products that add into the residual: about one 128 x 128 tile per compute unit
+    and a long K (the w2 product of a 2,048-token prompt), rounds that are little more than half full, narrower tiles
+    where those fill theirs better."""
+    assert ops.tiled_plan(1, M, N, K) == ("deep", expected)
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     want = back(a) @ back(w).T
@@ -513,19 +511,20 @@ def test_the_prompt_product_of_one_round_of_tiles_over_a_long_k(ops, M, N, K, ex
     ops.gemm(a, w, accumulate_into=residual)
     close(residual, before + want, torch.float32, 2.0)
     direct = before.float().to(DEV)
-    ops.gemm_deep(a, w, accumulate_into=direct, columns=columns)
+    ops.gemm_deep(a, w, accumulate_into=direct, columns=expected)
     assert torch.equal(direct, residual)
     close(ops.gemm(a, w, out_dtype=torch.float32), want, torch.float32, 2.0)
 
 
-@pytest.mark.parametrize("M,N,K,mode,columns", [(256, 6144, 2048, 0, 64), (500, 6100, 1984, 0, 128), (130, 6144, 2048, 0, 64),
+@pytest.mark.parametrize("M,N,K,mode,columns", [(256, 6144, 2048, 0, 64), (1100, 2048, 4096, 0, 128), (130, 6144, 2048, 0, 64),
                                                    (512, 2048, 2048, 1, 64), (320, 2048, 2048, 1, 64), (300, 3072, 1024, 0, 64),
-                                                   (256, 2048, 8192, 1, 0), (600, 6144, 2048, 0, 0), (256, 1024, 2048, 0, 0)])
+                                                   (256, 2048, 8192, 1, 0), (600, 6144, 2048, 0, 0), (500, 6100, 1984, 0, 0), (256, 1024, 2048, 0, 64)])
 def test_a_few_hundred_rows_go_to_the_tiles_whose_waves_split_k(ops, M, N, K, mode, columns):
     """A decode step of a few hundred requests: storing and short accumulating products take those
-    tiles when they are not too few (equal, bit for bit, to the kernel called by name); a long K,
-    more rows or too few tiles stay with the other products."""
-    assert ops._deep_columns_few_rows(mode, M, N, K) == columns
+    tiles (equal, bit for bit, to the kernel called by name); a long K of few rows has it cut over
+    workgroups, and wide outputs of some hundred rows go to the large tiles."""
+    kind, width = ops.tiled_plan(mode, M, N, K)
+    assert (width if kind == "deep" else 0) == columns
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     want = back(a) @ back(w).T
