@@ -151,24 +151,33 @@ class GatedDeltaRule(Mixer):
         """Whether the columns of state of a step that is walked token by token are shared out over 32 lanes (``row0``: the first row of each
         segment, and the end).
         A walk is bound by how fast one wave issues its chain of instructions, so half the arithmetic a wave pays as long as its
-        workgroups, of 8 value channels, have a compute unit each. 16 heads of 128 channels, prompts of 694 rows: one
-        173 -> 150 us, but two 177 -> 196 and four 222 -> 320; 4 heads: four prompts 173 -> 148, eight of 300 rows
-        82 -> 91. Single rows beside a prompt count too: their workgroups come and go, and the prompt's then share the compute
-        units unevenly (four layers, 1,500 rows beside 6 single ones: the step 4.05 ms, on 32 lanes 4.80)."""
+        workgroups, of 8 value channels, have a compute unit each. One segment of 64 / 95 rows (longer ones go in chunks), records included: 16
+        heads of 128 channels 26.8 -> 26.0, 34.8 -> 32.4 us, 8 of 256 38.2 -> 33.3, 51.2 -> 43.2, 16 of 192 37.7 -> 32.3, 50.2 -> 42.1; two of 694 rows
+        on 16 heads, beyond those compute units, 177 -> 196. Single rows beside a prompt count too: their workgroups come and go, and
+        the prompt's then share the compute units unevenly."""
         if self.dtype != torch.bfloat16 or self.dim <= 64:
             return False        # (a float32 run gives the same bits however a sequence is cut into steps: its prompts walk as its single rows do)
         return (len(row0) - 1) * self.heads * -(-self.vdim // 8) <= ops.COMPUTE_UNITS
 
+    # Rows that the longest segment must have beyond 96 for each head of each segment of one row, by the keys' width in 64 channels (or half
+    # the values', which weigh as much): a chunk's workgroup costs such a segment what it costs sixteen rows, and large heads take whole
+    # compute units.
+    CHUNK_ROWS = (0.14, 0.16, 0.3, 0.8)
+
     def chunked(self, row0) -> bool:
         """Whether a step's segments are walked sixteen tokens at a time (``row0``: the first row of each segment, and the end). That takes
-        one launch more and a chunk's work for a segment of one row, and gains 0.05 to 0.17 us a token of the longest segment. 16 heads of
-        128 channels, convolutions included: one prompt of 64 rows 25 -> 23 us, of 96 33 -> 26, of 1,111 272 -> 117, sixteen of 96 169 -> 112;
-        2 heads of 16 channels: 64 rows 16.5 -> 18.9, 96 rows 21.3 -> 20.4. Beside 24 single rows 64 rows lose (46 -> 56) and 128 gain
-        (70 -> 65), beside 60 single rows 128 lose (84 -> 116) and 500 gain (233 -> 150)."""
+        one launch more and a chunk's work for a segment of one row, and gains 0.05 to 0.35 us a token of the longest segment. 16 heads of
+        128 channels, convolutions included: one prompt of 64 rows 26 -> 23 us, of 95 32 -> 25, of 1,111 272 -> 117, sixteen of 96 169 -> 112;
+        2 heads of 16 channels: 64 rows 23.9 -> 20.8 (both bound by the host there). Segments of few rows beside the longest: 16 heads of
+        128, 24 single ones, 96 rows 57 -> 59, 128 68 -> 64, 256 118 -> 79, 60 single ones, 200 rows 113 -> 122, 256 136 -> 127; 48 heads, 24 single
+        ones, 160 rows 133 -> 151, 256 185 -> 169, 60 single ones, 256 rows 246 -> 360, 777 557 -> 477; 16 heads of 256, 24 single ones, 200
+        rows 203 -> 235, 400 309 -> 284, 60 single ones, 400 rows 433 -> 574, 777 667 -> 694; 32 heads of 64, 60 single ones, 200 rows 82 -> 93, 256
+        100 -> 96. The rule gives up what little there is to gain near its line rather than lose there."""
         if self.dtype != torch.bfloat16:
             return False        # (a float32 run gives the same bits however a sequence is cut into steps)
         lengths = [b - a for a, b in zip(row0, row0[1:])]
-        return max(lengths, default=0) >= 96 + 2 * sum(n < 16 for n in lengths)
+        short = sum(24 - n for n in lengths if n < 24) / 24         # segments of one row, those of up to 23 in part
+        return max(lengths, default=0) >= 96 + short * self.heads * self.CHUNK_ROWS[(max(self.dim, self.vdim // 2) - 1) // 64]
 
     def heads_output(self, h, ctx, cache) -> torch.Tensor:
         """The heads' normed and gated read-outs [rows, heads * vdim] in the activation dtype; the

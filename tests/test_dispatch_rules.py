@@ -32,11 +32,20 @@ def test_delta_rule_spreads_its_columns_while_every_workgroup_has_a_compute_unit
 
 
 @pytest.mark.parametrize("lengths,chunked", [
-    ([95], False), ([96], True), ([64] * 16, False), ([96] * 16, True), ([1111], True), ([1] * 24 + [128], False), ([1] * 24 + [144], True),
-    ([1] * 60 + [200], False), ([1] * 60 + [500], True), ([1] * 8, False), ([15, 300], True)])
+    ([95], False), ([96], True), ([64] * 16, False), ([96] * 16, True), ([1111], True), ([1] * 24 + [128], False), ([1] * 24 + [160], True),
+    ([1] * 60 + [200], False), ([1] * 60 + [256], True), ([1] * 60 + [500], True), ([1] * 8, False), ([15, 300], True)])
 def test_delta_rule_walks_prompts_in_chunks_where_those_are_faster(lengths, chunked):
     assert _delta_rule(16, 128, 128).chunked(_row0(lengths)) == chunked
     assert not _delta_rule(16, 128, 128, torch.float32).chunked(_row0(lengths))
+
+
+@pytest.mark.parametrize("heads,dim,vdim,lengths,chunked", [
+    (48, 128, 128, [1] * 24 + [200], False), (48, 128, 128, [1] * 60 + [400], False), (48, 128, 128, [1] * 60 + [777], True),
+    (16, 256, 256, [96], True), (16, 256, 256, [1] * 24 + [256], False), (16, 256, 256, [1] * 24 + [400], True), (16, 256, 256, [1] * 60 + [777], False),
+    (16, 256, 256, [17] * 40 + [192], False), (16, 64, 256, [1] * 60 + [200], False), (1, 256, 256, [1] * 60 + [160], True),
+    (32, 64, 64, [1] * 60 + [256], False), (2, 16, 16, [1] * 60 + [128], True), (256, 1, 1, [1] * 4 + [200], False)])
+def test_many_or_large_heads_beside_short_segments_keep_the_walk_token_by_token(heads, dim, vdim, lengths, chunked):
+    assert _delta_rule(heads, dim, vdim).chunked(_row0(lengths)) == chunked
 
 
 @pytest.mark.parametrize("heads,dim,lengths,cuts", [
