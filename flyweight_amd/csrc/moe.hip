@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const TA* __restrict_
 // bfloat16 operands, float32 accumulation (v_mfma_f32_32x32x16_bf16). A tile of places belongs to one
 // expert; both operands are k-contiguous, a slab of 64 k of each is copied per iteration: global ->
 // registers (two slabs ahead of the one multiplied) -> LDS (one ahead), two LDS buffers, one barrier an
-// iteration, LDS rows padded to 144 bytes. Two shapes of tile:
+// iteration. Two shapes of tile:
 //   BIG     128 places x 128 rows of W; four waves as 2 x 2, each 64 x 64. For steps in which an expert
 //           has hundreds of places (prompts) and that do not go straight to LDS (fw_grouped_gemm_large_fits): a clamped
 //           unit, a K that is no multiple of 32, few tiles over a long K.
@@ -399,7 +399,12 @@ typedef __attribute__((ext_vector_type(8))) __bf16 gg_bf16x8;
 typedef __attribute__((ext_vector_type(16))) float gg_f32x16;
 typedef __attribute__((ext_vector_type(4))) uint32_t gg_u32x4;
 #define GGM_TK 64
-#define GGM_ROW_BYTES 144
+// Where row r of a slab lies in LDS, and what n rows (an even number) take: 128 bytes a row and 16 behind every second one, so that 16-byte reads of
+// sixteen consecutive rows, two of which cover the 64 banks, meet no bank twice. A gated tile of 32 places is then 77 KB (with every row
+// padded to 144 bytes 81), and two workgroups share a compute unit: with one, and the tiles dealt evenly to the dies, the few tiles of a second round
+// took as long as a full one (gated 1,536 over 2,048, 4 of 32 experts, 12 / 24 / 40 rows, 270 to 380 tiles: 65.8 / 76.0 / 76.2 us while the
+// first dies had them all, 68.1 / 78.0 / 79.0 dealt evenly, 63.9 / 75.4 / 76.2 now; one row, 48 tiles 23.8 -> 23.1).
+static __host__ __device__ constexpr int ggm_row(int r) { return r * 128 + (r >> 1) * 16; }
 
 __device__ __forceinline__ float gg_silu(float g) {
     if (g >= 0.0f) return g / (1.0f + __expf(-g));
@@ -418,7 +423,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     constexpr int NI = TMR / (32 * WAVES_M);
     constexpr int BN = WAVES_N * NJ * 32;               // rows of W of a tile
     constexpr int A_CHUNKS = TMR / 32, W_CHUNKS = BN / 32;
-    constexpr int A_SLAB = TMR * GGM_ROW_BYTES, W_SLAB = BN * GGM_ROW_BYTES;
+    constexpr int A_SLAB = ggm_row(TMR), W_SLAB = ggm_row(BN);
     static_assert(!GATED || NJ == 2, "the gated tile holds gate and up side by side");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 
@@ -442,7 +447,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
         place = place < end ? place : end - 1;          // places past the expert's last are computed and dropped
         const int from = place_row ? place_row[place] : place;
         a_src[i] = a + (size_t)from * K;
-        a_at[i] = row * GGM_ROW_BYTES + (tid & 7) * 16;
+        a_at[i] = ggm_row(row) + (tid & 7) * 16;
     }
 #pragma unroll
     for (int i = 0; i < W_CHUNKS; ++i) {
@@ -457,7 +462,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
             wr = wr < N ? wr : N - 1;
         }
         w_src[i] = we + (size_t)wr * K;
-        w_at[i] = row * GGM_ROW_BYTES + (tid & 7) * 16;
+        w_at[i] = ggm_row(row) + (tid & 7) * 16;
     }
 
     gg_f32x16 acc[NI][NJ];
@@ -501,10 +506,10 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
             gg_bf16x8 fa[NI], fb[NJ];
 #pragma unroll
             for (int i = 0; i < NI; ++i)
-                fa[i] = *reinterpret_cast<const gg_bf16x8*>(sa + (a_row0 + 32 * i) * GGM_ROW_BYTES + k16 * 32 + k_lane);
+                fa[i] = *reinterpret_cast<const gg_bf16x8*>(sa + ggm_row(a_row0) + ggm_row(32 * i) + k16 * 32 + k_lane);
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
-                fb[j] = *reinterpret_cast<const gg_bf16x8*>(sb + b_row[j] * GGM_ROW_BYTES + k16 * 32 + k_lane);
+                fb[j] = *reinterpret_cast<const gg_bf16x8*>(sb + ggm_row(b_row[j]) + k16 * 32 + k_lane);
 #pragma unroll
             for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -582,7 +587,7 @@ static int grouped_mfma_launch(const void* a, const int32_t* place_row, const vo
     const long long tiles_n = fw_ceil_div(N, features);
     FW_REQUIRE(tiles_m * tiles_n < (1ll << 30), "grouped_gemm: too many tiles");
     const int per_xcd = (int)fw_ceil_div(tiles_m * tiles_n, 8);
-    const int lds_bytes = 2 * (TMR + BN) * GGM_ROW_BYTES;
+    const int lds_bytes = 2 * ggm_row(TMR + BN);
     static bool configured = false;     // per instantiation
     if (!configured) {
         hipError_t status = hipFuncSetAttribute((const void*)grouped_gemm_mfma_kernel<GATED, BIG, NJ, TO>,
