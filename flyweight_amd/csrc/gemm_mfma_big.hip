@@ -457,15 +457,8 @@ static BigPlan big_plan(int mode, int M, int N) {
     return best;
 }
 
-// How many tiles the kernel cuts a shape into, by the tile it will choose (the caller decides
-// whether that fills the chip); 0 if the kernel does not take the shape (K must be a multiple
-// of 32).
-extern "C" int fw_gemm_mfma_big_tiles(int mode, int M, int N, int K) {
-    if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1 || N > BN_MOST) return 0;
-    return big_plan(mode, M, N).tiles;
-}
-
-// The same with the tile's edges: what the caller needs to tell how much of the tiles the output fills.
+// How many tiles the kernel cuts a shape into, by the tile it will choose, and that tile's edges (the caller works out from them
+// whether that fills the chip); 0 if the kernel does not take the shape (K must be a multiple of 32).
 extern "C" int fw_gemm_mfma_big_plan(int mode, int M, int N, int K, int* rows, int* columns) {
     if (K <= 0 || K % BK || K > BK_MOST || M < 1 || N < 1 || N > BN_MOST) return 0;
     const BigPlan plan = big_plan(mode, M, N);

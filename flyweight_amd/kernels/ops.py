@@ -660,56 +660,7 @@ MEDIUM_MAX_ROWS = 64
 # 17.3, 3,072 at 384 rows 24.4 against 18.3, 16,384 gated at 128 rows 35 against 27), and so it does with a long K where the others' tiles
 # fill their round (fw_gemm_rows_round_fits).
 ROWS_MAX = 1024
-BIG_TILES_MIN = 192      # large tiles that are nearly a round over the 256 compute units
-DEEP_MIN_K = 1024         # adding into the residual (2,048 x 2,048 x 2,048: 31 vs 39 us; x 8,192: 83 vs 118 us; 2,048 x 1,024 x 1,024: 13 vs 15 us)
 DEEP_ROUND = 256          # tiles of a round: one per compute unit
-DEEP_FILL = 0.85          # least share of the rounds' places that the tiles must fill (640 narrow tiles, 0.83: 193 vs 189 us)
-# adding into the residual, 2,048 features: 144 wide tiles (1,152 rows) K 8,192 72 vs 103 us, K 2,048 28 vs 35 us; 160
-# narrow tiles (576 rows) 46 vs 65 us and 16.5 vs 27 us; 576 narrow (2,304 rows) 120 vs 135 us; 128 narrow tiles lose
-DEEP_FILL_ADDING = 0.55
-
-
-def _round_fill(tiles: int) -> float:
-    """The share of the places in whole rounds over the chip that the tiles fill."""
-    rounds = -(-tiles // DEEP_ROUND)
-    return tiles / (rounds * DEEP_ROUND) if tiles > 0 else 0.0
-
-
-def _deep_columns(mode: int, M: int, N: int, K: int) -> int:
-    """The width of the tiles whose waves split K that serves this shape: the width (128 or 64
-    columns) whose tiles fill their rounds over the chip better, the wider at a tie, if they fill
-    enough of them; else 0. A product that adds into the residual needs less (the other kernels
-    ask for the old values at the end of a tile, where nothing hides the read)."""
-    fills = {columns: _round_fill(library().fw_gemm_mfma_deep_tiles(mode, M, N, K, columns)) for columns in (128, 64)}
-    columns = 128 if fills[128] >= fills[64] else 64
-    return columns if fills[columns] >= (DEEP_FILL_ADDING if mode == 1 else DEEP_FILL) else 0
-
-
-DEEP_FEW_ROWS = 512       # up to here the tiles whose waves split K also serve a short K, if they are not too few
-DEEP_FEW_TILES_WIDE = 192   # tiles of 128 columns from which those are taken, else
-DEEP_FEW_TILES = 96       # tiles of 64 columns from which those are
-
-
-def _deep_columns_few_rows(mode: int, M: int, N: int, K: int) -> int:
-    """A few hundred rows (decode steps of that many requests, short prompts) give the 128 x 128
-    tiles of the register-staged product less than a round over the chip; the tiles whose waves
-    split K bring their operands straight into LDS, three slabs ahead, and a workgroup alone on
-    its compute unit keeps them coming. Measured against the products they replace, 8 in a row:
-    storing 6,144 features at 256 rows 16.0 vs 21.0 us, at 128 rows 15.0 vs 18.6; 3,072 features at
-    256 rows 15.0 vs 18.6, at 512 rows 15.9 vs 21.0 us; adding 2,048 features (K 2,048) at 512 rows
-    16.2 vs 23.0 us, at 320 rows 15.7 vs 21.5 us. With a long K (8,192) the product that cuts K over
-    workgroups is level with them."""
-    if mode not in (0, 1) or M > DEEP_FEW_ROWS or K > (LONG_K if mode == 1 else 1 << 30):
-        return 0
-    wide = library().fw_gemm_mfma_deep_tiles(mode, M, N, K, 128)
-    narrow = library().fw_gemm_mfma_deep_tiles(mode, M, N, K, 64)
-    if mode == 0 and DEEP_FEW_TILES_WIDE <= wide <= DEEP_ROUND:
-        return 128
-    if DEEP_FEW_TILES <= narrow <= 2 * DEEP_ROUND:
-        return 64
-    return 0
-
-
 BIG_MIN_ROWS = 128       # up to here a 256-row tile would be at least half empty (the head at 128 rows: 110 vs 78 us)
 _MEDIUM_COUNTERS = {}
 

@@ -1,5 +1,5 @@
-"""The product on tiles of 256 rows: every number of slabs of K up to where its turns repeat (its four stages half full, full, one
-turn, several), every shape of tile, rows and features that end inside one, its three epilogues."""
+"""The product on large tiles: every number of slabs of K up to where its turns repeat, every shape of tile, rows and features that end inside one,
+its epilogues in both output types."""
 
 import ctypes
 
@@ -19,13 +19,6 @@ def ops():
     return module
 
 
-def big(ops, a, w, out, mode, N):
-    M, K = a.shape
-    entry = ops.library().fw_gemm_mfma_big
-    ops._check(entry(ops._p(a), ops._p(w), None, ops._p(out), F32 if out.dtype == torch.float32 else BF16, mode, M, N, K, ops._stream()))
-    return out
-
-
 def draw(*shape, seed=0):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16)
 
@@ -35,31 +28,52 @@ def bound(a, w):
     return (a.shape[1] + 16) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
 
 
-# (rows, features) for each tile: 256 x 256, 256 x 192, 128 x 256, 128 x 192 by the count of rounds, and one row of one feature
-@pytest.mark.parametrize("M,N", [(256, 512), (300, 185), (129, 257), (77, 190), (1, 1)])
-@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 288, 1056])
-def test_every_number_of_slabs(ops, M, N, K):
-    a, w = draw(M, K), draw(2 * N, K, seed=1)
-    A, W = a.to(DEV), w.to(DEV)
-    exact, limit = a.double() @ w.double().T, bound(a, w)
-    plain = big(ops, A, W[:N], torch.empty(M, N, device=DEV), STORE, N).cpu().double()
-    assert ((plain - exact[:, :N]).abs() <= limit[:, :N]).all()
+# (rows, features) for each shape of tile, whole and ending inside one, the tile, and the features of the gated product on its 256 rows
+TILES = [(2048, 6144, (256, 192)), (1537, 6100, (256, 192)), (1536, 8192, (256, 256)), (1500, 8201, (256, 256)), (1920, 4096, (128, 256)),
+         (1900, 4001, (128, 256)), (256, 384, (128, 192)), (129, 257, (128, 192)), (1, 1, (128, 192))]
+
+
+@pytest.mark.parametrize("M,N,tile", TILES)
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 288, 544])
+def test_every_number_of_slabs(ops, M, N, tile, K):
+    """Every number of slabs of K up to where the turns of the loop repeat: its four stages half full, full, one turn, several."""
+    rows, columns = ctypes.c_int(0), ctypes.c_int(0)
+    for mode in (STORE, ADD):
+        assert ops.library().fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns)) > 0
+        assert (rows.value, columns.value) == tile
+    half = (N + 1) // 2                         # (of the gated product: the other rows of w)
+    a, w = draw(M, K), draw(max(N, 2 * half), K, seed=1)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2))
     residual = torch.randn(M, N, generator=torch.Generator().manual_seed(3))
-    total = big(ops, A, W[:N], residual.to(DEV), ADD, N).cpu().double()
-    assert ((total - exact[:, :N] - residual.double()).abs() <= limit[:, :N] + 2.0 ** -23 * total.abs()).all()
-    gate, up = exact[:, :N], exact[:, N:]
+    A, W, B = a.to(DEV), w.to(DEV), bias.to(DEV)
+    # (the products and their bounds on the GPU in float64, by the library: 16 million elements of a large one)
+    exact = A.double() @ W.double().T
+    limit = (K + 16) * 2.0 ** -24 * (A.double().abs() @ W.double().abs().T)
+
+    def run(mode, out, width, with_bias=False):
+        entry = ops.library().fw_gemm_mfma_big
+        ops._check(entry(ops._p(A), ops._p(W), ops._p(B) if with_bias else None, ops._p(out), F32 if out.dtype == torch.float32 else BF16, mode, M,
+                         width, K, ops._stream()))
+        return out.double()
+
+    want, room = exact[:, :N] + B.double(), limit[:, :N] + 2.0 ** -23 * (exact[:, :N].abs() + B.double().abs())
+    assert ((run(STORE, torch.empty(M, N, device=DEV), N, True) - want).abs() <= room).all()
+    assert ((run(STORE, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), N, True) - want).abs() <= room + 2.0 ** -8 * want.abs()).all()
+    total = run(ADD, residual.to(DEV), N)
+    assert ((total - exact[:, :N] - residual.to(DEV).double()).abs() <= limit[:, :N] + 2.0 ** -23 * total.abs()).all()
+    gate, up, gate_off, up_off = exact[:, :half], exact[:, half:2 * half], limit[:, :half], limit[:, half:2 * half]
     want = gate * torch.sigmoid(gate) * up
-    got = big(ops, A, W, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), GATED, N).cpu().double()
     # |d silu| <= 1.1 |d gate|, |silu| <= |gate|; the hardware's exponential and reciprocal 2^-20; one rounding to bfloat16
-    slack = 1.1 * limit[:, :N] * (up.abs() + limit[:, N:]) + gate.abs() * limit[:, N:] + 2.0 ** -20 * want.abs() + 2.0 ** -8 * want.abs() + 2.0 ** -133
-    assert ((got - want).abs() <= slack).all()
+    slack = 1.1 * gate_off * (up.abs() + up_off) + gate.abs() * up_off + 2.0 ** -20 * want.abs() + 2.0 ** -8 * want.abs() + 2.0 ** -133
+    assert ((run(GATED, torch.empty(M, half, device=DEV, dtype=torch.bfloat16), half) - want).abs() <= slack).all()
 
 
 def test_a_width_beyond_its_offsets_goes_elsewhere(ops):
-    rows, columns = ctypes.c_int(0), ctypes.c_int(0)
-    assert ops.library().fw_gemm_mfma_big_tiles(0, 4096, 8192, 1 << 22) > 0
-    assert ops.library().fw_gemm_mfma_big_tiles(0, 4096, 8192, (1 << 22) + 32) == 0
-    assert ops.library().fw_gemm_mfma_big_plan(0, 4096, 8192, (1 << 22) + 32, ctypes.byref(rows), ctypes.byref(columns)) == 0
+    plan = lambda M, N, K: ops.library().fw_gemm_mfma_big_plan(0, M, N, K, ctypes.byref(ctypes.c_int(0)), ctypes.byref(ctypes.c_int(0)))    # noqa: E731
+    assert plan(4096, 8192, 1 << 22) > 0
+    assert plan(4096, 8192, (1 << 22) + 32) == 0
+    assert plan(4096, 1 << 20, 64) > 0
+    assert plan(4096, (1 << 20) + 1, 64) == 0
 
 
 @pytest.mark.parametrize("shift", [0, 1])

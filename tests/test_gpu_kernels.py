@@ -419,30 +419,45 @@ def test_fast_gemm_every_epilogue(ops, M, N, K):
         close(ops.gemm_swiglu(a, w), act, torch.bfloat16, 0.4)
 
 
-@pytest.mark.parametrize("M,N,K,tiles", [(2048, 6144, 96, 256), (1500, 8200, 160, 198), (4000, 3100, 64, 208), (1800, 6000, 2080, 256),
-                                         (1536, 6100, 96, 192), (2048, 3072, 96, 256), (1990, 3000, 2080, 256), (1900, 4000, 160, 240)])
-def test_large_tile_prompt_product(ops, M, N, K, tiles):
-    """Shapes that the large-tile kernel cuts into at least 192 tiles go to it: every epilogue,
-    edges in both directions, few and many slabs. ``tiles`` tells which tile a storing or
-    accumulating product takes: 256 x 256 (the second and third shape), 256 x 192 (the first,
-    fourth and fifth: one round over the chip with the narrower tile), 128 x 192 (the sixth and
-    seventh: 128 tiles of 256 rows, 256 of 128) and 128 x 256 (the last); the gated product keeps
-    the 256 x 256 tiles."""
-    assert ops.library().fw_gemm_mfma_big_tiles(0, M, N, K) == tiles and tiles >= ops.BIG_TILES_MIN
-    assert not ops.library().fw_gemm_mfma_big_tiles(0, M, N, K + 8)
+def every_epilogue(ops, product, M, N, K):
+    """A tiled product called by name, ``product(a, w, bias, out, dtype code, mode, N)``: stored with a bias in float32, in bfloat16, added, gated;
+    twice the same bits."""
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     bias = gen(N, seed=2).float().to(DEV)
     want = back(a) @ back(w).T
-    close(ops.gemm(a, w, bias, out_dtype=torch.float32), want + bias.cpu().double(), torch.float32, 2.0)
-    close(ops.gemm(a, w), want, torch.bfloat16, 0.4)
+    first = product(a, w, bias, torch.empty(M, N, device=DEV), ops.F32, 0, N)
+    close(first, want + bias.cpu().double(), torch.float32, 2.0)
+    for _ in range(3):
+        assert torch.equal(product(a, w, bias, torch.empty(M, N, device=DEV), ops.F32, 0, N), first)
+    close(product(a, w, None, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), ops.BF16, 0, N), want, torch.bfloat16, 0.4)
     residual = gen(M, N, seed=3).float().to(DEV)
     before = residual.cpu().double()
-    ops.gemm(a, w, accumulate_into=residual)
-    close(residual, before + want, torch.float32, 2.0)
-    if N % 2 == 0 and ops.library().fw_gemm_mfma_big_tiles(2, M, N // 2, K) >= ops.BIG_TILES_MIN:
+    close(product(a, w, None, residual, ops.F32, 1, N), before + want, torch.float32, 2.0)
+    if N % 2 == 0:
         half = N // 2
-        close(ops.gemm_swiglu(a, w), F.silu(want[:, :half]) * want[:, half:], torch.bfloat16, 0.4)
+        out = torch.empty(M, half, device=DEV, dtype=torch.bfloat16)
+        close(product(a, w, None, out, ops.BF16, 2, half), F.silu(want[:, :half]) * want[:, half:], torch.bfloat16, 0.4)
+
+
+@pytest.mark.parametrize("M,N,K,rows,columns,tiles", [
+    (2048, 6144, 96, 256, 192, 256), (1500, 8200, 160, 256, 256, 198), (4000, 3100, 64, 256, 256, 208), (1800, 6000, 2080, 256, 192, 256),
+    (1536, 6100, 96, 256, 192, 192), (2048, 3072, 96, 128, 192, 256), (1990, 3000, 2080, 128, 192, 256), (1900, 4000, 160, 128, 256, 240)])
+def test_large_tile_prompt_product(ops, M, N, K, rows, columns, tiles):
+    """Every epilogue on every shape of the large tiles, edges in both directions, few and many slabs: 256 x 256, 256 x 192 (one round
+    over the chip with the narrower tile), 128 x 192 (128 tiles of 256 rows, 256 of 128) and 128 x 256; the gated product keeps 256 x 256."""
+    import ctypes
+    found = ctypes.c_int(0), ctypes.c_int(0)
+    plan = ops.library().fw_gemm_mfma_big_plan
+    for mode in (0, 1):
+        assert plan(mode, M, N, K, *map(ctypes.byref, found)) == tiles and [x.value for x in found] == [rows, columns]
+    assert not plan(0, M, N, K + 8, *map(ctypes.byref, found))
+
+    def product(a, w, bias, out, code, mode, N):
+        ops._check(ops.library().fw_gemm_mfma_big(ops._p(a), ops._p(w), ops._p(bias), ops._p(out), code, mode, M, N, K, ops._stream()))
+        return out
+
+    every_epilogue(ops, product, M, N, K)
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 2048, 2048), (128, 2048, 8192), (130, 104, 1032), (200, 3072, 2048), (300, 2500, 520),
@@ -450,28 +465,20 @@ def test_large_tile_prompt_product(ops, M, N, K, tiles):
 def test_tiled_product_cuts_k_into_slices(ops, M, N, K):
     """More than 64 rows but fewer tiles than compute units: K goes to several workgroups and the
     last one of a tile to arrive adds the slices in their order. Every epilogue, edges in rows,
-    features and K, twice in a row (the tickets are left at zero), and bitwise the same whichever
+    features and K, several times in a row (the tickets are left at zero), and bitwise the same whichever
     workgroup came last."""
     import ctypes
-    need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
-    assert ops.library().fw_gemm_mfma_split_plan(0, M, N, K, ctypes.byref(need_bytes), ctypes.byref(need_counters)) == 0
-    assert need_bytes.value > 0 and need_counters.value > 0, "the shape is meant to be cut"
-    a = as_dev(gen(M, K), torch.bfloat16)
-    w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
-    bias = gen(N, seed=2).float().to(DEV)
-    want = back(a) @ back(w).T
-    first = ops.gemm(a, w, bias, out_dtype=torch.float32)
-    close(first, want + bias.cpu().double(), torch.float32, 2.0)
-    for _ in range(3):
-        assert torch.equal(ops.gemm(a, w, bias, out_dtype=torch.float32), first)
-    close(ops.gemm(a, w), want, torch.bfloat16, 0.4)
-    residual = gen(M, N, seed=3).float().to(DEV)
-    before = residual.cpu().double()
-    ops.gemm(a, w, accumulate_into=residual)
-    close(residual, before + want, torch.float32, 2.0)
-    if N % 2 == 0:
-        half = N // 2
-        close(ops.gemm_swiglu(a, w), F.silu(want[:, :half]) * want[:, half:], torch.bfloat16, 0.4)
+
+    def product(a, w, bias, out, code, mode, N):
+        need_bytes, need_counters = ops._split_needs(mode, M, N, K)
+        assert need_bytes > 0 and need_counters > 0, "the shape is meant to be cut"
+        workspace = torch.empty(need_bytes // 4, device=DEV)
+        counters = ops._medium_counters(a.device, need_counters)
+        ops._check(ops.library().fw_gemm_mfma_split(ops._p(a), ops._p(w), ops._p(bias), ops._p(out), code, mode, M, N, K, ops._p(workspace),
+                                                    ctypes.c_size_t(need_bytes), ops._p(counters), counters.numel(), ops._stream()))
+        return out
+
+    every_epilogue(ops, product, M, N, K)
 
 
 @pytest.mark.parametrize("columns", [128, 64])
