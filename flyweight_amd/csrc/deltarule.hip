@@ -192,10 +192,12 @@ __device__ __forceinline__ float delta_lanes_sum(float x) {
 // block's 16 values. A thread copies the same pieces of every chunk (16-byte pieces: where each lies in
 // a token's record and in LDS is worked out once).
 // The walk is bound by how fast one wave a SIMD issues its chain (about 7 clocks an instruction, twice what several waves get):
-// a prompt's heads of more than 64 key channels take 32 lanes a column, half the arithmetic a wave on twice the
-// workgroups, while those have a compute unit each (the caller says: GatedDeltaRule.spread). 16 heads of 128 channels, 694 rows in the mean: 205 us with operands read one float at a time, 172 read four at a
-// time, 146 on 32 lanes. (Two tokens at a time, their sums travelling together, gained nothing more: 147; nor did chunks of 32
-// tokens.) Beyond that 32 lanes lose: four prompts of 694 rows 222 against 320 us, 8 single rows 8.9 against 12.1.
+// a portion's heads of more than 64 key channels take 32 lanes a column, half the arithmetic a wave on twice the
+// workgroups, while those have a compute unit each (the caller says: GatedDeltaRule.spread; longer segments of a bfloat16 run go in chunks,
+// deltarule_chunks.hip). With the records in front of it, 95 rows: 16 heads of 128 channels 34.8 -> 32.4 us, 8 of 256 51.2 -> 43.2. 694 rows of
+// 16 heads, as float32 runs walk them: 205 us with operands read one float at a time, 172 read four at a time. (Two tokens at a time, their
+// sums travelling together, gained nothing more, nor did chunks of 32 tokens.) Beyond that 32 lanes lose: four prompts of 694 rows 222 against
+// 320 us, 8 single rows 8.9 against 12.1.
 template <int RPT, int DELTA_LANES>
 __global__ __launch_bounds__(256) void gated_delta_rule_kernel(
     const float* __restrict__ records, float* __restrict__ state, float* __restrict__ out,

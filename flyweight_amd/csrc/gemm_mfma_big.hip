@@ -83,8 +83,8 @@ struct BigTile {
 // K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way), and at most BK_MOST (a
 // lane's place in a tile's 256 rows is 32 bits, as it is in the output: N at most BN_MOST).
 //
-// Bound by the matrix cores at the clock that their power leaves (1.5 to 1.7 GHz in long runs): 72 to 76 % of the cycles in MFMAs,
-// the rest between the steps and at a tile's start and end. 2,048 x 8,192 gated x 2,048: 128.2 -> 117.5 us against reads and loads
+// Bound by the matrix cores at the clock that their power leaves (1.5 to 1.7 GHz in long runs): 65 % of a wave's cycles in MFMAs inside a
+// prompt's step, 72 % of the gated product alone, 76 % of 8,192^3; the rest between the steps and at a tile's start and end. 2,048 x 8,192 gated x 2,048: 128.2 -> 117.5 us against reads and loads
 // spread over whole steps with 64-bit addresses in vector registers; 2,048 x 6,144: 51.9 -> 49.4; 8,192^3: 1,185 -> 1,296 TFLOP/s.
 // One barrier for two slabs (five stages) gave nothing more.
 // TN: 32-column product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144

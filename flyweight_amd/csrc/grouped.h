@@ -17,7 +17,7 @@ struct GroupedTile {
 // that read the same rows of W run side by side, and an expert's places stay in the L2 of the die that works through it. Workgroups are
 // dealt to the eight dies in turn; a die takes an eighth of the tiles THERE ARE, which the device alone knows (the grid holds as many as there can
 // be at most: dealt out by that number, the last dies had nothing to do. Eight rows of four of 32 experts, 252 tiles of at most
-// 396, left three of the eight idle). Every wave works it out for itself, in scalar
+// 396, 50 a die, left two of the eight idle and a third with two). Every wave works it out for itself, in scalar
 // registers: read with a shuffle the tile would count as different in every lane, and so would every address formed from it (each load to LDS then
 // runs in a loop over the lanes' addresses: gated, 2,048 rows, 32 experts 173 us against 158).
 __device__ __forceinline__ GroupedTile grouped_tile(const int32_t* __restrict__ begin, int experts, int rows, int columns) {
