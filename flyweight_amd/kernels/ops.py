@@ -593,22 +593,32 @@ def _split_needs(mode: int, M: int, N: int, K: int):
 # below zero: parts that were, fitted to shapes of few rounds, made many rounds over a short K free.
 _TIME_DEEP = {0: {128: (3.2, 9.1, 1.4, 4.76, 3.28), 64: (2.6, 3.9, 1.2, 3.56, 1.54)},
               1: {128: (2.7, 10.4, 1.9, 4.84, 2.64), 64: (2.4, 4.5, 1.3, 3.62, 1.26)}}
-_TIME_DEEP_FEW_ROWS = 1.25     # of a long K where at most three rows of tiles share what they read of the weights (256 x 2,112 over 7,872: 53 us, by the parts alone 38)
-# ... through registers, where two workgroups share a compute unit, two parts more: for each pair of rounds, for 1,024 k of it
+_TIME_DEEP_FEW_ROWS = 1.25     # 64 columns, a long K, at most three rows of tiles sharing what they read of the weights (256 x 2,112 over 7,872: 53 us, by the parts alone 38)
+# ... through registers, where two workgroups share a compute unit, two parts more: for each pair of rounds (a gated product's third round
+# and those behind it: half a pair each), for 1,024 k of it
 _TIME_TILES = {0: {128: (5.1, 0.0, 1.5, 6.32, 2.84, 6.2, 0.92), 64: (0.0, 0.3, 0.8, 3.64, 1.42, 6.2, 2.54)},
                1: {128: (0.3, 0.0, 6.1, 5.87, 1.06, 11.7, 3.78), 64: (0.0, 1.1, 1.3, 2.55, 2.66, 5.1, 3.81)},
-               2: {64: (3.4, 0.7, 0.6, 5.46, 1.69, 2.6, 3.74)}}
+               2: {64: (3.2, 0.8, 0.5, 5.52, 1.82, 2.8, 3.67)}}
 _TIME_RAGGED = 3.0       # ... adding into features that end inside a tile of 64, and the same with K cut: a branch and a load an element
 _TIME_BIG = {0: {128: (1.9, 2.0, 2.9, 0.337, 0.197), 256: (2.4, 4.4, 4.2, 0.174, 0.239)},     # by the tile's rows; walk and fill by 32 x 32 of its area
              1: {128: (0.6, 3.6, 3.9, 0.341, 0.192), 256: (0.7, 3.9, 13.9, 0.203, 0.21)}, 2: {256: (2.2, 4.4, 2.1, 0.247, 0.144)}}
 _TIME_BIG_ODD = 4.0      # a round more of gated products with an odd number of features, which leave element by element
+# A gated product whose second round of large tiles is at most half full costs a step more than its own time: a burst at full power, then idle compute
+# units, behind which the step's attention and products run at a lower clock. With 2,048 x 4,608 over K 1,024 (288 tiles; alone 57.1 us on large tiles,
+# 56.4 on small ones) a prompt of 16,384 tokens took 27.1 ms against 25.9, with 5,120 features 27.8 against 26.7, 5,632 28.4 / 28.2, 6,144 28.9 / 28.7, with
+# 4,096 (one round) 23.6 against 24.3, 7,168 29.7 against 30.6; over K 2,048 4,608 features 4.73 ms a step against 4.67, 6,144 5.03 against 5.24.
+_TIME_BIG_BURST = 10.0         # from K 1,024 on, in proportion below
+# Large tiles level with those whose waves split K leave the product to the latter, for the same reason (2,048 x 2,048 adding over K 2,048: alone 27.2 us,
+# large tiles 26.3; in a prompt's step 32.5, 33.4; 1,111 x 2,048 and 3,072 storing: two prompts of 1,111 and 277 rows 3,198 us, large tiles 3,209)
+_TIE = 0.93
 # ... with K cut: start, a slice's part in the sum at the end, 1,024 k of a slice in each round and for 256 workgroups, 256 workgroups
 _TIME_SPLIT = {0: (8.3, 0.44, 4.6, 3.4, 1.5), 1: (7.3, 0.55, 4.8, 4.55, 4.0), 2: (8.3, 0.77, 8.7, 3.96, 2.5)}
 
 
 def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: float, walk: float, fill: float, each_pair: float = 0.0,
-                walk_pair: float = 0.0) -> float:
-    rounds, pairs = -(-tiles // DEEP_ROUND), -(-tiles // (2 * DEEP_ROUND))
+                walk_pair: float = 0.0, gated: bool = False) -> float:
+    rounds = -(-tiles // DEEP_ROUND)
+    pairs = max(1.0, rounds / 2) if gated else -(-rounds // 2)
     share = tiles / DEEP_ROUND
     return (start + rounds * each_round + share * each_tile + pairs * each_pair
             + K / 1024 * (rounds * walk + share * fill + pairs * walk_pair))
@@ -618,8 +628,8 @@ def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: 
 def tiled_plan(mode: int, M: int, N: int, K: int):
     """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
     256 columns), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through registers), "split" (those with K cut over
-    workgroups). The least estimated time decides: on the shapes that it was fitted to 0.2 % above the fastest in the
-    geometric mean, on 430 others 0.2 to 0.6 %. Fixed numbers of tiles were 10 % above it (storing, 1,111 rows by 2,048 features over K 8,192 97 us
+    workgroups). The least estimated time decides, with what a tie costs inside a step: on the shapes that it was fitted to 0.2 to 0.4 % above the fastest
+    alone in the geometric mean. Fixed numbers of tiles were 10 % above it (storing, 1,111 rows by 2,048 features over K 8,192 97 us
     against 57, 640 by 2,048 over 2,048 22 against 14, 1,300 by 3,072 over 2,048 44 against 28; gated, 1,111 by 4,608 over 2,048 63 against 46), adding
     products of up to 2,048 features held to the tiles whose waves split K 5 % (6,200 by 2,048 over 7,168 269 against 163, 2,690 by 1,536 over 1,024 32
     against 18; they keep what is one round over a long K: 2,048 by 2,048 over 4,096 41 against 48)."""
@@ -627,20 +637,23 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
     wide, narrow = -(-M // 128) * -(-N // 128), -(-M // 128) * -(-N // 64)
     columns = 64 if mode == 2 or wide < DEEP_ROUND or (wide == DEEP_ROUND and K < LONG_K) else 128        # as fw_gemm_mfma chooses
     ragged = _TIME_RAGGED if mode == 1 and N % 64 else 0.0
-    times = {("tiles", 0): _tiled_time(narrow if columns == 64 else wide, K, *_TIME_TILES[mode][columns]) + (ragged if columns == 64 else 0.0)}
+    times = {("tiles", 0): _tiled_time(narrow if columns == 64 else wide, K, *_TIME_TILES[mode][columns], gated=mode == 2) + (ragged if columns == 64 else 0.0)}
     if mode != 2:
         for columns in (128, 64):
             tiles = lib.fw_gemm_mfma_deep_tiles(mode, M, N, K, columns)
             if tiles:
-                times["deep", columns] = _tiled_time(tiles, K, *_TIME_DEEP[mode][columns]) * (_TIME_DEEP_FEW_ROWS if columns == 64 and M <= 384 and K > 2560 else 1.0)
+                few = columns == 64 and M <= 384 and K > 2560
+                times["deep", columns] = _tiled_time(tiles, K, *_TIME_DEEP[mode][columns]) * (_TIME_DEEP_FEW_ROWS if few else 1.0)
     if M > BIG_MIN_ROWS:
         rows, columns = ctypes.c_int(0), ctypes.c_int(0)
         tiles = lib.fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns))
         if tiles:
             start, each_round, each_tile, walk, fill = _TIME_BIG[mode][rows.value]
             area = rows.value * (256 if mode == 2 else columns.value) / 1024        # (a gated tile has gate and up columns)
-            odd = _TIME_BIG_ODD if mode == 2 and N % 2 else 0.0
-            times["big", 0] = _tiled_time(tiles, K, start, each_round + odd, each_tile, walk * area, fill * area)
+            if mode == 2:
+                each_round += _TIME_BIG_ODD if N % 2 else 0.0
+                start += _TIME_BIG_BURST * min(1.0, K / 1024) if DEEP_ROUND < tiles <= 3 * DEEP_ROUND // 2 else 0.0
+            times["big", 0] = _tiled_time(tiles, K, start, each_round, each_tile, walk * area, fill * area)
     need_bytes, tiles = _split_needs(mode, M, N, K)
     if need_bytes:
         slices = need_bytes // (tiles * 128 * (128 if mode == 2 else 64) * 4)
@@ -649,7 +662,10 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
         share = workgroups / DEEP_ROUND
         times["split", 0] = (start + ragged + each * slices + share * all_at_once
                              + K / 1024 / slices * (walk * -(-workgroups // DEEP_ROUND) + fill * share))
-    return min(times, key=times.get)
+    least = min(times, key=times.get)
+    if least == ("big", 0) and ("deep", 128) in times and times["deep", 128] * _TIE <= times[least]:
+        return "deep", 128
+    return least
 
 
 MEDIUM_MAX_ROWS = 64
