@@ -4,13 +4,16 @@
 // the path would be busy all the time, and the kernel is bound by it at a third of the peak.
 // Twice the tile edge halves the bytes per flop, in the memory path and in LDS alike:
 //
-//  * a workgroup of four waves computes 256 x 256; each wave a 128 x 128 quarter as 4 x 4 tiles of
-//    v_mfma_f32_32x32x16_bf16, its 256 accumulators in the accumulation registers; one wave per
-//    SIMD, so the overlap of loads, LDS reads and MFMAs is inside the wave;
-//  * 256 x 32 slabs of both operands travel from global memory STRAIGHT into LDS
+//  * a workgroup of four waves computes 256 x 256; each wave a 128 x 128 quarter as 8 x 8 tiles of
+//    v_mfma_f32_16x16x32_bf16, its 256 accumulators in the accumulation registers; one wave per
+//    SIMD, so the overlap of loads, LDS reads and MFMAs is inside the wave. (The same products on
+//    v_mfma_f32_32x32x16_bf16 move twice the accumulators per flop and draw more power: 8,192^3 at 1.45 GHz
+//    against 1.6. Both give the same bits.);
+//  * 256 x 64 slabs of both operands travel from global memory STRAIGHT into LDS
 //    (buffer_load_dwordx4 .. lds: no staging registers, which the accumulators leave no room for),
-//    three slabs ahead of the one being multiplied, four stages, one barrier per slab; rows are
-//    not padded, their chunks are stored permuted against bank conflicts;
+//    two stages of a and three of w in all 160 KB, one barrier per slab; a row of a slab is a whole cache
+//    line (slabs of 32 k ask L2 for every line in two halves: twice the requests, 11 of the 16 a clock that a
+//    die's L2 takes); rows are not padded, their chunks are stored permuted against bank conflicts;
 //  * workgroups are numbered so that each XCD works on a compact group of tiles.
 //
 // A product whose 256-row tiles would leave compute units idle takes tiles of 128 rows (each wave
@@ -28,20 +31,19 @@
 #include "grouped.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
 #define BT 256                  // tile edge (rows: of the tall tiles)
-#define BK 32                   // k per slab: an LDS row is 64 bytes, four 16-byte chunks
-#define BSTAGES 4               // slabs in LDS: one is multiplied, three are on their way
-#define BSLAB (BT * BK * 2)     // bytes of one operand's slab
+#define BK 32                   // k of one step of products: K is a multiple of it
+#define BLDS 163840             // bytes of LDS of a compute unit
 #define BK_MOST (1 << 22)
 #define BN_MOST (1 << 20)       // 256 rows of the output lie below BOUNDS
 #define BOUNDS 0x80000000u
 #define BGROUP_M 4
-#define B_LOADS 4               // most wave-wide loads (16 rows of 64 bytes) per wave per operand per slab
+#define B_LOADS 8               // most wave-wide loads (1,024 bytes) per wave per operand per slab
 
 enum { MB_STORE = 0, MB_ACCUMULATE = 1, MB_SWIGLU = 2 };
 
@@ -71,33 +73,50 @@ struct BigGroups {
     int experts;
 };
 
-template <int TM, int TN>
+// A slab: 64 k of the tile's rows (an LDS row is 128 bytes, eight 16-byte chunks), or 32 where two workgroups share a compute unit. Chunk
+// c of a row lies in slot c ^ swap(row): a read of 16 rows by four chunks goes in groups of 16 lanes, 0-3, 12-15 and 20-27, then the 16
+// others of the first 32, and every group covers all 64 banks once.
+template <int DEPTH>
+__device__ __forceinline__ int chunk_swap(int row) {
+    if (DEPTH == 64) return (row >> 1) & 7;
+    const int low = (row >> 2) & 1, high = (row >> 3) & 1;      // 0, 2, 3, 1 for four rows each
+    return (low ^ high) * 2 + high;
+}
+
+template <int TM, int TN, int DEPTH>
 struct BigTile {
     static constexpr int ROWS = 2 * TM * 32;               // rows of a tile
     static constexpr int WIDE = 2 * TN * 32;               // columns of a tile
-    static constexpr int A_LOADS = ROWS / 64;              // wave-wide loads per wave for a slab of a (16 rows each)
-    static constexpr int W_LOADS = WIDE / 64;              // and for a slab of w
+    static constexpr int A_SLAB = ROWS * DEPTH * 2, W_SLAB = WIDE * DEPTH * 2;     // bytes
+    static constexpr int A_LOADS = A_SLAB / 4096;          // wave-wide loads per wave for a slab of a (1,024 bytes each)
+    static constexpr int W_LOADS = W_SLAB / 4096;          // and for a slab of w
     static constexpr int SLAB_LOADS = A_LOADS + W_LOADS;   // and for a slab of both operands
+    // slabs in LDS, the one that is multiplied among them: as many of both as fit, and one more of w if it fits beside them
+    static constexpr int LDS_MOST = DEPTH == 64 ? BLDS : BLDS / 2;
+    static constexpr int A_STAGES = LDS_MOST / (A_SLAB + W_SLAB) < 4 ? LDS_MOST / (A_SLAB + W_SLAB) : 4;
+    static constexpr int W_STAGES = A_STAGES < 3 && A_STAGES * A_SLAB + (A_STAGES + 1) * W_SLAB <= LDS_MOST ? A_STAGES + 1 : A_STAGES;
+    static constexpr int LDS = A_STAGES * A_SLAB + W_STAGES * W_SLAB;
 };
 
 // K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way), and at most BK_MOST (a
 // lane's place in a tile's 256 rows is 32 bits, as it is in the output: N at most BN_MOST).
 //
-// Bound by the matrix cores at the clock that their power leaves (1.5 to 1.7 GHz in long runs): 65 % of a wave's cycles in MFMAs inside a
-// prompt's step, 72 % of the gated product alone, 76 % of 8,192^3; the rest between the steps and at a tile's start and end. 2,048 x 8,192 gated x 2,048: 128.2 -> 117.5 us against reads and loads
-// spread over whole steps with 64-bit addresses in vector registers; 2,048 x 6,144: 51.9 -> 49.4; 8,192^3: 1,185 -> 1,296 TFLOP/s.
-// One barrier for two slabs (five stages) gave nothing more.
-// TN: 32-column product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144
+// Bound by the matrix cores at the clock that their power leaves (1.5 to 1.9 GHz): 77 % of a wave's cycles in MFMAs at 8,192^3, the rest at a tile's
+// start and end and where a slab's loads are waited for. Against slabs of 32 k on v_mfma_f32_32x32x16_bf16: 2,048 x 8,192 gated x 2,048 120.8 -> 104.7 us
+// (1,310 TFLOP/s), storing 2,048 x 6,144 x 2,048 52.8 -> 44.0, 2,048 x 3,072 x 2,048 30.7 -> 25.4, 1,111 x 16,384 x 2,048 90.4 -> 79.0, 8,192^3 1,254 -> 1,470
+// TFLOP/s. Where the loads stand among the MFMAs (behind every second to every eighth) changed nothing; two stages of w instead of three cost 1 to 8 %.
+// TN: 32-column pairs of product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144
 // features gives 192 tiles of 256 columns for 256 compute units, but exactly 256 tiles of 192).
-// TM: 32-row product tiles per wave, 4 (256 rows a tile) or 2 (128 rows).
-template <int MODE, typename TO, int TN, int TM, int STAGES, bool GROUPED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3 ? 2 : 1, STAGES == 3 ? 2 : 1))) void gemm_mfma_big_kernel(
+// TM: 32-row pairs of product tiles per wave, 4 (256 rows a tile) or 2 (128 rows). DEPTH: k of a slab, see BigTile.
+template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32 ? 2 : 1, DEPTH == 32 ? 2 : 1))) void gemm_mfma_big_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const float* __restrict__ bias,
     TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups) {
-    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [stage][a slab | w slab]
-    constexpr int ROWS = BigTile<TM, TN>::ROWS, WIDE = BigTile<TM, TN>::WIDE;
-    constexpr int A_LOADS = BigTile<TM, TN>::A_LOADS, W_LOADS = BigTile<TM, TN>::W_LOADS, SLAB_LOADS = BigTile<TM, TN>::SLAB_LOADS;
-    constexpr int A_SLAB = ROWS * BK * 2, STAGE = A_SLAB + WIDE * BK * 2;       // bytes
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [A_STAGES slabs of a][W_STAGES slabs of w]
+    typedef BigTile<TM, TN, DEPTH> Tile;
+    constexpr int ROWS = Tile::ROWS, WIDE = Tile::WIDE, A_SLAB = Tile::A_SLAB, W_SLAB = Tile::W_SLAB, A_STAGES = Tile::A_STAGES, W_STAGES = Tile::W_STAGES;
+    constexpr int A_LOADS = Tile::A_LOADS, W_LOADS = Tile::W_LOADS, SLAB_LOADS = Tile::SLAB_LOADS;
+    constexpr int PARTS = DEPTH / BK, CHUNKS = DEPTH / 8, LOAD_ROWS = 64 / CHUNKS;      // steps of a slab, chunks of a row, rows of a wave-wide load
     const int features = MODE == MB_SWIGLU ? BT / 2 : WIDE;
     static_assert(MODE != MB_SWIGLU || TN == 4, "the gated tile holds 128 gate and 128 up rows");
     int m0, n0;
@@ -130,11 +149,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3
     const int wm = wave >> 1, wn = wave & 1;
 
     // The copy: a wave-wide load writes 1,024 contiguous bytes of LDS, lane l its 16 bytes at
-    // l * 16: 16 rows of 64 bytes. Rows are not padded; instead the four chunks of a row are
-    // stored permuted (chunk c of row r in slot c ^ ((r / 4) % 4)), so that the 16-byte operand
-    // reads of 16 consecutive rows cover all 64 banks once (rows r, r + 4, r + 8, r + 12 would
-    // otherwise share theirs). Lane l therefore ASKS for chunk (l % 4) ^ ((r / 4) % 4) of row
-    // r = l / 4 of its 16 rows. Addresses are a base that the wave shares (the tile's first row; of a gated
+    // l * 16: 8 rows of 128 bytes (16 of 64). Rows are not padded; instead the chunks of a row are
+    // stored permuted (chunk_swap): lane l therefore ASKS for the chunk whose slot it fills. Addresses are a base that the wave shares (the tile's first row; of a gated
     // product's w the first gate or up row: a wave's loads of w are all of one kind), a 32-bit
     // offset of the lane, and the slab's offset in a scalar register: a slab costs no vector arithmetic.
     const int w_part = MODE == MB_SWIGLU && wave >= 2 ? 1 : 0;
@@ -144,170 +160,224 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3
     uint32_t a_at[A_LOADS], w_at[B_LOADS];
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
-        const int row = (wave * A_LOADS + i) * 16 + (lane >> 2);
-        const int chunk = (lane & 3) ^ ((row >> 2) & 3);
+        const int row = (wave * A_LOADS + i) * LOAD_ROWS + lane / CHUNKS;
+        const int chunk = (lane % CHUNKS) ^ chunk_swap<DEPTH>(row);
         uint32_t from = row < M - m0 ? row : M - m0 - 1;        // rows past the end are computed and dropped
         if (GROUPED && groups_rows) from = groups_rows[m0 + (int)from];
         a_at[i] = from * (uint32_t)(2 * K) + chunk * 16;
     }
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
-        const int row = (wave * W_LOADS + i) * 16 + (lane >> 2);
-        const int chunk = (lane & 3) ^ ((row >> 2) & 3);
+        const int row = (wave * W_LOADS + i) * LOAD_ROWS + lane / CHUNKS;
+        const int chunk = (lane % CHUNKS) ^ chunk_swap<DEPTH>(row);
         const int of_part = MODE == MB_SWIGLU ? row - w_part * (BT / 2) : row;
         w_at[i] = (uint32_t)(of_part < N - n0 ? of_part : N - n0 - 1) * (uint32_t)(2 * K) + chunk * 16;
     }
     const fw_buffer a_rows = fw_make_buffer(a_base), w_rows = fw_make_buffer(w_base);
-    // loads from .. to - 1 of this wave's SLAB_LOADS for a slab
-    auto request_part = [&](int slab, int from, int to) {
-        unsigned char* stage = lds + (slab % STAGES) * STAGE;
-        const int k0 = slab * (BK * 2);
+    // This wave's loads for a slab of either operand, into the stage at `stage`. A last slab of half the length has no upper
+    // chunks: the lower ones are read again in their place and never used.
+    const int whole = K / DEPTH, slabs = (K + DEPTH - 1) / DEPTH;
+    auto request_a = [&](int stage, int slab, int i) { fw_buffer_to_lds(a_rows, lds + stage + (wave * A_LOADS + i) * 1024, a_at[i], slab * (DEPTH * 2)); };
+    auto request_w = [&](int stage, int slab, int i) { fw_buffer_to_lds(w_rows, lds + stage + (wave * W_LOADS + i) * 1024, w_at[i], slab * (DEPTH * 2)); };
+    auto upper = [&](int first_row) { return ((lane % CHUNKS) ^ chunk_swap<DEPTH>(first_row + lane / CHUNKS)) >= CHUNKS / 2; };
+    auto request_slab_a = [&](int stage, int slab) {
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i)
-            if (i >= from && i < to) fw_buffer_to_lds(a_rows, stage + (wave * A_LOADS + i) * 1024, a_at[i], k0);
-#pragma unroll
-        for (int i = 0; i < W_LOADS; ++i)
-            if (A_LOADS + i >= from && A_LOADS + i < to) fw_buffer_to_lds(w_rows, stage + A_SLAB + (wave * W_LOADS + i) * 1024, w_at[i], k0);
+        for (int i = 0; i < A_LOADS; ++i) {
+            if (PARTS == 2 && slab >= whole && upper((wave * A_LOADS + i) * LOAD_ROWS)) a_at[i] -= BK * 2;
+            request_a(stage, slab, i);
+        }
     };
-    auto request = [&](int slab) { request_part(slab, 0, SLAB_LOADS); };
+    auto request_slab_w = [&](int stage, int slab) {
+#pragma unroll
+        for (int i = 0; i < W_LOADS; ++i) {
+            if (PARTS == 2 && slab >= whole && upper((wave * W_LOADS + i) * LOAD_ROWS)) w_at[i] -= BK * 2;
+            request_w(stage, slab, i);
+        }
+    };
 
-    f32x16 acc[TM][TN];
+    constexpr int TA = 2 * TM, TB = 2 * TN;     // 16-row and 16-column product tiles of the wave
+    f32x4 acc[TA][TB];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TA; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+        for (int j = 0; j < TB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // this wave's rows of the a slab, and its rows of the w slab: for SwiGLU the columns of a wave
-    // are 64 gate features (tiles 0, 1) and the 64 up features of the same columns (tiles 2, 3)
-    const int a_row0 = wm * (TM * 32) + (lane & 31);
-    int b_row[TN];
+    // are 64 gate features (tiles 0 to 3) and the 64 up features of the same columns (tiles 4 to 7).
+    // Every row this lane reads is (lane % 16) plus a multiple of 16: one permutation for all
+    int slot[PARTS];
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
-        b_row[j] = MODE == MB_SWIGLU ? (j >> 1) * (BT / 2) + wn * 64 + (j & 1) * 32 + (lane & 31) : wn * (TN * 32) + j * 32 + (lane & 31);
-    // every row this lane reads is (lane % 32) plus a multiple of 32: one permutation for all
-    const int swizzle = ((lane & 31) >> 2) & 3;
-    int slot[BK / 16];
-#pragma unroll
-    for (int t = 0; t < BK / 16; ++t) slot[t] = ((2 * t + (lane >> 5)) ^ swizzle) * 16;
+    for (int t = 0; t < PARTS; ++t) slot[t] = ((4 * t + (lane >> 4)) ^ chunk_swap<DEPTH>(lane & 15)) * 16;
+    const int a_row0 = wm * (TM * 32) + (lane & 15), b_row0 = (MODE == MB_SWIGLU ? wn * 64 : wn * (TN * 32)) + (lane & 15);
 
-    // operand registers of one k16 step: the wave's row tiles of a and column tiles of w
+    // operand registers of one step: the wave's row tiles of a and column tiles of w
     struct Operands {
-        bf16x8 fa[TM], fb[TN];
+        bf16x8 fa[TA], fb[TB];
     };
-    auto read = [&](Operands& f, int slab, int t) {
-        const unsigned char* sa = lds + (slab % STAGES) * STAGE;
-        const unsigned char* sb = sa + A_SLAB;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-            f.fa[i] = *reinterpret_cast<const bf16x8*>(sa + (a_row0 + 32 * i) * (BK * 2) + slot[t]);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-            f.fb[j] = *reinterpret_cast<const bf16x8*>(sb + b_row[j] * (BK * 2) + slot[t]);
+    constexpr int MFMAS = TA * TB, READS = TA + TB;
+    constexpr int W_FIRST = A_STAGES * A_SLAB, W_END = W_FIRST + W_STAGES * W_SLAB;
+    // the stages of slab s and the one behind it, and of w the one ahead of it
+    int a_now = 0, a_then = A_SLAB, w_now = W_FIRST, w_then = W_FIRST + W_SLAB, w_before = W_END - W_SLAB;
+    auto advance = [&]() {
+        a_now = a_then;
+        a_then = a_then + A_SLAB < W_FIRST ? a_then + A_SLAB : 0;
+        w_before = w_now;
+        w_now = w_then;
+        w_then = w_then + W_SLAB < W_END ? w_then + W_SLAB : W_FIRST;
     };
-    auto multiply = [&](const Operands& f, int first_row_tile, int row_tiles) {
-#pragma unroll
-        for (int i = first_row_tile; i < first_row_tile + row_tiles; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.fa[i], f.fb[j], acc[i][j], 0, 0, 0);
+    auto read_one = [&](Operands& f, int a_stage, int w_stage, int part, int which) {
+        if (which < TA) {
+            f.fa[which] = *reinterpret_cast<const bf16x8*>(lds + a_stage + slot[part] + (a_row0 + 16 * which) * (DEPTH * 2));
+        } else {
+            const int j = which - TA, row = MODE == MB_SWIGLU ? (j >> 2) * (BT / 2) + (j & 3) * 16 : j * 16;
+            f.fb[j] = *reinterpret_cast<const bf16x8*>(lds + w_stage + slot[part] + (b_row0 + row) * (DEPTH * 2));
+        }
     };
-    // Asks the scheduler to issue `count` times: `mfmas` MFMAs, then one instruction of `kind`
-    // (0x100 LDS read, 0x020 global load). A wave issues in order and an MFMA holds the matrix
-    // pipe for 32 clocks, so whatever sits between two MFMAs costs nothing.
-#define FW_INTERLEAVE(count, mfmas, kind)                          \
-    _Pragma("unroll") for (int u = 0; u < (count); ++u) {          \
-        __builtin_amdgcn_sched_group_barrier(0x008, (mfmas), 0);   \
-        __builtin_amdgcn_sched_group_barrier((kind), 1, 0);        \
-    }
+    auto read = [&](Operands& f, int a_stage, int w_stage, int part) {
+#pragma unroll
+        for (int u = 0; u < READS; ++u) read_one(f, a_stage, w_stage, part, u);
+    };
+    // product tile number `which`, row by row, every second row backwards
+    auto multiply_one = [&](const Operands& f, int which) {
+        const int i = which / TB, j = i & 1 ? TB - 1 - which % TB : which % TB;
+        if constexpr (DEPTH == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.fa[i], f.fb[j], acc[i][j], 0, 0, 0);
+        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f.fa[i]), "v"(f.fb[j]));
+    };
+    auto multiply = [&](const Operands& f) {
+#pragma unroll
+        for (int u = 0; u < MFMAS; ++u) multiply_one(f, u);
+    };
     // Tells the compiler that these operands are needed HERE, so that it waits for their LDS reads
     // before the next reads are issued and not, for all reads together, in front of the MFMAs.
     auto arrived = [&](const Operands& f) {
-        asm volatile("" ::"v"(f.fa[0]), "v"(f.fa[1]), "v"(f.fa[TM - 2]), "v"(f.fa[TM - 1]), "v"(f.fb[0]), "v"(f.fb[1]), "v"(f.fb[2]), "v"(f.fb[TN - 1]));
+#pragma unroll
+        for (int i = 0; i < TA; i += 2) asm volatile("" ::"v"(f.fa[i]), "v"(f.fa[i + 1]));
+#pragma unroll
+        for (int j = 0; j < TB; j += 2) asm volatile("" ::"v"(f.fb[j]), "v"(f.fb[j + 1]));
+        // two wait states between moves that have written an operand or an accumulator and the product that reads it: the compiler
+        // does not see a product in the assembly
+        asm volatile("s_nop 1");
     };
-    // waits until at most `slabs` of this wave's requested slabs are still on their way (SLAB_LOADS loads each)
+    // waits until at most `slabs` of this wave's requested slabs (of both operands, or of w alone where w has a stage more) are still on their way
+    constexpr int EACH = W_STAGES > A_STAGES ? W_LOADS : SLAB_LOADS;
     auto wait_for_all_but = [&](int slabs) {
-        if (slabs >= 3) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * SLAB_LOADS) : "memory");
-        else if (slabs == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * SLAB_LOADS) : "memory");
-        else if (slabs == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 * SLAB_LOADS) : "memory");
+        if (slabs >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * EACH) : "memory");
+        else if (slabs == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(1 * EACH) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     };
 
-    // Four stages: while slab s is multiplied, slabs s + 1 .. s + 3 are in LDS or on their way.
-    // The two k16 steps of a slab are software-pipelined by hand, because with one wave per SIMD
-    // nothing else hides the latency of LDS: the operands of the next step are read behind the first
-    // MFMAs of this one, a read each, so that they have arrived when the step is through. Between
-    // the two steps the wave makes sure that slab s + 1 has landed (its own loads: vmcnt;
-    // everybody's: the barrier), which also tells that every wave has read the last of slab s,
-    // whose stage then takes slab s + 4. Its loads are issued behind every second one of the later MFMAs, half
-    // of them in the next slab's step 0: a compute unit takes a wave's load in 16 clocks, and four
-    // waves that each issued one behind every MFMA (32 clocks) stood still at them.
-    const int steps = K / BK;
-    for (int s = 0; s < STAGES && s < steps; ++s) request(s);
-    wait_for_all_but((steps < STAGES ? steps : STAGES) - 1);
+    // With one wave per SIMD nothing else hides the latency of LDS: the operands of a step are read behind the MFMAs of the step
+    // before it. Ahead of a slab's last step the wave makes sure that the next slab has landed (its own loads: vmcnt; everybody's: the
+    // barrier), which also tells that every wave has read slab s. Its stages then take the slabs that come A_STAGES and W_STAGES later:
+    // that of a behind the MFMAs of the slab's last step, that of w behind those of the next slab's first (where a slab is one
+    // step, both behind its later MFMAs).
+    for (int u = 0; u < W_STAGES - 1; ++u) {
+        if (u < slabs) request_slab_a(u * A_SLAB, u);
+        if (u < slabs) request_slab_w(W_FIRST + u * W_SLAB, u);
+    }
+    if (A_STAGES == W_STAGES && A_STAGES <= slabs) request_slab_a((A_STAGES - 1) * A_SLAB, A_STAGES - 1);
+    if (PARTS == 1 && W_STAGES <= slabs) request_slab_w(W_END - W_SLAB, W_STAGES - 1);
+    if (slabs >= W_STAGES) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((A_STAGES - 1) * A_LOADS + (W_STAGES - (PARTS == 1 ? 1 : 2)) * W_LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     Operands f0, f1;
-    read(f0, 0, 0);
+    read(f0, a_now, w_now, 0);
     int s = 0;
-    constexpr int EARLY = SLAB_LOADS / 2;
-    // (where the reads outnumber the MFMAs the rest is left to the scheduler)
-#define FW_STEP_SCHEDULE()                                                                   \
-    FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)                          \
-    FW_INTERLEAVE((TM + TN < TM * TN ? (TM * TN - TM - TN) / 2 : 0), 2, 0x020)                \
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + STAGES < steps) {
-        read(f1, 0, 1);
-        multiply(f0, 0, TM);
-        FW_INTERLEAVE((TM + TN < TM * TN ? TM + TN : TM * TN), 1, 0x100)
-        __builtin_amdgcn_sched_barrier(0);
-        // a turn: step 1 of slab s and step 0 of slab s + 1, with the loads of slab s + STAGES. Nothing in it is
-        // conditional, so that each step is one run of instructions the scheduler can interleave
-        do {
-            arrived(f1);                                    // slab s has been read
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * SLAB_LOADS) : "memory");   // slab s + 1 has landed; those behind it may still fly
-            __builtin_amdgcn_s_barrier();
-            read(f0, s + 1, 0);
-            request_part(s + STAGES, 0, EARLY);
-            multiply(f1, 0, TM);
-            FW_STEP_SCHEDULE()
-            read(f1, s + 1, 1);
-            request_part(s + STAGES, EARLY, SLAB_LOADS);
-            multiply(f0, 0, TM);
-            FW_STEP_SCHEDULE()
-            ++s;
-        } while (s + STAGES < steps);
-        // step 1 of slab s = steps - STAGES, of which step 0 is done
-        arrived(f1);
-        wait_for_all_but(STAGES - 2);
+    // two MFMAs (32 clocks) to a read: four waves that read at once keep LDS busy for as long
+    constexpr int READ_GAP = 2 * READS <= MFMAS ? 2 : 1, A_GAP = MFMAS / A_LOADS, W_GAP = MFMAS / W_LOADS;
+    auto landed = [&](const Operands& f) {
+        arrived(f);                                         // slab s has been read
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((W_STAGES - 2) * EACH) : "memory");   // slab s + 1 has landed; those behind it may still fly
         __builtin_amdgcn_s_barrier();
-        read(f0, s + 1, 0);
-        multiply(f1, 0, TM);
-        __builtin_amdgcn_sched_barrier(0);
-        ++s;
-    }
-#undef FW_STEP_SCHEDULE
-    // the last slabs: nothing more to request
-    for (; s < steps; ++s) {
-        arrived(f0);
-        read(f1, s, 1);
-        multiply(f0, 0, TM);
-        __builtin_amdgcn_sched_barrier(0);
-        arrived(f1);
-        if (s + 1 < steps) {
-            wait_for_all_but(steps - 2 - s);                // slabs s + 2 .. may still fly
-            __builtin_amdgcn_s_barrier();
-            read(f0, s + 1, 0);
+    };
+    if constexpr (PARTS == 2) {
+        while (s + A_STAGES < whole) {
+            arrived(f0);
+#pragma unroll
+            for (int u = 0; u < MFMAS; ++u) {
+                if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f1, a_now, w_now, 1, u / READ_GAP);
+                if (u % W_GAP == 0 && u / W_GAP < W_LOADS) request_w(w_before, s + W_STAGES - 1, u / W_GAP);
+                multiply_one(f0, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            landed(f1);
+#pragma unroll
+            for (int u = 0; u < MFMAS; ++u) {
+                if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f0, a_then, w_then, 0, u / READ_GAP);
+                if (u % A_GAP == 0 && u / A_GAP < A_LOADS) request_a(a_now, s + A_STAGES, u / A_GAP);
+                multiply_one(f1, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            advance();
+            ++s;
         }
-        multiply(f1, 0, TM);
-        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        auto step = [&](const Operands& now, Operands& next) {
+            landed(now);
+#pragma unroll
+            for (int u = 0; u < MFMAS; ++u) {
+                if (u < READS) read_one(next, a_then, w_then, 0, u);
+                const int load = (u - READS) / 2;
+                if (u >= READS && (u - READS) % 2 == 0 && load < A_LOADS) request_a(a_now, s + A_STAGES, load);
+                if (u >= READS && (u - READS) % 2 == 0 && load >= A_LOADS && load < SLAB_LOADS) request_w(w_now, s + W_STAGES, load - A_LOADS);
+                multiply_one(now, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            advance();
+            ++s;
+        };
+        static_assert(PARTS == 2 || READS + 2 * SLAB_LOADS <= MFMAS, "the loads have MFMAs to go behind");
+        while (s + A_STAGES + 1 < slabs) {                  // two slabs a turn, so that the operand sets keep their names
+            step(f0, f1);
+            step(f1, f0);
+        }
     }
-#undef FW_INTERLEAVE
+    // the last slabs: asking for what is left to ask for; one of two steps may have half the length
+    for (; s < slabs; ++s) {
+        const int ahead = (slabs < s + W_STAGES ? slabs : s + W_STAGES) - (s + 2);      // slabs behind s + 1 that have been asked for
+        arrived(f0);
+        if constexpr (PARTS == 2) {
+            if (s < whole) read(f1, a_now, w_now, 1);
+            if (s + W_STAGES - 1 < slabs) request_slab_w(w_before, s + W_STAGES - 1);
+            multiply(f0);
+            __builtin_amdgcn_sched_barrier(0);
+            arrived(f1);
+        }
+        if (s + 1 < slabs) {
+            wait_for_all_but(ahead);
+            __builtin_amdgcn_s_barrier();
+            read(PARTS == 2 ? f0 : f1, a_then, w_then, 0);
+            if (s + A_STAGES < slabs) request_slab_a(a_now, s + A_STAGES);
+            if (PARTS == 1 && s + W_STAGES < slabs) request_slab_w(w_now, s + W_STAGES);
+        }
+        if constexpr (PARTS == 2) {
+            if (s < whole) multiply(f1);
+        } else {
+            multiply(f0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (s + 1 < slabs) {
+                arrived(f1);
+                f0 = f1;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        advance();
+    }
     fw_mfma_drain();     // branches follow that lead to code reading the accumulators
 
-    // D layout of the 32x32 product: lane holds column lane % 32; register r is row
-    // 8 * (r / 4) + 4 * (lane / 32) + r % 4
-    const int col = lane & 31, row_base = (lane >> 5) * 4;
+    // D layout of the 16x16 product: lane holds column lane % 16, register r is row 4 * (lane / 16) + r. Two neighbouring
+    // column tiles swap every second 16 lanes, so that a lane holds column lane % 32 of the pair and eight rows
+    // 8 * (lane / 32) + u of the row tile: a store then covers whole runs of 32 columns.
+    const int col = lane & 31, row_base = (lane >> 5) * 8;
+    auto paired = [](const float (&left)[4], const float (&right)[4], float (&rows)[8]) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const auto swapped = __builtin_amdgcn_permlane16_swap(__float_as_uint(left[r]), __float_as_uint(right[r]), false, false);
+            const uint32_t upper = swapped[0], lower = swapped[1];
+            rows[r] = __uint_as_float(upper);
+            rows[4 + r] = __uint_as_float(lower);
+        }
+    };
     // The output leaves through a buffer that ends behind the tile's last row, so that rows past the end are dropped by its
     // bounds and a lane of a column past the end by a place beyond them: no branch. (With a branch an element the last tile
     // of a ragged product took 5 us longer than a whole one, with one only a row 4 us: 192 x 1,536 gated x 1,024 28.7 us
@@ -322,50 +392,61 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3
     // (the grouped product has the unit of its form for few places, bit for bit)
     auto unit = [](float g) { return GROUPED ? silu_big(g) : silu_quick(g); };
     const uint32_t first_row = (uint32_t)(wm * (TM * 32) + row_base);      // of this lane, of the tile
+    // the eight rows of row tile i and pair j of column tiles that this lane holds: gated, or with the bias
+    constexpr int PAIRS = MODE == MB_SWIGLU ? 2 : TN;
+    auto values = [&](int i, int j, float b, float (&rows)[8]) {
+        float left[4], right[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (MODE == MB_SWIGLU) {
+                left[r] = fw_gate_of<TO>(acc[i][2 * j][r], unit) * acc[i][2 * j + 4][r];
+                right[r] = fw_gate_of<TO>(acc[i][2 * j + 1][r], unit) * acc[i][2 * j + 5][r];
+            } else {
+                left[r] = acc[i][2 * j][r];
+                right[r] = acc[i][2 * j + 1][r];
+            }
+        }
+        paired(left, right, rows);
+        if constexpr (MODE != MB_SWIGLU)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) rows[u] = fw_before_store<TO>(rows[u] + b);
+    };
     if (SIZE == 4 || ((N & 1) == 0 && (uintptr_t)out % 4 == 0)) {
 #pragma unroll
-        for (int j = 0; j < (MODE == MB_SWIGLU ? 2 : TN); ++j) {
+        for (int j = 0; j < PAIRS; ++j) {
             const int c = (MODE == MB_SWIGLU ? wn * 64 : wn * (TN * 32)) + j * 32 + col;        // column of the tile
             const bool there = n0 + c < N;
+            const float b = MODE != MB_SWIGLU && bias && there ? bias[n0 + c] : 0.0f;
             if constexpr (SIZE == 4) {
-                const float b = bias && there ? bias[n0 + c] : 0.0f;
                 const uint32_t at = there ? first_row * row_step + c * 4 : BOUNDS;
-                float old[MODE == MB_ACCUMULATE ? TM * 16 : 1];
+                float old[MODE == MB_ACCUMULATE ? TA * 8 : 1];
                 if constexpr (MODE == MB_ACCUMULATE) {
 #pragma unroll
-                    for (int u = 0; u < TM * 16; ++u)
-                        old[u] = fw_buffer_load_float(to, at + (uint32_t)((u >> 4) * 32 + 8 * ((u & 15) >> 2) + (u & 3)) * row_step);
+                    for (int u = 0; u < TA * 8; ++u) old[u] = fw_buffer_load_float(to, at + (uint32_t)((u >> 3) * 16 + (u & 7)) * row_step);
                 }
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < TA; ++i) {
+                    float rows[8];
+                    values(i, j, b, rows);
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        float value = acc[i][j][r] + b;
-                        if (MODE == MB_ACCUMULATE) value += old[i * 16 + r];
-                        fw_buffer_store(to, at + (uint32_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * row_step, __builtin_bit_cast(uint32_t, value));
+                    for (int u = 0; u < 8; ++u) {
+                        if (MODE == MB_ACCUMULATE) rows[u] += old[i * 8 + u];
+                        fw_buffer_store(to, at + (uint32_t)(i * 16 + u) * row_step, __builtin_bit_cast(uint32_t, rows[u]));
                     }
+                }
             } else {
-                const float b = MODE != MB_SWIGLU && bias && there ? bias[n0 + c] : 0.0f;
                 const uint32_t at = there ? (first_row + (odd ? 1 : 0)) * row_step + (c & ~1) * 2 : BOUNDS;
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < TA; ++i) {
+                    float rows[8];
+                    values(i, j, b, rows);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const int r = 4 * q + 2 * h;        // rows 8 q + 2 h and the one below, of row tile i
-                            float upper, lower;
-                            if constexpr (MODE == MB_SWIGLU) {
-                                upper = fw_gate_of<TO>(acc[i][j][r], unit) * acc[i][j + 2][r];
-                                lower = fw_gate_of<TO>(acc[i][j][r + 1], unit) * acc[i][j + 2][r + 1];
-                            } else {
-                                upper = fw_before_store<TO>(acc[i][j][r] + b);
-                                lower = fw_before_store<TO>(acc[i][j][r + 1] + b);
-                            }
-                            const float got = from_neighbour(odd ? upper : lower);
-                            const uint32_t word = odd ? pack_bf16x2(got, lower) : pack_bf16x2(upper, got);
-                            fw_buffer_store(to, at + (uint32_t)(i * 32 + 8 * q + 2 * h) * row_step, word);
-                        }
+                    for (int u = 0; u < 8; u += 2) {
+                        const float got = from_neighbour(odd ? rows[u] : rows[u + 1]);
+                        const uint32_t word = odd ? pack_bf16x2(got, rows[u + 1]) : pack_bf16x2(rows[u], got);
+                        fw_buffer_store(to, at + (uint32_t)(i * 16 + u) * row_step, word);
+                    }
+                }
             }
         }
         return;
@@ -374,33 +455,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(STAGES == 3
     // (with two an element 5,532 x 83 x 608 took 19.0 us against 11.5, 1,300 x 3,071 x 1,024 25.7 against 18.3).
     if constexpr (SIZE == 2) {
 #pragma unroll
-        for (int j = 0; j < (MODE == MB_SWIGLU ? 2 : TN); ++j) {
+        for (int j = 0; j < PAIRS; ++j) {
             const int c = (MODE == MB_SWIGLU ? wn * 64 : wn * (TN * 32)) + j * 32 + col;
             const bool there = n0 + c < N;
             const float b = MODE != MB_SWIGLU && bias && there ? bias[n0 + c] : 0.0f;
             const uint32_t at = there ? first_row * row_step + c * 2 : BOUNDS;
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TA; ++i) {
+                float rows[8];
+                values(i, j, b, rows);
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    float value;
-                    if constexpr (MODE == MB_SWIGLU) value = fw_gate_of<TO>(acc[i][j][r], unit) * acc[i][j + 2][r];
-                    else value = fw_before_store<TO>(acc[i][j][r] + b);
-                    fw_buffer_store(to, at + (uint32_t)(i * 32 + 8 * (r >> 2) + (r & 3)) * row_step, float_to_bf16_bits(value));
-                }
+                for (int u = 0; u < 8; ++u) fw_buffer_store(to, at + (uint32_t)(i * 16 + u) * row_step, float_to_bf16_bits(rows[u]));
+            }
         }
     }
 }
 
-template <int MODE, typename TO, int TN, int TM, int STAGES, bool GROUPED>
+template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED>
 static int launch_tiles(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, int tiles_m, const BigGroups& groups,
                         hipStream_t stream) {
-    const int tiles_n = fw_ceil_div(N, MODE == MB_SWIGLU ? BT / 2 : BigTile<TM, TN>::WIDE);
+    const int tiles_n = fw_ceil_div(N, MODE == MB_SWIGLU ? BT / 2 : BigTile<TM, TN, DEPTH>::WIDE);
     const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n, 8);
-    const int lds_bytes = STAGES * (BigTile<TM, TN>::ROWS + BigTile<TM, TN>::WIDE) * BK * 2;
+    const int lds_bytes = BigTile<TM, TN, DEPTH>::LDS;
     static bool configured = false;     // per instantiation
     if (!configured) {
-        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, STAGES, GROUPED>,
+        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (status != hipSuccess) {
             fw_set_error("gemm_mfma_big: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(status));
@@ -408,19 +487,22 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
         }
         configured = true;
     }
-    gemm_mfma_big_kernel<MODE, TO, TN, TM, STAGES, GROUPED><<<per_xcd * 8, 256, lds_bytes, stream>>>(
+    gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED><<<per_xcd * 8, 256, lds_bytes, stream>>>(
         (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups);
     return 0;
 }
 template <int MODE, typename TO, int TN = 4, int TM = 4>
 static int launch_big(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, hipStream_t stream) {
-    return launch_tiles<MODE, TO, TN, TM, BSTAGES, false>(a, w, bias, out, M, N, K, fw_ceil_div(M, BigTile<TM, TN>::ROWS), BigGroups(), stream);
+    return launch_tiles<MODE, TO, TN, TM, 64, false>(a, w, bias, out, M, N, K, fw_ceil_div(M, BigTile<TM, TN, 64>::ROWS), BigGroups(), stream);
 }
 
 // The grouped product of fw_grouped_gemm on tiles of 128 places by 256 rows of W, for K a multiple of 32 and a of less than 4 GB. Bound by
 // the experts' weights from memory (600 MB for both products of 32 experts of 1,536 features: 127 us) and by tiles that an expert's last places fill partly.
-// Two workgroups share a compute unit (three stages of 24 KB each), so that one multiplies while the other starts, ends or waits. 2,048 rows, 4 of 32
-// experts, gated 1,536 over 2,048: 158 us; with four stages and one workgroup 175, on tiles of 256 places 186; through registers (moe.hip) 241.
+// Slabs of 64 k leave room for one workgroup on a compute unit, slabs of 32 for two (three stages of 24 KB each), of which one multiplies while the other
+// starts, ends or waits: a short K and experts of less than a tile of places, whose weights are the load, take the latter. us, slabs of 64 / 32, gated and
+// down: 2,048 rows, 4 of 32 experts, 1,536 features over 2,048 146 / 147 and 90 / 99, 1,111 rows 108 / 115 and 49 / 53, 600 rows 109 / 105 and 37 / 37; 1,500
+// rows, 2 of 8 over 4,096 97 / 110; 3,000 rows, 4 of 16 over 1,280 91 / 85; 2,048 rows, 2 of 8 over 1,024 57 / 52, 6 of 64 62 / 54. (On v_mfma_f32_32x32x16_bf16 with
+// slabs of 32: 154 and 102, 120 and 57; tiles of 256 places 186; through registers, moe.hip, 241.)
 bool fw_grouped_big_takes(int a_rows, int N, int K) { return K % BK == 0 && K <= BK_MOST && N <= BN_MOST && 2ll * a_rows * K <= 0xffff0000ll; }
 int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
                           int experts, int N, int K, hipStream_t stream) {
@@ -428,8 +510,12 @@ int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w
     const int tiles_m = places / 128 + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
     // (what the product through registers, whose tiles have half the features, would refuse is refused here too)
     FW_REQUIRE((long long)tiles_m * fw_ceil_div(N, gated ? BT / 4 : BT / 2) < (1ll << 30), "grouped_gemm: too many tiles");
-    if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
-    return launch_tiles<MB_STORE, float, 4, 2, 3, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+    if (K >= 1536 && places >= 128 * experts) {
+        if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 64, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+        return launch_tiles<MB_STORE, float, 4, 2, 64, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+    }
+    if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 32, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+    return launch_tiles<MB_STORE, float, 4, 2, 32, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
 }
 
 // The tile a storing or accumulating product is cut into: 256 or 128 rows by 256 or 192 columns,

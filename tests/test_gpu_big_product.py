@@ -34,9 +34,9 @@ TILES = [(2048, 6144, (256, 192)), (1537, 6100, (256, 192)), (1536, 8192, (256, 
 
 
 @pytest.mark.parametrize("M,N,tile", TILES)
-@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 288, 544])
+@pytest.mark.parametrize("K", [32, 64, 96, 128, 160, 192, 256, 288, 352, 448, 544])
 def test_every_number_of_slabs(ops, M, N, tile, K):
-    """Every number of slabs of K up to where the turns of the loop repeat: its four stages half full, full, one turn, several."""
+    """Every number of slabs of K up to where the turns of the loop repeat: its two to four stages half full, full, one turn, several, the last slab whole and half."""
     rows, columns = ctypes.c_int(0), ctypes.c_int(0)
     for mode in (STORE, ADD):
         assert ops.library().fw_gemm_mfma_big_plan(mode, M, N, K, ctypes.byref(rows), ctypes.byref(columns)) > 0
@@ -106,3 +106,25 @@ def test_two_byte_outputs_of_any_width_and_place(ops, M, N, shift):
     # (the slope of the tanh form is below 1.13 as well)
     want = torch.nn.functional.gelu(gate, approximate="tanh") * up
     assert ((run(GATED, ops.BF16_GEGLU, False) - want).abs() <= 1.03 * slack + 1e-5 * (gate * up).abs() + 2.0 ** -7 * want.abs()).all()
+
+
+@pytest.mark.parametrize("rows,experts,top,K,N", [(384, 6, 2, 1536, 200), (383, 6, 2, 1536, 200), (700, 4, 1, 1568, 129), (513, 4, 2, 2048, 128),
+                                                  (384, 6, 2, 1504, 200), (300, 3, 1, 1536, 130), (640, 5, 3, 96, 257)])
+def test_grouped_product_on_slabs_of_either_depth(ops, rows, experts, top, K, N):
+    """Both sides of the rule: a long K and experts of 128 places in the mean, or slabs of half the depth; whole and half last slabs."""
+    generator = torch.Generator().manual_seed(rows + K)
+    chosen = torch.rand(rows, experts, generator=generator).topk(top, -1).indices.int().to(DEV)
+    begin, place_row, pair_place = ops.moe_arrange(chosen, experts)
+    a, w = draw(rows, K).to(DEV), draw(experts, 2 * N, K, seed=1).to(DEV)
+    gated = ops.grouped_gemm(a, place_row, w, begin, rows * top, gated=True, out_dtype=torch.bfloat16).double()
+    plain = ops.grouped_gemm(a, place_row, w, begin, rows * top, gated=False, out_dtype=torch.float32).double()
+    first, A = begin.tolist(), a.double()[place_row.long()]
+    for e in range(experts):
+        here = slice(first[e], first[e + 1])
+        exact = A[here] @ w[e].double().T
+        limit = (K + 16) * 2.0 ** -24 * (A[here].abs() @ w[e].double().abs().T)
+        assert ((plain[here] - exact).abs() <= limit).all()
+        gate, up, gate_off, up_off = exact[:, :N], exact[:, N:], limit[:, :N], limit[:, N:]
+        want = gate * torch.sigmoid(gate) * up
+        slack = 1.1 * gate_off * (up.abs() + up_off) + gate.abs() * up_off + 2.0 ** -20 * want.abs() + 2.0 ** -8 * want.abs() + 2.0 ** -133
+        assert ((gated[here] - want).abs() <= slack).all()
