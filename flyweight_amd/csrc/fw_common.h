@@ -83,6 +83,16 @@ __device__ __forceinline__ float fw_buffer_load_float(fw_buffer from, uint32_t a
 }
 __device__ __forceinline__ void fw_buffer_store(fw_buffer to, uint32_t at, uint32_t word) { __builtin_amdgcn_raw_buffer_store_b32(word, to, at, 0, 0); }
 __device__ __forceinline__ void fw_buffer_store(fw_buffer to, uint32_t at, uint16_t half) { __builtin_amdgcn_raw_buffer_store_b16(half, to, at, 0, 0); }
+// 16 bytes a lane at device scope (past the die's L2), at an offset of the lane and one that the wave shares
+typedef __attribute__((ext_vector_type(4))) float fw_f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t fw_buffer_words;
+#define FW_DEVICE_SCOPE 16      // sc1
+__device__ __forceinline__ void fw_buffer_store_device(fw_buffer to, uint32_t at, int shared_at, fw_f32x4 v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(fw_buffer_words, v), to, at, shared_at, FW_DEVICE_SCOPE);
+}
+__device__ __forceinline__ fw_f32x4 fw_buffer_load_device(fw_buffer from, uint32_t at, int shared_at) {
+    return __builtin_bit_cast(fw_f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, shared_at, FW_DEVICE_SCOPE));
+}
 __device__ __forceinline__ void fw_buffer_to_lds(fw_buffer from, void* lds, uint32_t at, int shared_at) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)lds, 16, at, shared_at, 0, 0);
 }

@@ -72,6 +72,10 @@ int fw_gemm_mfma_split_plan(int mode, int M, int N, int K, size_t* workspace_byt
 int fw_gemm_mfma_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode,
                        int M, int N, int K, void* workspace, size_t workspace_bytes, int* counters,
                        int counters_len, void* stream);
+// The same on tiles of 128 x 256, for modes 0 and 1; slices 0: the shape is not taken.
+int fw_gemm_mfma_big_split_plan(int mode, int M, int N, int K, int* slices, size_t* workspace_bytes, int* counters);
+int fw_gemm_mfma_big_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
+                           void* workspace, size_t workspace_bytes, int* counters, int counters_len, void* stream);
 // The same product for 1..64 rows with K split over workgroups, for the shapes that fw_gemm_rows serves worse.
 // fw_gemm_medium_plan says what a shape needs: bytes of workspace (0: none) and int32 counters (0: none) that are zero before
 // the first call; the kernel leaves them zero. Calls that overlap on one device need their own of both.

@@ -73,6 +73,13 @@ struct BigGroups {
     int experts;
 };
 
+// K cut over workgroups: `slices` of k_each, which meet in a workspace [slice][tile][product tile][thread][4] through a ticket a tile.
+struct BigSlices {
+    int slices, k_each;
+    float* partials;
+    int* counters;
+};
+
 // A slab: 64 k of the tile's rows (an LDS row is 128 bytes, eight 16-byte chunks), or 32 where two workgroups share a compute unit. Chunk
 // c of a row lies in slot c ^ swap(row): a read of 16 rows by four chunks goes in groups of 16 lanes, 0-3, 12-15 and 20-27, then the 16
 // others of the first 32, and every group covers all 64 banks once.
@@ -108,10 +115,10 @@ struct BigTile {
 // TN: 32-column pairs of product tiles per wave, 4 (a 256 x 256 tile) or 3 (256 x 192: a width of 6,144
 // features gives 192 tiles of 256 columns for 256 compute units, but exactly 256 tiles of 192).
 // TM: 32-row pairs of product tiles per wave, 4 (256 rows a tile) or 2 (128 rows). DEPTH: k of a slab, see BigTile.
-template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED>
+template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED, bool SPLIT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32 ? 2 : 1, DEPTH == 32 ? 2 : 1))) void gemm_mfma_big_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const float* __restrict__ bias,
-    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups) {
+    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups, const BigSlices cut) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [A_STAGES slabs of a][W_STAGES slabs of w]
     typedef BigTile<TM, TN, DEPTH> Tile;
     constexpr int ROWS = Tile::ROWS, WIDE = Tile::WIDE, A_SLAB = Tile::A_SLAB, W_SLAB = Tile::W_SLAB, A_STAGES = Tile::A_STAGES, W_STAGES = Tile::W_STAGES;
@@ -119,8 +126,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32
     constexpr int PARTS = DEPTH / BK, CHUNKS = DEPTH / 8, LOAD_ROWS = 64 / CHUNKS;      // steps of a slab, chunks of a row, rows of a wave-wide load
     const int features = MODE == MB_SWIGLU ? BT / 2 : WIDE;
     static_assert(MODE != MB_SWIGLU || TN == 4, "the gated tile holds 128 gate and 128 up rows");
-    int m0, n0;
+    int m0, n0, k_first = 0, k_length = K;
     const int32_t* groups_rows = nullptr;
+    int slice = 0, tile_number = 0;
     if constexpr (GROUPED) {
         const GroupedTile tile = grouped_tile(groups.begin, groups.experts, ROWS, tiles_n);
         const int expert = tile.expert;
@@ -135,8 +143,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32
         else a += (size_t)first * K;
     } else {
         const int total = tiles_m * tiles_n;
-        const int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-        if (logical >= total) return;
+        int logical = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+        if (logical >= total * (SPLIT ? cut.slices : 1)) return;
+        if constexpr (SPLIT) {              // slice by slice: a die's workgroups share what they read of a and w
+            slice = logical / total;
+            logical -= slice * total;
+            tile_number = logical;
+            k_first = slice * cut.k_each;
+            k_length = K - k_first < cut.k_each ? K - k_first : cut.k_each;
+        }
         const int width = BGROUP_M * tiles_n;
         const int group = logical / width;
         const int first_m = group * BGROUP_M;
@@ -173,10 +188,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32
         const int of_part = MODE == MB_SWIGLU ? row - w_part * (BT / 2) : row;
         w_at[i] = (uint32_t)(of_part < N - n0 ? of_part : N - n0 - 1) * (uint32_t)(2 * K) + chunk * 16;
     }
-    const fw_buffer a_rows = fw_make_buffer(a_base), w_rows = fw_make_buffer(w_base);
+    const fw_buffer a_rows = fw_make_buffer(a_base + k_first), w_rows = fw_make_buffer(w_base + k_first);
     // This wave's loads for a slab of either operand, into the stage at `stage`. A last slab of half the length has no upper
     // chunks: the lower ones are read again in their place and never used.
-    const int whole = K / DEPTH, slabs = (K + DEPTH - 1) / DEPTH;
+    const int whole = k_length / DEPTH, slabs = (k_length + DEPTH - 1) / DEPTH;
     auto request_a = [&](int stage, int slab, int i) { fw_buffer_to_lds(a_rows, lds + stage + (wave * A_LOADS + i) * 1024, a_at[i], slab * (DEPTH * 2)); };
     auto request_w = [&](int stage, int slab, int i) { fw_buffer_to_lds(w_rows, lds + stage + (wave * W_LOADS + i) * 1024, w_at[i], slab * (DEPTH * 2)); };
     auto upper = [&](int first_row) { return ((lane % CHUNKS) ^ chunk_swap<DEPTH>(first_row + lane / CHUNKS)) >= CHUNKS / 2; };
@@ -365,6 +380,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32
     }
     fw_mfma_drain();     // branches follow that lead to code reading the accumulators
 
+    // A slice's sums leave past the die's cache (device scope). Every wave waits until its own are acknowledged, then one thread takes the
+    // ticket, and the last workgroup of the tile adds the slices in their order.
+    if constexpr (SPLIT) {
+        const int total = tiles_m * tiles_n;
+        constexpr int TILE_BYTES = ROWS * WIDE * 4;
+        auto left_by = [&](int of) { return fw_make_buffer(cut.partials + ((size_t)of * total + tile_number) * (TILE_BYTES / 4), TILE_BYTES); };
+        const fw_buffer mine = left_by(slice);
+#pragma unroll
+        for (int u = 0; u < MFMAS; ++u) fw_buffer_store_device(mine, tid * 16, u * 4096, acc[u / TB][u % TB]);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int* ticket = reinterpret_cast<int*>(lds);
+        if (tid == 0) *ticket = __hip_atomic_fetch_add(&cut.counters[tile_number], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*ticket != cut.slices - 1) return;
+        if (tid == 0) __hip_atomic_store(&cut.counters[tile_number], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        f32x4 sum[TA][TB];
+        for (int of = 0; of < cut.slices; ++of) {
+            const fw_buffer theirs = left_by(of);
+            f32x4 part[TA][TB];
+#pragma unroll
+            for (int u = 0; u < MFMAS; ++u) part[u / TB][u % TB] = fw_buffer_load_device(theirs, tid * 16, u * 4096);
+#pragma unroll
+            for (int u = 0; u < MFMAS; ++u) sum[u / TB][u % TB] = of ? sum[u / TB][u % TB] + part[u / TB][u % TB] : part[u / TB][u % TB];
+        }
+#pragma unroll
+        for (int u = 0; u < MFMAS; ++u) acc[u / TB][u % TB] = sum[u / TB][u % TB];
+    }
+
     // D layout of the 16x16 product: lane holds column lane % 16, register r is row 4 * (lane / 16) + r. Two neighbouring
     // column tiles swap every second 16 lanes, so that a lane holds column lane % 32 of the pair and eight rows
     // 8 * (lane / 32) + u of the row tile: a store then covers whole runs of 32 columns.
@@ -471,15 +515,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DEPTH == 32
     }
 }
 
-template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED>
+template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED, bool SPLIT = false>
 static int launch_tiles(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, int tiles_m, const BigGroups& groups,
-                        hipStream_t stream) {
+                        hipStream_t stream, const BigSlices& cut = BigSlices()) {
     const int tiles_n = fw_ceil_div(N, MODE == MB_SWIGLU ? BT / 2 : BigTile<TM, TN, DEPTH>::WIDE);
-    const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n, 8);
+    const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n * (SPLIT ? cut.slices : 1), 8);
     const int lds_bytes = BigTile<TM, TN, DEPTH>::LDS;
     static bool configured = false;     // per instantiation
     if (!configured) {
-        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED>,
+        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED, SPLIT>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (status != hipSuccess) {
             fw_set_error("gemm_mfma_big: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(status));
@@ -487,8 +531,8 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
         }
         configured = true;
     }
-    gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED><<<per_xcd * 8, 256, lds_bytes, stream>>>(
-        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups);
+    gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED, SPLIT><<<per_xcd * 8, 256, lds_bytes, stream>>>(
+        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups, cut);
     return 0;
 }
 template <int MODE, typename TO, int TN = 4, int TM = 4>
@@ -586,5 +630,70 @@ extern "C" int fw_gemm_mfma_big(const void* a, const void* w, const float* bias,
     else status = launch_planned<MB_STORE, bf16_t>(plan, a, w, bias, out, M, N, K, s);
     if (status != 0) return status;
     FW_LAUNCH_CHECK("gemm_mfma_big");
+    return 0;
+}
+
+// ----- K cut into slices, for products with at most half as many tiles as compute units and a long K --------
+// A tile of 128 x 256 moves 48 bytes a clock of full MFMA rate through a compute unit's memory path, one of 128 x 128 all of its 64: two or three slices of K on
+// the larger tiles pay for their meeting (about 12 us: 128 KB a workgroup out past the dies' caches and back) where K is long. us, cut / 128 x 128 with
+// K dealt to the waves: storing 1,111 x 2,048 x 8,192 49.6 / 60.3, adding 2,048 x 2,048 x 8,192 72.2 / 70.5 alone and 8 us less of it in a prompt's step
+// (4,863 against 4,995 for 16 layers), storing 1,024 x 2,560 x 6,368 51.2 / 73 (whole large tiles). With four slices the sum at the end costs more than it
+// gives (adding 801 x 2,048 x 7,168 40.6 against 38.7 on 128 x 64), and so do slices of less than 512 k (2,048 x 1,024 x 1,024 21.2 / 12.2).
+struct BigSplitPlan {
+    int tiles, slices, k_each;
+    size_t workspace_bytes;
+};
+static BigSplitPlan big_split_plan(int M, int N, int K) {
+    BigSplitPlan plan = {0, 0, 0, 0};
+    const long long tiles = (long long)fw_ceil_div(M, BT / 2) * fw_ceil_div(N, BT);
+    if (tiles > 128) return plan;
+    int slices = (int)(256 / tiles);                    // at most a workgroup a compute unit
+    slices = slices > 3 ? 3 : slices;                   // the last workgroup of a tile adds them one after the other
+    const int most = K / 512;
+    slices = slices > most ? most : slices;
+    if (slices < 2) return plan;
+    plan.tiles = (int)tiles;
+    plan.k_each = fw_ceil_div(fw_ceil_div(K, slices), 64) * 64;
+    plan.slices = fw_ceil_div(K, plan.k_each);
+    plan.workspace_bytes = (size_t)plan.slices * plan.tiles * (BT / 2) * BT * sizeof(float);
+    return plan;
+}
+
+// What fw_gemm_mfma_big_split needs for a shape: its slices of K (0: it does not take the shape), bytes of float32 workspace and the number of
+// int32 counters (zero before the first call; left zero).
+extern "C" int fw_gemm_mfma_big_split_plan(int mode, int M, int N, int K, int* slices, size_t* workspace_bytes, int* counters) {
+    FW_REQUIRE(M >= 1 && N > 0 && K > 0 && mode >= 0 && mode <= 2, "gemm_mfma_big_split: M %d N %d K %d mode %d", M, N, K, mode);
+    BigSplitPlan plan = {0, 0, 0, 0};
+    if (mode != MB_SWIGLU && K % BK == 0 && K <= BK_MOST && N <= BN_MOST) plan = big_split_plan(M, N, K);
+    *slices = plan.slices;
+    *workspace_bytes = plan.workspace_bytes;
+    *counters = plan.tiles;
+    return 0;
+}
+
+// fw_gemm_mfma's contract for modes 0 and 1, with K cut into slices as fw_gemm_mfma_big_split_plan says, on tiles of 128 x 256. Calls that overlap on one
+// device must not share counters or workspace.
+extern "C" int fw_gemm_mfma_big_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
+                                      void* workspace, size_t workspace_bytes, int* counters, int counters_len, void* stream) {
+    int slices = 0, need_counters = 0;
+    size_t need_bytes = 0;
+    if (fw_gemm_mfma_big_split_plan(mode, M, N, K, &slices, &need_bytes, &need_counters)) return -1;
+    FW_REQUIRE(slices > 1, "gemm_mfma_big_split: this shape (M %d N %d K %d mode %d) is not cut", M, N, K, mode);
+    FW_REQUIRE(mode != MB_ACCUMULATE || out_dtype == FW_F32, "gemm_mfma_big_split: accumulation needs a float32 destination");
+    FW_REQUIRE(out_dtype == FW_F32 || out_dtype == FW_BF16 || (out_dtype == FW_BF16_GELU && mode == MB_STORE), "gemm_mfma_big_split: unknown out dtype %d", out_dtype);
+    FW_REQUIRE(((uintptr_t)a % 16 == 0) && ((uintptr_t)w % 16 == 0), "gemm_mfma_big_split: operands must be 16-byte aligned");
+    FW_REQUIRE(workspace != nullptr && workspace_bytes >= need_bytes && counters != nullptr && counters_len >= need_counters && (uintptr_t)workspace % 16 == 0,
+               "gemm_mfma_big_split: this shape needs %zu bytes of workspace and %d counters", need_bytes, need_counters);
+    const BigSplitPlan plan = big_split_plan(M, N, K);
+    const BigSlices cut = {plan.slices, plan.k_each, (float*)workspace, counters};
+    const int tiles_m = fw_ceil_div(M, BT / 2);
+    hipStream_t s = (hipStream_t)stream;
+    int status;
+    if (mode == MB_ACCUMULATE) status = launch_tiles<MB_ACCUMULATE, float, 4, 2, 64, false, true>(a, w, bias, out, M, N, K, tiles_m, BigGroups(), s, cut);
+    else if (out_dtype == FW_F32) status = launch_tiles<MB_STORE, float, 4, 2, 64, false, true>(a, w, bias, out, M, N, K, tiles_m, BigGroups(), s, cut);
+    else if (out_dtype == FW_BF16_GELU) status = launch_tiles<MB_STORE, gelu_bf16_t, 4, 2, 64, false, true>(a, w, bias, out, M, N, K, tiles_m, BigGroups(), s, cut);
+    else status = launch_tiles<MB_STORE, bf16_t, 4, 2, 64, false, true>(a, w, bias, out, M, N, K, tiles_m, BigGroups(), s, cut);
+    if (status != 0) return status;
+    FW_LAUNCH_CHECK("gemm_mfma_big_split");
     return 0;
 }

@@ -569,12 +569,13 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     if kind == "deep":
         _check(library().fw_gemm_mfma_deep(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, columns, _stream()))
         return
-    if kind == "split":
-        need_bytes, need_counters = _split_needs(mode, M, N, K)
+    if kind in ("split", "bigsplit"):
+        need_bytes, need_counters = (_split_needs if kind == "split" else _big_split_needs)(mode, M, N, K)[:2]
         workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
         counters = _medium_counters(a.device, need_counters)
-        _check(library().fw_gemm_mfma_split(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _p(workspace),
-                                            ctypes.c_size_t(need_bytes), _p(counters), counters.numel(), _stream()))
+        entry = library().fw_gemm_mfma_split if kind == "split" else library().fw_gemm_mfma_big_split
+        _check(entry(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _p(workspace), ctypes.c_size_t(need_bytes), _p(counters),
+                     counters.numel(), _stream()))
         return
     entry = library().fw_gemm_mfma_big if kind == "big" else library().fw_gemm_mfma
     _check(entry(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
@@ -585,6 +586,13 @@ def _split_needs(mode: int, M: int, N: int, K: int):
     need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
     _check(library().fw_gemm_mfma_split_plan(mode, M, N, K, ctypes.byref(need_bytes), ctypes.byref(need_counters)))
     return need_bytes.value, need_counters.value
+
+
+def _big_split_needs(mode: int, M: int, N: int, K: int):
+    """(bytes of workspace, counters, slices of K) of the product that cuts K over workgroups on large tiles; zeros where it does not take the shape."""
+    slices, need_bytes, need_counters = ctypes.c_int(0), ctypes.c_size_t(0), ctypes.c_int(0)
+    _check(library().fw_gemm_mfma_big_split_plan(mode, M, N, K, ctypes.byref(slices), ctypes.byref(need_bytes), ctypes.byref(need_counters)))
+    return need_bytes.value, need_counters.value, slices.value
 
 
 # What the tiled products take, us: start + rounds * round + tiles / 256 * tile + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of
@@ -600,19 +608,14 @@ _TIME_TILES = {0: {128: (5.1, 0.0, 1.5, 6.32, 2.84, 6.2, 0.92), 64: (0.0, 0.3, 0
                1: {128: (0.3, 0.0, 6.1, 5.87, 1.06, 11.7, 3.78), 64: (0.0, 1.1, 1.3, 2.55, 2.66, 5.1, 3.81)},
                2: {64: (3.2, 0.8, 0.5, 5.52, 1.82, 2.8, 3.67)}}
 _TIME_RAGGED = 3.0       # ... adding into features that end inside a tile of 64, and the same with K cut: a branch and a load an element
-_TIME_BIG = {0: {128: (1.9, 2.0, 2.9, 0.337, 0.197), 256: (2.4, 4.4, 4.2, 0.174, 0.239)},     # by the tile's rows; walk and fill by 32 x 32 of its area
-             1: {128: (0.6, 3.6, 3.9, 0.341, 0.192), 256: (0.7, 3.9, 13.9, 0.203, 0.21)}, 2: {256: (2.2, 4.4, 2.1, 0.247, 0.144)}}
+_TIME_BIG = {0: {128: (2.3, 2.8, 3.2, 0.301, 0.099), 256: (4.1, 2.3, 7.0, 0.219, 0.114)},     # by the tile's rows; walk and fill by 32 x 32 of its area
+             1: {128: (0.9, 5.1, 3.8, 0.301, 0.111), 256: (5.5, 0.9, 14.8, 0.217, 0.118)}, 2: {256: (1.8, 5.7, 1.6, 0.239, 0.095)}}
 _TIME_BIG_ODD = 4.0      # a round more of gated products with an odd number of features, which leave element by element
-# A gated product whose second round of large tiles is at most half full costs a step more than its own time: a burst at full power, then idle compute
-# units, behind which the step's attention and products run at a lower clock. With 2,048 x 4,608 over K 1,024 (288 tiles; alone 57.1 us on large tiles,
-# 56.4 on small ones) a prompt of 16,384 tokens took 27.1 ms against 25.9, with 5,120 features 27.8 against 26.7, 5,632 28.4 / 28.2, 6,144 28.9 / 28.7, with
-# 4,096 (one round) 23.6 against 24.3, 7,168 29.7 against 30.6; over K 2,048 4,608 features 4.73 ms a step against 4.67, 6,144 5.03 against 5.24.
-_TIME_BIG_BURST = 10.0         # from K 1,024 on, in proportion below
-# Large tiles level with those whose waves split K leave the product to the latter, for the same reason (2,048 x 2,048 adding over K 2,048: alone 27.2 us,
-# large tiles 26.3; in a prompt's step 32.5, 33.4; 1,111 x 2,048 and 3,072 storing: two prompts of 1,111 and 277 rows 3,198 us, large tiles 3,209)
-_TIE = 0.93
 # ... with K cut: start, a slice's part in the sum at the end, 1,024 k of a slice in each round and for 256 workgroups, 256 workgroups
 _TIME_SPLIT = {0: (8.3, 0.44, 4.6, 3.4, 1.5), 1: (7.3, 0.55, 4.8, 4.55, 4.0), 2: (8.3, 0.77, 8.7, 3.96, 2.5)}
+
+# ... large tiles with K cut: start, a slice's part in the sum at the end, 256 workgroups, 1,024 k of a slice and for 256 workgroups
+_TIME_BIG_SPLIT = {0: (8.4, 1.9, 5.5, 5.0, 8.6), 1: (10.6, 1.6, 5.6, 5.8, 7.9)}
 
 
 def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: float, walk: float, fill: float, each_pair: float = 0.0,
@@ -627,8 +630,8 @@ def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: 
 @functools.lru_cache(maxsize=4096)
 def tiled_plan(mode: int, M: int, N: int, K: int):
     """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
-    256 columns), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through registers), "split" (those with K cut over
-    workgroups). The least estimated time decides, with what a tie costs inside a step: on the shapes that it was fitted to 0.2 to 0.4 % above the fastest
+    256 columns), "bigsplit" (128 rows by 256, K cut over workgroups), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through
+    registers), "split" (those with K cut over workgroups). The least estimated time decides: on 780 shapes 0.1 to 0.7 % above the fastest
     alone in the geometric mean. Fixed numbers of tiles were 10 % above it (storing, 1,111 rows by 2,048 features over K 8,192 97 us
     against 57, 640 by 2,048 over 2,048 22 against 14, 1,300 by 3,072 over 2,048 44 against 28; gated, 1,111 by 4,608 over 2,048 63 against 46), adding
     products of up to 2,048 features held to the tiles whose waves split K 5 % (6,200 by 2,048 over 7,168 269 against 163, 2,690 by 1,536 over 1,024 32
@@ -652,7 +655,6 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
             area = rows.value * (256 if mode == 2 else columns.value) / 1024        # (a gated tile has gate and up columns)
             if mode == 2:
                 each_round += _TIME_BIG_ODD if N % 2 else 0.0
-                start += _TIME_BIG_BURST * min(1.0, K / 1024) if DEEP_ROUND < tiles <= 3 * DEEP_ROUND // 2 else 0.0
             times["big", 0] = _tiled_time(tiles, K, start, each_round, each_tile, walk * area, fill * area)
     need_bytes, tiles = _split_needs(mode, M, N, K)
     if need_bytes:
@@ -662,10 +664,13 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
         share = workgroups / DEEP_ROUND
         times["split", 0] = (start + ragged + each * slices + share * all_at_once
                              + K / 1024 / slices * (walk * -(-workgroups // DEEP_ROUND) + fill * share))
-    least = min(times, key=times.get)
-    if least == ("big", 0) and ("deep", 128) in times and times["deep", 128] * _TIE <= times[least]:
-        return "deep", 128
-    return least
+    if mode != 2 and M > BIG_MIN_ROWS:
+        need_bytes, tiles, slices = _big_split_needs(mode, M, N, K)
+        if slices:
+            start, each, all_at_once, walk, fill = _TIME_BIG_SPLIT[mode]
+            share = tiles * slices / DEEP_ROUND
+            times["bigsplit", 0] = start + each * slices + share * all_at_once + K / 1024 / slices * (walk + fill * share)
+    return min(times, key=times.get)
 
 
 MEDIUM_MAX_ROWS = 64

@@ -122,21 +122,21 @@ def test_products_beyond_64_rows_are_dealt_to_waves_where_that_is_faster(mode, M
 
 
 @pytest.mark.parametrize("mode,M,N,K,plan", [
-    (0, 1111, 2048, 8192, ("deep", 128)), (0, 1111, 2048, 2048, ("deep", 128)), (0, 640, 2048, 2048, ("deep", 64)), (0, 1111, 1024, 4608, ("deep", 64)),
+    (0, 1111, 2048, 8192, ("bigsplit", 0)), (0, 1111, 2048, 2048, ("big", 0)), (0, 640, 2048, 2048, ("deep", 64)), (0, 1111, 1024, 4608, ("deep", 64)),
     (0, 1300, 3072, 2048, ("big", 0)), (0, 801, 3072, 1024, ("big", 0)), (0, 2048, 6144, 2048, ("big", 0)), (0, 512, 6144, 1024, ("big", 0)),
-    (0, 320, 6144, 2048, ("deep", 128)), (0, 320, 1024, 8192, ("split", 0)), (0, 128, 3072, 8192, ("split", 0)), (0, 300, 2500, 520, ("tiles", 0)),
+    (0, 320, 6144, 2048, ("big", 0)), (0, 320, 1024, 8192, ("split", 0)), (0, 128, 3072, 8192, ("split", 0)), (0, 300, 2500, 520, ("tiles", 0)),
     (0, 100, 8192, 32, ("tiles", 0)), (2, 801, 1536, 2048, ("tiles", 0)), (2, 1111, 4608, 2048, ("big", 0)), (2, 640, 1536, 2048, ("split", 0)),
     (0, 1111, 64, 4096, ("split", 0)), (0, 2048, 64, 1024, ("deep", 64)), (2, 300, 64, 2048, ("split", 0)),
-    (2, 2048, 8192, 2048, ("big", 0)), (2, 128, 8192, 1024, ("tiles", 0)), (2, 2048, 2048, 2048, ("tiles", 0)),
-    (1, 2048, 2048, 8192, ("deep", 128)), (1, 2048, 1024, 1024, ("deep", 64)), (1, 512, 2048, 2048, ("deep", 64)), (1, 256, 2048, 8192, ("split", 0)),
+    (2, 2048, 8192, 2048, ("big", 0)), (2, 128, 8192, 1024, ("tiles", 0)), (2, 2048, 2048, 2048, ("big", 0)),
+    (1, 2048, 2048, 8192, ("bigsplit", 0)), (1, 2048, 1024, 1024, ("deep", 64)), (1, 512, 2048, 2048, ("deep", 64)), (1, 256, 2048, 8192, ("split", 0)),
     (1, 2048, 8192, 2048, ("big", 0)),
-    # ties inside a step, where a burst of large tiles slows what runs behind it
-    (2, 2048, 4608, 1024, ("tiles", 0)), (2, 2048, 5120, 1024, ("tiles", 0)), (2, 2048, 4608, 2048, ("tiles", 0)), (2, 2048, 4096, 1024, ("big", 0)),
-    (2, 2048, 7168, 1024, ("big", 0)), (2, 2048, 6144, 2048, ("big", 0)), (2, 1005, 11344, 192, ("big", 0)), (1, 2048, 2048, 2048, ("deep", 128)),
+    # a second round of large tiles that is little full
+    (2, 2048, 4608, 1024, ("big", 0)), (2, 2048, 5120, 1024, ("big", 0)), (2, 2048, 4608, 2048, ("big", 0)), (2, 2048, 4096, 1024, ("big", 0)),
+    (2, 2048, 7168, 1024, ("big", 0)), (2, 2048, 6144, 2048, ("big", 0)), (2, 1005, 11344, 192, ("big", 0)), (1, 2048, 2048, 2048, ("big", 0)),
     # many rounds of tiles, a short K, odd widths, few rows of tiles over a long K
-    (1, 6200, 2048, 7168, ("big", 0)), (1, 8192, 2048, 1024, ("big", 0)), (1, 2690, 1536, 1024, ("big", 0)), (1, 1700, 2048, 7168, ("deep", 128)),
+    (1, 6200, 2048, 7168, ("big", 0)), (1, 8192, 2048, 1024, ("big", 0)), (1, 2690, 1536, 1024, ("big", 0)), (1, 1700, 2048, 7168, ("bigsplit", 0)), (1, 2048, 2048, 4160, ("deep", 128)),
     (2, 13184, 3496, 352, ("big", 0)), (2, 5964, 4032, 128, ("big", 0)), (2, 2304, 1281, 128, ("tiles", 0)), (2, 512, 4480, 2560, ("tiles", 0)),
-    (0, 100, 65536, 2048, ("tiles", 0)), (0, 512, 65536, 2048, ("big", 0)), (0, 128, 4480, 2816, ("split", 0)), (1, 256, 2112, 7872, ("split", 0))])
+    (0, 100, 65536, 2048, ("tiles", 0)), (0, 512, 65536, 2048, ("big", 0)), (0, 128, 4480, 2816, ("split", 0)), (1, 256, 2112, 7872, ("bigsplit", 0))])
 def test_tiled_products_take_the_tiles_that_were_the_fastest(mode, M, N, K, plan):
     from flyweight_amd.kernels import ops
     assert ops.tiled_plan(mode, M, N, K) == plan

@@ -128,3 +128,46 @@ def test_grouped_product_on_slabs_of_either_depth(ops, rows, experts, top, K, N)
         want = gate * torch.sigmoid(gate) * up
         slack = 1.1 * gate_off * (up.abs() + up_off) + gate.abs() * up_off + 2.0 ** -20 * want.abs() + 2.0 ** -8 * want.abs() + 2.0 ** -133
         assert ((gated[here] - want).abs() <= slack).all()
+
+
+# (rows, features, K, slices): whole tiles and ragged ones, slices of equal and of unequal length, the last one with half a slab
+@pytest.mark.parametrize("M,N,K,slices", [(256, 512, 1024, 2), (2048, 2048, 2080, 2), (1111, 2048, 8192, 3), (129, 257, 1536, 3), (1, 1, 1568, 3), (1000, 2560, 3104, 3),
+                                          (130, 8191, 1056, 2)])
+def test_large_tiles_with_k_cut_over_workgroups(ops, M, N, K, slices):
+    need_bytes, need_counters, cut = ops._big_split_needs(STORE, M, N, K)
+    assert cut == slices and ops._big_split_needs(GATED, M, N, K) == (0, 0, 0)
+    a, w = draw(M, K).to(DEV), draw(N, K, seed=1).to(DEV)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(2)).to(DEV)
+    residual = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).to(DEV)
+    exact = a.double() @ w.double().T
+    limit = (K + 16) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    workspace = torch.full((need_bytes // 4,), float("nan"), device=DEV)
+    counters = torch.zeros(need_counters, dtype=torch.int32, device=DEV)
+
+    def run(mode, out, with_bias=False):
+        ops._check(ops.library().fw_gemm_mfma_big_split(ops._p(a), ops._p(w), ops._p(bias) if with_bias else None, ops._p(out), ops._code(out.dtype), mode, M,
+                                                        N, K, ops._p(workspace), need_bytes, ops._p(counters), counters.numel(), ops._stream()))
+        return out
+
+    want = exact + bias.double()
+    room = limit + 2.0 ** -23 * (exact.abs() + bias.double().abs())
+    stored = run(STORE, torch.empty(M, N, device=DEV), True)
+    assert ((stored.double() - want).abs() <= room).all()
+    assert ((run(STORE, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), True).double() - want).abs() <= room + 2.0 ** -8 * want.abs()).all()
+    total = run(ADD, residual.clone()).double()
+    assert ((total - exact - residual.double()).abs() <= limit + 2.0 ** -23 * total.abs()).all()
+    # whichever workgroup of a tile ends last, the slices are added in their order, and the counters are left at zero
+    for _ in range(3):
+        assert torch.equal(run(STORE, torch.empty(M, N, device=DEV), True), stored)
+    assert not counters.any()
+
+
+def test_large_tiles_with_k_cut_refuse_what_they_do_not_take(ops):
+    a, w, out = draw(128, 1024).to(DEV), draw(256, 1024, seed=1).to(DEV), torch.empty(128, 256, device=DEV)
+    call = lambda K, mode, bytes_, counters: ops._check(ops.library().fw_gemm_mfma_big_split(ops._p(a), ops._p(w), None, ops._p(out), F32, mode, 128, 256, K, ops._p(out),      # noqa: E731,E501
+                                                                                             bytes_, ops._p(counters), counters.numel(), ops._stream()))
+    one = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for K, mode, bytes_, counters, text in [(1000, 0, 1 << 20, one, "is not cut"), (992, 0, 1 << 20, one, "is not cut"), (1024, 2, 1 << 20, one, "is not cut"),
+                                            (1024, 0, 1000, one, "bytes of workspace"), (1024, 0, 1 << 20, one[:0], "counters")]:
+        with pytest.raises(ops.KernelError, match=text):
+            call(K, mode, bytes_, counters)
