@@ -491,6 +491,382 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu((HD
     }
 }
 
+// ---- prompt portions, heads of 64 or 128 channels two by two ------------------------------------
+// The same tiles and workgroups' order; a wave has 16 rows of two query heads of a kv group, so that an operand read from LDS serves
+// both. What it is bound by is the softmax: 168 vector instructions a wave and page, 34 of them exponentials at half the rate, about twice the clocks of
+// its 32 products (HD 64). So a wave's loop holds three pages at once: while the softmax of page i runs, the
+// matrix pipe works on the scores of page i + 1 and on the output of page i - 1, a product or two behind every few vector instructions, a
+// load behind every few more (issued together behind the barrier, eight waves' loads keep a compute unit's memory path for as long as a third of a page).
+// us, one head a workgroup or halves of attend_page / this: 16 heads in 8 groups of 64 channels, 2,048 rows behind 30,720 keys 442 / 359 (741 TFLOP/s), 32
+// heads behind 2,048 98 / 80, 6,144 rows behind 8,192 956 / 690 (822); 16 heads in 4 groups of 128, 2,048 rows with a window of 1,024 44.7 / 29.0, behind
+// 4,096 187 / 104 (828). In halves the eight waves meet at one barrier a page, which costs a tenth of what four-wave workgroups side by side reach. Three waves a
+// SIMD (168 registers) gave 3 % with work for all of them and spilled.
+//
+//  * keys and values travel straight into LDS (buffer_load .. lds), STG stages of each; rows are not padded, their 16-byte chunks are
+//    stored permuted so that a wave's reads meet no bank twice;
+//  * the 16 keys of a score tile are chosen so that a lane's eight scores of two tiles are those of eight keys in a row: key
+//    32 (tile / 2) + 8 (row / 4) + 4 (tile % 2) + row % 4. The second product's operand is then one 16-byte read of a channel's keys;
+//  * values past the last one written (a tile's last page) are zeroed in LDS ahead of their product.
+//
+// PARTS 2: eight waves, the pages dealt to two halves of four waves with stages of their own, which merge at the end.
+// The largest of three scores in one instruction. (fmaxf makes two, and one more for every score to quiet what might be a signalling NaN.) What
+// a matrix product has written is read here only behind fw_mfma_drain: the compiler does not see into the assembly.
+__device__ __forceinline__ float max_of(float a, float b, float c) {
+    float m;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+}
+__device__ __forceinline__ float quad_max_of(float x) {
+    float a, b, c, d;
+    fw_quad_partners16(x, a, b);
+    asm("v_max_f32 %0, %1, %2" : "=v"(c) : "v"(a), "v"(b));
+    fw_quad_partners32(c, a, b);
+    asm("v_max_f32 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+    return d;
+}
+
+template <int HD, int PARTS, int STG>
+__global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention_prompt_kernel(
+    const uint16_t* __restrict__ q, uint16_t* __restrict__ out, const uint16_t* __restrict__ k_pages,
+    const uint16_t* __restrict__ v_pages, const int32_t* __restrict__ block_table, int table_stride,
+    const int32_t* __restrict__ tile_seg, const int32_t* __restrict__ tile_row0, const int32_t* __restrict__ seg_row0,
+    const int32_t* __restrict__ row_pos, int num_heads, int num_kv_heads, float scale_log2, int window,
+    int chunk, float cap, float cap_scale, int keep_first, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[];     // [half][K stages | V stages]
+    constexpr int NH = 2, DC = HD / 32, VT = HD / 16;
+    constexpr int TILE = PAGE * HD * 2, LOADS = TILE / 4096;             // bytes of a page's keys (values) of a kv head; wave-wide loads per wave
+    constexpr int K_CHUNKS = HD / 8, K_ROWS = 64 / K_CHUNKS;            // chunks of a key's row, rows of a wave-wide load
+    const int half = PARTS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255;
+    unsigned char* lds = lds_raw + (size_t)half * 2 * STG * TILE;
+    unsigned char* lds_v = lds + STG * TILE;
+
+    const int group = num_heads / num_kv_heads, runs = group / NH;
+    const int per_tile = num_kv_heads * runs;
+    const int tile = blockIdx.x / per_tile, of_tile = blockIdx.x % per_tile;
+    const int kvh = of_tile / runs, first_head = kvh * group + (of_tile % runs) * NH;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, g = lane >> 4;
+    const int seg = tile_seg[tile];
+    const int tile_first_row = tile_row0[tile];
+    const int seg_end = seg_row0[seg + 1];
+    const int tile_rows = seg_end - tile_first_row < 64 ? seg_end - tile_first_row : 64;
+    const int row0 = tile_first_row + wave * 16;
+    const int rows = tile_rows - wave * 16 < 16 ? tile_rows - wave * 16 : 16;     // may be <= 0
+    const bool valid = i16 < rows;
+    const int my_row = valid ? row0 + i16 : tile_first_row;      // a lane without a row computes along with the tile's first and is not stored
+    const int my_pos = row_pos[my_row];
+    const int pos_lo = row_pos[tile_first_row], pos_hi = row_pos[tile_first_row + tile_rows - 1];
+    const int my_first = fw_first_visible(my_pos, window, chunk);
+    const int tile_first = fw_first_visible(pos_lo, window, chunk);
+
+    // The pages a tile walks: those of the kept first keys that lie before the window's first page, then the window's.
+    const int window_block = tile_first / PAGE, last_block = pos_hi / PAGE;
+    const int kept_blocks = (keep_first + PAGE - 1) / PAGE < window_block ? (keep_first + PAGE - 1) / PAGE : window_block;
+    const int last_step = kept_blocks + last_block - window_block;
+    auto block_of = [&](int step) { return step < kept_blocks ? step : window_block + step - kept_blocks; };
+    auto step_of = [&](int i) { return PARTS * i + half; };
+    const int pages = (last_step + PARTS) / PARTS;              // of the first half; the other may have one less (a page past the end, masked whole)
+    const int32_t* table = block_table + (size_t)seg * table_stride;
+
+    // what this lane asks for of a page: the chunk whose slot it fills
+    uint32_t k_at[LOADS], v_at[LOADS];
+#pragma unroll
+    for (int j = 0; j < LOADS; ++j) {
+        const int key = (wave * LOADS + j) * K_ROWS + lane / K_CHUNKS;
+        const int swap = HD == 64 ? ((key >> 1) & 1) | (((key >> 3) & 3) << 1) : (key & 3) | (((key >> 3) & 3) << 2);
+        k_at[j] = key * (HD * 2) + ((lane % K_CHUNKS) ^ swap) * 16;
+        const int channel = (wave * LOADS + j) * 8 + (lane >> 3);
+        v_at[j] = channel * (PAGE * 2) + ((lane & 7) ^ ((channel >> 1) & 7)) * 16;
+    }
+    // The numbers of 64 pages at a time, one a lane, and those of the next 64 on their way: a page's number read when it is needed would
+    // stand between a barrier and the loads behind it. (Past the end: the last one again, never counted.)
+    auto numbers = [&](int first) {
+        const int step = step_of(first + lane);
+        return table[block_of(step < last_step ? step : last_step)];
+    };
+    int held = numbers(0), ahead = numbers(64);
+    int page_k = 0, page_before = 0, page_v = 0;                // of keys i, i - 1, i - 2; values follow the keys by two
+    auto next_page = [&](int i) {
+        page_v = page_before;
+        page_before = page_k;
+        page_k = __builtin_amdgcn_readlane(held, i & 63);
+        if ((i & 63) == 63) {
+            held = ahead;
+            ahead = numbers(i + 65);
+        }
+    };
+    // load number `u` of a page: LOADS of keys i, then as many of values i - 2
+    auto request = [&](int i, int u) {
+        if (u < LOADS) {
+            const fw_buffer keys = fw_make_buffer(k_pages + ((size_t)page_k * num_kv_heads + kvh) * (PAGE * HD));
+            fw_buffer_to_lds(keys, lds + (i % STG) * TILE + (wave * LOADS + u) * 1024, k_at[u], 0);
+        } else {
+            const fw_buffer channels = fw_make_buffer(v_pages + ((size_t)page_v * num_kv_heads + kvh) * (PAGE * HD));
+            fw_buffer_to_lds(channels, lds_v + ((i + STG - 2) % STG) * TILE + (wave * LOADS + u - LOADS) * 1024, v_at[u - LOADS], 0);
+        }
+    };
+
+    Columns<HD> c[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) load_query<HD>(c[h], q + ((size_t)my_row * num_heads + first_head + h) * HD, HD, valid);
+    float dist[NH];
+#pragma unroll
+    for (int h = 0; h < NH; ++h) dist[h] = slopes ? slopes[first_head + h] * 1.4426950408889634f / scale_log2 : 0.0f;
+
+    // operands: unit u < PV_UNITS is a run of 32 keys of 16 channels of the values, the others 32 channels of 16 keys
+    constexpr int PV_UNITS = 2 * VT, UNITS = PV_UNITS + 4 * DC;
+    const int k_swap = HD == 64 ? ((i16 >> 1) & 1) | ((i16 >> 2) << 1) : i16;
+    const int k_row = (8 * (i16 >> 2) + (i16 & 3)) * (HD * 2);
+    int k_lane[DC], v_lane[2];
+#pragma unroll
+    for (int d = 0; d < DC; ++d) k_lane[d] = k_row + ((d * 4 + g) ^ k_swap) * 16;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) v_lane[kb] = i16 * (PAGE * 2) + ((kb * 4 + g) ^ ((i16 >> 1) & 7)) * 16;
+    auto read_k = [&](const unsigned char* stage, int kt, int d) {
+        return *reinterpret_cast<const bf16x8*>(stage + k_lane[d] + (32 * (kt >> 1) + 4 * (kt & 1)) * (HD * 2));
+    };
+    auto read_v = [&](const unsigned char* stage, int kb, int t) { return *reinterpret_cast<const bf16x8*>(stage + v_lane[kb] + t * 16 * (PAGE * 2)); };
+    // (two tiles of keys in turn, so that a product does not wait for the one it adds to)
+    auto tile_of = [](int u) { return 2 * ((u - PV_UNITS) / (2 * DC)) + (u - PV_UNITS) % 2; };
+    auto run_of = [](int u) { return (u - PV_UNITS) / 2 % DC; };
+    auto operand = [&](const unsigned char* k_stage, const unsigned char* v_stage, int u) {
+        return u < PV_UNITS ? read_v(v_stage, u / VT, u % VT) : read_k(k_stage, tile_of(u), run_of(u));
+    };
+
+    f32x4 s0[NH][4], s1[NH][4];
+    uint32_t p0[NH][4][2], p1[NH][4][2];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto work = [&](int u, const bf16x8& x, const uint32_t (&p)[NH][4][2], f32x4 (&s)[NH][4]) {
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            if (u < PV_UNITS) {
+                const int kb = u / VT, t = u % VT;
+                const u32x4 pw = {p[h][2 * kb][0], p[h][2 * kb][1], p[h][2 * kb + 1][0], p[h][2 * kb + 1][1]};
+                c[h].o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, __builtin_bit_cast(bf16x8, pw), c[h].o[t], 0, 0, 0);
+            } else {
+                const int kt = tile_of(u), d = run_of(u);
+                s[h][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, c[h].q[d], d ? s[h][kt] : zero, 0, 0, 0);
+            }
+        }
+    };
+    auto landed = [&](bool first) {
+        if (first) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((2 * STG - 3) * LOADS) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STG - 2) * 2 * LOADS) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    // One page: the softmax of scores `s` into `p`, beside it the output of the page before (weights `p_before`) and the scores of the next.
+    auto page = [&](int i, f32x4 (&s)[NH][4], f32x4 (&s_next)[NH][4], uint32_t (&p)[NH][4][2], const uint32_t (&p_before)[NH][4][2]) {
+        landed(false);
+        next_page(i + STG);
+        const int base = block_of(step_of(i)) * PAGE;           // (past the end: beyond every position)
+        const int lo = my_first - base, hi = my_pos - base, kept = keep_first - base;
+        if (cap > 0.0f) {       // s <- cap * tanh(s * scale / cap), as attend_page
+            const float twice = 2.0f * cap_scale * 1.4426950408889634f;
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float e = __builtin_amdgcn_exp2f(s[h][kt][r] * twice);
+                        s[h][kt][r] = cap - 2.0f * cap * __builtin_amdgcn_rcpf(1.0f + e);
+                    }
+        }
+        if (slopes) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        s[h][kt][r] = fmaf(-dist[h], (float)(hi - (32 * (kt >> 1) + 8 * g + 4 * (kt & 1) + r)), s[h][kt][r]);
+        }
+        if (!__all((lo <= 0 || kept >= lo) && hi >= PAGE - 1)) {
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int key = 32 * (kt >> 1) + 8 * g + 4 * (kt & 1) + r;
+                    const bool seen = (key >= lo || key < kept) && key <= hi;
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) s[h][kt][r] = seen ? s[h][kt][r] : NEG_BIG;
+                }
+        }
+        const unsigned char* k_stage = lds + ((i + 1) % STG) * TILE;
+        const unsigned char* v_stage = lds_v + ((i + STG - 1) % STG) * TILE;
+        // SLOTS runs of vector instructions, the units of products dealt to them evenly, an operand read AHEAD units before its product
+        constexpr int SLOTS = 14, AHEAD = HD == 64 ? 6 : 2;
+        bf16x8 ring[AHEAD + 1];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) ring[u] = operand(k_stage, v_stage, u);
+        auto units = [&](int slot) {
+#pragma unroll
+            for (int u = 0; u < 2 * LOADS; ++u)         // (a compute unit takes a wave's load in 16 clocks: all at once, they would be waited for)
+                if (u * SLOTS / (2 * LOADS) == slot) request(i + STG, u);
+#pragma unroll
+            for (int u = 0; u < UNITS; ++u)
+                if (u * SLOTS / UNITS == slot) {
+                    if (u + AHEAD < UNITS) ring[(u + AHEAD) % (AHEAD + 1)] = operand(k_stage, v_stage, u + AHEAD);
+                    work(u, ring[u % (AHEAD + 1)], p_before, s_next);
+                }
+        };
+        float top[NH], alpha[NH], shift[NH], sum[NH];
+        bool rose = false;
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+#pragma unroll
+            for (int part = 0; part < 2; ++part) {
+                units(h * 3 + part);
+                const f32x4 &a = s[h][2 * part], &b = s[h][2 * part + 1];
+                top[h] = max_of(part ? top[h] : a[0], a[0], a[1]);
+                top[h] = max_of(top[h], a[2], a[3]);
+                top[h] = max_of(top[h], b[0], b[1]);
+                top[h] = max_of(top[h], b[2], b[3]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            units(h * 3 + 2);
+            const float page_max = quad_max_of(top[h]);
+            // a column that has seen no key yet keeps NEG_BIG (the raw maximum times the scale would overflow)
+            const float new_max = fmaxf(c[h].m, page_max > 0.5f * NEG_BIG ? page_max * scale_log2 : NEG_BIG);
+            alpha[h] = __builtin_amdgcn_exp2f(c[h].m - new_max);
+            rose |= alpha[h] != 1.0f;
+            c[h].m = new_max;
+            shift[h] = new_max > 0.5f * NEG_BIG ? -new_max : 0.0f;
+            sum[h] = 0.0f;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                units(6 + h * 4 + kt);
+                float e[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) e[r] = __builtin_amdgcn_exp2f(fmaf(s[h][kt][r], scale_log2, shift[h]));
+                sum[h] += (e[0] + e[1]) + (e[2] + e[3]);
+                p[h][kt][0] = pack_bf16_pair(e[0], e[1]);
+                p[h][kt][1] = pack_bf16_pair(e[2], e[3]);
+                asm volatile("" : "+v"(p[h][kt][0]), "+v"(p[h][kt][1]), "+v"(sum[h]));      // here, among the products, and not behind the branch below
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int h = 0; h < NH; ++h) c[h].l = c[h].l * alpha[h] + sum[h];
+        fw_mfma_drain();            // a branch follows that leads to code reading what the products wrote
+        if (__any(rose)) {          // the output holds the pages up to i - 1 now
+#pragma unroll
+            for (int h = 0; h < NH; ++h)
+#pragma unroll
+                for (int t = 0; t < VT; ++t) c[h].o[t] *= alpha[h];
+        }
+    };
+
+    // the stage of the values of "page -1", whose weights are zero
+#pragma unroll
+    for (int u = 0; u < TILE / 4096; ++u) *reinterpret_cast<u32x4*>(lds_v + (STG - 1) * TILE + (u * 256 + tid) * 16) = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) p1[h][kt][0] = p1[h][kt][1] = 0u;
+#pragma unroll
+    for (int i = 0; i < STG; ++i) {
+        next_page(i);
+#pragma unroll
+        for (int u = 0; u < (i < 2 ? LOADS : 2 * LOADS); ++u) request(i, u);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    landed(true);
+    {
+        const unsigned char* k_stage = lds;
+#pragma unroll
+        for (int u = PV_UNITS; u < UNITS; ++u) work(u, operand(k_stage, lds_v, u), p1, s0);
+        fw_mfma_drain();
+    }
+    int i = 0;
+    for (; i + 1 < pages; i += 2) {
+        page(i, s0, s1, p0, p1);
+        page(i + 1, s1, s0, p1, p0);
+    }
+    if (i < pages) page(i, s0, s1, p0, p1);
+    // the output of the last page: the values past the last one written are zeroed first (whatever an earlier owner of the page left there
+    // must not meet a weight of 0)
+    const int last = pages - 1;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    unsigned char* v_last = lds_v + (last % STG) * TILE;
+    const int last_written = step_of(last) >= last_step ? pos_hi - last_block * PAGE : PAGE - 1;
+    if (last_written < PAGE - 1) {
+        for (int run = tid; run < HD * 8; run += 256) {
+            const int channel = run >> 3, first_key = ((run & 7) ^ ((channel >> 1) & 7)) * 8;
+            u32x4* at = reinterpret_cast<u32x4*>(v_last + run * 16);
+            u32x4 v = *at;
+#pragma unroll
+            for (int word = 0; word < 4; ++word) {
+                const int key = first_key + 2 * word;
+                v[word] &= key + 1 <= last_written ? 0xffffffffu : (key <= last_written ? 0xffffu : 0u);
+            }
+            *at = v;
+        }
+    }
+    __syncthreads();
+    if (pages & 1) {
+#pragma unroll
+        for (int u = 0; u < PV_UNITS; ++u) work(u, operand(lds, v_last, u), p0, s1);
+    } else {
+#pragma unroll
+        for (int u = 0; u < PV_UNITS; ++u) work(u, operand(lds, v_last, u), p1, s0);
+    }
+    fw_mfma_drain();
+    if constexpr (PARTS > 1) {
+        // the second half leaves its maximum, sum and output to the same lane of the first
+        constexpr int VALUES = HD / 4 + 2;
+        float* left = reinterpret_cast<float*>(lds_raw) + tid;                  // [NH][VALUES][256]
+        __syncthreads();
+        if (half == 1)
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                left[(h * VALUES + HD / 4) * 256] = c[h].m;
+                left[(h * VALUES + HD / 4 + 1) * 256] = c[h].l;
+#pragma unroll
+                for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) left[(h * VALUES + t * 4 + r) * 256] = c[h].o[t][r];
+            }
+        __syncthreads();
+        if (half == 1) return;
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const float other = left[(h * VALUES + HD / 4) * 256], top = fmaxf(c[h].m, other);
+            // (a half without any key of this row keeps NEG_BIG: its factor is 0)
+            const float mine = __builtin_amdgcn_exp2f(c[h].m - top), theirs = __builtin_amdgcn_exp2f(other - top);
+            c[h].m = top;
+            c[h].l = c[h].l * mine + left[(h * VALUES + HD / 4 + 1) * 256] * theirs;
+#pragma unroll
+            for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) c[h].o[t][r] = c[h].o[t][r] * mine + left[(h * VALUES + t * 4 + r) * 256] * theirs;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+        float l = fw_quad_sum(c[h].l);
+        if (!valid) continue;
+        float inv = 1.0f / l;
+        if (sinks) {        // one more term in the sum, with no value: exp(sink), not scaled
+            const float sink = sinks[first_head + h] * 1.4426950408889634f;
+            const float top = fmaxf(c[h].m, sink);
+            const float shrink = exp2f(c[h].m - top);
+            inv = shrink / (l * shrink + exp2f(sink - top));
+        }
+        uint16_t* dest = out + ((size_t)my_row * num_heads + first_head + h) * HD;
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t) {
+            u32x2 packed = {pack_bf16(c[h].o[t][0] * inv, c[h].o[t][1] * inv), pack_bf16(c[h].o[t][2] * inv, c[h].o[t][3] * inv)};
+            *reinterpret_cast<u32x2*>(dest + t * 16 + g * 4) = packed;
+        }
+    }
+}
+
 // ---- decode ------------------------------------------------------------------------------------
 #define MERGE_PARTS 64               // parts of a row up to which the last workgroup keeps their weights in LDS (a context of 16,384 tokens at one run each)
 #define DECODE_WORKGROUPS 512        // two per compute unit: beyond, longer splits serve better than more of them
@@ -889,7 +1265,8 @@ static int check_common(const char* name, int rows, int num_heads, int num_kv_he
 // 1.27 ms for 2,048 rows behind 30,720 tokens, 32 heads in 8 groups, head_dim 64), one gives four
 // times as many workgroups to even out tiles of unequal length (58 vs 81 us for the same rows
 // from position 0; equal behind 6,144 tokens). The caller, who knows the positions, says which;
-// 0: chosen here from the shape alone: 4 where that still leaves every compute unit four workgroups.
+// 0: one. halves: 1 as above (PARTS 2 of the kernel for any head size), 2 heads two by two (attention_prompt_kernel), 3 those with the pages
+// shared out between two halves.
 extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_pages, const void* v_pages,
                                     const int32_t* block_table, int table_stride, const int32_t* tile_seg,
                                     const int32_t* tile_row0, int tiles, const int32_t* seg_row0,
@@ -904,14 +1281,34 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
     const int most_together = widest <= 64 ? 4 : 1;
     FW_REQUIRE(heads_together == 0 || heads_together == 1 || (heads_together == 4 && most_together == 4),
                "attention_prefill: %d heads together with head_dim %d (1, or 4 up to head_dim 64)", heads_together, head_dim);
-    FW_REQUIRE(!halves || (widest <= 64 && heads_together == 0), "attention_prefill: the pages are shared out between halves up to head_dim 64, two heads together");
+    FW_REQUIRE(halves >= 0 && halves <= 3, "attention_prefill: halves %d", halves);
+    FW_REQUIRE(halves != 1 || (widest <= 64 && heads_together == 0), "attention_prefill: the pages are shared out between halves up to head_dim 64, two heads together");
     if (rows == 0 || tiles == 0) return 0;
     const int group = num_heads / num_kv_heads;
+    const bool paired = halves >= 2;
+    FW_REQUIRE(!paired || (heads_together == 0 && head_dim == v_dim && (head_dim == 64 || head_dim == 128) && group % 2 == 0),
+               "attention_prefill: heads two by two are taken with head_dim and v_dim 64 or 128 and an even number of heads a group");
     if (halves) heads_together = 2;
     if (heads_together == 0) heads_together = 1;
     const long long blocks = (long long)tiles * num_kv_heads * ((group + heads_together - 1) / heads_together);
     FW_REQUIRE(blocks < (1ll << 31), "attention_prefill: too many tiles and heads");
     dim3 grid((unsigned)blocks);
+#define LAUNCH_PROMPT(HD, PARTS, STG)                                                                               \
+    {                                                                                                              \
+        const int stage_bytes = PARTS * 2 * STG * PAGE * HD * 2, merge_bytes = PARTS > 1 ? 2 * (HD / 4 + 2) * 256 * 4 : 0;  \
+        const int bytes = stage_bytes > merge_bytes ? stage_bytes : merge_bytes;                                   \
+        static bool configured = false;                                                                            \
+        if (!configured) {                                                                                         \
+            hipError_t status = hipFuncSetAttribute((const void*)attention_prompt_kernel<HD, PARTS, STG>,          \
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, bytes);            \
+            FW_REQUIRE(status == hipSuccess, "attention_prefill: cannot reserve %d bytes of LDS", bytes);          \
+            configured = true;                                                                                     \
+        }                                                                                                          \
+        attention_prompt_kernel<HD, PARTS, STG><<<grid, 256 * PARTS, bytes, (hipStream_t)stream>>>(                 \
+            (const uint16_t*)q, (uint16_t*)out, (const uint16_t*)k_pages, (const uint16_t*)v_pages, block_table,    \
+            table_stride, tile_seg, tile_row0, seg_row0, row_pos, num_heads, num_kv_heads, rule.scale_log2,        \
+            window, chunk, rule.cap, rule.cap_scale, keep_first, sinks, slopes);                                   \
+    }
 #define LAUNCH(HD, NH, PARTS)                                                                                      \
     {                                                                                                              \
         const int lds_bytes = PARTS * 2 * (PAGE * (HD + KV_PAD) + v_dim * (PAGE + KV_PAD)) * 2;                    \
@@ -929,7 +1326,13 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
             table_stride, tile_seg, tile_row0, seg_row0, row_pos, num_heads, num_kv_heads, head_dim, v_dim,        \
             rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, keep_first, sinks, slopes);                  \
     }
-    if (widest <= 32) {
+    if (paired) {
+        if (head_dim == 64) {
+            if (halves == 3) LAUNCH_PROMPT(64, 2, 4) else LAUNCH_PROMPT(64, 1, 4)
+        } else {
+            if (halves == 3) LAUNCH_PROMPT(128, 2, 2) else LAUNCH_PROMPT(128, 1, 2)
+        }
+    } else if (widest <= 32) {
         if (halves) LAUNCH(32, 2, 2) else if (heads_together == 4) LAUNCH(32, 4, 1) else LAUNCH(32, 1, 1)
     } else if (widest <= 64) {
         if (halves) LAUNCH(64, 2, 2) else if (heads_together == 4) LAUNCH(64, 4, 1) else LAUNCH(64, 1, 1)
@@ -939,6 +1342,7 @@ extern "C" int fw_attention_prefill(const void* q, void* out, const void* k_page
         LAUNCH(256, 1, 1)
     }
 #undef LAUNCH
+#undef LAUNCH_PROMPT
     FW_LAUNCH_CHECK("attention_prefill");
     return 0;
 }

@@ -183,7 +183,8 @@ int fw_attention_generic(const void* q, void* out, int dtype, const void* k_page
 // that see the most keys first. heads_together: how many query heads of a kv group one workgroup takes, reading
 // the keys and values once for all of them (0 and 1: one; 4 up to head_dim 64, slower than one head or halves at every length
 // measured: 32 heads, 2,048 rows behind 0 / 2,048 / 8,192 keys 76 / 144 / 347 us against 44 / 133 / 327). halves (with heads_together
-// 0, up to head_dim 64): two heads together, a tile's pages shared out between two halves of a workgroup that merge at the end.
+// 0) 1, up to head_dim 64: two heads together, a tile's pages shared out between two halves of a workgroup that merge at the end; 2, with head_dim and v_dim
+// both 64 or both 128 and an even number of heads a group: two heads together, three pages of the loop in flight; 3: the same in halves.
 int fw_attention_prefill(const void* q, void* out, const void* k_pages, const void* v_pages,
                          const int32_t* block_table, int table_stride, const int32_t* tile_seg,
                          const int32_t* tile_row0, int tiles, const int32_t* seg_row0, const int32_t* row_pos,

@@ -1088,9 +1088,10 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
                       seg_row0: torch.Tensor, row_pos: torch.Tensor, scale: float, window: int = 0,
                       heads_together: int = 0, out: Optional[torch.Tensor] = None, v_dim: Optional[int] = None,
                       chunk: int = 0, softcap: float = 0.0, keep_first: int = 0, sinks: Optional[torch.Tensor] = None,
-                      slopes: Optional[torch.Tensor] = None, halves: bool = False) -> torch.Tensor:
+                      slopes: Optional[torch.Tensor] = None, halves: bool = False, paired: bool = False) -> torch.Tensor:
     """``heads_together``: query heads of a kv group per workgroup (0 and 1: one; 4 up to head_dim 64). ``halves`` (up
-    to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. Only the rows of the given tiles are written (into ``out`` if given)."""
+    to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. ``paired`` (head_dim and v_dim both
+    64 or both 128, an even number of heads a group): two heads per workgroup, whose loop has three pages in flight; with ``halves`` or without. Only the rows of the given tiles are written (into ``out`` if given)."""
     _dev(q, k_pages, v_pages, block_table, tile_seg, tile_row0, seg_row0, row_pos)
     _want(q, torch.bfloat16, "q")
     rows = q.shape[0]
@@ -1111,7 +1112,7 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
         _p(q), _p(out), _p(k_pages), _p(v_pages), _p(block_table), block_table.shape[1], _p(tile_seg), _p(tile_row0),
         tile_seg.numel(), _p(seg_row0), _p(row_pos), rows, num_heads, num_kv_heads, head_dim, v_dim, float(scale),
         int(window), int(chunk), float(softcap), *_sinks(sinks, num_heads, keep_first, window, chunk, slopes), PAGE_SIZE, pages,
-        int(heads_together), int(halves), _stream()))
+        int(heads_together), int(halves) + (2 if paired else 0), _stream()))
     return out
 
 
@@ -1241,6 +1242,39 @@ def prompt_halves(tiles: int, num_heads: int, num_kv_heads: int, widest: int, ke
     return workgroups >= fill * rounds * COMPUTE_UNITS and keys >= least
 
 
+# us of the paired form: a workgroup of four waves per page while it has a compute unit to itself, while two share one, and of many in line for
+# two places a unit; eight waves per page; start, end (and merge) of either
+_PAIRED = {64: (0.93, 1.2, 1.32, 0.73, 4.0, 7.0), 128: (1.6, 2.2, 2.4, 1.09, 4.0, 8.5)}
+
+
+def prompt_pairs(tiles: int, num_heads: int, num_kv_heads: int, head_dim: int, v_dim: int, keys: int, context: int):
+    """Whether a prompt's attention takes the heads of a group two by two (fw_attention_prefill), and if so whether in halves: None, False or True.
+    ``tiles`` tiles of rows, of which the rows see up to ``keys`` keys, the last of them ``context`` if no window held it. It does where its kernel is built (heads of 64 or 128 channels, an even number a
+    group); with heads of 64 from 640 keys on: in front of that its two operands in flight have no page to hide behind (us, one head a workgroup / two by two:
+    37 rows 6.4 / 7.0, 300 9.9 / 10.8, 500 12.9 / 13.7, 777 17.4 / 16.6, 2,048 45 / 39, behind 2,048 keys 104 / 85, 16 heads behind 30,720 442 / 359).
+    Heads of 128: 16 in 4 groups, 37 rows 8.9 / 8.8, 1,111 rows 36.5 / 27.2, 2,048 44.7 / 29.0 with a window of 1,024, behind 4,096 keys 187 / 104.
+    Eight waves a workgroup (halves) or four by the estimated time of either: pages of a tile run from what the last tile sees down to what the first one does;
+    the longest workgroup, or all of them over the places there are, or two rounds in line (us, four / eight: 32 heads, 777 rows 18.6 / 17.6, 1,500
+    30.7 / 27.5, 3,000 65 / 78, 1,300 behind 2,048 66 / 71; 16 heads, 4,096 rows 71 / 64, 2,048 behind 30,720 462 / 359)."""
+    group = num_heads // num_kv_heads
+    if head_dim != v_dim or head_dim not in _PAIRED or group % 2 or tiles < 1 or (head_dim == 64 and keys < 640):
+        return None
+    alone, shared, many, eight, start, start_eight = _PAIRED[head_dim]
+    workgroups = tiles * num_kv_heads * (group // 2)
+    longest, last = -(-keys // 64), -(-context // 64)
+    full = min(tiles, max(1, last - longest + 1))           # tiles that see as much as the last one does; a page less each from there on
+    least = max(1, longest - (tiles - full))
+    total = (full * longest + (tiles - full) * (longest - 1 + least) / 2) * (workgroups // tiles)
+    four = start + max(longest * (alone if workgroups <= COMPUTE_UNITS else shared), total * many / (2 * COMPUTE_UNITS) if workgroups > 2 * COMPUTE_UNITS else 0.0)
+    rounds = -(-workgroups // COMPUTE_UNITS)
+    halves = start_eight + longest * eight
+    if rounds == 2:         # the workgroup that ends its round first, and the first of the next
+        halves = max(halves, 2 * (start_eight + eight * max(least, min(longest, longest + full - tiles * COMPUTE_UNITS / workgroups))))
+    elif rounds > 2:
+        halves = max(halves, rounds * start_eight + total * eight / COMPUTE_UNITS)
+    return halves < four
+
+
 def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int, k_pages: torch.Tensor,
               v_pages: torch.Tensor, block_table: torch.Tensor, ctx, scale: float, window: int = 0,
               tile_seg: Optional[torch.Tensor] = None, tile_row0: Optional[torch.Tensor] = None,
@@ -1266,10 +1300,14 @@ def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
         single = getattr(ctx, "decode_prefix", 0)       # leading segments of one row: rows and tiles 0 .. single - 1
         lengths = getattr(ctx, "new_lengths", None)     # what each segment sees in the end; the single rows' contexts are not the tiles'
         keys = min([n for n in (window, chunk) if n] + [max(lengths[single:]) if lengths else ctx.max_context])
-        halves = prompt_halves(tile_seg.numel() - single, num_heads, num_kv_heads, max(head_dim, v_dim), keys)
+        context = max(lengths[single:]) if lengths else ctx.max_context
+        halves = prompt_pairs(tile_seg.numel() - single, num_heads, num_kv_heads, head_dim, v_dim, keys, context)
+        paired = halves is not None
+        if not paired:
+            halves = prompt_halves(tile_seg.numel() - single, num_heads, num_kv_heads, max(head_dim, v_dim), keys)
         if single == 0:
             return attention_prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, tile_seg,
-                                     tile_row0, ctx.seg_row0, ctx.row_pos, scale, window, halves=halves, v_dim=v_dim,
+                                     tile_row0, ctx.seg_row0, ctx.row_pos, scale, window, halves=halves, paired=paired, v_dim=v_dim,
                                      chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)
         out = torch.empty((q.shape[0], num_heads * v_dim), dtype=q.dtype, device=q.device)
         attention_decode(q[:single], num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, ctx.row_seg,
@@ -1277,7 +1315,7 @@ def attention(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
                          chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)
         return attention_prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table,
                                  tile_seg[single:], tile_row0[single:], ctx.seg_row0, ctx.row_pos, scale, window,
-                                 halves=halves, out=out, v_dim=v_dim, chunk=chunk, softcap=softcap,
+                                 halves=halves, paired=paired, out=out, v_dim=v_dim, chunk=chunk, softcap=softcap,
                                  keep_first=keep_first, sinks=sinks, slopes=slopes)
     return attention_generic(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, ctx.row_seg,
                              ctx.row_pos, scale, window, v_dim=v_dim, chunk=chunk, softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)

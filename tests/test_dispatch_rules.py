@@ -72,6 +72,19 @@ def test_prompt_attention_shares_pages_between_halves_where_its_rounds_are_full(
     assert ops.prompt_halves(-(-rows // 64), heads, groups, widest, rows + behind) == halves
 
 
+@pytest.mark.parametrize("rows,behind,heads,groups,dim,v_dim,window,form", [
+    (37, 0, 32, 8, 64, 64, 0, None), (576, 0, 32, 8, 64, 64, 0, None), (777, 0, 32, 8, 64, 64, 0, False), (1111, 0, 32, 8, 64, 64, 0, True),
+    (1300, 2048, 32, 8, 64, 64, 0, False), (2048, 0, 32, 8, 64, 64, 0, True), (2048, 2048, 32, 8, 64, 64, 0, False), (3000, 0, 32, 8, 64, 64, 0, False),
+    (100, 2000, 32, 8, 64, 64, 0, True), (4096, 0, 16, 8, 64, 64, 0, True), (2048, 30720, 16, 8, 64, 64, 0, True), (2048, 2048, 24, 8, 64, 64, 0, None),
+    (2048, 2048, 32, 8, 64, 48, 0, None), (2048, 2048, 32, 8, 80, 80, 0, None), (37, 0, 16, 4, 128, 128, 1024, False), (300, 0, 16, 4, 128, 128, 1024, False),
+    (1111, 0, 16, 4, 128, 128, 1024, True), (2048, 0, 16, 4, 128, 128, 1024, True), (3000, 0, 16, 4, 128, 128, 1024, False),
+    (4096, 0, 16, 4, 128, 128, 1024, False), (2048, 4096, 16, 4, 128, 128, 0, True), (2048, 4096, 8, 8, 128, 128, 0, None)])
+def test_prompt_attention_takes_heads_two_by_two_where_that_is_faster(rows, behind, heads, groups, dim, v_dim, window, form):
+    from flyweight_amd.kernels import ops
+    context = rows + behind
+    assert ops.prompt_pairs(-(-rows // 64), heads, groups, dim, v_dim, min(window or context, context), context) is form
+
+
 def test_decode_rows_do_not_choose_the_form_of_a_prompt_beside_them(monkeypatch):
     """A new prompt of 777 rows beside a request that decodes behind 20,000 keys takes the form that it takes alone."""
     from types import SimpleNamespace

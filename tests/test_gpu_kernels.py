@@ -732,6 +732,53 @@ def test_attention_prefill_whose_halves_share_the_pages(ops, nh, nkv, hd, window
         run(halves=True, heads_together=1)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,window,keep_first,sink,slope,softcap,chunk", [
+    (4, 2, 64, 0, 0, False, False, 0.0, 0), (6, 1, 64, 0, 0, True, False, 0.0, 0), (8, 4, 64, 70, 0, False, False, 0.0, 0), (4, 2, 64, 64, 5, True, False, 0.0, 0),
+    (4, 2, 64, 130, 70, False, False, 0.0, 0), (2, 1, 64, 0, 0, False, True, 0.0, 0), (4, 1, 64, 0, 0, False, False, 8.0, 0), (2, 1, 64, 0, 0, False, False, 0.0, 100),
+    (4, 2, 128, 0, 0, False, False, 0.0, 0), (2, 1, 128, 70, 0, True, False, 0.0, 0), (4, 2, 128, 64, 5, False, False, 0.0, 0), (4, 1, 128, 1, 0, False, False, 5.0, 0),
+    (8, 2, 128, 0, 0, False, True, 0.0, 0), (2, 1, 128, 0, 0, False, False, 0.0, 65)])
+def test_attention_prefill_of_heads_two_by_two(ops, nh, nkv, hd, window, keep_first, sink, slope, softcap, chunk):
+    """Tiles of one page to more pages than are in flight, whose last page is whole, full but for a row and nearly empty (what lies behind the last value
+    is not a number), 5,000 keys (the numbers of the pages come 64 at a time), with every mask and bias: as one head at a time, in four waves and in eight."""
+    lengths = [150, 200, 64, 65, 33, 320, 128, 5000]
+    starts = [0, 120, 63, 64, 16, 5, 100, 4930]
+    keys, values, table, k_pages, v_pages = _mfma_setup(nh, nkv, hd, lengths, num_pages=100, seed=5)
+    counts = [n - s for n, s in zip(lengths, starts)]
+    seg_row0 = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    row_pos = np.concatenate([np.arange(s, n) for s, n in zip(starts, lengths)]).astype(np.int32)
+    row_seg = np.concatenate([np.full(c, i) for i, c in enumerate(counts)]).astype(np.int32)
+    tile_seg, tile_row0 = ops.query_tiles(seg_row0.tolist())
+    rows = int(seg_row0[-1])
+    q = as_dev(gen(rows, nh * hd, seed=4), torch.bfloat16)
+    scale = 1 / math.sqrt(hd)
+    generator = torch.Generator().manual_seed(1)
+    sinks = torch.randn(nh, generator=generator).to(DEV) if sink else None
+    slopes = (0.05 * torch.rand(nh, generator=generator)).to(DEV) if slope else None
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    run = lambda **how: ops.attention_prefill(q, nh, nkv, hd, k_pages, v_pages, d(table), d(tile_seg), d(tile_row0), d(seg_row0),  # noqa: E731
+                                              d(row_pos), scale, window, keep_first=keep_first, sinks=sinks, slopes=slopes, softcap=softcap, chunk=chunk, **how)
+    plain = run(heads_together=1)
+    for halves in (False, True):
+        found = run(paired=True, halves=halves)
+        close(found, back(plain), torch.bfloat16)
+        if not (sink or keep_first or slope or softcap or chunk):
+            want = torch.stack([attention_reference(back(q)[r].reshape(nh, hd), keys[row_seg[r]], values[row_seg[r]], int(row_pos[r]),
+                                                    scale, window, nh // nkv).reshape(-1) for r in range(rows)])
+            close(found, want, torch.bfloat16)
+        assert torch.equal(found, run(paired=True, halves=halves))
+    with pytest.raises(ops.KernelError, match="two by two"):
+        run(paired=True, heads_together=1)
+
+
+def test_attention_prefill_of_heads_two_by_two_refuses_other_heads(ops):
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    for nh, nkv, hd in ((3, 1, 64), (4, 2, 48), (4, 2, 80)):
+        _, _, table, k_pages, v_pages = _mfma_setup(nh, nkv, hd, [70], num_pages=3, seed=5)
+        q = as_dev(gen(70, nh * hd, seed=4), torch.bfloat16)
+        with pytest.raises(ops.KernelError, match="two by two"):
+            ops.attention_prefill(q, nh, nkv, hd, k_pages, v_pages, d(table), d([0, 0]), d([0, 64]), d([0, 70]), d(np.arange(70)), 0.1, 0, paired=True)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,window", [(4, 2, 16, 0), (3, 1, 48, 0), (6, 3, 80, 0), (32, 8, 64, 0), (2, 2, 128, 0),
                                               (20, 1, 256, 0), (4, 2, 32, 300), (4, 4, 64, 64), (2, 1, 64, 1)])
 def test_attention_decode_on_the_matrix_cores(ops, nh, nkv, hd, window):
