@@ -129,8 +129,7 @@ __global__ __launch_bounds__(256) void rmsnorm_rows4_kernel(const float* __restr
         scale[u] = reinterpret_cast<const f32x4*>(weight)[piece < pieces ? piece : 0];
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-        sum += (held[u][0] * held[u][0] + held[u][1] * held[u][1]) + (held[u][2] * held[u][2] + held[u][3] * held[u][3]);
+    for (int u = 0; u < 4; ++u) sum += fw_sum_of_squares(held[u]);
     sum = block_sum(sum, scratch);
     const float inv = rsqrtf(sum / (float)hidden + eps);
     const float one = one_centered ? 1.0f : 0.0f;

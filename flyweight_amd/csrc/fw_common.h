@@ -155,6 +155,9 @@ template <> __device__ __forceinline__ float round_through<bf16_t>(float v) {
     return bf16_bits_to_float(float_to_bf16_bits(v));
 }
 
+// the squares of four neighbours of a row, as every kernel that sums a row's squares adds them
+template <typename V> __device__ __forceinline__ float fw_sum_of_squares(const V& v) { return (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]); }
+
 // ---- wave64 reductions (fixed butterfly order: the result does not depend on
 //      anything but the 64 inputs) -----------------------------------------------------
 __device__ __forceinline__ float wave_sum(float v) {

@@ -20,12 +20,15 @@
 //  * Every output is the sum over the same groups of the same four k in the same order, part by part, the parts
 //    four by four, whatever the tile: its value does not depend on M or on the other rows.
 //
+// One and two rows over K from 1,024 on go to gemm_float32_few.hip, which gives the same bits.
+//
 // Measured inside a request of the LFM2-350M shape in float32, before -> after: one row, 1,024 outputs (K 4,608 and 1,024
 // in the mean) 464 -> 9.3 us, gate|up (2 x 4,608, K 1,024) 171 + 5 -> 13.6 us (2.8 TB/s of W), 65,536 outputs 255 -> 49 us (5.4
 // TB/s); 301 rows, gate|up 222 + 5 -> 82 us (69 TFLOP/s), 1,024 outputs 523 -> 38 us; 2,048 rows by 1,024 outputs, K 4,608: 187 us
 // (103 TFLOP/s). The sums' distance from 64 bits in that request's logits fell from 8.8e-6 to 2.4e-6.
 #include "fw_common.h"
 #include "fw_kernels.h"
+#include "float32_few.h"
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -350,6 +353,7 @@ extern "C" int fw_gemm_float32(const float* a, const float* w, const float* bias
     FW_REQUIRE((long long)fw_ceil_div(M, 16) * fw_ceil_div(N, 8) < (1ll << 30), "gemm_float32: M=%d N=%d are too many tiles", M, N);
     if (M == 0) return 0;
     hipStream_t s = (hipStream_t)stream;
+    if (fw_gemm_float32_few_takes(M, N, K, mode, false)) return fw_launch_float32_few(a, nullptr, nullptr, 0.0f, 0, w, bias, out, out_dtype, mode, M, N, K, s);
     if (mode == MF_ACCUMULATE) choose<MF_ACCUMULATE, float>(a, w, bias, out, M, N, K, s);
     else if (mode == MF_SWIGLU) choose<MF_SWIGLU, float>(a, w, nullptr, out, M, N, K, s);
     else if (out_dtype == FW_F32) choose<MF_STORE, float>(a, w, bias, out, M, N, K, s);

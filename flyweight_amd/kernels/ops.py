@@ -285,6 +285,35 @@ def gemm_generic(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] 
     return target
 
 
+@functools.lru_cache(maxsize=4096)
+def float32_normed_takes(gated: bool, rows: int, features: int, k: int) -> bool:
+    """Whether a float32 product of few rows takes their RMS norm in front (``gemm_float32_normed``)."""
+    return bool(library().fw_gemm_float32_normed_takes(2 if gated else 0, rows, features, k))
+
+
+def gemm_float32_normed(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, one_centered: bool, w: torch.Tensor, bias: Optional[torch.Tensor] = None, *,
+                        row_index: Optional[torch.Tensor] = None, gated: bool = False) -> torch.Tensor:
+    """``rmsnorm_rows`` followed by the product with ``w`` (``gated``: silu(gate) * up of [gate rows; up rows]), float32 throughout, in one kernel and bit
+    for bit as the two give it; ``float32_normed_takes`` says which shapes."""
+    _dev(x, norm_weight, w, bias, row_index)
+    for name, t in (("x", x), ("norm_weight", norm_weight), ("w", w)) + ((("bias", bias),) if bias is not None else ()):
+        _want(t, torch.float32, name)
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or norm_weight.shape != (x.shape[1],):
+        raise KernelError(f"gemm_float32_normed: x is {tuple(x.shape)}, w {tuple(w.shape)}, the norm's weight {tuple(norm_weight.shape)}")
+    if row_index is not None:
+        _want(row_index, torch.int32, "row_index")
+    rows = x.shape[0] if row_index is None else row_index.numel()
+    features = w.shape[0] // 2 if gated else w.shape[0]
+    if (gated and w.shape[0] % 2) or (bias is not None and bias.shape != (w.shape[0],)):
+        raise KernelError("gemm_float32_normed: gate and up rows are even in number, a bias has a value per row of w")
+    if eps <= 0.0:
+        raise KernelError("gemm_float32_normed: eps must be positive")
+    out = torch.empty((rows, features), dtype=torch.float32, device=x.device)
+    _check(library().fw_gemm_float32_normed(_p(x), _p(norm_weight), _p(row_index), float(eps), int(one_centered), _p(w), _p(bias), _p(out), 2 if gated else 0, rows,
+                                            features, x.shape[1], _stream()))
+    return out
+
+
 def _float32_ok(a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the product runs on the float32 matrix instruction, whose lanes read four k at once; other operands and
     other K take the plain FMA tiles (one row, 1,024 outputs: 464 us against 9; 301 rows: 523 against 38)."""

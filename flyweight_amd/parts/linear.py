@@ -96,6 +96,11 @@ class Linear:
             return {}
         return {"squares": a.prepared.squares, "eps": a.rms_parameters()[1]}
 
+    def _normed(self, a: Input, features: int, gated: bool) -> bool:
+        """Few float32 rows whose norm has not run yet: their product takes it in front."""
+        return (isinstance(a, LazyNorm) and a.dtype == torch.float32 and self.weight.dtype == torch.float32 and a.pending
+                and ops.float32_normed_takes(gated, a.rows, features, self.in_features))
+
     # ----- products -----------------------------------------------------------------------
     def forward(self, a: Input, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
         out_dtype = out_dtype or a.dtype
@@ -105,6 +110,8 @@ class Linear:
         if self._fused(a, self.out_features, ops.EPILOGUE_STORE):
             return ops.gemm_decode(self._rows_of(a), self.weight, ops.EPILOGUE_STORE, bias=self.bias, out_dtype=out_dtype,
                                    w_tiled=self.tiled, **self._norm_arguments(a))
+        if out_dtype == torch.float32 and self._normed(a, self.out_features, False):
+            return ops.gemm_float32_normed(a.x, *a.rms_parameters(), self.weight, self.bias, row_index=a.row_index)
         return ops.gemm(self._tensor_of(a), self.weight, self.bias, out_dtype=out_dtype, w_tiled=self.tiled)
 
     def accumulate(self, a: torch.Tensor, residual: torch.Tensor, then=None) -> Optional[Prepared]:
@@ -142,6 +149,8 @@ class Linear:
         if self.bias is None and self._fused(a, self.out_features // 2, ops.EPILOGUE_SWIGLU):
             return ops.gemm_decode(self._rows_of(a), self.weight, ops.EPILOGUE_SWIGLU, out_dtype=torch.bfloat16,
                                    w_tiled=self.tiled, glu=glu, **self._norm_arguments(a))
+        if self.bias is None and not gelu and self._normed(a, self.out_features // 2, True):
+            return ops.gemm_float32_normed(a.x, *a.rms_parameters(), self.weight, row_index=a.row_index, gated=True)
         return ops.gemm_swiglu(self._tensor_of(a), self.weight, w_tiled=self.tiled, gelu=gelu)
 
     def gelu(self, a: torch.Tensor) -> torch.Tensor:

@@ -67,6 +67,12 @@ class LazyNorm:
     def dtype(self) -> torch.dtype:
         return self.norm.dtype
 
+    @property
+    def pending(self) -> bool:
+        """Whether the norm is a plain RMS norm over float32 rows that has not run yet, nor any part of it."""
+        return self._tensor is None and self.prepared is None and self.x.dtype == torch.float32 and self.x.is_contiguous() \
+            and self.x.data_ptr() % 16 == 0 and self.rms_parameters() is not None
+
     def rms_parameters(self):
         """(weight, eps, one_centered) if the norm is a plain RMS norm, else None."""
         return self.norm.rms_parameters() if hasattr(self.norm, "rms_parameters") else None

@@ -89,3 +89,75 @@ def test_what_its_loads_cannot_take_goes_to_the_plain_tiles(ops):
     b, v = flat[1:].view(5, 64), draw(40, 64, seed=1)
     exact = b.cpu().double() @ v.double().T
     assert ((ops.gemm(b, v.to(DEV)).cpu().double() - exact).abs() <= bound(b.cpu(), v)).all()
+
+
+# K of whole groups and parts, ending inside a group, inside a part, with parts that have nothing; the deeper ring; outputs at the edges of both tiles
+@pytest.mark.parametrize("K", [1024, 1028, 1040, 1280, 2052, 3900, 4096, 4100, 8192])
+@pytest.mark.parametrize("N", [1, 5, 1024, 3071, 3072, 3081])
+def test_few_rows_have_the_values_of_many(ops, N, K):
+    """One and two rows go to a kernel of their own, three and more to the matrix instruction: the same bits, with and without the norm in front."""
+    a, w = draw(19, K).to(DEV), draw(2 * N, K, seed=1).to(DEV)
+    bias, weight = draw(N, seed=2).to(DEV), draw(K, seed=3).to(DEV)
+    old = draw(19, N, seed=4).to(DEV)
+    for one_centered in (False, True):
+        if K > 4096 or (one_centered and N > 5):
+            break
+        normed = ops.rmsnorm_rows(a, weight, 1e-5, torch.float32, one_centered=one_centered)
+        stored, gated = ops.gemm(normed, w[:N], bias), ops.gemm_swiglu(normed, w)
+        index = torch.tensor([11, 4], dtype=torch.int32, device=DEV)
+        for rows in (1, 2):
+            of = index[:rows].long()
+            if ops.float32_normed_takes(False, rows, N, K):
+                assert torch.equal(ops.gemm_float32_normed(a, weight, 1e-5, one_centered, w[:N].contiguous(), bias, row_index=index[:rows]), stored[of])
+                assert torch.equal(ops.gemm_float32_normed(a[:rows].contiguous(), weight, 1e-5, one_centered, w[:N].contiguous(), bias), stored[:rows])
+            if ops.float32_normed_takes(True, rows, N, K):
+                assert torch.equal(ops.gemm_float32_normed(a, weight, 1e-5, one_centered, w, row_index=index[:rows], gated=True), gated[of])
+    stored, gated = ops.gemm(a, w[:N], bias), ops.gemm_swiglu(a, w)
+    total = ops.gemm(a, w[:N], accumulate_into=old.clone())
+    rounded = ops.gemm(a, w[:N], out_dtype=torch.bfloat16)
+    for rows in (1, 2):
+        few = a[:rows].contiguous()
+        assert torch.equal(ops.gemm(few, w[:N], bias), stored[:rows])
+        assert torch.equal(ops.gemm(few, w[:N], out_dtype=torch.bfloat16), rounded[:rows])
+        assert torch.equal(ops.gemm(few, w[:N], accumulate_into=old[:rows].clone()), total[:rows])
+        assert torch.equal(ops.gemm_swiglu(few, w), gated[:rows])
+
+
+def test_what_a_normed_product_of_few_rows_refuses(ops):
+    assert not ops.float32_normed_takes(False, 3, 64, 1024) and not ops.float32_normed_takes(False, 1, 64, 4100) and not ops.float32_normed_takes(False, 1, 64, 1020)
+    a, w, weight = draw(1, 1020).to(DEV), draw(64, 1020, seed=1).to(DEV), draw(1020, seed=2).to(DEV)
+    with pytest.raises(ops.KernelError, match="not taken"):
+        ops.gemm_float32_normed(a, weight, 1e-5, False, w)
+    with pytest.raises(ops.KernelError, match="norm"):
+        ops.gemm_float32_normed(a, weight[:1000].contiguous(), 1e-5, False, w)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,v_dim,window,keep_first,sink,slope,softcap,chunk", [
+    (4, 2, 64, 64, 0, 0, False, False, 0.0, 0), (6, 2, 64, 48, 70, 0, False, False, 0.0, 0), (4, 1, 128, 128, 100, 70, True, False, 0.0, 0),
+    (2, 2, 20, 320, 0, 0, False, True, 0.0, 0), (4, 2, 320, 64, 0, 0, False, False, 6.0, 0), (4, 2, 64, 1024, 0, 0, True, False, 0.0, 130)])
+def test_attention_of_few_rows_has_the_values_of_many(ops, nh, nkv, hd, v_dim, window, keep_first, sink, slope, softcap, chunk):
+    """Eight pages side by side, folded in their order: the same bits as a page after the other, for contexts of one page to more than two rounds of eight."""
+    lengths = [1, 63, 64, 65, 300, 512, 513, 1100]
+    generator = torch.Generator().manual_seed(1)
+    many = 300 // nh + 1                                    # copies of the rows: more rows times heads than compute units
+    pages = [(n + 63) // 64 for n in lengths]
+    order = torch.randperm(sum(pages), generator=generator).tolist()
+    table = torch.zeros(len(lengths), max(pages), dtype=torch.int32)
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.tensor([order.pop() for _ in range(n)])
+    k_pages, v_pages = draw(sum(pages), nkv, 64, hd, seed=2).to(DEV), draw(sum(pages), nkv, v_dim, 64, seed=3).to(DEV)
+    for i, n in enumerate(lengths):                         # what lies behind the last key is not a number
+        if n % 64:
+            v_pages[table[i, pages[i] - 1].item(), :, :, n % 64:] = float("nan")
+            k_pages[table[i, pages[i] - 1].item(), :, n % 64:] = float("nan")
+    sinks = draw(nh, seed=4).to(DEV) if sink else None
+    slopes = (0.05 * torch.rand(nh, generator=generator)).to(DEV) if slope else None
+    table = table.to(DEV)
+    for i, n in enumerate(lengths):
+        q = draw(1, nh * hd, seed=10 + i).to(DEV)
+        run = lambda copies: ops.attention_generic(q.repeat(copies, 1), nh, nkv, hd, k_pages, v_pages, table, torch.full((copies,), i, dtype=torch.int32, device=DEV),   # noqa: E731,E501,B023
+                                                   torch.full((copies,), n - 1, dtype=torch.int32, device=DEV), hd ** -0.5, window, v_dim=v_dim, chunk=chunk,      # noqa: B023
+                                                   softcap=softcap, keep_first=keep_first, sinks=sinks, slopes=slopes)
+        few, rows = run(1), run(many)
+        assert torch.isfinite(few).all()
+        assert torch.equal(rows, few.expand_as(rows))
