@@ -338,6 +338,115 @@ __global__ __launch_bounds__(64) void attention_generic_kernel(
     }
 }
 
+// The same for steps of few rows, float32, head sizes that are multiples of 4: a workgroup of eight waves per (row, head), which take eight pages side by
+// side. Scores, maxima, exponentials and a page's weighted sum are formed page by page as above, and the pages then folded in their order with the same
+// expressions: bit for bit the same results. What it saves is the chain from page to page: 16 heads of 64 channels, one row behind 301-308
+// keys 19.5 -> FW_PAGES_FIGURE us. With rows times heads enough to fill the chip the waves above have no idle compute units beside them.
+#define SIDE 8
+#define PAGES_MOST 256          // rows times heads: a workgroup a compute unit
+__global__ __launch_bounds__(64 * SIDE) void attention_pages_kernel(
+    const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
+    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ row_seg,
+    const int32_t* __restrict__ row_pos, int num_heads, int num_kv_heads, int head_dim, int v_dim, float scale, int window,
+    int chunk, float softcap, int keep_first, const float* __restrict__ sinks, const float* __restrict__ slopes) {
+    __shared__ __attribute__((aligned(16))) float qs[ATTN_MAX_HEAD_DIM];
+    __shared__ __attribute__((aligned(16))) float ps[SIDE][ATTN_PAGE];
+    __shared__ float page_max[SIDE], page_sum[SIDE], parts[SIDE][64 * SIDE];
+    const int row = blockIdx.x, head = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kvh = head / (num_heads / num_kv_heads);
+    const int pos = row_pos[row];
+    const int32_t* table = block_table + (size_t)row_seg[row] * table_stride;
+    const float* query = q + ((size_t)row * num_heads + head) * head_dim;
+    for (int d = tid; d < head_dim; d += 64 * SIDE) qs[d] = query[d];
+    const int first = fw_first_visible(pos, window, chunk);
+    const int kept = keep_first < first ? keep_first : first;
+    const int head_tiles = (kept + ATTN_PAGE - 1) / ATTN_PAGE < first / ATTN_PAGE ? (kept + ATTN_PAGE - 1) / ATTN_PAGE : first / ATTN_PAGE;
+    const int tiles = head_tiles + pos / ATTN_PAGE - first / ATTN_PAGE + 1;
+    float running_max = -INFINITY, running_sum = 0.0f, acc = 0.0f;         // acc: channel tid
+    for (int at0 = 0; at0 < tiles; at0 += SIDE) {
+        const int here = tiles - at0 < SIDE ? tiles - at0 : SIDE;
+        const bool busy = wave < here;
+        const int at = at0 + (busy ? wave : 0);
+        const int tile = at < head_tiles ? at : first / ATTN_PAGE + at - head_tiles;
+        const int page = table[tile];
+        const int t = tile * ATTN_PAGE + lane;
+        const bool valid = busy && (t >= first || t < kept) && t <= pos;
+        const float* values = v_pages + ((size_t)page * num_kv_heads + kvh) * v_dim * ATTN_PAGE;
+        float4 ahead[ATTN_PAGE / 4];
+        const float4* value_ahead = reinterpret_cast<const float4*>(values + (size_t)(lane < v_dim ? lane : 0) * ATTN_PAGE);
+        // (a load of 64 rows' pieces costs the compute unit 64 lookups: a wave without a page asks for nothing)
+        if (busy)
+#pragma unroll
+            for (int i = 0; i < ATTN_PAGE / 4; ++i) ahead[i] = value_ahead[i];
+        fw_lds_barrier();                                                   // the query is there; the parts before have been folded (the loads stay on their way)
+        float score = -INFINITY;
+        if (valid) {
+            const float4* key4 = reinterpret_cast<const float4*>(k_pages + (((size_t)page * num_kv_heads + kvh) * ATTN_PAGE + lane) * head_dim);
+            const float4* q4 = reinterpret_cast<const float4*>(qs);
+            float dot = 0.0f;
+#pragma unroll 16
+            for (int d = 0; d < head_dim / 4; ++d) {
+                const float4 k = key4[d], x = q4[d];
+                dot = fmaf(x.w, k.w, fmaf(x.z, k.z, fmaf(x.y, k.y, fmaf(x.x, k.x, dot))));
+            }
+            score = dot * scale;
+            if (softcap > 0.0f) score = softcap * tanhf(score / softcap);
+            if (slopes) score -= slopes[head] * (float)(pos - t);
+        }
+        const float most = wave_max(score);
+        if (busy && lane == 0) page_max[wave] = most;
+        fw_lds_barrier();
+        if (busy) {
+            float new_max = running_max;
+            for (int i = 0; i <= wave; ++i) new_max = fmaxf(new_max, page_max[i]);
+            const float p = valid ? expf(score - new_max) : 0.0f;
+            const float sum = wave_sum(p);
+            if (lane == 0) page_sum[wave] = sum;
+            ps[wave][lane] = p;
+            const int lo = (first - tile * ATTN_PAGE > 0 && kept <= tile * ATTN_PAGE) ? first - tile * ATTN_PAGE : 0;
+            const int hi = pos - tile * ATTN_PAGE < ATTN_PAGE - 1 ? pos - tile * ATTN_PAGE : ATTN_PAGE - 1;
+            const bool whole = lo == 0 && hi == ATTN_PAGE - 1;
+            const float4* p4 = reinterpret_cast<const float4*>(ps[wave]);   // (a wave's own: its writes are ahead of its reads)
+            for (int j = 0; 64 * j < v_dim; ++j) {
+                const int d = lane + 64 * j;
+                if (d < v_dim) {
+                    const float4* value4 = reinterpret_cast<const float4*>(values + (size_t)d * ATTN_PAGE);
+                    float part = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < ATTN_PAGE / 4; ++i) {
+                        float4 v = j == 0 ? ahead[i] : value4[i];
+                        const float4 w = p4[i];
+                        if (!whole) {
+                            v.x = 4 * i >= lo && 4 * i <= hi ? v.x : 0.0f;
+                            v.y = 4 * i + 1 >= lo && 4 * i + 1 <= hi ? v.y : 0.0f;
+                            v.z = 4 * i + 2 >= lo && 4 * i + 2 <= hi ? v.z : 0.0f;
+                            v.w = 4 * i + 3 >= lo && 4 * i + 3 <= hi ? v.w : 0.0f;
+                        }
+                        part = fmaf(w.w, v.w, fmaf(w.z, v.z, fmaf(w.y, v.y, fmaf(w.x, v.x, part))));
+                    }
+                    parts[wave][d] = part;
+                }
+            }
+        }
+        fw_lds_barrier();
+        for (int i = 0; i < here; ++i) {
+            const float new_max = fmaxf(running_max, page_max[i]);
+            const float alpha = expf(running_max - new_max);
+            running_sum = running_sum * alpha + page_sum[i];
+            running_max = new_max;
+            if (tid < v_dim) acc = acc * alpha + parts[i][tid];
+        }
+    }
+    float shrink = 1.0f;
+    if (sinks) {
+        const float sink = sinks[head];
+        const float new_max = fmaxf(running_max, sink);
+        shrink = expf(running_max - new_max);
+        running_sum = running_sum * shrink + expf(sink - new_max);
+    }
+    if (tid < v_dim) out[((size_t)row * num_heads + head) * v_dim + tid] = acc * shrink / running_sum;
+}
+
 extern "C" int fw_attention_generic(const void* q, void* out, int dtype, const void* k_pages,
                                     const void* v_pages, const int32_t* block_table, int table_stride,
                                     const int32_t* row_seg, const int32_t* row_pos, int rows, int num_heads,
@@ -359,7 +468,12 @@ extern "C" int fw_attention_generic(const void* q, void* out, int dtype, const v
     attention_generic_kernel<T, WIDE><<<grid, 64, 0, (hipStream_t)stream>>>(                                                      \
         (const T*)q, (T*)out, (const T*)k_pages, (const T*)v_pages, block_table, table_stride, row_seg, row_pos, num_heads,       \
         num_kv_heads, head_dim, v_dim, scale, window, chunk, softcap, keep_first, sinks, slopes)
-    if (dtype == FW_F32 && head_dim % 4 == 0 && ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0) FW_ATTENTION_LAUNCH(float, true);
+    const bool wide = dtype == FW_F32 && head_dim % 4 == 0 && ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
+    if (wide && v_dim <= 64 * SIDE && (long long)rows * num_heads <= PAGES_MOST)          // (a thread has a channel of the output)
+        attention_pages_kernel<<<grid, 64 * SIDE, 0, (hipStream_t)stream>>>(
+            (const float*)q, (float*)out, (const float*)k_pages, (const float*)v_pages, block_table, table_stride, row_seg, row_pos, num_heads, num_kv_heads,
+            head_dim, v_dim, scale, window, chunk, softcap, keep_first, sinks, slopes);
+    else if (wide) FW_ATTENTION_LAUNCH(float, true);
     else if (dtype == FW_F32) FW_ATTENTION_LAUNCH(float, false);
     else if (dtype == FW_BF16) FW_ATTENTION_LAUNCH(bf16_t, false);
 #undef FW_ATTENTION_LAUNCH
