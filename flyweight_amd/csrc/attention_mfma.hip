@@ -71,7 +71,7 @@ struct Columns {
 // (all pages but those on the diagonal, at a window's edge, and a sequence's last) skips the
 // mask. The scale is folded into the exponent's argument: the maximum is taken over the raw
 // scores (the scale is positive) and kept scaled.
-template <int HD, int NH, bool CLEAN_V, bool K_PADDED, bool EARLY_V = false>
+template <int HD, int NH, bool CLEAN_V, bool K_PADDED>
 __device__ __forceinline__ void attend_page(Columns<HD> (&c)[NH], const uint16_t* __restrict__ k_page,
                                             const uint16_t* __restrict__ v_page, int head_dim, int v_dim, float scale_log2,
                                             int lo, int hi, int last_written, int k_stride, int v_stride,
@@ -92,20 +92,6 @@ __device__ __forceinline__ void attend_page(Columns<HD> (&c)[NH], const uint16_t
                 if (dc * 32 + g * 8 < head_dim) kf[kt][dc] = *reinterpret_cast<const bf16x8*>(key + dc * 32);
             }
         }
-    }
-    // EARLY_V (pages read from global memory, one page per wave): the values are asked for
-    // together with the keys, so that they travel while the scores are formed, not after them.
-    u32x2 early_a[EARLY_V ? 2 : 1][EARLY_V ? HD / 16 : 1], early_b[EARLY_V ? 2 : 1][EARLY_V ? HD / 16 : 1];
-    if (EARLY_V) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-            for (int t = 0; t < HD / 16; ++t) {
-                const int channel = t * 16 + i16 < v_dim ? t * 16 + i16 : v_dim - 1;
-                const uint16_t* value = v_page + (size_t)channel * v_stride + kb * 32 + g * 4;
-                early_a[kb][t] = *reinterpret_cast<const u32x2*>(value);
-                early_b[kb][t] = *reinterpret_cast<const u32x2*>(value + 16);
-            }
     }
     // scores of all heads
     f32x4 s[NH][4];
@@ -236,14 +222,7 @@ __device__ __forceinline__ void attend_page(Columns<HD> (&c)[NH], const uint16_t
         for (int t = 0; t < HD / 16; ++t) {
             const int channel = t * 16 + i16 < v_dim ? t * 16 + i16 : v_dim - 1;
             const uint16_t* value = v_page + (size_t)channel * v_stride;
-            u32x2 va, vb;
-            if (EARLY_V) {
-                va = early_a[kb][t];
-                vb = early_b[kb][t];
-            } else {
-                va = *reinterpret_cast<const u32x2*>(value + key_a);
-                vb = *reinterpret_cast<const u32x2*>(value + key_b);
-            }
+            const u32x2 va = *reinterpret_cast<const u32x2*>(value + key_a), vb = *reinterpret_cast<const u32x2*>(value + key_b);
             u32x4 vw = {va[0], va[1], vb[0], vb[1]};
             if (CLEAN_V) vw = u32x4{va[0] & keep_a0, va[1] & keep_a1, vb[0] & keep_b0, vb[1] & keep_b1};
             const bf16x8 vf = __builtin_bit_cast(bf16x8, vw);
@@ -253,6 +232,139 @@ __device__ __forceinline__ void attend_page(Columns<HD> (&c)[NH], const uint16_t
     }
     // for the same reason the last products have left the pipe before control leaves this function
     fw_mfma_drain();
+}
+
+// ---- pages that stream through registers (decode, up to 128 channels) ---------------------------
+// The keys and values of a page on their way into a wave's registers. A matrix product sums over its
+// operands in any order, so the key that stands in row i of score tile kt is chosen to suit the values: 32 (kt / 2)
+// + 8 (i / 4) + 4 (kt % 2) + i % 4. Then the eight keys whose probabilities a lane holds for half a page
+// follow one another, and their values are one load of 16 bytes (four lanes together 64 bytes of a channel).
+template <int HD>
+struct PageOnWay {
+    u32x4 k[4][HD / 32], v[2][HD / 16];
+};
+// Every lane's byte offsets in a page. Loads go through a buffer descriptor that ends with the page: channels past
+// head_dim or v_dim give zeros, and a page that is not wanted has a descriptor of no bytes and costs no traffic.
+template <int HD>
+struct PageOffsets {
+    uint32_t k[4][HD / 32], v;
+    __device__ __forceinline__ PageOffsets(int head_dim) {
+        const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int dc = 0; dc < HD / 32; ++dc) {
+                const int key = (kt >> 1) * 32 + (i16 >> 2) * 8 + (kt & 1) * 4 + (i16 & 3), channel = dc * 32 + g * 8;
+                k[kt][dc] = channel < head_dim ? (uint32_t)(key * head_dim + channel) * 2 : 0x7ffffff0u;
+            }
+        v = (uint32_t)(i16 * PAGE + g * 8) * 2;
+    }
+};
+__device__ __forceinline__ u32x4 page_words(fw_buffer from, uint32_t at) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(from, at, 0, 0)); }
+template <int HD>
+__device__ __forceinline__ void ask_for_keys(PageOnWay<HD>& page, const PageOffsets<HD>& at, fw_buffer from) {
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int dc = 0; dc < HD / 32; ++dc) page.k[kt][dc] = page_words(from, at.k[kt][dc]);
+}
+template <int HD>
+__device__ __forceinline__ void ask_for_values(PageOnWay<HD>& page, const PageOffsets<HD>& at, fw_buffer from) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t) page.v[kb][t] = page_words(from, at.v + t * 16 * PAGE * 2 + kb * 64);
+}
+
+// One page against one set of columns, as attend_page takes it: the same scores, maxima and exponentials, summed in the
+// order of PageOnWay. As soon as the keys (values) have met their products, `ask_keys` (`ask_values`) asks for those of
+// a later page into the same registers, so that the wave's loads never pause.
+template <int HD, typename AskKeys, typename AskValues>
+__device__ __forceinline__ void attend_on_way(Columns<HD>& c, PageOnWay<HD>& page, float scale_log2, int lo, int hi, float cap, float cap_scale, int kept,
+                                              bool biased, float dist, AskKeys ask_keys, AskValues ask_values) {
+    const int g = (threadIdx.x & 63) >> 4;
+    f32x4 s[4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+        s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int dc = 0; dc < HD / 32; ++dc)
+            s[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, page.k[kt][dc]), c.q[dc], s[kt], 0, 0, 0);
+    }
+    fw_mfma_drain();        // the branches below read the scores
+    ask_keys();
+    // this lane's score [kt][r] is that of key 32 (kt / 2) + 8 g + 4 (kt % 2) + r
+    auto key_of = [&](int kt, int r) { return (kt >> 1) * 32 + g * 8 + (kt & 1) * 4 + r; };
+    if (cap > 0.0f) {
+        const float twice = 2.0f * cap_scale * 1.4426950408889634f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = __builtin_amdgcn_exp2f(s[kt][r] * twice);
+                s[kt][r] = cap - 2.0f * cap * __builtin_amdgcn_rcpf(1.0f + e);
+            }
+    }
+    if (biased) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[kt][r] = fmaf(-dist, (float)(hi - key_of(kt, r)), s[kt][r]);
+    }
+    // a page with keys that do not count: their scores leave the sum, and the values behind the row's own
+    // position (an earlier owner's, perhaps no numbers) are cleared before they meet a probability of 0
+    if (hi < PAGE - 1 || !(lo <= 0 || kept >= lo)) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int key = key_of(kt, r);
+                s[kt][r] = (key >= lo || key < kept) && key <= hi ? s[kt][r] : NEG_BIG;
+            }
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int key = kb * 32 + g * 8 + 2 * w;
+                const uint32_t keep = key + 1 <= hi ? 0xffffffffu : (key <= hi ? 0xffffu : 0u);
+#pragma unroll
+                for (int t = 0; t < HD / 16; ++t) page.v[kb][t][w] &= keep;
+            }
+    }
+    float page_max = NEG_BIG;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) page_max = fmaxf(page_max, s[kt][r]);
+    page_max = fw_quad_max(page_max);
+    // a column that has seen no key yet keeps NEG_BIG and subtracts nothing (attend_page)
+    const float new_max = fmaxf(c.m, page_max > 0.5f * NEG_BIG ? page_max * scale_log2 : NEG_BIG);
+    const float alpha = __builtin_amdgcn_exp2f(c.m - new_max);
+    const float shift = new_max > 0.5f * NEG_BIG ? -new_max : 0.0f;
+    c.m = new_max;
+#pragma unroll
+    for (int t = 0; t < HD / 16; ++t) c.o[t] *= alpha;
+    u32x4 p[2];
+    float sum = 0.0f;
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+        float e[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            e[r] = __builtin_amdgcn_exp2f(fmaf(s[kt][r], scale_log2, shift));
+            sum += e[r];
+        }
+        p[kt >> 1][(kt & 1) * 2] = pack_bf16_pair(e[0], e[1]);
+        p[kt >> 1][(kt & 1) * 2 + 1] = pack_bf16_pair(e[2], e[3]);
+    }
+    c.l = c.l * alpha + sum;
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t)
+            c.o[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, page.v[kb][t]), __builtin_bit_cast(bf16x8, p[kb]), c.o[t], 0, 0, 0);
+    fw_mfma_drain();        // before control leaves (attend_page)
+    ask_values();
 }
 
 template <int HD>
@@ -869,13 +981,23 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
 
 // ---- decode ------------------------------------------------------------------------------------
 #define MERGE_PARTS 64               // parts of a row up to which the last workgroup keeps their weights in LDS (a context of 16,384 tokens at one run each)
-#define DECODE_WORKGROUPS 512        // two per compute unit: beyond, longer splits serve better than more of them
+// One per compute unit: beyond, longer splits serve better than more of them. Mean over 37 steps (1 to 64 rows, contexts of 600 to 40,000
+// even and ragged, 64 and 128 channels) with the rounds rounded up for 200 / 256 / 384 workgroups: 27.2 / 27.0 / 29.1 us;
+// rounded down for 256 / 512: 28.3 / 30.0 us. (Sharing a row's runs out evenly between its splits gave nothing.)
+#define DECODE_WORKGROUPS 256
 // grid (rows, kv heads * head tiles, splits); four waves, each takes one page of the split's
 // SPLIT_PAGES, and their results are merged in LDS in the order of the keys. Columns are the
 // query heads of the kv group (16 per head tile). partial [rows][heads][max_splits][v_dim + 4]:
 // unnormalised output, then maximum and sum; a split with nothing to do writes nothing and takes
 // no ticket. The last workgroup of a (row, kv head, head tile) to arrive merges what the others
 // left; the only workgroup of a short row writes the result at once.
+// What bounds it is memory: bytes on their way to the compute units, for as long as the walk takes. Up to 128 channels a wave's
+// loads of a page's keys go out as soon as the page before has been scored, those of its values as soon as the values before are used, the
+// page's number one page earlier still, and the first page's while the fused variant forms the queries; each page in turn, with
+// its number looked up in front and nothing on its way during the arithmetic: 64 rows of 725..2,900 keys, 32 heads in 8 groups of 64 channels
+// 84 us, now 62 (4.2 TB/s); 24 rows 38, now 36; 8 rows of 2,048 keys 17.6, now 15.0; 8 rows of 32,768 keys, 16 heads
+// 100, now 98 (5.5 TB/s); groups of 16 heads of 128 channels, 64 rows 75, now 51. Two pages in the registers at a time did not fit (the compiler
+// copies between them and spills); 167 registers leave room for three waves a SIMD.
 // What the fused variant does in front of the attention: the step's raw projections (float32
 // [rows][(heads + kv heads) * head_dim + kv heads * v_dim]: queries, keys, values) get their per-head RMS norm and
 // rotation here, as qk_norm_rope_kv_write does in a kernel of its own (the same arithmetic in the
@@ -954,20 +1076,21 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     const int group = num_heads / num_kv_heads;
     const int head_tiles = (group + 15) / 16;
     const int kvh = blockIdx.y / head_tiles, head_tile = blockIdx.y % head_tiles;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
     const int pos = row_pos[row];
-    const int segment = row_seg[row];       // asked for together with the position, not behind the branch below
+    // asked for together with the position, not behind the branches below
+    const int segment = row_seg[row], step_runs = *(decode_work ? decode_work : row_seg);
     const int first = fw_first_visible(pos, window, chunk);
     // Splits are counted from the first page that holds a visible key; a split is `rounds` runs of
-    // SPLIT_PAGES pages. One run each serves while the step's runs (decode_work: over all its rows;
-    // times the kv heads and head tiles) are no more than about two workgroups per compute unit;
-    // beyond, fewer and longer workgroups read the cache faster, and a row has fewer parts to merge (one
-    // workgroup for a whole row needs no merge at all). Counting the step's work, not the row's, gives
+    // SPLIT_PAGES pages. One run each serves while the step's runs (decode_work: over all its rows, each with no
+    // more than the grid has splits, which is what a window leaves of it; times the kv heads and head tiles) are fewer
+    // than the compute units; beyond, fewer and longer workgroups read the cache faster, and a row has fewer
+    // parts to merge (one workgroup for a whole row needs no merge at all). Counting the step's work, not the row's, gives
     // a long row among short ones its share of the chip.
     int rounds = 1;
     if (decode_work) {
-        const long long workgroups = (long long)decode_work[0] * gridDim.y;
-        rounds = (int)(workgroups / DECODE_WORKGROUPS);
+        const long long most = (long long)gridDim.x * gridDim.z;
+        rounds = (int)(((step_runs < most ? step_runs : most) * gridDim.y + DECODE_WORKGROUPS - 1) / DECODE_WORKGROUPS);
         rounds = rounds < 1 ? 1 : rounds;
     }
     const int pages_per_split = SPLIT_PAGES * rounds;
@@ -984,6 +1107,44 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
 
     Columns<HD> columns_of_wave[1];
     Columns<HD>& c = columns_of_wave[0];
+    // the wave's pages: every SPLIT_PAGES-th step from its first one on; their numbers are asked for ahead
+    const int my_first = first_step + wave;
+    const int my_rounds = my_first > last_step ? 0 : (last_step - my_first) / SPLIT_PAGES + 1 < rounds ? (last_step - my_first) / SPLIT_PAGES + 1 : rounds;
+    auto block_of = [&](int round) {
+        const int step = my_first + round * SPLIT_PAGES;
+        return step < kept_blocks ? step : window_block + step - kept_blocks;
+    };
+    const int32_t* table = block_table + (size_t)segment * table_stride;
+    auto number_of = [&](int round) { return table[block_of(round < my_rounds ? round : my_rounds - 1)]; };
+    // Up to 128 channels the pages stream: STAGES of them are on their way at any time, the first ones while the queries are formed.
+    constexpr bool STREAMED = HD <= 128;
+    constexpr int STAGES = 1;
+    PageOnWay<STREAMED ? HD : 32> pages[STAGES];
+    const PageOffsets<STREAMED ? HD : 32> offsets(head_dim);
+    int next[STAGES];
+    auto keys_at = [&](int page, bool wanted) {
+        return fw_make_buffer(k_pages + ((size_t)page * num_kv_heads + kvh) * PAGE * head_dim, wanted ? (uint32_t)(PAGE * head_dim * 2) : 0u);
+    };
+    auto values_at = [&](int page, bool wanted) {
+        return fw_make_buffer(v_pages + ((size_t)page * num_kv_heads + kvh) * PAGE * v_dim, wanted ? (uint32_t)(PAGE * v_dim * 2) : 0u);
+    };
+    // this row's new key and value are stored below, and their page is asked for behind that
+    const int own_round = FUSED && fused.write_kv && my_rounds > 0 && my_first + (my_rounds - 1) * SPLIT_PAGES == last_step ? my_rounds - 1 : -1;
+    int first_page[STAGES];
+    if (STREAMED && my_rounds > 0) {
+#pragma unroll
+        for (int i = 0; i < STAGES; ++i) {
+            first_page[i] = number_of(i);
+            next[i] = number_of(STAGES + i);
+        }
+#pragma unroll
+        for (int i = 0; i < STAGES; ++i) {
+            first_page[i] = __builtin_amdgcn_readfirstlane(first_page[i]);
+            const bool wanted = i < my_rounds && i != own_round;
+            ask_for_keys(pages[i], offsets, keys_at(first_page[i], wanted));
+            ask_for_values(pages[i], offsets, values_at(first_page[i], wanted));
+        }
+    }
     if (FUSED) {
         const float* projections = fused.qkv + (size_t)row * fused.width;
         const int half = fused.rotary_dim / 2;
@@ -1023,16 +1184,45 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     }
     // this lane's column is a head: its slope of a bias by distance, in the units of the raw scores
     float dist[1] = {slopes ? slopes[head] * 1.4426950408889634f / scale_log2 : 0.0f};
-    for (int round = 0; round < rounds; ++round) {
-        const int step = first_step + round * SPLIT_PAGES + wave;
-        if (step > last_step) break;
-        const int block = step < kept_blocks ? step : window_block + step - kept_blocks;
-        const int page = block_table[(size_t)segment * table_stride + block];
-        const size_t at = ((size_t)page * num_kv_heads + kvh) * PAGE;
-        const int base = block * PAGE;
-        // a lane without a head computes along (q = 0, nothing of it is stored)
-        attend_page<HD, 1, true, false, (HD <= 128)>(columns_of_wave, k_pages + at * head_dim, v_pages + at * v_dim, head_dim, v_dim, scale_log2, first - base, pos - base, pos - base,
-                        head_dim, PAGE, cap, cap_scale, keep_first - base, slopes ? dist : nullptr);
+    if constexpr (STREAMED) {
+#pragma unroll
+        for (int i = 0; i < STAGES; ++i)
+            if (own_round == i) {
+                ask_for_keys(pages[i], offsets, keys_at(first_page[i], true));
+                ask_for_values(pages[i], offsets, values_at(first_page[i], true));
+                // waited for here: a wait in the loop that also allowed for this branch would hold up every round
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                    for (int dc = 0; dc < HD / 32; ++dc) asm volatile("" : "+v"(pages[i].k[kt][dc]));
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int t = 0; t < HD / 16; ++t) asm volatile("" : "+v"(pages[i].v[kb][t]));
+            }
+        for (int round = 0; round < my_rounds; round += STAGES) {
+#pragma unroll
+            for (int i = 0; i < STAGES; ++i) {
+                if (round + i >= my_rounds) break;
+                const int base = block_of(round + i) * PAGE;
+                const bool wanted = round + i + STAGES < my_rounds;
+                const int page = __builtin_amdgcn_readfirstlane(next[i]);
+                // a lane without a head computes along (q = 0, nothing of it is stored)
+                attend_on_way<HD>(c, pages[i], scale_log2, first - base, pos - base, cap, cap_scale, keep_first - base, slopes != nullptr, dist[0],
+                                  [&] {
+                                      next[i] = number_of(round + i + 2 * STAGES);
+                                      ask_for_keys(pages[i], offsets, keys_at(page, wanted));
+                                  },
+                                  [&] { ask_for_values(pages[i], offsets, values_at(page, wanted)); });
+            }
+        }
+    } else {
+        for (int round = 0; round < my_rounds; ++round) {
+            const int block = block_of(round), base = block * PAGE;
+            const size_t at = ((size_t)number_of(round) * num_kv_heads + kvh) * PAGE;
+            attend_page<HD, 1, true, false>(columns_of_wave, k_pages + at * head_dim, v_pages + at * v_dim, head_dim, v_dim, scale_log2, first - base, pos - base, pos - base,
+                                            head_dim, PAGE, cap, cap_scale, keep_first - base, slopes ? dist : nullptr);
+        }
     }
     const float l = fw_quad_sum(c.l);
 #pragma unroll
@@ -1398,7 +1588,7 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
 // max_splits must cover the keys such a row sees, in runs of 4 pages. decode_work: null, or one
 // int32 on the device: the runs of 4 pages that all the rows of the step see together (the sum over
 // the rows of ceil((position + 1) / 256)); with it a workgroup takes as many runs as bring the step
-// down to about 512 workgroups (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
+// down to about 256 workgroups (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
 // ceil(group / 16) int32 counters, zero before the first call and left zero; calls that overlap on
 // one device need their own (and their own workspace).
 extern "C" int fw_attention_decode(const void* q, void* out, float* partial, int max_splits, int max_context,

@@ -820,6 +820,63 @@ def test_attention_decode_on_the_matrix_cores(ops, nh, nkv, hd, window):
         ops._check(status)
 
 
+@pytest.mark.parametrize("nh,nkv,hd,v_dim,window,chunk,keep_first,softcap,sink,slope", [
+    (16, 8, 64, 64, 0, 0, 0, 0.0, False, False), (8, 8, 64, 32, 700, 0, 70, 0.0, True, False), (8, 8, 48, 64, 0, 600, 0, 7.0, False, False),
+    (16, 8, 128, 128, 0, 0, 0, 0.0, False, True), (8, 8, 80, 112, 900, 0, 0, 5.0, True, False), (8, 8, 16, 16, 0, 0, 0, 0.0, False, False),
+    (8, 8, 192, 192, 0, 0, 0, 0.0, False, False)])
+def test_attention_decode_streams_runs_of_pages(ops, nh, nkv, hd, v_dim, window, chunk, keep_first, softcap, sink, slope):
+    """Steps long enough that a workgroup walks several runs of pages: every remainder of runs and pages, heads narrower
+    than their template, and what a page asked for ahead must not bring in (pages past a row's last one, an earlier owner's
+    keys and values, which are no numbers here). The fused call stores the last key and value before it reads their page."""
+    lengths = [1, 64, 65, 257, 512, 513, 768, 1025, 1100, 1281, 1472, 1536] * 4
+    rng = np.random.default_rng(7)
+    order = rng.permutation(len(lengths) * 24).astype(np.int32).reshape(len(lengths), 24)
+    used = np.array([[b < (n + 63) // 64 for b in range(24)] for n in lengths])
+    table = torch.tensor(np.where(used, order, 0), device=DEV)
+    k_pages = as_dev(gen(order.size, nkv, 64, hd, seed=1), torch.bfloat16)
+    v_pages = as_dev(gen(order.size, nkv, v_dim, 64, seed=2), torch.bfloat16)
+    for i, n in enumerate(lengths):
+        if n % 64:
+            k_pages[order[i, n // 64], :, n % 64:] = float("nan")
+            v_pages[order[i, n // 64], :, :, n % 64:] = float("nan")
+    k_pages[torch.tensor(order[~used], device=DEV).long()] = float("nan")
+    v_pages[torch.tensor(order[~used], device=DEV).long()] = float("nan")
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    rows, positions = len(lengths), d([n - 1 for n in lengths])
+    sinks = gen(nh, seed=3).float().to(DEV) if sink else None
+    slopes = (gen(nh, seed=4).abs() * 0.01).float().to(DEV) if slope else None
+    qkv = gen(rows, (nh + nkv) * hd + nkv * v_dim, seed=5).float().to(DEV)
+    cos, sin = torch.cos(qkv[:, :8]).contiguous(), torch.sin(qkv[:, :8]).contiguous()
+    work = d([sum((n + 255) // 256 for n in lengths)])      # 168 runs on 8 kv heads: six of them to a workgroup
+    how = dict(window=window, chunk=chunk, keep_first=keep_first, softcap=softcap, sinks=sinks, slopes=slopes, v_dim=v_dim)
+    scale = hd ** -0.5
+    k_fused, v_fused = k_pages.clone(), v_pages.clone()
+    q = ops.qk_norm_rope_kv_write(qkv, nh, nkv, hd, None, None, 1e-5, cos, sin, 16, k_pages, v_pages, table, d(np.arange(rows)), positions, v_dim=v_dim)
+    run = lambda w: ops.attention_decode(q, nh, nkv, hd, k_pages, v_pages, table, d(np.arange(rows)), positions, scale, 1536, decode_work=w, **how)     # noqa: E731
+    out = run(work)
+    fused = ops.attention_decode_fused(qkv, nh, nkv, hd, None, None, 1e-5, cos, sin, 16, k_fused, v_fused, table, d(np.arange(rows)), positions, scale,
+                                       1536, decode_work=work, **how)
+    assert torch.equal(fused, out)
+    assert torch.equal(k_fused.view(torch.int16), k_pages.view(torch.int16)) and torch.equal(v_fused.view(torch.int16), v_pages.view(torch.int16))
+    close(run(None), back(out), torch.bfloat16)             # one run each
+    keys = back(k_pages)[torch.tensor(order).long()].transpose(2, 3).reshape(rows, 1536, nkv, hd)
+    values = back(v_pages)[torch.tensor(order).long()].permute(0, 1, 4, 2, 3).reshape(rows, 1536, nkv, v_dim)
+    qs = back(q).view(rows, nh, hd)
+    for r in range(12):
+        n, group = lengths[r], nh // nkv
+        pos, at = n - 1, torch.arange(n)
+        first = max(0, pos - window + 1) if window else pos // chunk * chunk if chunk else 0
+        want = torch.empty(nh, v_dim, dtype=torch.float64)
+        for h in range(nh):
+            s = keys[r, :n, h // group] @ qs[r, h] * scale
+            s = softcap * torch.tanh(s / softcap) if softcap else s
+            s = s - (float(slopes[h]) * (pos - at) if slope else 0.0)
+            s = s.masked_fill((at < first) & (at >= keep_first), float("-inf"))
+            s = torch.cat((s, torch.tensor([float(sinks[h])], dtype=torch.float64))) if sink else s
+            want[h] = torch.softmax(s, 0)[:n] @ values[r, :n, h // group]
+        close(out[r], want.reshape(-1), torch.bfloat16)
+
+
 def test_matrix_core_attention_finds_one_far_key_and_the_edges_of_a_window(ops):
     """The same single-dominant-key cases as for the generic kernel, for both fast kernels."""
     nh, nkv, hd, T = 8, 2, 64, 700
