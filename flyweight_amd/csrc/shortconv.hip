@@ -8,7 +8,8 @@
 //
 // A batch holds segments of several sequences. The general variant is two launches: the
 // outputs (state is only read), then the state update (one thread per segment and channel
-// reads what it needs, then writes). A batch of single-token segments runs one fused launch.
+// reads what it needs, then writes). A batch of single-token segments runs one fused launch, and so do
+// kernels of up to four taps over 32 rows and more.
 #include "fw_common.h"
 #include "fw_kernels.h"
 
@@ -47,35 +48,46 @@ __global__ void shortconv_rows_kernel(const T* __restrict__ bcx, TO* __restrict_
     store_from_float(out, (size_t)row * hidden + channel, gate * y);
 }
 
-// The same for kernels of up to four taps, eight consecutive rows of a channel per thread: the
+// The same for kernels of up to four taps, and the state with it in one launch. A thread takes up to eight consecutive rows of a channel: the
 // products B * x of the rows and of the three before them are formed once and slide through
 // the taps in registers (a row's product is otherwise read by as many threads as there are taps),
-// and the chain of dependent loads in front (segment of the row, its first row, its slot) is paid
+// and the chain of dependent loads in front (the segment, its rows, its slot) is paid
 // once for eight rows: with a thread per (row, channel) a prompt's 16 thousand workgroups were
 // bound by that chain. The taps are aligned to the end of a window of four: tap j of a kernel of L
 // taps sits at place j + 4 - L; the places in front are skipped. Sums in the order of the taps, as above.
+//
+// Tiles of eight rows are counted from the first row of their segment, so that only a segment's first tile reaches
+// back into the request's state; its threads read what they need of the state and are therefore free to write it as well, from the
+// segment's last rows. (A kernel of its own behind this one, for the few values of a state, took 4.7 us.) Segment s has the tiles from
+// row0 / 8 + s on, which is room for all its rows wherever they begin; the places left over end at once.
 #define CONV_TILE_ROWS 8
 #define CONV_TILE_HISTORY 3
 // C: channels side by side per thread (2: loads and stores of twice the width, where the model's width is
 // even and the input float32: 2,048 rows of 2,048 channels 19.4 -> 16.2 us; with 4, 19.2 us; a channel's
 // arithmetic is the same either way).
 template <typename T, typename TO, int C>
-__global__ __launch_bounds__(256) void shortconv_rows8_kernel(const T* __restrict__ bcx, TO* __restrict__ out,
+__global__ __launch_bounds__(256) void shortconv_tiles_kernel(const T* __restrict__ bcx, TO* __restrict__ out,
                                                               const float* __restrict__ taps, const float* __restrict__ conv_bias,
-                                                              const float* __restrict__ state, const int32_t* __restrict__ row_seg,
-                                                              const int32_t* __restrict__ seg_row0, const int32_t* __restrict__ seg_slot,
-                                                              int rows, int hidden, int kernel_size) {
+                                                              float* state, const int32_t* __restrict__ seg_row0,
+                                                              const int32_t* __restrict__ seg_slot, int segments, int across, int hidden, int kernel_size) {
     constexpr int R = CONV_TILE_ROWS, H = CONV_TILE_HISTORY;
-    const int r0 = blockIdx.y * R;
-    const int channel = (blockIdx.x * blockDim.x + threadIdx.x) * C;
-    if (channel >= hidden) return;
+    const int tile = blockIdx.x / across;
+    // the last segment whose tiles begin at or before this one: 64 segments are compared at a time
+    int seg = 0;
+    for (int left = segments; left > 1;) {
+        const int stride = (left + 63) / 64, at = (threadIdx.x & 63) * stride;
+        const bool reached = at == 0 || (at < left && seg_row0[seg + at] / R + seg + at <= tile);
+        const int last = (__popcll(__ballot(reached)) - 1) * stride;
+        seg += last;
+        left = left - last < stride ? left - last : stride;
+    }
+    seg = __builtin_amdgcn_readfirstlane(seg);
+    const int first = seg_row0[seg], end = seg_row0[seg + 1], slot = seg_slot[seg];
+    const int before = (tile - (first / R + seg)) * R;      // rows of the segment in front of the tile
+    const int r0 = first + before;
+    const int channel = ((blockIdx.x % across) * blockDim.x + threadIdx.x) * C;
+    if (r0 >= end || channel >= hidden) return;
     const int history = kernel_size - 1, unused = H - history;      // places of the window in front of tap 0
-    // every row's segment and place in it, asked for together and first (two dependent loads each)
-    int seg_of[R], offset_of[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) seg_of[i] = row_seg[r0 + i < rows ? r0 + i : rows - 1];
-#pragma unroll
-    for (int i = 0; i < R; ++i) offset_of[i] = r0 + i - seg_row0[seg_of[i]];
     // C values that lie side by side, as one load
     const auto load_run = [&](const T* from, float (&values)[C]) {
         if (C == 2 && sizeof(T) == 4) {
@@ -87,21 +99,23 @@ __global__ __launch_bounds__(256) void shortconv_rows8_kernel(const T* __restric
             for (int c = 0; c < C; ++c) values[c] = load_as_float(from, c);
         }
     };
-    // the products of rows r0 - 3 .. r0 + 7 (0 where that is no row of this step)
-    float product[R + H][C], gate[R][C];
-#pragma unroll
-    for (int p = 0; p < R + H; ++p) {
-        const int row = r0 - H + p;
-        const bool valid = row >= 0 && row < rows;
-        const T* source = bcx + (size_t)(valid ? row : 0) * 3 * hidden;
+    const auto product_of = [&](int row, float (&values)[C]) {
+        const T* source = bcx + (size_t)row * 3 * hidden;
         float b[C], x[C];
         load_run(source + channel, b);
         load_run(source + 2 * (size_t)hidden + channel, x);
 #pragma unroll
-        for (int c = 0; c < C; ++c) product[p][c] = valid ? b[c] * x[c] : 0.0f;
+        for (int c = 0; c < C; ++c) values[c] = b[c] * x[c];
+    };
+    // the products of rows r0 - 3 .. r0 + 7 (of a row beside the segment: those of its first or last one, not used)
+    float product[R + H][C], gate[R][C];
+#pragma unroll
+    for (int p = 0; p < R + H; ++p) {
+        const int row = r0 - H + p;
+        product_of(row < first ? first : row < end ? row : end - 1, product[p]);
     }
 #pragma unroll
-    for (int i = 0; i < R; ++i) load_run(bcx + (size_t)(r0 + i < rows ? r0 + i : rows - 1) * 3 * hidden + hidden + channel, gate[i]);
+    for (int i = 0; i < R; ++i) load_run(bcx + (size_t)(r0 + i < end ? r0 + i : end - 1) * 3 * hidden + hidden + channel, gate[i]);
     float tap[H + 1][C], bias[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
@@ -110,11 +124,39 @@ __global__ __launch_bounds__(256) void shortconv_rows8_kernel(const T* __restric
             tap[place][c] = place >= unused ? taps[(size_t)(channel + c) * kernel_size + (place - unused)] : 0.0f;
         bias[c] = conv_bias ? conv_bias[channel + c] : 0.0f;
     }
+    if (before == 0) {
+        float* own = state + ((size_t)slot * hidden + channel) * history;
+        // the last `history` products of the sequence: the segment's, or what the state keeps of older ones
+        const int count = end - first;
+        float next[H][C];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            if (k >= history) break;
+            const int offset = count - history + k;
+            if (offset >= 0) {
+                product_of(first + offset, next[k]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < C; ++c) next[k][c] = own[c * history + history + offset];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < H; ++p) {
+            if (p < unused) continue;
+#pragma unroll
+            for (int c = 0; c < C; ++c) product[p][c] = own[c * history + p - unused];
+        }
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            if (k >= history) break;
+#pragma unroll
+            for (int c = 0; c < C; ++c) own[c * history + k] = next[k][c];
+        }
+    }
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         const int row = r0 + i;
-        if (row >= rows) break;
-        const int seg = seg_of[i], offset_in_segment = offset_of[i];
+        if (row >= end) break;
         float result[C];
 #pragma unroll
         for (int c = 0; c < C; ++c) {
@@ -122,11 +164,7 @@ __global__ __launch_bounds__(256) void shortconv_rows8_kernel(const T* __restric
 #pragma unroll
             for (int place = 0; place <= H; ++place) {
                 if (place < unused) continue;       // in front of tap 0: not this kernel's (and never multiplied, not even by 0)
-                float value = product[i + place][c];
-                const int offset = offset_in_segment - H + place;       // where in the segment this place lies
-                if (offset < 0)                                         // in front of the segment: the request's state
-                    value = state[((size_t)seg_slot[seg] * hidden + channel + c) * history + history + offset];
-                y = fmaf(tap[place][c], value, y);
+                y = fmaf(tap[place][c], product[i + place][c], y);
             }
             y += bias[c];
             result[c] = gate[i][c] * y;
@@ -194,15 +232,16 @@ static void launch(const void* bcx, void* out, const float* taps, const float* c
         return;
     }
     if (kernel_size <= CONV_TILE_HISTORY + 1 && rows >= 4 * CONV_TILE_ROWS) {
-        if (hidden % 2 == 0 && sizeof(T) == 4)
-            shortconv_rows8_kernel<T, TO, 2><<<dim3(fw_ceil_div(hidden / 2, 256), fw_ceil_div(rows, CONV_TILE_ROWS)), 256, 0, stream>>>(
-                (const T*)bcx, (TO*)out, taps, conv_bias, state, row_seg, seg_row0, seg_slot, rows, hidden, kernel_size);
+        const int side = hidden % 2 == 0 && sizeof(T) == 4 ? 2 : 1, across = fw_ceil_div(hidden / side, 256);
+        const unsigned grid = (unsigned)(rows / CONV_TILE_ROWS + segments) * across;
+        if (side == 2)
+            shortconv_tiles_kernel<T, TO, 2><<<grid, 256, 0, stream>>>((const T*)bcx, (TO*)out, taps, conv_bias, state, seg_row0, seg_slot, segments, across, hidden, kernel_size);
         else
-            shortconv_rows8_kernel<T, TO, 1><<<dim3(bx, fw_ceil_div(rows, CONV_TILE_ROWS)), 256, 0, stream>>>(
-                (const T*)bcx, (TO*)out, taps, conv_bias, state, row_seg, seg_row0, seg_slot, rows, hidden, kernel_size);
-    } else
-        shortconv_rows_kernel<T, TO><<<dim3(bx, rows), 256, 0, stream>>>(
-            (const T*)bcx, (TO*)out, taps, conv_bias, state, row_seg, seg_row0, seg_slot, hidden, kernel_size);
+            shortconv_tiles_kernel<T, TO, 1><<<grid, 256, 0, stream>>>((const T*)bcx, (TO*)out, taps, conv_bias, state, seg_row0, seg_slot, segments, across, hidden, kernel_size);
+        return;
+    }
+    shortconv_rows_kernel<T, TO><<<dim3(bx, rows), 256, 0, stream>>>(
+        (const T*)bcx, (TO*)out, taps, conv_bias, state, row_seg, seg_row0, seg_slot, hidden, kernel_size);
     shortconv_state_kernel<T><<<dim3(bx, segments), 256, 0, stream>>>(
         (const T*)bcx, state, seg_row0, seg_slot, hidden, kernel_size);
 }

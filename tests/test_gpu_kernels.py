@@ -166,6 +166,24 @@ def test_shortconv_mixed_segments(ops, dtype, H, L, with_bias):
     close(dev_state, want_state1, torch.float32, 10.0 if dtype == torch.bfloat16 else 1.0)
 
 
+@pytest.mark.parametrize("dtype,out_dtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("H,L,counts", [
+    (514, 3, [37]), (70, 4, [1] * 6 + [8, 9, 16, 17, 7, 3, 2, 1, 24]), (33, 2, [1, 33]), (258, 3, [31, 1]), (64, 4, [2, 1, 3] * 30 + [20]), (40, 3, [1] * 4200 + [40])])
+def test_shortconv_tiles_of_segments(ops, dtype, out_dtype, H, L, counts):
+    """Tiles of eight rows counted from each segment's start, which also write its state: segments that begin anywhere, are shorter than the
+    kernel or end on a tile's edge, and as many as need one, two and three rounds of the search for a tile's segment."""
+    first = np.concatenate([[0], np.cumsum(counts)])
+    n, rows = len(counts), int(first[-1])
+    slots = np.random.default_rng(n).permutation(n + 1)[:n]
+    bcx, taps, state = as_dev(gen(rows, 3 * H), dtype), gen(H, L, seed=1).float(), gen(n + 1, H, L - 1, seed=3).float()
+    want_out, want_state = conv_reference(back(bcx), taps.double(), None, state.double(), [(int(f), c, int(s)) for f, c, s in zip(first, counts, slots)])
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    dev_state = state.to(DEV)
+    out = ops.shortconv(bcx, taps.to(DEV), None, dev_state, d(np.repeat(np.arange(n), counts)), d(first), d(slots), n, out_dtype=out_dtype)
+    close(out, want_out, out_dtype)
+    close(dev_state, want_state, torch.float32, 10.0 if dtype == torch.bfloat16 else 1.0)
+
+
 def rope_reference(x, cos, sin, rotary):
     half = rotary // 2
     a, b, rest = x[..., :half], x[..., half:rotary], x[..., rotary:]
