@@ -981,11 +981,13 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
 
 // ---- decode ------------------------------------------------------------------------------------
 #define MERGE_PARTS 64               // parts of a row up to which the last workgroup keeps their weights in LDS (a context of 16,384 tokens at one run each)
-// One per compute unit: beyond, longer splits serve better than more of them. Mean over 37 steps (1 to 64 rows, contexts of 600 to 40,000
-// even and ragged, 64 and 128 channels) with the rounds rounded up for 200 / 256 / 384 workgroups: 27.2 / 27.0 / 29.1 us;
-// rounded down for 256 / 512: 28.3 / 30.0 us. (Sharing a row's runs out evenly between its splits gave nothing.)
-#define DECODE_WORKGROUPS 256
-// grid (rows, kv heads * head tiles, splits); four waves, each takes one page of the split's
+// Workgroups a step is cut into at most (rounds rounded up): one per compute unit where every row is as long as the others, so that all end
+// together; where the lengths differ a half more of them fill up behind those of short rows. Mean of 12 steps of even rows (1 to 64 rows, 1,000 to
+// 40,000 keys) with 256 / 320 / 384 / 512 workgroups 24.9 / 27.8 / 27.6 / 26.4 us, of 48 ragged ones (3 to 64 rows of up to
+// 6,000 keys, 4 head shapes of 64 and 128 channels) 41.4 / 40.5 / 39.7 / 40.1.
+#define EVEN_WORKGROUPS 256
+#define RAGGED_WORKGROUPS 384
+// grid (kv heads * head tiles, rows, splits), or the first two changed over beyond 65,535 rows; four waves, each takes one page of the split's
 // SPLIT_PAGES, and their results are merged in LDS in the order of the keys. Columns are the
 // query heads of the kv group (16 per head tile). partial [rows][heads][max_splits][v_dim + 4]:
 // unnormalised output, then maximum and sum; a split with nothing to do writes nothing and takes
@@ -995,8 +997,8 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
 // loads of a page's keys go out as soon as the page before has been scored, those of its values as soon as the values before are used, the
 // page's number one page earlier still, and the first page's while the fused variant forms the queries; each page in turn, with
 // its number looked up in front and nothing on its way during the arithmetic: 64 rows of 725..2,900 keys, 32 heads in 8 groups of 64 channels
-// 84 us, now 62 (4.2 TB/s); 24 rows 38, now 36; 8 rows of 2,048 keys 17.6, now 15.0; 8 rows of 32,768 keys, 16 heads
-// 100, now 98 (5.5 TB/s); groups of 16 heads of 128 channels, 64 rows 75, now 51. Two pages in the registers at a time did not fit (the compiler
+// 84 us, now 56 (4.6 TB/s); 24 rows 38, now 36; 8 rows of 2,048 keys 17.6, now 15.0; 8 rows of 32,768 keys, 16 heads
+// 100, now 98 (5.5 TB/s); groups of 16 heads of 128 channels, 64 rows 75, now 47. Two pages in the registers at a time did not fit (the compiler
 // copies between them and spills); 167 registers leave room for three waves a SIMD.
 // What the fused variant does in front of the attention: the step's raw projections (float32
 // [rows][(heads + kv heads) * head_dim + kv heads * v_dim]: queries, keys, values) get their per-head RMS norm and
@@ -1065,40 +1067,43 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     const int32_t* __restrict__ row_seg, const int32_t* __restrict__ row_pos, int num_heads, int num_kv_heads,
     int head_dim, int v_dim, float scale_log2, int window, int chunk, float cap, float cap_scale, int max_splits,
     const int32_t* __restrict__ decode_work, const FusedProjections fused, int keep_first, const float* __restrict__ sinks,
-    const float* __restrict__ slopes) {
+    const float* __restrict__ slopes, bool heads_first) {
     __shared__ f32x4 shared_o[SPLIT_PAGES][HD / 16][64];
     __shared__ float shared_m[SPLIT_PAGES][16], shared_l[SPLIT_PAGES][16];
     __shared__ int ticket_shared;
     __shared__ float merge_w[MERGE_PARTS][16], merge_l[MERGE_PARTS][16];
     __shared__ __attribute__((aligned(16))) uint16_t fused_q[FUSED ? 16 : 1][FUSED ? HD : 8];
     __shared__ float fused_scratch[FUSED ? SPLIT_PAGES : 1][FUSED ? HD : 1];
-    const int row = blockIdx.x, split = blockIdx.z;
+    const int row = heads_first ? blockIdx.y : blockIdx.x, across = heads_first ? blockIdx.x : blockIdx.y, split = blockIdx.z;
+    const int rows = heads_first ? gridDim.y : gridDim.x, acrosses = heads_first ? gridDim.x : gridDim.y;
     const int group = num_heads / num_kv_heads;
     const int head_tiles = (group + 15) / 16;
-    const int kvh = blockIdx.y / head_tiles, head_tile = blockIdx.y % head_tiles;
+    const int kvh = across / head_tiles, head_tile = across % head_tiles;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
     const int pos = row_pos[row];
     // asked for together with the position, not behind the branches below
     const int segment = row_seg[row], step_runs = *(decode_work ? decode_work : row_seg);
     const int first = fw_first_visible(pos, window, chunk);
-    // Splits are counted from the first page that holds a visible key; a split is `rounds` runs of
-    // SPLIT_PAGES pages. One run each serves while the step's runs (decode_work: over all its rows, each with no
-    // more than the grid has splits, which is what a window leaves of it; times the kv heads and head tiles) are fewer
-    // than the compute units; beyond, fewer and longer workgroups read the cache faster, and a row has fewer
-    // parts to merge (one workgroup for a whole row needs no merge at all). Counting the step's work, not the row's, gives
-    // a long row among short ones its share of the chip.
-    int rounds = 1;
-    if (decode_work) {
-        const long long most = (long long)gridDim.x * gridDim.z;
-        rounds = (int)(((step_runs < most ? step_runs : most) * gridDim.y + DECODE_WORKGROUPS - 1) / DECODE_WORKGROUPS);
-        rounds = rounds < 1 ? 1 : rounds;
-    }
-    const int pages_per_split = SPLIT_PAGES * rounds;
     // The pages a row walks: those of the kept first keys that lie before the window's first page, then the
     // window's. They are numbered through (`step`), and the splits are counted over the steps.
     const int window_block = first / PAGE, last_block = pos / PAGE;
     const int kept_blocks = (keep_first + PAGE - 1) / PAGE < window_block ? (keep_first + PAGE - 1) / PAGE : window_block;
     const int last_step = kept_blocks + last_block - window_block;
+    // Splits are counted from the first page that holds a visible key; a split is `rounds` runs of
+    // SPLIT_PAGES pages. One run each serves while the step's runs (decode_work: over all its rows, each with no
+    // more than the grid has splits, which is what a window leaves of it; times the kv heads and head tiles) are fewer
+    // than the workgroups wanted; beyond, fewer and longer workgroups read the cache faster, and a row has fewer
+    // parts to merge (one workgroup for a whole row needs no merge at all). Counting the step's work, not the row's, gives
+    // a long row among short ones its share of the chip.
+    int rounds = 1;
+    if (decode_work) {
+        const long long most = (long long)rows * gridDim.z, runs = step_runs < most ? step_runs : most;
+        const long long beside = (long long)(last_step / SPLIT_PAGES + 1) * rows - runs;    // 0: every row is as long as this one
+        const int wanted = beside >= -rows && beside <= rows ? EVEN_WORKGROUPS : RAGGED_WORKGROUPS;
+        rounds = (int)((runs * acrosses + wanted - 1) / wanted);
+        rounds = rounds < 1 ? 1 : rounds;
+    }
+    const int pages_per_split = SPLIT_PAGES * rounds;
     const int first_step = split * pages_per_split;
     if (first_step > last_step) return;         // the whole workgroup
     const int in_group = head_tile * 16 + col;
@@ -1282,7 +1287,7 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     // takes the ticket. Nobody waits for another workgroup. The ticket counter is left at zero.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    int* ticket = tickets + (size_t)row * gridDim.y + blockIdx.y;
+    int* ticket = tickets + (size_t)row * acrosses + across;
     if (threadIdx.x == 0) ticket_shared = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (ticket_shared != row_splits - 1) return;
@@ -1566,17 +1571,21 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
     if (rows == 0) return 0;
     const ScoreRule rule = score_rule(scale, softcap);
     const int head_tiles = (num_heads / num_kv_heads + 15) / 16;
-    dim3 grid(rows, num_kv_heads * head_tiles, max_splits);
+    // Workgroups go to the eight dies in turn: the heads of a row first, so that a long row is spread over the dies (rows first, a
+    // step of 8 n rows puts all of a row on one die: 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 59.9 us, now 56.1; in 16 groups 117, now 107).
+    const bool heads_first = rows <= 65535;
+    const int across = num_kv_heads * head_tiles;
+    const dim3 grid(heads_first ? across : rows, heads_first ? rows : across, max_splits);
 
 #define CALL(HD)                                                                                                              \
     if (fused.qkv)                                                                                                            \
         attention_decode_split_kernel<HD, true><<<grid, 64 * SPLIT_PAGES, 0, (hipStream_t)stream>>>(                          \
             (const uint16_t*)q, (uint16_t*)out, partial, tickets, (uint16_t*)k_pages, (uint16_t*)v_pages, block_table,        \
-            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes); \
+            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first); \
     else                                                                                                                      \
         attention_decode_split_kernel<HD, false><<<grid, 64 * SPLIT_PAGES, 0, (hipStream_t)stream>>>(                         \
             (const uint16_t*)q, (uint16_t*)out, partial, tickets, (uint16_t*)k_pages, (uint16_t*)v_pages, block_table,        \
-            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes)
+            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first)
     FW_BY_HEAD_DIM((head_dim > v_dim ? head_dim : v_dim), CALL);
 #undef CALL
     FW_LAUNCH_CHECK("attention_decode");
@@ -1588,7 +1597,7 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
 // max_splits must cover the keys such a row sees, in runs of 4 pages. decode_work: null, or one
 // int32 on the device: the runs of 4 pages that all the rows of the step see together (the sum over
 // the rows of ceil((position + 1) / 256)); with it a workgroup takes as many runs as bring the step
-// down to about 256 workgroups (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
+// down to 256 to 384 workgroups (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
 // ceil(group / 16) int32 counters, zero before the first call and left zero; calls that overlap on
 // one device need their own (and their own workspace).
 extern "C" int fw_attention_decode(const void* q, void* out, float* partial, int max_splits, int max_context,
