@@ -87,10 +87,13 @@ class QueryTileArrays:
 class GQAttention(QueryTileArrays, Mixer):
     graph_safe = True
     accepts_lazy_norm = True
-    # Up to this many rows a decode step forms queries and keys inside the attention kernel (at 8 rows
-    # 18.9 us against 15.4 + 4.9 us in two kernels); with many rows the attention is bound by reading
-    # the cache and the work in front of it only delays every workgroup (64 rows: 74.1 against 65.9 + 7.2 us).
+    # Up to this many rows a decode step forms queries and keys inside the attention kernel, while its first pages are on
+    # their way: 17 / 32 / 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 22.6 / 38.8 / 63.6 us against 25.3 / 40.6 / 69.0 in two
+    # kernels, of 300 keys 11.4 / 10.9 / 14.1 against 12.9 / 12.7 / 19.4; with 128 channels 15.3 / 15.6 / 21.6 against 17.5 / 17.4 /
+    # 22.9 (128 rows of 3,000 keys 231 against 221). Every workgroup of a group forms all its queries: groups of 16 heads of 128 channels
+    # take 19.4 us at 17 rows of 300 keys against 17.4, so that groups of more than four stay with 16 rows.
     FUSED_DECODE_ROWS = 16
+    FUSED_DECODE_ROWS_OF_FEW_HEADS = 64
 
     def __init__(self, spec):
         super().__init__(spec)
@@ -270,7 +273,9 @@ class GQAttention(QueryTileArrays, Mixer):
         if self.shared_kv and cache.writes:
             raise ConfigError(f"{self.prefix}: the layer has no keys and values of its own; its schedule entry must read another's cache entry")
         mask = {"keep_first": self.keep_first if self.window else 0, "sinks": self.sinks, "slopes": self.slopes}
-        if ctx.all_decode and ctx.num_rows <= self.FUSED_DECODE_ROWS and qkv.dtype == torch.float32 and self.step_arrays_key() is not None:
+        few_heads = self.num_heads <= 4 * self.num_kv_heads
+        fused_rows = self.FUSED_DECODE_ROWS_OF_FEW_HEADS if few_heads else self.FUSED_DECODE_ROWS
+        if ctx.all_decode and ctx.num_rows <= fused_rows and qkv.dtype == torch.float32 and self.step_arrays_key() is not None:
             # a few single-token segments on the matrix cores: norm, rotation, cache write and attention in one kernel
             return ops.attention_decode_fused(
                 qkv, self.num_heads, self.num_kv_heads, self.head_dim, self.q_norm_weight, self.k_norm_weight, self.qk_norm_eps,
