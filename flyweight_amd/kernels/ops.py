@@ -626,7 +626,7 @@ def _big_split_needs(mode: int, M: int, N: int, K: int):
 
 # What the tiled products take, us: start + rounds * round + tiles / 256 * tile + K / 1,024 * (rounds * walk + tiles / 256 * fill), rounds those of
 # their tiles over the 256 compute units (a round that is little full is a little faster). By mode: storing, adding, gated. Fitted to 2,200
-# shapes of 65 to 16,384 rows by 32 to 16,384 features over K 32 to 12,288, the weights from memory, to 4 to 12 % (mean square), with no part
+# shapes (the large tiles: 852, when their loop changed) of 65 to 16,384 rows by 32 to 16,384 features over K 32 to 12,288, the weights from memory, to 4 to 12 % (mean square), with no part
 # below zero: parts that were, fitted to shapes of few rounds, made many rounds over a short K free.
 _TIME_DEEP = {0: {128: (3.2, 9.1, 1.4, 4.76, 3.28), 64: (2.6, 3.9, 1.2, 3.56, 1.54)},
               1: {128: (2.7, 10.4, 1.9, 4.84, 2.64), 64: (2.4, 4.5, 1.3, 3.62, 1.26)}}
@@ -660,11 +660,9 @@ def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: 
 def tiled_plan(mode: int, M: int, N: int, K: int):
     """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
     256 columns), "bigsplit" (128 rows by 256, K cut over workgroups), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through
-    registers), "split" (those with K cut over workgroups). The least estimated time decides: on 780 shapes 0.1 to 0.7 % above the fastest
-    alone in the geometric mean. Fixed numbers of tiles were 10 % above it (storing, 1,111 rows by 2,048 features over K 8,192 97 us
-    against 57, 640 by 2,048 over 2,048 22 against 14, 1,300 by 3,072 over 2,048 44 against 28; gated, 1,111 by 4,608 over 2,048 63 against 46), adding
-    products of up to 2,048 features held to the tiles whose waves split K 5 % (6,200 by 2,048 over 7,168 269 against 163, 2,690 by 1,536 over 1,024 32
-    against 18; they keep what is one round over a long K: 2,048 by 2,048 over 4,096 41 against 48)."""
+    registers), "split" (those with K cut over workgroups). The least estimated time decides. Fixed numbers of
+    tiles were 10 % above the fastest in the geometric mean, adding products of up to 2,048 features held to the tiles whose waves split K 5 %; K cut
+    over workgroups takes 1,111 rows by 2,048 features over K 8,192 in 50 us against 60 on the tiles whose waves split K."""
     lib = library()
     wide, narrow = -(-M // 128) * -(-N // 128), -(-M // 128) * -(-N // 64)
     columns = 64 if mode == 2 or wide < DEEP_ROUND or (wide == DEEP_ROUND and K < LONG_K) else 128        # as fw_gemm_mfma chooses
