@@ -97,9 +97,10 @@ class Linear:
         return {"squares": a.prepared.squares, "eps": a.rms_parameters()[1]}
 
     def _normed(self, a: Input, features: int, gated: bool) -> bool:
-        """Few float32 rows whose norm has not run yet: their product takes it in front."""
-        return (isinstance(a, LazyNorm) and a.dtype == torch.float32 and self.weight.dtype == torch.float32 and a.pending
-                and ops.float32_normed_takes(gated, a.rows, features, self.in_features))
+        """Few float32 rows whose norm has not run yet: their product takes it in front (operands that do not start at 16 bytes pass the
+        norm and the plain product)."""
+        return (isinstance(a, LazyNorm) and a.dtype == torch.float32 and self.weight.dtype == torch.float32 and self.weight.data_ptr() % 16 == 0
+                and a.pending and ops.float32_normed_takes(gated, a.rows, features, self.in_features))
 
     # ----- products -----------------------------------------------------------------------
     def forward(self, a: Input, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:

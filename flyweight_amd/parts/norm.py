@@ -69,9 +69,12 @@ class LazyNorm:
 
     @property
     def pending(self) -> bool:
-        """Whether the norm is a plain RMS norm over float32 rows that has not run yet, nor any part of it."""
-        return self._tensor is None and self.prepared is None and self.x.dtype == torch.float32 and self.x.is_contiguous() \
-            and self.x.data_ptr() % 16 == 0 and self.rms_parameters() is not None
+        """Whether the norm is a plain RMS norm over float32 rows that has not run yet, nor any part of it, and rows and weight can be read 16
+        bytes at a time."""
+        if self._tensor is not None or self.prepared is not None or self.x.dtype != torch.float32 or self.x.dim() != 2 or not self.x.is_contiguous():
+            return False
+        rms = self.rms_parameters()
+        return rms is not None and self.x.data_ptr() % 16 == 0 and rms[0].data_ptr() % 16 == 0
 
     def rms_parameters(self):
         """(weight, eps, one_centered) if the norm is a plain RMS norm, else None."""

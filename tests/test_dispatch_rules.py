@@ -153,3 +153,31 @@ def test_products_beyond_64_rows_are_dealt_to_waves_where_that_is_faster(mode, M
 def test_tiled_products_take_the_tiles_that_were_the_fastest(mode, M, N, K, plan):
     from flyweight_amd.kernels import ops
     assert ops.tiled_plan(mode, M, N, K) == plan
+
+
+def _at_an_odd_place(t):
+    """The same values from an address that is no multiple of 16 bytes."""
+    held = torch.empty(t.numel() + 4, dtype=t.dtype)
+    first = next(i for i in range(4) if (held.data_ptr() + i * t.element_size()) % 16)
+    odd = held[first:first + t.numel()].view(t.shape)
+    return odd.copy_(t)
+
+
+def _even(*shape):
+    t = torch.randn(*shape)
+    return t if t.data_ptr() % 16 == 0 else pytest.skip("the host's tensors do not start at 16 bytes")
+
+
+@pytest.mark.parametrize("odd", ["none", "rows", "weight", "norm"])
+def test_few_float32_rows_take_their_norm_in_front_only_where_every_operand_starts_at_16_bytes(odd):
+    """The kernel that takes the norm reads x, W and the norm's weight 16 bytes at a time; anything else goes through the norm and the product apart."""
+    from flyweight_amd.config.spec import PartSpec
+    from flyweight_amd.parts.linear import Linear
+    from flyweight_amd.parts.norm import LazyNorm, RMSNorm
+    x, w, weight = (_at_an_odd_place(t) if odd == name else t for name, t in (("rows", _even(1, 1024)), ("weight", _even(64, 1024)), ("norm", _even(1024))))
+    norm = RMSNorm(PartSpec("rmsnorm", {"size": 1024, "eps": 1e-5}))
+    norm.bind({norm.tensor_name: weight}, torch.float32, torch.device("cpu"))
+    linear = Linear(w)
+    for gated, features in ((False, 64), (True, 32)):
+        assert linear._normed(LazyNorm(norm, x, None), features, gated) == (odd == "none")
+    assert not linear._normed(LazyNorm(norm, x.view(1, 1, 1024), None), 64, False)       # (rows of another shape, which the norm by itself takes)

@@ -132,6 +132,35 @@ def test_what_a_normed_product_of_few_rows_refuses(ops):
         ops.gemm_float32_normed(a, weight[:1000].contiguous(), 1e-5, False, w)
 
 
+@pytest.mark.parametrize("odd", ["rows", "weight", "norm"])
+def test_one_normed_row_of_operands_at_odd_places(ops, odd):
+    """A linear part whose weight, norm or row does not start at 16 bytes: norm and product apart, as with more rows."""
+    from flyweight_amd.config.spec import PartSpec
+    from flyweight_amd.parts.linear import Linear
+    from flyweight_amd.parts.norm import LazyNorm, RMSNorm
+
+    def placed(name, t):
+        held = torch.zeros(t.numel() + 1, device=DEV)
+        held[1:] = t.to(DEV).reshape(-1)
+        return held[1:].view(t.shape) if name == odd else t.to(DEV)
+
+    x, w, weight, bias = draw(1, 1024), draw(64, 1024, seed=1), 1.0 + 0.1 * draw(1024, seed=2), draw(64, seed=3)
+    norm = RMSNorm(PartSpec("rmsnorm", {"size": 1024, "eps": 1e-5}))
+    norm.bind({norm.tensor_name: placed("norm", weight)}, torch.float32, torch.device(DEV))
+    X, W = placed("rows", x), placed("weight", w)
+    normed = x.double() * torch.rsqrt(x.double().pow(2).mean() + 1e-5) * weight.double()
+    # the row's mean of squares, root and two products are a few roundings each beside those of the product
+    limit = bound(normed, w) + 8 * 2.0 ** -24 * (normed.abs() @ w.double().abs().T)
+    sums = normed @ w.double().T
+    stored = Linear(W, bias.to(DEV)).forward(LazyNorm(norm, X, None), out_dtype=torch.float32).cpu().double()
+    assert ((stored - sums - bias.double()).abs() <= limit + 2.0 ** -23 * stored.abs()).all()
+    gated = Linear(W).swiglu(LazyNorm(norm, X, None)).cpu().double()
+    g, u = sums[:, :32], sums[:, 32:]
+    exact = torch.nn.functional.silu(g) * u
+    allowed = 1.1 * limit[:, :32] * u.abs() + limit[:, 32:] * g.abs() + 2.0 ** -20 * exact.abs() + 1e-12     # (as the gated product above)
+    assert ((gated - exact).abs() <= allowed).all()
+
+
 @pytest.mark.parametrize("nh,nkv,hd,v_dim,window,keep_first,sink,slope,softcap,chunk", [
     (4, 2, 64, 64, 0, 0, False, False, 0.0, 0), (6, 2, 64, 48, 70, 0, False, False, 0.0, 0), (4, 1, 128, 128, 100, 70, True, False, 0.0, 0),
     (2, 2, 20, 320, 0, 0, False, True, 0.0, 0), (4, 2, 320, 64, 0, 0, False, False, 6.0, 0), (4, 2, 64, 1024, 0, 0, True, False, 0.0, 130)])
