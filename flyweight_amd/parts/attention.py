@@ -92,8 +92,13 @@ class GQAttention(QueryTileArrays, Mixer):
     # kernels, of 300 keys 11.4 / 10.9 / 14.1 against 12.9 / 12.7 / 19.4; with 128 channels 15.3 / 15.6 / 21.6 against 17.5 / 17.4 /
     # 22.9 (128 rows of 3,000 keys 231 against 221). Every workgroup of a group forms all its queries: groups of 16 heads of 128 channels
     # take 19.4 us at 17 rows of 300 keys against 17.4, so that groups of more than four stay with 16 rows.
+    # Heads beyond 128 channels have no page on its way meanwhile (the registers would not hold it). They gain up to 32 rows, by the kernel
+    # that is saved, and lose beyond, where many workgroups wait for the queries: 16 heads in 4 groups of 192 channels, 24 / 32 rows of 2,900 keys 65.0 /
+    # 73.4 against 68.2 / 77.9, 48 / 64 rows 118.4 / 134.5 against 111.3 / 133.9; of 256 channels, 32 rows 88 against 94, 48 rows of 300 / 1,000 / 2,900 keys
+    # 31.7 / 74.1 / 141.9 against 30.8 / 70.1 / 135.0; 8 heads in 8 groups of 144 channels, 32 rows of 300 keys 23.3 against 24.9, 64 rows 46.4 against 45.8.
     FUSED_DECODE_ROWS = 16
     FUSED_DECODE_ROWS_OF_FEW_HEADS = 64
+    FUSED_DECODE_ROWS_OF_WIDE_HEADS = 32
 
     def __init__(self, spec):
         super().__init__(spec)
@@ -273,8 +278,9 @@ class GQAttention(QueryTileArrays, Mixer):
         if self.shared_kv and cache.writes:
             raise ConfigError(f"{self.prefix}: the layer has no keys and values of its own; its schedule entry must read another's cache entry")
         mask = {"keep_first": self.keep_first if self.window else 0, "sinks": self.sinks, "slopes": self.slopes}
-        few_heads = self.num_heads <= 4 * self.num_kv_heads
-        fused_rows = self.FUSED_DECODE_ROWS_OF_FEW_HEADS if few_heads else self.FUSED_DECODE_ROWS
+        fused_rows = self.FUSED_DECODE_ROWS
+        if self.num_heads <= 4 * self.num_kv_heads:
+            fused_rows = self.FUSED_DECODE_ROWS_OF_FEW_HEADS if max(self.head_dim, self.v_head_dim) <= 128 else self.FUSED_DECODE_ROWS_OF_WIDE_HEADS
         if ctx.all_decode and ctx.num_rows <= fused_rows and qkv.dtype == torch.float32 and self.step_arrays_key() is not None:
             # a few single-token segments on the matrix cores: norm, rotation, cache write and attention in one kernel
             return ops.attention_decode_fused(

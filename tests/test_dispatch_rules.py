@@ -181,3 +181,27 @@ def test_few_float32_rows_take_their_norm_in_front_only_where_every_operand_star
     for gated, features in ((False, 64), (True, 32)):
         assert linear._normed(LazyNorm(norm, x, None), features, gated) == (odd == "none")
     assert not linear._normed(LazyNorm(norm, x.view(1, 1, 1024), None), 64, False)       # (rows of another shape, which the norm by itself takes)
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,v_dim,rows,fused", [
+    (32, 8, 64, 64, 64, True), (32, 8, 64, 64, 65, False), (16, 4, 128, 128, 64, True), (16, 16, 80, 112, 64, True), (16, 4, 144, 144, 32, True),
+    (16, 4, 144, 144, 33, False), (8, 8, 256, 256, 32, True), (8, 8, 256, 256, 48, False), (8, 4, 64, 192, 33, False), (8, 4, 192, 64, 33, False),
+    (16, 1, 128, 128, 16, True), (16, 1, 128, 128, 17, False), (16, 1, 256, 256, 16, True), (16, 1, 256, 256, 17, False)])
+def test_decode_steps_form_queries_inside_the_attention_kernel_where_that_is_faster(monkeypatch, heads, kv_heads, dim, v_dim, rows, fused):
+    from types import SimpleNamespace
+    from flyweight_amd.config.spec import PartSpec
+    from flyweight_amd.kernels import ops
+    from flyweight_amd.parts.attention import GQAttention
+    took = []
+    monkeypatch.setattr(ops, "attention_decode_fused", lambda *a, **k: took.append(True))
+    monkeypatch.setattr(ops, "qk_norm_rope_kv_write", lambda *a, **k: None)
+    monkeypatch.setattr(ops, "attention", lambda *a, **k: took.append(False))
+    part = GQAttention(PartSpec("gqa_attention", {
+        "hidden_size": 64, "num_heads": heads, "num_kv_heads": kv_heads, "head_dim": dim, "v_head_dim": v_dim,
+        "position": PartSpec("rotary_neox", {"head_dim": dim, "theta": 1e4})}))
+    part.dtype, part.sinks, part.slopes, part.conv, part.q_norm_weight, part.k_norm_weight = torch.bfloat16, None, None, None, None, None
+    part.qkv = SimpleNamespace(forward=lambda h, out_dtype: torch.empty(0, dtype=out_dtype))
+    ctx = SimpleNamespace(all_decode=True, num_rows=rows, max_context=64, row_seg=None, row_pos=None,
+                          position_tables=lambda p: (None, None), step_arrays=lambda p: {})
+    part.attend(None, ctx, SimpleNamespace(writes=True, k_pages=None, v_pages=None, block_table=None))
+    assert took == [fused]
