@@ -981,12 +981,36 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
 
 // ---- decode ------------------------------------------------------------------------------------
 #define MERGE_PARTS 64               // parts of a row up to which the last workgroup keeps their weights in LDS (a context of 16,384 tokens at one run each)
-// Workgroups a step is cut into at most (rounds rounded up): one per compute unit where every row is as long as the others, so that all end
-// together; where the lengths differ a half more of them fill up behind those of short rows. Mean of 12 steps of even rows (1 to 64 rows, 1,000 to
-// 40,000 keys) with 256 / 320 / 384 / 512 workgroups 24.9 / 27.8 / 27.6 / 26.4 us, of 48 ragged ones (3 to 64 rows of up to
-// 6,000 keys, 4 head shapes of 64 and 128 channels) 41.4 / 40.5 / 39.7 / 40.1.
+// How a step is cut into workgroups. Where the rows are equally long, into whole splits of every row that fill the compute units once, each with a workgroup
+// of its own, so that all end together; where that leaves more than three tenths of them idle and the rows have LONG_RUNS runs, twice or three
+// times. Counted are the places of the grid, those of rows that fill a recorded step up among them: a workgroup that ends at once has still moved
+// the next one on by a compute unit. us of the best of 1 to 24 splits / this rule / as many splits as bring all the rows' runs below 256, mean of 560
+// steps (1 to 96 rows, a third of them filled up, 300 to 6,000 keys; 1 to 8 kv heads of 64 and 128 channels) 1 / 1.021 / 1.057: 20 rows filled up to 24 behind
+// 2,900 keys, 32 heads in 8 groups of 64 channels 28.0 / 28.0 / 33.3, 2 groups of 16 heads of 128 channels 24.6 / 24.6 / 32.0; 24 rows, 4 groups of 128
+// channels 37.6 / 37.6 / 47.0; 40 rows, the same, 1,000 keys (1 and 2 splits) 24.3 and 30.9, 2,900 (1, 2 and 3) 58.3, 65.4 and 51.7.
+// Where the lengths differ, RAGGED_WORKGROUPS at most (rounds rounded up): a half more than compute units fill up behind those of short rows. Mean of 48
+// ragged steps (3 to 64 rows of up to 6,000 keys, 4 head shapes of 64 and 128 channels) with 256 / 320 / 384 / 512 workgroups 41.4 / 40.5 / 39.7 / 40.1 us.
 #define EVEN_WORKGROUPS 256
 #define RAGGED_WORKGROUPS 384
+#define LONG_RUNS 8
+struct EvenSplits {
+    int plain, many;        // of a row; from LONG_RUNS runs on
+    int runs;               // that a window leaves of a row, most of the time (a row whose window ends inside a page sees a page more)
+};
+static EvenSplits even_splits(int rows, int across, int max_splits, int span, int keep_first) {
+    const int places = rows > 3 * EVEN_WORKGROUPS ? rows : rows * across;       // of one split
+    EvenSplits even = {places < EVEN_WORKGROUPS ? EVEN_WORKGROUPS / places : 1, 0, max_splits};
+    for (int times = 1; times <= 3 && even.many == 0; ++times) {
+        const int splits = times * EVEN_WORKGROUPS / places;
+        if (10 * splits * places >= 7 * times * EVEN_WORKGROUPS) even.many = splits;
+    }
+    if (even.many == 0) even.many = places < 3 * EVEN_WORKGROUPS ? 3 * EVEN_WORKGROUPS / places : 1;
+    if (span > 0) {
+        const int pages = (span - 1) / PAGE + 1 + (keep_first + PAGE - 1) / PAGE, runs = (pages + SPLIT_PAGES - 1) / SPLIT_PAGES;
+        even.runs = runs < max_splits ? runs : max_splits;
+    }
+    return even;
+}
 // grid (kv heads * head tiles, rows, splits), or the first two changed over beyond 65,535 rows; four waves, each takes one page of the split's
 // SPLIT_PAGES, and their results are merged in LDS in the order of the keys. Columns are the
 // query heads of the kv group (16 per head tile). partial [rows][heads][max_splits][v_dim + 4]:
@@ -1067,7 +1091,7 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     const int32_t* __restrict__ row_seg, const int32_t* __restrict__ row_pos, int num_heads, int num_kv_heads,
     int head_dim, int v_dim, float scale_log2, int window, int chunk, float cap, float cap_scale, int max_splits,
     const int32_t* __restrict__ decode_work, const FusedProjections fused, int keep_first, const float* __restrict__ sinks,
-    const float* __restrict__ slopes, bool heads_first) {
+    const float* __restrict__ slopes, bool heads_first, const EvenSplits even) {
     __shared__ f32x4 shared_o[SPLIT_PAGES][HD / 16][64];
     __shared__ float shared_m[SPLIT_PAGES][16], shared_l[SPLIT_PAGES][16];
     __shared__ int ticket_shared;
@@ -1090,17 +1114,21 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     const int kept_blocks = (keep_first + PAGE - 1) / PAGE < window_block ? (keep_first + PAGE - 1) / PAGE : window_block;
     const int last_step = kept_blocks + last_block - window_block;
     // Splits are counted from the first page that holds a visible key; a split is `rounds` runs of
-    // SPLIT_PAGES pages. One run each serves while the step's runs (decode_work: over all its rows, each with no
-    // more than the grid has splits, which is what a window leaves of it; times the kv heads and head tiles) are fewer
-    // than the workgroups wanted; beyond, fewer and longer workgroups read the cache faster, and a row has fewer
-    // parts to merge (one workgroup for a whole row needs no merge at all). Counting the step's work, not the row's, gives
-    // a long row among short ones its share of the chip.
+    // SPLIT_PAGES pages, the same number for every row of the step. One run each serves while there are few; beyond, fewer and longer workgroups
+    // read the cache faster, and a row has fewer parts to merge (one workgroup for a whole row needs no merge at all). decode_work says what
+    // the step holds: below zero that its rows are equally long and the runs of the longest; else the runs of all rows together, of which no more
+    // count than a window leaves of every row (rows that all reach it are equally long). Counting the step's work,
+    // not the row's, gives a long row among short ones its share of the chip.
     int rounds = 1;
     if (decode_work) {
-        const long long most = (long long)rows * gridDim.z, runs = step_runs < most ? step_runs : most;
-        const long long beside = (long long)(last_step / SPLIT_PAGES + 1) * rows - runs;    // 0: every row is as long as this one
-        const int wanted = beside >= -rows && beside <= rows ? EVEN_WORKGROUPS : RAGGED_WORKGROUPS;
-        rounds = (int)((runs * acrosses + wanted - 1) / wanted);
+        if (step_runs < 0 || step_runs >= (long long)rows * even.runs) {
+            const uint32_t seen = -(uint32_t)step_runs;
+            const int longest = step_runs < 0 && seen < (uint32_t)even.runs ? (int)seen : even.runs;
+            const int splits = longest >= LONG_RUNS ? even.many : even.plain;
+            rounds = splits == 1 ? (int)gridDim.z : (longest + splits - 1) / splits;
+        } else {
+            rounds = (int)(((long long)step_runs * acrosses + RAGGED_WORKGROUPS - 1) / RAGGED_WORKGROUPS);
+        }
         rounds = rounds < 1 ? 1 : rounds;
     }
     const int pages_per_split = SPLIT_PAGES * rounds;
@@ -1576,16 +1604,17 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
     const bool heads_first = rows <= 65535;
     const int across = num_kv_heads * head_tiles;
     const dim3 grid(heads_first ? across : rows, heads_first ? rows : across, max_splits);
+    const EvenSplits even = even_splits(rows, across, max_splits, visible_span(window, chunk), keep_first);
 
 #define CALL(HD)                                                                                                              \
     if (fused.qkv)                                                                                                            \
         attention_decode_split_kernel<HD, true><<<grid, 64 * SPLIT_PAGES, 0, (hipStream_t)stream>>>(                          \
             (const uint16_t*)q, (uint16_t*)out, partial, tickets, (uint16_t*)k_pages, (uint16_t*)v_pages, block_table,        \
-            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first); \
+            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first, even); \
     else                                                                                                                      \
         attention_decode_split_kernel<HD, false><<<grid, 64 * SPLIT_PAGES, 0, (hipStream_t)stream>>>(                         \
             (const uint16_t*)q, (uint16_t*)out, partial, tickets, (uint16_t*)k_pages, (uint16_t*)v_pages, block_table,        \
-            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first)
+            table_stride, row_seg, row_pos, num_heads, num_kv_heads, head_dim, v_dim, rule.scale_log2, window, chunk, rule.cap, rule.cap_scale, max_splits, decode_work, fused, keep_first, sinks, slopes, heads_first, even)
     FW_BY_HEAD_DIM((head_dim > v_dim ? head_dim : v_dim), CALL);
 #undef CALL
     FW_LAUNCH_CHECK("attention_decode");
@@ -1596,8 +1625,8 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
 // max_context: no row's position reaches it (the caller knows; the kernel cannot check);
 // max_splits must cover the keys such a row sees, in runs of 4 pages. decode_work: null, or one
 // int32 on the device: the runs of 4 pages that all the rows of the step see together (the sum over
-// the rows of ceil((position + 1) / 256)); with it a workgroup takes as many runs as bring the step
-// down to 256 to 384 workgroups (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
+// the rows of ceil((position + 1) / 256)), or, where the rows are equally long, the runs of the longest as a negative number; with it a workgroup
+// takes as many runs as bring the step down to about as many workgroups as compute units (it changes how the work is shared out, not what is computed). tickets: rows * kv heads *
 // ceil(group / 16) int32 counters, zero before the first call and left zero; calls that overlap on
 // one device need their own (and their own workspace).
 extern "C" int fw_attention_decode(const void* q, void* out, float* partial, int max_splits, int max_context,

@@ -201,8 +201,8 @@ int fw_attention_prefill(const void* q, void* out, const void* k_pages, const vo
 // [rows][heads][max_splits][v_dim + 4]; max_context: an upper bound on position + 1 of every
 // row, known to the caller; tickets: rows * kv_heads * ceil(heads / kv_heads / 16) int32 counters,
 // zero before the first call and left zero. decode_work: null, or one int32 on the device, the runs
-// of 4 pages that all the rows of the step see together; with it a workgroup takes as many runs as
-// bring the step down to 256 to 384 workgroups.
+// of 4 pages that all the rows of the step see together, or, as a negative number, those that the longest of equally long rows sees; with it a workgroup
+// takes as many runs as bring the step down to about as many workgroups as compute units.
 int fw_attention_decode(const void* q, void* out, float* partial, int max_splits, int max_context,
                         const int32_t* decode_work, int* tickets, int tickets_len, const void* k_pages, const void* v_pages, const int32_t* block_table, int table_stride,
                         const int32_t* row_seg, const int32_t* row_pos, int rows, int num_heads, int num_kv_heads,

@@ -1160,8 +1160,9 @@ def attention_decode(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_di
                       slopes: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One row per request; ``max_context`` bounds position + 1 of every row (the host knows it).
     ``decode_work``: one int32 on the device, the runs of 4 pages that the rows see together (the
-    sum of ceil((position + 1) / 256)): the kernel shares the work out by it (fewer, longer
-    workgroups once there are more runs than 256 to 384); without it, one run per workgroup."""
+    sum of ceil((position + 1) / 256)), or, where the rows are equally long, those of the longest as a negative number: the kernel shares
+    the work out by it (fewer, longer workgroups once there are more runs than about as many as compute units); without it, one
+    run per workgroup."""
     _dev(q, k_pages, v_pages, block_table, row_seg, row_pos)
     _want(q, torch.bfloat16, "q")
     rows = q.shape[0]

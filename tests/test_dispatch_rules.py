@@ -205,3 +205,16 @@ def test_decode_steps_form_queries_inside_the_attention_kernel_where_that_is_fas
                           position_tables=lambda p: (None, None), step_arrays=lambda p: {})
     part.attend(None, ctx, SimpleNamespace(writes=True, k_pages=None, v_pages=None, block_table=None))
     assert took == [fused]
+
+
+@pytest.mark.parametrize("positions,work", [
+    ([1999] * 9, -8), ([1999] * 9 + [0] * 7, -8), ([2000, 2040, 2047, 2048], -9), ([700, 2900, 1500], 21), ([700, 2900, 1500, 0], 21), ([300], -2),
+    ([0] * 4, 0), ([2560, 10], 12), ([2999] * 63 + [40], -12)])
+def test_decode_steps_tell_rows_of_one_length_from_rows_of_many(positions, work):
+    """Whatever rows fill a step up."""
+    from types import SimpleNamespace
+    from flyweight_amd.parts.attention import QueryTileArrays
+    rows = np.asarray(positions, dtype=np.int32)
+    assert QueryTileArrays()._decode_work(SimpleNamespace(num_rows=len(rows), all_decode=True, host_row_pos=rows)) == work
+    beside = SimpleNamespace(num_rows=len(rows) + 50, all_decode=False, decode_prefix=len(rows), host_row_pos=np.concatenate([rows, np.arange(50, dtype=np.int32)]))
+    assert QueryTileArrays()._decode_work(beside) == work

@@ -838,6 +838,27 @@ def test_attention_decode_on_the_matrix_cores(ops, nh, nkv, hd, window):
         ops._check(status)
 
 
+@pytest.mark.parametrize("rows,filled,window", [(1, 0, 0), (9, 7, 0), (9, 7, 300), (40, 0, 0), (33, 7, 0), (64, 0, 500), (97, 15, 0)])
+def test_attention_decode_of_equally_long_rows(ops, rows, filled, window):
+    """However many runs the longest row is said to see (fewer than there are, too: a row may have moved on), and with rows at position 0 behind the
+    step's: the same values as with a run to a workgroup, up to the order of the sums."""
+    nh, nkv, hd, n = 16, 8, 64, 1400
+    pages = (n + 63) // 64
+    d = lambda a: torch.tensor(np.asarray(a, dtype=np.int32), device=DEV)       # noqa: E731
+    order = np.random.default_rng(rows).permutation(300)
+    table = np.stack([np.roll(order, -7 * r)[:pages] for r in range(rows)] + [np.full(pages, order[299])] * filled)
+    k_pages, v_pages = as_dev(gen(300, nkv, 64, hd, seed=1), torch.bfloat16), as_dev(gen(300, nkv, hd, 64, seed=2), torch.bfloat16)
+    q = as_dev(gen(rows + filled, nh * hd), torch.bfloat16)
+    positions = d([n - 1 - 3 * r for r in range(rows)] + [0] * filled)
+    run = lambda work: ops.attention_decode(q, nh, nkv, hd, k_pages, v_pages, d(table), d(np.arange(rows + filled)), positions, hd ** -0.5, n, window,  # noqa: E731
+                                            decode_work=None if work is None else d([work]))
+    apart = back(run(None))
+    for work in (-1, -2, -5, -6, -7, -(1 << 30), -(1 << 31), 6 * rows, (1 << 31) - 1):
+        out = run(work)
+        close(out, apart, torch.bfloat16)
+        assert torch.equal(run(work), out)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,v_dim,window,chunk,keep_first,softcap,sink,slope", [
     (16, 8, 64, 64, 0, 0, 0, 0.0, False, False), (8, 8, 64, 32, 700, 0, 70, 0.0, True, False), (8, 8, 48, 64, 0, 600, 0, 7.0, False, False),
     (16, 8, 128, 128, 0, 0, 0, 0.0, False, True), (8, 8, 80, 112, 900, 0, 0, 5.0, True, False), (8, 8, 16, 16, 0, 0, 0, 0.0, False, False),
