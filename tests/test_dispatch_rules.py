@@ -149,7 +149,13 @@ def test_products_beyond_64_rows_are_dealt_to_waves_where_that_is_faster(mode, M
     # many rounds of tiles, a short K, odd widths, few rows of tiles over a long K
     (1, 6200, 2048, 7168, ("big", 0)), (1, 8192, 2048, 1024, ("big", 0)), (1, 2690, 1536, 1024, ("big", 0)), (1, 1700, 2048, 7168, ("bigsplit", 0)), (1, 2048, 2048, 4160, ("deep", 128)),
     (2, 13184, 3496, 352, ("big", 0)), (2, 5964, 4032, 128, ("big", 0)), (2, 2304, 1281, 128, ("tiles", 0)), (2, 512, 4480, 2560, ("tiles", 0)),
-    (0, 100, 65536, 2048, ("tiles", 0)), (0, 512, 65536, 2048, ("big", 0)), (0, 128, 4480, 2816, ("split", 0)), (1, 256, 2112, 7872, ("bigsplit", 0))])
+    (0, 100, 65536, 2048, ("tiles", 0)), (0, 512, 65536, 2048, ("big", 0)), (0, 128, 4480, 2816, ("split", 0)), (1, 256, 2112, 7872, ("bigsplit", 0)),
+    # what the GPU tests of these tiles compute
+    (1, 2048, 2048, 4096, ("big", 0)), (1, 1800, 1990, 4160, ("deep", 128)), (1, 2048, 1024, 2048, ("deep", 64)), (1, 1152, 2048, 2048, ("big", 0)),
+    (1, 576, 2048, 1024, ("deep", 64)), (1, 1100, 1024, 2048, ("deep", 64)), (1, 1664, 2048, 4096, ("deep", 128)), (0, 256, 6144, 2048, ("deep", 64)),
+    (0, 1100, 2048, 4096, ("bigsplit", 0)), (0, 130, 6144, 2048, ("deep", 64)), (1, 320, 2048, 2048, ("deep", 64)), (0, 300, 3072, 1024, ("deep", 64)),
+    (0, 600, 6144, 2048, ("big", 0)), (0, 700, 6144, 2048, ("big", 0)), (0, 500, 6100, 1984, ("big", 0)), (0, 256, 1024, 2048, ("deep", 64)),
+    (0, 1300, 2944, 7680, ("deep", 128))])
 def test_tiled_products_take_the_tiles_that_were_the_fastest(mode, M, N, K, plan):
     from flyweight_amd.kernels import ops
     assert ops.tiled_plan(mode, M, N, K) == plan

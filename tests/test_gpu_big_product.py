@@ -144,8 +144,8 @@ def test_large_tiles_with_k_cut_over_workgroups(ops, M, N, K, slices):
     workspace = torch.full((need_bytes // 4,), float("nan"), device=DEV)
     counters = torch.zeros(need_counters, dtype=torch.int32, device=DEV)
 
-    def run(mode, out, with_bias=False):
-        ops._check(ops.library().fw_gemm_mfma_big_split(ops._p(a), ops._p(w), ops._p(bias) if with_bias else None, ops._p(out), ops._code(out.dtype), mode, M,
+    def run(mode, out, with_bias=False, code=None):
+        ops._check(ops.library().fw_gemm_mfma_big_split(ops._p(a), ops._p(w), ops._p(bias) if with_bias else None, ops._p(out), code or ops._code(out.dtype), mode, M,
                                                         N, K, ops._p(workspace), need_bytes, ops._p(counters), counters.numel(), ops._stream()))
         return out
 
@@ -154,6 +154,10 @@ def test_large_tiles_with_k_cut_over_workgroups(ops, M, N, K, slices):
     stored = run(STORE, torch.empty(M, N, device=DEV), True)
     assert ((stored.double() - want).abs() <= room).all()
     assert ((run(STORE, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), True).double() - want).abs() <= room + 2.0 ** -8 * want.abs()).all()
+    # (gelu's slope is below 1.13; its short error function is within 1.5e-7, times half of z)
+    unit = run(STORE, torch.empty(M, N, device=DEV, dtype=torch.bfloat16), True, ops.BF16_GELU).double()
+    gelu = torch.nn.functional.gelu(want)
+    assert ((unit - gelu).abs() <= 1.13 * room + 1e-6 + 1e-6 * want.abs() + 2.0 ** -8 * gelu.abs()).all()
     total = run(ADD, residual.clone()).double()
     assert ((total - exact - residual.double()).abs() <= limit + 2.0 ** -23 * total.abs()).all()
     # whichever workgroup of a tile ends last, the slices are added in their order, and the counters are left at zero

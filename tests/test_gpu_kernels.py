@@ -521,13 +521,30 @@ def test_tiles_whose_waves_split_k(ops, M, N, K, columns):
         ops.gemm_deep(a[:, :K - 8].contiguous(), w[:, :K - 8].contiguous())
 
 
-@pytest.mark.parametrize("M,N,K,expected", [(2048, 2048, 4160, 128), (1800, 1990, 4160, 128), (2048, 1024, 2048, 64),
-                                            (1664, 2048, 4096, 128), (576, 2048, 1024, 64), (1100, 1024, 2048, 64)])
-def test_the_prompt_product_of_one_round_of_tiles_over_a_long_k(ops, M, N, K, expected):
-    """What the dispatch sends to those tiles of products that add into the residual: about one 128 x 128 tile per compute unit
-    and a long K (the w2 product of a 2,048-token prompt), rounds that are little more than half full, narrower tiles
-    where those fill theirs better."""
-    assert ops.tiled_plan(1, M, N, K) == ("deep", expected)
+def tiled_by_name(ops, kind, columns, a, w, mode, target):
+    """The product on tiles of both operands that is called `kind`, into `target` (float32)."""
+    lib, (M, K), N = ops.library(), a.shape, w.shape[0]
+    common = (ops._p(a), ops._p(w), None, ops._p(target), ops._code(target.dtype), mode, M, N, K)
+    if kind in ("split", "bigsplit"):
+        need_bytes, need_counters = (ops._split_needs if kind == "split" else ops._big_split_needs)(mode, M, N, K)[:2]
+        workspace = torch.empty(need_bytes // 4, device=DEV)
+        counters = torch.zeros(need_counters, dtype=torch.int32, device=DEV)
+        ops._check((lib.fw_gemm_mfma_split if kind == "split" else lib.fw_gemm_mfma_big_split)(
+            *common, ops._p(workspace), need_bytes, ops._p(counters), counters.numel(), ops._stream()))
+        torch.cuda.synchronize()
+        return
+    if kind == "deep":
+        common += (columns,)
+    ops._check({"big": lib.fw_gemm_mfma_big, "tiles": lib.fw_gemm_mfma, "deep": lib.fw_gemm_mfma_deep}[kind](*common, ops._stream()))
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 2048, 4096), (1800, 1990, 4160), (2048, 1024, 2048), (1152, 2048, 2048), (576, 2048, 1024), (1100, 1024, 2048),
+                                   (2048, 2048, 4160), (1664, 2048, 4096)])
+def test_the_prompt_product_of_one_round_of_tiles_over_a_long_k(ops, M, N, K):
+    """Products that add into the residual, of about one 128 x 128 tile per compute unit over a long K, of rounds that are little more than half
+    full, and of narrower tiles where those fill theirs better: the values, bit for bit those of the kernel that the plan names. (Which one that
+    is stands in test_dispatch_rules.)"""
+    kind, columns = ops.tiled_plan(1, M, N, K)
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     want = back(a) @ back(w).T
@@ -536,37 +553,35 @@ def test_the_prompt_product_of_one_round_of_tiles_over_a_long_k(ops, M, N, K, ex
     ops.gemm(a, w, accumulate_into=residual)
     close(residual, before + want, torch.float32, 2.0)
     direct = before.float().to(DEV)
-    ops.gemm_deep(a, w, accumulate_into=direct, columns=expected)
+    tiled_by_name(ops, kind, columns, a, w, 1, direct)
     assert torch.equal(direct, residual)
     close(ops.gemm(a, w, out_dtype=torch.float32), want, torch.float32, 2.0)
 
 
-@pytest.mark.parametrize("M,N,K,mode,columns", [(256, 6144, 2048, 0, 64), (1100, 2048, 4096, 0, 0), (130, 6144, 2048, 0, 64),
-                                                   (512, 2048, 2048, 1, 64), (320, 2048, 2048, 1, 64), (300, 3072, 1024, 0, 64),
-                                                   (256, 2048, 8192, 1, 0), (600, 6144, 2048, 0, 0), (700, 6144, 2048, 0, 0), (500, 6100, 1984, 0, 0), (256, 1024, 2048, 0, 64)])
-def test_a_few_hundred_rows_go_to_the_tiles_whose_waves_split_k(ops, M, N, K, mode, columns):
-    """A decode step of a few hundred requests: storing and short accumulating products take those
-    tiles (equal, bit for bit, to the kernel called by name); a long K of few rows has it cut over
-    workgroups, and wide outputs of some hundred rows go to the large tiles."""
-    kind, width = ops.tiled_plan(mode, M, N, K)
-    assert (width if kind == "deep" else 0) == columns
+@pytest.mark.parametrize("M,N,K,mode", [(256, 6144, 2048, 0), (1100, 2048, 4096, 0), (130, 6144, 2048, 0), (512, 2048, 2048, 1), (320, 2048, 2048, 1), (300, 3072, 1024, 0),
+                                        (256, 2048, 8192, 1), (600, 6144, 2048, 0), (700, 6144, 2048, 0), (500, 6100, 1984, 0), (256, 1024, 2048, 0), (1300, 2944, 7680, 0),
+                                        (100, 8192, 32, 0)])
+def test_a_few_hundred_rows_go_to_the_tiles_that_the_plan_names(ops, M, N, K, mode):
+    """A decode step of a few hundred requests, and storing products on every kind of tiles: the values, bit for bit those of the kernel that the
+    plan names. (Which one that is stands in test_dispatch_rules.)"""
+    kind, columns = ops.tiled_plan(mode, M, N, K)
     a = as_dev(gen(M, K), torch.bfloat16)
     w = as_dev(gen(N, K, seed=1, scale=K ** -0.5), torch.bfloat16)
     want = back(a) @ back(w).T
     if mode == 0:
         got = ops.gemm(a, w, out_dtype=torch.float32)
         close(got, want, torch.float32, 2.0)
-        if columns:
-            assert torch.equal(got, ops.gemm_deep(a, w, out_dtype=torch.float32, columns=columns))
+        direct = torch.empty_like(got)
+        tiled_by_name(ops, kind, columns, a, w, 0, direct)
+        assert torch.equal(got, direct)
     else:
         residual = gen(M, N, seed=3).float().to(DEV)
         before = residual.cpu().double()
         ops.gemm(a, w, accumulate_into=residual)
         close(residual, before + want, torch.float32, 2.0)
-        if columns:
-            direct = before.float().to(DEV)
-            ops.gemm_deep(a, w, accumulate_into=direct, columns=columns)
-            assert torch.equal(direct, residual)
+        direct = before.float().to(DEV)
+        tiled_by_name(ops, kind, columns, a, w, 1, direct)
+        assert torch.equal(direct, residual)
 
 
 def test_fast_gemm_rows_do_not_depend_on_the_batch(ops):
