@@ -1,4 +1,4 @@
-// gemm_float32_few.hip: products of up to four float32 rows, bit for bit those of gemm_float32.hip
+// gemm_float32_few.hip: products of one or two float32 rows, bit for bit those of gemm_float32.hip
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -39,7 +39,9 @@ int fw_gemm_generic(const void* a, int a_dtype, const void* w, int w_dtype, cons
 // rows then up rows, out (float32) = silu(a . gate^T) * (a . up^T), no bias.
 int fw_gemm_float32(const float* a, const float* w, const float* bias, void* out, int out_dtype, int mode,
                     int M, int N, int K, void* stream);
-// The same for up to four rows of x (row_index[m], or m) that pass an RMS norm first, bit for bit as fw_rmsnorm_rows followed by fw_gemm_float32; modes 0
+// 1 where a kernel for one or two rows takes that product, 0 where the matrix instruction does (the same bits either way).
+int fw_gemm_float32_few_rows(int mode, int M, int N, int K);
+// The same for one or two rows of x (row_index[m], or m) that pass an RMS norm first, bit for bit as fw_rmsnorm_rows followed by fw_gemm_float32; modes 0
 // and 2, float32 out. fw_gemm_float32_normed_takes: 1 where a shape is taken.
 int fw_gemm_float32_normed_takes(int mode, int M, int N, int K);
 int fw_gemm_float32_normed(const float* x, const float* norm_weight, const int32_t* row_index, float eps, int one_centered, const float* w, const float* bias,

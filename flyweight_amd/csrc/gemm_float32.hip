@@ -20,7 +20,8 @@
 //  * Every output is the sum over the same groups of the same four k in the same order, part by part, the parts
 //    four by four, whatever the tile: its value does not depend on M or on the other rows.
 //
-// One and two rows over K from 1,024 on go to gemm_float32_few.hip, which gives the same bits.
+// One row over K from 1,024 to 8,192 goes to gemm_float32_few.hip, which gives the same bits, and so do two rows below 32,768 features, adding over K up to
+// 4,096, storing and gated over K 1,024 (fw_gemm_float32_few_takes).
 //
 // Measured inside a request of the LFM2-350M shape in float32, before -> after: one row, 1,024 outputs (K 4,608 and 1,024
 // in the mean) 464 -> 9.3 us, gate|up (2 x 4,608, K 1,024) 171 + 5 -> 13.6 us (2.8 TB/s of W), 65,536 outputs 255 -> 49 us (5.4

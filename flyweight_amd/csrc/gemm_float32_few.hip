@@ -1,18 +1,19 @@
-// Matrix product of up to four rows, float32: out[M][N] = a[M][K] . w[N][K]^T, optionally with the rows' RMS norm in front. The float32 matrix
+// Matrix product of one or two rows, float32: out[M][N] = a[M][K] . w[N][K]^T, optionally with the rows' RMS norm in front. The float32 matrix
 // instruction (gemm_float32.hip) computes sixteen rows whether they are there or not, and a tile of sixteen features gives a product of 1,024
 // outputs 64 workgroups: a fourth of the chip streams W, through 4 us of matrix time. Here every output is formed by ordinary multiply-adds in the order
 // of that instruction (its four k one after the other, each a fused multiply-add: bit for bit the same on normal and subnormal numbers), so
 // that a value does not depend on the kernel that formed it:
 //
-//  * a workgroup has 4 or 16 rows of W and all of K, which is cut into sixteen parts: wave q has parts 4 q .. 4 q + 3, a lane one row of W, one part
-//    (and with 4 rows of W one row of a). A lane walks its part in groups of 16 k; the parts meet in LDS at the end and are added as there;
+//  * a workgroup has 4 or 16 rows of W and all of K, which is cut into sixteen parts: wave q has parts 4 q .. 4 q + 3, a lane one row of W and one part.
+//    With 16 rows of W a lane takes the rows of a in turn; with 4 a wave has four places for rows of a, of which two at most are filled and the others form
+//    the first row's sums once more. A lane walks its part in groups of 16 k; the parts meet in LDS at the end and are added as there;
 //  * W goes straight into LDS, each wave's into a ring of its own up to sixteen groups deep (64 KB a workgroup in flight), 64 contiguous bytes a row of W
 //    and part; no barrier in the loop;
 //  * the rows of a lie in LDS, normed on the way there. They are asked for ahead of W, so that nothing waits for W before it is needed; the norm's
 //    chain (load, sum over the workgroup, scale) runs while W is on its way and the kernel that did it alone is saved.
 //
-// Bound by the stream of W (1,024 x 4,608: 2.3 TB/s, 4,608 gated x 1,024 3.1, 65,536 x 1,024 5.4) and by the kernel's start and end. Four rows of W a workgroup up to
-// 3,072 outputs, 16 beyond (3,072 storing 5.7 with 16, 6.3 with 4; 2,048 5.1 and 4.8).
+// Bound by the stream of W (1,024 x 4,608: 2.3 TB/s, 4,608 gated x 1,024 3.1, 65,536 x 1,024 5.4) and by the kernel's start and end. Four rows of W a workgroup below
+// 3,072 outputs, 16 from there on and for gated products (3,072 storing 5.7 with 16, 6.3 with 4; 2,048 5.1 and 4.8).
 #include "fw_common.h"
 #include "fw_kernels.h"
 #include "float32_few.h"
@@ -325,7 +326,9 @@ int fw_launch_float32_few(const float* a, const float* norm_weight, const int32_
     return choose<MF_STORE, bf16_t>(a, norm_weight, row_index, eps, one_centered, w, bias, out, M, N, K, s);
 }
 
-// fw_gemm_float32 over rows that pass an RMS norm first, as fw_rmsnorm_rows gives it bit for bit. 0 rows taken: fw_gemm_float32_normed_takes.
+// fw_gemm_float32 over rows that pass an RMS norm first, as fw_rmsnorm_rows gives it bit for bit; fw_gemm_float32_normed_takes says for which shapes.
+// fw_gemm_float32_few_rows: whether fw_gemm_float32 itself comes here.
+extern "C" int fw_gemm_float32_few_rows(int mode, int M, int N, int K) { return fw_gemm_float32_few_takes(M, N, K, mode, false) ? 1 : 0; }
 extern "C" int fw_gemm_float32_normed_takes(int mode, int M, int N, int K) { return fw_gemm_float32_few_takes(M, N, K, mode, true) ? 1 : 0; }
 extern "C" int fw_gemm_float32_normed(const float* x, const float* norm_weight, const int32_t* row_index, float eps, int one_centered, const float* w,
                                       const float* bias, float* out, int mode, int M, int N, int K, void* stream) {

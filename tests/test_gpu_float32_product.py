@@ -95,7 +95,14 @@ def test_what_its_loads_cannot_take_goes_to_the_plain_tiles(ops):
 @pytest.mark.parametrize("K", [1024, 1028, 1040, 1280, 2052, 3900, 4096, 4100, 8192])
 @pytest.mark.parametrize("N", [1, 5, 1024, 3071, 3072, 3081])
 def test_few_rows_have_the_values_of_many(ops, N, K):
-    """One and two rows go to a kernel of their own, three and more to the matrix instruction: the same bits, with and without the norm in front."""
+    """One row, two over a short K or that add, go to a kernel of their own, more to the matrix instruction: the same bits, with and without the norm in front."""
+    # what the threads hold of the rows, and where two rows' multiply-adds in line are still the faster ones
+    takes = {(rows, mode): rows * K <= 8192 and (rows == 1 or mode == 1 or K == 1024) for rows in (1, 2) for mode in (0, 1, 2)}
+    for rows in (1, 2, 3):
+        for mode in (0, 1, 2):
+            assert bool(ops.library().fw_gemm_float32_few_rows(mode, rows, N, K)) == takes.get((rows, mode), False)
+            if mode != 1:
+                assert ops.float32_normed_takes(mode == 2, rows, N, K) == (takes.get((rows, mode), False) and K <= 4096)
     a, w = draw(19, K).to(DEV), draw(2 * N, K, seed=1).to(DEV)
     bias, weight = draw(N, seed=2).to(DEV), draw(K, seed=3).to(DEV)
     old = draw(19, N, seed=4).to(DEV)
@@ -107,10 +114,10 @@ def test_few_rows_have_the_values_of_many(ops, N, K):
         index = torch.tensor([11, 4], dtype=torch.int32, device=DEV)
         for rows in (1, 2):
             of = index[:rows].long()
-            if ops.float32_normed_takes(False, rows, N, K):
+            if takes[rows, 0]:
                 assert torch.equal(ops.gemm_float32_normed(a, weight, 1e-5, one_centered, w[:N].contiguous(), bias, row_index=index[:rows]), stored[of])
                 assert torch.equal(ops.gemm_float32_normed(a[:rows].contiguous(), weight, 1e-5, one_centered, w[:N].contiguous(), bias), stored[:rows])
-            if ops.float32_normed_takes(True, rows, N, K):
+            if takes[rows, 2]:
                 assert torch.equal(ops.gemm_float32_normed(a, weight, 1e-5, one_centered, w, row_index=index[:rows], gated=True), gated[of])
     stored, gated = ops.gemm(a, w[:N], bias), ops.gemm_swiglu(a, w)
     total = ops.gemm(a, w[:N], accumulate_into=old.clone())
