@@ -340,8 +340,12 @@ __global__ __launch_bounds__(64) void attention_generic_kernel(
 
 // The same for steps of few rows, float32, head sizes that are multiples of 4: a workgroup of eight waves per (row, head), which take eight pages side by
 // side. Scores, maxima, exponentials and a page's weighted sum are formed page by page as above, and the pages then folded in their order with the same
-// expressions: bit for bit the same results. What it saves is the chain from page to page: 16 heads of 64 channels, one row behind 301-308
-// keys 19.5 -> FW_PAGES_FIGURE us. With rows times heads enough to fill the chip the waves above have no idle compute units beside them.
+// expressions: bit for bit the same results. What it saves is the chain from page to page. us, a wave a row and head / eight pages, 16 heads in 8
+// groups of 64 channels, one row of 20 / 64 / 100 / 300 / 1,100 / 3,000 keys 5.4 / 5.5, 4.8 / 5.5, 7.9 / 6.6, 15.5 / 10.1, 47.5 / 27.8, 136 / 67; sixteen
+// rows 5.5 / 5.7, 5.0 / 5.7, 8.1 / 6.8, 17.9 / 11.0, 54.9 / 29.7, 161 / 75; 8 heads of 96 channels, 32 rows of 64 / 300 / 3,000 keys 7.4 / 7.8, 28.1 / 17.1,
+// 266 / 138; 4 heads of 256, 64 rows 10.3 / 9.2, 56.1 / 29.4, 586 / 252. A context of one page has nothing to take side by side and costs up to 0.8 us
+// more, with narrow heads; how long contexts are the caller of a recorded step does not know. With rows times heads
+// enough to fill the chip the waves above have no idle compute units beside them.
 #define SIDE 8
 #define PAGES_MOST 256          // rows times heads: a workgroup a compute unit
 __global__ __launch_bounds__(64 * SIDE) void attention_pages_kernel(
