@@ -987,7 +987,9 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
 // the next one on by a compute unit. us of the best of 1 to 24 splits / this rule / as many splits as bring all the rows' runs below 256, mean of 560
 // steps (1 to 96 rows, a third of them filled up, 300 to 6,000 keys; 1 to 8 kv heads of 64 and 128 channels) 1 / 1.021 / 1.057: 20 rows filled up to 24 behind
 // 2,900 keys, 32 heads in 8 groups of 64 channels 28.0 / 28.0 / 33.3, 2 groups of 16 heads of 128 channels 24.6 / 24.6 / 32.0; 24 rows, 4 groups of 128
-// channels 37.6 / 37.6 / 47.0; 40 rows, the same, 1,000 keys (1 and 2 splits) 24.3 and 30.9, 2,900 (1, 2 and 3) 58.3, 65.4 and 51.7.
+// channels 37.6 / 37.6 / 47.0; 40 rows, the same, 1,000 keys (1 and 2 splits) 24.3 and 30.9, 2,900 (1, 2 and 3) 58.3, 65.4 and 51.7. Heads of 144 to
+// 256 channels, which do not stream, are cut the same way: 230 steps, the best 1, by this rule 1.015, 1.028 with 256 workgroups (384 where rows fill the step up); 48
+// rows of 1,000 keys, 4 groups of 256 channels 55.5 by this rule, 63.1 by those, but of 2,900 keys 135.6 and 122.5.
 // Where the lengths differ, RAGGED_WORKGROUPS at most (rounds rounded up): a half more than compute units fill up behind those of short rows. Mean of 48
 // ragged steps (3 to 64 rows of up to 6,000 keys, 4 head shapes of 64 and 128 channels) with 256 / 320 / 384 / 512 workgroups 41.4 / 40.5 / 39.7 / 40.1 us.
 #define EVEN_WORKGROUPS 256
@@ -1020,9 +1022,9 @@ static EvenSplits even_splits(int rows, int across, int max_splits, int span, in
 // What bounds it is memory: bytes on their way to the compute units, for as long as the walk takes. Up to 128 channels a wave's
 // loads of a page's keys go out as soon as the page before has been scored, those of its values as soon as the values before are used, the
 // page's number one page earlier still, and the first page's while the fused variant forms the queries; each page in turn, with
-// its number looked up in front and nothing on its way during the arithmetic: 64 rows of 725..2,900 keys, 32 heads in 8 groups of 64 channels
-// 84 us, now 56 (4.6 TB/s); 24 rows 38, now 36; 8 rows of 2,048 keys 17.6, now 15.0; 8 rows of 32,768 keys, 16 heads
-// 100, now 98 (5.5 TB/s); groups of 16 heads of 128 channels, 64 rows 75, now 47. Two pages in the registers at a time did not fit (the compiler
+// its number looked up in front and nothing on its way during the arithmetic (and cut into up to 512 workgroups): 64 rows of 725..2,900 keys, 32 heads in 8
+// groups of 64 channels 72.6 us, now 54.8 (4.6 TB/s); 24 rows 35.3, now 30.5; 8 rows of 2,048 keys 15.7, now 14.6; 8 rows of 32,768 keys, 16 heads
+// 101.5, now 100.4 (5.4 TB/s); 16 heads in one group of 128 channels, 64 rows 40.1, now 33.1. Two pages in the registers at a time did not fit (the compiler
 // copies between them and spills); 167 registers leave room for three waves a SIMD.
 // What the fused variant does in front of the attention: the step's raw projections (float32
 // [rows][(heads + kv heads) * head_dim + kv heads * v_dim]: queries, keys, values) get their per-head RMS norm and
@@ -1600,7 +1602,7 @@ static int decode_launch(const void* q, void* out, float* partial, int max_split
     const ScoreRule rule = score_rule(scale, softcap);
     const int head_tiles = (num_heads / num_kv_heads + 15) / 16;
     // Workgroups go to the eight dies in turn: the heads of a row first, so that a long row is spread over the dies (rows first, a
-    // step of 8 n rows puts all of a row on one die: 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 59.9 us, now 56.1; in 16 groups 117, now 107).
+    // step of 8 n rows puts all of a row on one die: 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 59.9 us against 56.1; in 16 groups 117 against 107).
     const bool heads_first = rows <= 65535;
     const int across = num_kv_heads * head_tiles;
     const dim3 grid(heads_first ? across : rows, heads_first ? rows : across, max_splits);

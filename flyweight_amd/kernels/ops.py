@@ -1251,13 +1251,16 @@ def attention_is_tiled(head_dim: int) -> bool:
 def prompt_halves(tiles: int, num_heads: int, num_kv_heads: int, widest: int, keys: int) -> bool:
     """Whether a prompt's attention takes the form of two heads a workgroup (fw_attention_prefill), whose two halves share the
     pages out: ``tiles`` tiles of rows, of which the rows see up to ``keys`` keys, heads of up to ``widest`` channels.
+    It is asked where the heads of a group are not taken two by two (``prompt_pairs``): heads of 48 channels, or keys and values of 48 and 64.
     Its workgroups have a compute unit each, those of the form of one head share one by two to four. So it pays where
     its rounds over the chip are full, and where rows see enough keys for the merge at the end to be little. us, one head /
-    halves, heads of 64: 32 heads in 8 groups, 2,048 rows (2 rounds) behind 0 / 2,048 / 30,720 keys 44 / 45, 133 / 102, 1,084 /
-    870; 1,500 rows (1.5 rounds) behind 3,072 97 / 115; 1,700 (1.7) behind 2,048 123 / 95; 777 (0.8) behind 0 / 512 18.0 / 19.1,
-    27.2 / 26.2; 6,000 (5.9) behind 4,096 687 / 624, 3,500 (3.4) 329 / 336; 20 prompts of 300 (6.3) behind 1,300 188 / 202. 16
-    heads in 8 groups, 777 rows (0.4) behind 2,048 / 30,720 45.7 / 46.0, 453 / 430. With an odd number of heads a group one wave
-    in so many idles (24 in 8 groups, 2,048 rows behind 8,192 223 / 267), and heads of 32 channels leave LDS less to bound
+    halves, heads of 48: 32 heads in 8 groups, 2,048 rows (2 rounds) behind 0 / 2,048 / 30,720 keys 53.5 / 54.1, 120 / 109, 1,050 /
+    850; 1,500 rows (1.5 rounds) behind 3,072 100 / 121; 1,700 (1.7) behind 2,048 108 / 100; 777 (0.8) behind 0 / 512 19.5 / 19.5,
+    27.6 / 26.7; 6,000 (5.9) behind 4,096 642 / 642, 3,500 (3.4) 333 / 345; 16 heads in 8 groups, 777 rows (0.4) behind 2,048 45.0 /
+    45.7, 2,048 rows (1) behind 0 / 30,720 38.1 / 35.1, 544 / 438; keys of 64 and values of 48, 32 heads, 2,048 rows behind 0 / 2,048 53.1 /
+    54.2, 119 / 109, 6,000 behind 4,096 639 / 647; keys of 48 and values of 64, 16 heads, 2,048 rows behind 2,048 76 / 64. Over 52 such prompts
+    the rule's choice takes 0.1 % more than the better one. With an odd number of heads a group one wave
+    in so many idles (24 in 8 groups of 64 channels, 2,048 rows behind 8,192 223 / 267), and heads of 32 channels leave LDS less to bound
     (2,048 rows behind 8,192 188 / 213)."""
     group = num_heads // num_kv_heads
     if not 32 < widest <= 64 or group % 2:

@@ -93,14 +93,14 @@ class GQAttention(QueryTileArrays, Mixer):
     graph_safe = True
     accepts_lazy_norm = True
     # Up to this many rows a decode step forms queries and keys inside the attention kernel, while its first pages are on
-    # their way: 17 / 32 / 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 22.6 / 38.8 / 63.6 us against 25.3 / 40.6 / 69.0 in two
-    # kernels, of 300 keys 11.4 / 10.9 / 14.1 against 12.9 / 12.7 / 19.4; with 128 channels 15.3 / 15.6 / 21.6 against 17.5 / 17.4 /
-    # 22.9 (128 rows of 3,000 keys 231 against 221). Every workgroup of a group forms all its queries: groups of 16 heads of 128 channels
-    # take 19.4 us at 17 rows of 300 keys against 17.4, so that groups of more than four stay with 16 rows.
+    # their way: 17 / 32 / 64 ragged rows of up to 2,900 keys, 32 heads in 8 groups 29.3 / 38.4 / 59.9 us against 32.0 / 40.5 / 64.6 in two
+    # kernels, of 300 keys 10.5 / 11.7 / 16.3 against 12.5 / 13.8 / 21.3; with 128 channels 15.0 / 16.1 / 17.7 against 17.4 / 19.0 /
+    # 19.5 (128 rows of 3,000 keys 144 against 147). Every workgroup of a group forms all its queries: groups of 16 heads of 128 channels
+    # take 19.2 us at 17 rows of 300 keys against 17.1, so that groups of more than four stay with 16 rows.
     # Heads beyond 128 channels have no page on its way meanwhile (the registers would not hold it). They gain up to 32 rows, by the kernel
-    # that is saved, and lose beyond, where many workgroups wait for the queries: 16 heads in 4 groups of 192 channels, 24 / 32 rows of 2,900 keys 65.0 /
-    # 73.4 against 68.2 / 77.9, 48 / 64 rows 118.4 / 134.5 against 111.3 / 133.9; of 256 channels, 32 rows 88 against 94, 48 rows of 300 / 1,000 / 2,900 keys
-    # 31.7 / 74.1 / 141.9 against 30.8 / 70.1 / 135.0; 8 heads in 8 groups of 144 channels, 32 rows of 300 keys 23.3 against 24.9, 64 rows 46.4 against 45.8.
+    # that is saved, and no more beyond, where many workgroups wait for the queries: 16 heads in 4 groups of 192 channels, 24 / 32 rows of 2,900 keys 69.8 /
+    # 74.1 against 74.2 / 79.0, 48 / 64 rows 119.3 / 128.4 against 121.1 / 129.3; of 256 channels, 32 rows 88.0 against 94.0, 48 rows of 300 / 1,000 / 2,900 keys
+    # 33.5 / 63.2 / 148.4 against 32.3 / 63.0 / 147.9; 8 heads in 8 groups of 144 channels, 32 rows of 300 keys 24.6 against 26.4, 64 rows 45.8 against 45.3.
     FUSED_DECODE_ROWS = 16
     FUSED_DECODE_ROWS_OF_FEW_HEADS = 64
     FUSED_DECODE_ROWS_OF_WIDE_HEADS = 32
