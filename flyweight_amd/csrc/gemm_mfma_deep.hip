@@ -1,5 +1,6 @@
 // Tiled matrix product for prompts whose output is too narrow for the 256 x 256 tiles to fill the
-// chip (2,048 rows x 2,048 features: 64 large tiles for 256 compute units): out[M][N] =
+// chip (2,048 rows x 1,024 features: 32 large tiles for 256 compute units; into 2,048 features
+// the large tiles have become the faster ones, over a long K with K cut over workgroups): out[M][N] =
 // a[M][K] . w[N][K]^T with 128 x 128 tiles in which the four waves split K, not the tile.
 //
 // With a 128 x 128 tile cut into four 64 x 64 quarters, one per wave, every k16 step of a wave
