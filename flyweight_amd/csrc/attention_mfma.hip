@@ -1153,7 +1153,7 @@ __global__ __launch_bounds__(64 * SPLIT_PAGES) __attribute__((amdgpu_waves_per_e
     auto number_of = [&](int round) { return table[block_of(round < my_rounds ? round : my_rounds - 1)]; };
     // Up to 128 channels the pages stream: STAGES of them are on their way at any time, the first ones while the queries are formed.
     constexpr bool STREAMED = HD <= 128;
-    constexpr int STAGES = 1;
+    constexpr int STAGES = 1;       // (written out without the loops over them the compiler keeps the pages otherwise: heads of 128 channels spill)
     PageOnWay<STREAMED ? HD : 32> pages[STAGES];
     const PageOffsets<STREAMED ? HD : 32> offsets(head_dim);
     int next[STAGES];
