@@ -33,15 +33,6 @@
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-#define PARTS 16
-
-enum { MF_STORE = 0, MF_ACCUMULATE = 1, MF_SWIGLU = 2 };
-
-__device__ __forceinline__ float sigmoid_float32(float x) {
-    const float e = expf(x >= 0.0f ? -x : x);
-    return x >= 0.0f ? 1.0f / (1.0f + e) : e / (1.0f + e);
-}
-
 // A group of 16 k of 16 rows is 1 KB of LDS: row r at 64 r, its four pieces (of four k) permuted, piece p in place
 // p ^ (r / 4 % 4), so that the reads of one piece of 16 rows cover all banks once. Instruction j of a group takes
 // component j of every lane's piece, so its four k are j, 4 + j, 8 + j, 12 + j of the group.

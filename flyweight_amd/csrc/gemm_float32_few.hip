@@ -20,18 +20,10 @@
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-#define PARTS 16
 #define FEW_WIDE 3072                   // outputs from which a workgroup has 16 rows of W
 #define FEW_ROWS 2
 #define FEW_HOLD 8                      // runs of four floats of the rows that a thread holds on their way to LDS
 #define NORM_RUNS 4                     // of one row with a norm: K up to 4,096
-
-enum { MF_STORE = 0, MF_ACCUMULATE = 1, MF_SWIGLU = 2 };
-
-__device__ __forceinline__ float sigmoid_float32(float x) {
-    const float e = expf(x >= 0.0f ? -x : x);
-    return x >= 0.0f ? 1.0f / (1.0f + e) : e / (1.0f + e);
-}
 
 // A workgroup barrier that orders LDS traffic alone. (fw_lds_barrier waits for loads to LDS as well, here for all of W that is on its way.)
 __device__ __forceinline__ void meet() {
