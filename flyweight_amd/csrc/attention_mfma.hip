@@ -367,6 +367,61 @@ __device__ __forceinline__ void attend_on_way(Columns<HD>& c, PageOnWay<HD>& pag
     ask_values();
 }
 
+// The second of two halves that shared a tile's pages out leaves its maximum, sum and output to the same lane of the first, which joins them with its own.
+template <int HD, int NH>
+__device__ __forceinline__ void leave_columns(const Columns<HD> (&c)[NH], float* left) {        // left: [NH][HD / 4 + 2][256], this thread's place
+    constexpr int VALUES = HD / 4 + 2;
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+        left[(h * VALUES + HD / 4) * 256] = c[h].m;
+        left[(h * VALUES + HD / 4 + 1) * 256] = c[h].l;
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) left[(h * VALUES + t * 4 + r) * 256] = c[h].o[t][r];
+    }
+}
+template <int HD, int NH>
+__device__ __forceinline__ void join_columns(Columns<HD> (&c)[NH], const float* left) {
+    constexpr int VALUES = HD / 4 + 2;
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+        const float other = left[(h * VALUES + HD / 4) * 256], top = fmaxf(c[h].m, other);
+        // (a half without any key of this row keeps NEG_BIG: its factor is 0)
+        const float mine = __builtin_amdgcn_exp2f(c[h].m - top), theirs = __builtin_amdgcn_exp2f(other - top);
+        c[h].m = top;
+        c[h].l = c[h].l * mine + left[(h * VALUES + HD / 4 + 1) * 256] * theirs;
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c[h].o[t][r] = c[h].o[t][r] * mine + left[(h * VALUES + t * 4 + r) * 256] * theirs;
+    }
+}
+
+// The output of a lane's row for the first `heads` of its columns' heads, `v_dim` channels each from `dest` on; sinks: of those heads, or null
+template <int HD, int NH>
+__device__ __forceinline__ void store_columns(const Columns<HD> (&c)[NH], bool valid, int heads, const float* __restrict__ sinks, uint16_t* __restrict__ dest, int v_dim) {
+    const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+        float l = fw_quad_sum(c[h].l);
+        if (!valid || h >= heads) continue;
+        float inv = 1.0f / l;
+        if (sinks) {        // one more term in the sum, with no value: exp(sink), not scaled
+            const float sink = sinks[h] * 1.4426950408889634f;
+            const float top = fmaxf(c[h].m, sink);
+            const float shrink = exp2f(c[h].m - top);
+            inv = shrink / (l * shrink + exp2f(sink - top));
+        }
+#pragma unroll
+        for (int t = 0; t < HD / 16; ++t) {
+            if (t * 16 >= v_dim) break;
+            u32x2 packed = {pack_bf16(c[h].o[t][0] * inv, c[h].o[t][1] * inv), pack_bf16(c[h].o[t][2] * inv, c[h].o[t][3] * inv)};
+            *reinterpret_cast<u32x2*>(dest + (size_t)h * v_dim + t * 16 + g * 4) = packed;
+        }
+    }
+}
+
 template <int HD>
 __device__ __forceinline__ void load_query(Columns<HD>& c, const uint16_t* __restrict__ q_row, int head_dim, bool valid) {
     const int g = (threadIdx.x & 63) >> 4;
@@ -553,54 +608,15 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu((HD
         fw_lds_barrier();
     }
     if constexpr (PARTS > 1) {
-        // the second half leaves its maximum, sum and output to the same lane of the first
-        constexpr int VALUES = HD / 4 + 2;
-        float* left = reinterpret_cast<float*>(lds_raw) + tid;                  // [NH][VALUES][256]
+        float* left = reinterpret_cast<float*>(lds_raw) + tid;
         __syncthreads();
-        if (half == 1)
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                left[(h * VALUES + HD / 4) * 256] = c[h].m;
-                left[(h * VALUES + HD / 4 + 1) * 256] = c[h].l;
-#pragma unroll
-                for (int t = 0; t < HD / 16; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) left[(h * VALUES + t * 4 + r) * 256] = c[h].o[t][r];
-            }
+        if (half == 1) leave_columns(c, left);
         __syncthreads();
         if (half == 1) return;
-#pragma unroll
-        for (int h = 0; h < NH; ++h) {
-            const float other = left[(h * VALUES + HD / 4) * 256], top = fmaxf(c[h].m, other);
-            // (a half without any key of this row keeps NEG_BIG: its factor is 0)
-            const float mine = __builtin_amdgcn_exp2f(c[h].m - top), theirs = __builtin_amdgcn_exp2f(other - top);
-            c[h].m = top;
-            c[h].l = c[h].l * mine + left[(h * VALUES + HD / 4 + 1) * 256] * theirs;
-#pragma unroll
-            for (int t = 0; t < HD / 16; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) c[h].o[t][r] = c[h].o[t][r] * mine + left[(h * VALUES + t * 4 + r) * 256] * theirs;
-        }
+        join_columns(c, left);
     }
-#pragma unroll
-    for (int h = 0; h < NH; ++h) {
-        float l = fw_quad_sum(c[h].l);
-        if (!valid || first_in_group + h >= group) continue;
-        float inv = 1.0f / l;
-        if (sinks) {        // one more term in the sum, with no value: exp(sink), not scaled
-            const float sink = sinks[kvh * group + first_in_group + h] * 1.4426950408889634f;
-            const float top = fmaxf(c[h].m, sink);
-            const float shrink = exp2f(c[h].m - top);
-            inv = shrink / (l * shrink + exp2f(sink - top));
-        }
-        uint16_t* dest = out + ((size_t)my_row * num_heads + kvh * group + first_in_group + h) * v_dim;
-#pragma unroll
-        for (int t = 0; t < HD / 16; ++t) {
-            if (t * 16 >= v_dim) break;
-            u32x2 packed = {pack_bf16(c[h].o[t][0] * inv, c[h].o[t][1] * inv), pack_bf16(c[h].o[t][2] * inv, c[h].o[t][3] * inv)};
-            *reinterpret_cast<u32x2*>(dest + t * 16 + g * 4) = packed;
-        }
-    }
+    const int first_head = kvh * group + first_in_group;
+    store_columns(c, valid, group - first_in_group, sinks ? sinks + first_head : nullptr, out + ((size_t)my_row * num_heads + first_head) * v_dim, v_dim);
 }
 
 // ---- prompt portions, heads of 64 or 128 channels two by two ------------------------------------
@@ -930,53 +946,14 @@ __global__ __launch_bounds__(256 * PARTS) __attribute__((amdgpu_waves_per_eu(2, 
     }
     fw_mfma_drain();
     if constexpr (PARTS > 1) {
-        // the second half leaves its maximum, sum and output to the same lane of the first
-        constexpr int VALUES = HD / 4 + 2;
-        float* left = reinterpret_cast<float*>(lds_raw) + tid;                  // [NH][VALUES][256]
+        float* left = reinterpret_cast<float*>(lds_raw) + tid;
         __syncthreads();
-        if (half == 1)
-#pragma unroll
-            for (int h = 0; h < NH; ++h) {
-                left[(h * VALUES + HD / 4) * 256] = c[h].m;
-                left[(h * VALUES + HD / 4 + 1) * 256] = c[h].l;
-#pragma unroll
-                for (int t = 0; t < HD / 16; ++t)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) left[(h * VALUES + t * 4 + r) * 256] = c[h].o[t][r];
-            }
+        if (half == 1) leave_columns(c, left);
         __syncthreads();
         if (half == 1) return;
-#pragma unroll
-        for (int h = 0; h < NH; ++h) {
-            const float other = left[(h * VALUES + HD / 4) * 256], top = fmaxf(c[h].m, other);
-            // (a half without any key of this row keeps NEG_BIG: its factor is 0)
-            const float mine = __builtin_amdgcn_exp2f(c[h].m - top), theirs = __builtin_amdgcn_exp2f(other - top);
-            c[h].m = top;
-            c[h].l = c[h].l * mine + left[(h * VALUES + HD / 4 + 1) * 256] * theirs;
-#pragma unroll
-            for (int t = 0; t < HD / 16; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) c[h].o[t][r] = c[h].o[t][r] * mine + left[(h * VALUES + t * 4 + r) * 256] * theirs;
-        }
+        join_columns(c, left);
     }
-#pragma unroll
-    for (int h = 0; h < NH; ++h) {
-        float l = fw_quad_sum(c[h].l);
-        if (!valid) continue;
-        float inv = 1.0f / l;
-        if (sinks) {        // one more term in the sum, with no value: exp(sink), not scaled
-            const float sink = sinks[first_head + h] * 1.4426950408889634f;
-            const float top = fmaxf(c[h].m, sink);
-            const float shrink = exp2f(c[h].m - top);
-            inv = shrink / (l * shrink + exp2f(sink - top));
-        }
-        uint16_t* dest = out + ((size_t)my_row * num_heads + first_head + h) * HD;
-#pragma unroll
-        for (int t = 0; t < HD / 16; ++t) {
-            u32x2 packed = {pack_bf16(c[h].o[t][0] * inv, c[h].o[t][1] * inv), pack_bf16(c[h].o[t][2] * inv, c[h].o[t][3] * inv)};
-            *reinterpret_cast<u32x2*>(dest + t * 16 + g * 4) = packed;
-        }
-    }
+    store_columns(c, valid, NH, sinks ? sinks + first_head : nullptr, out + ((size_t)my_row * num_heads + first_head) * HD, HD);
 }
 
 // ---- decode ------------------------------------------------------------------------------------
