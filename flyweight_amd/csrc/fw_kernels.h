@@ -83,6 +83,13 @@ int fw_gemm_mfma_split(const void* a, const void* w, const float* bias, void* ou
 int fw_gemm_mfma_big_split_plan(int mode, int M, int N, int K, int* slices, size_t* workspace_bytes, int* counters);
 int fw_gemm_mfma_big_split(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K,
                            void* workspace, size_t workspace_bytes, int* counters, int counters_len, void* stream);
+// fw_gemm_mfma's contract on the large tile named: rows x columns (64 to 256 by 128 to 320; a gated tile has as many gate as up columns), workgroups on a compute
+// unit (2: tiles of up to 128 x 128), slices of K (more than one: storing and adding products on 64 x 128, 128 x 128 and 128 x 256). ..._needs: bytes of float32
+// workspace and int32 counters (zero before the first call, left zero), or -1 where there is no such tile or it does not take the shape. Calls with K cut that
+// overlap on one device need their own of both.
+int fw_gemm_mfma_big_tile_needs(int mode, int M, int N, int K, int rows, int columns, int each_cu, int slices, size_t* workspace_bytes, int* counters);
+int fw_gemm_mfma_big_tile(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K, int rows,
+                          int columns, int each_cu, int slices, void* workspace, size_t workspace_bytes, int* counters, int counters_len, void* stream);
 // The same product for 1..64 rows with K split over workgroups, for the shapes that fw_gemm_rows serves worse.
 // fw_gemm_medium_plan says what a shape needs: bytes of workspace (0: none) and int32 counters (0: none) that are zero before
 // the first call; the kernel leaves them zero. Calls that overlap on one device need their own of both.

@@ -583,11 +583,22 @@ def rows_fit(mode: int, M: int, N: int, K: int) -> bool:
 def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                w_tiled: Optional[torch.Tensor] = None) -> None:
     """bfloat16 operands on the matrix cores: up to 16 rows of a short K the skinny kernel; up to 64 rows, and with weights in operand tiles as long as its tiles are one
-    round over the chip, the product whose waves split K; the tiled ones beyond."""
+    round over the chip, the product whose waves split K; the tiled ones beyond, with weights in operand tiles the large tile that ``large_tile`` names."""
     M, K = a.shape
     if M <= DECODE_MAX_ROWS and skinny_takes(M, N, K):
         _check(library().fw_gemm_skinny(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, _stream()))
         return
+    if w_tiled is not None and M > MEDIUM_MAX_ROWS:
+        tile = large_tile(mode, M, N, K)
+        if tile is not None:
+            *named, need_bytes, need_counters = tile
+            workspace = counters = None
+            if need_bytes:
+                workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
+                counters = _medium_counters(a.device, need_counters)
+            _check(library().fw_gemm_mfma_big_tile(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, *named, _p(workspace), need_bytes, _p(counters),
+                                                   need_counters, _stream()))
+            return
     if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and rows_fit(mode, M, N, K)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
             gemm_medium_into(a, w, bias, target, BF16, mode, N, w_tiled=w_tiled, glu=GEGLU)
@@ -656,13 +667,8 @@ def _tiled_time(tiles: int, K: int, start: float, each_round: float, each_tile: 
             + K / 1024 * (rounds * walk + share * fill + pairs * walk_pair))
 
 
-@functools.lru_cache(maxsize=4096)
-def tiled_plan(mode: int, M: int, N: int, K: int):
-    """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
-    256 columns), "bigsplit" (128 rows by 256, K cut over workgroups), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through
-    registers), "split" (those with K cut over workgroups). The least estimated time decides. Fixed numbers of
-    tiles were 10 % above the fastest in the geometric mean, adding products of up to 2,048 features held to the tiles whose waves split K 5 %; K cut
-    over workgroups takes 1,111 rows by 2,048 features over K 8,192 in 50 us against 60 on the tiles whose waves split K."""
+def _tiled_times(mode: int, M: int, N: int, K: int):
+    """The estimated time of every product on tiles of both operands that takes the shape, by (kind, columns)."""
     lib = library()
     wide, narrow = -(-M // 128) * -(-N // 128), -(-M // 128) * -(-N // 64)
     columns = 64 if mode == 2 or wide < DEEP_ROUND or (wide == DEEP_ROUND and K < LONG_K) else 128        # as fw_gemm_mfma chooses
@@ -697,7 +703,88 @@ def tiled_plan(mode: int, M: int, N: int, K: int):
             start, each, all_at_once, walk, fill = _TIME_BIG_SPLIT[mode]
             share = tiles * slices / DEEP_ROUND
             times["bigsplit", 0] = start + each * slices + share * all_at_once + K / 1024 / slices * (walk + fill * share)
+    return times
+
+
+@functools.lru_cache(maxsize=4096)
+def tiled_plan(mode: int, M: int, N: int, K: int):
+    """Which of the products on tiles of both operands takes a shape, as (kind, columns of its tiles or 0): "big" (256 or 128 rows by up to
+    256 columns), "bigsplit" (128 rows by 256, K cut over workgroups), "deep" (128 rows by 128 or 64, the waves split K), "tiles" (128 rows, through
+    registers), "split" (those with K cut over workgroups). The least estimated time decides. Fixed numbers of
+    tiles were 10 % above the fastest in the geometric mean, adding products of up to 2,048 features held to the tiles whose waves split K 5 %; K cut
+    over workgroups takes 1,111 rows by 2,048 features over K 8,192 in 50 us against 60 on the tiles whose waves split K."""
+    times = _tiled_times(mode, M, N, K)
     return min(times, key=times.get)
+
+
+# The large tiles one by one, us, by (rows, columns, workgroups on a compute unit): start + rounds * round + tiles / 256 * tile + K / 1,024 * (rounds * walk +
+# tiles / 256 * fill) + MB of weights * memory, rounds those of the tiles over the 256 compute units (over 512 places where two workgroups share one). Fitted to
+# 420 shapes a mode (65 to 4,096 rows by 64 to 14,000 features over K 256 to 10,752, the weights from memory, no launch in the time) to 2.4 to 11 % (mean square).
+_TIME_LARGE = {
+    0: {(64, 128, 1): (1.479, 2.7, 0.387, 3.672, 1.243, 0.132), (64, 128, 2): (2.751, 0.488, 0.848, 3.974, 2.614, 0.122), (128, 128, 1): (2.133, 2.631, 1.925, 5.279, 1.699, 0.102),
+        (128, 128, 2): (3.379, 0.0, 2.127, 6.304, 3.248, 0.071), (192, 128, 1): (2.607, 2.755, 2.626, 7.1, 2.099, 0.048), (64, 192, 1): (1.898, 2.731, 0.665, 4.762, 1.757, 0.176),
+        (128, 192, 1): (2.073, 3.337, 1.99, 7.08, 1.83, 0.124), (128, 256, 1): (2.277, 3.438, 2.524, 8.98, 2.227, 0.135), (192, 192, 1): (2.267, 3.91, 3.176, 9.708, 2.078, 0.042),
+        (192, 256, 1): (1.621, 5.112, 3.981, 12.299, 2.613, 0.049), (256, 192, 1): (1.774, 4.865, 3.937, 12.25, 2.695, 0.032), (256, 256, 1): (1.564, 6.259, 5.049, 15.86, 3.458, 0.02),
+        (256, 320, 1): (0.0, 8.431, 3.819, 20.043, 4.24, 0.163)},
+    1: {(64, 128, 1): (1.548, 2.711, 0.962, 3.716, 1.22, 0.147), (64, 128, 2): (2.46, 0.722, 1.346, 4.101, 2.628, 0.134), (128, 128, 1): (1.304, 3.83, 2.21, 5.427, 1.382, 0.115),
+        (128, 128, 2): (1.934, 1.583, 3.413, 6.501, 2.787, 0.08), (192, 128, 1): (0.752, 5.218, 3.532, 7.165, 1.608, 0.073), (64, 192, 1): (1.554, 3.171, 1.097, 4.877, 1.585, 0.206),
+        (128, 192, 1): (1.169, 4.72, 2.821, 7.253, 1.656, 0.135), (128, 256, 1): (1.68, 4.487, 5.011, 9.231, 1.665, 0.151), (192, 192, 1): (1.434, 5.569, 5.932, 9.822, 1.757, 0.049),
+        (192, 256, 1): (0.797, 7.165, 7.688, 12.428, 2.505, 0.053), (256, 192, 1): (0.951, 6.927, 7.95, 12.431, 2.596, 0.003), (256, 256, 1): (0.0, 9.246, 10.769, 16.027, 3.126, 0.002),
+        (256, 320, 1): (0.0, 10.509, 10.441, 20.3, 3.87, 0.144)},
+    2: {(64, 128, 1): (1.537, 2.467, 0.0, 3.851, 1.227, 0.112), (64, 128, 2): (2.328, 0.577, 0.346, 4.133, 2.77, 0.106), (128, 128, 1): (1.606, 3.179, 0.278, 5.465, 1.516, 0.095),
+        (128, 128, 2): (1.835, 1.195, 0.853, 6.48, 3.039, 0.082), (192, 128, 1): (1.821, 3.503, 0.574, 7.149, 1.813, 0.069), (64, 192, 1): (1.519, 2.702, 0.0, 5.07, 1.556, 0.141),
+        (128, 192, 1): (1.393, 3.791, 0.244, 7.286, 1.741, 0.105), (128, 256, 1): (1.358, 3.944, 0.448, 9.29, 1.927, 0.109), (192, 192, 1): (1.796, 4.198, 0.672, 9.826, 1.84, 0.058),
+        (192, 256, 1): (1.5, 5.095, 0.671, 12.494, 2.431, 0.049), (256, 192, 1): (1.514, 5.132, 0.447, 12.374, 2.544, 0.037), (256, 256, 1): (1.951, 5.817, 1.116, 15.924, 3.445, 0.013),
+        (256, 320, 1): (1.562, 6.131, 1.696, 20.857, 3.561, 0.095)}}
+# ... with K cut over workgroups: start, a slice's part in the sum at the end, 256 workgroups, 1,024 k of a slice and for 256 workgroups, MB of weights
+_TIME_LARGE_CUT = {0: {(64, 128): (5.054, 0.448, 4.393, 3.678, 0.047, 0.083), (128, 128): (6.172, 0.703, 6.135, 5.315, 0.43, 0.068)},
+                   1: {(64, 128): (6.096, 0.4, 3.895, 3.5, 0.874, 0.069), (128, 128): (7.824, 0.499, 5.709, 5.176, 0.861, 0.069)}}
+# ... of the product whose waves split K (fw_gemm_rows): start, 1,024 k, and for 256 rows, for 4,096 rows of W, a million outputs, and 1,024 k of them
+_TIME_ROWS = {0: (3.585, 0.562, 0.112, 1.194, 4.492, 3.142), 1: (3.719, 0.601, 0.108, 1.152, 4.71, 2.926),
+              2: (4.209, 0.786, 0.139, 1.173, 3.606, 2.155)}
+_TIME_OLDER = 1.05       # what the products of `_tiled_times` took of those shapes, by their estimates
+_LARGE_LEAST_SLICE = 384     # k
+
+
+@functools.lru_cache(maxsize=4096)
+def large_tile(mode: int, M: int, N: int, K: int):
+    """The large tile that takes a product of more than 64 rows by weights that a model holds (they come with their operand tiles; a bare product keeps to
+    ``tiled_plan``, whose sums its callers know by the kernel's name): (rows, columns, workgroups on a compute unit, slices of K, bytes of workspace, counters),
+    or None where the product whose waves split K or one of ``tiled_plan`` is estimated to be faster. Chosen so, the 420 shapes a mode take 1.8 (storing,
+    adding) and 1.0 % (gated) more than with the fastest product each, and 12, 13 and 26 % less than without these tiles; no shape loses more than 15 %
+    (adding 2,048 x 1,024 over K 1,024 13.3 -> 10.3 us, 801 x 2,048 over 7,168 43.3 -> 36.1, gated 500 x 4,608 over 1,024 24.8 -> 16.4, 2,048 x 4,608 55 -> 38)."""
+    if K % 32 or K > 1 << 22 or N > 1 << 20:
+        return None
+    k, megabytes = K / 1024, N * (2 if mode == 2 else 1) * K * 2e-6
+    best, least = None, 1e30
+    for (rows, columns, each), (start, each_round, each_tile, walk, fill, memory) in _TIME_LARGE[mode].items():
+        tiles = -(-M // rows) * -(-N // (columns // 2 if mode == 2 else columns))
+        rounds, share = -(-tiles // (DEEP_ROUND * each)), tiles / DEEP_ROUND
+        if mode == 2 and N % 2:
+            each_round += _TIME_BIG_ODD
+        time = start + rounds * each_round + share * each_tile + k * (rounds * walk + share * fill) + megabytes * memory
+        if time < least:
+            best, least = (rows, columns, each, 1), time
+    for (rows, columns), (start, each_slice, all_at_once, walk, fill, memory) in _TIME_LARGE_CUT.get(mode, {}).items():
+        tiles = -(-M // rows) * -(-N // columns)
+        for slices in range(2, 9):
+            if tiles * slices > DEEP_ROUND or K < slices * _LARGE_LEAST_SLICE:
+                break
+            share = tiles * slices / DEEP_ROUND
+            time = start + slices * each_slice + share * all_at_once + k / slices * (walk + fill * share) + megabytes * memory
+            if time < least and -(-K // slices // 64) * 64 * (slices - 1) < K:
+                best, least = (rows, columns, 1, slices), time
+    if rows_fit(mode, M, N, K):
+        start, walk, by_rows, by_width, outputs, by_outputs = _TIME_ROWS[mode]
+        width = N * (2 if mode == 2 else 1)
+        other = start + k * (walk + by_rows * M / 256 + by_width * width / 4096) + M * width * 1e-6 * (outputs + by_outputs * k)
+    else:
+        other = _TIME_OLDER * min(_tiled_times(mode, M, N, K).values())
+    if other <= least:
+        return None
+    need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
+    _check(library().fw_gemm_mfma_big_tile_needs(mode, M, N, K, *best, ctypes.byref(need_bytes), ctypes.byref(need_counters)))
+    return (*best, need_bytes.value, need_counters.value)
 
 
 MEDIUM_MAX_ROWS = 64
