@@ -437,6 +437,10 @@ int fw_moe_arrange(const int32_t* chosen, int32_t* expert_begin, int32_t* place_
 int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                     const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
                     float glu_limit, float glu_alpha, float glu_shift, void* stream);
+// The same for steps of a few places an expert: bfloat16 a and w, w's rows [experts * N, or 2 N][K] in operand tiles (K a multiple of 32), out bfloat16 (gated)
+// or float32.
+int fw_grouped_gemm_few(const void* a, const int32_t* place_row, const void* w_tiled, const int32_t* expert_begin, void* out, int gated, int places,
+                        int experts, int N, int K, int place_tiles, float glu_limit, float glu_alpha, float glu_shift, void* stream);
 // 1: with bfloat16 operands, the plain unit and an output of bfloat16 (gated) or float32 the large tiles take it
 int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int experts, int N, int K);
 // x[r] += sum_j weight[r][j] * y[pair_place[r][j]], j in order, and with b (null: none) + sigmoid(gate[r * gate_stride]) b[r]; float32

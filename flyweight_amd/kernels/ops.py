@@ -838,6 +838,18 @@ def tile_weights(w: torch.Tensor) -> Optional[torch.Tensor]:
     return w.view(padded // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
 
 
+def tile_expert_weights(w: torch.Tensor) -> Optional[torch.Tensor]:
+    """The experts' stacked weights [experts, rows, K] once more in operand tiles, for steps of a few places an expert; None where the layout does not apply
+    or the copy would leave less than half of the device's memory free (experts are most of a large mixture's weights)."""
+    if not w.is_cuda or w.dtype != torch.bfloat16 or w.shape[2] % 32:
+        return None
+    free, total = torch.cuda.mem_get_info(w.device)
+    reserved = torch.cuda.memory_reserved(w.device) - torch.cuda.memory_allocated(w.device)
+    if free + reserved - w.numel() * w.element_size() < total // 2:
+        return None
+    return tile_weights(w.view(-1, w.shape[2]))
+
+
 def _tiled_for(w: torch.Tensor, w_tiled: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``w_tiled`` if it is ``w`` in operand tiles (checked by its shape), else an error."""
     if w_tiled is None:
@@ -2083,11 +2095,20 @@ def moe_arrange(chosen: torch.Tensor, experts: int):
     return expert_begin, place_row, pair_place
 
 
+def grouped_few_tiles(places: int, experts: int) -> int:
+    """Tiles of 16 places to a workgroup of the grouped product whose experts' weights come in operand tiles (fw_grouped_gemm_few), 0 where the tiles
+    of moe.hip and gemm_mfma_big.hip are faster. By places an expert in the mean, us for both products (those tiles / one / two): 32 experts of 1,536 features over 2,048,
+    4 a row, 1 / 8 / 32 / 64 / 96 / 128 rows 37 / 21 / 23, 87 / 65 / 67, 122 / 95 / 97, 126 / 101 / 103, 127 / 112 / 109, 128 / 145 / 118; 8 of 4,096 over 2,048, 2 a row, 8 / 32 /
+    64 / 128 rows 95 / 58 / 63, 108 / 73 / 78, 109 / 94 / 86, 112 / 153 / 149."""
+    return 1 if places <= 8 * experts else 2 if places <= 16 * experts else 0
+
+
 def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: torch.Tensor, expert_begin: torch.Tensor, places: int,
-                 gated: bool, out_dtype: torch.dtype, glu: Optional[tuple] = None) -> torch.Tensor:
+                 gated: bool, out_dtype: torch.dtype, glu: Optional[tuple] = None, w_tiled: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[place] = a[place_row[place]] . w[expert of place]^T (``place_row`` None: a[place]); ``w`` [experts, N, K], or
     with ``gated`` [experts, 2 N, K] (gate rows, then up rows) and out = silu(gate) * up, or with ``glu`` = (limit, alpha,
-    shift) the unit with clamped halves. Returns [places, N]."""
+    shift) the unit with clamped halves. ``w_tiled``: the rows of ``w`` [experts * N, K] once more in operand tiles
+    (``tile_weights``), for steps of a few places an expert. Returns [places, N]."""
     _dev(a, place_row, w, expert_begin)
     experts, n_rows, K = w.shape
     N = n_rows // 2 if gated else n_rows
@@ -2101,6 +2122,13 @@ def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: torch.Te
     elif a.shape[0] < places:
         raise KernelError("grouped_gemm: fewer rows than places")
     out = torch.empty((places, N), dtype=out_dtype, device=a.device)
+    if w_tiled is not None and a.dtype == torch.bfloat16 and out_dtype == (torch.bfloat16 if gated else torch.float32) and a.data_ptr() % 16 == 0:
+        place_tiles = grouped_few_tiles(places, experts)
+        if place_tiles:
+            w_tiled = _tiled_for(w.view(experts * n_rows, K), w_tiled)
+            _check(library().fw_grouped_gemm_few(_p(a), _p(place_row), _p(w_tiled), _p(expert_begin), _p(out), int(gated), int(places), experts, N, K, place_tiles,
+                                                 *_glu(glu if gated else None), _stream()))
+            return out
     _check(library().fw_grouped_gemm(_p(a), _code(a.dtype), a.shape[0], _p(place_row), _p(w), _code(w.dtype), _p(expert_begin), _p(out),
                                      _code(out_dtype), int(gated), int(places), experts, N, K, *_glu(glu if gated else None), _stream()))
     return out

@@ -124,12 +124,13 @@ class MoeSwiGLU(FeedForward):
         self.gate_up = torch.stack([torch.cat([tensors[self._expert(e, "gate")], tensors[self._expert(e, "up")]], dim=0)
                                     for e in range(self.experts)]).contiguous()
         self.down = torch.stack([tensors[self._expert(e, "down")] for e in range(self.experts)]).contiguous()
+        self.gate_up_tiled, self.down_tiled = ops.tile_expert_weights(self.gate_up), ops.tile_expert_weights(self.down)
         if self.shared is not None:
             self.shared.bind(tensors, dtype, device)
 
     # ----- what a step reads and computes (the experts' weights are read only where tokens chose them) --------
     def gathered_tensors(self):
-        return (self.gate_up, self.down)
+        return tuple(t for t in (self.gate_up, self.down, self.gate_up_tiled, self.down_tiled) if t is not None)
 
     def chosen_weight_bytes(self, rows: int) -> float:
         """Bytes of the experts that ``rows`` tokens are expected to choose, each ``top`` different ones and
@@ -161,8 +162,9 @@ class MoeSwiGLU(FeedForward):
         chosen, weight = self._choose(logits)
         begin, place_row, pair_place = ops.moe_arrange(chosen, self.experts)
         places = rows.shape[0] * self.top
-        hidden = ops.grouped_gemm(rows, place_row, self.gate_up, begin, places, gated=True, out_dtype=rows.dtype, glu=self.glu)
-        return ops.grouped_gemm(hidden, None, self.down, begin, places, gated=False, out_dtype=torch.float32), weight, pair_place, gate
+        hidden = ops.grouped_gemm(rows, place_row, self.gate_up, begin, places, gated=True, out_dtype=rows.dtype, glu=self.glu, w_tiled=self.gate_up_tiled)
+        outputs = ops.grouped_gemm(hidden, None, self.down, begin, places, gated=False, out_dtype=torch.float32, w_tiled=self.down_tiled)
+        return outputs, weight, pair_place, gate
 
     def _shared_output(self, h, rows, ctx):
         if self.shared is None:
