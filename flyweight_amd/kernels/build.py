@@ -15,6 +15,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import time
 import zlib
@@ -261,6 +262,56 @@ def ensure_host_built() -> str:
         raise
 
 
+# ----- the launches of a prompt's step as a Python module: host code over torch's headers ---------------
+LAUNCH_SOURCE = os.path.join(CSRC, "launch", "launch.cpp")
+LAUNCH_NAME = "fw_launch"
+
+
+def _launch_command() -> List[str]:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    return ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-I{root}/include", f"-I{root}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", LAUNCH_SOURCE,
+            f"-L{root}/lib", "-lc10", "-ltorch_cpu", "-ltorch_python", f"-Wl,-rpath,{root}/lib"]
+
+
+def _launch_fingerprint() -> str:
+    import torch
+    digest = hashlib.sha256()
+    for path in (LAUNCH_SOURCE, HEADER):
+        with open(path, "rb") as handle:
+            digest.update(handle.read())
+    digest.update(" ".join([torch.__version__, sys.version, *_launch_command()[:6]]).encode())
+    return digest.hexdigest()
+
+
+def build_launch(verbose: bool = True) -> str:
+    folder = _writable_dir()
+    started = time.time()
+    lib = os.path.join(folder, LAUNCH_NAME + ".so")
+    partial = lib + f".{os.getpid()}.tmp"
+    result = subprocess.run([_host_compiler(), *_launch_command(), "-o", partial], capture_output=True, text=True)
+    if result.returncode != 0:
+        raise RuntimeError(f"building {LAUNCH_NAME} failed:\n{result.stderr}")
+    os.replace(partial, lib)
+    with open(os.path.join(folder, "launch.stamp"), "w", encoding="utf-8") as handle:
+        handle.write(_launch_fingerprint())
+    if verbose:
+        _say(f"built {lib} in {time.time() - started:.0f} s")
+    return lib
+
+
+def ensure_launch_built() -> str:
+    wanted = _launch_fingerprint()
+    for folder in build_dirs():
+        lib, stamp = os.path.join(folder, LAUNCH_NAME + ".so"), os.path.join(folder, "launch.stamp")
+        if os.path.isfile(lib) and os.path.isfile(stamp):
+            with open(stamp, "r", encoding="utf-8") as handle:
+                if handle.read().strip() == wanted:
+                    return lib
+    return build_launch()
+
+
 # ----- the plain C++ references of the kernels: host code, for tests ------------------------------
 REFERENCE_DIR = os.path.join(CSRC, "reference")
 REFERENCE_LIB_NAME = "libflyweight_reference.so"
@@ -308,4 +359,5 @@ def ensure_reference_built() -> str:
 if __name__ == "__main__":
     build()
     build_host()
+    build_launch()
     build_reference()

@@ -9,8 +9,11 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import importlib.util
 import os
+import sys
 import time
+import warnings
 from typing import Dict, Optional
 
 import torch
@@ -128,10 +131,40 @@ def library():
             raise KernelError(f"{path}: kernel library ABI {lib.fw_abi_version()} != {wanted}; rebuild it")
         _declare(lib)
         _lib = lib
+        _load_native(lib)
         if os.environ.get("FLYWEIGHT_KERNEL_PROFILE", "")[:1] == "1":
             kernel_profile(True)
             return _profiled
     return _lib
+
+
+# The launches of a prompt's step as functions of a native module (csrc/launch): checks, allocations and the call in one. The general paths below serve whatever
+# it hands back (NotImplemented), everything while kernels are timed one by one, and everything where it could not be built.
+_native = None
+_NATIVE_ENTRIES = ("fw_gemm_rows", "fw_gemm_medium", "fw_gemm_mfma_big_tile", "fw_rmsnorm_rows", "fw_shortconv", "fw_qk_norm_rope_kv_write", "fw_attention_prefill",
+                   "fw_last_error")
+
+
+def _load_native(lib) -> None:
+    global _native
+    _native = None
+    module = sys.modules.get(_build.LAUNCH_NAME)
+    if module is None:
+        try:
+            spec = importlib.util.spec_from_file_location(_build.LAUNCH_NAME, _build.ensure_launch_built())
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+        except (RuntimeError, OSError, ImportError) as error:
+            warnings.warn(f"the native launches cannot be had; steps with prompts take longer on the host: {error}")
+            return
+        sys.modules[_build.LAUNCH_NAME] = module
+    module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _NATIVE_ENTRIES}, KernelError, torch.OutOfMemoryError)
+    _native = module
+
+
+def native_launches() -> bool:
+    """Whether launches go through the native module."""
+    return _native is not None and _profiled is None
 
 
 def library_path() -> str:
@@ -140,7 +173,7 @@ def library_path() -> str:
 
 
 def _check(status: int) -> None:
-    if status != 0:
+    if status:
         raise KernelError(library().fw_last_error().decode("utf-8", "replace"))
 
 
@@ -154,12 +187,8 @@ def _code(dtype: torch.dtype) -> int:
 
 def _dev(*tensors: Optional[torch.Tensor]) -> None:
     for t in tensors:
-        if t is None:
-            continue
-        if not t.is_cuda:
-            raise KernelError("kernels run on the GPU only; got a CPU tensor")
-        if not t.is_contiguous():
-            raise KernelError("kernels need contiguous tensors")
+        if t is not None and not (t.is_cuda and t.is_contiguous()):
+            raise KernelError("kernels need contiguous tensors" if t.is_cuda else "kernels run on the GPU only; got a CPU tensor")
 
 
 def _dev_rows(t: torch.Tensor, name: str) -> None:
@@ -233,6 +262,10 @@ def scale_softcap_(x: torch.Tensor, scale: float = 1.0, cap: float = 0.0) -> tor
 def rmsnorm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.dtype,
                  row_index: Optional[torch.Tensor] = None, one_centered: bool = False,
                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    if _native is not None and _profiled is None and out is None and x.is_cuda and (out_dtype == torch.bfloat16 or out_dtype == torch.float32):
+        made = _native.rmsnorm(x, weight, row_index, out_dtype == torch.bfloat16, eps, one_centered, _stream())
+        if made is not NotImplemented:
+            return made
     _dev(x, weight, row_index, out)
     _want(x, torch.float32, "x")
     _want(weight, torch.float32, "weight")
@@ -243,11 +276,11 @@ def rmsnorm_rows(x: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: t
     if row_index is not None:
         _want(row_index, torch.int32, "row_index")
     if out is None:
-        out = torch.empty((rows, hidden), dtype=out_dtype, device=x.device)
-    if out.shape != (rows, hidden) or out.dtype != out_dtype:
+        out = torch.empty(rows, hidden, dtype=out_dtype, device=x.device)
+    elif out.shape != (rows, hidden) or out.dtype != out_dtype:
         raise KernelError("rmsnorm: out has the wrong shape or dtype")
-    _check(library().fw_rmsnorm_rows(_p(x), _p(weight), _p(out), _code(out_dtype), _p(row_index), rows, hidden,
-                                     float(eps), int(one_centered), _stream()))
+    _check(library().fw_rmsnorm_rows(x.data_ptr(), weight.data_ptr(), out.data_ptr(), _code(out_dtype), _p(row_index), rows, hidden, float(eps), 1 if one_centered else 0,
+                                     _stream()))
     return out
 
 
@@ -365,6 +398,10 @@ def shortconv(bcx: torch.Tensor, taps: torch.Tensor, conv_bias: Optional[torch.T
               out_dtype: Optional[torch.dtype] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """state [slots, H, L-1] is read and updated in place. ``bcx`` may be float32 beside a
     bfloat16 output."""
+    if _native is not None and _profiled is None and out is None and bcx.is_cuda and (out_dtype == torch.bfloat16 or out_dtype == torch.float32):
+        made = _native.shortconv(bcx, taps, conv_bias, state, row_seg, seg_row0, seg_slot, segments, out_dtype == torch.bfloat16, _stream())
+        if made is not NotImplemented:
+            return made
     _dev(bcx, taps, conv_bias, state, row_seg, seg_row0, seg_slot, out)
     out_dtype = out_dtype or bcx.dtype
     rows, width = bcx.shape
@@ -379,16 +416,18 @@ def shortconv(bcx: torch.Tensor, taps: torch.Tensor, conv_bias: Optional[torch.T
         _want(conv_bias, torch.float32, "conv_bias")
         if conv_bias.shape != (hidden,):
             raise KernelError("shortconv: bias has the wrong shape")
-    for name, t, n in (("row_seg", row_seg, rows), ("seg_row0", seg_row0, segments + 1), ("seg_slot", seg_slot, segments)):
-        _want(t, torch.int32, name)
-        if t.numel() < n:
-            raise KernelError(f"shortconv: {name} holds {t.numel()} entries, needs {n}")
+    if (row_seg.dtype != torch.int32 or seg_row0.dtype != torch.int32 or seg_slot.dtype != torch.int32 or row_seg.numel() < rows
+            or seg_row0.numel() <= segments or seg_slot.numel() < segments):
+        for name, t, n in (("row_seg", row_seg, rows), ("seg_row0", seg_row0, segments + 1), ("seg_slot", seg_slot, segments)):
+            _want(t, torch.int32, name)
+            if t.numel() < n:
+                raise KernelError(f"shortconv: {name} holds {t.numel()} entries, needs {n}")
     if out is None:
-        out = torch.empty((rows, hidden), dtype=out_dtype, device=bcx.device)
-    if out.shape != (rows, hidden) or out.dtype != out_dtype:
+        out = torch.empty(rows, hidden, dtype=out_dtype, device=bcx.device)
+    elif out.shape != (rows, hidden) or out.dtype != out_dtype:
         raise KernelError("shortconv: out has the wrong shape or dtype")
-    _check(library().fw_shortconv(_p(bcx), _code(bcx.dtype), _p(out), _code(out_dtype), _p(taps), _p(conv_bias), _p(state), _p(row_seg),
-                                  _p(seg_row0), _p(seg_slot), rows, segments, hidden, kernel, state.shape[0], _stream()))
+    _check(library().fw_shortconv(bcx.data_ptr(), _code(bcx.dtype), out.data_ptr(), _code(out_dtype), taps.data_ptr(), _p(conv_bias), state.data_ptr(),
+                                  row_seg.data_ptr(), seg_row0.data_ptr(), seg_slot.data_ptr(), rows, segments, hidden, kernel, state.shape[0], _stream()))
     return out
 
 
@@ -417,6 +456,11 @@ def qk_norm_rope_kv_write(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, 
     ``q_row_scale`` (float32 [rows]): a factor on each row's finished queries.
     ``v_dim``: the size of a value head where it is not ``head_dim``. ``interleaved``: channel 2i turns
     with channel 2i + 1 instead of channel i with channel i + rotary_dim / 2."""
+    if _native is not None and _profiled is None and qkv.is_cuda:
+        made = _native.qk_norm(qkv, num_heads, num_kv_heads, head_dim, q_norm_weight, k_norm_weight, eps, cos, sin, rotary_dim, k_pages, v_pages, block_table, row_seg,
+                               row_pos, write_kv, head_dim if v_dim is None else v_dim, interleaved, q_only, q_row_scale, PAGE_SIZE, _stream())
+        if made is not NotImplemented:
+            return made
     _dev(q_norm_weight, k_norm_weight, cos, sin, k_pages, v_pages, block_table, row_seg, row_pos)
     _dev_rows(qkv, "qkv")
     rows, width = qkv.shape
@@ -591,13 +635,13 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     if w_tiled is not None and M > MEDIUM_MAX_ROWS:
         tile = large_tile(mode, M, N, K)
         if tile is not None:
-            *named, need_bytes, need_counters = tile
-            workspace = counters = None
+            rows, columns, each, slices, need_bytes, need_counters = tile
+            workspace_at = counters_at = None
             if need_bytes:
                 workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
-                counters = _medium_counters(a.device, need_counters)
-            _check(library().fw_gemm_mfma_big_tile(_p(a), _p(w), _p(bias), _p(target), out_code, mode, M, N, K, *named, _p(workspace), need_bytes, _p(counters),
-                                                   need_counters, _stream()))
+                workspace_at, counters_at = workspace.data_ptr(), _medium_counters(a.device, need_counters).data_ptr()
+            _check(library().fw_gemm_mfma_big_tile(a.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), target.data_ptr(), out_code, mode, M, N, K,
+                                                   rows, columns, each, slices, workspace_at, need_bytes, counters_at, need_counters, _stream()))
             return
     if M <= MEDIUM_MAX_ROWS or (w_tiled is not None and rows_fit(mode, M, N, K)):
         if out_code == BF16_GEGLU:      # that product is told by its unit, not by the output's type
@@ -850,13 +894,18 @@ def tile_expert_weights(w: torch.Tensor) -> Optional[torch.Tensor]:
     return tile_weights(w.view(-1, w.shape[2]))
 
 
+@functools.lru_cache(maxsize=4096)
+def _tiled_shape(rows: int, K: int) -> Optional[torch.Size]:
+    return None if K % 32 else torch.Size(((rows + 15) // 16, K // 32, 4, 16, 8))
+
+
 def _tiled_for(w: torch.Tensor, w_tiled: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     """``w_tiled`` if it is ``w`` in operand tiles (checked by its shape), else an error."""
     if w_tiled is None:
         return None
     rows, K = w.shape
-    if (w_tiled.dtype != torch.bfloat16 or K % 32 or tuple(w_tiled.shape) != ((rows + 15) // 16, K // 32, 4, 16, 8)
-            or not w_tiled.is_contiguous() or w_tiled.device != w.device):
+    if (w_tiled.dtype != torch.bfloat16 or w_tiled.shape != _tiled_shape(rows, K) or not w_tiled.is_contiguous()
+            or w_tiled.get_device() != w.get_device()):
         raise KernelError(f"weights in operand tiles for w {tuple(w.shape)} are bfloat16 [{(rows + 15) // 16}, {K // 32}, 4, 16, 8], "
                           f"found {tuple(w_tiled.shape)}")
     return w_tiled
@@ -910,6 +959,16 @@ def _medium_plan(mode: int, M: int, N: int, K: int):
     return need_bytes.value, need_counters.value, squares_rows.value
 
 
+@functools.lru_cache(maxsize=4096)
+def _few_plan(mode: int, M: int, N: int, K: int):
+    """Of a product of a few dozen rows: whether K is split over workgroups, then its bytes of workspace, counters and rows of sums of squares, and the rows
+    of sums of squares of the kernel whose waves split K."""
+    squares_rows = library().fw_gemm_rows_square_tiles(M, N)
+    if M <= MEDIUM_MAX_ROWS and medium_splits_k(mode, M, N, K):
+        return (True, *_medium_plan(mode, M, N, K), squares_rows)
+    return False, 0, 0, 0, squares_rows
+
+
 def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out_code: int, mode: int, N: int,
                      next_norm_weight: Optional[torch.Tensor] = None, next_one_centered: bool = False,
                      squares: Optional[torch.Tensor] = None, eps: float = 0.0, w_tiled: Optional[torch.Tensor] = None,
@@ -919,37 +978,83 @@ def gemm_medium_into(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tenso
     formed from those sums. With ``next_norm_weight`` (accumulating product) returns what the
     norm after it needs: (activations x * w_next, sums of squares)."""
     M, K = a.shape
-    next_activations = next_squares = None
     stride = 16 if M <= DECODE_MAX_ROWS else 64
-    if squares is not None and (squares.dtype != torch.float32 or squares.dim() != 2 or squares.shape[1] != stride
-                                or not squares.is_contiguous()):
-        raise KernelError(f"gemm_medium: sums of squares for {M} rows are float32 [n, {stride}]")
-    squares_rows = 0 if squares is None else squares.shape[0]
-    w_tiled = _tiled_for(w, w_tiled)
-    operand = w if w_tiled is None else w_tiled
-    splits_k = M <= MEDIUM_MAX_ROWS and medium_splits_k(mode, M, N, K) and target.data_ptr() % 16 == 0
-    if splits_k:
-        need_bytes, need_counters, prepared_rows = _medium_plan(mode, M, N, K)
+    squares_at, squares_rows = None, 0
+    if squares is not None:
+        if squares.dtype != torch.float32 or squares.dim() != 2 or squares.shape[1] != stride or not squares.is_contiguous():
+            raise KernelError(f"gemm_medium: sums of squares for {M} rows are float32 [n, {stride}]")
+        squares_at, squares_rows = squares.data_ptr(), squares.shape[0]
+    operand, tiled = (w, 0) if w_tiled is None else (_tiled_for(w, w_tiled), 1)
+    splits_k, need_bytes, need_counters, prepared_rows, whole_rows = _few_plan(mode, M, N, K)
+    target_at = target.data_ptr()
+    splits_k = splits_k and target_at % 16 == 0
+    next_activations = next_squares = weight_at = activations_at = next_at = None
     if next_norm_weight is not None:
-        rows = prepared_rows if splits_k else library().fw_gemm_rows_square_tiles(M, N)
-        next_activations = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-        next_squares = torch.empty((rows, stride), dtype=torch.float32, device=a.device)
+        device = a.device
+        next_activations = torch.empty(M, N, dtype=torch.bfloat16, device=device)
+        next_squares = torch.empty(prepared_rows if splits_k else whole_rows, stride, dtype=torch.float32, device=device)
+        weight_at, activations_at, next_at = next_norm_weight.data_ptr(), next_activations.data_ptr(), next_squares.data_ptr()
+    bias_at = None if bias is None else bias.data_ptr()
+    limit, alpha, shift = _SWIGLU if glu is None else _glu(glu)
     if splits_k:
-        workspace = counters = None
+        workspace_at = counters_at = None
+        counters_len = 0
         if need_bytes:
             workspace = torch.empty(need_bytes // 4, dtype=torch.float32, device=a.device)
             counters = _medium_counters(a.device, need_counters)
-        _check(library().fw_gemm_medium(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
-                                        _p(workspace), need_bytes, _p(counters), 0 if counters is None else counters.numel(),
-                                        _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
-                                        squares_rows, float(eps), *_glu(glu), _stream()))
+            workspace_at, counters_at, counters_len = workspace.data_ptr(), counters.data_ptr(), counters.numel()
+        _check(library().fw_gemm_medium(a.data_ptr(), operand.data_ptr(), tiled, bias_at, target_at, out_code, mode, M, N, K,
+                                        workspace_at, need_bytes, counters_at, counters_len, weight_at, 1 if next_one_centered else 0, activations_at, next_at,
+                                        squares_at, squares_rows, float(eps), limit, alpha, shift, _stream()))
     else:
-        _check(library().fw_gemm_rows(_p(a), _p(operand), int(w_tiled is not None), _p(bias), _p(target), out_code, mode, M, N, K,
-                                      _p(next_norm_weight), int(next_one_centered), _p(next_activations), _p(next_squares), _p(squares),
-                                      squares_rows, float(eps), *_glu(glu), _stream()))
+        _check(library().fw_gemm_rows(a.data_ptr(), operand.data_ptr(), tiled, bias_at, target_at, out_code, mode, M, N, K,
+                                      weight_at, 1 if next_one_centered else 0, activations_at, next_at, squares_at, squares_rows, float(eps), limit, alpha, shift,
+                                      _stream()))
     if next_norm_weight is not None:
         return next_activations, next_squares
     return None
+
+
+@functools.lru_cache(maxsize=8192)
+def _native_plan(few: bool, tiled: bool, mode: int, M: int, N: int, K: int):
+    """How the native module launches a product: (0, *_few_plan) or (1, *large_tile), None for the general path. ``few``: the product of a few dozen rows was
+    asked for by name."""
+    if K % 8 or M < 1:
+        return None
+    if not few:
+        if M <= DECODE_MAX_ROWS and skinny_takes(M, N, K):
+            return None
+        tile = large_tile(mode, M, N, K) if tiled and M > MEDIUM_MAX_ROWS else None
+        if tile is not None:
+            return (1, *tile)
+        if M > MEDIUM_MAX_ROWS and not (tiled and rows_fit(mode, M, N, K)):
+            return None
+    elif M > MEDIUM_MAX_ROWS:
+        return None
+    return (0, *_few_plan(mode, M, N, K))
+
+
+def _native_product(few: bool, a: torch.Tensor, w: torch.Tensor, w_tiled, bias, target, mode: int, out_dtype, gelu: bool = False, glu=None,
+                    next_norm_weight=None, next_one_centered: bool = False, squares=None, eps: float = 0.0):
+    """A product through the native module: what ``gemm_medium`` (``few``), ``gemm`` or ``gemm_swiglu`` return, or NotImplemented."""
+    if not a.is_cuda or a.dim() != 2 or w.dim() != 2 or (out_dtype != torch.bfloat16 and out_dtype != torch.float32):
+        return NotImplemented
+    M, K = a.shape
+    rows = w.shape[0]
+    plan = _native_plan(few, w_tiled is not None, mode, M, rows // 2 if mode == 2 else rows, K)
+    if plan is None:
+        return NotImplemented
+    tickets = plan[6] if plan[0] else plan[3]
+    counters = _medium_counters(a.device, tickets) if tickets else None
+    rounded = out_dtype == torch.bfloat16
+    code = BF16 if rounded else F32
+    if gelu:
+        code = BF16_GELU
+    elif glu == GEGLU and plan[0]:      # (the products of few rows are told by the unit, not by the output's type)
+        code, glu = BF16_GEGLU, None
+    limit, alpha, shift = _SWIGLU if glu is None else _glu(glu)
+    return _native.product(a, w, w_tiled, bias, target, mode, code, rounded, next_norm_weight, next_one_centered, squares, eps, limit, alpha, shift, plan, counters,
+                           _stream())
 
 
 def gemm_medium(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Optional[torch.Tensor] = None,
@@ -961,15 +1066,22 @@ def gemm_medium(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Option
     ACCUMULATE / SWIGLU): returns the output, or for an accumulation with ``next_norm_weight``
     what the norm after it needs. ``glu`` (with EPILOGUE_SWIGLU): (limit, alpha, shift) of a gated
     unit with clamped halves instead of SwiGLU."""
+    if _native is not None and _profiled is None and epilogue in (0, 1, 2) and (not gelu or (epilogue == EPILOGUE_STORE and (out_dtype or torch.bfloat16) == torch.bfloat16)):
+        made = _native_product(True, a, w, w_tiled, bias, accumulate_into, epilogue,
+                               torch.bfloat16 if epilogue == EPILOGUE_SWIGLU else torch.float32 if epilogue == EPILOGUE_ACCUMULATE else out_dtype or torch.bfloat16,
+                               gelu, glu if epilogue == EPILOGUE_SWIGLU else None, next_norm_weight, next_one_centered, squares, eps)
+        if made is not NotImplemented:
+            return made
     _dev(a, w, bias, accumulate_into, squares, next_norm_weight)
     _want(a, torch.bfloat16, "a")
     _want(w, torch.bfloat16, "w")
     M, K = a.shape
+    w_rows, w_k = w.shape
     kinds = 2 if epilogue == EPILOGUE_SWIGLU else 1
-    if not 1 <= M <= MEDIUM_MAX_ROWS or w.shape[1] != K or w.shape[0] % kinds or K % 8 or epilogue not in (0, 1, 2):
+    if not 1 <= M <= MEDIUM_MAX_ROWS or w_k != K or w_rows % kinds or K % 8 or epilogue not in (0, 1, 2):
         raise KernelError(f"gemm_medium: a is {tuple(a.shape)}, w is {tuple(w.shape)}, epilogue {epilogue}")
-    N = w.shape[0] // kinds
-    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (w.shape[0],)):
+    N = w_rows // kinds
+    if bias is not None and (bias.dtype != torch.float32 or bias.shape != (w_rows,)):
         raise KernelError("gemm_medium: bias must be float32, one entry per row of w")
     if next_norm_weight is not None and (epilogue != EPILOGUE_ACCUMULATE or next_norm_weight.dtype != torch.float32
                                          or next_norm_weight.shape != (N,)):
@@ -981,7 +1093,7 @@ def gemm_medium(a: torch.Tensor, w: torch.Tensor, epilogue: int, *, bias: Option
         left = gemm_medium_into(a, w, bias, accumulate_into, F32, 1, N, next_norm_weight, next_one_centered, squares, eps, w_tiled=w_tiled)
         return accumulate_into if left is None else left
     out_dtype = torch.bfloat16 if epilogue == EPILOGUE_SWIGLU else (out_dtype or torch.bfloat16)
-    out = torch.empty((M, N), dtype=out_dtype, device=a.device)
+    out = torch.empty(M, N, dtype=out_dtype, device=a.device)
     if gelu and (epilogue != EPILOGUE_STORE or out_dtype != torch.bfloat16):
         raise KernelError("gemm_medium: gelu goes with a storing product of bfloat16")
     gemm_medium_into(a, w, bias, out, BF16_GELU if gelu else _code(out_dtype), epilogue, N, squares=squares, eps=eps, w_tiled=w_tiled, glu=glu)
@@ -1026,6 +1138,11 @@ def gemm(a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     the float32 sums, rounded once (the matrix-core products form it as they store)."""
     if gelu and accumulate_into is not None:
         raise KernelError("gemm: gelu goes with a product that stores")
+    if _native is not None and _profiled is None and a.dtype == torch.bfloat16 and (not gelu or (out_dtype or a.dtype) == torch.bfloat16):
+        made = _native_product(False, a, w, w_tiled, bias, accumulate_into, 0 if accumulate_into is None else 1,
+                               out_dtype or a.dtype if accumulate_into is None else torch.float32, gelu)
+        if made is not NotImplemented:
+            return made
     if gelu and (not _fast_ok(a, w) or (out_dtype or a.dtype) != torch.bfloat16):
         return gelu_rows(gemm(a, w, bias, out_dtype=torch.float32, w_tiled=w_tiled), out_dtype or a.dtype)
     if not _fast_ok(a, w):
@@ -1054,6 +1171,10 @@ def gemm_swiglu(a: torch.Tensor, w_gate_up: torch.Tensor, w_tiled: Optional[torc
     in place of silu).
     The activation is formed from the float32 sums inside the product's kernel; where the operands fit none of those the
     [M, 2I] intermediate is float32 and a second kernel forms it."""
+    if _native is not None and _profiled is None and a.dtype == torch.bfloat16:
+        made = _native_product(False, a, w_gate_up, w_tiled, None, None, 2, torch.bfloat16, glu=GEGLU if gelu else None)
+        if made is not NotImplemented:
+            return made
     rows2, K = w_gate_up.shape
     if rows2 % 2:
         raise KernelError("gemm_swiglu: the operand holds gate and up rows; their number must be even")
@@ -1079,6 +1200,7 @@ EPILOGUE_STORE, EPILOGUE_ACCUMULATE, EPILOGUE_SWIGLU, EPILOGUE_CONV = 0, 1, 2, 3
 
 
 GEGLU = "gelu_tanh"       # in place of a clamped unit's three numbers
+_SWIGLU = (0.0, 1.0, 0.0)
 
 
 def _glu(glu):
@@ -1218,6 +1340,12 @@ def attention_prefill(q: torch.Tensor, num_heads: int, num_kv_heads: int, head_d
     """``heads_together``: query heads of a kv group per workgroup (0 and 1: one; 4 up to head_dim 64). ``halves`` (up
     to head_dim 64): two heads per workgroup, whose two halves share a tile's pages out and merge. ``paired`` (head_dim and v_dim both
     64 or both 128, an even number of heads a group): two heads per workgroup, whose loop has three pages in flight; with ``halves`` or without. Only the rows of the given tiles are written (into ``out`` if given)."""
+    if _native is not None and _profiled is None and out is None and q.is_cuda:
+        made = _native.prefill(q, num_heads, num_kv_heads, head_dim, k_pages, v_pages, block_table, tile_seg, tile_row0, seg_row0, row_pos, scale, window, heads_together,
+                               head_dim if v_dim is None else v_dim, chunk, softcap, keep_first, sinks, slopes, (1 if halves else 0) + (2 if paired else 0), PAGE_SIZE,
+                               _stream())
+        if made is not NotImplemented:
+            return made
     _dev(q, k_pages, v_pages, block_table, tile_seg, tile_row0, seg_row0, row_pos)
     _want(q, torch.bfloat16, "q")
     rows = q.shape[0]

@@ -35,13 +35,17 @@ class Linear:
         # kilobytes per wave: a decode step is bound by how fast the weights stream); the prompt kernels
         # read the row-major one. None where that layout does not apply.
         self.tiled = ops.tile_weights(self.weight)
+        # the fewest rows that go to the products of a few dozen rows, which take bfloat16 operands whose rows lie at 16 bytes
+        self._rounded = self.weight.dtype == torch.bfloat16
+        large = self.weight.numel() >= (self.LARGE if self.tiled is None else self.LARGE_TILED)
+        self._medium_from = (self.LARGE_MIN_ROWS if self.tiled is None else self.LARGE_TILED_MIN_ROWS) if large else ops.DECODE_MAX_ROWS + 1
+        if not self._rounded or self.in_features % 8:
+            self._medium_from = 1 << 30
 
     # ----- which path ---------------------------------------------------------------------
     def _fused(self, a: Input, features: int, epilogue: int) -> bool:
-        if self.weight.dtype != torch.bfloat16 or a.dtype != torch.bfloat16:
-            return False
         rows = a.rows if isinstance(a, LazyNorm) else a.shape[0]
-        if not 1 <= rows <= ops.DECODE_MAX_ROWS:
+        if not (1 <= rows <= ops.DECODE_MAX_ROWS and self._rounded and a.dtype == torch.bfloat16):
             return False
         if isinstance(a, LazyNorm) and (a.rms_parameters() is None or (features >= self.WIDE and a.prepared is None)):
             return False        # very wide outputs (a vocabulary): norming once beats norming in every workgroup
@@ -79,16 +83,9 @@ class Linear:
     def _medium(self, a: Input) -> bool:
         """17..64 rows of a bfloat16 model, and fewer rows of a large weight: the products of a few dozen
         rows, which take prepared activations and prepare the next norm as the fused decode product does."""
-        if self.weight.dtype != torch.bfloat16 or a.dtype != torch.bfloat16 or self.in_features % 8:
-            return False
-        rows = a.rows if isinstance(a, LazyNorm) else a.shape[0]
-        if self.tiled is None:
-            few = self.LARGE_MIN_ROWS <= rows <= ops.DECODE_MAX_ROWS and self.weight.numel() >= self.LARGE
-        else:
-            few = self.LARGE_TILED_MIN_ROWS <= rows <= ops.DECODE_MAX_ROWS and self.weight.numel() >= self.LARGE_TILED
-        if not (few or ops.DECODE_MAX_ROWS < rows <= ops.MEDIUM_MAX_ROWS):
-            return False
-        return not isinstance(a, LazyNorm) or a.prepared is not None
+        if isinstance(a, LazyNorm):
+            return a.prepared is not None and self._medium_from <= a.rows <= ops.MEDIUM_MAX_ROWS and a.dtype == torch.bfloat16
+        return self._medium_from <= a.shape[0] <= ops.MEDIUM_MAX_ROWS and a.dtype == torch.bfloat16
 
     @staticmethod
     def _prepared_arguments(a: Input) -> dict:
@@ -99,7 +96,7 @@ class Linear:
     def _normed(self, a: Input, features: int, gated: bool) -> bool:
         """Few float32 rows whose norm has not run yet: their product takes it in front (operands that do not start at 16 bytes pass the
         norm and the plain product)."""
-        return (isinstance(a, LazyNorm) and a.dtype == torch.float32 and self.weight.dtype == torch.float32 and self.weight.data_ptr() % 16 == 0
+        return (not self._rounded and isinstance(a, LazyNorm) and a.dtype == torch.float32 and self.weight.dtype == torch.float32 and self.weight.data_ptr() % 16 == 0
                 and a.pending and ops.float32_normed_takes(gated, a.rows, features, self.in_features))
 
     # ----- products -----------------------------------------------------------------------

@@ -51,13 +51,13 @@ class LazyNorm:
     def __init__(self, norm: Norm, x: torch.Tensor, ctx, row_index: Optional[torch.Tensor] = None,
                  prepared: Optional[Prepared] = None):
         self.norm, self.x, self.ctx, self.row_index = norm, x, ctx, row_index
+        self.prepared = self._tensor = None
         # only what was made for this very norm and these rows counts
-        ok = prepared is not None and prepared.norm is norm and row_index is None \
-            and prepared.activations.shape == x.shape
-        self._tensor = None
-        if ok and isinstance(prepared, NormedRows):     # the norm has run already
-            self._tensor, ok = prepared.activations, False
-        self.prepared = prepared if ok else None
+        if prepared is not None and prepared.norm is norm and row_index is None and prepared.activations.shape == x.shape:
+            if isinstance(prepared, NormedRows):        # the norm has run already
+                self._tensor = prepared.activations
+            else:
+                self.prepared = prepared
 
     @property
     def rows(self) -> int:

@@ -1,0 +1,136 @@
+"""The native module of launches: bit for bit what the general paths give, over every form that it accepts; what it does not take goes to them and is served or refused as
+they do."""
+
+import pytest
+import torch
+
+DEV = "cuda:0"
+BF, F32 = torch.bfloat16, torch.float32
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from flyweight_amd.kernels import ops as module
+    module.library()
+    assert module.native_launches()
+    return module
+
+
+def draw(*shape, dtype=BF, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV)
+
+
+def both(ops, monkeypatch, call):
+    """What the call gives natively and on the general path."""
+    taken = []
+    real = ops._native
+
+    class Counted:
+        def __getattr__(self, name):
+            def function(*args):
+                made = getattr(real, name)(*args)
+                taken.append(made is not NotImplemented)
+                return made
+            return function
+
+    monkeypatch.setattr(ops, "_native", Counted())
+    native = call()
+    monkeypatch.setattr(ops, "_native", None)
+    general = call()
+    monkeypatch.setattr(ops, "_native", real)
+    assert taken and all(taken)
+    return native, general
+
+
+def same(a, b):
+    if isinstance(a, tuple):
+        return len(a) == len(b) and all(same(x, y) for x, y in zip(a, b))
+    return a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 2048, 4096), (16, 2048, 8192), (17, 96, 520), (37, 3072, 1024), (64, 515, 168), (65, 1000, 1024), (130, 2048, 4608), (300, 1536, 512), (801, 2048, 2048)])
+@pytest.mark.parametrize("tiled", [False, True])
+def test_products(ops, monkeypatch, M, N, K, tiled):
+    a, w, bias, old = draw(M, K), draw(2 * N, K, seed=1), draw(N, dtype=F32, seed=2), draw(M, N, dtype=F32, seed=3)
+    own = w[:N].contiguous()
+    t, t2 = (ops.tile_weights(own), ops.tile_weights(w)) if tiled else (None, None)
+    if tiled and t is None:
+        return
+    taken = ops._native_plan(False, tiled, 0, M, N, K) is not None
+    if taken:
+        for how in ({}, {"out_dtype": F32}, {"bias": bias, "out_dtype": F32}, {"gelu": True}):
+            assert same(*both(ops, monkeypatch, lambda: ops.gemm(a, own, w_tiled=t, **how)))
+    if ops._native_plan(False, tiled, 1, M, N, K) is not None:
+        assert same(*both(ops, monkeypatch, lambda: ops.gemm(a, own, bias, accumulate_into=old.clone(), w_tiled=t)))
+    if ops._native_plan(False, tiled, 2, M, N, K) is not None:
+        for gelu in (False, True):
+            assert same(*both(ops, monkeypatch, lambda: ops.gemm_swiglu(a, w, w_tiled=t2, gelu=gelu)))
+    if M <= 64:
+        squares = draw(5, 16 if M <= 16 else 64, dtype=F32, seed=4).abs()
+        weight = draw(N, dtype=F32, seed=5)
+        assert same(*both(ops, monkeypatch, lambda: ops.gemm_medium(a, own, ops.EPILOGUE_STORE, squares=squares, eps=1e-5, bias=bias, out_dtype=F32, w_tiled=t)))
+        for glu in (None, ops.GEGLU, (7.0, 1.702, 1.0)):
+            assert same(*both(ops, monkeypatch, lambda: ops.gemm_medium(a, w, ops.EPILOGUE_SWIGLU, glu=glu, w_tiled=t2)))
+        for centered in (False, True):
+            def add():
+                into = old.clone()
+                return (*ops.gemm_medium(a, own, ops.EPILOGUE_ACCUMULATE, accumulate_into=into, next_norm_weight=weight, next_one_centered=centered, w_tiled=t), into)
+            (x, sums, into), (x2, sums2, into2) = both(ops, monkeypatch, add)
+            assert same(x, x2) and same(into, into2) and same(sums[:, :M], sums2[:, :M])
+
+
+@pytest.mark.gpu
+def test_norm_convolution_and_attention(ops, monkeypatch):
+    x, weight, index = draw(40, 512, dtype=F32), draw(512, dtype=F32, seed=1), torch.tensor([3, 39, 3], dtype=torch.int32, device=DEV)
+    for dtype in (BF, F32):
+        for rows in (None, index):
+            assert same(*both(ops, monkeypatch, lambda: ops.rmsnorm_rows(x, weight, 1e-5, dtype, row_index=rows, one_centered=rows is not None)))
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)    # noqa: E731
+    bcx, taps, state = draw(40, 3 * 512, dtype=F32), draw(512, 3, dtype=F32), draw(4, 512, 2, dtype=F32)
+    seg, row0, slot = ints(*([0] * 33 + [1] * 7)), ints(0, 33, 40), ints(2, 0)
+
+    def conv():
+        own = state.clone()
+        return ops.shortconv(bcx, taps, weight, own, seg, row0, slot, 2, out_dtype=BF), own
+    assert same(*both(ops, monkeypatch, conv))
+    heads, kv, d, rows = 8, 2, 64, 40
+    qkv, q_weight = draw(rows, (heads + 2 * kv) * d, dtype=F32), draw(d, dtype=F32, seed=2)
+    cos, sin = draw(rows, d // 2, dtype=F32, seed=3), draw(rows, d // 2, dtype=F32, seed=4)
+    table, pos = ints(0, 1).view(2, 1).contiguous(), ints(*list(range(33)) + list(range(7)))
+
+    def attend():
+        k_pages, v_pages = torch.zeros(3, kv, 64, d, dtype=BF, device=DEV), torch.zeros(3, kv, d, 64, dtype=BF, device=DEV)
+        q = ops.qk_norm_rope_kv_write(qkv, heads, kv, d, q_weight, q_weight, 1e-5, cos, sin, d, k_pages, v_pages, table, seg, pos)
+        tile_seg, tile_row0 = ops.query_tiles([0, 33, 40])
+        out = ops.attention_prefill(q, heads, kv, d, k_pages, v_pages, table, ints(*tile_seg), ints(*tile_row0), row0, pos, d ** -0.5, sinks=draw(heads, dtype=F32))
+        return q, k_pages, v_pages, out
+    assert same(*both(ops, monkeypatch, attend))
+
+
+@pytest.mark.gpu
+def test_what_it_does_not_take_is_served_or_refused_as_before(ops):
+    a, w = draw(40, 256), draw(96, 256, seed=1)
+    with pytest.raises(ops.KernelError, match="contiguous"):
+        ops.gemm(a.t().contiguous().t(), w)
+    with pytest.raises(ops.KernelError, match="gemm: a is"):
+        ops.gemm(a[:, :128].contiguous(), w)
+    with pytest.raises(ops.KernelError, match="destination"):
+        ops.gemm(a, w, accumulate_into=torch.zeros(40, 95, device=DEV))
+    with pytest.raises(ops.KernelError, match="sums of squares"):
+        ops.gemm_medium(a, w, ops.EPILOGUE_STORE, squares=torch.zeros(2, 16, device=DEV))
+    with pytest.raises(ops.KernelError, match="operand tiles"):
+        ops.gemm_medium(a, w, ops.EPILOGUE_STORE, w_tiled=ops.tile_weights(w)[:-1].contiguous())
+    with pytest.raises(ops.KernelError, match="row width"):
+        ops.rmsnorm_rows(a.float(), torch.zeros(255, device=DEV), 1e-5, BF)
+    odd = torch.empty(40 * 256 + 1, dtype=BF, device=DEV)[1:].view(40, 256).copy_(a)       # at no multiple of 16 bytes
+    assert torch.allclose(ops.gemm(odd, w, out_dtype=F32), a.float() @ w.float().T, atol=1e-3)
+
+
+def test_tensors_of_the_host_are_left_to_the_general_path(ops):
+    a, w = torch.zeros(20, 64, dtype=BF), torch.zeros(32, 64, dtype=BF)
+    assert ops._native_product(False, a, w, None, None, None, 0, BF) is NotImplemented
+    with pytest.raises(ops.KernelError, match="GPU only"):
+        ops.rmsnorm_rows(torch.zeros(2, 8), torch.zeros(8), 1e-5, BF)
+    with pytest.raises(TypeError):
+        ops._native.rmsnorm(a)
