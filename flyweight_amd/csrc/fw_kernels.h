@@ -441,8 +441,10 @@ int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place
 // or float32.
 int fw_grouped_gemm_few(const void* a, const int32_t* place_row, const void* w_tiled, const int32_t* expert_begin, void* out, int gated, int places,
                         int experts, int N, int K, int place_tiles, float glu_limit, float glu_alpha, float glu_shift, void* stream);
-// 1: with bfloat16 operands, the plain unit and an output of bfloat16 (gated) or float32 the large tiles take it
+// 1: with bfloat16 operands, the plain unit and an output of bfloat16 (gated) or float32 the product is worth tiles of more than 128 places
 int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int experts, int N, int K);
+// the places and the columns (gate and up together) of the tile that it then has; tall: tiles of more than 128 places are worth it
+int fw_grouped_gemm_tile(int gated, int places, int experts, int N, int K, int tall, int* rows, int* columns);
 // x[r] += sum_j weight[r][j] * y[pair_place[r][j]], j in order, and with b (null: none) + sigmoid(gate[r * gate_stride]) b[r]; float32
 int fw_moe_combine(float* x, const float* y, const float* weight, const int32_t* pair_place, const float* b, const float* gate,
                    int gate_stride, int rows, int top, int hidden, void* stream);

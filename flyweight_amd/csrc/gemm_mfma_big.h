@@ -41,6 +41,7 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 
 #define BT 256                  // tile edge (rows: of the tall tiles)
 #define BK 32                   // k of one step of products: K is a multiple of it
+#define BSLAB 64                // k of a slab, two steps
 #define BLDS 163840             // bytes of LDS of a compute unit
 #define BK_MOST (1 << 22)
 #define BN_MOST (1 << 20)       // 256 rows of the output lie below BOUNDS
@@ -83,32 +84,27 @@ struct BigSlices {
     int* counters;
 };
 
-// A slab: 64 k of the tile's rows (an LDS row is 128 bytes, eight 16-byte chunks), or 32 where two workgroups share a compute unit. Chunk
+// A slab: 64 k of the tile's rows (an LDS row is 128 bytes, eight 16-byte chunks). Chunk
 // c of a row lies in slot c ^ swap(row): a read of 16 rows by four chunks goes in groups of 16 lanes, 0-3, 12-15 and 20-27, then the 16
 // others of the first 32, and every group covers all 64 banks once.
-template <int DEPTH>
-__device__ __forceinline__ int chunk_swap(int row) {
-    if (DEPTH == 64) return (row >> 1) & 7;
-    const int low = (row >> 2) & 1, high = (row >> 3) & 1;      // 0, 2, 3, 1 for four rows each
-    return (low ^ high) * 2 + high;
-}
+__device__ __forceinline__ int chunk_swap(int row) { return (row >> 1) & 7; }
 
-template <int TM, int TN, int DEPTH, int EACH_CU = DEPTH == 64 ? 1 : 2>
+template <int TM, int TN, int EACH_CU>
 struct BigTile {
     static constexpr int ROWS = 2 * TM * 32;               // rows of a tile
     static constexpr int WIDE = 2 * TN * 32;               // columns of a tile
-    static constexpr int A_SLAB = ROWS * DEPTH * 2, W_SLAB = WIDE * DEPTH * 2;     // bytes
+    static constexpr int A_SLAB = ROWS * BSLAB * 2, W_SLAB = WIDE * BSLAB * 2;     // bytes
     static constexpr int A_LOADS = A_SLAB / 4096;          // wave-wide loads per wave for a slab of a (1,024 bytes each)
     static constexpr int W_LOADS = W_SLAB / 4096;          // and for a slab of w
     static constexpr int SLAB_LOADS = A_LOADS + W_LOADS;   // and for a slab of both operands
     // slabs in LDS, the one that is multiplied among them: as many of both as fit, and one more of w if it fits beside them
-    static constexpr int LDS_MOST = BLDS / EACH_CU, MOST_STAGES = DEPTH == 64 && TM * TN <= 4 ? 6 : 4;
+    static constexpr int LDS_MOST = BLDS / EACH_CU, MOST_STAGES = TM * TN <= 4 ? 6 : 4;
     static constexpr int A_STAGES = LDS_MOST / (A_SLAB + W_SLAB) < MOST_STAGES ? LDS_MOST / (A_SLAB + W_SLAB) : MOST_STAGES;
     static constexpr int W_STAGES = A_STAGES < 3 && A_STAGES * A_SLAB + (A_STAGES + 1) * W_SLAB <= LDS_MOST ? A_STAGES + 1 : A_STAGES;
     static constexpr int LDS = A_STAGES * A_SLAB + W_STAGES * W_SLAB;
-    // whether w is asked for together with a, behind the products that follow a slab's last read: where a slab is one step, and where w has
-    // two stages (asked for a step later its slab would have one step to arrive)
-    static constexpr bool TOGETHER = DEPTH == BK || W_STAGES == 2;
+    // whether w is asked for together with a, behind the products that follow a slab's last read: where w has two stages (asked for a step later its
+    // slab would have one step to arrive)
+    static constexpr bool TOGETHER = W_STAGES == 2;
 };
 
 // K must be a multiple of BK (the loads go straight to LDS: nothing can be zeroed on the way), and at most BK_MOST (a
@@ -119,17 +115,18 @@ struct BigTile {
 // (1,310 TFLOP/s), storing 2,048 x 6,144 x 2,048 52.8 -> 44.0, 2,048 x 3,072 x 2,048 30.7 -> 25.4, 1,111 x 16,384 x 2,048 90.4 -> 79.0, 8,192^3 1,254 -> 1,470
 // TFLOP/s. Where the loads stand among the MFMAs (behind every second to every eighth) changed nothing; two stages of w instead of three cost 1 to 8 %.
 // TN: 32-column pairs of product tiles per wave, 2 (128 columns a tile) to 5 (320). TM: 32-row pairs of product tiles per wave, 1 (64 rows a tile) to
-// 4. DEPTH: k of a slab, EACH_CU: workgroups on a compute unit, see BigTile.
-template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED, bool SPLIT, int EACH_CU>
+// 4. EACH_CU: workgroups on a compute unit.
+template <int MODE, typename TO, int TN, int TM, bool GROUPED, bool SPLIT, int EACH_CU>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EACH_CU))) void gemm_mfma_big_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const float* __restrict__ bias,
     TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups, const BigSlices cut) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [A_STAGES slabs of a][W_STAGES slabs of w]
-    typedef BigTile<TM, TN, DEPTH, EACH_CU> Tile;
+    typedef BigTile<TM, TN, EACH_CU> Tile;
     constexpr int ROWS = Tile::ROWS, WIDE = Tile::WIDE, A_SLAB = Tile::A_SLAB, W_SLAB = Tile::W_SLAB, A_STAGES = Tile::A_STAGES, W_STAGES = Tile::W_STAGES;
     constexpr int A_LOADS = Tile::A_LOADS, W_LOADS = Tile::W_LOADS, SLAB_LOADS = Tile::SLAB_LOADS;
     constexpr bool TOGETHER = Tile::TOGETHER;
-    constexpr int PARTS = DEPTH / BK, CHUNKS = DEPTH / 8, LOAD_ROWS = 64 / CHUNKS;      // steps of a slab, chunks of a row, rows of a wave-wide load
+    constexpr int PARTS = BSLAB / BK, CHUNKS = BSLAB / 8, LOAD_ROWS = 64 / CHUNKS;      // steps of a slab, chunks of a row, rows of a wave-wide load
+    static_assert(PARTS == 2, "the loop has two steps a slab");
     constexpr int features = MODE == MB_SWIGLU ? WIDE / 2 : WIDE;       // a gated tile holds as many gate as up rows
     int m0, n0, k_first = 0, k_length = K;
     const int32_t* groups_rows = nullptr;
@@ -181,7 +178,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
         const int row = (wave * A_LOADS + i) * LOAD_ROWS + lane / CHUNKS;
-        const int chunk = (lane % CHUNKS) ^ chunk_swap<DEPTH>(row);
+        const int chunk = (lane % CHUNKS) ^ chunk_swap(row);
         uint32_t from = row < M - m0 ? row : M - m0 - 1;        // rows past the end are computed and dropped
         if (GROUPED && groups_rows) from = groups_rows[m0 + (int)from];
         a_at[i] = from * (uint32_t)(2 * K) + chunk * 16;
@@ -189,28 +186,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
 #pragma unroll
     for (int i = 0; i < W_LOADS; ++i) {
         const int row = (wave * W_LOADS + i) * LOAD_ROWS + lane / CHUNKS;
-        const int chunk = (lane % CHUNKS) ^ chunk_swap<DEPTH>(row);
+        const int chunk = (lane % CHUNKS) ^ chunk_swap(row);
         const int of_part = MODE == MB_SWIGLU ? row - w_part * features : row;
         w_at[i] = (uint32_t)(of_part < N - n0 ? of_part : N - n0 - 1) * (uint32_t)(2 * K) + chunk * 16;
     }
     const fw_buffer a_rows = fw_make_buffer(a_base + k_first), w_rows = fw_make_buffer(w_base + k_first);
     // This wave's loads for a slab of either operand, into the stage at `stage`. A last slab of half the length has no upper
     // chunks: the lower ones are read again in their place and never used.
-    const int whole = k_length / DEPTH, slabs = (k_length + DEPTH - 1) / DEPTH;
-    auto request_a = [&](int stage, int slab, int i) { fw_buffer_to_lds(a_rows, lds + stage + (wave * A_LOADS + i) * 1024, a_at[i], slab * (DEPTH * 2)); };
-    auto request_w = [&](int stage, int slab, int i) { fw_buffer_to_lds(w_rows, lds + stage + (wave * W_LOADS + i) * 1024, w_at[i], slab * (DEPTH * 2)); };
-    auto upper = [&](int first_row) { return ((lane % CHUNKS) ^ chunk_swap<DEPTH>(first_row + lane / CHUNKS)) >= CHUNKS / 2; };
+    const int whole = k_length / BSLAB, slabs = (k_length + BSLAB - 1) / BSLAB;
+    auto request_a = [&](int stage, int slab, int i) { fw_buffer_to_lds(a_rows, lds + stage + (wave * A_LOADS + i) * 1024, a_at[i], slab * (BSLAB * 2)); };
+    auto request_w = [&](int stage, int slab, int i) { fw_buffer_to_lds(w_rows, lds + stage + (wave * W_LOADS + i) * 1024, w_at[i], slab * (BSLAB * 2)); };
+    auto upper = [&](int first_row) { return ((lane % CHUNKS) ^ chunk_swap(first_row + lane / CHUNKS)) >= CHUNKS / 2; };
     auto request_slab_a = [&](int stage, int slab) {
 #pragma unroll
         for (int i = 0; i < A_LOADS; ++i) {
-            if (PARTS == 2 && slab >= whole && upper((wave * A_LOADS + i) * LOAD_ROWS)) a_at[i] -= BK * 2;
+            if (slab >= whole && upper((wave * A_LOADS + i) * LOAD_ROWS)) a_at[i] -= BK * 2;
             request_a(stage, slab, i);
         }
     };
     auto request_slab_w = [&](int stage, int slab) {
 #pragma unroll
         for (int i = 0; i < W_LOADS; ++i) {
-            if (PARTS == 2 && slab >= whole && upper((wave * W_LOADS + i) * LOAD_ROWS)) w_at[i] -= BK * 2;
+            if (slab >= whole && upper((wave * W_LOADS + i) * LOAD_ROWS)) w_at[i] -= BK * 2;
             request_w(stage, slab, i);
         }
     };
@@ -227,7 +224,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     // Every row this lane reads is (lane % 16) plus a multiple of 16: one permutation for all
     int slot[PARTS];
 #pragma unroll
-    for (int t = 0; t < PARTS; ++t) slot[t] = ((4 * t + (lane >> 4)) ^ chunk_swap<DEPTH>(lane & 15)) * 16;
+    for (int t = 0; t < PARTS; ++t) slot[t] = ((4 * t + (lane >> 4)) ^ chunk_swap(lane & 15)) * 16;
     const int a_row0 = wm * (TM * 32) + (lane & 15), b_row0 = wn * (MODE == MB_SWIGLU ? TN * 16 : TN * 32) + (lane & 15);
 
     // operand registers of one step: the wave's row tiles of a and column tiles of w
@@ -247,10 +244,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     };
     auto read_one = [&](Operands& f, int a_stage, int w_stage, int part, int which) {
         if (which < TA) {
-            f.fa[which] = *reinterpret_cast<const bf16x8*>(lds + a_stage + slot[part] + (a_row0 + 16 * which) * (DEPTH * 2));
+            f.fa[which] = *reinterpret_cast<const bf16x8*>(lds + a_stage + slot[part] + (a_row0 + 16 * which) * (BSLAB * 2));
         } else {
             const int j = which - TA, row = MODE == MB_SWIGLU ? (j / TN) * features + (j % TN) * 16 : j * 16;
-            f.fb[j] = *reinterpret_cast<const bf16x8*>(lds + w_stage + slot[part] + (b_row0 + row) * (DEPTH * 2));
+            f.fb[j] = *reinterpret_cast<const bf16x8*>(lds + w_stage + slot[part] + (b_row0 + row) * (BSLAB * 2));
         }
     };
     auto read = [&](Operands& f, int a_stage, int w_stage, int part) {
@@ -260,8 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     // product tile number `which`, row by row, every second row backwards
     auto multiply_one = [&](const Operands& f, int which) {
         const int i = which / TB, j = i & 1 ? TB - 1 - which % TB : which % TB;
-        if constexpr (DEPTH == 32) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.fa[i], f.fb[j], acc[i][j], 0, 0, 0);
-        else if (i * TB + j < 64) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f.fa[i]), "v"(f.fb[j]));
+        if (i * TB + j < 64) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(f.fa[i]), "v"(f.fb[j]));
         else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(f.fa[i]), "v"(f.fb[j]));      // (256 accumulation registers)
     };
     auto multiply = [&](const Operands& f) {
@@ -290,8 +286,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     // With one wave per SIMD nothing else hides the latency of LDS: the operands of a step are read behind the MFMAs of the step
     // before it. Ahead of a slab's last step the wave makes sure that the next slab has landed (its own loads: vmcnt; everybody's: the
     // barrier), which also tells that every wave has read slab s. Its stages then take the slabs that come A_STAGES and W_STAGES later:
-    // that of a behind the MFMAs of the slab's last step, that of w behind those of the next slab's first (where a slab is one
-    // step, both behind its later MFMAs).
+    // that of a behind the MFMAs of the slab's last step, that of w behind those of the next slab's first.
     for (int u = 0; u < W_STAGES - 1; ++u) {
         if (u < slabs) request_slab_a(u * A_SLAB, u);
         if (u < slabs) request_slab_w(W_FIRST + u * W_SLAB, u);
@@ -311,77 +306,44 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((W_STAGES - 2) * EACH) : "memory");   // slab s + 1 has landed; those behind it may still fly
         __builtin_amdgcn_s_barrier();
     };
-    if constexpr (PARTS == 2) {
-        while (s + A_STAGES < whole) {
-            arrived(f0);
+    while (s + A_STAGES < whole) {
+        arrived(f0);
 #pragma unroll
-            for (int u = 0; u < MFMAS; ++u) {
-                if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f1, a_now, w_now, 1, u / READ_GAP);
-                if (!TOGETHER && u % W_GAP == 0 && u / W_GAP < W_LOADS) request_w(w_before, s + W_STAGES - 1, u / W_GAP);
-                multiply_one(f0, u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            landed(f1);
-#pragma unroll
-            for (int u = 0; u < MFMAS; ++u) {
-                if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f0, a_then, w_then, 0, u / READ_GAP);
-                if (u % A_GAP == 0 && u / A_GAP < A_LOADS) request_a(a_now, s + A_STAGES, u / A_GAP);
-                if (TOGETHER && u % W_GAP == W_GAP / 2 && u / W_GAP < W_LOADS) request_w(w_now, s + W_STAGES, u / W_GAP);
-                multiply_one(f1, u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            advance();
-            ++s;
+        for (int u = 0; u < MFMAS; ++u) {
+            if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f1, a_now, w_now, 1, u / READ_GAP);
+            if (!TOGETHER && u % W_GAP == 0 && u / W_GAP < W_LOADS) request_w(w_before, s + W_STAGES - 1, u / W_GAP);
+            multiply_one(f0, u);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    } else {
-        auto step = [&](const Operands& now, Operands& next) {
-            landed(now);
+        landed(f1);
 #pragma unroll
-            for (int u = 0; u < MFMAS; ++u) {
-                if (u < READS) read_one(next, a_then, w_then, 0, u);
-                const int load = (u - READS) / 2;
-                if (u >= READS && (u - READS) % 2 == 0 && load < A_LOADS) request_a(a_now, s + A_STAGES, load);
-                if (u >= READS && (u - READS) % 2 == 0 && load >= A_LOADS && load < SLAB_LOADS) request_w(w_now, s + W_STAGES, load - A_LOADS);
-                multiply_one(now, u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            advance();
-            ++s;
-        };
-        static_assert(PARTS == 2 || READS + 2 * SLAB_LOADS <= MFMAS, "the loads have MFMAs to go behind");
-        while (s + A_STAGES + 1 < slabs) {                  // two slabs a turn, so that the operand sets keep their names
-            step(f0, f1);
-            step(f1, f0);
+        for (int u = 0; u < MFMAS; ++u) {
+            if (u % READ_GAP == 0 && u / READ_GAP < READS) read_one(f0, a_then, w_then, 0, u / READ_GAP);
+            if (u % A_GAP == 0 && u / A_GAP < A_LOADS) request_a(a_now, s + A_STAGES, u / A_GAP);
+            if (TOGETHER && u % W_GAP == W_GAP / 2 && u / W_GAP < W_LOADS) request_w(w_now, s + W_STAGES, u / W_GAP);
+            multiply_one(f1, u);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        advance();
+        ++s;
     }
     // the last slabs: asking for what is left to ask for; one of two steps may have half the length
     for (; s < slabs; ++s) {
         const int ahead = (slabs < s + W_STAGES ? slabs : s + W_STAGES) - (s + 2);      // slabs behind s + 1 that have been asked for
         arrived(f0);
-        if constexpr (PARTS == 2) {
-            if (s < whole) read(f1, a_now, w_now, 1);
-            if (!TOGETHER && s + W_STAGES - 1 < slabs) request_slab_w(w_before, s + W_STAGES - 1);
-            multiply(f0);
-            __builtin_amdgcn_sched_barrier(0);
-            arrived(f1);
-        }
+        if (s < whole) read(f1, a_now, w_now, 1);
+        if (!TOGETHER && s + W_STAGES - 1 < slabs) request_slab_w(w_before, s + W_STAGES - 1);
+        multiply(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived(f1);
         if (s + 1 < slabs) {
             wait_for_all_but(ahead);
             __builtin_amdgcn_s_barrier();
-            read(PARTS == 2 ? f0 : f1, a_then, w_then, 0);
+            read(f0, a_then, w_then, 0);
             if (s + A_STAGES < slabs) request_slab_a(a_now, s + A_STAGES);
             if (TOGETHER && s + W_STAGES < slabs) request_slab_w(w_now, s + W_STAGES);
         }
-        if constexpr (PARTS == 2) {
-            if (s < whole) multiply(f1);
-        } else {
-            multiply(f0);
-            __builtin_amdgcn_sched_barrier(0);
-            if (s + 1 < slabs) {
-                arrived(f1);
-                f0 = f1;
-            }
-        }
+        if (s < whole) multiply(f1);
         __builtin_amdgcn_sched_barrier(0);
         advance();
     }
@@ -574,15 +536,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     }
 }
 
-template <int MODE, typename TO, int TN, int TM, int DEPTH, bool GROUPED, bool SPLIT = false, int EACH_CU = DEPTH == 64 ? 1 : 2>
+template <int MODE, typename TO, int TN, int TM, bool GROUPED, bool SPLIT, int EACH_CU>
 static int launch_tiles(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, int tiles_m, const BigGroups& groups,
                         hipStream_t stream, const BigSlices& cut = BigSlices()) {
-    const int tiles_n = fw_ceil_div(N, BigTile<TM, TN, DEPTH, EACH_CU>::WIDE / (MODE == MB_SWIGLU ? 2 : 1));
+    const int tiles_n = fw_ceil_div(N, BigTile<TM, TN, EACH_CU>::WIDE / (MODE == MB_SWIGLU ? 2 : 1));
     const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n * (SPLIT ? cut.slices : 1), 8);
-    const int lds_bytes = BigTile<TM, TN, DEPTH, EACH_CU>::LDS;
+    const int lds_bytes = BigTile<TM, TN, EACH_CU>::LDS;
     static bool configured = false;     // per instantiation
     if (!configured) {
-        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED, SPLIT, EACH_CU>,
+        hipError_t status = hipFuncSetAttribute((const void*)gemm_mfma_big_kernel<MODE, TO, TN, TM, GROUPED, SPLIT, EACH_CU>,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (status != hipSuccess) {
             fw_set_error("gemm_mfma_big: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(status));
@@ -590,7 +552,7 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
         }
         configured = true;
     }
-    gemm_mfma_big_kernel<MODE, TO, TN, TM, DEPTH, GROUPED, SPLIT, EACH_CU><<<per_xcd * 8, 256, lds_bytes, stream>>>(
+    gemm_mfma_big_kernel<MODE, TO, TN, TM, GROUPED, SPLIT, EACH_CU><<<per_xcd * 8, 256, lds_bytes, stream>>>(
         (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups, cut);
     return 0;
 }
@@ -599,5 +561,5 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
 template <int MODE, typename TO, int TN, int TM, int EACH_CU, bool SPLIT>
 static int launch_big(const BigCall& c) {
     const BigSlices cut = {c.slices, c.k_each, c.partials, c.counters};
-    return launch_tiles<MODE, TO, TN, TM, 64, false, SPLIT, EACH_CU>(c.a, c.w, c.bias, c.out, c.M, c.N, c.K, fw_ceil_div(c.M, TM * 64), BigGroups(), c.stream, cut);
+    return launch_tiles<MODE, TO, TN, TM, false, SPLIT, EACH_CU>(c.a, c.w, c.bias, c.out, c.M, c.N, c.K, fw_ceil_div(c.M, TM * 64), BigGroups(), c.stream, cut);
 }

@@ -1,27 +1,98 @@
 // The products on large tiles that are asked for by shape: the plan of the tile, K cut over workgroups, the experts' grouped product, and the tile named
 // by the caller. The kernel is gemm_mfma_big.h.
+#include <math.h>
+
 #include "gemm_mfma_big.h"
 
-// The grouped product of fw_grouped_gemm on tiles of 128 places by 256 rows of W, for K a multiple of 32 and a of less than 4 GB. Bound by
-// the experts' weights from memory (600 MB for both products of 32 experts of 1,536 features: 127 us) and by tiles that an expert's last places fill partly.
-// Slabs of 64 k leave room for one workgroup on a compute unit, slabs of 32 for two (three stages of 24 KB each), of which one multiplies while the other
-// starts, ends or waits: a short K and experts of less than a tile of places, whose weights are the load, take the latter. us, slabs of 64 / 32, gated and
-// down: 2,048 rows, 4 of 32 experts, 1,536 features over 2,048 146 / 147 and 90 / 99, 1,111 rows 108 / 115 and 49 / 53, 600 rows 109 / 105 and 37 / 37; 1,500
-// rows, 2 of 8 over 4,096 97 / 110; 3,000 rows, 4 of 16 over 1,280 91 / 85; 2,048 rows, 2 of 8 over 1,024 57 / 52, 6 of 64 62 / 54. (On v_mfma_f32_32x32x16_bf16 with
-// slabs of 32: 154 and 102, 120 and 57; tiles of 256 places 186; through registers, moe.hip, 241.)
+// The grouped product of fw_grouped_gemm, for K a multiple of 32 and a of less than 4 GB. Bound by the experts' weights from memory (600 MB for both products
+// of 32 experts of 1,536 features: 127 us), by tiles that an expert's last places fill partly and by rounds of them that the chip is not full with: the tile
+// follows from how many places an expert has in the mean. us, tiles of 128 x 256 alone / chosen, gated and down: 32 experts of 1,536 features over 2,048, four
+// a row, 2,048 rows 160 / 145 and 93 / 77, 1,111 rows 129 / 105 and 65 / 49, 600 rows 103 / 97 and 50 / 45; 16 of 1,024 over 4,096, two a row, 2,048 rows 123 / 88 and
+// 66 / 55; 64 of 768 over 1,024, six a row, 3,000 rows 109 / 91 and 60 / 50. All tiles give the same bits.
 bool fw_grouped_big_takes(int a_rows, int N, int K) { return K % BK == 0 && K <= BK_MOST && N <= BN_MOST && 2ll * a_rows * K <= 0xffff0000ll; }
-int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
-                          int experts, int N, int K, hipStream_t stream) {
-    const BigGroups groups = {place_row, expert_begin, experts};
-    const int tiles_m = places / 128 + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
-    // (what the product through registers, whose tiles have half the features, would refuse is refused here too)
-    FW_REQUIRE((long long)tiles_m * fw_ceil_div(N, gated ? BT / 4 : BT / 2) < (1ll << 30), "grouped_gemm: too many tiles");
-    if (K >= 1536 && places >= 128 * experts) {
-        if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 64, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
-        return launch_tiles<MB_STORE, float, 4, 2, 64, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+
+// What a tile takes, us: start + rounds * round + tiles / 256 * tile + K / 1,024 * (rounds * walk + tiles / 256 * fill) + MB of all experts' weights * memory,
+// rounds those of the tiles over 256 compute units (512 places where two workgroups share one). Fitted to 60 shapes a form (8 to 128 experts, 200 to
+// 4,000 rows) to 5 to 10 % (mean square); so chosen they take 1.5 (gated) and 2.4 % (down) more than with the fastest tile each, and 9 and 12 % less than with one tile.
+struct GroupedTime {
+    int rows, columns, each_cu;
+    float start, round, tile, walk, fill, memory;
+};
+static const GroupedTime grouped_times[2][7] = {
+    {{64, 128, 2, 0.00f, 1.69f, 0.31f, 1.81f, 4.66f, 0.10f},
+     {128, 128, 2, 0.00f, 4.18f, 0.00f, 3.18f, 6.26f, 0.07f},
+     {128, 192, 1, 0.00f, 0.00f, 4.39f, 5.27f, 6.19f, 0.09f},
+     {128, 256, 1, 0.00f, 5.89f, 0.00f, 7.40f, 4.88f, 0.09f},
+     {192, 192, 1, 0.00f, 0.00f, 5.07f, 7.64f, 7.53f, 0.06f},
+     {192, 256, 1, 0.00f, 7.53f, 0.00f, 10.33f, 7.58f, 0.05f},
+     {256, 256, 1, 0.00f, 10.03f, 0.00f, 12.41f, 5.93f, 0.06f}},
+    {{64, 128, 2, 1.16f, 0.00f, 0.96f, 5.69f, 1.95f, 0.11f},
+     {128, 128, 2, 4.24f, 2.27f, 0.00f, 3.57f, 5.23f, 0.09f},
+     {128, 192, 1, 4.36f, 4.89f, 0.00f, 8.30f, 1.44f, 0.09f},
+     {128, 256, 1, 0.32f, 5.96f, 0.38f, 7.08f, 3.95f, 0.11f},
+     {192, 192, 1, 0.69f, 7.95f, 0.00f, 10.28f, 1.73f, 0.07f},
+     {192, 256, 1, 11.21f, 5.31f, 0.00f, 5.18f, 11.60f, 0.07f},
+     {256, 256, 1, 10.72f, 7.17f, 0.00f, 8.36f, 13.75f, 0.04f}}};
+
+// Tiles of `rows` places that experts of `mean` places in the mean have, their numbers spread as independent choices spread them (the device alone knows them):
+// the sum over j of the chance that an expert has more than j * rows.
+static double expected_tiles(double mean, int rows) {
+    double tiles = 0.0;
+    for (int j = 0;; ++j) {
+        const double chance = 0.5 * erfc((j * (double)rows + 0.5 - mean) / sqrt(2.0 * mean));
+        if (chance < 1e-3) return tiles;
+        tiles += chance;
     }
-    if (gated) return launch_tiles<MB_SWIGLU, bf16_t, 4, 2, 32, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
-    return launch_tiles<MB_STORE, float, 4, 2, 32, true>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream);
+}
+
+static const GroupedTime& grouped_plan(int gated, int places, int experts, int N, int K, bool tall) {
+    const GroupedTime* best = nullptr;
+    double least = 0.0;
+    for (const GroupedTime& t : grouped_times[gated]) {
+        if (t.rows > 128 && !tall) continue;
+        const double tiles = expected_tiles((double)places / experts, t.rows) * experts * fw_ceil_div(N, gated ? t.columns / 2 : t.columns), share = tiles / 256.0;
+        const double rounds = ceil(tiles / (256.0 * t.each_cu)), k = K / 1024.0;
+        const double time = t.start + rounds * t.round + share * t.tile + k * (rounds * t.walk + share * t.fill) + 2e-6 * experts * (gated ? 2.0 : 1.0) * N * K * t.memory;
+        if (!best || time < least) {
+            best = &t;
+            least = time;
+        }
+    }
+    return *best;
+}
+
+// The tile of a grouped product that goes straight to LDS.
+extern "C" int fw_grouped_gemm_tile(int gated, int places, int experts, int N, int K, int tall, int* rows, int* columns) {
+    FW_REQUIRE(places >= 1 && experts >= 1 && N >= 1 && K >= 1, "grouped_gemm_tile: bad sizes places=%d experts=%d N=%d K=%d", places, experts, N, K);
+    const GroupedTime& plan = grouped_plan(gated ? 1 : 0, places, experts, N, K, tall != 0);
+    *rows = plan.rows;
+    *columns = plan.columns;
+    return 0;
+}
+
+// `tall`: tiles of more than 128 places are worth a look (fw_grouped_gemm_large_fits)
+int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
+                          int experts, int N, int K, bool tall, hipStream_t stream) {
+    const BigGroups groups = {place_row, expert_begin, experts};
+    const GroupedTime& plan = grouped_plan(gated, places, experts, N, K, tall);
+    const int tiles_m = places / plan.rows + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
+    // (what the product through registers, whose tiles have half the features, would refuse is refused here too)
+    FW_REQUIRE((long long)(places / 128 + (experts < places ? experts : places)) * fw_ceil_div(N, gated ? BT / 4 : BT / 2) < (1ll << 30), "grouped_gemm: too many tiles");
+    FW_REQUIRE((long long)tiles_m * fw_ceil_div(N, gated ? plan.columns / 2 : plan.columns) < (1ll << 30), "grouped_gemm: too many tiles");
+#define FW_GROUPED_TILE(ROWS, COLUMNS, EACH)                                                                                                                   \
+    if (plan.rows == ROWS && plan.columns == COLUMNS && plan.each_cu == EACH)                                                                                  \
+        return gated ? launch_tiles<MB_SWIGLU, bf16_t, COLUMNS / 64, ROWS / 64, true, false, EACH>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream) \
+                     : launch_tiles<MB_STORE, float, COLUMNS / 64, ROWS / 64, true, false, EACH>(a, w, nullptr, out, places, N, K, tiles_m, groups, stream)
+    FW_GROUPED_TILE(64, 128, 2);
+    FW_GROUPED_TILE(128, 128, 2);
+    FW_GROUPED_TILE(128, 192, 1);
+    FW_GROUPED_TILE(128, 256, 1);
+    FW_GROUPED_TILE(192, 192, 1);
+    FW_GROUPED_TILE(192, 256, 1);
+    FW_GROUPED_TILE(256, 256, 1);
+#undef FW_GROUPED_TILE
+    fw_set_error("grouped_gemm: no tile of %d x %d", plan.rows, plan.columns);
+    return -1;
 }
 
 // The tile a storing or accumulating product is cut into: 256 or 128 rows by 256 or 192 columns,

@@ -386,8 +386,8 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(const TA* __restrict_
 // registers (two slabs ahead of the one multiplied) -> LDS (one ahead), two LDS buffers, one barrier an
 // iteration. Two shapes of tile:
 //   BIG     128 places x 128 rows of W; four waves as 2 x 2, each 64 x 64. For steps in which an expert
-//           has hundreds of places (prompts) and that do not go straight to LDS (fw_grouped_gemm_large_fits): a clamped
-//           unit, a K that is no multiple of 32, few tiles over a long K.
+//           has many places (prompts) and that do not go straight to LDS (gemm_mfma_big.hip): a clamped
+//           unit, a K that is no multiple of 32, few tiles over the longest K.
 //   small    32 places x (128 NJ) rows of W; four waves side by side, each 32 x (32 NJ). For steps of
 //           few places an expert (decoding): the product is bound by how fast the experts' weights stream,
 //           and every workgroup streams rows of W that no other reads.
@@ -600,12 +600,8 @@ static int grouped_mfma_launch(const void* a, const int32_t* place_row, const vo
     return 0;
 }
 
-// Whether a product of many places an expert (bfloat16, the plain unit) goes straight to LDS on the large tiles: with a short K, and where
-// they are about a round over the chip (every expert's last tile half full in the mean). Fewer of them over a long K leave the streaming of W
-// to too few workgroups: 8 experts, 200 / 384 / 1,111 places, 1,024 features over K 2,048 28 / 29 / 29 us against 25 / 26 / 28 through registers, 32
-// experts of 100 places, 288 over 16,832 311 against 173; over K 576 to 960 they win down to 8 tiles (10.5 us against 11.6, 14.3 against 15.3).
-// 140 tiles over K 1,952 35.5 against 42.8, but 148 over 3,232 53.7 against 45.5. Tiles that are half padding win while they are less than a round (10.9 us
-// against 12.8) and lose beyond (32 features of 128 experts, 41,352 places 12.3 against 11.5).
+// Whether a product of many places an expert (bfloat16, the plain unit) is worth tiles of more than 128 places: where tiles of 128 x 256 are about a round over the
+// chip (every expert's last tile half full in the mean), or K is short. Elsewhere the lower ones stream W through more workgroups.
 extern "C" int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int experts, int N, int K) {
     if ((long long)places < 48ll * experts || !fw_grouped_big_takes(a_rows, N, K)) return 0;
     const int features = gated ? 128 : 256;
@@ -629,8 +625,13 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
         (out_dtype == FW_F32 || (out_dtype == FW_BF16 && gated))) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
-        if (glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K))
-            status = fw_launch_grouped_big(a, place_row, w, expert_begin, out, gated, places, experts, N, K, s);
+        // ... straight to LDS, on the tile that the experts' places ask for, from 24 places an expert, with a short K from 48 (fewer leave most of a tile of 64
+        // empty: 64 experts, 768 features over 1,024, 19 places an expert, down 18.7 us on tiles of 32 and 19.4; 40 of 3,000 over 320, 25 places 18.2 / 19.6; but 32 of 2,048
+        // over 1,536, 25 places 48.7 / 41.5, 8 of 1,024 over 2,048, 48 places, gated 31.1 / 16.9), not over the longest K (32 of 288 over 16,832, 100 places 175 / 191)
+        const bool tall = fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) != 0;
+        const bool straight = tall || (K <= 16384 && (long long)places >= (K >= 1024 ? 24ll : 48ll) * experts && fw_grouped_big_takes(a_rows, N, K));
+        if (glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && straight)
+            status = fw_launch_grouped_big(a, place_row, w, expert_begin, out, gated, places, experts, N, K, tall, s);
         else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
                                 : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);
         else status = big ? grouped_mfma_launch<false, true, 2, float>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
