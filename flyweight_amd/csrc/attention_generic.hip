@@ -169,6 +169,168 @@ __global__ __launch_bounds__(64) void qk_norm_rope_kv_write_rows_kernel(
     }
 }
 
+// The same once more for heads of 64 and 128 channels and values of whole 64s whose rows lie at 16 bytes: a lane holds four neighbouring channels, HEAD_LANES
+// lanes a head, 64 / HEAD_LANES rows side by side, eight rows of a head-vector to a wave; a value's 64 channels a lane each, as above. With a channel a lane a
+// wave's eight rows were eight sums over 64 lanes one behind the other, six trips through the LDS crossbar each, and every query waited for its row's
+// position, segment and page, which keys and values alone need. What is left is the memory's: float32 sums in, bfloat16 out. 2,048 rows of 32 + 16 heads of 64
+21.3 -> 12.9 us (2.9 TB/s), 801 rows 12.7 -> 8.2; 1,111 rows of 16 + 8 heads of 128 15.2 -> 10.8. The same bits: the squares
+// are added in the order of the sum over a wave, channels 64 apart, then 32, 16, 8 and 4 over the lanes, 2 and 1 in the lane.
+template <typename TI> struct four_of { typedef float4 vector; };
+template <> struct four_of<bf16_t> { typedef uint2 vector; };
+__device__ __forceinline__ void four_floats(const float4 v, float (&x)[4]) { x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w; }
+__device__ __forceinline__ void four_floats(const uint2 v, float (&x)[4]) {
+    x[0] = bf16_bits_to_float(v.x & 0xffff), x[1] = bf16_bits_to_float(v.x >> 16);
+    x[2] = bf16_bits_to_float(v.y & 0xffff), x[3] = bf16_bits_to_float(v.y >> 16);
+}
+__device__ __forceinline__ void store_four(float* to, const float (&x)[4]) { *reinterpret_cast<float4*>(to) = make_float4(x[0], x[1], x[2], x[3]); }
+__device__ __forceinline__ void store_four(bf16_t* to, const float (&x)[4]) {
+    *reinterpret_cast<uint2*>(to) = make_uint2((uint32_t)float_to_bf16_bits(x[0]) | ((uint32_t)float_to_bf16_bits(x[1]) << 16),
+                                               (uint32_t)float_to_bf16_bits(x[2]) | ((uint32_t)float_to_bf16_bits(x[3]) << 16));
+}
+// the value of the lane N below in a row of 16 lanes, round its end
+template <int N> __device__ __forceinline__ float turned_by(float v) { return __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(v), 0x120 + N, 0xF, 0xF, true)); }
+template <typename TI, typename T, int HEAD_LANES>
+__global__ __launch_bounds__(256) void qk_norm_rope_kv_write_wide_kernel(
+    const TI* __restrict__ qkv, T* __restrict__ q_out, const float* __restrict__ q_norm_weight,
+    const float* __restrict__ k_norm_weight, float eps, const float* __restrict__ cos_table,
+    const float* __restrict__ sin_table, int rotary_dim, T* __restrict__ k_pages, T* __restrict__ v_pages,
+    const int32_t* __restrict__ block_table, int table_stride, const int32_t* __restrict__ row_seg,
+    const int32_t* __restrict__ row_pos, int num_heads, int num_kv_heads, int v_dim, int rows, int interleaved, int width,
+    const float* __restrict__ q_row_scale, int units) {
+    constexpr int D = 4 * HEAD_LANES, SIDE = 64 / HEAD_LANES, PASSES = QK_ROWS / SIDE;
+    const int r0 = blockIdx.x * QK_ROWS, lane = threadIdx.x & 63;
+    const int unit = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (unit >= units) return;
+    if (unit >= num_heads + num_kv_heads) {     // 64 channels of a value head: transposed store
+        const int blocks = v_dim / 64, kvh = (unit - num_heads - num_kv_heads) / blocks, d = (unit - num_heads - num_kv_heads) % blocks * 64 + lane;
+        const size_t first = (size_t)(num_heads + num_kv_heads) * D + (size_t)kvh * v_dim + d;
+        int pos[QK_ROWS], page[QK_ROWS];
+        float v[QK_ROWS];
+#pragma unroll
+        for (int i = 0; i < QK_ROWS; ++i) {
+            const int row = r0 + i < rows ? r0 + i : rows - 1;
+            v[i] = load_as_float(qkv + (size_t)row * width, first);
+            pos[i] = row_pos[row];
+            page[i] = row_seg[row];
+        }
+#pragma unroll
+        for (int i = 0; i < QK_ROWS; ++i) page[i] = block_table[(size_t)page[i] * table_stride + pos[i] / ATTN_PAGE];
+        // eight rows that follow each other in one page leave as one store (see above)
+        bool together = sizeof(T) == 2 && r0 + QK_ROWS <= rows && pos[0] % 8 == 0 && (uintptr_t)v_pages % 16 == 0;
+#pragma unroll
+        for (int i = 1; i < QK_ROWS; ++i) together = together && page[i] == page[0] && pos[i] == pos[0] + i;
+        if (together) {
+            uint32_t packed[QK_ROWS / 2];
+#pragma unroll
+            for (int i = 0; i < QK_ROWS / 2; ++i) packed[i] = (uint32_t)float_to_bf16_bits(v[2 * i]) | ((uint32_t)float_to_bf16_bits(v[2 * i + 1]) << 16);
+            T* to = v_pages + (((size_t)page[0] * num_kv_heads + kvh) * v_dim + d) * ATTN_PAGE + pos[0] % ATTN_PAGE;
+            *reinterpret_cast<uint4*>(to) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < QK_ROWS; ++i)
+            if (r0 + i < rows) store_from_float(v_pages, (((size_t)page[i] * num_kv_heads + kvh) * v_dim + d) * ATTN_PAGE + pos[i] % ATTN_PAGE, v[i]);
+        return;
+    }
+    const bool is_query = unit < num_heads;
+    const int own = lane % HEAD_LANES, half = rotary_dim / 2;      // this lane's channels are 4 own .. 4 own + 3
+    const bool turned = 4 * own < rotary_dim;
+    const bool is_first = 4 * own < half;                          // halves: the four channels are all in one of them
+    const int pair = interleaved ? 2 * own : (is_first ? 4 * own : 4 * own - half);
+    const float* weight = is_query ? q_norm_weight : k_norm_weight;
+    int row_of[PASSES], pos[PASSES], page[PASSES];
+    typename four_of<TI>::vector got[PASSES];
+    float4 c[PASSES] = {}, s[PASSES] = {};
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const int row = r0 + i * SIDE + lane / HEAD_LANES;
+        row_of[i] = row < rows ? row : rows - 1;
+        if (!is_query) {                                            // asked for ahead of the rows: the page is another trip behind them
+            pos[i] = row_pos[row_of[i]];
+            page[i] = row_seg[row_of[i]];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        got[i] = *reinterpret_cast<const typename four_of<TI>::vector*>(qkv + (size_t)row_of[i] * width + (size_t)unit * D + 4 * own);
+        if (turned) {
+            const float *from_c = cos_table + (size_t)row_of[i] * half + pair, *from_s = sin_table + (size_t)row_of[i] * half + pair;
+            if (interleaved) {
+                const float2 two_c = *reinterpret_cast<const float2*>(from_c), two_s = *reinterpret_cast<const float2*>(from_s);
+                c[i] = make_float4(two_c.x, two_c.x, two_c.y, two_c.y);
+                s[i] = make_float4(-two_s.x, two_s.x, -two_s.y, two_s.y);
+            } else {
+                c[i] = *reinterpret_cast<const float4*>(from_c);
+                const float4 four = *reinterpret_cast<const float4*>(from_s);
+                s[i] = is_first ? make_float4(-four.x, -four.y, -four.z, -four.w) : four;
+            }
+        }
+    }
+    T* dest[PASSES];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        if (is_query) {
+            dest[i] = q_out + ((size_t)row_of[i] * num_heads + unit) * D;
+        } else {
+            page[i] = block_table[(size_t)page[i] * table_stride + pos[i] / ATTN_PAGE];
+            dest[i] = k_pages + (((size_t)page[i] * num_kv_heads + (unit - num_heads)) * ATTN_PAGE + pos[i] % ATTN_PAGE) * D;
+        }
+    }
+    const float4 w4 = weight ? *reinterpret_cast<const float4*>(weight + 4 * own) : make_float4(1.f, 1.f, 1.f, 1.f);
+    const int partner = (lane & ~(HEAD_LANES - 1)) | (turned ? (is_first ? own + half / 4 : own - half / 4) : own);
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        float x[4];
+        four_floats(got[i], x);
+        if (weight) {
+            float square[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) square[u] = fmaf(x[u], x[u], 0.0f);     // rounded: a plain product would be fused with the sum behind it
+            if constexpr (HEAD_LANES == 32) {
+                // the sum that a lane of a wave holds of its two channels: the second joins the first's square in one fused step
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    float low, high;
+                    fw_quad_partners16(x[u], low, high);
+                    square[u] = fmaf(high, high, low * low);
+                }
+            }
+            // turned by 8, 4, 2 and 1 lanes, the sums of a step repeat at that distance: each is its partner's of a butterfly
+#pragma unroll
+            for (int u = 0; u < 4; ++u) square[u] += turned_by<8>(square[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) square[u] += turned_by<4>(square[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) square[u] += turned_by<2>(square[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) square[u] += turned_by<1>(square[u]);
+            const float sum = (square[0] + square[2]) + (square[1] + square[3]);
+            const float inv = rsqrtf(sum / (float)D + eps);
+            x[0] = x[0] * inv * w4.x, x[1] = x[1] * inv * w4.y, x[2] = x[2] * inv * w4.z, x[3] = x[3] * inv * w4.w;
+        }
+        if (rotary_dim) {
+            float other[4];
+            if (interleaved) other[0] = x[1], other[1] = x[0], other[2] = x[3], other[3] = x[2];
+            else if (half == 32)        // eight lanes on, of sixteen
+#pragma unroll
+                for (int u = 0; u < 4; ++u) other[u] = turned_by<8>(x[u]);
+            else
+#pragma unroll
+                for (int u = 0; u < 4; ++u) other[u] = __shfl(x[u], partner, 64);
+            if (turned) {
+                x[0] = fmaf(x[0], c[i].x, other[0] * s[i].x), x[1] = fmaf(x[1], c[i].y, other[1] * s[i].y);
+                x[2] = fmaf(x[2], c[i].z, other[2] * s[i].z), x[3] = fmaf(x[3], c[i].w, other[3] * s[i].w);
+            }
+        }
+        if (is_query && q_row_scale) {
+            const float factor = q_row_scale[row_of[i]];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] *= factor;
+        }
+        if (r0 + i * SIDE + lane / HEAD_LANES < rows) store_four(dest[i] + 4 * own, x);
+    }
+}
+
 extern "C" int fw_qk_norm_rope_kv_write(const void* qkv, int in_dtype, int row_stride, void* q_out, int dtype, const float* q_norm_weight,
                                         const float* k_norm_weight, float eps, const float* cos_table,
                                         const float* sin_table, int rotary_dim, void* k_pages, void* v_pages,
@@ -194,7 +356,30 @@ extern "C" int fw_qk_norm_rope_kv_write(const void* qkv, int in_dtype, int row_s
     FW_REQUIRE(vectors <= 65535, "qk_norm_rope: too many heads (%d)", vectors);
     dim3 grid(rows, vectors);
     hipStream_t s = (hipStream_t)stream;
-    if (head_dim <= 64 && v_dim == head_dim && rows >= 8 * QK_ROWS) {    // a prompt's rows, eight to a wave
+    // a prompt's rows, four channels to a lane, where 16 bytes of a row (8 in bfloat16) lie at such a place in everything that is read or stored so
+    auto at = [](const void* p, int bytes) { return (uintptr_t)p % bytes == 0; };
+    const int in_size = in_dtype == FW_F32 ? 4 : 2, out_size = dtype == FW_F32 ? 4 : 2;
+    if ((head_dim == 64 || head_dim == 128) && v_dim % 64 == 0 && rows >= 8 * QK_ROWS && width % 4 == 0 && rotary_dim % 8 == 0 && at(qkv, 4 * in_size) &&
+        at(q_out, 4 * out_size) && at(k_pages, 4 * out_size) && at(q_norm_weight, 16) && at(k_norm_weight, 16) && at(cos_table, 16) && at(sin_table, 16)) {
+        const int units = write_kv ? num_heads + num_kv_heads + num_kv_heads * (v_dim / 64) : num_heads;
+        dim3 wide((rows + QK_ROWS - 1) / QK_ROWS, (units + 3) / 4);
+#define FW_QK_WIDE_LAUNCH(TI, T, LANES)                                                                              \
+    qk_norm_rope_kv_write_wide_kernel<TI, T, LANES><<<wide, 256, 0, s>>>(                                            \
+        (const TI*)qkv, (T*)q_out, q_norm_weight, k_norm_weight, eps, cos_table, sin_table, rotary_dim, (T*)k_pages, \
+        (T*)v_pages, block_table, table_stride, row_seg, row_pos, num_heads, num_kv_heads, v_dim, rows, interleaved, width, q_row_scale, units)
+#define FW_QK_WIDE(TI, T)                                \
+    if (head_dim == 64) FW_QK_WIDE_LAUNCH(TI, T, 16);    \
+    else FW_QK_WIDE_LAUNCH(TI, T, 32)
+        if (in_dtype == FW_F32 && dtype == FW_F32) { FW_QK_WIDE(float, float); }
+        else if (in_dtype == FW_F32 && dtype == FW_BF16) { FW_QK_WIDE(float, bf16_t); }
+        else if (in_dtype == FW_BF16 && dtype == FW_BF16) { FW_QK_WIDE(bf16_t, bf16_t); }
+        else FW_REQUIRE(false, "qk_norm_rope: unsupported dtypes in=%d out=%d", in_dtype, dtype);
+#undef FW_QK_WIDE
+#undef FW_QK_WIDE_LAUNCH
+        FW_LAUNCH_CHECK("qk_norm_rope_kv_write");
+        return 0;
+    }
+    if (head_dim <= 64 && v_dim == head_dim && rows >= 8 * QK_ROWS) {    // smaller heads, eight rows to a wave
         dim3 by_rows((rows + QK_ROWS - 1) / QK_ROWS, vectors);
 #define FW_QK_ROWS_LAUNCH(TI, T)                                                                                     \
     qk_norm_rope_kv_write_rows_kernel<TI, T><<<by_rows, 64, 0, s>>>(                                                 \
