@@ -90,6 +90,9 @@ int fw_gemm_mfma_big_split(const void* a, const void* w, const float* bias, void
 int fw_gemm_mfma_big_tile_needs(int mode, int M, int N, int K, int rows, int columns, int each_cu, int slices, size_t* workspace_bytes, int* counters);
 int fw_gemm_mfma_big_tile(const void* a, const void* w, const float* bias, void* out, int out_dtype, int mode, int M, int N, int K, int rows,
                           int columns, int each_cu, int slices, void* workspace, size_t workspace_bytes, int* counters, int counters_len, void* stream);
+// The gated product with clamped halves (as fw_clamped_glu) on the tile named, out bfloat16.
+int fw_gemm_mfma_big_tile_clamped(const void* a, const void* w, void* out, int M, int N, int K, int rows, int columns, int each_cu, float limit, float alpha,
+                                  float shift, void* stream);
 // The same product for 1..64 rows with K split over workgroups, for the shapes that fw_gemm_rows serves worse.
 // fw_gemm_medium_plan says what a shape needs: bytes of workspace (0: none) and int32 counters (0: none) that are zero before
 // the first call; the kernel leaves them zero. Calls that overlap on one device need their own of both.

@@ -1,4 +1,4 @@
-// The product on large tiles, called by the tile (gemm_mfma_big.h has the kernel; each of the three sources below compiles one epilogue of it).
+// The product on large tiles, called by the tile (gemm_mfma_big.h has the kernel; each of the four sources below compiles one epilogue of it).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -14,6 +14,7 @@ struct BigCall {
     float* partials;
     int* counters;
     hipStream_t stream;
+    float limit = 0.0f, alpha = 0.0f, shift = 0.0f;     // of the gated unit with clamped halves
 };
 
 // whether there is such a tile: `slices` tells those with K cut from the others
@@ -31,3 +32,4 @@ __host__ __device__ inline bool fw_big_tile_exists(int mode, int rows, int colum
 __attribute__((visibility("hidden"))) int fw_launch_big_store(const BigCall& call);
 __attribute__((visibility("hidden"))) int fw_launch_big_add(const BigCall& call);
 __attribute__((visibility("hidden"))) int fw_launch_big_gated(const BigCall& call);
+__attribute__((visibility("hidden"))) int fw_launch_big_clamped(const BigCall& call);

@@ -84,6 +84,16 @@ struct BigSlices {
     int* counters;
 };
 
+// A gated product with this output type stores the unit with clamped halves (fw_gated_unit) in bfloat16.
+struct clamped_bf16_t {
+    uint16_t bits;
+};
+struct BigUnit {
+    float limit, alpha, shift;
+};
+template <typename TO> struct big_clamps { static constexpr bool value = false; };
+template <> struct big_clamps<clamped_bf16_t> { static constexpr bool value = true; };
+
 // A slab: 64 k of the tile's rows (an LDS row is 128 bytes, eight 16-byte chunks). Chunk
 // c of a row lies in slot c ^ swap(row): a read of 16 rows by four chunks goes in groups of 16 lanes, 0-3, 12-15 and 20-27, then the 16
 // others of the first 32, and every group covers all 64 banks once.
@@ -119,7 +129,7 @@ struct BigTile {
 template <int MODE, typename TO, int TN, int TM, bool GROUPED, bool SPLIT, int EACH_CU>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EACH_CU))) void gemm_mfma_big_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ w, const float* __restrict__ bias,
-    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups, const BigSlices cut) {
+    TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int per_xcd, int up_offset, const BigGroups groups, const BigSlices cut, const BigUnit halves) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];      // [A_STAGES slabs of a][W_STAGES slabs of w]
     typedef BigTile<TM, TN, EACH_CU> Tile;
     constexpr int ROWS = Tile::ROWS, WIDE = Tile::WIDE, A_SLAB = Tile::A_SLAB, W_SLAB = Tile::W_SLAB, A_STAGES = Tile::A_STAGES, W_STAGES = Tile::W_STAGES;
@@ -424,6 +434,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     const bool odd = lane & 1;
     // (the grouped product has the unit of its form for few places, bit for bit)
     auto unit = [](float g) { return GROUPED ? silu_big(g) : silu_quick(g); };
+    auto gated = [&](float g, float u) {
+        if constexpr (big_clamps<TO>::value) {
+            g = fminf(g, halves.limit);
+            u = fminf(fmaxf(u, -halves.limit), halves.limit);
+            return g * __builtin_amdgcn_rcpf(1.0f + __expf(-halves.alpha * g)) * (u + halves.shift);
+        } else {
+            return fw_gate_of<TO>(g, unit) * u;
+        }
+    };
     const uint32_t first_row = (uint32_t)(wm * (TM * 32) + row_base);      // of this lane, of the tile
     // the eight rows of row tile i and pair j of column tiles that this lane holds: gated, or with the bias
     constexpr int SHARE = MODE == MB_SWIGLU ? TN * 16 : TN * 32, PAIRS = SHARE / 32;       // columns of the output that a wave holds
@@ -432,8 +451,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             if constexpr (MODE == MB_SWIGLU) {
-                left[r] = fw_gate_of<TO>(acc[i][2 * j][r], unit) * acc[i][2 * j + TN][r];
-                right[r] = fw_gate_of<TO>(acc[i][2 * j + 1][r], unit) * acc[i][2 * j + 1 + TN][r];
+                left[r] = gated(acc[i][2 * j][r], acc[i][2 * j + TN][r]);
+                right[r] = gated(acc[i][2 * j + 1][r], acc[i][2 * j + 1 + TN][r]);
             } else {
                 left[r] = acc[i][2 * j][r];
                 right[r] = acc[i][2 * j + 1][r];
@@ -450,7 +469,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
     const uint32_t lone_row = (uint32_t)(wm * (TM * 32) + (lane >> 4) * 4);
     auto lone_values = [&](int i, float (&rows)[4]) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) rows[r] = fw_gate_of<TO>(acc[i][TN - 1][r], unit) * acc[i][2 * TN - 1][r];
+        for (int r = 0; r < 4; ++r) rows[r] = gated(acc[i][TN - 1][r], acc[i][2 * TN - 1][r]);
     };
     if (SIZE == 4 || ((N & 1) == 0 && (uintptr_t)out % 4 == 0)) {
 #pragma unroll
@@ -538,7 +557,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
 
 template <int MODE, typename TO, int TN, int TM, bool GROUPED, bool SPLIT, int EACH_CU>
 static int launch_tiles(const void* a, const void* w, const float* bias, void* out, int M, int N, int K, int tiles_m, const BigGroups& groups,
-                        hipStream_t stream, const BigSlices& cut = BigSlices()) {
+                        hipStream_t stream, const BigSlices& cut = BigSlices(), const BigUnit& halves = BigUnit()) {
     const int tiles_n = fw_ceil_div(N, BigTile<TM, TN, EACH_CU>::WIDE / (MODE == MB_SWIGLU ? 2 : 1));
     const int per_xcd = fw_ceil_div((long long)tiles_m * tiles_n * (SPLIT ? cut.slices : 1), 8);
     const int lds_bytes = BigTile<TM, TN, EACH_CU>::LDS;
@@ -553,7 +572,7 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
         configured = true;
     }
     gemm_mfma_big_kernel<MODE, TO, TN, TM, GROUPED, SPLIT, EACH_CU><<<per_xcd * 8, 256, lds_bytes, stream>>>(
-        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups, cut);
+        (const uint16_t*)a, (const uint16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, per_xcd, N, groups, cut, halves);
     return 0;
 }
 
@@ -561,5 +580,5 @@ static int launch_tiles(const void* a, const void* w, const float* bias, void* o
 template <int MODE, typename TO, int TN, int TM, int EACH_CU, bool SPLIT>
 static int launch_big(const BigCall& c) {
     const BigSlices cut = {c.slices, c.k_each, c.partials, c.counters};
-    return launch_tiles<MODE, TO, TN, TM, false, SPLIT, EACH_CU>(c.a, c.w, c.bias, c.out, c.M, c.N, c.K, fw_ceil_div(c.M, TM * 64), BigGroups(), c.stream, cut);
+    return launch_tiles<MODE, TO, TN, TM, false, SPLIT, EACH_CU>(c.a, c.w, c.bias, c.out, c.M, c.N, c.K, fw_ceil_div(c.M, TM * 64), BigGroups(), c.stream, cut, {c.limit, c.alpha, c.shift});
 }

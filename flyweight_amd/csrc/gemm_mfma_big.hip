@@ -248,3 +248,21 @@ extern "C" int fw_gemm_mfma_big_tile(const void* a, const void* w, const float* 
     FW_LAUNCH_CHECK("gemm_mfma_big_tile");
     return 0;
 }
+
+// The gated product with clamped halves on the tile named: out bfloat16 [M][N] = g sigmoid(alpha g) (u + shift), g = min(gate, limit), u = clamp(up, -limit,
+// limit), formed from the float32 sums. The sums in memory and a pass over them took 83 + 23 us of 1,111 x 8,192 over K 2,048, this 75 (tiles of 192 x 128); 277 rows 30 + 6 and 29.
+extern "C" int fw_gemm_mfma_big_tile_clamped(const void* a, const void* w, void* out, int M, int N, int K, int rows, int columns, int each_cu, float limit, float alpha,
+                                             float shift, void* stream) {
+    size_t need_bytes = 0;
+    int need_counters = 0;
+    if (check_operands(a, w, nullptr, FW_BF16, MB_SWIGLU, M, N, K)) return -1;
+    if (fw_gemm_mfma_big_tile_needs(MB_SWIGLU, M, N, K, rows, columns, each_cu, 1, &need_bytes, &need_counters)) return -1;
+    FW_REQUIRE(limit > 0.0f, "gemm_mfma_big_tile_clamped: the limit must be positive");
+    BigCall call = {a, w, nullptr, out, FW_BF16, M, N, K, rows, columns, each_cu, 1, K, nullptr, nullptr, (hipStream_t)stream};
+    call.limit = limit;
+    call.alpha = alpha;
+    call.shift = shift;
+    if (fw_launch_big_clamped(call)) return -1;
+    FW_LAUNCH_CHECK("gemm_mfma_big_tile_clamped");
+    return 0;
+}

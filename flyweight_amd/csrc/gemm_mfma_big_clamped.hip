@@ -1,0 +1,28 @@
+// The large tiles' gated products whose unit clamps its halves (gemm_mfma_big.h), on the tile that the call names.
+#include "gemm_mfma_big.h"
+
+template <typename TO>
+static int launch(const BigCall& c) {
+#define FW_TILE(ROWS, COLUMNS, EACH, CUT) \
+    if (c.rows == ROWS && c.columns == COLUMNS && c.each_cu == EACH && (c.slices > 1) == CUT) return launch_big<MB_SWIGLU, TO, COLUMNS / 64, ROWS / 64, EACH, CUT>(c)
+    FW_TILE(64, 128, 1, false);
+    FW_TILE(64, 128, 2, false);
+    FW_TILE(128, 128, 1, false);
+    FW_TILE(128, 128, 2, false);
+    FW_TILE(192, 128, 1, false);
+    FW_TILE(64, 192, 1, false);
+    FW_TILE(128, 192, 1, false);
+    FW_TILE(192, 192, 1, false);
+    FW_TILE(256, 192, 1, false);
+    FW_TILE(128, 256, 1, false);
+    FW_TILE(192, 256, 1, false);
+    FW_TILE(256, 256, 1, false);
+    FW_TILE(256, 320, 1, false);
+#undef FW_TILE
+    fw_set_error("gemm_mfma_big: no tile of %d x %d, %d on a compute unit, K in %d slices", c.rows, c.columns, c.each_cu, c.slices);
+    return -1;
+}
+
+int fw_launch_big_clamped(const BigCall& c) {
+    return launch<clamped_bf16_t>(c);
+}

@@ -1910,6 +1910,22 @@ def clamped_glu(gate_up: torch.Tensor, limit: float, alpha: float, shift: float,
     return out
 
 
+def gemm_clamped_glu(a: torch.Tensor, w_gate_up: torch.Tensor, limit: float, alpha: float, shift: float) -> Optional[torch.Tensor]:
+    """clamped_glu(a . [gate | up]^T) in bfloat16 for more than 64 rows by weights that a model holds, the unit in the product's epilogue; None where no large
+    tile takes the product (``large_tile``)."""
+    rows2, K = w_gate_up.shape
+    M = a.shape[0]
+    if rows2 % 2 or a.shape[1] != K or M <= MEDIUM_MAX_ROWS or not _fast_ok(a, w_gate_up) or not limit > 0.0:
+        return None
+    tile = large_tile(2, M, rows2 // 2, K)
+    if tile is None:
+        return None
+    _dev(a, w_gate_up)
+    out = torch.empty((M, rows2 // 2), dtype=torch.bfloat16, device=a.device)
+    _check(library().fw_gemm_mfma_big_tile_clamped(a.data_ptr(), w_gate_up.data_ptr(), out.data_ptr(), M, rows2 // 2, K, *tile[:3], limit, alpha, shift, _stream()))
+    return out
+
+
 # ---- a sublayer between two norms, layer norm, the gate on a second token table ------------------------------
 NEXT_NOTHING, NEXT_ROUNDED, NEXT_RMS, NEXT_CENTERED = 0, 1, 2, 3
 

@@ -162,14 +162,18 @@ class Linear:
 
     def clamped_glu(self, a: Input, limit: float, alpha: float, shift: float) -> torch.Tensor:
         """The weight holds gate rows then up rows: g * sigmoid(alpha g) * (u + shift) with g = min(gate,
-        limit), u = clamp(up, -limit, limit). In the products of few rows the unit is the product's
-        epilogue, as SwiGLU is; a prompt's product leaves float32 sums and a kernel of its own forms it."""
+        limit), u = clamp(up, -limit, limit). In the products of few rows and on
+        the large tiles the unit is the product's epilogue, as SwiGLU is; the others leave float32 sums and a kernel of its own forms it."""
         if self.bias is None and self._medium(a):
             return ops.gemm_medium(self._rows_of(a), self.weight, ops.EPILOGUE_SWIGLU, w_tiled=self.tiled, glu=(limit, alpha, shift),
                                    **self._prepared_arguments(a))
         if self.bias is None and self._fused(a, self.out_features // 2, ops.EPILOGUE_SWIGLU):
             return ops.gemm_decode(self._rows_of(a), self.weight, ops.EPILOGUE_SWIGLU, out_dtype=torch.bfloat16,
                                    w_tiled=self.tiled, glu=(limit, alpha, shift), **self._norm_arguments(a))
+        if self.bias is None and self.tiled is not None and a.dtype == torch.bfloat16:
+            made = ops.gemm_clamped_glu(self._tensor_of(a), self.weight, limit, alpha, shift)
+            if made is not None:
+                return made
         return ops.clamped_glu(self.forward(a, out_dtype=torch.float32), limit, alpha, shift, a.dtype)
 
     def short_conv_decode(self, a: Input, taps: torch.Tensor, conv_bias: Optional[torch.Tensor], state: torch.Tensor,
