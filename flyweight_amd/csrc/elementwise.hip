@@ -52,6 +52,39 @@ __global__ __launch_bounds__(256) void embed_copies_kernel(const bf16_t* __restr
     }
 }
 
+// One copy of a prompt's rows, four channels to a thread where table and rows lie so (the same bits). 2,048 rows of 2,048 18.1 -> 10.4 us, with a vector per
+// position 22.9 -> 13.0.
+template <typename W> __device__ __forceinline__ void embed_four(const W* from, float (&v)[4]);
+template <> __device__ __forceinline__ void embed_four<float>(const float* from, float (&v)[4]) {
+    const float4 four = *reinterpret_cast<const float4*>(from);
+    v[0] = four.x, v[1] = four.y, v[2] = four.z, v[3] = four.w;
+}
+template <> __device__ __forceinline__ void embed_four<bf16_t>(const bf16_t* from, float (&v)[4]) {
+    const uint2 four = *reinterpret_cast<const uint2*>(from);
+    v[0] = bf16_bits_to_float(four.x & 0xffff), v[1] = bf16_bits_to_float(four.x >> 16);
+    v[2] = bf16_bits_to_float(four.y & 0xffff), v[3] = bf16_bits_to_float(four.y >> 16);
+}
+template <typename W, typename P>
+__global__ __launch_bounds__(256) void embed_rows_wide_kernel(const W* __restrict__ table, const int32_t* __restrict__ ids, float* __restrict__ out, int hidden,
+                                                              float scale, const P* __restrict__ places_table, const int32_t* __restrict__ places) {
+    const int row = blockIdx.y;
+    const size_t base = (size_t)ids[row] * hidden, place = places ? (size_t)places[row] * hidden : 0;
+    for (int i = (blockIdx.x * 256 + threadIdx.x) * 4; i < hidden; i += gridDim.x * 1024) {
+        float v[4], p[4];
+        embed_four<W>(table + base + i, v);
+        if (places) {
+#pragma clang fp contract(off)          // the product is rounded by itself, as above
+            embed_four<P>(places_table + place + i, p);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = v[e] * scale + p[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] *= scale;
+        }
+        *reinterpret_cast<float4*>(out + (size_t)row * hidden + i) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
 extern "C" int fw_embed_rows(const void* table, int table_dtype, const int32_t* ids, float* out,
                              int rows, int hidden, int vocab, float scale, const void* places_table, int places_dtype,
                              const int32_t* places, int places_entries, int copies, void* stream) {
@@ -69,6 +102,19 @@ extern "C" int fw_embed_rows(const void* table, int table_dtype, const int32_t* 
         return 0;
     }
     if (places == nullptr) places_dtype = table_dtype;
+    auto lies = [](const void* p, int dtype) { return (uintptr_t)p % (dtype == FW_F32 ? 16 : 8) == 0; };
+    if (copies == 1 && rows >= 64 && hidden % 4 == 0 && lies(table, table_dtype) && lies(out, FW_F32) && (places == nullptr || lies(places_table, places_dtype))) {
+        const dim3 by_four(fw_ceil_div(hidden, 1024) > 64 ? 64 : fw_ceil_div(hidden, 1024), rows);
+#define FW_EMBED_WIDE(W, P) embed_rows_wide_kernel<W, P><<<by_four, 256, 0, s>>>((const W*)table, ids, out, hidden, scale, (const P*)places_table, places)
+        if (table_dtype == FW_F32 && places_dtype == FW_F32) FW_EMBED_WIDE(float, float);
+        else if (table_dtype == FW_BF16 && places_dtype == FW_BF16) FW_EMBED_WIDE(bf16_t, bf16_t);
+        else if (table_dtype == FW_BF16 && places_dtype == FW_F32) FW_EMBED_WIDE(bf16_t, float);
+        else if (table_dtype == FW_F32 && places_dtype == FW_BF16) FW_EMBED_WIDE(float, bf16_t);
+        else FW_REQUIRE(false, "embed_rows: unknown table dtypes %d, %d", table_dtype, places_dtype);
+#undef FW_EMBED_WIDE
+        FW_LAUNCH_CHECK("embed_rows");
+        return 0;
+    }
 #define FW_EMBED_LAUNCH(W, P) \
     embed_rows_kernel<W, P><<<grid, 256, 0, s>>>((const W*)table, ids, out, hidden, scale, (const P*)places_table, places, copies)
     if (table_dtype == FW_F32 && places_dtype == FW_F32) FW_EMBED_LAUNCH(float, float);

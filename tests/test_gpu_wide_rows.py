@@ -44,3 +44,16 @@ def test_sum_of_a_rows_experts(rows, hidden, top, shared):
     more = {"shared": b, "gate": gate} if shared else {}
     want = ops.moe_combine_(off(x), y, weight, place, **more)
     assert torch.equal(ops.moe_combine_(x.clone(), y, weight, place, **more), want)
+
+
+@pytest.mark.parametrize("table_dtype,places_dtype", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, None), (torch.float32, None)])
+@pytest.mark.parametrize("rows,hidden", [(64, 4), (65, 1028), (300, 2048), (64, 66000)])
+def test_rows_of_a_table(rows, hidden, table_dtype, places_dtype):
+    from flyweight_amd.kernels import ops
+    print(rows, hidden, table_dtype, places_dtype, flush=True)
+    g = torch.Generator().manual_seed(rows)
+    table, places = torch.randn(50, hidden, generator=g).to(DEV, table_dtype), torch.randn(400, hidden, generator=g).to(DEV, places_dtype or table_dtype)
+    ids, at = (torch.randint(0, n, (rows,), generator=g).to(DEV, torch.int32) for n in (50, 400))
+    more = {} if places_dtype is None else {"places_table": places, "places": at}
+    want = ops.embed_rows(off(table), ids, scale=1.7, **more)
+    assert torch.equal(ops.embed_rows(table, ids, scale=1.7, **more), want)
