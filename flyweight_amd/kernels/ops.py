@@ -2240,10 +2240,10 @@ def moe_arrange(chosen: torch.Tensor, experts: int):
 
 
 def grouped_few_tiles(places: int, experts: int) -> int:
-    """Tiles of 16 places to a workgroup of the grouped product whose experts' weights come in operand tiles (fw_grouped_gemm_few), 0 where the tiles
-    of moe.hip and gemm_mfma_big.hip are faster. By places an expert in the mean, us for both products (those tiles / one / two): 32 experts of 1,536 features over 2,048,
-    4 a row, 1 / 8 / 32 / 64 / 96 / 128 rows 37 / 21 / 23, 87 / 65 / 67, 122 / 95 / 97, 126 / 101 / 103, 127 / 112 / 109, 128 / 145 / 118; 8 of 4,096 over 2,048, 2 a row, 8 / 32 /
-    64 / 128 rows 95 / 58 / 63, 108 / 73 / 78, 109 / 94 / 86, 112 / 153 / 149."""
+    """Tiles of 16 places to a wave of the grouped product whose experts' weights come in operand tiles (fw_grouped_gemm_few), 0 where the tiles
+    of moe.hip and gemm_mfma_big.hip are faster (the bits are the same). By places an expert in the mean, us for both products (those tiles / one / two): 32 experts of
+    1,536 features over 2,048, 4 a row, 1 / 8 / 32 / 64 / 96 / 128 rows 37 / 19 / -, 87 / 64 / -, 121 / 92 / 93, 126 / 99 / 97, 127 / 109 / 101, 128 / 143 / 108; 8 of 4,096
+    over 2,048, 2 a row, 8 / 32 / 64 rows 90 / 58 / 58, 109 / 71 / 72, 110 / 89 / 74."""
     return 1 if places <= 8 * experts else 2 if places <= 16 * experts else 0
 
 

@@ -74,6 +74,30 @@ def test_a_places_sums_do_not_depend_on_the_step(ops, monkeypatch):
         assert torch.equal(run(first, count, place_tiles), everything[first:first + count])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("experts,top,K,N", [(4, 2, 1536, 96), (5, 1, 2080, 41), (8, 4, 544, 264)])
+@pytest.mark.parametrize("glu", [None, (1.0, 1.702, 1.0)])
+def test_a_row_has_the_same_bits_alone_and_among_hundreds(ops, experts, top, K, N, glu):
+    """Steps of a few places an expert, of the tiles of 32 places beside them (17 to 23 an expert) and of prompts: every place's sums have one order of k."""
+    rows, rng = 200 * experts // top, np.random.default_rng(K)
+    g = torch.Generator().manual_seed(K)
+    a, w = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(DEV), (torch.randn(experts, 2 * N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    tiled, chosen = ops.tile_weights(w.view(-1, K)), torch.from_numpy(np.stack([rng.permutation(experts)[:top] for _ in range(rows)]).astype(np.int32)).to(DEV)
+
+    def run(first, count):
+        begin, place_row, pair_place = ops.moe_arrange(chosen[first:first + count].contiguous(), experts)
+        own = a[first:first + count].contiguous()
+        return [ops.grouped_gemm(own, place_row, w, begin, count * top, gated=gated, out_dtype=dtype, glu=glu if gated else None, w_tiled=tiled)[pair_place.long()]
+                for gated, dtype in ((True, torch.bfloat16), (False, torch.float32))]
+
+    everything, taken = run(0, rows), set()
+    for first, count in ((0, 1), (rows - 3, 3), (7, 7 * experts // top), (3, 14 * experts // top), (1, 20 * experts // top)):
+        taken.add(ops.grouped_few_tiles(count * top, experts))
+        for part, whole in zip(run(first, count), everything):
+            assert torch.equal(part, whole[first:first + count])
+    assert taken == {0, 1, 2}
+
+
 @pytest.mark.parametrize("places,experts,tiles", [(1, 32, 1), (256, 32, 1), (257, 32, 2), (512, 32, 2), (513, 32, 0), (8192, 32, 0)])
 def test_tiles_of_places(ops, places, experts, tiles):
     assert ops.grouped_few_tiles(places, experts) == tiles
