@@ -8,6 +8,7 @@
 // dtype codes used across the C ABI
 #define FW_F32 0
 #define FW_BF16 1
+#define FW_BF16_TILES 4     // bfloat16 weights in operand tiles: 16 rows x 32 columns, 1 KB each, [ceil(rows / 16)][K / 32][4][16][8]
 
 // ---- error channel: every entry point returns 0 or -1 and leaves a message ---------
 void fw_set_error(const char* format, ...);

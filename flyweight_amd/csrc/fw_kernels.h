@@ -436,7 +436,8 @@ int fw_moe_arrange(const int32_t* chosen, int32_t* expert_begin, int32_t* place_
 // out[place] = a[place_row ? place_row[place] : place] . w[expert of place]^T; w [experts][N][K], or with
 // gated [experts][2 N][K] (gate rows, then up rows) and out = silu(gate) * up, or with a glu_limit > 0 the clamped
 // unit g sigmoid(glu_alpha g) (u + glu_shift), g = min(gate, limit), u = clamp(up, -limit, limit). out [places][N].
-// a holds a_rows rows; place_row names no other.
+// a holds a_rows rows; place_row names no other. w_dtype FW_BF16_TILES: w's rows, all experts' one behind the other, in operand tiles (a bfloat16 at 16 bytes, K a multiple
+// of 32, out bfloat16 (gated) or float32); the same bits.
 int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                     const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
                     float glu_limit, float glu_alpha, float glu_shift, void* stream);

@@ -70,10 +70,10 @@ extern "C" int fw_grouped_gemm_tile(int gated, int places, int experts, int N, i
     return 0;
 }
 
-// `tall`: tiles of more than 128 places are worth a look (fw_grouped_gemm_large_fits)
-int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated, int places,
+// `tiled`: w in operand tiles; `tall`: tiles of more than 128 places are worth a look (fw_grouped_gemm_large_fits)
+int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, bool tiled, const int32_t* expert_begin, void* out, int gated, int places,
                           int experts, int N, int K, bool tall, hipStream_t stream) {
-    const BigGroups groups = {place_row, expert_begin, experts};
+    const BigGroups groups = {place_row, expert_begin, experts, tiled};
     const GroupedTime& plan = grouped_plan(gated, places, experts, N, K, tall);
     const int tiles_m = places / plan.rows + (experts < places ? experts : places);       // at most: every expert's last tile may not be full
     // (what the product through registers, whose tiles have half the features, would refuse is refused here too)

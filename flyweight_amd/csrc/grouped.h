@@ -5,8 +5,8 @@
 
 // gemm_mfma_big.hip: fw_grouped_gemm on large tiles, for bfloat16 operands, the plain unit and outputs of bfloat16 (gated) or float32
 __attribute__((visibility("hidden"))) bool fw_grouped_big_takes(int a_rows, int N, int K);
-__attribute__((visibility("hidden"))) int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int gated,
-                                                                int places, int experts, int N, int K, bool tall, hipStream_t stream);
+__attribute__((visibility("hidden"))) int fw_launch_grouped_big(const void* a, const int32_t* place_row, const void* w, bool tiled, const int32_t* expert_begin, void* out,
+                                                                int gated, int places, int experts, int N, int K, bool tall, hipStream_t stream);
 
 struct GroupedTile {
     int expert, row_tile, column_tile;      // expert < 0: none

@@ -416,7 +416,7 @@ template <bool GATED, bool BIG, int NJ, typename TO>
 __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     const uint16_t* __restrict__ a, const int32_t* __restrict__ place_row, const uint16_t* __restrict__ w,
     const int32_t* __restrict__ expert_begin, TO* __restrict__ out, int experts, int N, int K, int tiles_n,
-    const GatedUnit unit) {
+    bool tiled, const GatedUnit unit) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     constexpr int TMR = BIG ? 128 : 32;                 // places of a tile
     constexpr int WAVES_M = BIG ? 2 : 1, WAVES_N = 4 / WAVES_M;
@@ -434,12 +434,14 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     const int features = GATED ? BN / 2 : BN;
     const int n0 = tile.column_tile * features;
     const int wm = BIG ? wave >> 1 : 0, wn = BIG ? wave & 1 : wave;
-    const uint16_t* we = w + (size_t)expert * (GATED ? 2 : 1) * N * K;
 
     const uint16_t* a_src[A_CHUNKS];
     const uint16_t* w_src[W_CHUNKS];
     int a_at[A_CHUNKS], w_at[W_CHUNKS];
     const int kc = (tid & 7) * 8;
+    // this thread's rows and k of W: of operand tiles a wave takes one whole (rows 0 to 15 or 16 to 31 of 32, k 0 to 31 or 32 to 63); both products of 32 experts of 1,536
+    // features over 2,048, 18 places an expert, by rows / tiles 130 / 113 us
+    const int w_row0 = tiled ? (wave >> 1) * 16 + (lane & 15) : tid >> 3, w_kc = tiled ? (wave & 1) * 32 + (lane >> 4) * 8 : kc;
 #pragma unroll
     for (int i = 0; i < A_CHUNKS; ++i) {
         const int row = (tid >> 3) + 32 * i;
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     }
 #pragma unroll
     for (int i = 0; i < W_CHUNKS; ++i) {
-        const int row = (tid >> 3) + 32 * i;
+        const int row = w_row0 + 32 * i;
         int wr;
         if (GATED) {
             wr = row < BN / 2 ? n0 + row : n0 + row - BN / 2;
@@ -461,8 +463,9 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
             wr = n0 + row;
             wr = wr < N ? wr : N - 1;
         }
-        w_src[i] = we + (size_t)wr * K;
-        w_at[i] = ggm_row(row) + (tid & 7) * 16;
+        const size_t w_row = (size_t)expert * (GATED ? 2 : 1) * N + wr;
+        w_src[i] = w + (tiled ? (w_row & ~(size_t)15) * K + (w_row & 15) * 8 : w_row * K);
+        w_at[i] = ggm_row(row) + w_kc * 2;
     }
 
     gg_f32x16 acc[NI][NJ];
@@ -479,18 +482,19 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
     // until it moves to LDS, so that the loads of two slabs stay in flight while a third is multiplied.
     auto fetch = [&](gg_u32x4 (&ra)[A_CHUNKS], gg_u32x4 (&rw)[W_CHUNKS], int k0) {
         const int from = k0 + kc < K ? k0 + kc : 0;     // K is a multiple of 8: columns 0..7 always exist
+        const int w_k = k0 + w_kc < K ? k0 + w_kc : 0, w_from = tiled ? (w_k >> 5) * 512 + (w_k & 24) * 16 : w_k;      // (a tile: 32 k, 8 k in 128 numbers)
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) ra[i] = *reinterpret_cast<const gg_u32x4*>(a_src[i] + from);
 #pragma unroll
-        for (int i = 0; i < W_CHUNKS; ++i) rw[i] = *reinterpret_cast<const gg_u32x4*>(w_src[i] + from);
+        for (int i = 0; i < W_CHUNKS; ++i) rw[i] = *reinterpret_cast<const gg_u32x4*>(w_src[i] + w_from);
     };
     auto stash = [&](const gg_u32x4 (&ra)[A_CHUNKS], const gg_u32x4 (&rw)[W_CHUNKS], int buffer, int k0) {
         unsigned char* base = lds + buffer * (A_SLAB + W_SLAB);
-        const bool ok = k0 + kc < K;                    // a past the end of K is zero; W may then be anything finite
+        const bool ok = k0 + kc < K, w_ok = k0 + w_kc < K;      // a past the end of K is zero; W may then be anything finite
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) *reinterpret_cast<gg_u32x4*>(base + a_at[i]) = ok ? ra[i] : zero;
 #pragma unroll
-        for (int i = 0; i < W_CHUNKS; ++i) *reinterpret_cast<gg_u32x4*>(base + A_SLAB + w_at[i]) = ok ? rw[i] : zero;
+        for (int i = 0; i < W_CHUNKS; ++i) *reinterpret_cast<gg_u32x4*>(base + A_SLAB + w_at[i]) = w_ok ? rw[i] : zero;
     };
     const int a_row0 = wm * 32 * NI + (lane & 31);
     int b_row[NJ];
@@ -578,7 +582,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_mfma_kernel(
 }
 
 template <bool GATED, bool BIG, int NJ, typename TO>
-static int grouped_mfma_launch(const void* a, const int32_t* place_row, const void* w, const int32_t* expert_begin, void* out, int places,
+static int grouped_mfma_launch(const void* a, const int32_t* place_row, const void* w, bool tiled, const int32_t* expert_begin, void* out, int places,
                                int experts, int N, int K, const GatedUnit unit, hipStream_t stream) {
     constexpr int TMR = BIG ? 128 : 32;
     constexpr int BN = (BIG ? 2 : 4) * NJ * 32;
@@ -596,7 +600,7 @@ static int grouped_mfma_launch(const void* a, const int32_t* place_row, const vo
         configured = true;
     }
     grouped_gemm_mfma_kernel<GATED, BIG, NJ, TO><<<per_xcd * 8, 256, lds_bytes, stream>>>(
-        (const uint16_t*)a, place_row, (const uint16_t*)w, expert_begin, (TO*)out, experts, N, K, (int)tiles_n, unit);
+        (const uint16_t*)a, place_row, (const uint16_t*)w, expert_begin, (TO*)out, experts, N, K, (int)tiles_n, tiled, unit);
     return 0;
 }
 
@@ -621,7 +625,10 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
     hipStream_t s = (hipStream_t)stream;
     // bfloat16 operands go to the matrix cores: tiles of 128 places where experts have many, of 32 where few (32 experts, gated 1,536 over
     // 2,048, 37 / 48 / 75 places an expert: tiles of 128 104 / 104 / 101 us, of 32 106 / 118 / 119)
-    if (a_dtype == FW_BF16 && w_dtype == FW_BF16 && K % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0 &&
+    const bool tiled = w_dtype == FW_BF16_TILES;
+    FW_REQUIRE(!tiled || (a_dtype == FW_BF16 && K % 32 == 0 && out_dtype == (gated ? FW_BF16 : FW_F32) && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0),
+               "grouped_gemm: operand tiles take bfloat16 rows at 16 bytes, K a multiple of 32 and leave bfloat16 (gated) or float32");
+    if (a_dtype == FW_BF16 && (w_dtype == FW_BF16 || tiled) && K % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0 &&
         (out_dtype == FW_F32 || (out_dtype == FW_BF16 && gated))) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
@@ -631,11 +638,11 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
         const bool tall = fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) != 0;
         const bool straight = tall || (K <= 16384 && (long long)places >= (K >= 1024 ? 24ll : 48ll) * experts && fw_grouped_big_takes(a_rows, N, K));
         if (glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && straight)
-            status = fw_launch_grouped_big(a, place_row, w, expert_begin, out, gated, places, experts, N, K, tall, s);
-        else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
-                                : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);
-        else status = big ? grouped_mfma_launch<false, true, 2, float>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s)
-                          : grouped_mfma_launch<false, false, 1, float>(a, place_row, w, expert_begin, out, places, experts, N, K, unit, s);
+            status = fw_launch_grouped_big(a, place_row, w, tiled, expert_begin, out, gated, places, experts, N, K, tall, s);
+        else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s)
+                                : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s);
+        else status = big ? grouped_mfma_launch<false, true, 2, float>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s)
+                          : grouped_mfma_launch<false, false, 1, float>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s);
         if (status != 0) return status;
         FW_LAUNCH_CHECK("grouped_gemm");
         return 0;

@@ -14,14 +14,14 @@ import os
 import sys
 import time
 import warnings
-from typing import Dict, Optional
+from typing import Dict, Optional, Union
 
 import torch
 
 from . import build as _build
 
 # (the last two: a storing product leaves gelu of its float32 sums; a gated product gelu_tanh(gate) * up)
-F32, BF16, BF16_GELU, BF16_GEGLU = 0, 1, 2, 3
+F32, BF16, BF16_GELU, BF16_GEGLU, BF16_TILES = 0, 1, 2, 3, 4
 PAGE_SIZE = 64          # tokens per cache page: the width of a wavefront
 COMPUTE_UNITS = 256     # of the chip
 MAX_HEAD_DIM = 256          # of the matrix-core attention kernels
@@ -882,16 +882,29 @@ def tile_weights(w: torch.Tensor) -> Optional[torch.Tensor]:
     return w.view(padded // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous()
 
 
-def tile_expert_weights(w: torch.Tensor) -> Optional[torch.Tensor]:
-    """The experts' stacked weights [experts, rows, K] once more in operand tiles, for steps of a few places an expert; None where the layout does not apply
-    or the copy would leave less than half of the device's memory free (experts are most of a large mixture's weights)."""
-    if not w.is_cuda or w.dtype != torch.bfloat16 or w.shape[2] % 32:
-        return None
-    free, total = torch.cuda.mem_get_info(w.device)
-    reserved = torch.cuda.memory_reserved(w.device) - torch.cuda.memory_allocated(w.device)
-    if free + reserved - w.numel() * w.element_size() < total // 2:
-        return None
-    return tile_weights(w.view(-1, w.shape[2]))
+class ExpertWeights:
+    """The weights [rows, K] of every expert, held once for ``grouped_gemm``: in operand tiles where that layout applies (``tile_weights``), which steps of
+    a few places an expert stream in whole kilobytes and the other products read as they read rows; else one behind the other. ``pieces``: called with an
+    expert's number."""
+
+    def __init__(self, experts: int, pieces):
+        first = pieces(0).contiguous()
+        rows, K = first.shape
+        self.shape = (experts, rows, K)
+        self.rows = self.tiled = None
+        laid = tile_weights(first)
+        if laid is None:
+            self.rows = torch.stack([first, *(pieces(e) for e in range(1, experts))])
+        elif rows % 16:             # experts that meet inside a tile
+            self.tiled = tile_weights(torch.cat([first, *(pieces(e) for e in range(1, experts))]))
+        else:
+            self.tiled = laid.new_empty((experts * laid.shape[0], *laid.shape[1:]))
+            for e, own in enumerate(self.tiled.chunk(experts)):
+                own.copy_(laid if e == 0 else tile_weights(pieces(e).contiguous()))
+
+    @property
+    def held(self) -> torch.Tensor:
+        return self.rows if self.tiled is None else self.tiled
 
 
 @functools.lru_cache(maxsize=4096)
@@ -2247,17 +2260,20 @@ def grouped_few_tiles(places: int, experts: int) -> int:
     return 1 if places <= 8 * experts else 2 if places <= 16 * experts else 0
 
 
-def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: torch.Tensor, expert_begin: torch.Tensor, places: int,
+def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: Union[torch.Tensor, ExpertWeights], expert_begin: torch.Tensor, places: int,
                  gated: bool, out_dtype: torch.dtype, glu: Optional[tuple] = None, w_tiled: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out[place] = a[place_row[place]] . w[expert of place]^T (``place_row`` None: a[place]); ``w`` [experts, N, K], or
     with ``gated`` [experts, 2 N, K] (gate rows, then up rows) and out = silu(gate) * up, or with ``glu`` = (limit, alpha,
     shift) the unit with clamped halves. ``w_tiled``: the rows of ``w`` [experts * N, K] once more in operand tiles
-    (``tile_weights``), for steps of a few places an expert. Returns [places, N]."""
+    (``tile_weights``), for steps of a few places an expert; an ``ExpertWeights`` holds its rows in them alone. Returns [places, N]."""
+    shape = w.shape
+    if isinstance(w, ExpertWeights):
+        w, w_tiled = w.rows, w.tiled
     _dev(a, place_row, w, expert_begin)
-    experts, n_rows, K = w.shape
+    experts, n_rows, K = shape
     N = n_rows // 2 if gated else n_rows
     if a.dim() != 2 or a.shape[1] != K or (gated and n_rows % 2) or expert_begin.numel() != experts + 1:
-        raise KernelError(f"grouped_gemm: a is {tuple(a.shape)}, w {tuple(w.shape)}, {expert_begin.numel()} expert bounds")
+        raise KernelError(f"grouped_gemm: a is {tuple(a.shape)}, w {tuple(shape)}, {expert_begin.numel()} expert bounds")
     _want(expert_begin, torch.int32, "expert_begin")
     if place_row is not None:
         _want(place_row, torch.int32, "place_row")
@@ -2266,14 +2282,18 @@ def grouped_gemm(a: torch.Tensor, place_row: Optional[torch.Tensor], w: torch.Te
     elif a.shape[0] < places:
         raise KernelError("grouped_gemm: fewer rows than places")
     out = torch.empty((places, N), dtype=out_dtype, device=a.device)
+    if w is None and a.data_ptr() % 16:
+        a = a.clone()
     if w_tiled is not None and a.dtype == torch.bfloat16 and out_dtype == (torch.bfloat16 if gated else torch.float32) and a.data_ptr() % 16 == 0:
         place_tiles = grouped_few_tiles(places, experts)
         if place_tiles:
-            w_tiled = _tiled_for(w.view(experts * n_rows, K), w_tiled)
+            if w is not None:
+                w_tiled = _tiled_for(w.view(experts * n_rows, K), w_tiled)
             _check(library().fw_grouped_gemm_few(_p(a), _p(place_row), _p(w_tiled), _p(expert_begin), _p(out), int(gated), int(places), experts, N, K, place_tiles,
                                                  *_glu(glu if gated else None), _stream()))
             return out
-    _check(library().fw_grouped_gemm(_p(a), _code(a.dtype), a.shape[0], _p(place_row), _p(w), _code(w.dtype), _p(expert_begin), _p(out),
+    held, held_code = (w_tiled, BF16_TILES) if w is None else (w, _code(w.dtype))
+    _check(library().fw_grouped_gemm(_p(a), _code(a.dtype), a.shape[0], _p(place_row), _p(held), held_code, _p(expert_begin), _p(out),
                                      _code(out_dtype), int(gated), int(places), experts, N, K, *_glu(glu if gated else None), _stream()))
     return out
 

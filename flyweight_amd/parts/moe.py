@@ -5,7 +5,7 @@ logits are chosen (ties: the lowest id) and weighted by the softmax over the cho
 W_down (silu(W_gate h) * (W_up h)) without biases; the output is the weighted sum of the chosen experts'
 outputs, summed in the order of the choices. ``shared_intermediate_size``: one more unit of that width runs for
 every token and is added. The experts' weights lie stacked ([experts, 2 ff, hidden] gate rows then up rows,
-[experts, hidden, ff]); a step sorts its (token, choice) pairs by expert on the device and runs each expert's
+[experts, hidden, ff], in bfloat16 in operand tiles), once; a step sorts its (token, choice) pairs by expert on the device and runs each expert's
 pairs as tiles of one grouped product, so nothing crosses to the host and a decode step can be recorded.
 
 ``router_scores`` "softmax_all": the scores are the softmax over all experts, and the chosen experts' scores divided by
@@ -121,21 +121,19 @@ class MoeSwiGLU(FeedForward):
         self.router = Linear(router)
         self.correction = tensors[self.prefix + self.names["correction"]] if self.has_correction else None
         self.bias = tensors[self.prefix + self.names["router_bias"]] if self.router_bias else None
-        self.gate_up = torch.stack([torch.cat([tensors[self._expert(e, "gate")], tensors[self._expert(e, "up")]], dim=0)
-                                    for e in range(self.experts)]).contiguous()
-        self.down = torch.stack([tensors[self._expert(e, "down")] for e in range(self.experts)]).contiguous()
-        self.gate_up_tiled, self.down_tiled = ops.tile_expert_weights(self.gate_up), ops.tile_expert_weights(self.down)
+        self.gate_up = ops.ExpertWeights(self.experts, lambda e: torch.cat([tensors[self._expert(e, "gate")], tensors[self._expert(e, "up")]], dim=0))
+        self.down = ops.ExpertWeights(self.experts, lambda e: tensors[self._expert(e, "down")])
         if self.shared is not None:
             self.shared.bind(tensors, dtype, device)
 
     # ----- what a step reads and computes (the experts' weights are read only where tokens chose them) --------
     def gathered_tensors(self):
-        return tuple(t for t in (self.gate_up, self.down, self.gate_up_tiled, self.down_tiled) if t is not None)
+        return (self.gate_up.held, self.down.held)
 
     def chosen_weight_bytes(self, rows: int) -> float:
         """Bytes of the experts that ``rows`` tokens are expected to choose, each ``top`` different ones and
         every expert as likely as any other: experts * (1 - (1 - top / experts) ** rows) of them."""
-        per_expert = (self.gate_up[0].numel() + self.down[0].numel()) * self.gate_up.element_size()
+        per_expert = 3 * self.hidden * self.intermediate * self.gate_up.held.element_size()
         return self.experts * (1.0 - (1.0 - self.top / self.experts) ** max(int(rows), 0)) * per_expert
 
     def chosen_flops_per_token(self) -> int:
@@ -162,8 +160,8 @@ class MoeSwiGLU(FeedForward):
         chosen, weight = self._choose(logits)
         begin, place_row, pair_place = ops.moe_arrange(chosen, self.experts)
         places = rows.shape[0] * self.top
-        hidden = ops.grouped_gemm(rows, place_row, self.gate_up, begin, places, gated=True, out_dtype=rows.dtype, glu=self.glu, w_tiled=self.gate_up_tiled)
-        outputs = ops.grouped_gemm(hidden, None, self.down, begin, places, gated=False, out_dtype=torch.float32, w_tiled=self.down_tiled)
+        hidden = ops.grouped_gemm(rows, place_row, self.gate_up, begin, places, gated=True, out_dtype=rows.dtype, glu=self.glu)
+        outputs = ops.grouped_gemm(hidden, None, self.down, begin, places, gated=False, out_dtype=torch.float32)
         return outputs, weight, pair_place, gate
 
     def _shared_output(self, h, rows, ctx):
