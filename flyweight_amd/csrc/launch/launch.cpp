@@ -2,6 +2,8 @@
 // library's entry points. A step runs some hundred of them one by one, and a short prompt's step is bound by that: written in Python (checks, allocations, an
 // address per argument, ctypes) a product took 11 us of the host's time, of which the launch itself is 3; see ops.py for what each function computes.
 //
+// As with ctypes, other Python threads run while memory is found and the kernel library called: either may wait (for the driver, for room in a queue).
+//
 // A function returns NotImplemented wherever something about its arguments is not as the plain case has it; its caller then takes the general path, which
 // also knows what to refuse and how to say so.
 #include <torch/csrc/autograd/python_variable.h>
@@ -53,6 +55,17 @@ bool same_device(const at::Tensor& a, std::initializer_list<const at::Tensor*> o
 at::Tensor make(const at::Tensor& like, int64_t rows, int64_t columns, at::ScalarType type) { return at::empty({rows, columns}, like.options().dtype(type)); }
 bool fits(int64_t v) { return v >= 0 && v < (1ll << 31); }
 
+// The interpreter's lock is let go while this lives: nothing of Python's is touched meanwhile.
+struct Unlocked {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename Call>
+int unlocked(Call call) {
+    const Unlocked others;
+    return call();
+}
+
 int whole(PyObject* o) { return (int)PyLong_AsLong(o); }
 float number(PyObject* o) { return (float)PyFloat_AsDouble(o); }
 void* stream_of(PyObject* o) { return PyLong_AsVoidPtr(o); }
@@ -93,52 +106,42 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (squares && squares->size(1) != stride) return other_path();
     PyObject* plan = args[15];
     if (!PyTuple_Check(plan) || PyTuple_GET_SIZE(plan) < 6) return other_path();
-    auto planned = [&](int i) { return PyLong_AsSsize_t(PyTuple_GET_ITEM(plan, i)); };
+    const bool large = PyLong_AsSsize_t(PyTuple_GET_ITEM(plan, 0)) == 1;
+    Py_ssize_t planned[7] = {};
+    if (large && (PyTuple_GET_SIZE(plan) != 7 || next_weight || squares)) return other_path();
+    for (int i = 1; i < (large ? 7 : 6); ++i) planned[i] = PyLong_AsSsize_t(PyTuple_GET_ITEM(plan, i));
     const float eps = number(args[11]), limit = number(args[12]), alpha = number(args[13]), shift = number(args[14]);
     void* stream = stream_of(args[17]);
     if (PyErr_Occurred()) return nullptr;
+    // the large tile that is named, K split over workgroups or the product whose waves split K
+    const bool split = !large && planned[1] && (!target || (uintptr_t)target->data_ptr() % 16 == 0);
+    const size_t bytes = large ? (size_t)planned[5] : split ? (size_t)planned[2] : 0;
+    const int tickets = large ? (int)planned[6] : (int)planned[3];
+    if (bytes && (!is(counters, at::kInt, 1) || counters->size(0) < tickets)) return other_path();
 
-    at::Tensor out = target ? *target : make(*a, M, N, rounded ? at::kBFloat16 : at::kFloat);
-    void* to = out.data_ptr();
-    at::Tensor workspace, activations, next_squares;
-    int status;
-    if (planned(0) == 1) {
-        if (next_weight || squares || PyTuple_GET_SIZE(plan) != 7) return other_path();
-        const size_t bytes = (size_t)planned(5);
-        const int tickets = (int)planned(6);
-        if (bytes) {
-            if (!is(counters, at::kInt, 1) || counters->size(0) < tickets) return other_path();
-            workspace = at::empty({(int64_t)(bytes / 4)}, a->options().dtype(at::kFloat));
-        }
-        status = entry.big_tile(a->data_ptr(), w->data_ptr(), at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K, (int)planned(1), (int)planned(2),
-                                (int)planned(3), (int)planned(4), bytes ? workspace.data_ptr() : nullptr, bytes, bytes ? at_of<int>(counters) : nullptr, tickets, stream);
-    } else {
-        const bool split = planned(1) && (uintptr_t)to % 16 == 0;
+    at::Tensor out, workspace, activations, next_squares;
+    const int status = unlocked([&] {
+        out = target ? *target : make(*a, M, N, rounded ? at::kBFloat16 : at::kFloat);
+        if (bytes) workspace = at::empty({(int64_t)(bytes / 4)}, a->options().dtype(at::kFloat));
         if (next_weight) {
             activations = make(*a, M, N, at::kBFloat16);
-            next_squares = make(*a, split ? planned(4) : planned(5), stride, at::kFloat);
+            next_squares = make(*a, split ? planned[4] : planned[5], stride, at::kFloat);
         }
+        void *to = out.data_ptr(), *room = bytes ? workspace.data_ptr() : nullptr, *next = next_weight ? activations.data_ptr() : nullptr;
         const void* operand = (tiled ? tiled : w)->data_ptr();
-        void* next = next_weight ? activations.data_ptr() : nullptr;
+        int* ticket = bytes ? at_of<int>(counters) : nullptr;
         float* next_sums = next_weight ? static_cast<float*>(next_squares.data_ptr()) : nullptr;
         const int squares_rows = squares ? (int)squares->size(0) : 0;
-        if (split) {
-            const size_t bytes = (size_t)planned(2);
-            const int tickets = (int)planned(3);
-            if (bytes) {
-                if (!is(counters, at::kInt, 1) || counters->size(0) < tickets) return other_path();
-                workspace = at::empty({(int64_t)(bytes / 4)}, a->options().dtype(at::kFloat));
-            }
-            status = entry.gemm_medium(a->data_ptr(), operand, tiled != nullptr, at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K,
-                                       bytes ? workspace.data_ptr() : nullptr, bytes, bytes ? at_of<int>(counters) : nullptr, bytes ? (int)counters->size(0) : 0,
-                                       at_of<const float>(next_weight), one_centered, next, next_sums, at_of<const float>(squares), squares_rows, eps, limit, alpha,
-                                       shift, stream);
-        } else {
-            status = entry.gemm_rows(a->data_ptr(), operand, tiled != nullptr, at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K,
-                                     at_of<const float>(next_weight), one_centered, next, next_sums, at_of<const float>(squares), squares_rows, eps, limit, alpha, shift,
-                                     stream);
-        }
-    }
+        if (large)
+            return entry.big_tile(a->data_ptr(), w->data_ptr(), at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K, (int)planned[1], (int)planned[2],
+                                  (int)planned[3], (int)planned[4], room, bytes, ticket, tickets, stream);
+        if (split)
+            return entry.gemm_medium(a->data_ptr(), operand, tiled != nullptr, at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K, room, bytes, ticket,
+                                     bytes ? (int)counters->size(0) : 0, at_of<const float>(next_weight), one_centered, next, next_sums, at_of<const float>(squares),
+                                     squares_rows, eps, limit, alpha, shift, stream);
+        return entry.gemm_rows(a->data_ptr(), operand, tiled != nullptr, at_of<const float>(bias), to, out_code, mode, (int)M, (int)N, (int)K,
+                               at_of<const float>(next_weight), one_centered, next, next_sums, at_of<const float>(squares), squares_rows, eps, limit, alpha, shift, stream);
+    });
     if (status) return answer(status, nullptr);
     if (next_weight) {
         PyObject* pair = PyTuple_New(2);
@@ -164,13 +167,16 @@ PyObject* rmsnorm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (hidden < 1 || weight->size(0) != hidden) return other_path();
     const int64_t rows = index ? index->numel() : x->numel() / hidden;
     if (!fits(rows) || !fits(hidden)) return other_path();
-    const int rounded = PyObject_IsTrue(args[3]);
+    const int rounded = PyObject_IsTrue(args[3]), one_centered = PyObject_IsTrue(args[5]);
     const float eps = number(args[4]);
     void* stream = stream_of(args[6]);
     if (PyErr_Occurred()) return nullptr;
-    at::Tensor out = make(*x, rows, hidden, rounded ? at::kBFloat16 : at::kFloat);
-    const int status = entry.rmsnorm_rows(at_of<const float>(x), at_of<const float>(weight), out.data_ptr(), rounded ? BF16 : F32, at_of<const int32_t>(index), (int)rows,
-                                          (int)hidden, eps, PyObject_IsTrue(args[5]), stream);
+    at::Tensor out;
+    const int status = unlocked([&] {
+        out = make(*x, rows, hidden, rounded ? at::kBFloat16 : at::kFloat);
+        return entry.rmsnorm_rows(at_of<const float>(x), at_of<const float>(weight), out.data_ptr(), rounded ? BF16 : F32, at_of<const int32_t>(index), (int)rows,
+                                  (int)hidden, eps, one_centered, stream);
+    });
     return status ? answer(status, nullptr) : THPVariable_Wrap(std::move(out));
 }
 
@@ -190,10 +196,13 @@ PyObject* shortconv(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (bcx->size(1) != 3 * hidden || state->size(1) != hidden || state->size(2) != kernel - 1 || !size_is(bias, hidden) || row_seg->numel() < rows ||
         seg_row0->numel() < segments + 1 || seg_slot->numel() < segments || !fits(rows) || !fits(state->size(0)))
         return other_path();
-    at::Tensor out = make(*bcx, rows, hidden, rounded ? at::kBFloat16 : at::kFloat);
-    const int status = entry.shortconv(bcx->data_ptr(), bcx->scalar_type() == at::kFloat ? F32 : BF16, out.data_ptr(), rounded ? BF16 : F32, at_of<const float>(taps),
-                                       at_of<const float>(bias), at_of<float>(state), at_of<const int32_t>(row_seg), at_of<const int32_t>(seg_row0),
-                                       at_of<const int32_t>(seg_slot), (int)rows, (int)segments, (int)hidden, (int)kernel, (int)state->size(0), stream);
+    at::Tensor out;
+    const int status = unlocked([&] {
+        out = make(*bcx, rows, hidden, rounded ? at::kBFloat16 : at::kFloat);
+        return entry.shortconv(bcx->data_ptr(), bcx->scalar_type() == at::kFloat ? F32 : BF16, out.data_ptr(), rounded ? BF16 : F32, at_of<const float>(taps),
+                               at_of<const float>(bias), at_of<float>(state), at_of<const int32_t>(row_seg), at_of<const int32_t>(seg_row0),
+                               at_of<const int32_t>(seg_slot), (int)rows, (int)segments, (int)hidden, (int)kernel, (int)state->size(0), stream);
+    });
     return status ? answer(status, nullptr) : THPVariable_Wrap(std::move(out));
 }
 
@@ -230,12 +239,14 @@ PyObject* qk_norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (rotary && (!is(t, at::kFloat, 2) || t->size(0) != rows || t->size(1) != rotary / 2)) return other_path();
         if (!rotary && t && !t->is_contiguous()) return other_path();
     }
-    at::Tensor out = make(*qkv, rows, heads * head_dim, k->scalar_type());
-    const int status = entry.qk_norm(qkv->data_ptr(), qkv->scalar_type() == at::kFloat ? F32 : BF16, (int)width, out.data_ptr(), k->scalar_type() == at::kFloat ? F32 : BF16,
-                                     at_of<const float>(qw), at_of<const float>(kw), eps, at_of<const float>(cos), at_of<const float>(sin), (int)rotary, k->data_ptr(),
-                                     v->data_ptr(), at_of<const int32_t>(table), (int)table->size(1), at_of<const int32_t>(row_seg), at_of<const int32_t>(row_pos), (int)rows,
-                                     (int)heads, (int)kv_heads, (int)head_dim, (int)v_dim, (int)page, (int)k->size(0), write, interleaved, q_only,
-                                     at_of<const float>(scale), stream);
+    at::Tensor out;
+    const int status = unlocked([&] {
+        out = make(*qkv, rows, heads * head_dim, k->scalar_type());
+        return entry.qk_norm(qkv->data_ptr(), qkv->scalar_type() == at::kFloat ? F32 : BF16, (int)width, out.data_ptr(), k->scalar_type() == at::kFloat ? F32 : BF16,
+                             at_of<const float>(qw), at_of<const float>(kw), eps, at_of<const float>(cos), at_of<const float>(sin), (int)rotary, k->data_ptr(),
+                             v->data_ptr(), at_of<const int32_t>(table), (int)table->size(1), at_of<const int32_t>(row_seg), at_of<const int32_t>(row_pos), (int)rows,
+                             (int)heads, (int)kv_heads, (int)head_dim, (int)v_dim, (int)page, (int)k->size(0), write, interleaved, q_only, at_of<const float>(scale), stream);
+    });
     return status ? answer(status, nullptr) : THPVariable_Wrap(std::move(out));
 }
 
@@ -261,11 +272,14 @@ PyObject* prefill(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (q->size(1) != heads * head_dim || row_pos->numel() < rows || tile_seg->numel() != tile_row0->numel() || kept < 0 || (kept && chunk) || !fits(rows) ||
         !fits(table->size(1)))
         return other_path();
-    at::Tensor out = make(*q, rows, heads * v_dim, at::kBFloat16);
-    const int status = entry.prefill(q->data_ptr(), out.data_ptr(), k->data_ptr(), v->data_ptr(), at_of<const int32_t>(table), (int)table->size(1),
-                                     at_of<const int32_t>(tile_seg), at_of<const int32_t>(tile_row0), (int)tile_seg->numel(), at_of<const int32_t>(seg_row0),
-                                     at_of<const int32_t>(row_pos), (int)rows, (int)heads, (int)kv_heads, (int)head_dim, (int)v_dim, scale, window, chunk, softcap,
-                                     window ? kept : 0, at_of<const float>(sinks), at_of<const float>(slopes), (int)page, (int)k->size(0), together, form, stream);
+    at::Tensor out;
+    const int status = unlocked([&] {
+        out = make(*q, rows, heads * v_dim, at::kBFloat16);
+        return entry.prefill(q->data_ptr(), out.data_ptr(), k->data_ptr(), v->data_ptr(), at_of<const int32_t>(table), (int)table->size(1),
+                             at_of<const int32_t>(tile_seg), at_of<const int32_t>(tile_row0), (int)tile_seg->numel(), at_of<const int32_t>(seg_row0),
+                             at_of<const int32_t>(row_pos), (int)rows, (int)heads, (int)kv_heads, (int)head_dim, (int)v_dim, scale, window, chunk, softcap,
+                             window ? kept : 0, at_of<const float>(sinks), at_of<const float>(slopes), (int)page, (int)k->size(0), together, form, stream);
+    });
     return status ? answer(status, nullptr) : THPVariable_Wrap(std::move(out));
 }
 

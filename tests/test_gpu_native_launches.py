@@ -1,6 +1,8 @@
 """The native module of launches: bit for bit what the general paths give, over every form that it accepts; what it does not take goes to them and is served or refused as
 they do."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -134,3 +136,33 @@ def test_tensors_of_the_host_are_left_to_the_general_path(ops):
         ops.rmsnorm_rows(torch.zeros(2, 8), torch.zeros(8), 1e-5, BF)
     with pytest.raises(TypeError):
         ops._native.rmsnorm(a)
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_launch_waits(ops):
+    """The module lets go of the interpreter's lock around the kernel library's calls, as ctypes does. In place of the entry points here stands
+    PyGILState_Check, which says 1 (a refused call) to a thread that holds it."""
+    held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+    real = {name: ctypes.cast(getattr(ops._lib, name), ctypes.c_void_p).value for name in ops._NATIVE_ENTRIES}
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)    # noqa: E731
+    x, weight, pages, cos = draw(40, 256, dtype=F32), draw(256, dtype=F32), torch.zeros(2, 1, 64, 64, dtype=BF, device=DEV), draw(40, 32, dtype=F32)
+    seg, row0, pos, table = ints(*[0] * 40), ints(0, 40), ints(*range(40)), ints(0, 1).view(1, 2)
+    native, stream = ops._native, ops._stream()
+    products = [(few, M, N, K, t) for few, M, N, K, t in ((True, 2, 2048, 256, False), (False, 40, 96, 256, False), (True, 16, 256, 8192, True), (False, 300, 1536, 512, True),
+                                                          (False, 801, 2048, 7168, True))]
+    plans = [ops._native_plan(few, t, 0, M, N, K) for few, M, N, K, t in products]
+    assert all(plans) and {plan[0] for plan in plans} == {0, 1} and {plan[1] for plan in plans if not plan[0]} == {False, True} and plans[-1][4] > 1
+    operands = [(draw(M, K), w, ops.tile_weights(w) if t else None) for _, M, N, K, t in products for w in (draw(N, K),)]
+    counters = ops._medium_counters(x.device, 1)
+    calls = [lambda a=a, w=w, t=t, plan=plan: native.product(a, w, t, None, None, 0, ops.F32, False, None, False, None, 0.0, 0.0, 1.0, 0.0, plan, counters, stream)
+             for (a, w, t), plan in zip(operands, plans)]
+    calls += [lambda: native.rmsnorm(x, weight, None, True, 1e-5, False, stream),
+              lambda: native.shortconv(draw(40, 768, dtype=F32), draw(256, 3, dtype=F32), None, draw(1, 256, 2, dtype=F32), seg, row0, ints(0), 1, True, stream),
+              lambda: native.qk_norm(draw(40, 256, dtype=F32), 2, 1, 64, None, None, 1e-5, cos, cos, 64, pages, pages, table, seg, pos, True, 64, False, False, None, 64, stream),
+              lambda: native.prefill(draw(40, 128), 2, 1, 64, pages, pages, table, ints(0), ints(0), row0, pos, 0.125, 0, 0, 64, 0, 0.0, 0, None, None, 0, 64, stream)]
+    try:
+        native.bind({name: at if name == "fw_last_error" else held for name, at in real.items()}, ops.KernelError, torch.OutOfMemoryError)
+        for call in calls:
+            assert isinstance(call(), torch.Tensor)
+    finally:
+        native.bind(real, ops.KernelError, torch.OutOfMemoryError)
