@@ -791,15 +791,9 @@ _LARGE_LEAST_SLICE = 384     # k
 
 
 @functools.lru_cache(maxsize=4096)
-def large_tile(mode: int, M: int, N: int, K: int):
-    """The large tile that takes a product of more than 64 rows by weights that a model holds (they come with their operand tiles; a bare product keeps to
-    ``tiled_plan``, whose sums its callers know by the kernel's name): (rows, columns, workgroups on a compute unit, slices of K, bytes of workspace, counters),
-    or None where the product whose waves split K or one of ``tiled_plan`` is estimated to be faster. Chosen so, the 420 shapes a mode take 1.8 (storing,
-    adding) and 1.0 % (gated) more than with the fastest product each, and 12, 13 and 26 % less than without these tiles; no shape loses more than 15 %
-    (adding 2,048 x 1,024 over K 1,024 13.3 -> 10.3 us, 801 x 2,048 over 7,168 43.3 -> 36.1, gated 500 x 4,608 over 1,024 24.8 -> 16.4, 2,048 x 4,608 55 -> 38)."""
-    if K % 32 or K > 1 << 22 or N > 1 << 20:
-        return None
-    k, megabytes = K / 1024, N * (2 if mode == 2 else 1) * K * 2e-6
+def _fastest_large(mode: int, rows64: int, N: int, K: int):
+    """The large tile with the least estimated time for (rows64 - 1) * 64 + 1 to rows64 * 64 rows, its needs (``large_tile``) and that time: a tile's rows are a multiple of 64."""
+    M, k, megabytes = rows64 * 64, K / 1024, N * (2 if mode == 2 else 1) * K * 2e-6
     best, least = None, 1e30
     for (rows, columns, each), (start, each_round, each_tile, walk, fill, memory) in _TIME_LARGE[mode].items():
         tiles = -(-M // rows) * -(-N // (columns // 2 if mode == 2 else columns))
@@ -818,17 +812,36 @@ def large_tile(mode: int, M: int, N: int, K: int):
             time = start + slices * each_slice + share * all_at_once + k / slices * (walk + fill * share) + megabytes * memory
             if time < least and -(-K // slices // 64) * 64 * (slices - 1) < K:
                 best, least = (rows, columns, 1, slices), time
-    if rows_fit(mode, M, N, K):
-        start, walk, by_rows, by_width, outputs, by_outputs = _TIME_ROWS[mode]
-        width = N * (2 if mode == 2 else 1)
-        other = start + k * (walk + by_rows * M / 256 + by_width * width / 4096) + M * width * 1e-6 * (outputs + by_outputs * k)
-    else:
-        other = _TIME_OLDER * min(_tiled_times(mode, M, N, K).values())
-    if other <= least:
-        return None
     need_bytes, need_counters = ctypes.c_size_t(0), ctypes.c_int(0)
     _check(library().fw_gemm_mfma_big_tile_needs(mode, M, N, K, *best, ctypes.byref(need_bytes), ctypes.byref(need_counters)))
-    return (*best, need_bytes.value, need_counters.value)
+    return (*best, need_bytes.value, need_counters.value), least
+
+
+@functools.lru_cache(maxsize=4096)
+def _fastest_older(mode: int, rows128: int, N: int, K: int) -> float:
+    """... and of ``tiled_plan``'s products, whose tiles (and the lines between them) are multiples of 128 rows."""
+    return min(_tiled_times(mode, rows128 * 128, N, K).values())
+
+
+@functools.lru_cache(maxsize=4096)
+def large_tile(mode: int, M: int, N: int, K: int):
+    """The large tile that takes a product of more than 64 rows by weights that a model holds (they come with their operand tiles; a bare product keeps to
+    ``tiled_plan``, whose sums its callers know by the kernel's name): (rows, columns, workgroups on a compute unit, slices of K, bytes of workspace, counters),
+    or None where the product whose waves split K or one of ``tiled_plan`` is estimated to be faster. Chosen so, the 420 shapes a mode take 1.8 (storing,
+    adding) and 1.0 % (gated) more than with the fastest product each, and 12, 13 and 26 % less than without these tiles; no shape loses more than 15 %
+    (adding 2,048 x 1,024 over K 1,024 13.3 -> 10.3 us, 801 x 2,048 over 7,168 43.3 -> 36.1, gated 500 x 4,608 over 1,024 24.8 -> 16.4, 2,048 x 4,608 55 -> 38).
+    The estimates are kept by 64 (128) rows, since nearly every prompt has a length of its own: 400 lengths up to 2,048 took 17 to 23 us a product on the host
+    when each was searched for anew, 4 to 6 now."""
+    if K % 32 or K > 1 << 22 or N > 1 << 20:
+        return None
+    tile, least = _fastest_large(mode, -(-M // 64), N, K)
+    if rows_fit(mode, M, N, K):
+        start, walk, by_rows, by_width, outputs, by_outputs = _TIME_ROWS[mode]
+        k, width = K / 1024, N * (2 if mode == 2 else 1)
+        other = start + k * (walk + by_rows * M / 256 + by_width * width / 4096) + M * width * 1e-6 * (outputs + by_outputs * k)
+    else:
+        other = _TIME_OLDER * _fastest_older(mode, -(-M // 128), N, K)
+    return None if other <= least else tile
 
 
 MEDIUM_MAX_ROWS = 64
