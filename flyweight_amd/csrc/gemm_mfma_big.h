@@ -60,6 +60,16 @@ __device__ __forceinline__ float silu_big(float g) {
 // far below the bfloat16 the result is rounded to). exp(-g) overflows to infinity for very
 // negative g, whose reciprocal is 0: the result is -0, as it should be.
 __device__ __forceinline__ float silu_quick(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
+// The logistic function as exact as with expf and a division, without their cases (two prompts of four layers with 8,192 gated features over 2,048, 2,618 us: 10 us more
+// than with the hardware's alone; with expf and a division 44): e^-|z| as 2^t (1 + rest) with the product's rounding in the rest, and one step of Newton's behind the reciprocal. Largest error, -8 to 8 / -20 to -8 / -86 to -20:
+// 2^-22.6 / 2^-22.3 / 2^-22.6 of the value; expf and a division 2^-22.4 / 2^-22.4 / 2^-23.5; the hardware's exponential and reciprocal alone 2^-20.9 / 2^-19.9 / 2^-18.
+__device__ __forceinline__ float sigmoid_big(float z) {
+    const float x = fmaxf(-fabsf(z), -150.0f);                             // (2^t is zero from there on)
+    const float t = x * 1.44269504f, rest = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -t));        // log2 e in two parts
+    const float power = __builtin_amdgcn_exp2f(t), e = fmaf(power, rest * 0.693147181f, power);
+    const float r = __builtin_amdgcn_rcpf(1.0f + e);
+    return (z >= 0.0f ? 1.0f : e) * fmaf(fmaf(-(1.0f + e), r, 1.0f), r, r);
+}
 // two floats -> two bfloat16 in one word, round to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     const f32x2 v = {lo, hi};
@@ -87,7 +97,7 @@ struct BigSlices {
     int* counters;
 };
 
-// A gated product with this output type stores the unit with clamped halves (fw_gated_unit) in bfloat16.
+// A gated product with this output type stores the unit with clamped halves (as fw_clamped_glu forms it) in bfloat16.
 struct clamped_bf16_t {
     uint16_t bits;
 };
@@ -453,7 +463,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EACH_CU, EA
         if constexpr (big_clamps<TO>::value) {
             g = fminf(g, halves.limit);
             u = fminf(fmaxf(u, -halves.limit), halves.limit);
-            return g * __builtin_amdgcn_rcpf(1.0f + __expf(-halves.alpha * g)) * (u + halves.shift);
+            return g * sigmoid_big(halves.alpha * g) * (u + halves.shift);
         } else {
             return fw_gate_of<TO>(g, unit) * u;
         }

@@ -42,3 +42,24 @@ def test_a_models_weights_take_it_and_infinities_are_clamped(ops):  # noqa: F811
     assert torch.equal(got[3].isinf(), want[3].isinf())
     with pytest.raises(ops.KernelError):
         ops._check(ops.library().fw_gemm_mfma_big_tile_clamped(ops._p(a), ops._p(w), ops._p(got), 200, 1536, 512, 128, 256, 1, 0.0, 1.7, 1.0, ops._stream()))
+
+
+@pytest.mark.parametrize("tile", [(128, 256, 1), (192, 192, 1), (64, 128, 2)])
+@pytest.mark.parametrize("limit,alpha,shift", [(7.0, 1.0, 1.0), (30.0, 4.0, 0.0), (1000.0, 16.0, 0.0)])
+def test_the_unit_is_as_exact_as_on_float32_sums_in_memory(ops, tile, limit, alpha, shift):  # noqa: F811
+    """One number a sum and an alpha that is a power of two, so that the sigmoid's argument is exact; gates of many sizes, to where it leaves float32. What stands before the
+    rounding to bfloat16 may be 2^-21.5 of the value away (the sigmoid 2^-22.3, three roundings of 2^-24; the hardware's exponential gives zero below 2^-126): only a value that
+    near to the middle between two bfloat16 may be rounded to the other one. (Where the argument is rounded, that alone moves the sigmoid by |alpha g| 2^-24 of it.)"""
+    M, N, K = 700, 1000, 32
+    g = torch.Generator().manual_seed(3)
+    a, w = torch.zeros(M, K), torch.zeros(2 * N, K)
+    a[:, 0] = torch.randn(M, generator=g).exp()
+    w[:, 0] = torch.randn(2 * N, generator=g)
+    a, w = a.to(torch.bfloat16).to(DEV), w.to(torch.bfloat16).to(DEV)
+    out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+    ops._check(ops.library().fw_gemm_mfma_big_tile_clamped(ops._p(a), ops._p(w), ops._p(out), M, N, K, *tile, limit, alpha, shift, ops._stream()))
+    sums = a[:, :1].double() * w[:, 0].double()
+    gate, up = sums[:, :N].clamp(max=limit), sums[:, N:].clamp(-limit, limit)
+    want = gate * torch.sigmoid(alpha * gate) * (up + shift)
+    slack = 2.0 ** -21.5 * want.abs() + 2.0 ** -125 * (gate * (up + shift)).abs() + 2.0 ** -126
+    assert ((out.double() >= (want - slack).to(torch.bfloat16).double()) & (out.double() <= (want + slack).to(torch.bfloat16).double())).all()
