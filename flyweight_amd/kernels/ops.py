@@ -635,6 +635,8 @@ def _fast_gemm(a: torch.Tensor, w: torch.Tensor, bias, target: torch.Tensor, out
     if w_tiled is not None and M > MEDIUM_MAX_ROWS:
         tile = large_tile(mode, M, N, K)
         if tile is not None:
+            if rows_fit(mode, M, N, K):     # where the tiles could be read they have to be w's
+                _tiled_for(w, w_tiled)
             rows, columns, each, slices, need_bytes, need_counters = tile
             workspace_at = counters_at = None
             if need_bytes:

@@ -123,6 +123,12 @@ def test_what_it_does_not_take_is_served_or_refused_as_before(ops):
         ops.gemm_medium(a, w, ops.EPILOGUE_STORE, squares=torch.zeros(2, 16, device=DEV))
     with pytest.raises(ops.KernelError, match="operand tiles"):
         ops.gemm_medium(a, w, ops.EPILOGUE_STORE, w_tiled=ops.tile_weights(w)[:-1].contiguous())
+    for mode, M, N, K in ((0, 300, 1536, 512), (1, 200, 1024, 256), (2, 100, 512, 256)):         # on a large tile, which reads w, where the operand tiles could be read
+        assert ops._native_plan(False, True, mode, M, N, K)[0] == 1 and ops.rows_fit(mode, M, N, K)
+        x, own, into = draw(M, K), draw(2 * N if mode == 2 else N, K, seed=1), torch.zeros(M, N, device=DEV)
+        for wrong in (ops.tile_weights(own)[:-1].contiguous(), ops.tile_weights(own).float()):
+            with pytest.raises(ops.KernelError, match="operand tiles"):
+                ops.gemm_swiglu(x, own, w_tiled=wrong) if mode == 2 else ops.gemm(x, own, accumulate_into=into if mode else None, w_tiled=wrong)
     with pytest.raises(ops.KernelError, match="row width"):
         ops.rmsnorm_rows(a.float(), torch.zeros(255, device=DEV), 1e-5, BF)
     odd = torch.empty(40 * 256 + 1, dtype=BF, device=DEV)[1:].view(40, 256).copy_(a)       # at no multiple of 16 bytes
