@@ -629,7 +629,7 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
     FW_REQUIRE(!tiled || (a_dtype == FW_BF16 && K % 32 == 0 && out_dtype == (gated ? FW_BF16 : FW_F32) && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0),
                "grouped_gemm: operand tiles take bfloat16 rows at 16 bytes, K a multiple of 32 and leave bfloat16 (gated) or float32");
     if (a_dtype == FW_BF16 && (w_dtype == FW_BF16 || tiled) && K % 8 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0 &&
-        (out_dtype == FW_F32 || (out_dtype == FW_BF16 && gated))) {
+        out_dtype == (gated ? FW_BF16 : FW_F32)) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
         // ... straight to LDS, on the tile that the experts' places ask for, from 24 places an expert, with a short K from 48 (fewer leave most of a tile of 64
@@ -637,7 +637,7 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
         // over 1,536, 25 places 48.7 / 41.5, 8 of 1,024 over 2,048, 48 places, gated 31.1 / 16.9), not over the longest K (32 of 288 over 16,832, 100 places 175 / 191)
         const bool tall = fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) != 0;
         const bool straight = tall || (K <= 16384 && (long long)places >= (K >= 1024 ? 24ll : 48ll) * experts && fw_grouped_big_takes(a_rows, N, K));
-        if (glu_limit == 0.0f && out_dtype == (gated ? FW_BF16 : FW_F32) && straight)
+        if (glu_limit == 0.0f && straight)
             status = fw_launch_grouped_big(a, place_row, w, tiled, expert_begin, out, gated, places, experts, N, K, tall, s);
         else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s)
                                 : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s);

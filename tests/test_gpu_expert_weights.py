@@ -75,3 +75,20 @@ def test_what_operand_tiles_do_not_take_is_refused(ops):
         ops.grouped_gemm(torch.zeros(4, 64, dtype=torch.bfloat16, device=DEV), place_row, held, begin, 4, gated=False, out_dtype=torch.bfloat16)
     with pytest.raises(ops.KernelError, match="grouped_gemm: a is"):
         ops.grouped_gemm(torch.zeros(4, 96, dtype=torch.bfloat16, device=DEV), place_row, held, begin, 4, gated=False, out_dtype=torch.float32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,K", [(4, 64), (300, 64), (9, 72)])
+def test_gated_float32_outputs_of_bfloat16_rows(ops, rows, K):
+    """... hold float32 (K + 16 rounded sums of exact products, the unit's slopes as elsewhere), and the rows behind them are untouched."""
+    experts, N = 3, 24
+    begin, place_row, _ = step(ops, rows, experts, 2)
+    g = torch.Generator().manual_seed(rows)
+    a, w = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(DEV), (torch.randn(experts, 2 * N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(DEV)
+    got, own, b = ops.grouped_gemm(a, place_row, w, begin, 2 * rows, gated=True, out_dtype=torch.float32), a.index_select(0, place_row.long()), begin.tolist()
+    for e in range(experts):
+        x, part = own[b[e]:b[e + 1]].double(), got[b[e]:b[e + 1]].double()
+        exact, limit = x @ w[e].double().T, (K + 16) * 2.0 ** -24 * (x.abs() @ w[e].double().abs().T)
+        gate, up, lg, lu = exact[:, :N], exact[:, N:], limit[:, :N], limit[:, N:]
+        want = gate * torch.sigmoid(gate) * up
+        assert ((part - want).abs() <= 1.13 * lg * (up.abs() + lu) + gate.abs() * lu + 2.0 ** -20 * (gate * up).abs() + 2.0 ** -133).all()
