@@ -445,7 +445,9 @@ int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place
 // or float32.
 int fw_grouped_gemm_few(const void* a, const int32_t* place_row, const void* w_tiled, const int32_t* expert_begin, void* out, int gated, int places,
                         int experts, int N, int K, int place_tiles, float glu_limit, float glu_alpha, float glu_shift, void* stream);
-// 1: with bfloat16 operands, the plain unit and an output of bfloat16 (gated) or float32 the product is worth tiles of more than 128 places
+// 1: with bfloat16 operands, the plain unit and an output of bfloat16 (gated) or float32 the product goes straight to LDS, on fw_grouped_gemm_tile's tile
+int fw_grouped_gemm_straight(int gated, int a_rows, int places, int experts, int N, int K);
+// 1: ... it is worth tiles of more than 128 places
 int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int experts, int N, int K);
 // the places and the columns (gate and up together) of the tile that it then has; tall: tiles of more than 128 places are worth it
 int fw_grouped_gemm_tile(int gated, int places, int experts, int N, int K, int tall, int* rows, int* columns);

@@ -614,6 +614,15 @@ extern "C" int fw_grouped_gemm_large_fits(int gated, int a_rows, int places, int
     return K <= 1024 || tiles >= 192;
 }
 
+// Whether a product of bfloat16 operands and the plain unit goes straight to LDS, on the tile that the experts' places ask for (fw_grouped_gemm_tile): from 24 places an expert,
+// with a short K from 48 (fewer leave most of a tile of 64 empty: 64 experts, 768 features over 1,024, 19 places an expert, down 18.7 us on tiles of 32 and 19.4; 40 of 3,000
+// over 320, 25 places 18.2 / 19.6; but 32 of 2,048 over 1,536, 25 places 48.7 / 41.5, 8 of 1,024 over 2,048, 48 places, gated 31.1 / 16.9), not over the longest K (32 of
+// 288 over 16,832, 100 places 175 / 191).
+extern "C" int fw_grouped_gemm_straight(int gated, int a_rows, int places, int experts, int N, int K) {
+    return fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) ||
+           (K <= 16384 && (long long)places >= (K >= 1024 ? 24ll : 48ll) * experts && fw_grouped_big_takes(a_rows, N, K));
+}
+
 extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int32_t* place_row, const void* w, int w_dtype,
                                const int32_t* expert_begin, void* out, int out_dtype, int gated, int places, int experts, int N, int K,
                                float glu_limit, float glu_alpha, float glu_shift, void* stream) {
@@ -632,13 +641,9 @@ extern "C" int fw_grouped_gemm(const void* a, int a_dtype, int a_rows, const int
         out_dtype == (gated ? FW_BF16 : FW_F32)) {
         const bool big = (long long)places >= 48ll * experts;
         int status;
-        // ... straight to LDS, on the tile that the experts' places ask for, from 24 places an expert, with a short K from 48 (fewer leave most of a tile of 64
-        // empty: 64 experts, 768 features over 1,024, 19 places an expert, down 18.7 us on tiles of 32 and 19.4; 40 of 3,000 over 320, 25 places 18.2 / 19.6; but 32 of 2,048
-        // over 1,536, 25 places 48.7 / 41.5, 8 of 1,024 over 2,048, 48 places, gated 31.1 / 16.9), not over the longest K (32 of 288 over 16,832, 100 places 175 / 191)
-        const bool tall = fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) != 0;
-        const bool straight = tall || (K <= 16384 && (long long)places >= (K >= 1024 ? 24ll : 48ll) * experts && fw_grouped_big_takes(a_rows, N, K));
-        if (glu_limit == 0.0f && straight)
-            status = fw_launch_grouped_big(a, place_row, w, tiled, expert_begin, out, gated, places, experts, N, K, tall, s);
+        if (glu_limit == 0.0f && fw_grouped_gemm_straight(gated, a_rows, places, experts, N, K))
+            status = fw_launch_grouped_big(a, place_row, w, tiled, expert_begin, out, gated, places, experts, N, K,
+                                           fw_grouped_gemm_large_fits(gated, a_rows, places, experts, N, K) != 0, s);
         else if (gated) status = big ? grouped_mfma_launch<true, true, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s)
                                 : grouped_mfma_launch<true, false, 2, bf16_t>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s);
         else status = big ? grouped_mfma_launch<false, true, 2, float>(a, place_row, w, tiled, expert_begin, out, places, experts, N, K, unit, s)

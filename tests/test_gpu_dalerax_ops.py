@@ -305,22 +305,24 @@ def test_grouped_gemm(ops, dtype, rows, experts, top, K, N):
     assert out.shape == (places, K) and np.abs(host(out) - want).max() <= limit * np.abs(want).max()
 
 
-@pytest.mark.parametrize("rows,experts,top,K,N,gated,large", [
+@pytest.mark.parametrize("rows,experts,top,K,N,gated,straight", [
     (300, 4, 2, 96, 200, True, True), (300, 4, 2, 96, 200, False, True),        # tiles that end inside the features
     (500, 3, 1, 160, 129, True, True), (500, 3, 1, 160, 257, False, True),      # odd widths, one feature more than a tile
     (2100, 70, 2, 64, 300, True, True), (2100, 70, 2, 64, 300, False, True),    # more than 64 experts
-    (300, 4, 2, 100, 200, True, False), (200, 8, 2, 2048, 520, False, False), (2000, 2, 2, 64, 40, True, True),
-    (20000, 64, 2, 32, 24, True, False), (9000, 4, 2, 1056, 700, False, True)])
-def test_grouped_gemm_on_its_large_tiles(ops, rows, experts, top, K, N, gated, large):
-    """Products of prompts straight to LDS, and those beside them that go through registers: few tiles over a long K, more than a round of tiles
-    that are half empty, a K that is no multiple of 32. (K + 16) rounded sums of exact products; the unit as elsewhere."""
+    (200, 8, 2, 2048, 520, False, True), (2000, 2, 2, 64, 40, True, True), (20000, 64, 2, 32, 24, True, True), (9000, 4, 2, 1056, 700, False, True),
+    (300, 4, 2, 100, 200, True, False), (300, 4, 2, 100, 200, False, False),    # through registers: K no multiple of 32
+    (120, 2, 1, 16416, 40, True, False), (120, 2, 1, 16416, 70, False, False),  # the longest K
+    (90, 8, 2, 2048, 520, True, False), (90, 8, 2, 2048, 520, False, False), (170, 8, 2, 512, 72, True, False)])     # few places an expert
+def test_grouped_gemm_on_its_large_tiles(ops, rows, experts, top, K, N, gated, straight):
+    """Products of prompts straight to LDS, and those beside them that go through registers: a K that is no multiple of 32, the longest, few places an expert (a
+    clamped unit does too: test_gpu_telapel_ops). (K + 16) rounded sums of exact products; the unit as elsewhere."""
     rng = np.random.default_rng(rows + N)
     chosen = np.stack([rng.permutation(experts)[:top] for _ in range(rows)]).astype(np.int32)
     begin, place_row, _ = ops.moe_arrange(ints(chosen), experts)
     a = dev(rng.normal(size=(rows, K)), torch.bfloat16)
     w = dev(rng.normal(size=(experts, 2 * N if gated else N, K)), torch.bfloat16)
     places = rows * top
-    assert ops.library().fw_grouped_gemm_large_fits(int(gated), rows, places, experts, N, K) == large
+    assert ops.library().fw_grouped_gemm_straight(int(gated), rows, places, experts, N, K) == straight
     found = ops.grouped_gemm(a, place_row, w, begin, places, gated=gated, out_dtype=torch.bfloat16 if gated else torch.float32).cpu().double()
     b, at, A, W = begin.tolist(), place_row.long().cpu(), a.cpu().double(), w.cpu().double()
     for e in range(experts):
