@@ -17,15 +17,17 @@ struct BigCall {
     float limit = 0.0f, alpha = 0.0f, shift = 0.0f;     // of the gated unit with clamped halves
 };
 
+// Every tile there is, as T(rows, columns, workgroups on a compute unit), and those that storing and adding products also have with K cut.
+#define FW_BIG_WHOLE_TILES(T)                                                                                                                       \
+    T(64, 128, 1) T(64, 128, 2) T(128, 128, 1) T(128, 128, 2) T(192, 128, 1) T(64, 192, 1) T(128, 192, 1) T(192, 192, 1) T(256, 192, 1) T(128, 256, 1) \
+    T(192, 256, 1) T(256, 256, 1) T(256, 320, 1)
+#define FW_BIG_CUT_TILES(T) T(64, 128, 1) T(128, 128, 1) T(128, 256, 1)
+
 // whether there is such a tile: `slices` tells those with K cut from the others
 __host__ __device__ inline bool fw_big_tile_exists(int mode, int rows, int columns, int each_cu, int slices) {
-    if (slices > 1) return mode != 2 && each_cu == 1 && ((columns == 128 && (rows == 64 || rows == 128)) || (columns == 256 && rows == 128));
-    if (each_cu == 2) return columns == 128 && (rows == 64 || rows == 128);
-    if (each_cu != 1) return false;
-    if (columns == 128) return rows == 64 || rows == 128 || rows == 192;
-    if (columns == 192) return rows == 64 || rows == 128 || rows == 192 || rows == 256;
-    if (columns == 256) return rows == 128 || rows == 192 || rows == 256;
-    return columns == 320 && rows == 256;
+#define FW_IS(ROWS, COLUMNS, EACH) (rows == ROWS && columns == COLUMNS && each_cu == EACH) ||
+    return slices > 1 ? mode != 2 && (FW_BIG_CUT_TILES(FW_IS) false) : (FW_BIG_WHOLE_TILES(FW_IS) false);
+#undef FW_IS
 }
 
 // 0, or -1 with the error set

@@ -3,24 +3,13 @@
 
 template <typename TO>
 static int launch(const BigCall& c) {
-#define FW_TILE(ROWS, COLUMNS, EACH, CUT) \
-    if (c.rows == ROWS && c.columns == COLUMNS && c.each_cu == EACH && (c.slices > 1) == CUT) return launch_big<MB_STORE, TO, COLUMNS / 64, ROWS / 64, EACH, CUT>(c)
-    FW_TILE(64, 128, 1, false);
-    FW_TILE(64, 128, 2, false);
-    FW_TILE(128, 128, 1, false);
-    FW_TILE(128, 128, 2, false);
-    FW_TILE(192, 128, 1, false);
-    FW_TILE(64, 192, 1, false);
-    FW_TILE(128, 192, 1, false);
-    FW_TILE(192, 192, 1, false);
-    FW_TILE(256, 192, 1, false);
-    FW_TILE(128, 256, 1, false);
-    FW_TILE(192, 256, 1, false);
-    FW_TILE(256, 256, 1, false);
-    FW_TILE(256, 320, 1, false);
-    FW_TILE(64, 128, 1, true);
-    FW_TILE(128, 128, 1, true);
-    FW_TILE(128, 256, 1, true);
+#define FW_TILE(ROWS, COLUMNS, EACH) \
+    if (c.slices <= 1 && c.rows == ROWS && c.columns == COLUMNS && c.each_cu == EACH) return launch_big<MB_STORE, TO, COLUMNS / 64, ROWS / 64, EACH, false>(c);
+    FW_BIG_WHOLE_TILES(FW_TILE)
+#undef FW_TILE
+#define FW_TILE(ROWS, COLUMNS, EACH) \
+    if (c.slices > 1 && c.rows == ROWS && c.columns == COLUMNS && c.each_cu == EACH) return launch_big<MB_STORE, TO, COLUMNS / 64, ROWS / 64, EACH, true>(c);
+    FW_BIG_CUT_TILES(FW_TILE)
 #undef FW_TILE
     fw_set_error("gemm_mfma_big: no tile of %d x %d, %d on a compute unit, K in %d slices", c.rows, c.columns, c.each_cu, c.slices);
     return -1;

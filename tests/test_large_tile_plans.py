@@ -25,6 +25,17 @@ def test_the_tiles_rows_are_multiples_of_64():
         assert all(tile[0] % 64 == 0 for tile in table)
 
 
+def test_the_estimates_are_of_every_tile_there_is():
+    """The tables' tiles and the kernels' are the same, K cut on those that have it (and on 128 x 256, which a rule of its own chooses)."""
+    have = ctypes.c_size_t(0), ctypes.c_int(0)
+    for mode in range(3):
+        takes = lambda tile, slices: ops.library().fw_gemm_mfma_big_tile_needs(mode, 1000, 1000, 4096, *tile, slices, *map(ctypes.byref, have)) == 0    # noqa: E731
+        tiles = [(rows, columns, each) for rows in range(32, 353, 32) for columns in range(32, 417, 32) for each in (1, 2, 3)]
+        assert {tile for tile in tiles if takes(tile, 1)} == set(ops._TIME_LARGE[mode])
+        cut = {(rows, columns, 1) for rows, columns in ops._TIME_LARGE_CUT.get(mode, {})}
+        assert {tile for tile in tiles if takes(tile, 2)} == (cut | {(128, 256, 1)} if cut else set())
+
+
 def test_what_the_plans_are_made_of_changes_at_their_lines_alone():
     def needs(mode, M, N, K, tile):
         have = ctypes.c_size_t(0), ctypes.c_int(0)
