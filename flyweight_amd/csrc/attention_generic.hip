@@ -173,8 +173,9 @@ __global__ __launch_bounds__(64) void qk_norm_rope_kv_write_rows_kernel(
 // lanes a head, 64 / HEAD_LANES rows side by side, eight rows of a head-vector to a wave; a value's 64 channels a lane each, as above. With a channel a lane a
 // wave's eight rows were eight sums over 64 lanes one behind the other, six trips through the LDS crossbar each, and every query waited for its row's
 // position, segment and page, which keys and values alone need. What is left is the memory's: float32 sums in, bfloat16 out. 2,048 rows of 32 + 16 heads of 64
-// 21.3 -> 12.9 us (2.9 TB/s), 801 rows 12.7 -> 8.2; 1,111 rows of 16 + 8 heads of 128 15.2 -> 10.8. The same bits: the squares
-// are added in the order of the sum over a wave, channels 64 apart, then 32, 16, 8 and 4 over the lanes, 2 and 1 in the lane.
+// 21.3 -> 13.1 us (2.9 TB/s), 801 rows 12.7 -> 8.2; 1,111 rows of 16 + 8 heads of 128 15.2 -> 10.3. The bits of one row to a wave: the squares
+// are rounded and added in the order of the sum over a wave, channels 64 apart, then 32, 16, 8 and 4 over the lanes, 2 and 1 in the lane. (Eight rows one behind the other, as
+// above, have a square fused with the first sum: float32 outputs that are normed were one unit in the last place away from those of fewer rows.)
 template <typename TI> struct four_of { typedef float4 vector; };
 template <> struct four_of<bf16_t> { typedef uint2 vector; };
 __device__ __forceinline__ void four_floats(const float4 v, float (&x)[4]) { x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w; }

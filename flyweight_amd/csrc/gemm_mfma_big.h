@@ -19,7 +19,7 @@
 // The same loop runs on smaller and on wider tiles, 64 to 256 rows by 128 to 320 columns: a round of tiles that the chip's 256 compute units
 // are not full with is as long as a whole one, so the tile follows the shape. 2,048 rows by 3,072 features are 128 tiles of 256 x 192 but exactly 256 of
 // 128 x 192; 2,048 x 4,608 gated over K 1,024 is 288 tiles of 256 x 256, two rounds and 55 us, but 232 of 256 x 320, one and 38; 1,111 x 2,048 over K 2,048 are
-// 40 tiles of 256 x 256 and 153 of 64 x 256: 22 -> 18 us on 128 x 128; 300 x 8,192 gated over K 2,048 42 -> 31. A smaller tile moves more bytes per flop
+// 40 tiles of 256 x 256, 41 us with the launch, and 198 of 64 x 192, 21; 300 x 8,192 gated over K 2,048 42 us on 256 x 256 and 31 on 192 x 128. A smaller tile moves more bytes per flop
 // through LDS and the memory path (which its six stages, or a second workgroup on the compute unit, keep busy), so it is used only where it fills the
 // chip better: the caller compares the products' estimated times.
 //
